@@ -789,6 +789,26 @@ size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, si
     return quant_scratch_bytes(m, layer->in_features) + split_scratch_bytes(m, layer->in_features, layer->out_features);
 }
 
+size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,
+                                            int sum_order)
+{
+    if (!layer || m == 0) return 0;
+    const size_t in = layer->in_features;
+    if (gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, row_blocks(layer->out_features))) return 0;
+    return bitnet_hip_bitlinear_workspace_size(layer, m);
+}
+
+size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
+                                                  const float *gamma, int sum_order)
+{
+    if (!layers || count == 0 || m == 0) return 0;
+    for (size_t j = 0; j < count; ++j)
+        if (!layers[j]) return 0;
+    const size_t in = layers[0]->in_features;
+    if (gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, launch_group_blocks(layers, count))) return 0;
+    return quant_scratch_bytes(m, in);
+}
+
 int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, const size_t *dims, int rank,
                                  const float *gamma, float eps, int sum_order, const float *residual, float *out,
                                  void *workspace, size_t workspace_bytes, int8_t *dbg_q, float *dbg_a_scale,

@@ -1,8 +1,10 @@
-"""ctypes binding of libbitnet_hip.so (the C ABI declared in include/bitnet_hip.h).
+"""Binding of libbitnet_hip.so (the C ABI declared in include/bitnet_hip.h) through ctypes, with the calls a token loop
+makes (BitLinear.forward, forward_multi, DecoderProjections.decode) in a small native module beside this file (_call, built
+from native/call.cpp): the plain call goes through it, anything unusual through the code here, which checks and explains.
 
 The library is the product; this module only moves pointers.  torch is used for device memory and
 streams, nothing else: no function here computes a result on the host or through torch operators, and
-loading fails loudly if the HIP library has not been built.
+loading fails loudly if the HIP library or the native module has not been built.
 
 Class and method names mirror the reference's Rust API so call sites read alike:
   BitLinearConfig / BitLinear      bitnet-quant/src/bitlinear/layer.rs:20-109, forward.rs:14-51
@@ -69,11 +71,12 @@ class BitLinearError(RuntimeError):
 
 
 _lib = None
+_native = None  # the native module; loaded with the library
 
 
 def load_library() -> C.CDLL:
     """Loads the built library; raises if it is missing (there is no fallback path)."""
-    global _lib
+    global _lib, _native
     if _lib is not None:
         return _lib
     if not LIB_PATH.exists():
@@ -123,6 +126,8 @@ def load_library() -> C.CDLL:
         "bitnet_hip_bitlinear_set_bias": (i32, [vp, vp, sz, i32, vp]),
         "bitnet_hip_bitlinear_get_quantized": (i32, [vp, C.POINTER(f32), vp, sz]),
         "bitnet_hip_bitlinear_workspace_size": (sz, [vp, sz]),
+        "bitnet_hip_bitlinear_forward_scratch": (sz, [vp, vp, sz, vp, i32]),
+        "bitnet_hip_bitlinear_forward_multi_scratch": (sz, [C.POINTER(vp), sz, vp, sz, vp, i32]),
         "bitnet_hip_bitlinear_forward": (i32, [vp, vp, C.POINTER(sz), i32, vp, f32, i32, vp, vp, vp, sz, vp, vp, vp, vp]),
         "bitnet_hip_bitlinear_forward_noalloc": (i32, [vp, vp, C.POINTER(sz), i32, vp, f32, i32, vp, vp, vp]),
         "bitnet_hip_bitlinear_forward_multi": (i32, [C.POINTER(vp), sz, vp, sz, vp, f32, i32, C.POINTER(vp), vp, sz, vp]),
@@ -150,7 +155,11 @@ def load_library() -> C.CDLL:
         fn.restype = res
         fn.argtypes = args
     lib._bitnet_declared = tuple(sig)
-    _lib = lib
+    try:
+        from . import _call as native
+    except ImportError as exc:
+        raise ImportError(f"the native call path is not built ({exc}): run `make -C {_PKG_ROOT}`") from exc
+    _lib, _native = lib, native
     return lib
 
 
@@ -866,6 +875,8 @@ class BitLinearConfig:
 class BitLinear:
     """Mirror of BitLinear + BitLinearForward (layer.rs:82-109,113-179; forward.rs:14-136)."""
 
+    _key = None
+
     def __init__(self, config: BitLinearConfig, layer_name: str = "", _handle=None, _owner=None):
         self.config = config
         self.layer_name = layer_name
@@ -873,10 +884,11 @@ class BitLinear:
         lib = load_library()
         if _handle is not None:
             self._h = _handle
-            return
-        h = C.c_void_p()
-        _check(lib.bitnet_hip_bitlinear_create(config.in_features, config.out_features, int(config.use_bias), C.byref(h)))
-        self._h = h
+        else:
+            h = C.c_void_p()
+            _check(lib.bitnet_hip_bitlinear_create(config.in_features, config.out_features, int(config.use_bias), C.byref(h)))
+            self._h = h
+        self._key = (self._h.value, config.in_features, config.out_features)  # what the native call path reads
 
     def __del__(self):
         if getattr(self, "_owner", None) is None and getattr(self, "_h", None) and _lib is not None:
@@ -937,6 +949,11 @@ class BitLinear:
                 workspace: Optional[torch.Tensor] = None):
         """BitLinearForward::forward (forward.rs:55-92).  x: [m,in] or [b,s,in] f32 on the GPU.  out and workspace
         (uint8, at least workspace_size(m) bytes) may be supplied by callers that must not allocate per call."""
+        if self._key is not None and not debug and workspace is None:
+            cfg = self.config
+            y = _native.forward(self._key, x, gamma, residual, out, cfg.rms_norm_eps, cfg.sum_order, stream)
+            if y is not None:
+                return y
         _dev(x, torch.float32, "input")
         _check_optional_operands(self, x, gamma, residual)
         lib = load_library()
@@ -1047,6 +1064,11 @@ class BitLinear:
 
 def forward_multi(layers: Sequence["BitLinear"], x: torch.Tensor, gamma: Optional[torch.Tensor] = None, stream=None):
     """Several BitLinear layers on one input [m, in] (q/k/v, gate/up): one activation quantisation, shared launches."""
+    if _native is not None:
+        cfg = layers[0].config
+        outs = _native.forward_multi(layers, x, gamma, cfg.rms_norm_eps, cfg.sum_order, stream)
+        if outs is not None:
+            return outs
     _dev(x, torch.float32, "input")
     if x.dim() != 2:
         raise BitLinearError(SHAPE_MISMATCH, "forward_multi takes a [m, in] input", [1, layers[0].config.in_features],
@@ -1114,6 +1136,10 @@ class DecoderProjections:
     def decode(self, x: torch.Tensor, out: Optional[torch.Tensor] = None, want_qk: bool = False, stream=None,
                layers: Optional[Sequence[int]] = None):
         """One decode step through all blocks, or through blocks layers[0] .. layers[1]-1 only."""
+        if not want_qk and layers is None and self._h:
+            y = _native.decode(self._h.value, self.hidden, 0, self.layers, x, out, stream)
+            if y is not None:
+                return y
         _dev(x, torch.float32, "x")
         if x.dim() != 2 or x.shape[1] != self.hidden:
             raise BitLinearError(SHAPE_MISMATCH, "decode input", [x.shape[0] if x.dim() else 1, self.hidden], list(x.shape))

@@ -1,0 +1,275 @@
+// The call path of the Python binding for tensors that need no explanation.
+//
+// A decode-sized call (one token through one projection) takes the GPU 3.6 us.  Through ctypes the same call costs the
+// host about 13 us: attribute look-ups and checks in Python, fifteen boxed arguments, two or three allocations through
+// torch.empty and a stream object, each a microsecond or so.  These functions do the same checks on the tensors
+// themselves, allocate the result, call the C ABI and return; what is left of the host's time is the launch.
+//
+// Every function answers None where anything at all is unusual (another type, device, layout or shape than the plain
+// call takes, a status other than OK): the caller then runs its Python path, which makes the same call with every check
+// spelled out and reports the error.  Nothing is computed here.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/impl/DeviceGuardImplInterface.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../../include/bitnet_hip.h"
+
+namespace {
+
+PyObject *raw_stream_of = nullptr;   // torch._C._cuda_getCurrentRawStream
+PyObject *name_cuda_stream = nullptr, *name_key = nullptr;
+
+// The layer's (handle, in_features, out_features), which the binding keeps as the attribute `_key`.
+struct Layer {
+    bitnet_hip_bitlinear *handle = nullptr;
+    int64_t in = 0, out = 0;
+};
+bool read_layer(PyObject *key, Layer &l)
+{
+    if (!PyTuple_CheckExact(key) || PyTuple_GET_SIZE(key) != 3) return false;
+    l.handle = static_cast<bitnet_hip_bitlinear *>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(key, 0)));
+    l.in = PyLong_AsLongLong(PyTuple_GET_ITEM(key, 1));
+    l.out = PyLong_AsLongLong(PyTuple_GET_ITEM(key, 2));
+    return !PyErr_Occurred() && l.handle && l.in > 0 && l.out > 0;
+}
+
+// A dense f32 tensor on the current device, or null.
+const at::Tensor *plain_f32(PyObject *obj, c10::Device &device)
+{
+    if (!THPVariable_CheckExact(obj)) return nullptr;
+    const at::Tensor &t = THPVariable_Unpack(obj);
+    if (!t.is_cuda() || t.scalar_type() != at::kFloat || !t.is_contiguous()) return nullptr;
+    if (device.index() < 0) {
+        device = t.device();
+        if (c10::impl::getDeviceGuardImpl(at::kCUDA)->getDevice() != device) return nullptr;
+    } else if (t.device() != device) {
+        return nullptr;
+    }
+    return &t;
+}
+
+// An optional operand of exactly `count` elements: true with *ptr set (null if absent), false if it is not plain.
+bool optional_f32(PyObject *obj, int64_t count, c10::Device &device, const float **ptr)
+{
+    *ptr = nullptr;
+    if (obj == Py_None) return true;
+    const at::Tensor *t = plain_f32(obj, device);
+    if (!t || t->numel() != count) return false;
+    *ptr = t->const_data_ptr<float>();
+    return true;
+}
+
+bool stream_handle(PyObject *obj, const c10::Device &device, void **stream)
+{
+    PyObject *v;
+    if (obj == Py_None) {
+        PyObject *index = PyLong_FromLong(device.index());
+        if (!index) return false;
+        v = PyObject_CallOneArg(raw_stream_of, index);
+        Py_DECREF(index);
+    } else {
+        v = PyObject_GetAttr(obj, name_cuda_stream);
+    }
+    if (!v) return false;
+    *stream = PyLong_AsVoidPtr(v);
+    Py_DECREF(v);
+    return !PyErr_Occurred();
+}
+
+PyObject *unusual()
+{
+    PyErr_Clear();
+    Py_RETURN_NONE;
+}
+
+at::Tensor new_f32(at::IntArrayRef shape, const at::Tensor &like)
+{
+    at::AutoDispatchBelowADInplaceOrView below;
+    return at::empty(shape, like.options());
+}
+
+// forward(key, x, gamma, residual, out, eps, sum_order, stream)
+PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 8) return unusual();
+    Layer l;
+    c10::Device device(at::kCUDA, -1);
+    if (!read_layer(args[0], l)) return unusual();
+    const at::Tensor *x = plain_f32(args[1], device);
+    if (!x) return unusual();
+    const int64_t rank = x->dim();
+    if ((rank != 2 && rank != 3) || x->size(rank - 1) != l.in) return unusual();
+    const int64_t m = rank == 2 ? x->size(0) : x->size(0) * x->size(1);
+    const float *gamma, *residual;
+    if (m == 0 || !optional_f32(args[2], l.in, device, &gamma) || !optional_f32(args[3], m * l.out, device, &residual))
+        return unusual();
+    const double eps = PyFloat_AsDouble(args[5]);
+    const long order = PyLong_AsLong(args[6]);
+    void *stream;
+    if (PyErr_Occurred() || !stream_handle(args[7], device, &stream)) return unusual();
+    size_t dims[3] = {(size_t)x->size(0), (size_t)x->size(1), rank == 3 ? (size_t)x->size(2) : 0};
+    try {
+        at::Tensor made;
+        const at::Tensor *y;
+        if (args[4] == Py_None) {
+            const int64_t shape[3] = {x->size(0), rank == 3 ? x->size(1) : l.out, l.out};
+            made = new_f32(at::IntArrayRef(shape, rank), *x);
+            y = &made;
+        } else {
+            y = plain_f32(args[4], device);
+            if (!y || y->dim() != rank || y->size(rank - 1) != l.out || y->numel() != m * l.out || y->size(0) != x->size(0))
+                return unusual();
+        }
+        // scratch only where the call runs the stand-alone quantiser; from torch's allocator, in the order of the stream
+        // the tensors are used on
+        const float *xp = x->const_data_ptr<float>();
+        const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch(l.handle, xp, (size_t)m, gamma, (int)order);
+        at::Tensor ws;
+        if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+        float *yp = y->data_ptr<float>();
+        void *wp = ws_bytes ? ws.data_ptr() : nullptr;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = bitnet_hip_bitlinear_forward(l.handle, xp, dims, (int)rank, gamma, (float)eps, (int)order, residual, yp, wp, ws_bytes,
+                                          nullptr, nullptr, nullptr, stream);
+        Py_END_ALLOW_THREADS
+        if (rc != BITNET_HIP_OK) return unusual();
+        if (args[4] != Py_None) {
+            Py_INCREF(args[4]);
+            return args[4];
+        }
+        return THPVariable_Wrap(made);
+    } catch (...) {
+        return unusual();
+    }
+}
+
+// forward_multi(layers, x, gamma, eps, sum_order, stream)
+PyObject *forward_multi(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 6) return unusual();
+    constexpr Py_ssize_t MOST = 16;
+    PyObject *seq = args[0];
+    const bool list = PyList_CheckExact(seq);
+    if (!list && !PyTuple_CheckExact(seq)) return unusual();
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(seq);
+    if (count < 1 || count > MOST) return unusual();
+    bitnet_hip_bitlinear *handles[MOST];
+    int64_t widths[MOST];
+    c10::Device device(at::kCUDA, -1);
+    const at::Tensor *x = plain_f32(args[1], device);
+    if (!x || x->dim() != 2) return unusual();
+    const int64_t m = x->size(0), k = x->size(1);
+    for (Py_ssize_t j = 0; j < count; ++j) {
+        PyObject *key = PyObject_GetAttr(PySequence_Fast_GET_ITEM(seq, j), name_key);
+        Layer l;
+        const bool ok = key && read_layer(key, l) && l.in == k;
+        Py_XDECREF(key);
+        if (!ok) return unusual();
+        handles[j] = l.handle;
+        widths[j] = l.out;
+    }
+    const float *gamma;
+    if (m == 0 || !optional_f32(args[2], k, device, &gamma)) return unusual();
+    const double eps = PyFloat_AsDouble(args[3]);
+    const long order = PyLong_AsLong(args[4]);
+    void *stream;
+    if (PyErr_Occurred() || !stream_handle(args[5], device, &stream)) return unusual();
+    try {
+        at::Tensor outs[MOST];
+        float *ptrs[MOST];
+        for (Py_ssize_t j = 0; j < count; ++j) {
+            outs[j] = new_f32({m, widths[j]}, *x);
+            ptrs[j] = outs[j].data_ptr<float>();
+        }
+        const float *xp = x->const_data_ptr<float>();
+        const size_t ws_bytes = bitnet_hip_bitlinear_forward_multi_scratch(handles, (size_t)count, xp, (size_t)m, gamma, (int)order);
+        at::Tensor ws;
+        if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+        void *wp = ws_bytes ? ws.data_ptr() : nullptr;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = bitnet_hip_bitlinear_forward_multi(handles, (size_t)count, xp, (size_t)m, gamma, (float)eps, (int)order, ptrs, wp,
+                                                ws_bytes, stream);
+        Py_END_ALLOW_THREADS
+        if (rc != BITNET_HIP_OK) return unusual();
+        PyObject *res = PyList_New(count);
+        if (!res) return nullptr;
+        for (Py_ssize_t j = 0; j < count; ++j) {
+            PyObject *t = THPVariable_Wrap(outs[j]);
+            if (!t) {
+                Py_DECREF(res);
+                return nullptr;
+            }
+            PyList_SET_ITEM(res, j, t);
+        }
+        return res;
+    } catch (...) {
+        return unusual();
+    }
+}
+
+// decode(decoder, hidden, begin, end, x, out, stream)
+PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    if (nargs != 7) return unusual();
+    auto *dec = static_cast<bitnet_hip_decoder *>(PyLong_AsVoidPtr(args[0]));
+    const int64_t hidden = PyLong_AsLongLong(args[1]), begin = PyLong_AsLongLong(args[2]), end = PyLong_AsLongLong(args[3]);
+    c10::Device device(at::kCUDA, -1);
+    if (PyErr_Occurred() || !dec || begin < 0 || end < begin) return unusual();
+    const at::Tensor *x = plain_f32(args[4], device);
+    if (!x || x->dim() != 2 || x->size(1) != hidden) return unusual();
+    void *stream;
+    if (!stream_handle(args[6], device, &stream)) return unusual();
+    try {
+        at::Tensor made;
+        const at::Tensor *y;
+        if (args[5] == Py_None) {
+            made = new_f32(x->sizes(), *x);
+            y = &made;
+        } else {
+            y = plain_f32(args[5], device);
+            if (!y || y->sizes() != x->sizes()) return unusual();
+        }
+        const float *xp = x->const_data_ptr<float>();
+        float *yp = y->data_ptr<float>();
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = bitnet_hip_decoder_decode_layers(dec, (size_t)begin, (size_t)end, xp, (size_t)x->size(0), yp, nullptr, nullptr, stream);
+        Py_END_ALLOW_THREADS
+        if (rc != BITNET_HIP_OK) return unusual();
+        if (args[5] != Py_None) {
+            Py_INCREF(args[5]);
+            return args[5];
+        }
+        return THPVariable_Wrap(made);
+    } catch (...) {
+        return unusual();
+    }
+}
+
+PyMethodDef methods[] = {
+    {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
+    {"forward_multi", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward_multi)), METH_FASTCALL, nullptr},
+    {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__call()
+{
+    PyObject *torch_c = PyImport_ImportModule("torch._C");
+    if (!torch_c) return nullptr;
+    raw_stream_of = PyObject_GetAttrString(torch_c, "_cuda_getCurrentRawStream");
+    Py_DECREF(torch_c);
+    name_cuda_stream = PyUnicode_InternFromString("cuda_stream");
+    name_key = PyUnicode_InternFromString("_key");
+    if (!raw_stream_of || !name_cuda_stream || !name_key) return nullptr;
+    return PyModule_Create(&module);
+}

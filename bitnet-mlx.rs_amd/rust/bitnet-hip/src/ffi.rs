@@ -124,6 +124,10 @@ extern "C" {
     pub fn bitnet_hip_bitlinear_get_quantized(layer: *mut bitnet_hip_bitlinear, w_scale: *mut f32, packed: *mut u8,
                                               packed_len: usize) -> c_int;
     pub fn bitnet_hip_bitlinear_workspace_size(layer: *const bitnet_hip_bitlinear, m: usize) -> usize;
+    pub fn bitnet_hip_bitlinear_forward_scratch(layer: *const bitnet_hip_bitlinear, x: *const f32, m: usize, gamma: *const f32,
+                                                sum_order: c_int) -> usize;
+    pub fn bitnet_hip_bitlinear_forward_multi_scratch(layers: *const *mut bitnet_hip_bitlinear, count: usize, x: *const f32,
+                                                      m: usize, gamma: *const f32, sum_order: c_int) -> usize;
     pub fn bitnet_hip_bitlinear_forward(layer: *mut bitnet_hip_bitlinear, x: *const f32, dims: *const usize,
                                         rank: c_int, gamma: *const f32, eps: f32, sum_order: c_int,
                                         residual: *const f32, out: *mut f32, workspace: *mut c_void,

@@ -330,6 +330,10 @@ int bitnet_hip_bitlinear_get_quantized(bitnet_hip_bitlinear *layer, float *w_sca
  * rounded up to 256, plus two arrays of 4 * m bytes rounded up to 256, plus 256) and then runs without the split:
  * same results, 10 to 20 % slower in that range. */
 size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, size_t m);
+/* The same for one particular call: 0 where forward quantises inside its only launch and needs no workspace (decode token
+ * counts on aligned rows), else workspace_size(m).  For callers that allocate per call. */
+size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,
+                                            int sum_order);
 
 /* BitLinearForward::forward (forward.rs:55-92) / BitLinearLayer::forward (transformer_layers.rs:119-201):
  * x has `rank` dimensions `dims` (HOST array); rank 2 [m, in] or rank 3 [b, s, in] (flattened to
@@ -367,6 +371,9 @@ int bitnet_hip_bitlinear_forward_noalloc(bitnet_hip_bitlinear *layer, const floa
 int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
                                        const float *gamma, float eps, int sum_order, float *const *outs,
                                        void *workspace, size_t workspace_bytes, void *stream);
+/* Bytes of workspace that call needs; 0 where it needs none (as bitnet_hip_bitlinear_forward_scratch). */
+size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
+                                                  const float *gamma, int sum_order);
 
 /* The contraction + epilogue of a layer on activations that are already quantised:
  * TernaryProcessor::ternary_matmul (bitnet-inference/src/engine/ternary_operations.rs:87-113) /

@@ -1434,3 +1434,36 @@ def test_launch_chain_and_hand_over_diagnostics():
     assert intact
     with pytest.raises(bh.BitLinearError):
         bh.measure_hop(0, hops=5)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 33, 256), (8, 100, 2560), (9, 33, 260), (40, 64, 301), (130, 96, 512)])
+def test_native_call_path_matches_the_checked_one(m, n, k):
+    """The binding's native call path (plain tensors) against the Python one (taken when a workspace is supplied): the same
+    bits with every combination of operands, two- and three-dimensional inputs, a given output and a given stream; what the
+    native path does not take reaches the Python checks and raises."""
+    rng = np.random.default_rng(m + n + k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "native")
+    layer.update_weights(dev(synth_weights(rng, n, k)))
+    x, g = dev(synth_activations(rng, m, k, outliers=True)), dev(rng.standard_normal(k, dtype=f32))
+    res = dev(rng.standard_normal((m, n), dtype=f32))
+    ws = torch.empty((layer.workspace_size(m),), dtype=torch.uint8, device="cuda")
+    side = torch.cuda.Stream()
+    for gamma in (None, g):
+        for residual in (None, res):
+            want = layer.forward(x, gamma=gamma, residual=residual, workspace=ws)
+            assert torch.equal(layer.forward(x, gamma=gamma, residual=residual), want)
+            assert torch.equal(layer.forward(x.view(1, m, k), gamma=gamma, residual=residual), want.view(1, m, n))
+            out = torch.full((m, n), float("nan"), device="cuda")
+            assert layer.forward(x, gamma=gamma, residual=residual, out=out) is out and torch.equal(out, want)
+            torch.cuda.synchronize()
+            on_side = layer.forward(x, gamma=gamma, residual=residual, stream=side)
+            torch.cuda.synchronize()
+            assert torch.equal(on_side, want)
+    for a, b in zip(bh.forward_multi([layer, layer], x, gamma=g), bh.forward_multi((layer, layer), x, gamma=g, stream=torch.cuda.current_stream())):
+        assert torch.equal(a, b) and torch.equal(a, layer.forward(x, gamma=g))
+    for bad in (lambda: layer.forward(x.cpu()), lambda: layer.forward(x.double()), lambda: layer.forward(x[:, :-1].contiguous()),
+                lambda: layer.forward(x, gamma=g[:-1]), lambda: layer.forward(x, residual=res[:, :-1]), lambda: layer.forward(x[0]),
+                lambda: layer.forward(x, out=torch.empty((m + 1, n), device="cuda")), lambda: bh.forward_multi([layer], x.t()),
+                lambda: bh.BitLinear(layer.config, "no weights").forward(x)):
+        with pytest.raises(bh.BitLinearError):
+            bad()
