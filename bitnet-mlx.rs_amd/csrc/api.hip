@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "staging.hpp"
 
 namespace bitnet {
 
@@ -124,8 +125,10 @@ struct bitnet_hip_bitlinear {
     // readers: forward; writer: set_weights / set_bias (the reference guards weights with a RwLock)
     mutable std::shared_mutex lock;
 
+    bitnet_hip_bitlinear() { staging_retain(); }
     ~bitnet_hip_bitlinear()
     {
+        staging_release();
         if (packed) (void)hipFree(packed);
         if (tiled) (void)hipFree(tiled);
         if (w_scale) (void)hipFree(w_scale);
@@ -371,13 +374,10 @@ int bitnet_hip_absmax_quantize_activations(const float *x, size_t count, int pre
         return fail(BITNET_HIP_UNSUPPORTED, "absmax_quantize_activations: unsupported precision %d", precision);
     if (!stats) return fail(BITNET_HIP_NULL_POINTER, "absmax_quantize_activations: stats is required");
     if (count != 0 && (!x || !values)) return fail(BITNET_HIP_NULL_POINTER, "absmax_quantize_activations: null buffer");
-    DeviceTemp scratch;
-    int rc = scratch.alloc(absmax_quantize_scratch_bytes(count));
+    StreamScratch scratch;
+    int rc = scratch.alloc(absmax_quantize_scratch_bytes(count), as_stream(stream));
     if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_absmax_quantize(x, count, precision, scratch.ptr, values, stats, as_stream(stream));
-    if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipStreamSynchronize(as_stream(stream)));  // the scratch is released on return
-    return BITNET_HIP_OK;
+    return launch_absmax_quantize(x, count, precision, scratch.ptr, values, stats, as_stream(stream));
 }
 
 int bitnet_hip_abs_max(const float *x, size_t count, float *abs_max, void *stream)
@@ -386,14 +386,18 @@ int bitnet_hip_abs_max(const float *x, size_t count, float *abs_max, void *strea
     *abs_max = 0.0f;
     if (count == 0) return BITNET_HIP_OK;
     if (!x) return fail(BITNET_HIP_NULL_POINTER, "abs_max: null buffer");
-    DeviceTemp scratch;
-    int rc = scratch.alloc(absmax_quantize_scratch_bytes(count));
+    HostParts parts;
+    int rc = parts.acquire();
     if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_abs_max(x, count, scratch.ptr, as_stream(stream));
+    const int workgroups = abs_max_workgroups(count, HostParts::MOST);
+    rc = launch_abs_max(x, count, workgroups, parts.answers, parts.ticket, as_stream(stream));
     if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipMemcpyAsync(abs_max, scratch.ptr, sizeof(float), hipMemcpyDeviceToHost, as_stream(stream)));
-    BITNET_HIP_TRY(hipStreamSynchronize(as_stream(stream)));  // the value is the caller's on return, as to_scalar() is
-    return BITNET_HIP_OK;
+    // the value is the caller's on return, as to_scalar() is
+    return parts.wait(as_stream(stream), workgroups, [&](unsigned bits) {
+        float part;
+        memcpy(&part, &bits, sizeof part);
+        *abs_max = part > *abs_max ? part : *abs_max;
+    });
 }
 
 int bitnet_hip_quantize_activations_scaled(const float *x, size_t count, int precision, float scale, int reference_u8,
@@ -402,7 +406,16 @@ int bitnet_hip_quantize_activations_scaled(const float *x, size_t count, int pre
     if (precision != BITNET_HIP_PRECISION_ONE_FIVE_FIVE_BIT && precision != BITNET_HIP_PRECISION_EIGHT_BIT)
         return fail(BITNET_HIP_UNSUPPORTED, "quantize_activations_scaled: unsupported precision %d", precision);
     if (count != 0 && (!x || !values)) return fail(BITNET_HIP_NULL_POINTER, "quantize_activations_scaled: null buffer");
-    return launch_scaled_quantize(x, count, precision, scale, reference_u8 != 0, values, as_stream(stream));
+    return launch_scaled_quantize(x, count, precision, scale, reference_u8 != 0, values, nullptr, as_stream(stream));
+}
+
+int bitnet_hip_quantize_activations_scaled_keep(const float *x, size_t count, int precision, float scale, int reference_u8,
+                                                int8_t *values, float *scale_out, void *stream)
+{
+    if (precision != BITNET_HIP_PRECISION_ONE_FIVE_FIVE_BIT && precision != BITNET_HIP_PRECISION_EIGHT_BIT)
+        return fail(BITNET_HIP_UNSUPPORTED, "quantize_activations_scaled_keep: unsupported precision %d", precision);
+    if (!scale_out || (count != 0 && (!x || !values))) return fail(BITNET_HIP_NULL_POINTER, "quantize_activations_scaled_keep: null buffer");
+    return launch_scaled_quantize(x, count, precision, scale, reference_u8 != 0, values, scale_out, as_stream(stream));
 }
 
 // ---- lookup-table kernels ----------------------------------------------------------------------------
@@ -486,14 +499,17 @@ int bitnet_hip_quantize_weights(const float *w, size_t n, size_t k, int method, 
                                                      threshold_factor, packed, w_scale, q_i8, nullptr, stream);
     if (method != BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP && method != BITNET_HIP_TERNARY_MEAN_THRESHOLD)
         return fail(BITNET_HIP_INVALID_CONFIG, "quantize_weights: unknown method %d", method);
-    DeviceTemp row_sums;
-    int rc = row_sums.alloc(sizeof(double) * (n ? n : 1));
-    if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_quantize_weights(w, n, k, method, threshold_factor, static_cast<double *>(row_sums.ptr), packed,
-                                 w_scale, q_i8, as_stream(stream));
-    if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipStreamSynchronize(as_stream(stream)));  // row_sums is released on return
-    return BITNET_HIP_OK;
+    // The row sums (8 bytes a row) are done with before the codes are written: they take the codes' place where a row has
+    // 8 bytes of them.
+    StreamScratch scratch;
+    void *row_sums = packed;
+    if (k < 32 || (reinterpret_cast<uintptr_t>(packed) & 7) != 0) {
+        int rc = scratch.alloc(sizeof(double) * (n ? n : 1), as_stream(stream));
+        if (rc != BITNET_HIP_OK) return rc;
+        row_sums = scratch.ptr;
+    }
+    return launch_quantize_weights(w, n, k, method, threshold_factor, static_cast<double *>(row_sums), packed,
+                                   w_scale, q_i8, as_stream(stream));
 }
 
 int bitnet_hip_quantize_weights_reference(const float *w, size_t n, size_t k, int ternary_method, int normalize_weights,
@@ -507,14 +523,11 @@ int bitnet_hip_quantize_weights_reference(const float *w, size_t n, size_t k, in
     // WeightQuantizationConfig::validate (weights.rs:120-150)
     if (outlier_threshold < 0.0f) return fail(BITNET_HIP_INVALID_CONFIG, "Outlier threshold cannot be negative");
     if (custom_threshold_factor > 2.0f) return fail(BITNET_HIP_INVALID_CONFIG, "Custom threshold factor must be in range (0, 2]");
-    DeviceTemp scratch;
-    int rc = scratch.alloc(quantize_weights_reference_scratch_bytes(n));
+    StreamScratch scratch;
+    int rc = scratch.alloc(quantize_weights_reference_scratch_bytes(n), as_stream(stream));
     if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_quantize_weights_reference(w, n, k, ternary_method, normalize_weights != 0, outlier_threshold,
-                                           custom_threshold_factor, scratch.ptr, packed, w_scale, q_i8, stats, as_stream(stream));
-    if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipStreamSynchronize(as_stream(stream)));  // the scratch is released on return
-    return BITNET_HIP_OK;
+    return launch_quantize_weights_reference(w, n, k, ternary_method, normalize_weights != 0, outlier_threshold,
+                                             custom_threshold_factor, scratch.ptr, packed, w_scale, q_i8, stats, as_stream(stream));
 }
 
 size_t bitnet_hip_tiled_size(size_t n, size_t k) { return tiled_bytes(n, k); }
@@ -631,26 +644,25 @@ int bitnet_hip_bitlinear_set_weights_f32(bitnet_hip_bitlinear *layer, const floa
         return fail_shape(e, 2, a, 2, "weight matrix");  // BitLinear::update_weights, layer.rs:301-307
     }
     hipStream_t s = as_stream(stream);
-    DeviceTemp w_dev, flat;
+    StreamScratch w_dev;
+    Upload up;
     const float *src = w;
+    int rc = BITNET_HIP_OK;
     if (!on_device) {
-        int rc = w_dev.alloc(sizeof(float) * n * k);
+        rc = w_dev.alloc(sizeof(float) * n * k, s);
+        if (rc == BITNET_HIP_OK) rc = up.copy(w_dev.ptr, w, sizeof(float) * n * k, s);
         if (rc != BITNET_HIP_OK) return rc;
-        BITNET_HIP_TRY(hipMemcpyAsync(w_dev.ptr, w, sizeof(float) * n * k, hipMemcpyHostToDevice, s));
         src = static_cast<const float *>(w_dev.ptr);
     }
-    int rc = flat.alloc((n * k + 3) / 4);
-    if (rc != BITNET_HIP_OK) return rc;
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
-    rc = bitnet_hip_quantize_weights(src, rows, cols, method, threshold_factor, static_cast<uint8_t *>(flat.ptr),
-                                     layer->w_scale, nullptr, stream);
+    // the codes in the source's orientation first; [in, out] ones give way to the canonical [out, in] bytes after the re-tiling
+    rc = bitnet_hip_quantize_weights(src, rows, cols, method, threshold_factor, layer->packed, layer->w_scale, nullptr, stream);
     if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_retile(static_cast<const uint8_t *>(flat.ptr), n, k, layout, layer->tiled, s);
-    if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_untile(layer->tiled, n, k, layer->packed, s);  // canonical [out, in] bytes
+    rc = launch_retile(layer->packed, n, k, layout, layer->tiled, s, layout == BITNET_HIP_LAYOUT_OUT_IN ? nullptr : layer->packed);
     if (rc != BITNET_HIP_OK) return rc;
     BITNET_HIP_TRY(hipStreamSynchronize(s));
+    up.done();
     layer->has_weights = true;
     return BITNET_HIP_OK;
 }
@@ -668,11 +680,14 @@ int bitnet_hip_bitlinear_set_weights_packed(bitnet_hip_bitlinear *layer, const u
     hipStream_t s = as_stream(stream);
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
-    BITNET_HIP_TRY(hipMemcpyAsync(layer->packed, packed, need, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-    BITNET_HIP_TRY(hipMemcpyAsync(layer->w_scale, &w_scale, sizeof(float), hipMemcpyHostToDevice, s));
-    int rc = launch_retile(layer->packed, n, k, BITNET_HIP_LAYOUT_OUT_IN, layer->tiled, s);
+    int rc = BITNET_HIP_OK;
+    Upload up;
+    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(layer->packed, packed, need, hipMemcpyDeviceToDevice, s));
+    else rc = up.copy(layer->packed, packed, need, s);
+    if (rc == BITNET_HIP_OK) rc = launch_retile(layer->packed, n, k, BITNET_HIP_LAYOUT_OUT_IN, layer->tiled, s, nullptr, w_scale, layer->w_scale);
     if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipStreamSynchronize(s));  // w_scale is read from the caller's stack
+    BITNET_HIP_TRY(hipStreamSynchronize(s));  // forwards on other streams may follow
+    up.done();
     layer->has_weights = true;
     return BITNET_HIP_OK;
 }
@@ -687,22 +702,23 @@ int bitnet_hip_bitlinear_set_weights_base3(bitnet_hip_bitlinear *layer, const ui
         return fail_shape(e, 1, a, 1, "base-3 packed weight bytes");
     }
     hipStream_t s = as_stream(stream);
-    DeviceTemp staged;  // the base-3 bytes on the device
+    StreamScratch staged;  // the base-3 bytes on the device
+    Upload up;
     const uint8_t *src = packed;
     if (!on_device) {
-        int rc = staged.alloc(need);
+        int rc = staged.alloc(need, s);
+        if (rc == BITNET_HIP_OK) rc = up.copy(staged.ptr, packed, need, s);
         if (rc != BITNET_HIP_OK) return rc;
-        BITNET_HIP_TRY(hipMemcpyAsync(staged.ptr, packed, need, hipMemcpyHostToDevice, s));
         src = static_cast<const uint8_t *>(staged.ptr);
     }
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
     int rc = launch_base3_to_2bit(src, n * k, layer->packed, s);
     if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipMemcpyAsync(layer->w_scale, &w_scale, sizeof(float), hipMemcpyHostToDevice, s));
-    rc = launch_retile(layer->packed, n, k, BITNET_HIP_LAYOUT_OUT_IN, layer->tiled, s);
+    rc = launch_retile(layer->packed, n, k, BITNET_HIP_LAYOUT_OUT_IN, layer->tiled, s, nullptr, w_scale, layer->w_scale);
     if (rc != BITNET_HIP_OK) return rc;
-    BITNET_HIP_TRY(hipStreamSynchronize(s));  // w_scale is read from the caller's stack; `staged` is freed on return
+    BITNET_HIP_TRY(hipStreamSynchronize(s));  // forwards on other streams may follow
+    up.done();
     layer->has_weights = true;
     return BITNET_HIP_OK;
 }
@@ -731,19 +747,18 @@ int bitnet_hip_bitlinear_set_weights_gguf(bitnet_hip_bitlinear *layer, const uin
     else memcpy(header, data, 8);
     if (scale_out) *scale_out = header[0];
     if (offset_out) *offset_out = header[1];
-    // the codes start 8 bytes into the tensor: stage them at an aligned device address, in their own orientation
-    DeviceTemp flat;
-    int rc = flat.alloc(codes);
-    if (rc != BITNET_HIP_OK) return rc;
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
-    BITNET_HIP_TRY(hipMemcpyAsync(flat.ptr, data + 8, codes, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-    BITNET_HIP_TRY(hipMemcpyAsync(layer->w_scale, &header[0], sizeof(float), hipMemcpyHostToDevice, s));
-    rc = launch_retile(static_cast<const uint8_t *>(flat.ptr), n, k, layout, layer->tiled, s);
-    if (rc != BITNET_HIP_OK) return rc;
-    rc = launch_untile(layer->tiled, n, k, layer->packed, s);  // canonical [out, in] bytes, code 3 stored as code 1
+    // The codes start 8 bytes into the tensor; they go to an aligned address, the layer's own bytes, in their own orientation,
+    // and give way there to the canonical form ([out, in] order, code 3 stored as code 1).
+    Upload up;
+    int rc = BITNET_HIP_OK;
+    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(layer->packed, data + 8, codes, hipMemcpyDeviceToDevice, s));
+    else rc = up.copy(layer->packed, data + 8, codes, s);
+    if (rc == BITNET_HIP_OK) rc = launch_retile(layer->packed, n, k, layout, layer->tiled, s, layer->packed, header[0], layer->w_scale);
     if (rc != BITNET_HIP_OK) return rc;
     BITNET_HIP_TRY(hipStreamSynchronize(s));
+    up.done();
     layer->has_weights = true;
     return BITNET_HIP_OK;
 }
@@ -770,15 +785,13 @@ int bitnet_hip_bitlinear_get_quantized(bitnet_hip_bitlinear *layer, float *w_sca
     std::shared_lock<std::shared_mutex> guard(layer->lock);
     if (!layer->has_weights) return fail(BITNET_HIP_NOT_INITIALIZED, "get_quantized: the layer has no weights yet");
     BITNET_HIP_TRY(hipDeviceSynchronize());
-    if (w_scale) BITNET_HIP_TRY(hipMemcpy(w_scale, layer->w_scale, sizeof(float), hipMemcpyDeviceToHost));
-    if (packed) {
-        size_t need = (layer->in_features * layer->out_features + 3) / 4;
-        if (packed_len < need) {
-            size_t e[1] = {need}, a[1] = {packed_len};
-            return fail_shape(e, 1, a, 1, "packed weight bytes");
-        }
-        BITNET_HIP_TRY(hipMemcpy(packed, layer->packed, need, hipMemcpyDeviceToHost));
+    const size_t need = (layer->in_features * layer->out_features + 3) / 4;
+    if (packed && packed_len < need) {
+        size_t e[1] = {need}, a[1] = {packed_len};
+        return fail_shape(e, 1, a, 1, "packed weight bytes");
     }
+    if (packed) return download(packed, layer->packed, need, w_scale ? layer->w_scale : nullptr, w_scale, nullptr);
+    if (w_scale) BITNET_HIP_TRY(hipMemcpy(w_scale, layer->w_scale, sizeof(float), hipMemcpyDeviceToHost));
     return BITNET_HIP_OK;
 }
 

@@ -24,10 +24,14 @@ int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size
 // bytes; stats: 4 floats (scale, mse, min, max)
 size_t absmax_quantize_scratch_bytes(size_t n);
 int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratch, int8_t *q, float *stats, hipStream_t stream);
-// max |x| of a tensor into the first float of `scratch` (absmax_quantize_scratch_bytes(n) bytes), and the quantiser of
-// DynamicActivationQuantizer with the scale given from outside (activations.rs:269-294, 315-360)
-int launch_abs_max(const float *x, size_t n, void *scratch, hipStream_t stream);
-int launch_scaled_quantize(const float *x, size_t n, int precision, float scale, int reference_u8, int8_t *q, hipStream_t stream);
+// max |x| of a tensor for the waiting host, a partial maximum from each of `workgroups` (answers and ticket of a HostParts,
+// staging.hpp; abs_max_workgroups: how many the tensor is worth, at most `most`), and the quantiser of
+// DynamicActivationQuantizer with the scale given from outside (activations.rs:269-294, 315-360), which also stores the
+// scale to scale_out unless that is null
+int abs_max_workgroups(size_t n, int most);
+int launch_abs_max(const float *x, size_t n, int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream);
+int launch_scaled_quantize(const float *x, size_t n, int precision, float scale, int reference_u8, int8_t *q, float *scale_out,
+                           hipStream_t stream);
 
 // weight_prep.hip
 int launch_pack_2bit(const int8_t *q, size_t count, uint8_t *packed, hipStream_t stream);
@@ -47,7 +51,10 @@ size_t quantize_weights_reference_scratch_bytes(size_t n);
 int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int method, int normalize, float outlier_threshold,
                                       float custom_factor, void *scratch, uint8_t *packed, float *w_scale, int8_t *q_i8,
                                       float *stats, hipStream_t stream);
-int launch_retile(const uint8_t *packed, size_t n, size_t k, int layout, uint8_t *tiled, hipStream_t stream);
+// canonical (optional): the weights back in flat [n, k] order with code 3 stored as code 1; w_scale_out (optional): receives
+// w_scale (a value the host holds, stored without a copy of its own)
+int launch_retile(const uint8_t *packed, size_t n, size_t k, int layout, uint8_t *tiled, hipStream_t stream,
+                  uint8_t *canonical = nullptr, float w_scale = 0.0f, float *w_scale_out = nullptr);
 int launch_untile(const uint8_t *tiled, size_t n, size_t k, uint8_t *packed, hipStream_t stream);
 
 // gemv_base3.hip: the decode GEMV on base-3 bytes (five values per byte) in their own streaming layout

@@ -104,61 +104,154 @@ __device__ __forceinline__ double wave_sum_f64(double p)
     return p;
 }
 
+// Element c of a row for c = lane, lane + 64, .. below k, in ascending order, with up to U loads in flight: the f64 chains
+// of the row sums fix the order of the additions, not that of the loads.
+template <int U, typename F>
+__device__ __forceinline__ void for_row(const float *row, size_t k, int lane, F &&add)
+{
+    size_t c = lane;
+    for (size_t end = 64 * U; end <= k; end += 64 * U, c += 64 * U) {  // uniform: every lane of the wavefront is in it
+        float v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) v[i] = row[c + 64 * i];
+#pragma unroll
+        for (int i = 0; i < U; ++i) add(v[i], c + 64 * i);
+    }
+    for (; c < k; c += 64) add(row[c], c);
+}
+
 // Sum of |w| of one row in f64: lane l adds columns l, l+64, ... in ascending order, then the
-// butterfly.  One wavefront per row.
+// butterfly.  One wavefront per row.  Bound by the read of the matrix (6912 x 2560: 12 us with ten loads in flight, 16.7 with one).
 __global__ __launch_bounds__(256) void absmean_rows_kernel(const float *w, size_t n, size_t k, double *row_sums)
 {
     const int lane = threadIdx.x;
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (row >= n) return;
-    const float *wr = w + row * k;
     double s = 0.0;
-    for (size_t c = lane; c < k; c += 64) s = s + (double)fabsf(wr[c]);
+    for_row<10>(w + row * k, k, lane, [&](float v, size_t) { s = s + (double)fabsf(v); });
     s = wave_sum_f64(s);
     if (lane == 0) row_sums[row] = s;
 }
 
-// Combines the row sums the same way (lane l takes rows l, l+64, ...) and writes mean|W| as f32.
-__global__ __launch_bounds__(64) void absmean_final_kernel(const double *row_sums, size_t n, size_t k, float *w_scale)
+// The row sums of NACC accumulators (accumulator a at row_sums + a * n), combined in the declared order: lane l takes rows
+// l, l+64, ..., then the butterfly.  One workgroup of 1024 threads: all of them bring a round of rows into LDS, loads in
+// flight together; the chain of additions belongs to one wavefront per accumulator.  6912 rows: 26 us as one wavefront that
+// waits for every load, 5 us with the rows through LDS.  The result is valid in wavefront a for accumulator a.
+template <int NACC>
+__device__ __forceinline__ double combine_row_sums(const double *row_sums, size_t n)
 {
-    const int lane = threadIdx.x;
+    constexpr int CH = 7168 / NACC / 64 * 64, U = (NACC * CH + 1023) / 1024;  // rows a round: 56 KiB of LDS
+    __shared__ double sh[NACC * CH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     double s = 0.0;
-    for (size_t r = lane; r < n; r += 64) s = s + row_sums[r];
-    s = wave_sum_f64(s);
-    if (lane == 0) *w_scale = (n == 0 || k == 0) ? 0.0f : (float)(s / ((double)n * (double)k));
-}
-
-__device__ __forceinline__ int ternarize_one(float w, int method, float s, float thr)
-{
-    if (method == BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP) {
-        // RoundClip(w / s, -1, 1); s == 0 gives 0
-        if (s == 0.0f) return 0;
-        float r = roundf(f32_div(w, s));
-        if (r != r) return 0;
-        r = fminf(fmaxf(r, -1.0f), 1.0f);
-        return (int)r;
+    for (size_t r0 = 0; r0 < n; r0 += CH) {
+        const int rows = n - r0 < (size_t)CH ? (int)(n - r0) : CH;
+        double v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int e = tid + 1024 * i, a = min(e / CH, NACC - 1), r = min(e - a * CH, rows - 1);
+            v[i] = row_sums[a * n + r0 + r];
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+            if (tid + 1024 * i < NACC * CH) sh[tid + 1024 * i] = v[i];
+        __syncthreads();
+        if (wave < NACC) {
+            const double *mine = sh + wave * CH;
+            int r = lane;
+            for (; r + 15 * 64 < rows; r += 16 * 64) {
+                double t[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) t[i] = mine[r + 64 * i];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s = s + t[i];
+            }
+            for (; r < rows; r += 64) s = s + mine[r];
+        }
+        __syncthreads();
     }
-    return w > thr ? 1 : (w < -thr ? -1 : 0);  // strict comparisons, bitnet-quant/src/simd/ternary.rs:75-83
+    return wave_sum_f64(s);
 }
 
+// Writes mean|W| as f32.
+__global__ __launch_bounds__(1024) void absmean_final_kernel(const double *row_sums, size_t n, size_t k, float *w_scale)
+{
+    const double s = combine_row_sums<1>(row_sums, n);
+    if (threadIdx.x == 0) *w_scale = (n == 0 || k == 0) ? 0.0f : (float)(s / ((double)n * (double)k));
+}
+
+// What turns a weight into -1, 0 or +1: +1 where w >= hi (or w > hi if strict), -1 where -w does.
+struct TernaryRule {
+    float hi;
+    bool strict;
+};
+// RoundClip(w / s, -1, 1) is +1 exactly where the correctly rounded quotient is at least 1/2, that is where w / s is at
+// least 1/2 - 2^-26 (halfway to the float below 1/2; the tie goes to 1/2, whose significand is even), so where w is at
+// least the smallest float not below s * (1/2 - 2^-26), a product that is exact in f64 (24 + 25 significand bits).  One
+// comparison per weight in place of a division and a rounding.  s = 0 and a non-finite s make every weight 0.
+__device__ __forceinline__ TernaryRule ternary_rule(int method, float factor, float s)
+{
+    if (method != BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP) return {f32_mul(factor, s), true};  // strict, bitnet-quant/src/simd/ternary.rs:75-83
+    if (!(s > 0.0f) || s == __builtin_inff()) return {__builtin_nanf(""), true};  // no comparison holds
+    const double bound = (double)s * (0.5 - 0x1p-26);
+    float hi = (float)bound;
+    if ((double)hi < bound) hi = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, hi) + 1u);  // the next float up (hi >= 0)
+    return {hi, false};
+}
+__device__ __forceinline__ int ternarize_one(float w, const TernaryRule &t)
+{
+    return t.strict ? (w > t.hi ? 1 : (w < -t.hi ? -1 : 0)) : (w >= t.hi ? 1 : (w <= -t.hi ? -1 : 0));
+}
+
+// Four lanes that hold the code bytes of four consecutive groups of four weights each end up with the dword of all four.
+__device__ __forceinline__ uint32_t quad_dword(uint32_t byte, int lane)
+{
+    uint32_t w = byte << (8 * (lane & 3));
+    w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);
+    w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x4E, 0xf, 0xf, true);
+    return w;
+}
+
+// A wavefront takes 1024 consecutive weights: load i (of four) is one 16-byte chunk a lane, chunks in lane order, so loads
+// are dense; lane l keeps the dword of group i = l mod 4 of its quad and stores it: 256 bytes a wavefront.  Bound by the
+// read (6912 x 2560: 24 us as a thread per byte with four scalar loads and a division each, 10 us now).
 __global__ __launch_bounds__(256) void ternarize_pack_kernel(const float *w, size_t count, int method,
                                                              float factor, const float *w_scale,
-                                                             uint8_t *packed, int8_t *q_i8, size_t nbytes)
+                                                             uint8_t *packed, int8_t *q_i8, bool dense)
 {
-    size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbytes) return;
-    const float s = *w_scale;
-    const float thr = f32_mul(factor, s);
-    unsigned byte = 0;
-    for (int j = 0; j < 4; ++j) {
-        size_t i = 4 * b + j;
-        if (i < count) {
-            int t = ternarize_one(w[i], method, s, thr);
-            if (q_i8) q_i8[i] = (int8_t)t;
-            byte |= ((unsigned)(t + 1) & 3u) << (2 * j);
+    const int lane = threadIdx.x & 63;
+    const TernaryRule rule = ternary_rule(method, factor, *w_scale);
+    size_t base = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 1024;
+    for (; dense && base + 1024 <= count; base += (size_t)gridDim.x * 4096) {
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const float4 *>(w + base + 256 * i + 4 * lane);
+        uint32_t mine = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t0 = ternarize_one(v[i].x, rule), t1 = ternarize_one(v[i].y, rule), t2 = ternarize_one(v[i].z, rule),
+                      t3 = ternarize_one(v[i].w, rule);
+            if (q_i8)
+                *reinterpret_cast<uint32_t *>(q_i8 + base + 256 * i + 4 * lane) =
+                    (uint32_t)(t0 & 0xff) | ((uint32_t)(t1 & 0xff) << 8) | ((uint32_t)(t2 & 0xff) << 16) | ((uint32_t)(t3 & 0xff) << 24);
+            const uint32_t d = quad_dword((uint32_t)((t0 + 1) | ((t1 + 1) << 2) | ((t2 + 1) << 4) | ((t3 + 1) << 6)), lane);
+            if ((lane & 3) == i) mine = d;
+        }
+        *reinterpret_cast<uint32_t *>(packed + base / 4 + 64 * (lane & 3) + (lane & ~3)) = mine;
+    }
+    // the end of the matrix, and buffers that are not aligned: a byte per lane and round
+    for (; base < count; base += (size_t)gridDim.x * 4096) {
+        const size_t end = base + 1024 < count ? base + 1024 : count;
+        for (size_t e = base + 4 * lane; e < end; e += 256) {
+            unsigned byte = 0;
+            for (int j = 0; j < 4 && e + j < end; ++j) {
+                const int t = ternarize_one(w[e + j], rule);
+                if (q_i8) q_i8[e + j] = (int8_t)t;
+                byte |= (unsigned)(t + 1) << (2 * j);
+            }
+            packed[e / 4] = (uint8_t)byte;
         }
     }
-    packed[b] = (uint8_t)byte;
 }
 
 // ---- BitNetWeightQuantizer::quantize, the reference's weight pipeline (bitnet-quant/src/quantization/weights.rs:568-611)
@@ -169,11 +262,12 @@ __global__ __launch_bounds__(256) void ternarize_pack_kernel(const float *w, siz
 //   q = sign(w'') * [|w''| > thr]                        apply_ternary_quantization, :482-496
 //   scale = sum(w''*q) / sum(q*q)                        compute_ternary_scale, :546-559
 //
-// Nothing but the packed codes and the scale is written: w'' is recomputed from w wherever it is needed (two
-// f32 operations and a clamp).  Every tensor-wide sum is carried in f64 in the order of the absmean kernels above
-// (per row: lane l adds columns l, l+64, ..., then the butterfly; the row sums the same way), so the f32 scalars
-// have the bits the CPU restatement of the same order has.  The scalars stay on the device in WqState; one
-// wavefront finishes each reduction and derives the next stage's scalars.
+// Nothing but the packed codes and the scale is written: w'' is recomputed from w wherever it is needed (the short
+// division by the deviation, which is the same for the whole tensor, and a clamp).  Every tensor-wide sum is carried in f64
+// in the order of the absmean kernels above (per row: lane l adds columns l, l+64, ..., then the butterfly; the row sums
+// the same way), so the f32 scalars have the bits the CPU restatement of the same order has.  The scalars stay on the
+// device in WqState; one workgroup finishes each reduction and derives the next stage's scalars.  The last pass (the
+// scale's sums) knows the threshold, so it writes the codes too where rows start on bytes.
 struct WqState {
     float mean, sd;            // normalisation (0, 1 when switched off)
     float clip_mean, clip_mad; // centre and mean |.| of the normalised tensor
@@ -187,16 +281,46 @@ static_assert(sizeof(WqState) == 12 * sizeof(float), "stats are returned as 12 f
 enum WqPass { WQ_SUM = 0, WQ_SQDIFF, WQ_CLIP_STATS, WQ_ABS_STATS, WQ_OPTIMAL, WQ_SCALE };
 constexpr int WQ_MAX_ACC = 10;
 
-__device__ __forceinline__ float wq_normalised(float w, const WqState &st, bool normalize)
+__device__ __forceinline__ void wq_publish(const WqState &st, int clip, float *w_scale, float *stats)
 {
-    return normalize ? f32_div(w - st.mean, st.sd) : w;
+    *w_scale = st.scale;
+    if (stats) {
+        const float v[12] = {st.mean, st.sd, st.clip_mean, st.clip_mad, clip ? st.lo : 0.0f, clip ? st.hi : 0.0f,
+                             st.mean_abs, st.max_abs, st.thr, st.num, st.den, st.scale};
+        for (int i = 0; i < 12; ++i) stats[i] = v[i];
+    }
 }
-__device__ __forceinline__ float wq_processed(float w, const WqState &st, bool normalize, bool clip)
+
+// The scalars of a pass: the state, and the divisor of the normalisation prepared for div_by_invariant (ieee.hpp).
+struct WqView {
+    WqState st;
+    float recip;
+    bool fast, normalize, clip;
+};
+__device__ __forceinline__ WqView wq_view(const WqState *state, int normalize, int clip)
 {
-    float x = wq_normalised(w, st, normalize);
-    if (clip) {
-        x = x > st.hi ? st.hi : x;
-        x = x < st.lo ? st.lo : x;
+    WqView v;
+    v.st = *state;
+    v.recip = f32_div(1.0f, v.st.sd);
+    v.fast = invariant_divisor_ok(v.st.sd);
+    v.normalize = normalize != 0;
+    v.clip = clip != 0;
+    return v;
+}
+__device__ __forceinline__ float wq_normalised(float w, const WqView &p)
+{
+    if (!p.normalize) return w;
+    const float d = w - p.st.mean;
+    // the short division where every lane's dividend allows it: the same bits as the plain one
+    if (p.fast && __builtin_amdgcn_ballot_w64(!dividend_ok(d)) == 0) return div_by_invariant_unchecked(d, p.st.sd, p.recip);
+    return f32_div(d, p.st.sd);
+}
+__device__ __forceinline__ float wq_processed(float w, const WqView &p)
+{
+    float x = wq_normalised(w, p);
+    if (p.clip) {
+        x = x > p.st.hi ? p.st.hi : x;
+        x = x < p.st.lo ? p.st.lo : x;
     }
     return x;
 }
@@ -204,58 +328,69 @@ __device__ __forceinline__ float wq_code(float x, float thr) { return x > thr ? 
 
 __constant__ float wq_factors[10] = {0.3f, 0.4f, 0.5f, 0.6f, 0.7f, 0.8f, 0.9f, 1.0f, 1.1f, 1.2f};
 
+constexpr int wq_accumulators(int pass) { return pass == WQ_OPTIMAL ? 10 : ((pass == WQ_CLIP_STATS || pass == WQ_SCALE) ? 2 : 1); }
+
 // One wavefront per row; accumulator a of row r goes to row_sums[a * n + r] (and the row's max |.| to row_max[r]).
+// packed (WQ_SCALE, k a multiple of 4, else null): the codes of the row, four columns a byte, put together by the quad of
+// lanes that holds them; q_i8 as ever optional.  Bound by the read of the matrix.
 template <int PASS>
 __global__ __launch_bounds__(256) void wq_rows_kernel(const float *w, size_t n, size_t k, const WqState *state, int normalize,
-                                                      int clip, double *row_sums, float *row_max)
+                                                      int clip, double *row_sums, float *row_max, uint8_t *packed, int8_t *q_i8)
 {
-    constexpr int NACC = PASS == WQ_OPTIMAL ? 10 : ((PASS == WQ_CLIP_STATS || PASS == WQ_SCALE) ? 2 : 1);
+    constexpr int NACC = wq_accumulators(PASS);
     const int lane = threadIdx.x;
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (row >= n) return;
-    const WqState st = *state;
-    const float *wr = w + row * k;
+    const WqView p = wq_view(state, normalize, clip);
     double acc[NACC];
 #pragma unroll
     for (int a = 0; a < NACC; ++a) acc[a] = 0.0;
     float mx = 0.0f;
+    int nonzero = 0;  // of the row
     float cand[PASS == WQ_OPTIMAL ? 10 : 1];
     if constexpr (PASS == WQ_OPTIMAL) {
 #pragma unroll
-        for (int f = 0; f < 10; ++f) cand[f] = f32_mul(st.mean_abs, wq_factors[f]);
+        for (int f = 0; f < 10; ++f) cand[f] = f32_mul(p.st.mean_abs, wq_factors[f]);
     }
-    for (size_t c = lane; c < k; c += 64) {
-        const float v = wr[c];
+    for_row<PASS == WQ_OPTIMAL ? 4 : 10>(w + row * k, k, lane, [&](float v, size_t c) {
         if constexpr (PASS == WQ_SUM) {
             acc[0] = acc[0] + (double)v;
         } else if constexpr (PASS == WQ_SQDIFF) {
-            const float d = v - st.mean;
+            const float d = v - p.st.mean;
             acc[0] = acc[0] + (double)f32_mul(d, d);
         } else if constexpr (PASS == WQ_CLIP_STATS) {
-            const float x = wq_normalised(v, st, normalize != 0);
+            const float x = wq_normalised(v, p);
             acc[0] = acc[0] + (double)x;
             acc[1] = acc[1] + (double)fabsf(x);
         } else if constexpr (PASS == WQ_ABS_STATS) {
-            const float ax = fabsf(wq_processed(v, st, normalize != 0, clip != 0));
+            const float ax = fabsf(wq_processed(v, p));
             acc[0] = acc[0] + (double)ax;
             mx = fmaxf(mx, ax);
         } else if constexpr (PASS == WQ_OPTIMAL) {
-            const float x = wq_processed(v, st, normalize != 0, clip != 0);
+            const float x = wq_processed(v, p);
 #pragma unroll
             for (int f = 0; f < 10; ++f) {
                 const float d = x - wq_code(x, cand[f]);
                 acc[f] = acc[f] + (double)f32_mul(d, d);
             }
         } else {
-            const float x = wq_processed(v, st, normalize != 0, clip != 0);
-            const float q = wq_code(x, st.thr);
+            const float x = wq_processed(v, p);
+            const float q = wq_code(x, p.st.thr);
             acc[0] = acc[0] + (double)f32_mul(x, q);
-            acc[1] = acc[1] + (double)f32_mul(q, q);
+            nonzero += __popcll(__builtin_amdgcn_ballot_w64(q != 0.0f));  // sum of q * q: a count, exact in any order
+            if (packed) {  // k % 4 == 0: the four columns of a byte are active together
+                const int t = (int)q;
+                if (q_i8) q_i8[row * k + c] = (int8_t)t;
+                uint32_t b = (uint32_t)(t + 1) << (2 * (lane & 3));
+                b |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0xB1, 0xf, 0xf, true);
+                b |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, 0x4E, 0xf, 0xf, true);
+                if ((lane & 3) == 0) packed[(row * k + c) / 4] = (uint8_t)b;
+            }
         }
-    }
+    });
 #pragma unroll
     for (int a = 0; a < NACC; ++a) {
-        const double s = wave_sum_f64(acc[a]);
+        const double s = PASS == WQ_SCALE && a == 1 ? (double)nonzero : wave_sum_f64(acc[a]);
         if (lane == 0) row_sums[(size_t)a * n + row] = s;
     }
     if constexpr (PASS == WQ_ABS_STATS) {
@@ -265,28 +400,29 @@ __global__ __launch_bounds__(256) void wq_rows_kernel(const float *w, size_t n, 
     }
 }
 
-// One wavefront: combines the row sums of every accumulator (lane l takes rows l, l+64, ...; butterfly) and derives
-// the scalars of the next stage.  method: TernaryMethod 0..4; custom <= 0: the method's own factor.
+// One workgroup: combines the row sums of every accumulator and derives the scalars of the next stage.  method:
+// TernaryMethod 0..4; custom <= 0: the method's own factor.  WQ_SCALE, the last stage, also publishes the scale and
+// (optionally) the twelve scalars.
 template <int PASS>
-__global__ __launch_bounds__(64) void wq_final_kernel(const double *row_sums, const float *row_max, size_t n, size_t k,
-                                                      WqState *state, int method, float outlier_threshold, float custom)
+__global__ __launch_bounds__(1024) void wq_final_kernel(const double *row_sums, const float *row_max, size_t n, size_t k,
+                                                        WqState *state, int method, float outlier_threshold, float custom,
+                                                        int clip, float *w_scale, float *stats)
 {
-    constexpr int NACC = PASS == WQ_OPTIMAL ? 10 : ((PASS == WQ_CLIP_STATS || PASS == WQ_SCALE) ? 2 : 1);
-    const int lane = threadIdx.x;
-    double tot[NACC];
-#pragma unroll
-    for (int a = 0; a < NACC; ++a) {
-        double s = 0.0;
-        for (size_t r = lane; r < n; r += 64) s = s + row_sums[(size_t)a * n + r];
-        tot[a] = wave_sum_f64(s);
-    }
-    float mx = 0.0f;
+    constexpr int NACC = wq_accumulators(PASS);
+    __shared__ double tot[NACC];
+    __shared__ float maxima[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if constexpr (PASS == WQ_ABS_STATS) {
-        for (size_t r = lane; r < n; r += 64) mx = fmaxf(mx, row_max[r]);
+        float mx = 0.0f;
+        for (size_t r = threadIdx.x; r < n; r += 1024) mx = fmaxf(mx, row_max[r]);
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        if (lane == 0) maxima[wave] = mx;
     }
-    if (lane != 0) return;
+    const double s = combine_row_sums<NACC>(row_sums, n);
+    if (lane == 0 && wave < NACC) tot[wave] = s;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
     const double count = (double)n * (double)k;
     WqState st = *state;
     if constexpr (PASS == WQ_SUM) {
@@ -301,6 +437,8 @@ __global__ __launch_bounds__(64) void wq_final_kernel(const double *row_sums, co
         st.lo = st.clip_mean - spread;
         st.hi = st.clip_mean + spread;
     } else if constexpr (PASS == WQ_ABS_STATS) {
+        float mx = 0.0f;
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, maxima[i]);
         st.mean_abs = (float)(tot[0] / count);
         st.max_abs = mx;
         const bool has_custom = custom > 0.0f;
@@ -323,31 +461,33 @@ __global__ __launch_bounds__(64) void wq_final_kernel(const double *row_sums, co
         st.num = (float)tot[0];
         st.den = (float)tot[1];
         st.scale = fabsf(st.den) < 1.1920929e-07f ? 1.0f : f32_div(st.num, st.den);
+        wq_publish(st, clip, w_scale, stats);
     }
     *state = st;
 }
 
-__global__ void wq_init_kernel(WqState *state)
+__global__ void wq_init_kernel(WqState *state, int empty, int clip, float *w_scale, float *stats)
 {
     WqState st;
     st.mean = 0.0f; st.sd = 1.0f; st.clip_mean = 0.0f; st.clip_mad = 0.0f; st.lo = -__builtin_inff(); st.hi = __builtin_inff();
     st.mean_abs = 0.0f; st.max_abs = 0.0f; st.thr = 0.0f; st.num = 0.0f; st.den = 0.0f; st.scale = 1.0f;
     *state = st;
+    if (empty) wq_publish(st, clip, w_scale, stats);  // an empty tensor: no pass follows
 }
 
-// Ternarise the processed tensor with the threshold found, pack; thread b builds byte b.  Also publishes the scale and
-// (optionally) the twelve scalars.
+// Ternarise the processed tensor with the threshold found, pack; thread b builds byte b (widths that are no multiple of 4,
+// where a byte holds columns of two rows).
 __global__ __launch_bounds__(256) void wq_ternarize_pack_kernel(const float *w, size_t count, const WqState *state, int normalize,
                                                                 int clip, uint8_t *packed, int8_t *q_i8, size_t nbytes)
 {
     size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nbytes) return;
-    const WqState st = *state;
+    const WqView p = wq_view(state, normalize, clip);
     unsigned byte = 0;
     for (int j = 0; j < 4; ++j) {
         size_t i = 4 * b + j;
         if (i < count) {
-            const int t = (int)wq_code(wq_processed(w[i], st, normalize != 0, clip != 0), st.thr);
+            const int t = (int)wq_code(wq_processed(w[i], p), p.st.thr);
             if (q_i8) q_i8[i] = (int8_t)t;
             byte |= ((unsigned)(t + 1) & 3u) << (2 * j);
         }
@@ -355,70 +495,136 @@ __global__ __launch_bounds__(256) void wq_ternarize_pack_kernel(const float *w, 
     packed[b] = (uint8_t)byte;
 }
 
-__global__ void wq_publish_kernel(const WqState *state, int clip, float *w_scale, float *stats)
+// Codes of 16 consecutive elements e0 .. e0 + 15 (element j at bits 2j), code 3 as code 1; elements from `valid` on hold
+// code 1.  Reads the bytes that hold valid elements and no others.
+__device__ __forceinline__ uint32_t load_codes16(const uint8_t *packed, size_t e0, int valid, bool dwords)
 {
-    const WqState st = *state;
-    *w_scale = st.scale;
-    if (stats) {
-        const float v[12] = {st.mean, st.sd, st.clip_mean, st.clip_mad, clip ? st.lo : 0.0f, clip ? st.hi : 0.0f,
-                             st.mean_abs, st.max_abs, st.thr, st.num, st.den, st.scale};
-        for (int i = 0; i < 12; ++i) stats[i] = v[i];
-    }
-}
-
-__device__ __forceinline__ unsigned code_at(const uint8_t *packed, size_t e)
-{
-    return (packed[e >> 2] >> (2 * (e & 3))) & 3u;
-}
-
-// One thread builds one dword (16 weights of one row) of the tiled layout.
-__global__ __launch_bounds__(256) void retile_kernel(const uint8_t *packed, size_t n, size_t k, int layout,
-                                                     uint32_t *tiled, size_t kt_count, size_t total_dwords)
-{
-    size_t d = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= total_dwords) return;
-    size_t tile = d >> 8;
-    unsigned wd = (unsigned)(d & 255);
-    unsigned slot = wd >> 2, t = wd & 3;
-    unsigned r = slot & 15, g = 4 * t + (slot >> 4);
-    size_t rb = tile / kt_count, kt = tile % kt_count;
-    size_t row = rb * TILE_ROWS + r;
-    size_t kbase = kt * TILE_K + (size_t)g * 16;
-    uint32_t word = 0;
-    for (int j = 0; j < 16; ++j) {
-        size_t kk = kbase + j;
-        unsigned code = 1;
-        if (row < n && kk < k) {
-            size_t e = layout == BITNET_HIP_LAYOUT_OUT_IN ? row * k + kk : kk * n + row;
-            code = code_at(packed, e);
-            if (code == 3) code = 1;
+    uint32_t s = 0x55555555u;
+    if (valid > 0) {
+        if (dwords && valid >= 16) {  // e0 a multiple of 16, packed aligned to 4 bytes
+            s = reinterpret_cast<const uint32_t *>(packed)[e0 >> 4];
+        } else {
+            const int n = valid < 16 ? valid : 16;
+            const unsigned first = 2 * (unsigned)(e0 & 3);  // bit of element e0 in its byte
+            const size_t b0 = e0 >> 2, bytes = (first + 2 * n + 7) >> 3;
+            unsigned long long v = 0;
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+                if ((size_t)i < bytes) v |= (unsigned long long)packed[b0 + i] << (8 * i);
+            s = (uint32_t)(v >> first);
+            if (n < 16) s = (s & ((1u << (2 * n)) - 1u)) | (0x55555555u & ~((1u << (2 * n)) - 1u));
         }
-        word |= code << (2 * (j >> 2) + 8 * (j & 3));
     }
-    tiled[d] = word;
+    const uint32_t three = s & (s >> 1) & 0x55555555u;
+    return s & ~(three << 1);
 }
 
-// Inverse: one thread rebuilds one byte of the flat [n, k] packing.
+// 4 x 4 transposition of the 2-bit fields of a dword: field 4q + b (flat order) <-> bits 2q + 8b (tile order).  Its own inverse.
+__device__ __forceinline__ uint32_t interleave16(uint32_t s)
+{
+    uint32_t t = ((s >> 6) ^ s) & 0x00cc00ccu;
+    s ^= t ^ (t << 6);
+    t = ((s >> 12) ^ s) & 0x0000f0f0u;
+    return s ^ t ^ (t << 12);
+}
+
+// [out, in] source: one thread builds one dword (16 weights of one row) of the tiled layout.  A workgroup reads whole
+// 64-byte pieces of 16 rows and writes 1 KiB, for RETILE_KT k-tiles of a row block (a workgroup per tile is bound by the
+// dispatch of workgroups).  canonical (optional; rows of whole dwords only): the same codes back in flat order.  w_scale_out
+// (optional): receives w_scale.  (6912 x 2560: 37 us element by element.)
+constexpr unsigned RETILE_KT = 5;
+__global__ __launch_bounds__(256) void retile_kernel(const uint8_t *packed, size_t n, size_t k, uint32_t *tiled, unsigned kt_count,
+                                                     bool dwords, uint32_t *canonical, float w_scale, float *w_scale_out)
+{
+    const unsigned kt0 = blockIdx.x * RETILE_KT, rb = blockIdx.y + gridDim.y * blockIdx.z;
+    if (kt0 == 0 && rb == 0 && threadIdx.x == 0 && w_scale_out) *w_scale_out = w_scale;
+    if ((size_t)rb * TILE_ROWS >= n) return;
+    const unsigned slot = threadIdx.x >> 2, t = threadIdx.x & 3;
+    const size_t row = (size_t)rb * TILE_ROWS + (slot & 15);
+    uint32_t s[RETILE_KT];
+    int valid[RETILE_KT];
+#pragma unroll
+    for (unsigned i = 0; i < RETILE_KT; ++i) {
+        const size_t col = (size_t)(kt0 + i) * TILE_K + 64 * t + 16 * (slot >> 4);
+        valid[i] = row < n && col < k ? (int)(k - col < 16 ? k - col : 16) : 0;
+        s[i] = load_codes16(packed, row * k + col, valid[i], dwords);
+    }
+#pragma unroll
+    for (unsigned i = 0; i < RETILE_KT; ++i) {
+        if (kt0 + i >= kt_count) break;  // uniform
+        const size_t col = (size_t)(kt0 + i) * TILE_K + 64 * t + 16 * (slot >> 4);
+        if (canonical && valid[i]) canonical[(row * k + col) >> 4] = s[i];
+        tiled[((size_t)rb * kt_count + kt0 + i) * 256 + threadIdx.x] = interleave16(s[i]);
+    }
+}
+
+// [in, out] source: one thread takes the 16 columns of one dword position for all 16 rows of a row block (16 codes of 16
+// source rows each), transposes them in registers and stores 16 dwords.  Consecutive lanes take consecutive row blocks, so
+// they read consecutive dwords of a source row.
+__global__ __launch_bounds__(64) void retile_in_out_kernel(const uint8_t *packed, size_t n, size_t k, uint32_t *tiled, unsigned kt_count,
+                                                           bool dwords, float w_scale, float *w_scale_out)
+{
+    const size_t rb = (size_t)blockIdx.x * 64 + threadIdx.x;
+    const unsigned piece = blockIdx.y + gridDim.y * blockIdx.z;
+    const unsigned g = piece & 15, kt = piece >> 4;  // column group: columns 64 * (g >> 2) + 16 * (g & 3) of the tile
+    if (rb == 0 && piece == 0 && w_scale_out) *w_scale_out = w_scale;
+    if (rb * TILE_ROWS >= n || kt >= kt_count) return;
+    const unsigned t = g >> 2, kq = g & 3;
+    const size_t row0 = rb * TILE_ROWS, col0 = (size_t)kt * TILE_K + 64 * t + 16 * kq;
+    const int rows = (int)(n - row0 < 16 ? n - row0 : 16);
+    uint32_t src[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) src[j] = load_codes16(packed, (col0 + j) * n + row0, col0 + j < k ? rows : 0, dwords);
+    uint32_t *out = tiled + (rb * kt_count + kt) * 256 + 64 * kq + t;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        uint32_t word = 0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) word |= ((src[j] >> (2 * r)) & 3u) << (2 * (j >> 2) + 8 * (j & 3));
+        out[4 * r] = word;
+    }
+}
+
+// Inverse, rows of whole dwords (k a multiple of 16): one thread rebuilds the 16 elements of one dword of the flat packing.
+__global__ __launch_bounds__(256) void untile_rows_kernel(const uint32_t *tiled, unsigned dwords_per_row, size_t n, uint32_t *packed,
+                                                          unsigned kt_count)
+{
+    const unsigned d = blockIdx.x * 256 + threadIdx.x;
+    const size_t row = blockIdx.y + (size_t)gridDim.y * blockIdx.z;
+    if (d >= dwords_per_row || row >= n) return;
+    const unsigned kt = d >> 4, g = d & 15;
+    const size_t tile = (row / TILE_ROWS) * kt_count + kt;
+    packed[row * dwords_per_row + d] = interleave16(tiled[tile * 256 + 64 * (g & 3) + 4 * (row % TILE_ROWS) + (g >> 2)]);
+}
+
+// Inverse, any width: one thread rebuilds one byte of the flat [n, k] packing.
 __global__ __launch_bounds__(256) void untile_kernel(const uint32_t *tiled, size_t n, size_t k, uint8_t *packed,
                                                      size_t kt_count, size_t nbytes)
 {
     size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nbytes) return;
     const size_t count = n * k;
+    size_t row = 4 * b / k, kk = 4 * b - row * k;
     unsigned byte = 0;
     for (int j = 0; j < 4; ++j) {
-        size_t e = 4 * b + j;
-        if (e >= count) break;
-        size_t row = e / k, kk = e % k;
+        if (4 * b + j >= count) break;
         size_t tile = (row / TILE_ROWS) * kt_count + kk / TILE_K;
         unsigned g = (unsigned)((kk % TILE_K) / 16), c = (unsigned)(kk % 16);
         unsigned wd = (((g & 3) * 16 + (unsigned)(row % TILE_ROWS)) << 2) + (g >> 2);
         uint32_t word = tiled[tile * 256 + wd];
         byte |= ((word >> (2 * (c >> 2) + 8 * (c & 3))) & 3u) << (2 * j);
+        if (++kk == k) { kk = 0; ++row; }
     }
     packed[b] = (uint8_t)byte;
 }
 
+// Grid dimensions y and z that together cover `items` (y is limited to 65535).
+inline dim3 rows_grid(unsigned x, size_t items)
+{
+    const unsigned y = items < 32768 ? (unsigned)items : 32768u;
+    return dim3(x, y, (unsigned)((items + y - 1) / y));
+}
+inline bool aligned(const void *ptr, size_t a) { return (reinterpret_cast<uintptr_t>(ptr) % a) == 0; }
 inline unsigned blocks_for(size_t items, unsigned per_block) { return (unsigned)((items + per_block - 1) / per_block); }
 
 }  // namespace
@@ -481,12 +687,15 @@ int launch_quantize_weights(const float *w, size_t n, size_t k, int method, floa
         hipLaunchKernelGGL(absmean_rows_kernel, dim3(blocks_for(n, 4)), dim3(64, 4), 0, stream, w, n, k, row_sums);
         BITNET_HIP_CHECK_LAUNCH("absmean_rows_kernel");
     }
-    hipLaunchKernelGGL(absmean_final_kernel, dim3(1), dim3(64), 0, stream, row_sums, n, k, w_scale);
+    hipLaunchKernelGGL(absmean_final_kernel, dim3(1), dim3(1024), 0, stream, row_sums, n, k, w_scale);
     BITNET_HIP_CHECK_LAUNCH("absmean_final_kernel");
-    size_t count = n * k, nbytes = (count + 3) / 4;
-    if (nbytes == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(ternarize_pack_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, w, count,
-                       method, threshold_factor, w_scale, packed, q_i8, nbytes);
+    const size_t count = n * k;
+    if (count == 0) return BITNET_HIP_OK;
+    const bool dense = aligned(w, 16) && aligned(packed, 4) && (!q_i8 || aligned(q_i8, 4));
+    // at most eight workgroups a compute unit: one round, and no more dispatches than that
+    const unsigned blocks = blocks_for(count, 4096);
+    hipLaunchKernelGGL(ternarize_pack_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, stream, w, count,
+                       method, threshold_factor, w_scale, packed, q_i8, dense);
     BITNET_HIP_CHECK_LAUNCH("ternarize_pack_kernel");
     return BITNET_HIP_OK;
 }
@@ -505,54 +714,72 @@ int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int me
     double *row_sums = reinterpret_cast<double *>(static_cast<uint8_t *>(scratch) + 256);
     float *row_max = reinterpret_cast<float *>(row_sums + WQ_MAX_ACC * (n ? n : 1));
     const int clip = outlier_threshold > 0.0f ? 1 : 0;
-    hipLaunchKernelGGL(wq_init_kernel, dim3(1), dim3(1), 0, stream, state);
-    BITNET_HIP_CHECK_LAUNCH("wq_init_kernel");
     const size_t count = n * k, nbytes = (count + 3) / 4;
-    if (count != 0) {
-        const dim3 rgrid(blocks_for(n, 4)), rblock(64, 4);
+    hipLaunchKernelGGL(wq_init_kernel, dim3(1), dim3(1), 0, stream, state, count == 0 ? 1 : 0, clip, w_scale, stats);
+    BITNET_HIP_CHECK_LAUNCH("wq_init_kernel");
+    if (count == 0) return BITNET_HIP_OK;
+    const dim3 rgrid(blocks_for(n, 4)), rblock(64, 4);
+    uint8_t *packed_rows = k % 4 == 0 ? packed : nullptr;  // rows of whole bytes: the last pass writes the codes
 #define BITNET_WQ_PASS(PASS)                                                                                              \
     do {                                                                                                                  \
         hipLaunchKernelGGL((wq_rows_kernel<PASS>), rgrid, rblock, 0, stream, w, n, k, state, normalize, clip, row_sums,  \
-                           row_max);                                                                                      \
+                           row_max, packed_rows, q_i8);                                                                   \
         BITNET_HIP_CHECK_LAUNCH("wq_rows_kernel");                                                                        \
-        hipLaunchKernelGGL((wq_final_kernel<PASS>), dim3(1), dim3(64), 0, stream, row_sums, row_max, n, k, state, method, \
-                           outlier_threshold, custom_factor);                                                             \
+        hipLaunchKernelGGL((wq_final_kernel<PASS>), dim3(1), dim3(1024), 0, stream, row_sums, row_max, n, k, state,       \
+                           method, outlier_threshold, custom_factor, clip, w_scale, stats);                               \
         BITNET_HIP_CHECK_LAUNCH("wq_final_kernel");                                                                       \
     } while (0)
-        if (normalize) {
-            BITNET_WQ_PASS(WQ_SUM);
-            BITNET_WQ_PASS(WQ_SQDIFF);
-        }
-        if (clip) BITNET_WQ_PASS(WQ_CLIP_STATS);
-        BITNET_WQ_PASS(WQ_ABS_STATS);
-        if (method == 3 && !(custom_factor > 0.0f)) BITNET_WQ_PASS(WQ_OPTIMAL);
-        BITNET_WQ_PASS(WQ_SCALE);
+    if (normalize) {
+        BITNET_WQ_PASS(WQ_SUM);
+        BITNET_WQ_PASS(WQ_SQDIFF);
+    }
+    if (clip) BITNET_WQ_PASS(WQ_CLIP_STATS);
+    BITNET_WQ_PASS(WQ_ABS_STATS);
+    if (method == 3 && !(custom_factor > 0.0f)) BITNET_WQ_PASS(WQ_OPTIMAL);
+    BITNET_WQ_PASS(WQ_SCALE);
 #undef BITNET_WQ_PASS
+    if (!packed_rows) {
         hipLaunchKernelGGL(wq_ternarize_pack_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, w, count, state,
                            normalize, clip, packed, q_i8, nbytes);
         BITNET_HIP_CHECK_LAUNCH("wq_ternarize_pack_kernel");
     }
-    hipLaunchKernelGGL(wq_publish_kernel, dim3(1), dim3(1), 0, stream, state, clip, w_scale, stats);
-    BITNET_HIP_CHECK_LAUNCH("wq_publish_kernel");
     return BITNET_HIP_OK;
 }
 
-int launch_retile(const uint8_t *packed, size_t n, size_t k, int layout, uint8_t *tiled, hipStream_t stream)
+int launch_retile(const uint8_t *packed, size_t n, size_t k, int layout, uint8_t *tiled, hipStream_t stream, uint8_t *canonical,
+                  float w_scale, float *w_scale_out)
 {
-    size_t total_dwords = tiled_bytes(n, k) / 4;
-    if (total_dwords == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(retile_kernel, dim3(blocks_for(total_dwords, 256)), dim3(256), 0, stream, packed, n, k,
-                       layout, reinterpret_cast<uint32_t *>(tiled), k_tiles(k), total_dwords);
-    BITNET_HIP_CHECK_LAUNCH("retile_kernel");
-    return BITNET_HIP_OK;
+    if (tiled_bytes(n, k) == 0) return BITNET_HIP_OK;
+    uint32_t *out = reinterpret_cast<uint32_t *>(tiled);
+    const unsigned kt_count = (unsigned)k_tiles(k);
+    if (layout == BITNET_HIP_LAYOUT_OUT_IN) {
+        const bool dwords = k % 16 == 0 && aligned(packed, 4);
+        uint32_t *back = canonical && k % 16 == 0 && aligned(canonical, 4) ? reinterpret_cast<uint32_t *>(canonical) : nullptr;
+        hipLaunchKernelGGL(retile_kernel, rows_grid((kt_count + RETILE_KT - 1) / RETILE_KT, row_blocks(n)), dim3(256), 0, stream, packed, n, k, out, kt_count, dwords,
+                           back, w_scale, w_scale_out);
+        BITNET_HIP_CHECK_LAUNCH("retile_kernel");
+        if (back || !canonical) return BITNET_HIP_OK;
+    } else {
+        hipLaunchKernelGGL(retile_in_out_kernel, rows_grid(blocks_for(row_blocks(n), 64), 16 * (size_t)kt_count), dim3(64), 0, stream,
+                           packed, n, k, out, kt_count, n % 16 == 0 && aligned(packed, 4), w_scale, w_scale_out);
+        BITNET_HIP_CHECK_LAUNCH("retile_in_out_kernel");
+        if (!canonical) return BITNET_HIP_OK;
+    }
+    return launch_untile(tiled, n, k, canonical, stream);
 }
 
 int launch_untile(const uint8_t *tiled, size_t n, size_t k, uint8_t *packed, hipStream_t stream)
 {
     size_t nbytes = (n * k + 3) / 4;
     if (nbytes == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(untile_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream,
-                       reinterpret_cast<const uint32_t *>(tiled), n, k, packed, k_tiles(k), nbytes);
+    const uint32_t *src = reinterpret_cast<const uint32_t *>(tiled);
+    if (k % 16 == 0 && aligned(packed, 4)) {
+        hipLaunchKernelGGL(untile_rows_kernel, rows_grid(blocks_for(k / 16, 256), n), dim3(256), 0, stream, src, (unsigned)(k / 16), n,
+                           reinterpret_cast<uint32_t *>(packed), (unsigned)k_tiles(k));
+        BITNET_HIP_CHECK_LAUNCH("untile_rows_kernel");
+        return BITNET_HIP_OK;
+    }
+    hipLaunchKernelGGL(untile_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, src, n, k, packed, k_tiles(k), nbytes);
     BITNET_HIP_CHECK_LAUNCH("untile_kernel");
     return BITNET_HIP_OK;
 }

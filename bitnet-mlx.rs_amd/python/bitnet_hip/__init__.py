@@ -98,6 +98,7 @@ def load_library() -> C.CDLL:
         "bitnet_hip_absmax_quantize_activations": (i32, [vp, sz, i32, vp, vp, vp]),
         "bitnet_hip_abs_max": (i32, [vp, sz, C.POINTER(C.c_float), vp]),
         "bitnet_hip_quantize_activations_scaled": (i32, [vp, sz, i32, f32, i32, vp, vp]),
+        "bitnet_hip_quantize_activations_scaled_keep": (i32, [vp, sz, i32, f32, i32, vp, vp, vp]),
         "bitnet_hip_lookup_compute": (i32, [i32, vp, sz, vp, sz, vp, sz, vp]),
         "bitnet_hip_packed_size": (sz, [sz]),
         "bitnet_hip_pack_ternary_2bit": (i32, [vp, sz, vp, vp]),
@@ -465,6 +466,10 @@ class DynamicScaleState:
 
 def abs_max(x: torch.Tensor, stream=None) -> float:
     """max |x| over the tensor, on the host (activations.abs().max_all().to_scalar())."""
+    if _native is not None:
+        v = _native.abs_max(x, stream)
+        if v is not None:
+            return v
     _dev(x, torch.float32, "x")
     out = C.c_float(0.0)
     _check(load_library().bitnet_hip_abs_max(_ptr(x), x.numel(), C.byref(out), _stream(stream)))
@@ -474,11 +479,20 @@ def abs_max(x: torch.Tensor, stream=None) -> float:
 def quantize_activations_scaled(x: torch.Tensor, precision: int, scale: float, reference_u8: bool = False, stream=None) -> torch.Tensor:
     """DynamicActivationQuantizer::quantize with the scale given: int8 values (uint8 with reference_u8, the reference's
     literal clamp(0, 255) of its 8-bit branch)."""
-    _dev(x, torch.float32, "x")
-    values = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-    _check(load_library().bitnet_hip_quantize_activations_scaled(_ptr(x), x.numel(), precision, float(scale),
-                                                                 1 if reference_u8 else 0, _ptr(values), _stream(stream)))
-    return values.view(torch.uint8) if reference_u8 and precision == QuantizationPrecision.EightBit else values
+    return _quantize_scaled(x, precision, scale, reference_u8, stream)[0]
+
+
+def _quantize_scaled(x: torch.Tensor, precision: int, scale: float, reference_u8: bool, stream=None):
+    """(values, the scale as a [1] tensor on the device)"""
+    pair = _native.quantize_scaled(x, precision, float(scale), reference_u8, stream) if _native is not None else None
+    if pair is None:
+        lib = load_library()
+        _dev(x, torch.float32, "x")
+        pair = (torch.empty(x.shape, dtype=torch.int8, device=x.device), torch.empty((1,), dtype=torch.float32, device=x.device))
+        _check(lib.bitnet_hip_quantize_activations_scaled_keep(_ptr(x), x.numel(), precision, float(scale), 1 if reference_u8 else 0,
+                                                               _ptr(pair[0]), _ptr(pair[1]), _stream(stream)))
+    values, scales = pair
+    return (values.view(torch.uint8) if reference_u8 and precision == QuantizationPrecision.EightBit else values), scales
 
 
 class DynamicActivationQuantizer:
@@ -509,10 +523,9 @@ class DynamicActivationQuantizer:
         x = activations if activations.dtype == torch.float32 else activations.float()
         x = x.contiguous()
         scale = float(self.state.ema_scale) if self.state.ema_scale is not None else abs_max(x)
-        values = quantize_activations_scaled(x, self.config.precision, scale, self.reference_u8)
+        values, scales = _quantize_scaled(x, self.config.precision, scale, self.reference_u8)
         bits = 1.58 if self.config.precision == QuantizationPrecision.OneFiveFiveBit else 8.0
         stats = {"elements_count": activations.numel(), "scale_factor": scale, "compression_ratio": 32.0 / bits}
-        scales = torch.tensor([scale], dtype=torch.float32, device=activations.device)
         return QuantizedActivation(values, scales, None, tuple(activations.shape), self.config.precision, stats)
 
     def dequantize(self, quantized: QuantizedActivation) -> torch.Tensor:

@@ -252,7 +252,58 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     }
 }
 
+// abs_max(x, stream): the float, or None
+PyObject *abs_max(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    c10::Device device(at::kCUDA, -1);
+    if (nargs != 2) return unusual();
+    const at::Tensor *x = plain_f32(args[0], device);
+    void *stream;
+    if (!x || !stream_handle(args[1], device, &stream)) return unusual();
+    const float *xp = x->const_data_ptr<float>();
+    const size_t count = (size_t)x->numel();
+    float v = 0.0f;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bitnet_hip_abs_max(xp, count, &v, stream);
+    Py_END_ALLOW_THREADS
+    return rc == BITNET_HIP_OK ? PyFloat_FromDouble(v) : unusual();
+}
+
+// quantize_scaled(x, precision, scale, reference_u8, stream): (int8 values, scale tensor [1])
+PyObject *quantize_scaled(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    c10::Device device(at::kCUDA, -1);
+    if (nargs != 5) return unusual();
+    const at::Tensor *x = plain_f32(args[0], device);
+    const long precision = PyLong_AsLong(args[1]);
+    const double scale = PyFloat_AsDouble(args[2]);
+    const int u8 = PyObject_IsTrue(args[3]);
+    void *stream;
+    if (!x || PyErr_Occurred() || u8 < 0 || !stream_handle(args[4], device, &stream)) return unusual();
+    try {
+        at::Tensor values, scales;
+        {
+            at::AutoDispatchBelowADInplaceOrView below;
+            values = at::empty(x->sizes(), x->options().dtype(at::kChar));
+            scales = at::empty({1}, x->options());
+        }
+        if (bitnet_hip_quantize_activations_scaled_keep(x->const_data_ptr<float>(), (size_t)x->numel(), (int)precision, (float)scale, u8,
+                                                        values.data_ptr<int8_t>(), scales.data_ptr<float>(), stream) != BITNET_HIP_OK)
+            return unusual();
+        PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales);
+        PyObject *pair = v && sc ? PyTuple_Pack(2, v, sc) : nullptr;
+        Py_XDECREF(v);
+        Py_XDECREF(sc);
+        return pair;
+    } catch (...) {
+        return unusual();
+    }
+}
+
 PyMethodDef methods[] = {
+    {"abs_max", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(abs_max)), METH_FASTCALL, nullptr},
+    {"quantize_scaled", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize_scaled)), METH_FASTCALL, nullptr},
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
     {"forward_multi", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward_multi)), METH_FASTCALL, nullptr},
     {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, nullptr},

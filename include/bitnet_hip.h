@@ -154,7 +154,7 @@ int bitnet_hip_absmax_quantize_activations(const float *x, size_t count, int pre
 /* The two device steps of DynamicActivationQuantizer (bitnet-quant/src/quantization/activations.rs:203-454), whose
  * state (exponential moving average of the scale, history window, warm-up counter) lives on the host, where the
  * reference keeps it:
- *   bitnet_hip_abs_max: max |x| over the tensor into *abs_max, a HOST float; waits for the stream, as
+ *   bitnet_hip_abs_max: max |x| over the tensor into *abs_max, a HOST float; waits for the result, as
  *     activations.abs().max_all().to_scalar() does (compute_dynamic_scale, :241-267; calibrate, :472-475).
  *   bitnet_hip_quantize_activations_scaled: DynamicActivationQuantizer::quantize with the scale given
  *     (quantize_int8 :269-275, quantize_ternary_activation :277-294): y = x * (float)(1.0 / (double)scale);
@@ -163,6 +163,9 @@ int bitnet_hip_absmax_quantize_activations(const float *x, size_t count, int pre
 int bitnet_hip_abs_max(const float *x, size_t count, float *abs_max, void *stream);
 int bitnet_hip_quantize_activations_scaled(const float *x, size_t count, int precision, float scale, int reference_u8,
                                            int8_t *values, void *stream);
+/* The same, and the scale into *scale_out (one DEVICE float: the scale tensor of the QuantizedActivation). */
+int bitnet_hip_quantize_activations_scaled_keep(const float *x, size_t count, int precision, float scale, int reference_u8,
+                                                int8_t *values, float *scale_out, void *stream);
 
 /* ---- lookup-table kernels --------------------------------------------------------------------- */
 

@@ -1467,3 +1467,51 @@ def test_native_call_path_matches_the_checked_one(m, n, k):
                 lambda: bh.BitLinear(layer.config, "no weights").forward(x)):
         with pytest.raises(bh.BitLinearError):
             bad()
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (9000, 8), (1025, 33), (3, 600), (64, 700), (20, 1300), (100, 6404)])
+@pytest.mark.parametrize("method", [None, bh.TernaryMethod.MeanThreshold, bh.TernaryMethod.OptimalThreshold])
+def test_weight_quantisers_at_the_edges_of_their_batches(n, k, method):
+    """Rows shorter and longer than a batch of loads, rows that share bytes, more rows than one round of the final sums, and an
+    absmean whose rounding boundary is hit exactly (half the mean, and its neighbours)."""
+    rng = np.random.default_rng(n + k)
+    w = synth_weights(rng, n, k)
+    if method is None:
+        w[:] = np.where(rng.random((n, k)) < 0.5, f32(0.0137) * f32(0.5), f32(0.0137) * f32(1.5))
+        for _ in range(3):  # the mean settles: half of it and the floats around it, in either sign, replace the small half
+            s = orc.quantize_weights_absmean(w)[1]
+            half = s * f32(0.5)
+            edge = np.array([half, np.nextafter(half, f32(0)), np.nextafter(half, f32(1))], dtype=f32)
+            w = np.where(np.abs(w) < s, rng.choice(np.concatenate([edge, -edge]), size=w.shape), w).astype(f32)
+        q, s = orc.quantize_weights_absmean(w)
+        packed, scale, q_dev = bh.quantize_weights(dev(w), want_i8=True)
+        assert np.array_equal(host(q_dev), q) and f32(host(scale)[0]) == s and np.array_equal(host(packed), orc.pack_2bit(q))
+        off = torch.empty((n * k + 1,), device="cuda")[1:].view(n, k)  # not 16-byte aligned
+        off.copy_(dev(w))
+        assert torch.equal(bh.quantize_weights(off)[0], packed)
+    else:
+        got = bh.BitNetWeightQuantizer(bh.WeightQuantizationConfig(ternary_method=method)).quantize(dev(w))
+        q, scale, _, stats = orc.quantize_weights_reference(w, method=method, want_details=True)
+        assert np.array_equal(host(got.values), q) and np.array_equal(host(got.packed), orc.pack_2bit(q))
+        assert host(got.scales)[0] == scale and all(f32(got.stats[name]) == v for name, v in stats.items())
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (17, 257), (40, 1000), (33, 48), (2048, 4100), (1040, 2064)])
+@pytest.mark.parametrize("layout", [bh.LAYOUT_OUT_IN, bh.LAYOUT_IN_OUT])
+def test_layers_loaded_from_the_host_give_their_bytes_back(n, k, layout):
+    """GGUF codes through the pinned chunks (more than one of them, a last one that is not full) and below their size, re-tiled
+    from both orientations at widths that are and are not whole dwords, code 3 included: the layer's bytes and tiles."""
+    rng = np.random.default_rng(n + k)
+    raw = rng.integers(0, 256, size=(n * k + 3) // 4, dtype=np.uint8)
+    w = orc.unpack_2bit(raw, n * k)
+    w = w.reshape(n, k) if layout == bh.LAYOUT_OUT_IN else np.ascontiguousarray(w.reshape(k, n).T)
+    header = np.array([0.75, 0.0], dtype=f32).view(np.uint8)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "loaded")
+    for data in (torch.from_numpy(np.concatenate([header, raw])), dev(np.concatenate([header, raw]))):
+        assert layer.load_gguf_ternary(data, layout=layout) == (0.75, 0.0)
+        packed, scale = layer.get_quantized_weights()
+        assert scale == 0.75 and np.array_equal(packed.numpy(), orc.pack_2bit(w))
+        tiled = bh.retile_weights(dev(raw), n, k, layout)
+        assert np.array_equal(host(bh.untile_weights(tiled, n, k)), orc.pack_2bit(w))
+        x = synth_activations(rng, 2, k)
+        assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, orc.pack_2bit(w), n, f32(0.75))[0])
