@@ -2,12 +2,13 @@
 // declared summation order are in rowquant.hpp; the decode GEMV runs the same code inside its prologue).
 //
 // Three launch shapes, same bits:
-//   act_quant_block_kernel    one 256-thread workgroup per token row, the row held in registers between the three
+//   act_quant_block_kernel    256-thread workgroups that take token rows in turn, a row held in registers between the three
 //                             passes (sum of squares, absmax, quantise): 4*K bytes read once, K + 8 bytes written.
-//                             The usual shape (k <= 7168 with aligned rows), for one row or thousands.
-//   act_quant_block16_kernel  one 1024-thread workgroup per token row: up to 16 rows (a decode batch), where the
-//                             launch is as long as one row takes.
-//   act_quant_wave_kernel     one wavefront per token row: many rows of any length or alignment.
+//                             The usual shape, for one row or thousands.
+//   act_quant_row_kernel      a workgroup of up to 16 wavefronts per token row, one chunk of 4 (two above 4096 columns) per
+//                             thread: as many rows as run at once (a decode batch), where the launch is as long as one
+//                             row takes.
+//   act_quant_wave_kernel     one wavefront per token row: many rows of at most 1024 columns.
 #include "kernels.hpp"
 #include "rowquant.hpp"
 
@@ -22,6 +23,7 @@ struct ActQuantParams {
     int32_t *a_sum;
     float *y;
     size_t m;
+    size_t ldq;      // row stride of q: k, or more with the bytes from k on (up to the next multiple of 256) cleared
     int seq_in_lds;  // the launch carries LDS for the row's squares (literal summation order: sum_sequential_lds)
     unsigned *zero;  // optional: zero[0 .. zero_n) is cleared by the first workgroup (counters of the launch that follows)
     int zero_n;
@@ -36,96 +38,96 @@ __device__ __forceinline__ void clear_counters(const ActQuantParams &p)
     }
 }
 
-// NCH > 0: a lane keeps its NCH chunks in registers (K <= 256*NCH).  NCH == 0: any K, the row is
-// re-read (from cache) in each pass.
-template <int MODE, int NCH, bool VEC>
+constexpr size_t ROW_QUANT_MAX_ROWS = 512;
+
+// Where the int8 row goes.
+struct RowPlace {
+    size_t base;
+    __device__ __forceinline__ size_t chunk(int c) const { return base + 4 * (size_t)c; }
+};
+__device__ __forceinline__ RowPlace row_place(size_t row, size_t ldq) { return {row * ldq}; }
+
+// One quantised chunk (elements 4c .. 4c + 3 of the row; those from k on are +0 in `e`) to the int8 row, and to y if asked for.
+template <bool VEC>
+__device__ __forceinline__ void store_chunk(const ActQuantParams &p, const RowPlace &place, size_t row, int c, const float4 &e, float scale, int *isum)
+{
+    const int k = p.src.k;
+    const size_t at = place.chunk(c), base = row * (size_t)k + 4 * (size_t)c;
+    if (VEC || p.ldq > (size_t)k) {  // rows start on a dword and have room for a whole last one
+        *reinterpret_cast<uint32_t *>(p.q + at) = quant4_packed(e, scale, isum);
+        if constexpr (VEC) {
+            if (p.y) *reinterpret_cast<float4 *>(p.y + base) = e;
+            return;
+        }
+        if (!p.y) return;
+        const float es[4] = {e.x, e.y, e.z, e.w};
+        for (int j = 0; j < 4; ++j)
+            if (4 * c + j < k) p.y[base + j] = es[j];
+        return;
+    }
+    const float es[4] = {e.x, e.y, e.z, e.w};
+    for (int j = 0; j < 4; ++j) {
+        if (4 * c + j < k) {
+            const int qv = quant1(es[j], scale);
+            p.q[at + j] = (int8_t)qv;
+            if (p.y) p.y[base + j] = es[j];
+            *isum += qv;
+        }
+    }
+}
+// Chunk c lies past the row: cleared where the rows are padded.
+__device__ __forceinline__ void clear_pad(const ActQuantParams &p, const RowPlace &place, int c)
+{
+    if (4 * (size_t)c < p.ldq) *reinterpret_cast<uint32_t *>(p.q + place.chunk(c)) = 0u;
+}
+
+// One wavefront per row of at most 1024 columns: four chunks a lane, no barriers.  (A workgroup per row leaves most of its
+// threads without a chunk there.)
+template <int MODE, bool VEC>
 __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 {
+    constexpr int NCH = 4;
     const RowSource &src = p.src;
     const int lane = threadIdx.x;
     clear_counters(p);
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (row >= p.m) return;  // uniform per wavefront: a wavefront is one row
-    const int k = src.k;
-    const int chunks = (k + 3) >> 2;
-    const int nloop = NCH > 0 ? NCH : (chunks + 63) >> 6;
-    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int chunks = (src.k + 3) >> 2;
 
-    float4 v[NCH > 0 ? NCH : 1];
-    if constexpr (NCH > 0) {
+    float4 v[NCH];
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            int c = lane + 64 * i;
-            v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : zero4;
-        }
+    for (int i = 0; i < NCH; ++i) {
+        int c = lane + 64 * i;
+        v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    auto chunk_at = [&](int i, int c) -> float4 {
-        if constexpr (NCH > 0) return v[i];
-        else return c < chunks ? load_chunk<MODE, VEC>(src, row, c) : zero4;
-    };
-
-    RowDivisor rdiv = {1.0f, 1.0f, false};
-    const bool norm = src.gamma != nullptr;
-    if (norm) {
+    if (src.gamma) {
         float ss;
         if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
             ss = sum_squares_sequential<MODE>(src, row);
         } else {
-            // chunk c = lane + 64*i is virtual lane c mod 256 = lane + 64*(i mod 4): four partials per lane
-            float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (NCH > 0) {
+            // chunk lane + 64*i belongs to virtual lane lane + 64*i: four partials per lane
+            float part[NCH];
 #pragma unroll
-                for (int i = 0; i < NCH; ++i) part[i & 3] = sum_squares4(part[i & 3], v[i]);
-            } else {
-                for (int i = 0; i < nloop; i += 4)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) part[g] = sum_squares4(part[g], chunk_at(i + g, lane + 64 * (i + g)));
-            }
-            ss = f32_add(f32_add(f32_add(wave_sum_f32(part[0]), wave_sum_f32(part[1])), wave_sum_f32(part[2])),
-                         wave_sum_f32(part[3]));
+            for (int i = 0; i < NCH; ++i) part[i] = wave_sum_f32(sum_squares4(0.0f, v[i]));
+            ss = f32_add(f32_add(f32_add(part[0], part[1]), part[2]), part[3]);
         }
-        rdiv = make_row_divisor(rms_from_ss(ss, k, src.eps));
+        const Divisor rdiv = make_divisor(rms_from_ss(ss, src.k, src.eps));
+#pragma unroll
+        for (int i = 0; i < NCH; ++i)
+            if (lane + 64 * i < chunks) v[i] = normalize4(v[i], rdiv, load_gamma_chunk(src, lane + 64 * i, VEC));
     }
-
     float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < nloop; ++i) {
-        int c = lane + 64 * i;
-        float4 e = chunk_at(i, c);
-        if (norm && c < chunks) e = normalize4(e, rdiv, load_gamma_chunk(src, c, VEC));
-        if constexpr (NCH > 0) v[i] = e;
-        amax = absmax4(amax, e);
-    }
-    amax = wave_max_f32(amax);
-    const float scale = scale_from_absmax(amax);
+    for (int i = 0; i < NCH; ++i) amax = absmax4(amax, v[i]);
+    const float scale = scale_from_absmax(wave_max_f32(amax));
 
     int isum = 0;
+    const RowPlace place = row_place(row, p.ldq);
 #pragma unroll
-    for (int i = 0; i < nloop; ++i) {
-        int c = lane + 64 * i;
-        if (c >= chunks) continue;
-        float4 e;
-        if constexpr (NCH > 0) {
-            e = v[i];
-        } else {
-            e = load_chunk<MODE, VEC>(src, row, c);
-            if (norm) e = normalize4(e, rdiv, load_gamma_chunk(src, c, VEC));
-        }
-        size_t base = row * (size_t)k + 4 * (size_t)c;
-        if constexpr (VEC) {
-            *reinterpret_cast<uint32_t *>(p.q + base) = quant4_packed(e, scale, &isum);
-            if (p.y) *reinterpret_cast<float4 *>(p.y + base) = e;
-        } else {
-            float es[4] = {e.x, e.y, e.z, e.w};
-            for (int j = 0; j < 4; ++j) {
-                if (4 * c + j < k) {
-                    int qv = quant1(es[j], scale);
-                    p.q[base + j] = (int8_t)qv;
-                    if (p.y) p.y[base + j] = es[j];
-                    isum += qv;
-                }
-            }
-        }
+    for (int i = 0; i < NCH; ++i) {
+        const int c = lane + 64 * i;
+        if (c < chunks) store_chunk<VEC>(p, place, row, c, v[i], scale, &isum);
+        else clear_pad(p, place, c);
     }
     isum = wave_sum_i32(isum);
     if (lane == 0) {
@@ -134,7 +136,9 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
     }
 }
 
-// One workgroup per row.  NCH chunks per thread in registers (K <= 1024*NCH), NCH == 0: re-read.
+// A workgroup per row; NCH chunks per thread in registers (K <= 1024*NCH), NCH == 0: re-read.  A row is three dependent steps
+// with barriers between them: the loads of one workgroup overlap the arithmetic of the others on the compute unit.  (1024
+// workgroups that take rows in turn and fetch the next one early are slower: 15.8 us against 12.7 us at 2048 x 6912.)
 template <int MODE, int NCH, bool VEC>
 __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
 {
@@ -143,11 +147,12 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
     const RowSource &src = p.src;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     clear_counters(p);
-    const size_t row = blockIdx.x;
     const int k = src.k;
     const int chunks = (k + 3) >> 2;
     const int nloop = NCH > 0 ? NCH : (chunks + 255) >> 8;
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool norm = src.gamma != nullptr;
+    const size_t row = blockIdx.x;
 
     float4 v[NCH > 0 ? NCH : 1];
     if constexpr (NCH > 0) {
@@ -162,8 +167,7 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
         else return c < chunks ? load_chunk<MODE, VEC>(src, row, c) : zero4;
     };
 
-    RowDivisor rdiv = {1.0f, 1.0f, false};
-    const bool norm = src.gamma != nullptr;
+    Divisor rdiv = {1.0f, 1.0f, false};
     if (norm) {
         float ss;
         if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
@@ -174,7 +178,7 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
                     const int c = tid + 256 * i;
                     if (c < chunks) store_squares4(sq_lds, c, chunk_at(i, c));
                 }
-                __syncthreads();
+                lds_barrier();
                 ss = sum_sequential_lds(sq_lds, k);
             } else {
                 ss = sum_squares_sequential<MODE>(src, row);
@@ -185,10 +189,10 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
             for (int i = 0; i < nloop; ++i) part = sum_squares4(part, chunk_at(i, tid + 256 * i));
             part = wave_sum_f32(part);
             if (lane == 0) red_f[0][wave] = part;
-            __syncthreads();
+            lds_barrier();
             ss = f32_add(f32_add(f32_add(red_f[0][0], red_f[0][1]), red_f[0][2]), red_f[0][3]);
         }
-        rdiv = make_row_divisor(rms_from_ss(ss, k, src.eps));
+        rdiv = make_divisor(rms_from_ss(ss, k, src.eps));
     }
 
     float amax = 0.0f;
@@ -202,15 +206,19 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
     }
     amax = wave_max_f32(amax);
     if (lane == 0) red_f[1][wave] = amax;
-    __syncthreads();
+    lds_barrier();
     amax = fmaxf(fmaxf(red_f[1][0], red_f[1][1]), fmaxf(red_f[1][2], red_f[1][3]));
     const float scale = scale_from_absmax(amax);
 
     int isum = 0;
+    const RowPlace place = row_place(row, p.ldq);
 #pragma unroll
     for (int i = 0; i < nloop; ++i) {
         int c = tid + 256 * i;
-        if (c >= chunks) continue;
+        if (c >= chunks) {
+            clear_pad(p, place, c);
+            continue;
+        }
         float4 e;
         if constexpr (NCH > 0) {
             e = v[i];
@@ -218,146 +226,90 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
             e = load_chunk<MODE, VEC>(src, row, c);
             if (norm) e = normalize4(e, rdiv, load_gamma_chunk(src, c, VEC));
         }
-        size_t base = row * (size_t)k + 4 * (size_t)c;
-        if constexpr (VEC) {
-            *reinterpret_cast<uint32_t *>(p.q + base) = quant4_packed(e, scale, &isum);
-            if (p.y) *reinterpret_cast<float4 *>(p.y + base) = e;
-        } else {
-            float es[4] = {e.x, e.y, e.z, e.w};
-            for (int j = 0; j < 4; ++j) {
-                if (4 * c + j < k) {
-                    int qv = quant1(es[j], scale);
-                    p.q[base + j] = (int8_t)qv;
-                    if (p.y) p.y[base + j] = es[j];
-                    isum += qv;
-                }
-            }
-        }
+        store_chunk<VEC>(p, place, row, c, e, scale, &isum);
     }
     isum = wave_sum_i32(isum);
     if (lane == 0) red_i[wave] = isum;
-    __syncthreads();
+    lds_barrier();
     if (tid == 0) {
         p.a_scale[row] = scale;
         if (p.a_sum) p.a_sum[row] = red_i[0] + red_i[1] + red_i[2] + red_i[3];
     }
 }
 
-// One workgroup of 16 wavefronts per row, for the few rows of a decode batch: a row is then one workgroup's whole
-// work, so its time is the row's arithmetic divided by the threads that share it.  Thread t owns chunks t, t + 1024
-// (NCHB of them; k <= 4096 * NCHB, 16-byte aligned rows).  The sum of squares keeps the declared order: chunk c belongs
-// to virtual lane c % 256, so threads 0..255 also fetch the chunks of their lane and run its chain, then the four 64-lane
-// butterflies.  Same bits as the other two kernels.
-template <int MODE, int NCHB>
-__global__ __launch_bounds__(1024) void act_quant_block16_kernel(const float *hot_x, int hot_ldx, int hot_k, const float *hot_x2,
-                                                                const float *hot_gamma, int hot_head_dim, int hot_gqa_group,
-                                                                ActQuantParams p)
+// A workgroup of up to 16 wavefronts per row (Row16, rowquant.hpp), for the rows of a decode batch: the launch is as long as one
+// row takes, which is a chain of dependent steps.  What the first loads need arrives preloaded; the other arguments are one
+// scalar load while the row is on its way.  k % 4 == 0 up to 8192, 16-byte aligned rows, the declared summation order.
+struct RowQuantArgs {
+    int8_t *q;
+    float *a_scale;
+    int32_t *a_sum;
+    float *y;
+    unsigned *zero;
+    int zero_n;
+    int ldq;
+    int unused[4];
+};
+static_assert(sizeof(RowQuantArgs) == 64, "one scalar load");
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int ROW_QUANT_ARGS_AT = 48;  // its offset in the argument buffer: three pointers and six 4-byte arguments before it
+
+template <int MODE, bool NORM, int NCHB>
+__global__ __launch_bounds__(1024) void act_quant_row_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_chunks,
+                                                            int hot_nw, int hot_ldx, float hot_eps, int hot_m, [[maybe_unused]] RowQuantArgs args)
 {
     __shared__ float red_f[2][16];
-    __shared__ int red_i[16];
-    // the leading scalar arguments repeat what the first loads need; they are preloaded into registers (see the Makefile)
-    RowSource src = p.src;
-    src.x = hot_x; src.ldx = (size_t)hot_ldx; src.k = hot_k; src.x2 = hot_x2; src.gamma = hot_gamma;
-    src.head_dim = hot_head_dim; src.gqa_group = hot_gqa_group;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ int sum_s;
     const size_t row = blockIdx.x;
-    const int k = src.k, chunks = k >> 2;
-    const bool norm = src.gamma != nullptr;
-    constexpr int NSS = 4 * NCHB;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = hot_nw, chunks = hot_k >> 2;
+    const float *x = hot_x + row * (size_t)hot_ldx;
+    const float *x2 = MODE == BITNET_HIP_INPUT_RELU2_MUL ? hot_x2 + row * (size_t)hot_ldx : nullptr;
+    const uint64_t magics = MODE == BITNET_HIP_INPUT_GQA_BROADCAST ? reinterpret_cast<uintptr_t>(hot_x2) : 0;
+    Row16<NORM, NCHB> row16;
+    row16.template load<MODE>(x, x2, magics, hot_head_chunks, hot_gamma, chunks, nw, wave, tid, tid & 63);
+    __builtin_amdgcn_sched_barrier(0);
+    typedef const __attribute__((address_space(4))) v16u *arg_ptr;
+    v16u block = *(arg_ptr)((uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + ROW_QUANT_ARGS_AT);
+    if (tid < 16 && tid >= nw) red_f[1][tid] = 0.0f;
+    if (tid == 0) sum_s = 0;
+    float k_f = (float)hot_k, k_recip = recip_of_ok_divisor(k_f);
+    asm volatile("" : "+s"(block), "+v"(k_recip));
+    const global_ptr<int8_t> q = pointer_at<int8_t>(block, 0);
+    const global_ptr<float> a_scale = pointer_at<float>(block, 2), y = pointer_at<float>(block, 6);
+    const global_ptr<int32_t> a_sum = pointer_at<int32_t>(block, 4);
+    const global_ptr<unsigned> zero = pointer_at<unsigned>(block, 8);
+    const int zero_n = (int)block[10], ldq = (int)block[11];
+    const RowPlace place = row_place(row, (size_t)ldq);
 
-    // all loads up front, unconditional (clamped indices, values discarded), addressed by the preloaded arguments alone:
-    // the argument buffer is read only once they are on their way (wavefronts 0..3 fetch their lanes' chunks whatever
-    // the summation order turns out to be)
-    float4 v[NCHB], gm[NCHB], vs[NSS];
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i) v[i] = load_chunk<MODE, true>(src, row, min(tid + 1024 * i, chunks - 1));
-    if (norm && wave < 4) {
-#pragma unroll
-        for (int i = 0; i < NSS; ++i) vs[i] = load_chunk<MODE, true>(src, row, min(tid + 256 * i, chunks - 1));
-    }
-    if (norm) {
-#pragma unroll
-        for (int i = 0; i < NCHB; ++i) gm[i] = load_gamma_chunk(src, min(tid + 1024 * i, chunks - 1), true);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // nothing below moves above: the first wait for the argument buffer comes here
-    clear_counters(p);
-    const bool chain = norm && src.sum_order != BITNET_HIP_SUM_SEQUENTIAL && wave < 4;
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i)
-        if (tid + 1024 * i >= chunks) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-
-    if (norm) {
-        float ss;
-        if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
-            if (p.seq_in_lds) {
-                extern __shared__ float sq_lds[];  // squares_lds_bytes(k)
-#pragma unroll
-                for (int i = 0; i < NCHB; ++i)
-                    if (tid + 1024 * i < chunks) store_squares4(sq_lds, tid + 1024 * i, v[i]);
-                lds_barrier();
-                ss = sum_sequential_lds(sq_lds, k);
-            } else {
-                ss = sum_squares_sequential<MODE>(src, row);
-            }
-        } else {
-            if (chain) {  // thread tid < 256 is virtual lane tid
-                float part = 0.0f;
-#pragma unroll
-                for (int i = 0; i < NSS; ++i)
-                    if (tid + 256 * i < chunks) part = sum_squares4(part, vs[i]);  // chunks past the end would add +0
-                part = wave_sum_f32(part);
-                if (lane == 0) red_f[0][wave] = part;
-            }
-            lds_barrier();
-            ss = f32_add(f32_add(f32_add(red_f[0][0], red_f[0][1]), red_f[0][2]), red_f[0][3]);
-        }
-        const RowDivisor rdiv = make_row_divisor(rms_from_ss(ss, k, src.eps));
-#pragma unroll
-        for (int i = 0; i < NCHB; ++i)
-            if (tid + 1024 * i < chunks) v[i] = normalize4(v[i], rdiv, gm[i]);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i) amax = absmax4(amax, v[i]);
-    amax = wave_max_f32(amax);
-    if (lane == 0) red_f[1][wave] = amax;
-    lds_barrier();
-    amax = red_f[1][0];
-#pragma unroll
-    for (int w = 1; w < 16; ++w) amax = fmaxf(amax, red_f[1][w]);
-    const float scale = scale_from_absmax(amax);
-
-    int isum = 0;
+    uint32_t packed[NCHB];
+    const float scale = row16.quantise(chunks, k_f, k_recip, hot_eps, wave, tid, red_f, packed);
+    int sum = 0;
 #pragma unroll
     for (int i = 0; i < NCHB; ++i) {
-        const int c = tid + 1024 * i;
-        if (c < chunks) {
-            const size_t base = row * (size_t)k + 4 * (size_t)c;
-            *reinterpret_cast<uint32_t *>(p.q + base) = quant4_packed(v[i], scale, &isum);
-            if (p.y) *reinterpret_cast<float4 *>(p.y + base) = v[i];
-        }
+        const int c = row16.chunk[i];
+        if (4 * c < ldq) *(global_ptr<uint32_t>)(q + place.chunk(c)) = packed[i];  // chunks past the row hold zeros
+        if (y && c < chunks) *(global_ptr<v4f>)(y + (row * (size_t)hot_k + 4 * (size_t)c)) = (v4f){row16.v[i].x, row16.v[i].y, row16.v[i].z, row16.v[i].w};
+        sum = __builtin_amdgcn_sdot4((int)packed[i], 0x01010101, sum, false);
     }
-    isum = wave_sum_i32(isum);
-    if (lane == 0) red_i[wave] = isum;
-    lds_barrier();
-    if (tid == 0) {
-        p.a_scale[row] = scale;
-        if (p.a_sum) {
-            int total = 0;
-#pragma unroll
-            for (int w = 0; w < 16; ++w) total += red_i[w];
-            p.a_sum[row] = total;
-        }
+    if (tid == 0) a_scale[row] = scale;
+    if (zero && row == 0)
+        for (int i = tid; i < zero_n; i += 64 * nw) zero[i] = 0u;
+    if (a_sum) {
+        sum = wave_sum_i32(sum);
+        if ((tid & 63) == 0) atomicAdd(&sum_s, sum);
+        lds_barrier();
+        if (tid == 0) a_sum[row] = sum_s;
     }
 }
 
-template <int MODE, int NCH, bool VEC>
+template <int MODE, bool VEC>
 void launch_wave(const ActQuantParams &p, hipStream_t s)
 {
     const int rows_per_block = 4;
     dim3 block(64, rows_per_block);
     dim3 grid((unsigned)((p.m + rows_per_block - 1) / rows_per_block));
-    hipLaunchKernelGGL((act_quant_wave_kernel<MODE, NCH, VEC>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((act_quant_wave_kernel<MODE, VEC>), grid, block, 0, s, p);
 }
 
 // LDS for the row's squares where the literal summation order is asked for and a row fits the default limit
@@ -380,36 +332,45 @@ template <int MODE>
 void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
 {
     const int chunks = (p.src.k + 3) >> 2;
-    // Few rows (a decode batch): 16 wavefronts per row.
-    if (p.m <= 16 && vec && chunks <= 2048 && p.src.ldx < (1u << 31)) {
-#define BITNET_HOT_ARGS p.src.x, (int)p.src.ldx, p.src.k, p.src.x2, p.src.gamma, p.src.head_dim, p.src.gqa_group
-        ActQuantParams q = p;
-        const size_t lds = launch_squares_lds(p);
-        q.seq_in_lds = lds != 0;
-        if (chunks <= 1024) hipLaunchKernelGGL((act_quant_block16_kernel<MODE, 1>), dim3((unsigned)p.m), dim3(1024), lds, s, BITNET_HOT_ARGS, q);
-        else hipLaunchKernelGGL((act_quant_block16_kernel<MODE, 2>), dim3((unsigned)p.m), dim3(1024), lds, s, BITNET_HOT_ARGS, q);
+    // Rows that all run at once: up to 16 wavefronts per row.
+    const bool ordered = !p.src.gamma || p.src.sum_order == BITNET_HIP_SUM_BLOCK256;
+    if ((p.m <= ROW_QUANT_MAX_ROWS || chunks > 1792) && vec && ordered && chunks <= 2048 && p.src.ldx < (1u << 31)) {
+        const float *x2 = p.src.x2;
+        uint64_t magics = 0;
+        bool in_range = true;
+        if (MODE == BITNET_HIP_INPUT_GQA_BROADCAST) {
+            in_range = row16_magics(p.src.head_dim, p.src.gqa_group, &magics);
+            x2 = reinterpret_cast<const float *>(static_cast<uintptr_t>(magics));
+        }
+        if (in_range) {
+            const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, p.zero, p.zero_n, (int)p.ldq, {0, 0, 0, 0}};
+            const int kt = (p.src.k + 255) >> 8, nchb = kt > 16 ? 2 : 1;
+            const int nw = nchb == 2 ? (kt + 1) / 2 : row_workgroup_waves(p.src.k);
+            const dim3 grid((unsigned)p.m), block(64u * (unsigned)nw);
+#define BITNET_HOT_ARGS p.src.x, x2, p.src.gamma, p.src.k, p.src.head_dim / 4, nw, (int)p.src.ldx, p.src.eps, (int)p.m, args
+            if (p.src.gamma) {
+                if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+            } else {
+                if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+            }
 #undef BITNET_HOT_ARGS
-        return;
+            return;
+        }
     }
-    // A workgroup per row for few rows, and for any number of rows whose chunks fit the threads' registers: with
-    // more, shorter-lived workgroups in flight the load latency of one overlaps the arithmetic of others (measured
-    // at 2048 rows: 8.0 us against 9.0 us at k = 2560, 16.9 us against 23.1 us at k = 6912).
-    if (p.m <= 32 || (vec && ((chunks + 255) >> 8) <= 7)) {
-        if (!vec) return launch_block<MODE, 0, false>(p, s);
-        const int per_thread = (chunks + 255) >> 8;
+    if (p.m > 32 && chunks <= 256) return vec ? launch_wave<MODE, true>(p, s) : launch_wave<MODE, false>(p, s);
+    const int per_thread = (chunks + 255) >> 8;
+    if (vec) {
         if (per_thread <= 3) return launch_block<MODE, 3, true>(p, s);
         if (per_thread <= 7) return launch_block<MODE, 7, true>(p, s);
         if (per_thread <= 16) return launch_block<MODE, 16, true>(p, s);
         return launch_block<MODE, 0, true>(p, s);
     }
-    if (!vec) return launch_wave<MODE, 0, false>(p, s);
-    const int per_lane = (chunks + 63) >> 6;
-    if (per_lane <= 4) return launch_wave<MODE, 4, true>(p, s);
-    if (per_lane <= 10) return launch_wave<MODE, 10, true>(p, s);
-    if (per_lane <= 16) return launch_wave<MODE, 16, true>(p, s);
-    if (per_lane <= 27) return launch_wave<MODE, 27, true>(p, s);
-    if (per_lane <= 32) return launch_wave<MODE, 32, true>(p, s);
-    return launch_wave<MODE, 0, true>(p, s);
+    if (per_thread <= 3) return launch_block<MODE, 3, false>(p, s);
+    if (per_thread <= 7) return launch_block<MODE, 7, false>(p, s);
+    if (per_thread <= 16) return launch_block<MODE, 16, false>(p, s);
+    return launch_block<MODE, 0, false>(p, s);
 }
 
 inline bool aligned(const void *ptr, size_t a) { return (reinterpret_cast<uintptr_t>(ptr) % a) == 0; }
@@ -645,15 +606,18 @@ int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratc
 
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
-                     int8_t *q, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero, size_t zero_n)
+                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero, size_t zero_n)
 {
     ActQuantParams p;
+    p.ldq = ldq;
     p.zero = zero; p.zero_n = (int)zero_n;
     p.src.x = x; p.src.x2 = x2; p.src.gamma = gamma; p.src.ldx = ldx; p.src.k = (int)k;
     p.src.head_dim = (int)(head_dim ? head_dim : 1); p.src.gqa_group = (int)(gqa_group ? gqa_group : 1);
     p.src.sum_order = sum_order; p.src.eps = eps;
     p.q = q; p.a_scale = a_scale; p.a_sum = a_sum; p.y = y; p.m = m; p.seq_in_lds = 0;
 
+    if (ldq != k && (ldq % 4 != 0 || !aligned(q, 4) || ldq < k || ldq > (k + 255) / 256 * 256))
+        return fail(BITNET_HIP_INVALID_CONFIG, "activation quantiser: int8 row stride %zu for %zu columns", ldq, k);
     bool vec = (k % 4 == 0) && (ldx % 4 == 0) && aligned(x, 16) && aligned(q, 4) && (!x2 || aligned(x2, 16)) &&
                (!y || aligned(y, 16)) && (!gamma || aligned(gamma, 16));
     if (input_mode == BITNET_HIP_INPUT_GQA_BROADCAST) vec = vec && (head_dim % 4 == 0);

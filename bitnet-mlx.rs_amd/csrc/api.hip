@@ -153,14 +153,15 @@ size_t launch_group_blocks(bitnet_hip_bitlinear *const *layers, size_t count)
 // Runs `count` projections that share one input row block [m, k].  At decode token counts the quantiser runs
 // inside the GEMV launch (up to GEMV_MAX_PROJ projections per launch); otherwise the stand-alone quantiser
 // fills q / a_scale / a_sum (scratch the caller provides) and the GEMV or GEMM kernels consume them.
-// residual / out / acc are per-projection arrays (entries of residual and acc may be null, and so may the arrays).
+// residual / out / acc are per-projection arrays (entries of residual and acc may be null, and so may the arrays).  ldq: row
+// stride of q, in_features or padded_k(in_features).
 int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float *x, const float *x2, size_t ldx,
                     size_t m, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,
                     int sum_order, const float *const *residual, float *const *out, int32_t *const *acc, int8_t *q,
-                    float *a_scale, int32_t *a_sum, bool want_quant_outputs, hipStream_t s,
+                    size_t ldq, float *a_scale, int32_t *a_sum, bool want_quant_outputs, hipStream_t s,
                     const GemmSplitScratch *split = nullptr)
 {
-    const size_t k = layers[0]->in_features;
+    size_t k = layers[0]->in_features;
     auto proj_of = [&](int j) {
         bitnet_hip_bitlinear *bl = layers[j];
         GemvProj pj = {bl->tiled, bl->w_scale, bl->use_bias ? bl->bias : nullptr, residual ? residual[j] : nullptr,
@@ -184,10 +185,11 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
     for (int j = 0; j < count; ++j) n_blocks += row_blocks(layers[j]->out_features);
     // A GEMM that splits k across workgroups finds its tile counters zeroed by the quantiser launched in front of it.  One
     // scratch serves one launch: more projections than one launch takes run without the split.
-    const bool use_split = split && split->counters && count <= GEMM_MAX_PROJ && !gemv_takes(m, k, n_blocks, q);
-    int rc = launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, a_scale, a_sum,
+    const bool use_split = split && split->counters && count <= GEMM_MAX_PROJ && !gemv_takes(m, ldq, n_blocks, q);
+    int rc = launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, ldq, a_scale, a_sum,
                               nullptr, s, use_split ? split->counters : nullptr, use_split ? split->counter_count : 0);
     if (rc != BITNET_HIP_OK) return rc;
+    k = ldq;  // the columns past in_features are zero in the rows and in the tiles
     if (gemv_takes(m, k, n_blocks, q)) {
         for (int j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
             GemvProj pjs[GEMV_MAX_PROJ];
@@ -217,7 +219,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
     return BITNET_HIP_OK;
 }
 
-// Scratch for the quantised activations of m rows of width k: q [m*k] int8, a_scale [m] f32, a_sum [m] int32.
+// Scratch for the quantised activations of m rows of width (or row stride) k: q [m*k] int8, a_scale [m] f32, a_sum [m] int32.
 struct QuantScratch {
     int8_t *q;
     float *a_scale;
@@ -363,7 +365,7 @@ int bitnet_hip_quantize_activations_i8(const float *x, const float *x2, size_t l
         size_t e[2] = {m, src_cols}, a[2] = {m, ldx};
         return fail_shape(e, 2, a, 2, "row stride smaller than the row");
     }
-    return launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, a_scale,
+    return launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, k, a_scale,
                             a_sum, y_f32, as_stream(stream));
 }
 
@@ -799,7 +801,8 @@ size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, si
 {
     if (!layer) return 0;
     // the quantised activations, and the partial tiles of a GEMM that splits k across workgroups where one would run
-    return quant_scratch_bytes(m, layer->in_features) + split_scratch_bytes(m, layer->in_features, layer->out_features);
+    const size_t kp = padded_k(layer->in_features);
+    return quant_scratch_bytes(m, kp) + split_scratch_bytes(m, kp, layer->out_features);
 }
 
 size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,
@@ -819,7 +822,7 @@ size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *l
         if (!layers[j]) return 0;
     const size_t in = layers[0]->in_features;
     if (gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, launch_group_blocks(layers, count))) return 0;
-    return quant_scratch_bytes(m, in);
+    return quant_scratch_bytes(m, padded_k(in));
 }
 
 int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, const size_t *dims, int rank,
@@ -856,20 +859,23 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     bool own_ws = false;
     QuantScratch sc = {dbg_q, dbg_a_scale, nullptr};
     GemmSplitScratch split;
+    size_t ldq = in;
     if (!fused || debug) {  // the fused decode launch needs no scratch unless the caller wants q / a_scale back
-        const size_t need = quant_scratch_bytes(m, in), extra = split_scratch_bytes(m, in, layer->out_features);
+        const size_t least = quant_scratch_bytes(m, in);
+        if (!dbg_q && (!ws || workspace_bytes >= quant_scratch_bytes(m, padded_k(in)))) ldq = padded_k(in);
+        const size_t need = quant_scratch_bytes(m, ldq), extra = split_scratch_bytes(m, ldq, layer->out_features);
         bool with_split = extra != 0;
         if (!ws) {
             hipError_t e = hipMallocAsync(&ws, need + extra, s);
             if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward: hipMallocAsync(%zu) failed: %s", need + extra, hipGetErrorString(e));
             own_ws = true;
-        } else if (workspace_bytes < need) {
-            return fail(BITNET_HIP_MEMORY_ERROR, "forward: workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+        } else if (workspace_bytes < least) {
+            return fail(BITNET_HIP_MEMORY_ERROR, "forward: workspace of %zu bytes given, %zu needed", workspace_bytes, least);
         } else if (workspace_bytes < need + extra) {
             with_split = false;  // room for the quantised activations only: the GEMM walks k without the split
         }
-        sc = carve_scratch(ws, m, in);
-        if (with_split) split = carve_split(ws, m, in, layer->out_features);
+        sc = carve_scratch(ws, m, ldq);
+        if (with_split) split = carve_split(ws, m, ldq, layer->out_features);
         if (dbg_q) sc.q = dbg_q;
         if (dbg_a_scale) sc.a_scale = dbg_a_scale;
     }
@@ -878,7 +884,7 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     float *outs[1] = {out};
     int32_t *accs[1] = {dbg_acc};
     int rc = run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                             accs, sc.q, sc.a_scale, sc.a_sum, debug, s, split.partials ? &split : nullptr);
+                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, split.partials ? &split : nullptr);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -925,12 +931,13 @@ int bitnet_hip_bitlinear_forward_noalloc(bitnet_hip_bitlinear *layer, const floa
 
     std::shared_lock<std::shared_mutex> guard(layer->lock);
     if (!layer->has_weights) return fail(BITNET_HIP_NOT_INITIALIZED, "forward_noalloc: the layer has no weights yet");
-    const QuantScratch sc = carve_scratch(ws, m, in);
+    const size_t ldq = quant_scratch_bytes(m, padded_k(in)) <= NOALLOC_SCRATCH_BYTES ? padded_k(in) : in;
+    const QuantScratch sc = carve_scratch(ws, m, ldq);
     bitnet_hip_bitlinear *layers[1] = {layer};
     const float *res[1] = {residual};
     float *outs[1] = {out};
     return run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                           nullptr, sc.q, sc.a_scale, sc.a_sum, false, as_stream(stream));
+                           nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, as_stream(stream));
 }
 
 int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
@@ -957,8 +964,10 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {nullptr, nullptr, nullptr};
+    size_t ldq = in;
     if (!fused) {
-        const size_t need = quant_scratch_bytes(m, in);
+        if (!ws || workspace_bytes >= quant_scratch_bytes(m, padded_k(in))) ldq = padded_k(in);
+        const size_t need = quant_scratch_bytes(m, ldq);
         if (!ws) {
             hipError_t e = hipMallocAsync(&ws, need, s);
             if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward_multi: hipMallocAsync(%zu) failed: %s", need, hipGetErrorString(e));
@@ -966,10 +975,10 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
         } else if (workspace_bytes < need) {
             return fail(BITNET_HIP_MEMORY_ERROR, "forward_multi: workspace of %zu bytes given, %zu needed", workspace_bytes, need);
         }
-        sc = carve_scratch(ws, m, in);
+        sc = carve_scratch(ws, m, ldq);
     }
     int rc = run_projections(layers, (int)count, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order,
-                             nullptr, outs, nullptr, sc.q, sc.a_scale, sc.a_sum, false, s);
+                             nullptr, outs, nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, s);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -1066,7 +1075,7 @@ int bitnet_hip_decoder_create(size_t layers, size_t hidden, size_t ffn, size_t q
             rc = bitnet_hip_bitlinear_create(ins[p], outs[p], 0, &bl);
             if (rc == BITNET_HIP_OK) d->proj.push_back(bl);
         }
-    const size_t widest = hidden > ffn ? hidden : ffn;
+    const size_t widest = padded_k(hidden > ffn ? hidden : ffn);
     auto dev_alloc = [&](auto **ptr, size_t bytes) {
         if (rc != BITNET_HIP_OK) return;
         hipError_t e = hipMalloc(reinterpret_cast<void **>(ptr), bytes);
@@ -1189,7 +1198,7 @@ int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin
         BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));  // the previous decode used these buffers on another stream
     // One chain: rows [row0, row0 + rows) through blocks layer_begin .. layer_end-1 on stream cs, in its own rows of the
     // decoder's activation buffers.
-    const size_t widest = H > F ? H : F;
+    const size_t widest = padded_k(H > F ? H : F);
     auto run_chain = [&](size_t row0, size_t rows, hipStream_t cs) {
         // one launch group: `count` projections reading the same (transformed) input
         auto run = [&](bitnet_hip_bitlinear *const *layers, int count, const float *x, const float *x2, size_t ldx, int mode,
@@ -1197,7 +1206,8 @@ int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin
             if (rc != BITNET_HIP_OK) return;
             const float *res[GEMV_MAX_PROJ] = {res0, nullptr, nullptr};
             rc = run_projections(layers, count, x, x2, ldx, rows, mode, group, dec->head_dim, gamma, dec->eps, dec->sum_order,
-                                 res, outs, nullptr, dec->a8 + row0 * widest, dec->a_scale + row0, dec->a_sum + row0, false, cs);
+                                 res, outs, nullptr, dec->a8 + row0 * widest, padded_k(layers[0]->in_features), dec->a_scale + row0,
+                                 dec->a_sum + row0, false, cs);
         };
         float *qb = dec->qb + row0 * H, *kb = dec->kb + row0 * KV, *vb = dec->vb + row0 * KV, *x1 = dec->x1 + row0 * H;
         float *gate = dec->gate + row0 * F, *up = dec->up + row0 * F, *ping = dec->ping + row0 * H;
@@ -1383,7 +1393,7 @@ size_t decoder_device_bytes(const bitnet_hip_decoder *d)
         total += (p->in_features * p->out_features + 3) / 4 + tiled_bytes(p->out_features, p->in_features) + sizeof(float);
         if (p->use_bias) total += sizeof(float) * p->out_features;
     }
-    const size_t kv = d->kv_heads * d->head_dim, widest = d->hidden > d->ffn ? d->hidden : d->ffn, t = d->max_tokens;
+    const size_t kv = d->kv_heads * d->head_dim, widest = padded_k(d->hidden > d->ffn ? d->hidden : d->ffn), t = d->max_tokens;
     total += sizeof(float) * d->layers * 2 * d->hidden;                                        // norms
     total += t * widest + 2 * sizeof(float) * t;                                               // a8, a_scale, a_sum
     total += sizeof(float) * t * (d->hidden /*q*/ + 2 * kv + d->hidden /*x1*/ + 2 * d->ffn + d->hidden /*ping*/);

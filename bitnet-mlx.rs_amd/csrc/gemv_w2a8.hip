@@ -33,6 +33,8 @@
 // int8 activation matrix, which stays in L2; its B operand is a decoded weight dword, exactly as in the
 // prefill GEMM), so up to 16 tokens cost what one costs in weight traffic and instructions.  A workgroup
 // owns RB adjacent 16-row blocks so that the activation matrix is re-read by fewer workgroups.
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "rowquant.hpp"
 #include "tiledot.hpp"
@@ -44,7 +46,7 @@ namespace {
 
 constexpr int MODE_PREQUANT = -1;
 constexpr int GEMV_FUSED_MAX_ROWS = 8;   // tokens per fused quantiser + GEMV launch (a set of workgroups per token)
-constexpr int GEMV_FUSED_MAX_WGS = 512;  // and its workgroups over all tokens: one round on 256 compute units
+constexpr int GEMV_FUSED_MAX_WGS = 256;  // and its workgroups over all tokens: one per compute unit
 constexpr int FUSED_NCH = 7;  // 16-byte f32 chunks per thread kept in registers: K <= 7168
 
 struct GemvProjDev {
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(256) void gemv_tiled_kernel(GemvParams p)
                 if (t == 0) v[i] = v0[i];
                 else v[i] = c < chunks ? load_chunk<MODE, true>(src, (size_t)t, c) : make_float4(0.f, 0.f, 0.f, 0.f);
             }
-            RowDivisor rdiv = {1.0f, 1.0f, false};
+            Divisor rdiv = {1.0f, 1.0f, false};
             if (norm) {
                 float ss;
                 if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
@@ -183,7 +185,7 @@ __global__ __launch_bounds__(256) void gemv_tiled_kernel(GemvParams p)
                     __syncthreads();
                     ss = f32_add(f32_add(f32_add(red_f[t][0][0], red_f[t][0][1]), red_f[t][0][2]), red_f[t][0][3]);
                 }
-                rdiv = make_row_divisor(rms_from_ss(ss, p.k, src.eps));
+                rdiv = make_divisor(rms_from_ss(ss, p.k, src.eps));
             }
             float amax = 0.0f;
 #pragma unroll
@@ -337,7 +339,7 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvParams p)
         if (tid + 256 * i >= chunks) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 
     // thread tid is virtual lane tid of the declared summation order
-    RowDivisor rdiv = {1.0f, 1.0f, false};
+    Divisor rdiv = {1.0f, 1.0f, false};
     if constexpr (NORM) {
         float ss;
         if (p.src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvParams p)
             lds_barrier();
             ss = f32_add(f32_add(f32_add(red_f[0][0], red_f[0][1]), red_f[0][2]), red_f[0][3]);
         }
-        rdiv = make_row_divisor(rms_from_ss(ss, p.k, p.src.eps));
+        rdiv = make_divisor(rms_from_ss(ss, p.k, p.src.eps));
     }
     float amax = 0.0f;
 #pragma unroll
@@ -425,219 +427,215 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvParams p)
     }
 }
 
-// The same launch with up to 16 wavefronts per workgroup.  The prologue of gemv_fused_kernel is redundant arithmetic on
-// one wavefront per SIMD (normalise, absmax, quantise: about half of the dependent work of a launch); a thread per
-// chunk does the element-wise part four times faster.  A workgroup has nw wavefronts (bs = 64 nw threads), thread t
-// owns chunks t, t + bs (NCHB of them) and wavefront w the k-tiles w, w + nw; the sum of squares
-// keeps the declared order: chunk c belongs to virtual lane c % 256, whose chain runs over its chunks in ascending
-// order, so threads 0..255 (one per virtual lane) also fetch their lane's chunks (from L2, with the first loads of the
-// kernel) and add the squares up in that order, then the four 64-lane butterflies as before.
-// A 256-column k-tile is the 64 chunks one wavefront quantises, so every wavefront multiplies the tiles of its own
-// chunks (for each of the workgroup's RBW row blocks) straight after writing them to LDS, without a workgroup barrier
-// between quantiser and dot products; the partial sums of a row meet in LDS atomics.
+// The same launch with up to 16 wavefronts per workgroup: the default.  One wavefront per 256-column k-tile (nw wavefronts;
+// NCHB = 2: two tiles each, w and w + nw), a lane per 16-byte chunk of the tile: the element-wise steps run once, in
+// parallel, and what the launch takes is the chain of dependent steps.  At the decode shapes that chain, not memory, is
+// the bound: a launch whose workgroups only read the row and their cold weight tiles behind a barrier takes 2.2 us, and the
+// stack is as fast on weights that fit the last-level cache as on ones that do not.  So everything here is about the chain:
+//   * All arguments are in registers before the first barrier.  Scalar loads that the compiler places at their use (the
+//     width, eps, the output pointers) each cost a trip to L2 between two barriers.  What the first loads need arrives
+//     preloaded; the rest is fetched while the row is on its way, and pinned.
+//   * A lane's chunk is chosen so that the quantised row never goes through LDS.  Inside a tile, lane 16 kq + 4 t + u takes chunk
+//     16 t + 4 kq + u (columns 64 t + 16 kq + 4 u .. + 3), so that row broadcasts bring a lane the 16 columns 64 t + 16 kq .. + 15
+//     that dword t of its weight slot stands for: the A operand of MFMA t, all 16 rows of it the one row there is.  With four
+//     and more row blocks per workgroup taking the codes apart is what the matrix part waits for: MFMA u then takes the codes
+//     at bits 2u of all four dwords, for u < 3 in place (dword & (3 << 2u); the factor 4^u is shifted out between the
+//     MFMAs), 20 vector operations a tile instead of 28, and its A operand is the broadcasts of t = 0..3 for that u.
+//   * The row's sum for the code offset is an MFMA on a constant operand.
+//   * Wavefront reductions end in lane 63 by DPP row broadcasts, one instruction a step.
+// The sum of squares keeps the declared order: chunk c belongs to virtual lane c % 256, whose chain runs over its chunks in
+// ascending order, so threads 0..255 (one per virtual lane) also fetch their lane's chunks (from L2, with the first loads of
+// the kernel) and add the squares up in that order, then the four 64-lane butterflies as before.  The partial sums of a
+// row meet in LDS atomics (int32: any order gives the same sum).
+// A block of the 30-block stack (2560 / 6912), replayed, at one token: 16.5 us before these points, 14.8 with them; at four tokens
+// 23.9 and 22.3.
+
+// The arguments behind the preloaded ones, in blocks of 64 bytes: each is one scalar load.
+struct Fused16Proj {
+    const uint8_t *w;
+    const float *w_scale, *bias, *residual;
+    float *out;
+    int32_t *acc;
+    int n;
+    int rb_end;  // groups of RBW row blocks of projections 0..this one, cumulative
+    uint64_t unused;
+};
+struct Fused16Params {
+    int kt_count;
+    float eps;
+    uint64_t reserved;
+    int8_t *q_out;  // optional copies of what the prologue produced (written by the first group of row blocks)
+    float *a_scale_out;
+    int32_t *a_sum_out;
+    uint64_t unused[3];
+    Fused16Proj proj[GEMV_MAX_PROJ];
+};
+static_assert(sizeof(Fused16Proj) == 64 && sizeof(Fused16Params) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
+constexpr int FUSED16_ARGS_AT = 48;  // offset of the Fused16Params in the argument buffer: three pointers and six ints before it
+
+// The value of a lane of the own 16 lanes (a constant once unrolled): a row broadcast, 0x150 + lane.
+template <int LANE>
+__device__ __forceinline__ int row_lane_at(int v) { return dpp_i32<0x150 + LANE>(v); }
+__device__ __forceinline__ int row_lane(uint32_t packed, int at)
+{
+    const int v = (int)packed;
+    switch (at) {
+        case 0: return row_lane_at<0>(v); case 1: return row_lane_at<1>(v); case 2: return row_lane_at<2>(v); case 3: return row_lane_at<3>(v);
+        case 4: return row_lane_at<4>(v); case 5: return row_lane_at<5>(v); case 6: return row_lane_at<6>(v); case 7: return row_lane_at<7>(v);
+        case 8: return row_lane_at<8>(v); case 9: return row_lane_at<9>(v); case 10: return row_lane_at<10>(v); case 11: return row_lane_at<11>(v);
+        case 12: return row_lane_at<12>(v); case 13: return row_lane_at<13>(v); case 14: return row_lane_at<14>(v); default: return row_lane_at<15>(v);
+    }
+}
+typedef int v4i __attribute__((ext_vector_type(4)));
 
 template <int MODE, bool NORM, int NCHB, int RBW>
-__global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_dim,
-                                                           int hot_gqa_group, int hot_ldx, GemvParams p)
+__global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_chunks,
+                                                           int hot_nw, int hot_ldx, int hot_end0, int hot_end1, [[maybe_unused]] Fused16Params args)
 {
     // A launch has one to eight tokens (input rows), each with its own workgroups.  Workgroup (x, y) of the grid works on
     // token x / 8 and on group 8y + x % 8 of row blocks: the workgroups of one group are neighbours in dispatch order and,
     // workgroups going to the XCDs in turn, run on the same XCD, so its L2 fetches their weight tiles once.
-    // The leading scalar arguments repeat what the first loads need (input rows, RMSNorm weights, k): the file is
-    // compiled with kernel-argument preloading, so they arrive in registers with the wavefront instead of through a
-    // load from the argument buffer that the first address computation would have to wait for.
-    RowSource hot;
-    hot.x = hot_x; hot.x2 = hot_x2; hot.gamma = hot_gamma; hot.ldx = (size_t)hot_ldx; hot.k = hot_k; hot.head_dim = hot_head_dim;
-    hot.gqa_group = hot_gqa_group & 0xffff; hot.sum_order = BITNET_HIP_SUM_BLOCK256; hot.eps = 0.0f;
-    const size_t tok = blockIdx.x >> 3;
-    const int group = (int)blockIdx.y * 8 + (int)(blockIdx.x & 7);  // may lie past the last group: such workgroups leave below
-    extern __shared__ uint4 lds_a[];  // int8 activations, zero past K
+    // The leading scalar arguments are what the first loads need (input rows, RMSNorm weights, k): the file is compiled with
+    // kernel-argument preloading, so they arrive in registers with the wavefront.
     __shared__ float red_f[2][16];
-    __shared__ int red_i[16];
     __shared__ int tot[RBW][TILE_ROWS];
+    __shared__ int asum_s;
 
+    const size_t tok = blockIdx.x >> 3;
+    const int group = (int)blockIdx.y * 8 + (int)(blockIdx.x & 7);  // may lie past the last group: such workgroups store nothing
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int chunks = hot_k >> 2;
-    // A row of at most 1024 chunks is launched with one wavefront per k-tile (at least the four of the summation order)
-    // instead of 16: wavefronts without a chunk would only add their share of the redundant arithmetic between the
-    // barriers to the SIMDs' queues.  Their slots of the cross-wavefront reductions hold the neutral element.
-    const int nw = hot_gqa_group >> 16, bs = nw << 6;  // wavefronts and threads of the workgroup (preloaded with the GQA group)
-    if (tid < 16 && tid >= nw) {
-        red_f[1][tid] = 0.0f;
-        red_i[tid] = 0;
-    }
+    const int nw = hot_nw, chunks = hot_k >> 2;
+    const float *row = hot_x + tok * (size_t)hot_ldx;
+    const float *row2 = MODE == BITNET_HIP_INPUT_RELU2_MUL ? hot_x2 + tok * (size_t)hot_ldx : nullptr;
+    const uint64_t magics = MODE == BITNET_HIP_INPUT_GQA_BROADCAST ? reinterpret_cast<uintptr_t>(hot_x2) : 0;
 
-    // Every load is unconditional (clamped indices, values discarded), in the order in which the data is needed.
-    // First what the preloaded arguments alone address: the input row and the RMSNorm weights.  The argument buffer is
-    // read once these loads are on their way (it takes as long to arrive as the row: both come from memory), then
-    // the sum of squares, so that the two latencies run side by side.
-    float4 v[NCHB], gm[NORM ? NCHB : 1];
-    constexpr int NSS = NORM ? 4 * NCHB : 1;  // chunks per virtual lane of the summation order
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i) v[i] = load_chunk<MODE, true>(hot, tok, min(tid + bs * i, chunks - 1));
-    float4 vs[NSS];
-    if constexpr (NORM) {
-        if (wave < 4) {  // thread tid < 256 is virtual lane tid: it fetches the lane's chunks itself (from L2)
-#pragma unroll
-            for (int i = 0; i < NSS; ++i) vs[i] = load_chunk<MODE, true>(hot, tok, min(tid + 256 * i, chunks - 1));
-        }
-#pragma unroll
-        for (int i = 0; i < NCHB; ++i) gm[i] = load_gamma_chunk(hot, min(tid + bs * i, chunks - 1), true);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // nothing below moves above: the first wait for the argument buffer comes here
+    // The loads that need no argument but the preloaded ones, unconditional (clamped indices, values discarded).
+    const int in_tile = 16 * ((lane >> 2) & 3) + 4 * (lane >> 4) + (lane & 3);
+    Row16<NORM, NCHB> row16;
+    row16.template load<MODE>(row, row2, magics, hot_head_chunks, hot_gamma, chunks, nw, wave, tid, in_tile);
+    __builtin_amdgcn_sched_barrier(0);
 
-    const int lds_words = p.kt_count * 64;
-    int pj = 0;
-#pragma unroll
-    for (int j = 0; j < GEMV_MAX_PROJ - 1; ++j)
-        if (j + 1 < p.nproj && group >= p.proj[j].rb_end) pj = j + 1;
-    const GemvProjDev &P = p.proj[pj];
-    const int rb0 = (group - (pj ? p.proj[pj - 1].rb_end : 0)) * RBW;  // rb_end counts groups of RBW row blocks
-    const int rb_count = (P.n + TILE_ROWS - 1) / TILE_ROWS;
-    const uint4 *tiles = reinterpret_cast<const uint4 *>(P.w) + lane;
-    // k-tile kt holds chunks 64*kt .. 64*kt + 63: exactly what wavefront kt % 16 quantises, so a wavefront multiplies
-    // the tiles of its own chunks (tiles and row blocks past the end repeat the last one; their results are not added).
-    // When the tiles are requested (measured on the 30-block token step, replayed from a graph): with RMSNorm, once
-    // the argument buffer has arrived, ahead of the sum of squares (483.4 us a step against 489.7 behind the first
-    // barrier); without it, behind the absmax barrier (requested as early there the step takes 494 us: the weight
-    // stream then competes with the input row, which the kernel's chain of reductions hangs on).
-    uint4 wt[RBW][NCHB];
-    auto request_weight_tiles = [&]() {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int r = 0; r < RBW; ++r)
-#pragma unroll
-            for (int i = 0; i < NCHB; ++i)
-                wt[r][i] = load_weight_slot(tiles + ((size_t)min(rb0 + r, rb_count - 1) * p.kt_count + min(wave + nw * i, p.kt_count - 1)) * 64);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // epilogue operands: absent ones read the input row instead (always there) and are not used; the weight scale goes
-    // through a per-lane address so that it is a vector load, which nothing waits for before the epilogue
-    const int e_n = min((rb0 + (tid >> 4)) * TILE_ROWS + (tid & 15), P.n - 1);  // meaningful for tid < 16 * RBW
-    int lane_zero = 0;
-    asm volatile("" : "+v"(lane_zero));
-    const float e_ws = (P.out ? P.w_scale : hot_x)[lane_zero];
-    const float e_bias = *(P.bias ? P.bias + e_n : hot_x);
-    const float e_res = *(P.residual ? P.residual + (tok * (size_t)P.n + e_n) : hot_x);
+    // The other arguments, all at once, and pinned here.  Which projection a workgroup serves it knows from the preloaded
+    // ends of the first two (INT_MAX where there is no next one).
+    typedef const __attribute__((address_space(4))) v16u *arg_ptr;
+    const arg_ptr blocks = (arg_ptr)((uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + FUSED16_ARGS_AT);
+    const int pj = group < hot_end0 ? 0 : (group < hot_end1 ? 1 : 2), first_group = group < hot_end0 ? 0 : (group < hot_end1 ? hot_end0 : hot_end1);
+    v16u common = blocks[0], P = blocks[1 + pj];
     if (tid < RBW * TILE_ROWS) tot[tid >> 4][tid & 15] = 0;
+    if (tid < 16 && tid >= nw) red_f[1][tid] = 0.0f;  // the slots of absent wavefronts hold the neutral element
+    if (tid == 0) asum_s = 0;
+    float k_f = (float)hot_k, k_recip = recip_of_ok_divisor(k_f);  // k <= 8192: a divisor the short division accepts
+    asm volatile("" : "+s"(common), "+s"(P), "+v"(k_recip));
+    const int kt_count = (int)common[0];
+    const float eps = __builtin_bit_cast(float, (unsigned)common[1]);
+    const global_ptr<uint32_t> q_out = pointer_at<uint32_t>(common, 4);
+    const global_ptr<float> a_scale_out = pointer_at<float>(common, 6);
+    const global_ptr<int32_t> a_sum_out = pointer_at<int32_t>(common, 8);
+    const global_ptr<const float> absent = (global_ptr<const float>)(uintptr_t)hot_x;
+    const global_ptr<const float> w_scale = pointer_at<const float>(P, 2), bias = pointer_at<const float>(P, 4), residual = pointer_at<const float>(P, 6);
+    const global_ptr<float> out = pointer_at<float>(P, 8);
+    const global_ptr<int32_t> acc_out = pointer_at<int32_t>(P, 10);
+    const int P_n = (int)P[12];
+    const int rb0 = (group - first_group) * RBW;  // rb_end counts groups of RBW row blocks
+    const int rb_count = (P_n + TILE_ROWS - 1) / TILE_ROWS;
+    // Epilogue operands, fetched by the wavefronts that store; absent ones read the input row instead (always there) and are
+    // not used.  The weight scale goes through a per-lane address so that it is a vector load, which nothing waits for
+    // before the epilogue.
+    float e_ws = 0.0f, e_bias = 0.0f, e_res = 0.0f;
+    if (64 * wave < TILE_ROWS * RBW) {
+        const int e_n = min((rb0 + (tid >> 4)) * TILE_ROWS + (tid & 15), P_n - 1);
+        int lane_zero = 0;
+        asm volatile("" : "+v"(lane_zero));
+        e_ws = (out ? w_scale : absent)[lane_zero];
+        e_bias = *(bias ? bias + e_n : absent);
+        e_res = *(residual ? residual + (tok * (size_t)P_n + e_n) : absent);
+    }
+    // The weight tiles (tiles and row blocks past the end repeat the last one; their results are not added), non-temporal.
+    // The vector memory of a compute unit answers in the order of the requests, whichever wavefront they are from: a tile
+    // that comes from memory would hold up the input row of a wavefront that asked a little later.  So all wavefronts meet
+    // once their row is requested, and ask for the tiles then.
+    typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
+    const global_ptr<const v4u_t> tiles = pointer_at<const v4u_t>(P, 0) + lane;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    v4u_t wt[RBW][NCHB];
 #pragma unroll
-    for (int i = 0; i < NCHB; ++i)
-        if (tid + bs * i >= chunks) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-
-    if constexpr (NORM) {
-        request_weight_tiles();
-        if (wave < 4) {
-            float part = 0.0f;
-#pragma unroll
-            for (int i = 0; i < NSS; ++i)
-                if (tid + 256 * i < chunks) part = sum_squares4(part, vs[i]);  // chunks past the end would add +0
-            part = wave_sum_f32(part);
-            if (lane == 0) red_f[0][wave] = part;
-        }
-        lds_barrier();
-        const float ss = f32_add(f32_add(f32_add(red_f[0][0], red_f[0][1]), red_f[0][2]), red_f[0][3]);
-        const RowDivisor rdiv = make_row_divisor(rms_from_ss(ss, p.k, p.src.eps));
+    for (int r = 0; r < RBW; ++r)
 #pragma unroll
         for (int i = 0; i < NCHB; ++i)
-            if (tid + bs * i < chunks) v[i] = normalize4(v[i], rdiv, gm[i]);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i) amax = absmax4(amax, v[i]);
-    amax = wave_max_f32(amax);
-    if (lane == 0) red_f[1][wave] = amax;
-    lds_barrier();
-    if constexpr (!NORM) request_weight_tiles();
-    amax = red_f[1][0];
-#pragma unroll
-    for (int w = 1; w < 16; ++w) amax = fmaxf(amax, red_f[1][w]);
-    const float scale = scale_from_absmax(amax);
-    uint32_t *lds_w = reinterpret_cast<uint32_t *>(lds_a);
-    int isum = 0;
-#pragma unroll
-    for (int i = 0; i < NCHB; ++i) {
-        const int c = tid + bs * i;
-        if (c < chunks) {
-            const uint32_t packed = quant4_packed(v[i], scale, &isum);
-            lds_w[c] = packed;
-            if (p.q_out && group == 0) reinterpret_cast<uint32_t *>(p.q_out + tok * (size_t)hot_k)[c] = packed;
-        } else if (c < lds_words) {
-            lds_w[c] = 0;
-        }
-    }
-    isum = wave_sum_i32(isum);
-    if (lane == 0) red_i[wave] = isum;
-    // the int8 values this wavefront reads back below are its own: no workgroup barrier, only the LDS queue of the wavefront
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+            wt[r][i] = __builtin_nontemporal_load(tiles + ((size_t)min(rb0 + r, rb_count - 1) * kt_count + min(wave + nw * i, kt_count - 1)) * 64);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t packed[NCHB];
+    const float scale = row16.quantise(chunks, k_f, k_recip, eps, wave, tid, red_f, packed);
 
-    // Dot products on the matrix unit: the tile's 16 rows are the B operand of v_mfma_i32_16x16x64_i8 (lane l: row l mod 16,
-    // columns 64t + 16kq .. +15 for dword t, kq = l / 16), the activations are row 0 of the A operand (lanes 0, 16, 32, 48
-    // hold the four column groups; the other 15 rows are zero), so result register 0 of lanes 0..15 is the sum over the
-    // 64 columns of step t for rows 0..15.  Against dot4 this leaves only the unpacking of the 2-bit codes on the VALU.
-    typedef int v4i_t __attribute__((ext_vector_type(4)));
-    const int kq = lane >> 4;
-    const bool row0 = (lane & 15) == 0;
+    v4i acc[RBW], sums = {0, 0, 0, 0};
+#pragma unroll
+    for (int r = 0; r < RBW; ++r) acc[r] = (v4i){0, 0, 0, 0};
+    constexpr bool IN_PLACE = RBW >= 4;
 #pragma unroll
     for (int i = 0; i < NCHB; ++i) {
-        const int kt = wave + nw * i;
-        if (kt < p.kt_count) {  // uniform over the wavefront
-            // row blocks in batches of at most four: the accumulators of a batch are 16 registers
-            constexpr int RBB = RBW < 4 ? RBW : 4;
+        if (NCHB > 1 && wave + nw * i >= kt_count) break;  // uniform over the wavefront
+        if (q_out && group == 0 && row16.chunk[i] < chunks) q_out[tok * (size_t)chunks + row16.chunk[i]] = packed[i];
+        const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+        v4i af[4];  // the A operands: chunk (t, u) of a column group is in its lane 4t + u
 #pragma unroll
-            for (int r0 = 0; r0 < RBW; r0 += RBB) {
-                v4i_t acc[RBB];
+        for (int j = 0; j < 4; ++j)
+            af[j] = IN_PLACE ? (v4i){row_lane(packed[i], j), row_lane(packed[i], 4 + j), row_lane(packed[i], 8 + j), row_lane(packed[i], 12 + j)}
+                             : (v4i){row_lane(packed[i], 4 * j), row_lane(packed[i], 4 * j + 1), row_lane(packed[i], 4 * j + 2), row_lane(packed[i], 4 * j + 3)};
 #pragma unroll
-                for (int r = 0; r < RBB; ++r) acc[r] = (v4i_t){0, 0, 0, 0};
+        for (int j = 0; j < 4; ++j) sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[j], ones, sums, 0, 0, 0);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    v4i_t af = (v4i_t){0, 0, 0, 0};
-                    if (row0) af = *reinterpret_cast<const v4i_t *>(lds_a + kt * 16 + 4 * t + kq);
+        for (int r = 0; r < RBW; ++r) {
+            const v4u_t w4 = wt[r][i];
+            if constexpr (IN_PLACE) {
+                auto codes = [&](unsigned mask, int shift) {
+                    return (v4i){(int)((w4[0] >> shift) & mask), (int)((w4[1] >> shift) & mask), (int)((w4[2] >> shift) & mask), (int)((w4[3] >> shift) & mask)};
+                };
+                v4i part = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[2], codes(0x30303030u, 0), (v4i){0, 0, 0, 0}, 0, 0, 0);
+                part[0] >>= 2;  // 16 times the sum; only the first result register is used
+                part = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[1], codes(0x0c0c0c0cu, 0), part, 0, 0, 0);
+                part[0] >>= 2;
+                part = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[0], codes(0x03030303u, 0), part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[3], codes(0x03030303u, 6), part, 0, 0, 0);
+                acc[r][0] += part[0];
+            } else {
 #pragma unroll
-                    for (int r = 0; r < RBB; ++r) {
-                        const uint4 w4 = wt[r0 + r][i];
-                        const uint32_t wd = t == 0 ? w4.x : (t == 1 ? w4.y : (t == 2 ? w4.z : w4.w));
-                        v4i_t bf;
-                        bf[0] = (int)(wd & 0x03030303u);
-                        bf[1] = (int)((wd >> 2) & 0x03030303u);
-                        bf[2] = (int)((wd >> 4) & 0x03030303u);
-                        bf[3] = (int)((wd >> 6) & 0x03030303u);
-                        acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf, acc[r], 0, 0, 0);
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < RBB; ++r)
-                    if (lane < TILE_ROWS) atomicAdd(&tot[r0 + r][lane], acc[r][0]);  // int32: any order gives the same sum
+                for (int t = 0; t < 4; ++t)
+                    acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[t], (v4i){(int)(w4[t] & 0x03030303u), (int)((w4[t] >> 2) & 0x03030303u),
+                                                                                (int)((w4[t] >> 4) & 0x03030303u), (int)((w4[t] >> 6) & 0x03030303u)},
+                                                                   acc[r], 0, 0, 0);
             }
         }
     }
+    if (wave < kt_count && lane < TILE_ROWS) {  // wavefronts beyond the row's tiles hold a repeated tile: nothing of theirs is added
+#pragma unroll
+        for (int r = 0; r < RBW; ++r) atomicAdd(&tot[r][lane], acc[r][0] - sums[0]);
+        if (a_sum_out && lane == 0) atomicAdd(&asum_s, sums[0]);
+    }
+    const float s_recip = recip_of_ok_divisor(scale);
+    const bool divisor_fits = invariant_divisor_ok(scale);
     lds_barrier();
 
     if (tid < TILE_ROWS * RBW) {
-        const int r = tid >> 4, row = tid & 15;
-        const int n = (rb0 + r) * TILE_ROWS + row;
-        int asum = 0;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) asum += red_i[w];
-        if (group == 0 && tid == 0) {
-            if (p.a_scale_out) p.a_scale_out[tok] = scale;
-            if (p.a_sum_out) p.a_sum_out[tok] = asum;
+        const int r = tid >> 4, rw = tid & 15;
+        const int n = (rb0 + r) * TILE_ROWS + rw;
+        const int total = tot[r][rw];
+        const float scaled = f32_mul((float)total, e_ws);
+        float y = div_by_invariant_unchecked(scaled, scale, s_recip);
+        if (__builtin_expect(!(divisor_fits && dividend_ok(scaled)), 0)) y = f32_div(scaled, scale);
+        if (bias) y = f32_add(y, e_bias);
+        if (residual) y = f32_add(y, e_res);
+        if (n < P_n) {
+            if (acc_out) acc_out[tok * (size_t)P_n + n] = total;
+            if (out) out[tok * (size_t)P_n + n] = y;
         }
-        if (n < P.n) {
-            const int total = tot[r][row] - asum;
-            if (P.acc) P.acc[tok * (size_t)P.n + n] = total;
-            if (P.out) {
-                float y = f32_mul((float)total, e_ws);
-                y = f32_div(y, scale);
-                if (P.bias) y = f32_add(y, e_bias);
-                if (P.residual) y = f32_add(y, e_res);
-                P.out[tok * (size_t)P.n + n] = y;
-            }
+        if (group == 0 && tid == 0) {
+            if (a_scale_out) a_scale_out[tok] = scale;
+            if (a_sum_out) a_sum_out[tok] = asum_s;
         }
     }
 }
-
-typedef int v4i __attribute__((ext_vector_type(4)));
 
 struct GemvMfmaParams {
     GemvProjDev proj[GEMV_MAX_PROJ];  // rb_end counts groups of RB row blocks
@@ -1262,31 +1260,31 @@ int launch_fused_mode(const GemvParams &p, hipStream_t stream)
 }
 
 template <int MODE, int RBW>
-int launch_fused16_mode(const GemvParams &p, hipStream_t stream)
+int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src, int m, hipStream_t stream)
 {
-    const bool norm = p.src.gamma != nullptr;
-    const size_t lds = (size_t)p.kt_count * 16 * sizeof(uint4);
-    const dim3 grid(8u * (unsigned)p.m, ((unsigned)p.proj[p.nproj - 1].rb_end + 7u) / 8u);
+    const bool norm = src.gamma != nullptr;
+    const dim3 grid(8u * (unsigned)m, ((unsigned)p.proj[nproj - 1].rb_end + 7u) / 8u);
     // One wavefront per k-tile (at least the four of the summation order) for rows of up to 16 k-tiles, one chunk per
-    // thread; 16 wavefronts and two chunks per thread above.  Fewer wavefronts with more chunks each are slower (the
-    // element-wise steps lose their parallelism: 2560 columns on 5 wavefronts 581 us per 30-layer step against 507 on 10).
+    // thread; 16 wavefronts and two chunks per thread above.
     const int nchb = p.kt_count <= 16 ? 1 : 2;
-    const int nw = p.kt_count <= 16 ? row_workgroup_waves(p.src.k) : 16;
-    if (p.src.gqa_group < 0 || p.src.gqa_group > 0xffff) return fail(BITNET_HIP_INVALID_CONFIG, "GQA group %d out of range", p.src.gqa_group);
+    const int nw = p.kt_count <= 16 ? row_workgroup_waves(src.k) : 16;
     const dim3 block(64u * (unsigned)nw);
-#define BITNET_HOT_ARGS p.src.x, p.src.x2, p.src.gamma, p.src.k, p.src.head_dim, p.src.gqa_group | (nw << 16), (int)p.src.ldx
+    const float *x2 = src.x2;
+    if (MODE == BITNET_HIP_INPUT_GQA_BROADCAST) {
+        uint64_t magics = 0;
+        if (!row16_magics(src.head_dim, src.gqa_group, &magics))
+            return fail(BITNET_HIP_INVALID_CONFIG, "GQA group of %d heads of %d out of range", src.gqa_group, src.head_dim);
+        x2 = reinterpret_cast<const float *>(static_cast<uintptr_t>(magics));
+    }
+    const int end0 = nproj > 1 ? p.proj[0].rb_end : 0x7fffffff, end1 = nproj > 2 ? p.proj[1].rb_end : 0x7fffffff;
+#define BITNET_HOT_ARGS src.x, x2, src.gamma, src.k, src.head_dim / 4, nw, (int)src.ldx, end0, end1
 #define BITNET_F16_LAUNCH(NCHB) \
     do { \
-        if (norm) hipLaunchKernelGGL((gemv_fused16_kernel<MODE, true, NCHB, RBW>), grid, block, lds, stream, BITNET_HOT_ARGS, p); \
-        else hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, NCHB, RBW>), grid, block, lds, stream, BITNET_HOT_ARGS, p); \
+        if (norm) hipLaunchKernelGGL((gemv_fused16_kernel<MODE, true, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
+        else hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
     } while (0)
-    if (nchb == 1) {
-        BITNET_F16_LAUNCH(1);
-    } else if constexpr (RBW <= 8) {  // two k-tiles per wavefront: the tiles of 16 row blocks would not fit the registers
-        BITNET_F16_LAUNCH(2);
-    } else {
-        return fail(BITNET_HIP_UNSUPPORTED, "gemv_fused16: %d row blocks per workgroup with %d k-tiles", RBW, p.kt_count);
-    }
+    if (nchb == 1) BITNET_F16_LAUNCH(1);
+    else BITNET_F16_LAUNCH(2);
 #undef BITNET_F16_LAUNCH
 #undef BITNET_HOT_ARGS
     BITNET_HIP_CHECK_LAUNCH("gemv_fused16_kernel");
@@ -1294,12 +1292,14 @@ int launch_fused16_mode(const GemvParams &p, hipStream_t stream)
 }
 
 // rbw: row blocks per workgroup (rb_end then counts groups of rbw row blocks, per projection)
-int fill_projs(GemvParams &p, const GemvProj *projs, int nproj, size_t t0, size_t k, int rbw = 1)
+// Params: GemvParams or Fused16Params
+template <typename Params>
+int fill_projs(Params &p, const GemvProj *projs, int nproj, size_t t0, size_t k, int rbw = 1)
 {
     int rb_end = 0;
     for (int j = 0; j < nproj; ++j) {
         const GemvProj &s = projs[j];
-        GemvProjDev &d = p.proj[j];
+        auto &d = p.proj[j];
         d.w = s.tiled; d.w_scale = s.w_scale; d.bias = s.bias; d.n = (int)s.n;
         d.residual = s.residual ? s.residual + t0 * s.n : nullptr;
         d.out = s.out ? s.out + t0 * s.n : nullptr;
@@ -1308,8 +1308,6 @@ int fill_projs(GemvParams &p, const GemvProj *projs, int nproj, size_t t0, size_
         d.rb_end = rb_end;
     }
     for (int j = nproj; j < GEMV_MAX_PROJ; ++j) p.proj[j] = p.proj[nproj - 1];
-    p.nproj = nproj;
-    p.k = (int)k;
     p.kt_count = (int)k_tiles(k);
     return rb_end;
 }
@@ -1459,6 +1457,8 @@ int launch_gemv_tiled(const GemvProj *projs, int nproj, const int8_t *a, const f
         return fail(BITNET_HIP_UNSUPPORTED, "decode GEMV: k=%zu does not fit the LDS activation buffer", k);
     GemvParams p = {};
     if (fill_projs(p, projs, nproj, 0, k) == 0) return BITNET_HIP_OK;
+    p.k = (int)k;
+    p.nproj = nproj;
     p.m = 1;
     p.a = a;
     p.a_scale = a_scale;
@@ -1467,8 +1467,7 @@ int launch_gemv_tiled(const GemvProj *projs, int nproj, const int8_t *a, const f
 
 // Row blocks per workgroup of gemv_fused16_kernel.  Every workgroup quantises its token's input row for itself: that
 // arithmetic is repeated by every workgroup of the launch, and two workgroups on one compute unit take turns on its
-// SIMDs, so the launch is sized to about one workgroup per compute unit where the registers allow (a wavefront holds
-// the tiles of all its row blocks: 16 of them for rows of up to 16 k-tiles, 8 above).
+// SIMDs, so the launch is sized to about one workgroup per compute unit.
 int fused16_row_blocks_per_workgroup(size_t m, size_t k, size_t blocks)
 {
     if (m == 1) {
@@ -1477,11 +1476,11 @@ int fused16_row_blocks_per_workgroup(size_t m, size_t k, size_t blocks)
         return (blocks > 256 && k <= 4096) ? 2 : 1;
     }
     // Several tokens, each with its own workgroups: the fewest row blocks per workgroup that keep the launch within one
-    // workgroup per compute unit, at most 8 (16 lose: the dot products of 16 row blocks are a wavefront's serial work).
-    // 30-block step at 2 / 3 / 4 / 6 / 8 tokens: 578 / 662 / 713 / 778 / 901 us; with a limit of 512 workgroups and at
-    // most 4 row blocks each 646 / 733 / 779 / 1023 / 1150 us.
+    // workgroup per compute unit, at most 8 (4 of rows above 4096 columns, whose wavefronts hold two tiles of each).  30-block
+    // step at 2 / 3 / 4 / 6 tokens: 541 / 593 / 667 / 713 us; with launches of up to 512 workgroups 541 / 606 / 670 / 713.
     int rbw = 1;
-    while (rbw < 8 && (blocks + rbw - 1) / rbw * m > 256) rbw *= 2;
+    const int most = k_tiles(k) > 16 ? 4 : 8;
+    while (rbw < most && (blocks + rbw - 1) / rbw * m > 256) rbw *= 2;
     return rbw;
 }
 
@@ -1519,21 +1518,19 @@ int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const fl
         // a wavefront to hold the tiles of several row blocks (one token, gate alone, 432 row blocks: 4.50 us with one
         // row block per workgroup, 3.82 us with two)
         const int rbw16 = fused16_row_blocks_per_workgroup(m, k, blocks);
-        GemvParams p = {};
+        Fused16Params p = {};
         if (fill_projs(p, projs, nproj, 0, k, rbw16) == 0) return BITNET_HIP_OK;
-        p.m = (int)m;
-        p.src.x = x; p.src.x2 = x2; p.src.gamma = gamma; p.src.ldx = ldx; p.src.k = (int)k;
-        p.src.head_dim = (int)(head_dim ? head_dim : 1); p.src.gqa_group = (int)(gqa_group ? gqa_group : 1);
-        p.src.sum_order = sum_order; p.src.eps = eps;
-        p.q_out = q_out; p.a_scale_out = a_scale_out; p.a_sum_out = a_sum_out;
+        RowSource src = {};
+        src.x = x; src.x2 = x2; src.gamma = gamma; src.ldx = ldx; src.k = (int)k;
+        src.head_dim = (int)(head_dim ? head_dim : 1); src.gqa_group = (int)(gqa_group ? gqa_group : 1);
+        p.eps = eps; p.q_out = q_out; p.a_scale_out = a_scale_out; p.a_sum_out = a_sum_out;
 #define BITNET_F16_MODES(RBW) \
     switch (input_mode) { \
-        case BITNET_HIP_INPUT_PLAIN: return launch_fused16_mode<BITNET_HIP_INPUT_PLAIN, RBW>(p, stream); \
-        case BITNET_HIP_INPUT_RELU2_MUL: return launch_fused16_mode<BITNET_HIP_INPUT_RELU2_MUL, RBW>(p, stream); \
-        default: return launch_fused16_mode<BITNET_HIP_INPUT_GQA_BROADCAST, RBW>(p, stream); \
+        case BITNET_HIP_INPUT_PLAIN: return launch_fused16_mode<BITNET_HIP_INPUT_PLAIN, RBW>(p, nproj, src, (int)m, stream); \
+        case BITNET_HIP_INPUT_RELU2_MUL: return launch_fused16_mode<BITNET_HIP_INPUT_RELU2_MUL, RBW>(p, nproj, src, (int)m, stream); \
+        default: return launch_fused16_mode<BITNET_HIP_INPUT_GQA_BROADCAST, RBW>(p, nproj, src, (int)m, stream); \
     }
         switch (rbw16) {
-            case 16: BITNET_F16_MODES(16)
             case 8: BITNET_F16_MODES(8)
             case 4: BITNET_F16_MODES(4)
             case 2: BITNET_F16_MODES(2)
@@ -1544,6 +1541,8 @@ int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const fl
     const int rbw = (blocks > 512 && k <= 3 * 1024) ? 2 : 1;
     GemvParams p = {};
     if (fill_projs(p, projs, nproj, 0, k, rbw) == 0) return BITNET_HIP_OK;
+    p.k = (int)k;
+    p.nproj = nproj;
     p.m = (int)m;
     p.src.x = x; p.src.x2 = x2; p.src.gamma = gamma; p.src.ldx = ldx; p.src.k = (int)k;
     p.src.head_dim = (int)(head_dim ? head_dim : 1); p.src.gqa_group = (int)(gqa_group ? gqa_group : 1);

@@ -36,10 +36,66 @@ __device__ __forceinline__ bool dividend_ok(float x)
     const unsigned mag = __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
     return mag == 0u || (mag >= (64u << 23) && mag < (190u << 23));  // 0, or 2^-63 <= |x| < 2^63
 }
+// SIGNED_ZERO false: a zero dividend may lose its sign (one operation less, for callers that round to an integer next).
+template <bool SIGNED_ZERO = true>
 __device__ __forceinline__ float div_by_invariant_unchecked(float x, float d, float recip)
 {
     const float q0 = x * recip;
     const float rem = __builtin_fmaf(-q0, d, x);
-    return __builtin_copysignf(__builtin_fmaf(rem, recip, q0), x);  // d > 0: the quotient has x's sign (also for -0)
+    const float q = __builtin_fmaf(rem, recip, q0);
+    return SIGNED_ZERO ? __builtin_copysignf(q, x) : q;  // d > 0: the quotient has x's sign (also for -0)
+}
+
+// The correctly rounded 1/d of a divisor that invariant_divisor_ok accepts: the hardware's approximation (within one ulp)
+// and one Newton step (Markstein: correctly rounded from there except for a significand of all ones).  Three dependent
+// operations in place of the nine of the full division.  Compared with 1.0f / d for every float of the accepted
+// exponents on the device: no difference.
+__device__ __forceinline__ float recip_of_ok_divisor(float d)
+{
+    const float r = __builtin_amdgcn_rcpf(d);
+    return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+}
+
+// The one significand that invariant_divisor_ok excludes.
+__device__ __forceinline__ bool significand_ok(float d) { return (__builtin_bit_cast(unsigned, d) & 0x7fffffu) != 0x7fffffu; }
+
+// A divisor shared by many dividends, ready for use.
+struct Divisor {
+    float d, recip;
+    bool fast;
+};
+__device__ __forceinline__ Divisor make_divisor(float d)
+{
+    Divisor v;
+    v.d = d;
+    v.fast = invariant_divisor_ok(d);
+    v.recip = recip_of_ok_divisor(d);  // not used unless fast
+    return v;
+}
+// x / d for values that are the same in every lane of the wavefront (or where a full division in all lanes is as cheap).
+__device__ __forceinline__ float div_uniform(float x, const Divisor &v)
+{
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(v.fast && dividend_ok(x))) == 0, 1)) return div_by_invariant_unchecked(x, v.d, v.recip);
+    return f32_div(x, v.d);
+}
+
+// Square root for exponents 2^-62 .. 2^62: Goldschmidt's iteration from the hardware's reciprocal square root with a final
+// residual correction (Markstein).  Compared with the correctly rounded root for every float of that range on the device:
+// no difference.
+__device__ __forceinline__ float sqrt_in_range(float a)
+{
+    const float r = __builtin_amdgcn_rsqf(a);
+    float g = a * r, h = 0.5f * r;
+    const float e = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    h = __builtin_fmaf(h, e, h);
+    return __builtin_fmaf(__builtin_fmaf(-g, g, a), h, g);
+}
+// The square root of a value that is the same in every lane: the plain one outside that range.
+__device__ __forceinline__ float sqrt_uniform(float a)
+{
+    const unsigned expo = __builtin_bit_cast(unsigned, a) >> 23;  // the sign counts as a large exponent
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(expo > 64u && expo < 190u)) == 0, 1)) return sqrt_in_range(a);
+    return f32_sqrt(a);
 }
 }  // namespace bitnet

@@ -17,8 +17,11 @@ inline size_t tiled_bytes(size_t n, size_t k) { return row_blocks(n) * k_tiles(k
 // act_quant.hip
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
-                     int8_t *q, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero = nullptr,
+                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero = nullptr,
                      size_t zero_n = 0);  // zero[0 .. zero_n): cleared by the launch (tile counters of the GEMM behind it)
+// ldq: row stride of q, k or padded_k(k).  Padded rows end in zeros, so the contraction may take padded_k(k) for k: its weight
+// tiles are padded with zero weights, and every width then has the aligned rows the LDS-direct and the batched kernels need.
+inline size_t padded_k(size_t k) { return (k + TILE_K - 1) / TILE_K * TILE_K; }
 
 // absmax_quantize_activations (activations.rs:530-641): one scale per tensor; scratch of absmax_quantize_scratch_bytes(n)
 // bytes; stats: 4 floats (scale, mse, min, max)

@@ -1515,3 +1515,35 @@ def test_layers_loaded_from_the_host_give_their_bytes_back(n, k, layout):
         assert np.array_equal(host(bh.untile_weights(tiled, n, k)), orc.pack_2bit(w))
         x = synth_activations(rng, 2, k)
         assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, orc.pack_2bit(w), n, f32(0.75))[0])
+
+
+@pytest.mark.parametrize("m,k", [(512, 516), (513, 516), (300, 4096), (300, 4100), (513, 7168), (513, 7172), (3, 8192), (513, 1024), (513, 301)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_activation_quant_at_the_edges_of_its_kernels(m, k, norm):
+    """Rows on both sides of each line between the quantiser's kernels: rows that all run at once and more, one and two chunks per
+    thread, rows too long for a 256-thread workgroup's registers, short rows, rows that start unaligned."""
+    rng = np.random.default_rng(m + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    x[1] = 0.0
+    x[2, ::7] *= f32(2.0**-70)
+    g = rng.standard_normal(k, dtype=f32) if norm else None
+    q, s, asum, _ = bh.quantize_activations_i8(dev(x), dev(g) if norm else None, eps=1e-5, want_sum=True)
+    q_ref, s_ref, rs_ref = orc.rmsnorm_quantize_i8(x, g, 1e-5, orc.SUM_BLOCK256)
+    assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), rs_ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 40, 301), (130, 96, 441), (100, 330, 260), (300, 200, 3201)])
+def test_forward_of_padded_widths_bit_exact(m, n, k):
+    """Widths that are no multiple of a tile run on padded int8 rows; a workspace without room for the padding still serves."""
+    rng = np.random.default_rng(m + n + k)
+    w, x = synth_weights(rng, n, k), synth_activations(rng, m, k, outliers=True)
+    g = rng.standard_normal(k, dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "padded")
+    layer.update_weights(dev(w))
+    qw, ws_ = orc.quantize_weights_absmean(w)
+    ref = orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_, g=g, eps=1e-5)[0]
+    up = lambda v: (v + 255) // 256 * 256
+    least = torch.empty((up(m * k) + 2 * up(4 * m) + 256,), dtype=torch.uint8, device="cuda")
+    assert least.numel() < layer.workspace_size(m)
+    for ws in (None, least, torch.empty((layer.workspace_size(m),), dtype=torch.uint8, device="cuda")):
+        assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g), workspace=ws)), ref)
