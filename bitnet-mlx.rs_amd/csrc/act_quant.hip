@@ -24,6 +24,7 @@ struct ActQuantParams {
     float *y;
     size_t m;
     size_t ldq;      // row stride of q: k, or more with the bytes from k on (up to the next multiple of 256) cleared
+    int tiled;       // layout of q: see RowPlace
     int seq_in_lds;  // the launch carries LDS for the row's squares (literal summation order: sum_sequential_lds)
     unsigned *zero;  // optional: zero[0 .. zero_n) is cleared by the first workgroup (counters of the launch that follows)
     int zero_n;
@@ -40,12 +41,20 @@ __device__ __forceinline__ void clear_counters(const ActQuantParams &p)
 
 constexpr size_t ROW_QUANT_MAX_ROWS = 512;
 
-// Where the int8 row goes.
+// Where the int8 row goes: row-major (stride ldq), or by ActRows::TILES16: the rows of a group of 16 (rows_here of them in the
+// last group) interleaved in pieces of 16 bytes, row-fastest, so that a tile of 16 rows by 64 columns is contiguous.
 struct RowPlace {
     size_t base;
-    __device__ __forceinline__ size_t chunk(int c) const { return base + 4 * (size_t)c; }
+    unsigned piece;  // from one 16-byte piece of the row to the next
+    __device__ __forceinline__ size_t chunk(int c) const { return base + (size_t)((unsigned)(c >> 2) * piece) + (unsigned)(c & 3) * 4u; }
 };
-__device__ __forceinline__ RowPlace row_place(size_t row, size_t ldq) { return {row * ldq}; }
+__device__ __forceinline__ RowPlace row_place(size_t row, size_t m, size_t ldq, bool tiled)
+{
+    if (!tiled) return {row * ldq, 16u};
+    const size_t group = row >> 4;
+    const unsigned rows_here = (unsigned)min((size_t)16, m - group * 16);
+    return {group * 16 * ldq + (row & 15) * 16, 16u * rows_here};
+}
 
 // One quantised chunk (elements 4c .. 4c + 3 of the row; those from k on are +0 in `e`) to the int8 row, and to y if asked for.
 template <bool VEC>
@@ -122,7 +131,7 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
     const float scale = scale_from_absmax(wave_max_f32(amax));
 
     int isum = 0;
-    const RowPlace place = row_place(row, p.ldq);
+    const RowPlace place = row_place(row, p.m, p.ldq, p.tiled != 0);
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
         const int c = lane + 64 * i;
@@ -211,7 +220,7 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
     const float scale = scale_from_absmax(amax);
 
     int isum = 0;
-    const RowPlace place = row_place(row, p.ldq);
+    const RowPlace place = row_place(row, p.m, p.ldq, p.tiled != 0);
 #pragma unroll
     for (int i = 0; i < nloop; ++i) {
         int c = tid + 256 * i;
@@ -248,7 +257,8 @@ struct RowQuantArgs {
     unsigned *zero;
     int zero_n;
     int ldq;
-    int unused[4];
+    int tiled;
+    int unused[3];
 };
 static_assert(sizeof(RowQuantArgs) == 64, "one scalar load");
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -280,7 +290,7 @@ __global__ __launch_bounds__(1024) void act_quant_row_kernel(const float *hot_x,
     const global_ptr<int32_t> a_sum = pointer_at<int32_t>(block, 4);
     const global_ptr<unsigned> zero = pointer_at<unsigned>(block, 8);
     const int zero_n = (int)block[10], ldq = (int)block[11];
-    const RowPlace place = row_place(row, (size_t)ldq);
+    const RowPlace place = row_place(row, (size_t)hot_m, (size_t)ldq, block[12] != 0);
 
     uint32_t packed[NCHB];
     const float scale = row16.quantise(chunks, k_f, k_recip, hot_eps, wave, tid, red_f, packed);
@@ -343,7 +353,7 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
             x2 = reinterpret_cast<const float *>(static_cast<uintptr_t>(magics));
         }
         if (in_range) {
-            const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, p.zero, p.zero_n, (int)p.ldq, {0, 0, 0, 0}};
+            const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, p.zero, p.zero_n, (int)p.ldq, p.tiled, {0, 0, 0}};
             const int kt = (p.src.k + 255) >> 8, nchb = kt > 16 ? 2 : 1;
             const int nw = nchb == 2 ? (kt + 1) / 2 : row_workgroup_waves(p.src.k);
             const dim3 grid((unsigned)p.m), block(64u * (unsigned)nw);
@@ -606,9 +616,10 @@ int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratc
 
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
-                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero, size_t zero_n)
+                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero, size_t zero_n, ActRows rows)
 {
     ActQuantParams p;
+    p.tiled = rows == ActRows::TILES16;
     p.ldq = ldq;
     p.zero = zero; p.zero_n = (int)zero_n;
     p.src.x = x; p.src.x2 = x2; p.src.gamma = gamma; p.src.ldx = ldx; p.src.k = (int)k;
@@ -618,6 +629,7 @@ int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size
 
     if (ldq != k && (ldq % 4 != 0 || !aligned(q, 4) || ldq < k || ldq > (k + 255) / 256 * 256))
         return fail(BITNET_HIP_INVALID_CONFIG, "activation quantiser: int8 row stride %zu for %zu columns", ldq, k);
+    if (p.tiled && ldq % 256 != 0) return fail(BITNET_HIP_INVALID_CONFIG, "activation quantiser: tiles of rows of %zu columns", ldq);
     bool vec = (k % 4 == 0) && (ldx % 4 == 0) && aligned(x, 16) && aligned(q, 4) && (!x2 || aligned(x2, 16)) &&
                (!y || aligned(y, 16)) && (!gamma || aligned(gamma, 16));
     if (input_mode == BITNET_HIP_INPUT_GQA_BROADCAST) vec = vec && (head_dim % 4 == 0);

@@ -186,8 +186,11 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
     // A GEMM that splits k across workgroups finds its tile counters zeroed by the quantiser launched in front of it.  One
     // scratch serves one launch: more projections than one launch takes run without the split.
     const bool use_split = split && split->counters && count <= GEMM_MAX_PROJ && !gemv_takes(m, ldq, n_blocks, q);
-    int rc = launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, ldq, a_scale, a_sum,
-                              nullptr, s, use_split ? split->counters : nullptr, use_split ? split->counter_count : 0);
+    // Rows for the token GEMV go straight into the order that it reads, unless the caller wants to see them.
+    const bool tiles = !want_quant_outputs && gemv_rows_takes(m, ldq, n_blocks, q);
+    int rc = launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, ldq, a_scale, tiles ? nullptr : a_sum,
+                              nullptr, s, use_split ? split->counters : nullptr, use_split ? split->counter_count : 0,
+                              tiles ? ActRows::TILES16 : ActRows::ROW_MAJOR);
     if (rc != BITNET_HIP_OK) return rc;
     k = ldq;  // the columns past in_features are zero in the rows and in the tiles
     if (gemv_takes(m, k, n_blocks, q)) {
@@ -195,7 +198,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
             GemvProj pjs[GEMV_MAX_PROJ];
             const int nj = count - j0 < GEMV_MAX_PROJ ? count - j0 : GEMV_MAX_PROJ;
             for (int j = 0; j < nj; ++j) pjs[j] = proj_of(j0 + j);
-            rc = launch_gemv_tiled(pjs, nj, q, a_scale, m, k, s);
+            rc = tiles ? launch_gemv_rows(pjs, nj, q, a_scale, m, k, s) : launch_gemv_tiled(pjs, nj, q, a_scale, m, k, s);
             if (rc != BITNET_HIP_OK) return rc;
         }
         return BITNET_HIP_OK;

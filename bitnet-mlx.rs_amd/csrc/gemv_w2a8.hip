@@ -28,7 +28,8 @@
 // HBM traffic per call: n*k/4 weight bytes; the input row (K or 4K bytes per workgroup) comes from L2.
 // gemv_fused16_kernel is this launch with 16 wavefronts per workgroup (the default for one token; see its comment).
 //
-// gemv_mfma_kernel is the same weight-streaming scheme for 2..16 token rows: the 16 x 16 x 64 int8 MFMA takes
+// gemv_rows_kernel serves several tokens whose rows the quantiser laid out for it.  gemv_mfma_kernel is the same
+// weight-streaming scheme for 2..16 row-major token rows: the 16 x 16 x 64 int8 MFMA takes
 // the place of the dot-product chain (its A operand is 16 token rows x 64 columns, loaded straight from the
 // int8 activation matrix, which stays in L2; its B operand is a decoded weight dword, exactly as in the
 // prefill GEMM), so up to 16 tokens cost what one costs in weight traffic and instructions.  A workgroup
@@ -1186,6 +1187,187 @@ __global__ __launch_bounds__(256) void gemv_mfma_tg_kernel(const int8_t *hot_a, 
     }
 }
 
+// Several tokens on rows that the quantiser laid out for it (ActRows::TILES16): a workgroup of up to 16 wavefronts takes RB row
+// blocks and one group of up to 16 tokens, a wavefront the k-tiles wave, wave + nw, ... of them.  The tile of a token group by 64
+// columns is contiguous, so an A operand is one dense load into the registers the MFMA reads: no copy through LDS, no
+// gathers of 16 bytes per row, and no barrier before the products.  NT tiles are requested at once (LOOP: more than 16 NT tiles,
+// in batches of NT with the next batch in flight).  The rows' sums for the code offset are an MFMA on a constant operand and
+// leave the wavefront subtracted; the partial results of the wavefronts meet in LDS, and every thread finishes its own
+// outputs.  What a launch takes is one trip to memory, the MFMAs of a wavefront and that exchange.  6912 -> 2560, 16 tokens: 4.1 us
+// (gathering the rows from memory 7.6); a block of the 30-block stack: 25.7 us at 8 tokens, 35.8 at 42 (rows copied to LDS first
+// 30.0 and 50.2).
+// Everything that the loads need arrives preloaded, the weights' addresses too: a scalar load of an argument takes as long as
+// the weights do, and the two would add up (2560 columns, 160 row blocks: 0.55 us of 3.4).  Counts of row blocks and their
+// groups are packed, 16 bits each: rows and k-tiles; groups of projection 0, and of 0 and 1 (0xffff where there is no next
+// projection); row blocks of projections 0 and 1; row blocks of projection 2 and the wavefronts.
+struct RowsParams {
+    Fused16Proj proj[GEMV_MAX_PROJ];  // rb_end counts groups of RB row blocks
+    int kt_count;
+};
+constexpr int ROWS_ARGS_AT = 56;  // its offset in the argument buffer: five pointers and four ints before it
+
+template <int RB, int NT, bool LOOP>
+__global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, const uint8_t *hot_w0, const uint8_t *hot_w1, const uint8_t *hot_w2, unsigned hot_m_kt,
+                                                        unsigned hot_ends, unsigned hot_blocks, unsigned hot_blocks_nw, const float *a_scale,
+                                                        [[maybe_unused]] RowsParams args)
+{
+    extern __shared__ v4i part[];  // [nw][RB][64]
+    typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
+    // workgroup (x, y): token group x / 8, group 8y + x % 8 of row blocks, as in gemv_fused16_kernel: the token groups of one group
+    // of row blocks run on the same XCD
+    const int tg = (int)(blockIdx.x >> 3);
+    const int group = (int)blockIdx.y * 8 + (int)(blockIdx.x & 7);  // may lie past the last group: such workgroups store nothing
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = (int)(hot_m_kt & 0xffffu), kt_count = (int)(hot_m_kt >> 16), nw = (int)(hot_blocks_nw >> 16);
+    const int end0 = (int)(hot_ends & 0xffffu), end1 = (int)(hot_ends >> 16);
+    const int pj = group < end0 ? 0 : (group < end1 ? 1 : 2);
+    // the other arguments: asked for first, used once all loads of the products are on their way
+    typedef const __attribute__((address_space(4))) v16u *arg_ptr;
+    v16u P = ((arg_ptr)((uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + ROWS_ARGS_AT))[pj];
+    __builtin_amdgcn_sched_barrier(0);
+    const int rows_here = min(16, m - tg * 16);
+    const bool row_ok = (lane & 15) < rows_here;
+
+    // A operand of lane 16 g + r: row r, columns 16 g .. + 15 of a tile; lanes without a row load nothing (the results of their
+    // row are not used)
+    const global_ptr<const uint8_t> a_lane = (global_ptr<const uint8_t>)(uintptr_t)hot_a + (size_t)tg * 16 * TILE_K * kt_count +
+                                             (unsigned)(((lane >> 4) * rows_here + (lane & 15)) * 16);
+    auto load_a = [&](v4i (&af)[NT][4], int kt0) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) asm("" : "=v"(af[u][t]));
+        if (row_ok) {
+#pragma unroll
+            for (int u = 0; u < NT; ++u)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    af[u][t] = *(global_ptr<const v4i>)(a_lane + (unsigned)((min(kt0 + nw * u, kt_count - 1) * 4 + t) * 64 * rows_here));
+        }
+    };
+    v4i af[NT][4];
+    load_a(af, wave);
+    __builtin_amdgcn_sched_barrier(0);
+
+    const int rb0 = (group - (pj == 0 ? 0 : (pj == 1 ? end0 : end1))) * RB;
+    const int rb_count = (int)(pj == 0 ? hot_blocks & 0xffffu : (pj == 1 ? hot_blocks >> 16 : hot_blocks_nw & 0xffffu));
+    const global_ptr<const v4u_t> tiles = (global_ptr<const v4u_t>)(uintptr_t)(pj == 0 ? hot_w0 : (pj == 1 ? hot_w1 : hot_w2)) + lane;
+    auto load_w = [&](v4u_t (&w)[NT][RB], int kt0) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+                w[u][r] = __builtin_nontemporal_load(tiles + ((size_t)min(rb0 + r, rb_count - 1) * kt_count + min(kt0 + nw * u, kt_count - 1)) * 64);
+    };
+    v4u_t w[NT][RB];
+    load_w(w, wave);
+    __builtin_amdgcn_sched_barrier(0);
+
+    asm volatile("" : "+s"(P));
+    const global_ptr<const float> scales = (global_ptr<const float>)(uintptr_t)a_scale, absent = scales;
+    const global_ptr<const float> w_scale = pointer_at<const float>(P, 2), bias = pointer_at<const float>(P, 4), residual = pointer_at<const float>(P, 6);
+    const global_ptr<float> out = pointer_at<float>(P, 8);
+    const global_ptr<int32_t> acc_out = pointer_at<int32_t>(P, 10);
+    const int P_n = (int)P[12];
+
+    // Output e of the workgroup: token e / (16 RB), row block (e / 16) % RB, row e % 16.  Thread tid finishes the outputs tid, tid +
+    // 64 nw, ..: RB at most (a workgroup has four wavefronts at least).  Their operands are requested now, behind the tiles.
+    const int outputs = rows_here * RB * TILE_ROWS, step = 64 * nw;
+    float e_ws = 0.0f, e_bias[RB], e_res[RB], e_scale[RB];
+    {
+        int lane_zero = 0;
+        asm volatile("" : "+v"(lane_zero));
+        e_ws = (out ? w_scale : absent)[lane_zero];
+    }
+#pragma unroll
+    for (int s = 0; s < RB; ++s) {
+        e_bias[s] = 0.0f; e_res[s] = 0.0f; e_scale[s] = 1.0f;
+        if (64 * wave + s * step < outputs) {  // uniform over the wavefront
+            const int e = min(tid + s * step, outputs - 1);
+            const int n = min((rb0 + ((e >> 4) & (RB - 1))) * TILE_ROWS + (e & 15), P_n - 1), t = tg * 16 + e / (16 * RB);
+            e_scale[s] = (out ? scales + t : absent)[0];
+            e_bias[s] = (bias ? bias + n : absent)[0];
+            e_res[s] = (residual ? residual + ((size_t)t * P_n + n) : absent)[0];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    v4i acc[RB], sums = {0, 0, 0, 0};
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+    for (int r = 0; r < RB; ++r) acc[r] = (v4i){0, 0, 0, 0};
+    auto multiply = [&](const v4i (&a)[NT][4], const v4u_t (&wt)[NT][RB], int kt0) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            if (kt0 + nw * u >= kt_count) break;  // uniform over the wavefront
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][t], ones, sums, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    const unsigned wd = wt[u][r][t];
+                    const v4i bf = {(int)(wd & 0x03030303u), (int)((wd >> 2) & 0x03030303u), (int)((wd >> 4) & 0x03030303u), (int)((wd >> 6) & 0x03030303u)};
+                    acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][t], bf, acc[r], 0, 0, 0);
+                }
+            }
+        }
+    };
+    if constexpr (LOOP) {
+        for (int kt0 = wave; kt0 < kt_count; kt0 += nw * NT) {  // uniform over the wavefront
+            v4i a_next[NT][4];
+            v4u_t w_next[NT][RB];
+            load_a(a_next, kt0 + nw * NT);
+            load_w(w_next, kt0 + nw * NT);
+            multiply(af, w, kt0);
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) af[u][t] = a_next[u][t];
+#pragma unroll
+                for (int r = 0; r < RB; ++r) w[u][r] = w_next[u][r];
+            }
+        }
+    } else {
+        multiply(af, w, wave);
+    }
+    // Component i of a lane's result is token 4 (lane / 16) + i, row lane % 16.  It is stored at component (i + r) % 4, so that the
+    // reads below, of RB row blocks and 16 rows at once, spread over the banks.
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        const v4i d = acc[r] - sums;
+        part[((size_t)wave * RB + r) * 64 + lane] = (v4i){d[(0 - r) & 3], d[(1 - r) & 3], d[(2 - r) & 3], d[(3 - r) & 3]};
+    }
+    lds_barrier();
+    const int *part_i = reinterpret_cast<const int *>(part);
+#pragma unroll
+    for (int s = 0; s < RB; ++s) {
+        const int e = tid + s * step;
+        if (e >= outputs) break;
+        const int r = (e >> 4) & (RB - 1), tl = e / (16 * RB), lr = e & 15;
+        const int *from = part_i + r * 256 + ((tl >> 2) * 16 + lr) * 4 + ((tl + r) & 3);
+        int total = 0;
+        for (int v = 0; v < nw; v += 4) {  // past the last wavefront: its slot again, not added
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int got = from[min(v + j, nw - 1) * (RB * 256)];
+                total += v + j < nw ? got : 0;
+            }
+        }
+        const int n = (rb0 + r) * TILE_ROWS + lr;
+        if (n >= P_n) continue;
+        const size_t o = (size_t)(tg * 16 + tl) * P_n + n;
+        if (acc_out) acc_out[o] = total;
+        if (out) {
+            const float scaled = f32_mul((float)total, e_ws);
+            float y = div_by_invariant_unchecked(scaled, e_scale[s], recip_of_ok_divisor(e_scale[s]));
+            if (__builtin_expect(!(invariant_divisor_ok(e_scale[s]) && dividend_ok(scaled)), 0)) y = f32_div(scaled, e_scale[s]);
+            if (bias) y = f32_add(y, e_bias[s]);
+            if (residual) y = f32_add(y, e_res[s]);
+            out[o] = y;
+        }
+    }
+}
+
 // The reference's flat row-major packing, any n and k (rows need not start on a byte boundary).
 // One wavefront per output row; lane l takes columns 4l..4l+3, 4l+256.., gathers their codes one by one.
 __global__ __launch_bounds__(256) void gemv_rowmajor_kernel(const uint8_t *packed, const int8_t *a,
@@ -1310,6 +1492,19 @@ int fill_projs(Params &p, const GemvProj *projs, int nproj, size_t t0, size_t k,
     for (int j = nproj; j < GEMV_MAX_PROJ; ++j) p.proj[j] = p.proj[nproj - 1];
     p.kt_count = (int)k_tiles(k);
     return rb_end;
+}
+
+template <int RB, int NT, bool LOOP>
+int launch_rows(const RowsParams &p, int nproj, const int8_t *a, const float *a_scale, size_t m, int nw, hipStream_t stream)
+{
+    const dim3 grid(8u * (unsigned)((m + 15) / 16), ((unsigned)p.proj[nproj - 1].rb_end + 7u) / 8u);
+    const unsigned end0 = nproj > 1 ? (unsigned)p.proj[0].rb_end : 0xffffu, end1 = nproj > 2 ? (unsigned)p.proj[1].rb_end : 0xffffu;
+    auto blocks = [&](int j) { return (unsigned)row_blocks((size_t)p.proj[j].n); };
+    hipLaunchKernelGGL((gemv_rows_kernel<RB, NT, LOOP>), grid, dim3(64u * (unsigned)nw), (size_t)nw * RB * 1024, stream, a, p.proj[0].w, p.proj[1].w,
+                       p.proj[2].w, (unsigned)m | ((unsigned)p.kt_count << 16), end0 | (end1 << 16), blocks(0) | (blocks(1) << 16),
+                       blocks(2) | ((unsigned)nw << 16), a_scale, p);
+    BITNET_HIP_CHECK_LAUNCH("gemv_rows_kernel");
+    return BITNET_HIP_OK;
 }
 
 template <int RB, int MT>
@@ -1463,6 +1658,39 @@ int launch_gemv_tiled(const GemvProj *projs, int nproj, const int8_t *a, const f
     p.a = a;
     p.a_scale = a_scale;
     return launch_mode<MODE_PREQUANT>(p, stream);
+}
+
+int launch_gemv_rows(const GemvProj *projs, int nproj, const int8_t *a, const float *a_scale, size_t m, size_t k, hipStream_t stream)
+{
+    if (m == 0 || nproj <= 0) return BITNET_HIP_OK;
+    size_t blocks = 0;
+    for (int j = 0; j < nproj; ++j) blocks += row_blocks(projs[j].n);
+    // Row blocks per workgroup: the fewest that keep the launch within one workgroup per compute unit, at most 4 (within two: 36.9
+    // against 36.0 us a block of the stack at 42 tokens, 28.7 against 29.1 at 16).
+    const size_t tgroups = (m + 15) / 16;
+    int rb = 1;
+    while (rb < 4 && (blocks + rb - 1) / rb * tgroups > 256) rb *= 2;
+    const int kt = (int)k_tiles(k);
+    // One k-tile per wavefront up to 16, then two; more go through the loop with 16 wavefronts.
+    const int nt = kt <= 16 ? 1 : 2;
+    const int nw = kt > 32 ? 16 : ((kt + nt - 1) / nt < 4 ? 4 : (kt + nt - 1) / nt);
+    RowsParams p = {};
+    if (fill_projs(p, projs, nproj, 0, k, rb) == 0) return BITNET_HIP_OK;
+#define BITNET_ROWS(RB, NT, LOOP) return launch_rows<RB, NT, LOOP>(p, nproj, a, a_scale, m, nw, stream)
+    if (kt > 32) {
+        if (rb == 4) BITNET_ROWS(4, 1, true);
+        if (rb == 2) BITNET_ROWS(2, 2, true);
+        BITNET_ROWS(1, 2, true);
+    }
+    if (nt == 2) {
+        if (rb == 4) BITNET_ROWS(4, 2, false);
+        if (rb == 2) BITNET_ROWS(2, 2, false);
+        BITNET_ROWS(1, 2, false);
+    }
+    if (rb == 4) BITNET_ROWS(4, 1, false);
+    if (rb == 2) BITNET_ROWS(2, 1, false);
+    BITNET_ROWS(1, 1, false);
+#undef BITNET_ROWS
 }
 
 // Row blocks per workgroup of gemv_fused16_kernel.  Every workgroup quantises its token's input row for itself: that

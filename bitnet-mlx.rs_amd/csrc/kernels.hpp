@@ -15,10 +15,14 @@ inline size_t k_tiles(size_t k) { return (k + TILE_K - 1) / TILE_K; }
 inline size_t tiled_bytes(size_t n, size_t k) { return row_blocks(n) * k_tiles(k) * (size_t)TILE_BYTES; }
 
 // act_quant.hip
+// Layout of the int8 rows.  TILES16 (row stride a multiple of 256): what launch_gemv_rows reads, the 16 rows of a group
+// interleaved in pieces of 16 bytes; byte b of piece c of row r lies at 16 g ldq + (c R + r % 16) 16 + b, with g = r / 16 and R the
+// rows of that group (16; fewer in the last one).
+enum class ActRows { ROW_MAJOR, TILES16 };
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
                      int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero = nullptr,
-                     size_t zero_n = 0);  // zero[0 .. zero_n): cleared by the launch (tile counters of the GEMM behind it)
+                     size_t zero_n = 0, ActRows rows = ActRows::ROW_MAJOR);  // zero[0 .. zero_n): cleared by the launch (tile counters of the GEMM behind it)
 // ldq: row stride of q, k or padded_k(k).  Padded rows end in zeros, so the contraction may take padded_k(k) for k: its weight
 // tiles are padded with zero weights, and every width then has the aligned rows the LDS-direct and the batched kernels need.
 inline size_t padded_k(size_t k) { return (k + TILE_K - 1) / TILE_K * TILE_K; }
@@ -101,6 +105,14 @@ struct GemvProj {
 // activations already int8 ([m, k], a_scale [m]); any m (launched in groups of up to GEMV_MAX_M rows)
 int launch_gemv_tiled(const GemvProj *projs, int nproj, const int8_t *a, const float *a_scale, size_t m, size_t k,
                       hipStream_t stream);
+// the same for rows in ActRows::TILES16 order, where gemv_rows_takes says so
+constexpr size_t GEMV_ROWS_MAX_BLOCKS = 0xfff0;  // 16-row blocks of a launch (counts of 16 bits in its arguments)
+inline bool gemv_rows_takes(size_t m, size_t k, size_t n_blocks, const void *a)
+{
+    return m >= 2 && k % TILE_K == 0 && n_blocks <= GEMV_ROWS_MAX_BLOCKS && k_tiles(k) <= 0xffff && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
+           gemv_takes(m, k, n_blocks, a);
+}
+int launch_gemv_rows(const GemvProj *projs, int nproj, const int8_t *a, const float *a_scale, size_t m, size_t k, hipStream_t stream);
 // f32 input quantised inside the GEMV launch; only where gemv_fused_supported() says so.  q_out / a_scale_out /
 // a_sum_out (each optional) receive the quantiser's results.
 bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,

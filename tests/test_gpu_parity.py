@@ -1547,3 +1547,19 @@ def test_forward_of_padded_widths_bit_exact(m, n, k):
     assert least.numel() < layer.workspace_size(m)
     for ws in (None, least, torch.empty((layer.workspace_size(m),), dtype=torch.uint8, device="cuda")):
         assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g), workspace=ws)), ref)
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 95])
+@pytest.mark.parametrize("n,k", [(1, 4), (33, 260), (300, 1025), (700, 2560), (1400, 4352), (260, 8192), (700, 8448), (1400, 8448)])
+def test_forward_token_groups_bit_exact(m, n, k):
+    """The token GEMV on rows laid out by the quantiser: last token groups of one to sixteen rows, one, two and four row blocks per
+    workgroup, one and two k-tiles per wavefront and the loop over more, fewer tiles than wavefronts, row blocks past the end."""
+    rng = np.random.default_rng(m + n + k)
+    w, x = synth_weights(rng, n, k), synth_activations(rng, m, k, outliers=True)
+    bias, res = rng.standard_normal(n, dtype=f32), rng.standard_normal((m, n), dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "groups")
+    layer.update_weights(dev(w))
+    layer.update_bias(dev(bias))
+    qw, ws_ = orc.quantize_weights_absmean(w)
+    ref = orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_, eps=1e-5, bias=bias, residual=res)[0]
+    assert np.array_equal(host(layer.forward(dev(x), residual=dev(res))), ref)
