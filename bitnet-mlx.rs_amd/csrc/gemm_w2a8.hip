@@ -38,6 +38,8 @@
 // loads of stage s+1 are issued before the 4 k-steps of stage s are computed and written to LDS after them,
 // one barrier per stage.  Rows are padded to 272 bytes so that the 16-byte fragment reads of 8 consecutive
 // lanes fall in distinct banks.
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "ldsdma.hpp"
 
@@ -46,6 +48,7 @@ namespace bitnet {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 struct GemmProjDev {  // one projection of a launch of the LDS-direct kernels
     const uint8_t *w;
@@ -290,39 +293,87 @@ __device__ __forceinline__ void fetch_row_operands(const GemmParams &p, int m0, 
 
 // The epilogue of one wavefront's fragments on the usual path: f32 output only, n % 4 == 0, w_scale and every
 // a_scale of the tile suited to the short division (the caller checks).  Straight-line code: per output element
-// a subtraction, a conversion, two multiplications, two FMAs and a sign copy; one 16-byte store per fragment row.
+// a subtraction, a conversion, two multiplications, two FMAs and a sign copy; 16-byte stores, 128 contiguous bytes a row.
 // Fragment i of lane l holds token row rows[i], columns col0 + 16*j + 0..3.  FULL: the tile lies inside the
 // matrix, no bounds checks.  EXTRA: bias and / or residual may be present.
+// The stores are a quarter of a short-k launch (8192 x 2560 x 6912: 118 us of 153 without them), and the loads of the other
+// workgroups of the compute unit wait behind them: so they write whole 128-byte lines, non-temporal.  In 64-byte pieces 1024 x
+// 2560 x 6912 took 26.0 us (now 23.9), 2048 x 6912 x 2560 36.5 (34.8), 333 x 3328 x 8640 21.0 (19.5).
 template <int NI, int FN, bool FULL, bool EXTRA>
 __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], const int (&rs)[NI], const float (&as)[NI],
                                                      const float (&rcp)[NI], float ws, const GemmProjDev &PJ, int m,
                                                      const int (&rows)[NI], int col0)
 {
+    const int lr = threadIdx.x & 15;
+    const bool hi = lr >= 8;
+    auto scaled4 = [&](const v4i &c, int i) {
+        v4f v;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        if (!FULL && rows[i] >= m) continue;
-        const size_t o = (size_t)rows[i] * PJ.n + col0;
-        float *orow = PJ.out + o;
+        for (int r = 0; r < 4; ++r) v[r] = div_by_invariant_unchecked(f32_mul((float)(c[r] - rs[i]), ws), as[i], rcp[i]);
+        return v;
+    };
+    // Store k of fragment row i, FN of them.  Fragments 32 columns apart by pairs (j, j + 1): lanes of rows 8..15 of j change places
+    // with lanes of rows 0..7 of j + 1 (a rotation by 8 of the 16 lanes), and each of the two stores then writes eight rows of 128
+    // contiguous bytes.  Pairs begin at multiples of 32 columns; a fragment without a partner is stored as it is.
+    const bool odd = ((col0 - ((threadIdx.x >> 4) & 3) * 4) >> 4) & 1;  // uniform over the wavefront
+    auto place = [&](auto is_odd, int i, int k, int *row, int *col) {
+        constexpr int FIRST = decltype(is_odd)::value ? 1 : 0, PAIRED = (FN - FIRST) / 2 * 2;
+        const bool single = k < FIRST || k >= FIRST + PAIRED;
+        const int second = (k - FIRST) & 1;
+        *row = single ? rows[i] : rows[i] - (lr & 8) + 8 * second;
+        *col = col0 + (single ? k : k - second + (hi ? 1 : 0)) * 16;
+        return FULL || (*row < m && *col < PJ.n);  // n % 4 == 0: a fragment row is inside or outside as a whole
+    };
+    auto run = [&](auto is_odd) {
+        constexpr int FIRST = decltype(is_odd)::value ? 1 : 0, PAIRED = (FN - FIRST) / 2 * 2;
+        // The residuals of a fragment row are requested together, ahead of its arithmetic; where the registers allow it, while the
+        // row before it is finished.  (A lane reads no element that another lane writes: out may be the residual's memory.)
+        constexpr bool AHEAD = NI * FN <= 10;
+        v4f res[AHEAD ? 2 : 1][FN];
+        auto fetch = [&](int i) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            if (!FULL && col0 + j * 16 >= PJ.n) continue;  // n % 4 == 0: a fragment row is inside or outside as a whole
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[r] = div_by_invariant_unchecked(f32_mul((float)(acc[i][j][r] - rs[i]), ws), as[i], rcp[i]);
-            if (EXTRA) {
-                if (PJ.bias) {
-                    const float4 b = *reinterpret_cast<const float4 *>(PJ.bias + col0 + j * 16);
-                    v[0] = f32_add(v[0], b.x); v[1] = f32_add(v[1], b.y); v[2] = f32_add(v[2], b.z); v[3] = f32_add(v[3], b.w);
-                }
-                if (PJ.residual) {
-                    const float4 q = *reinterpret_cast<const float4 *>(PJ.residual + o + j * 16);
-                    v[0] = f32_add(v[0], q.x); v[1] = f32_add(v[1], q.y); v[2] = f32_add(v[2], q.z); v[3] = f32_add(v[3], q.w);
-                }
+            for (int k = 0; k < FN; ++k) {
+                int row, col;
+                const bool inside = place(is_odd, i, k, &row, &col);
+                res[AHEAD ? i & 1 : 0][k] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+                if (inside) res[AHEAD ? i & 1 : 0][k] = *reinterpret_cast<const v4f *>(PJ.residual + (size_t)row * PJ.n + col);
             }
-            *reinterpret_cast<float4 *>(orow + j * 16) = make_float4(v[0], v[1], v[2], v[3]);
+        };
+        if (AHEAD && EXTRA && PJ.residual) fetch(0);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if (EXTRA && PJ.residual && (AHEAD ? i + 1 < NI : true)) fetch(AHEAD ? i + 1 : i);
+            v4f v[FN];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) v[j] = scaled4(acc[i][j], i);
+#pragma unroll
+            for (int j = FIRST; j < FIRST + PAIRED; j += 2)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float a = v[j][r], b = v[j + 1][r];
+                    const int got = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, hi ? a : b), 0x128, 0xf, 0xf, true);
+                    v[j][r] = hi ? __builtin_bit_cast(float, got) : a;
+                    v[j + 1][r] = hi ? b : __builtin_bit_cast(float, got);
+                }
+#pragma unroll
+            for (int k = 0; k < FN; ++k) {
+                int row, col;
+                if (!place(is_odd, i, k, &row, &col)) continue;
+                v4f y = v[k];
+                if (EXTRA && PJ.bias) {
+                    const v4f b = *reinterpret_cast<const v4f *>(PJ.bias + col);
+                    y = (v4f){f32_add(y[0], b[0]), f32_add(y[1], b[1]), f32_add(y[2], b[2]), f32_add(y[3], b[3])};
+                }
+                if (EXTRA && PJ.residual) {
+                    const v4f q = res[AHEAD ? i & 1 : 0][k];
+                    y = (v4f){f32_add(y[0], q[0]), f32_add(y[1], q[1]), f32_add(y[2], q[2]), f32_add(y[3], q[3])};
+                }
+                __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(PJ.out + (size_t)row * PJ.n + col));
+            }
         }
-    }
+    };
+    if (odd) run(std::true_type{});
+    else run(std::false_type{});
 }
 
 // The epilogue for every other case (int32 accumulator output, n % 4 != 0, scales outside the short division's
