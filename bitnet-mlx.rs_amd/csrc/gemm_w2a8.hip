@@ -991,7 +991,10 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
 {
     if (m == 0 || nproj <= 0) return BITNET_HIP_OK;
     if (nproj > GEMM_MAX_PROJ) return BITNET_HIP_UNSUPPORTED;
-    bool dma_ok = a_sum != nullptr && m >= 96 && k % 256 == 0 && k >= 512 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
+    // One k-tile is enough for the LDS-direct kernels (two load stages: their prologue issues what there is); the eight-wavefront
+    // one wants two.  Through the register-staged kernel 1151 x 256 -> 1024 + 1024 took 37.9 us, now 10.5; 334 x 256 -> 2700
+    // with residual 24.7, now 9.6.
+    bool dma_ok = a_sum != nullptr && m >= 96 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
                   m * k < (1ull << 32);  // 32-bit lane offsets
     size_t tiles = 0, tiles128 = 0, tiles64 = 0, tiles32 = 0;  // 128 x 160 tiles; 128 x 128 tiles, or 0 if a projection is not a multiple of 128 wide
     bool all128 = true;
@@ -1036,7 +1039,7 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     // 2560 -> 6912 at 192 tokens 17.5 -> 13.6 us, at 384 tokens 20.0 -> 17.7 us.
     if (tiles < 100 && tiles32 <= 704) return launch_dma<64, 32, 4, 4>(p, stream);
     if (tiles <= 140 && tiles64 <= 768) return launch_dma<64, 64, 4, 3>(p, stream);
-    if (tiles >= 100 && tiles <= 256) return launch_ld8<128, 160>(p, stream);
+    if (tiles >= 100 && tiles <= 256 && k >= 512) return launch_ld8<128, 160>(p, stream);
     // between one and 2.5 tiles of 128 x 160 per compute unit: 128 x 128 tiles when they divide every projection and
     // fill the 768 workgroup slots almost three times (q + k + v at 3072 tokens: 33.0 us against 37.9 us with 64 x 160)
     if (tiles > 256 && tiles128 >= 640) return launch_dma<128, 128, 2, 3>(p, stream);

@@ -1563,3 +1563,14 @@ def test_forward_token_groups_bit_exact(m, n, k):
     qw, ws_ = orc.quantize_weights_absmean(w)
     ref = orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_, eps=1e-5, bias=bias, residual=res)[0]
     assert np.array_equal(host(layer.forward(dev(x), residual=dev(res))), ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(96, 33, 256), (130, 2049, 256), (700, 300, 256), (2000, 1600, 200), (1100, 2700, 256), (2500, 8200, 250)])
+def test_gemm_of_one_weight_tile_per_row_bit_exact(m, n, k):
+    """The shortest contraction of the LDS-direct kernels, two load stages, at each of their tile shapes."""
+    rng = np.random.default_rng(m + n)
+    w, x = synth_weights(rng, n, k), synth_activations(rng, m, k, outliers=True)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "short")
+    layer.update_weights(dev(w))
+    qw, ws_ = orc.quantize_weights_absmean(w)
+    assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_)[0])
