@@ -1007,6 +1007,30 @@ int bitnet_hip_bitlinear_matmul(bitnet_hip_bitlinear *layer, const int8_t *a, co
 // ---------------------------------------------------------------------------------------------------
 constexpr size_t DECODER_MAX_CHAINS = 8;
 
+namespace {
+// What the launches of a decode step depend on.
+struct StepKey {
+    size_t layer_begin = 0, layer_end = 0, m = 0;
+    const float *x_in = nullptr;
+    float *x_out = nullptr, *q_last = nullptr, *k_last = nullptr;
+    bool operator==(const StepKey &o) const
+    {
+        return layer_begin == o.layer_begin && layer_end == o.layer_end && m == o.m && x_in == o.x_in && x_out == o.x_out &&
+               q_last == o.q_last && k_last == o.k_last;
+    }
+};
+struct StepGraph {
+    StepKey key;
+    hipGraphExec_t exec = nullptr;
+    uint64_t used = 0;  // step_clock of its last replay
+};
+constexpr int STEP_GRAPHS = 4, STEP_SEEN = 8;
+// Which steps are worth a recording: blocks of up to STEP_SMALL_BLOCK weights from the second block on (896 to 1536 wide: 17 to
+// 40 us a block launch by launch, 12 to 27 us recorded); larger blocks keep the GPU busy for as long as the host needs to
+// enqueue them, and a graph starts 7 us later than a launch, so those only where that is under 2 % of the step.
+constexpr size_t STEP_MIN_BLOCKS = 2, STEP_MIN_LARGE_BLOCKS = 12, STEP_SMALL_BLOCK = 70000000;
+}  // namespace
+
 struct bitnet_hip_decoder {
     size_t layers = 0, hidden = 0, ffn = 0, q_heads = 0, kv_heads = 0, head_dim = 0, max_tokens = 0;
     float eps = 1e-5f;
@@ -1035,6 +1059,21 @@ struct bitnet_hip_decoder {
     size_t chains = 0;
     hipStream_t side[DECODER_MAX_CHAINS - 1] = {};
     hipEvent_t fork = nullptr, join[DECODER_MAX_CHAINS - 1] = {};
+    // Steps that come again with the same tensors (a generation loop: the allocator hands the loop the same buffers every
+    // time round) are recorded on their third call and replayed from then on (repeated_step_graph).  Guarded by decode_lock.
+    StepGraph steps[STEP_GRAPHS];
+    StepKey seen[STEP_SEEN] = {};
+    unsigned seen_count[STEP_SEEN] = {}, seen_next = 0;
+    uint64_t step_clock = 0, step_replays = 0, step_recordings = 0;
+    bool step_recording_failed = false;
+
+    void drop_step_graphs()
+    {
+        for (StepGraph &g : steps) {
+            if (g.exec) (void)hipGraphExecDestroy(g.exec);
+            g = StepGraph();
+        }
+    }
 
     ~bitnet_hip_decoder()
     {
@@ -1042,6 +1081,7 @@ struct bitnet_hip_decoder {
         void *bufs[] = {gamma, a8, a_scale, a_sum, qb, kb, vb, x1, gate, up, ping};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
+        drop_step_graphs();  // behind the hipFree calls, which wait for the device
         if (done) (void)hipEventDestroy(done);
         if (fork) (void)hipEventDestroy(fork);
         for (hipEvent_t e : join)
@@ -1168,37 +1208,17 @@ size_t bitnet_hip_decoder_weight_bytes(const bitnet_hip_decoder *dec)
     return total;
 }
 
-int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin, size_t layer_end,
-                                     const float *x_in, size_t m, float *x_out, float *q_last, float *k_last,
-                                     void *stream)
+}  // extern "C"
+
+// Enqueues the launches of a step on s.  The caller holds decode_lock and the read side of every projection involved.
+static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_t s)
 {
-    if (!dec || !x_in || !x_out) return fail(BITNET_HIP_NULL_POINTER, "decoder_decode: null argument");
-    if (layer_begin > layer_end || layer_end > dec->layers)
-        return fail(BITNET_HIP_INVALID_CONFIG, "decoder_decode: layer range [%zu, %zu) outside [0, %zu)", layer_begin,
-                    layer_end, dec->layers);
-    if (m == 0 || layer_begin == layer_end) return BITNET_HIP_OK;
-    if (m > dec->max_tokens) {
-        size_t e[2] = {dec->max_tokens, dec->hidden}, a[2] = {m, dec->hidden};
-        return fail_shape(e, 2, a, 2, "tokens per decode step exceed max_tokens");
-    }
-    hipStream_t s = as_stream(stream);
+    const size_t layer_begin = step.layer_begin, layer_end = step.layer_end, m = step.m;
+    const float *x_in = step.x_in;
+    float *x_out = step.x_out, *q_last = step.q_last, *k_last = step.k_last;
     const size_t H = dec->hidden, F = dec->ffn, KV = dec->kv_heads * dec->head_dim;
     const size_t group = dec->q_heads / dec->kv_heads;
     int rc = BITNET_HIP_OK;
-    // readers of every projection involved (weight updates take the write lock and wait for the GPU), and one
-    // decode at a time on this decoder's buffers
-    std::vector<std::shared_lock<std::shared_mutex>> guards;
-    guards.reserve((layer_end - layer_begin) * 7);
-    for (size_t i = layer_begin * 7; i < layer_end * 7; ++i) {
-        guards.emplace_back(dec->proj[i]->lock);
-        if (!dec->proj[i]->has_weights)
-            return fail(BITNET_HIP_NOT_INITIALIZED, "decoder_decode: a projection has no weights yet");
-    }
-    std::lock_guard<std::mutex> one_decode(dec->decode_lock);
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(s, &capturing);
-    if (dec->done_recorded && dec->done_stream != s && capturing == hipStreamCaptureStatusNone)
-        BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));  // the previous decode used these buffers on another stream
     // One chain: rows [row0, row0 + rows) through blocks layer_begin .. layer_end-1 on stream cs, in its own rows of the
     // decoder's activation buffers.
     const size_t widest = padded_k(H > F ? H : F);
@@ -1257,6 +1277,108 @@ int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin
                 rc = fail(BITNET_HIP_DEVICE_ERROR, "decoder_decode: joining a row-group chain: %s", hipGetErrorString(e));
         }
     }
+    return rc;
+}
+
+// The recorded form of a step, or null where it is to be enqueued launch by launch.  A launch costs the host 2.3 to 4.5 us and
+// a block is four to eight of them, which the GPU runs in 12 to 25 us where the model is small or the step one token: the
+// host was the slower side.  A graph costs it 13 us whatever it holds (120 launches of a 30-block step: 15 us).  Recording
+// costs about a millisecond, so only a step that has come twice before is recorded, and, once STEP_GRAPHS have been, no
+// more than one for every 64 replays: a program whose tensors never lie where they lay before does not pay for it.
+static hipGraphExec_t repeated_step_graph(bitnet_hip_decoder *dec, const StepKey &step)
+{
+    const size_t blocks = step.layer_end - step.layer_begin;
+    const size_t weights = dec->hidden * (2 * dec->hidden + 2 * dec->kv_heads * dec->head_dim + 3 * dec->ffn);  // of one block
+    if (dec->chains > 1 || dec->step_recording_failed ||
+        blocks < (weights <= STEP_SMALL_BLOCK ? STEP_MIN_BLOCKS : STEP_MIN_LARGE_BLOCKS))
+        return nullptr;
+    ++dec->step_clock;
+    StepGraph *oldest = &dec->steps[0];
+    for (StepGraph &g : dec->steps) {
+        if (g.exec && g.key == step) {
+            g.used = dec->step_clock;
+            ++dec->step_replays;
+            return g.exec;
+        }
+        if (g.used < oldest->used) oldest = &g;
+    }
+    int at = 0;
+    while (at < STEP_SEEN && !(dec->seen_count[at] && dec->seen[at] == step)) ++at;
+    if (at == STEP_SEEN) {
+        at = (int)(dec->seen_next++ % STEP_SEEN);
+        dec->seen[at] = step;
+        dec->seen_count[at] = 0;
+    }
+    if (++dec->seen_count[at] <= 2 || dec->step_recordings >= STEP_GRAPHS + dec->step_replays / 64) return nullptr;
+    hipStream_t cs = nullptr;
+    hipGraph_t recorded = nullptr;
+    hipGraphExec_t exec = nullptr;
+    // on a stream of its own: nothing runs, and what the caller's stream holds is not touched
+    bool ok = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) == hipSuccess;
+    if (ok && hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        ok = enqueue_step(dec, step, cs) == BITNET_HIP_OK;
+        ok = hipStreamEndCapture(cs, &recorded) == hipSuccess && ok;
+    } else {
+        ok = false;
+    }
+    ok = ok && hipGraphInstantiate(&exec, recorded, nullptr, nullptr, 0) == hipSuccess;
+    if (recorded) (void)hipGraphDestroy(recorded);
+    if (cs) (void)hipStreamDestroy(cs);
+    if (!ok) {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        (void)hipGetLastError();
+        dec->step_recording_failed = true;  // launch by launch from now on
+        return nullptr;
+    }
+    if (oldest->exec) {
+        // its last replay may still be running: as when a layer's weights change, an event that is rare waits for the device
+        if (hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGraphExecDestroy(exec);
+            return nullptr;
+        }
+        (void)hipGraphExecDestroy(oldest->exec);
+    }
+    ++dec->step_recordings;
+    dec->seen_count[at] = 0;
+    oldest->key = step; oldest->exec = exec; oldest->used = dec->step_clock;
+    return exec;
+}
+
+extern "C" {
+
+int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin, size_t layer_end,
+                                     const float *x_in, size_t m, float *x_out, float *q_last, float *k_last,
+                                     void *stream)
+{
+    if (!dec || !x_in || !x_out) return fail(BITNET_HIP_NULL_POINTER, "decoder_decode: null argument");
+    if (layer_begin > layer_end || layer_end > dec->layers)
+        return fail(BITNET_HIP_INVALID_CONFIG, "decoder_decode: layer range [%zu, %zu) outside [0, %zu)", layer_begin,
+                    layer_end, dec->layers);
+    if (m == 0 || layer_begin == layer_end) return BITNET_HIP_OK;
+    if (m > dec->max_tokens) {
+        size_t e[2] = {dec->max_tokens, dec->hidden}, a[2] = {m, dec->hidden};
+        return fail_shape(e, 2, a, 2, "tokens per decode step exceed max_tokens");
+    }
+    hipStream_t s = as_stream(stream);
+    // readers of every projection involved (weight updates take the write lock and wait for the GPU), and one
+    // decode at a time on this decoder's buffers
+    std::vector<std::shared_lock<std::shared_mutex>> guards;
+    guards.reserve((layer_end - layer_begin) * 7);
+    for (size_t i = layer_begin * 7; i < layer_end * 7; ++i) {
+        guards.emplace_back(dec->proj[i]->lock);
+        if (!dec->proj[i]->has_weights)
+            return fail(BITNET_HIP_NOT_INITIALIZED, "decoder_decode: a projection has no weights yet");
+    }
+    std::lock_guard<std::mutex> one_decode(dec->decode_lock);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(s, &capturing);
+    if (dec->done_recorded && dec->done_stream != s && capturing == hipStreamCaptureStatusNone)
+        BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));  // the previous decode used these buffers on another stream
+    const StepKey step = {layer_begin, layer_end, m, x_in, x_out, q_last, k_last};
+    int rc = BITNET_HIP_OK;
+    hipGraphExec_t recorded = capturing == hipStreamCaptureStatusNone ? repeated_step_graph(dec, step) : nullptr;
+    if (recorded) BITNET_HIP_TRY(hipGraphLaunch(recorded, s));
+    else rc = enqueue_step(dec, step, s);
     if (rc == BITNET_HIP_OK && capturing == hipStreamCaptureStatusNone) {
         BITNET_HIP_TRY(hipEventRecord(dec->done, s));
         dec->done_stream = s;
@@ -1455,6 +1577,31 @@ int bitnet_hip_backend_optimize_model(bitnet_hip_backend *backend, bitnet_hip_de
     return BITNET_HIP_OK;
 }
 
+static hipError_t move_rows(float *stage, const float *const *from, float *const *to, const size_t *rows, size_t begin, size_t end,
+                            size_t width, hipStream_t s)
+{
+    Pieces p = {};
+    int n = 0;
+    size_t at = 0;
+    hipError_t e = hipSuccess;
+    for (size_t t = begin; t < end && e == hipSuccess; ++t) {
+        // a piece counts its floats in 32 bits: a longer input is cut into whole rows
+        const size_t per = width < (1u << 30) ? (1u << 30) / width : 1;
+        for (size_t r = 0; r < rows[t] && e == hipSuccess; r += per) {
+            const size_t take = rows[t] - r < per ? rows[t] - r : per;
+            p.dst[n] = to ? to[t] + r * width : stage + at;
+            p.src[n] = to ? stage + at : from[t] + r * width;
+            p.count[n] = (unsigned)(take * width);
+            at += take * width;
+            if (++n == Pieces::MOST) {
+                e = launch_move_pieces(p, n, s);
+                n = 0;
+            }
+        }
+    }
+    return e == hipSuccess && n ? launch_move_pieces(p, n, s) : e;
+}
+
 int bitnet_hip_backend_execute_batch(bitnet_hip_backend *backend, const float *const *inputs, const size_t *rows,
                                      size_t count, float *const *outputs, void *stream)
 {
@@ -1488,21 +1635,11 @@ int bitnet_hip_backend_execute_batch(bitnet_hip_backend *backend, const float *c
             int rc = bitnet_hip_decoder_decode(dec, inputs[i], rows[i], outputs[i], nullptr, nullptr, stream);
             if (rc != BITNET_HIP_OK) return rc;
         } else {
-            size_t at = 0;
             staged = true;
-            for (size_t t = i; t < j; ++t) {
-                if (rows[t] == 0) continue;
-                BITNET_HIP_TRY(hipMemcpyAsync(backend->stage_in + at * H, inputs[t], sizeof(float) * rows[t] * H, hipMemcpyDeviceToDevice, s));
-                at += rows[t];
-            }
+            BITNET_HIP_TRY(move_rows(backend->stage_in, inputs, nullptr, rows, i, j, H, s));
             int rc = bitnet_hip_decoder_decode(dec, backend->stage_in, total, backend->stage_out, nullptr, nullptr, stream);
             if (rc != BITNET_HIP_OK) return rc;
-            at = 0;
-            for (size_t t = i; t < j; ++t) {
-                if (rows[t] == 0) continue;
-                BITNET_HIP_TRY(hipMemcpyAsync(outputs[t], backend->stage_out + at * H, sizeof(float) * rows[t] * H, hipMemcpyDeviceToDevice, s));
-                at += rows[t];
-            }
+            BITNET_HIP_TRY(move_rows(backend->stage_out, nullptr, outputs, rows, i, j, H, s));
         }
         i = j;
     }

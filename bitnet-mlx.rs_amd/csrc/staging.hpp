@@ -45,6 +45,15 @@ private:
 // The other way: returns with `dst` complete.  `scalar` (optional): one device float that comes along, into *scalar_host.
 // (4.4 MB into pageable memory through hipMemcpy: 250 us.)
 int download(void *dst, const void *src, size_t bytes, const float *scalar, float *scalar_host, hipStream_t stream);
+// Up to MOST separate pieces of device memory moved by one launch (a copy through the runtime costs the host 5 to 6 us each:
+// twelve requests gathered and scattered again, 130 us of a batch).
+struct Pieces {
+    static constexpr int MOST = 32;
+    float *dst[MOST];
+    const float *src[MOST];
+    unsigned count[MOST];  // floats
+};
+hipError_t launch_move_pieces(const Pieces &pieces, int n, hipStream_t stream);
 // The chunks exist while layers do: made by the first copy that wants them, given back with the last layer.
 void staging_retain();
 void staging_release();

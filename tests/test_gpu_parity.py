@@ -1565,6 +1565,54 @@ def test_forward_token_groups_bit_exact(m, n, k):
     assert np.array_equal(host(layer.forward(dev(x), residual=dev(res))), ref)
 
 
+@pytest.mark.parametrize("m", [1, 3, 20])
+def test_decoder_steps_that_repeat_match_the_oracle(m):
+    """The same tensors step after step (recorded on the third call and replayed), other tensors and row counts in between, more of
+    them than the decoder keeps recordings for, and weights that change under a recording."""
+    dims = (256, 512, 4, 2, 64)
+    rng = np.random.default_rng(m)
+    dec, ref = build_decoder(rng, 3, *dims, max_tokens=20)
+    xs = [synth_activations(rng, m, 256) for _ in range(6)]
+    ins, outs = [dev(x) for x in xs], [torch.empty((m, 256), device="cuda") for _ in xs]
+    want = [oracle_stack(ref, x, *dims)[0] for x in xs]
+    for step in range(5):
+        for i in range(6 if step < 4 else 2):
+            outs[i].fill_(float("nan"))
+            dec.decode(ins[i], out=outs[i])
+            assert np.array_equal(host(outs[i]), want[i])
+        ins[0].copy_(dev(xs[step]))  # new values in the same buffer
+        want[0] = want[step] if step else want[0]
+        xs[0] = xs[step]
+    w = synth_weights(rng, *dec.proj_shape(0))
+    dec.projection(0, 0).update_weights(dev(w))
+    dec.set_norm(1, 0, torch.full((256,), 1.25))
+    qw, s = orc.quantize_weights_absmean(w)
+    ref[0][0][0], ref[0][1][0] = orc.pack_2bit(qw), s
+    ref[1] = (ref[1][0], ref[1][1], np.full(256, 1.25, dtype=f32), ref[1][3])
+    want[1] = oracle_stack(ref, xs[1], *dims)[0]
+    side = torch.cuda.Stream()
+    for stream in (None, side, None):
+        dec.decode(ins[1], out=outs[1], stream=stream)
+        torch.cuda.synchronize()
+        assert np.array_equal(host(outs[1]), want[1])
+
+
+def test_inference_backend_moves_many_unaligned_inputs():
+    """More inputs than one launch moves, some at addresses that are no multiple of 16 bytes, rows longer than one workgroup's share."""
+    dims = (1280, 512, 20, 5, 64)
+    rng = np.random.default_rng(5)
+    dec, ref = build_decoder(rng, 1, *dims, max_tokens=64)
+    backend = bh.create_backend("hip:0")
+    backend.optimize_model(dec)
+    xs = [synth_activations(rng, 7 if i == 3 else 1 + i % 2, dims[0]) for i in range(36)]
+    ins = []
+    for i, x in enumerate(xs):
+        flat = torch.empty((x.size + 1,), device="cuda")
+        ins.append(flat[i % 2:i % 2 + x.size].view(x.shape).copy_(dev(x)))
+    for x, o in zip(xs, backend.execute_batch(ins)):
+        assert np.array_equal(host(o), oracle_stack(ref, x, *dims)[0])
+
+
 @pytest.mark.parametrize("m,n,k", [(96, 33, 256), (130, 2049, 256), (700, 300, 256), (2000, 1600, 200), (1100, 2700, 256), (2500, 8200, 250)])
 def test_gemm_of_one_weight_tile_per_row_bit_exact(m, n, k):
     """The shortest contraction of the LDS-direct kernels, two load stages, at each of their tile shapes."""
