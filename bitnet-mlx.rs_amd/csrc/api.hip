@@ -598,7 +598,7 @@ int bitnet_hip_matmul_w2a8(const uint8_t *tiled, const int8_t *a, const int32_t 
     if (reinterpret_cast<uintptr_t>(tiled) % 16)
         return fail(BITNET_HIP_INVALID_CONFIG, "matmul_w2a8: tiled weights must be 16-byte aligned");
     if (n > 0x7fffffffu || k > 0x7fffffffu) return fail(BITNET_HIP_UNSUPPORTED, "matmul_w2a8: dimension too large");
-    if (gemv_takes(m, k, row_blocks(n), a)) {
+    if (gemv_takes(m, k, row_blocks(n), a) || (!a_sum && m <= (size_t)GEMV_MAX_M)) {  // the GEMM that counts the rows' sums itself is slower
         GemvProj pj = {tiled, w_scale, bias, residual, out, acc, n};
         return launch_gemv_tiled(&pj, 1, a, a_scale, m, k, as_stream(stream));
     }

@@ -994,7 +994,7 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     // One k-tile is enough for the LDS-direct kernels (two load stages: their prologue issues what there is); the eight-wavefront
     // one wants two.  Through the register-staged kernel 1151 x 256 -> 1024 + 1024 took 37.9 us, now 10.5; 334 x 256 -> 2700
     // with residual 24.7, now 9.6.
-    bool dma_ok = a_sum != nullptr && m >= 96 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
+    bool dma_ok = a_sum != nullptr && m > 32 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
                   m * k < (1ull << 32);  // 32-bit lane offsets
     size_t tiles = 0, tiles128 = 0, tiles64 = 0, tiles32 = 0;  // 128 x 160 tiles; 128 x 128 tiles, or 0 if a projection is not a multiple of 128 wide
     bool all128 = true;

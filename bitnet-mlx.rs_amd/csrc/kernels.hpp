@@ -73,7 +73,7 @@ int launch_gemv_base3(const uint8_t *tiled, const int8_t *a, int32_t *acc, float
 // gemv_w2a8.hip
 int launch_gemv_rowmajor(const uint8_t *packed, const int8_t *a, int32_t *out, size_t n, size_t k,
                          hipStream_t stream);
-constexpr int GEMV_MAX_M = 95;      // token rows the decode-GEMV path always takes
+constexpr int GEMV_MAX_M = 95;      // token rows that the decode-GEMV path takes but for long outputs (gemm_takes_tokens)
 // More rows go to the prefill GEMM, except where the token-group GEMV (gemv_mfma_tg_kernel: k a multiple of 256 up to
 // 8192, 16-byte aligned rows) runs as a single round of workgroups: it then beats a GEMM that is too small to fill the
 // chip (6912 -> 2560 at 96 tokens: 13.6 us against 18.9 us; 2560 -> 2560 up to 192 tokens: 8.4 .. 9.8 us against
@@ -81,9 +81,19 @@ constexpr int GEMV_MAX_M = 95;      // token rows the decode-GEMV path always ta
 // against 19.1 us).  n_blocks: 16-row blocks of all projections of the launch.  The row blocks per workgroup and
 // the workgroup slots follow launch_gemv_tiled.
 constexpr int GEMV_WIDE_MAX_M = 512;
+// From 33 tokens on a token GEMV of many workgroups (four row blocks by 16 tokens each) is bound by the exchange of its partial results
+// and the GEMM is ahead, where its 64 x 32 tiles fit the chip at once or there is work for its larger ones.  In us, GEMV / GEMM,
+// quantiser included: 1536 -> 16384 at 33 / 49 / 65 tokens 9.0 / 9.5, 11.4 / 9.7, 13.7 / 11.1; 2560 -> 13824 at 33 / 49 / 95 11.0 /
+// 11.4, 14.2 / 11.5, 18.8 / 13.9; 2560 -> 24576 at 33 / 49 / 95 15.9 / 16.9, 21.1 / 17.4, 28.6 / 18.2; 8192 -> 8192 at 95 23.1 / 24.2.
+inline bool gemm_takes_tokens(size_t m, size_t k, size_t n_blocks, const void *a)
+{
+    const size_t wgs = (n_blocks + 3) / 4 * ((m + 15) / 16), tiles32 = (m + 63) / 64 * ((n_blocks + 1) / 2);
+    return m > 32 && wgs >= 800 && (tiles32 <= 704 || (wgs >= 1500 && k >= 1536)) && k % TILE_K == 0 && n_blocks * k < (1ull << 29) &&
+           (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+}
 inline bool gemv_takes(size_t m, size_t k, size_t n_blocks, const void *a)
 {
-    if (m <= (size_t)GEMV_MAX_M) return true;
+    if (m <= (size_t)GEMV_MAX_M) return !gemm_takes_tokens(m, k, n_blocks, a);
     if (m > (size_t)GEMV_WIDE_MAX_M || k % 256 != 0 || k > 8192 || (reinterpret_cast<uintptr_t>(a) & 15) != 0) return false;
     const size_t tgroups = (m + 15) / 16, slots = k <= 3072 ? 768 : 256;
     const size_t rb = n_blocks * tgroups > 2 * slots ? 4 : (n_blocks * tgroups > slots ? 2 : 1);

@@ -1622,3 +1622,14 @@ def test_gemm_of_one_weight_tile_per_row_bit_exact(m, n, k):
     layer.update_weights(dev(w))
     qw, ws_ = orc.quantize_weights_absmean(w)
     assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_)[0])
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 17100, 256), (49, 12900, 300), (65, 10300, 512), (80, 24700, 1600)])
+def test_forward_of_long_outputs_at_few_tokens_bit_exact(m, n, k):
+    """Few tokens and many outputs: the shapes on which the GEMM takes over below 96 tokens, incomplete row tiles."""
+    rng = np.random.default_rng(m)
+    x = synth_activations(rng, m, k, outliers=True)
+    pk = random_packed_ternary(rng, n, k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "long")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, pk, n, f32(0.02))[0])
