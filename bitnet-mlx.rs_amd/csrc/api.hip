@@ -139,7 +139,7 @@ struct bitnet_hip_bitlinear {
 namespace {
 
 // Row blocks of the largest launch group (up to GEMV_MAX_PROJ projections share a decode launch).
-size_t launch_group_blocks(bitnet_hip_bitlinear *const *layers, size_t count)
+size_t launch_group_blocks(const bitnet_hip_bitlinear *const *layers, size_t count)
 {
     size_t most = 0;
     for (size_t j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
@@ -148,6 +148,14 @@ size_t launch_group_blocks(bitnet_hip_bitlinear *const *layers, size_t count)
         most = sum > most ? sum : most;
     }
     return most;
+}
+
+// Whether projections of plain rows [m, in] need no scratch: the quantiser runs inside the launch.
+bool quantises_in_launch(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order)
+{
+    const size_t in = layers[0]->in_features, blocks = launch_group_blocks(layers, count);
+    return gemv_rowq_takes(x, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, sum_order, blocks, true) ||
+           gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, blocks);
 }
 
 // Runs `count` projections that share one input row block [m, k].  At decode token counts the quantiser runs
@@ -159,15 +167,27 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
                     size_t m, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,
                     int sum_order, const float *const *residual, float *const *out, int32_t *const *acc, int8_t *q,
                     size_t ldq, float *a_scale, int32_t *a_sum, bool want_quant_outputs, hipStream_t s,
-                    const GemmSplitScratch *split = nullptr)
+                    const GemmSplitScratch *split = nullptr, bool alone = true)
 {
     size_t k = layers[0]->in_features;
+    const bool short_rows = !want_quant_outputs && gemv_rowq_takes(x, ldx, m, k, input_mode, gqa_group, head_dim, gamma, sum_order,
+                                                                   launch_group_blocks(layers, count), alone);
     auto proj_of = [&](int j) {
         bitnet_hip_bitlinear *bl = layers[j];
         GemvProj pj = {bl->tiled, bl->w_scale, bl->use_bias ? bl->bias : nullptr, residual ? residual[j] : nullptr,
                        out[j], acc ? acc[j] : nullptr, bl->out_features};
         return pj;
     };
+    if (short_rows) {
+        for (int j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
+            GemvProj pjs[GEMV_MAX_PROJ];
+            const int nj = count - j0 < GEMV_MAX_PROJ ? count - j0 : GEMV_MAX_PROJ;
+            for (int j = 0; j < nj; ++j) pjs[j] = proj_of(j0 + j);
+            const int rc = launch_gemv_rowq(pjs, nj, x, m, k, input_mode, gqa_group, head_dim, gamma, eps, s);
+            if (rc != BITNET_HIP_OK) return rc;
+        }
+        return BITNET_HIP_OK;
+    }
     if (gemv_fused_supported(x, x2, ldx, m, k, input_mode, head_dim, gamma, sum_order, launch_group_blocks(layers, count))) {
         for (int j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
             GemvProj pjs[GEMV_MAX_PROJ];
@@ -813,7 +833,7 @@ size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, c
 {
     if (!layer || m == 0) return 0;
     const size_t in = layer->in_features;
-    if (gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, row_blocks(layer->out_features))) return 0;
+    if (quantises_in_launch(&layer, 1, x, m, gamma, sum_order)) return 0;
     return bitnet_hip_bitlinear_workspace_size(layer, m);
 }
 
@@ -824,7 +844,7 @@ size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *l
     for (size_t j = 0; j < count; ++j)
         if (!layers[j]) return 0;
     const size_t in = layers[0]->in_features;
-    if (gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, launch_group_blocks(layers, count))) return 0;
+    if (quantises_in_launch(layers, count, x, m, gamma, sum_order)) return 0;
     return quant_scratch_bytes(m, padded_k(in));
 }
 
@@ -857,7 +877,7 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
 
     hipStream_t s = as_stream(stream);
     const bool debug = dbg_q || dbg_a_scale || dbg_acc;
-    const bool fused = gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, row_blocks(layer->out_features));
+    const bool fused = quantises_in_launch(&layer, 1, x, m, gamma, sum_order);
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {dbg_q, dbg_a_scale, nullptr};
@@ -963,7 +983,7 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     }
     const size_t in = layers[0]->in_features;
     hipStream_t s = as_stream(stream);
-    const bool fused = gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, launch_group_blocks(layers, count));
+    const bool fused = quantises_in_launch(layers, count, x, m, gamma, sum_order);
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {nullptr, nullptr, nullptr};
@@ -1230,7 +1250,7 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
             const float *res[GEMV_MAX_PROJ] = {res0, nullptr, nullptr};
             rc = run_projections(layers, count, x, x2, ldx, rows, mode, group, dec->head_dim, gamma, dec->eps, dec->sum_order,
                                  res, outs, nullptr, dec->a8 + row0 * widest, padded_k(layers[0]->in_features), dec->a_scale + row0,
-                                 dec->a_sum + row0, false, cs);
+                                 dec->a_sum + row0, false, cs, nullptr, false);
         };
         float *qb = dec->qb + row0 * H, *kb = dec->kb + row0 * KV, *vb = dec->vb + row0 * KV, *x1 = dec->x1 + row0 * H;
         float *gate = dec->gate + row0 * F, *up = dec->up + row0 * F, *ping = dec->ping + row0 * H;

@@ -1624,6 +1624,40 @@ def test_gemm_of_one_weight_tile_per_row_bit_exact(m, n, k):
     assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_)[0])
 
 
+@pytest.mark.parametrize("m", [9, 12, 16, 17, 33, 95])
+@pytest.mark.parametrize("n,k", [(1, 4), (33, 260), (300, 1024), (1400, 768), (2200, 512), (5000, 100)])
+def test_forward_of_short_rows_in_one_launch_bit_exact(m, n, k):
+    """Rows that every workgroup quantises for itself (and their neighbours beyond its lines): one to sixteen rows in the last token
+    group, widths that are no multiple of a piece or a tile, one to four row blocks a workgroup, groups past the end; with and
+    without norm, a zero row, one too small and one too large for the short division."""
+    rng = np.random.default_rng(m + n + k)
+    w, x = synth_weights(rng, n, k), synth_activations(rng, m, k, outliers=True)
+    x[1] = 0.0
+    x[2] *= f32(2.0**-70)
+    x[3] *= f32(2.0**70)
+    g, bias, res = rng.standard_normal(k, dtype=f32), rng.standard_normal(n, dtype=f32), rng.standard_normal((m, n), dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "short rows")
+    layer.update_weights(dev(w))
+    layer.update_bias(dev(bias))
+    qw, ws_ = orc.quantize_weights_absmean(w)
+    ref = orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_, eps=1e-5, bias=bias, residual=res)[0]
+    assert np.array_equal(host(layer.forward(dev(x), residual=dev(res))), ref)
+    ref = orc.bitlinear_forward(x, orc.pack_2bit(qw), n, ws_, g=g, eps=1e-5, bias=bias)[0]
+    assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g))), ref)
+    outs = bh.forward_multi([layer] * 4, dev(x), gamma=dev(g))
+    assert all(np.array_equal(host(o), ref) for o in outs)
+
+
+@pytest.mark.parametrize("dims,m", [((2560, 256, 20, 5, 128), 8), ((192, 320, 12, 3, 16), 9), ((4352, 64, 34, 2, 128), 17), ((4096, 64, 64, 8, 64), 13)])
+def test_decoder_output_projection_reads_distinct_heads(dims, m):
+    """The attention output projection on its distinct columns: groups of one to seventeen query heads, one and two k-tiles a
+    wavefront, heads of one piece, row counts on both sides of a token group."""
+    rng = np.random.default_rng(m)
+    dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
+    x = synth_activations(rng, m, dims[0])
+    assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 17100, 256), (49, 12900, 300), (65, 10300, 512), (80, 24700, 1600)])
 def test_forward_of_long_outputs_at_few_tokens_bit_exact(m, n, k):
     """Few tokens and many outputs: the shapes on which the GEMM takes over below 96 tokens, incomplete row tiles."""
