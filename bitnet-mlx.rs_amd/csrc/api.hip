@@ -425,6 +425,29 @@ int bitnet_hip_abs_max(const float *x, size_t count, float *abs_max, void *strea
     });
 }
 
+int bitnet_hip_quantize_activations_dynamic(const float *x, size_t count, int precision, const float *average, float decay, int reference_u8,
+                                            int8_t *values, float *scale_out, float *abs_max, float *scratch, void *stream)
+{
+    if (precision != BITNET_HIP_PRECISION_ONE_FIVE_FIVE_BIT && precision != BITNET_HIP_PRECISION_EIGHT_BIT)
+        return fail(BITNET_HIP_UNSUPPORTED, "quantize_activations_dynamic: unsupported precision %d", precision);
+    if (count == 0) return fail(BITNET_HIP_INVALID_CONFIG, "quantize_activations_dynamic: an empty tensor has no scale");
+    if (!x || !values || !scale_out || !abs_max || !scratch) return fail(BITNET_HIP_NULL_POINTER, "quantize_activations_dynamic: null buffer");
+    HostParts parts;
+    int rc = parts.acquire();
+    if (rc != BITNET_HIP_OK) return rc;
+    const DynamicScale d = {average != nullptr, average ? *average : 0.0f, decay};
+    const int workgroups = count <= (size_t)DYNAMIC_SMALL ? 1 : abs_max_workgroups(count, HostParts::MOST);
+    rc = launch_dynamic_quantize(x, count, precision, d, reference_u8 != 0, values, scale_out, scratch, workgroups, parts.answers, parts.ticket,
+                                 as_stream(stream));
+    if (rc != BITNET_HIP_OK) return rc;
+    *abs_max = 0.0f;
+    return parts.wait(as_stream(stream), workgroups, [&](unsigned bits) {
+        float part;
+        memcpy(&part, &bits, sizeof part);
+        *abs_max = part > *abs_max ? part : *abs_max;
+    });
+}
+
 int bitnet_hip_quantize_activations_scaled(const float *x, size_t count, int precision, float scale, int reference_u8,
                                            int8_t *values, void *stream)
 {

@@ -36,7 +36,16 @@ int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratc
 // DynamicActivationQuantizer with the scale given from outside (activations.rs:269-294, 315-360), which also stores the
 // scale to scale_out unless that is null
 int abs_max_workgroups(size_t n, int most);
-int launch_abs_max(const float *x, size_t n, int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream);
+int launch_abs_max(const float *x, size_t n, int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream, float *parts = nullptr);
+// Both at once, the scale computed on the device from the maximum and the moving average before this step.  parts: 256 floats of
+// device scratch; answers receives one word (n <= DYNAMIC_SMALL) or one from each of `workgroups`.
+struct DynamicScale {
+    int has_average;
+    float average, decay;
+};
+constexpr int DYNAMIC_SMALL = 32768;
+int launch_dynamic_quantize(const float *x, size_t n, int precision, const DynamicScale &d, int reference_u8, int8_t *q, float *scale_out, float *parts,
+                            int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream);
 int launch_scaled_quantize(const float *x, size_t n, int precision, float scale, int reference_u8, int8_t *q, float *scale_out,
                            hipStream_t stream);
 

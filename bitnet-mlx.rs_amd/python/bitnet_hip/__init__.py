@@ -99,6 +99,7 @@ def load_library() -> C.CDLL:
         "bitnet_hip_abs_max": (i32, [vp, sz, C.POINTER(C.c_float), vp]),
         "bitnet_hip_quantize_activations_scaled": (i32, [vp, sz, i32, f32, i32, vp, vp]),
         "bitnet_hip_quantize_activations_scaled_keep": (i32, [vp, sz, i32, f32, i32, vp, vp, vp]),
+        "bitnet_hip_quantize_activations_dynamic": (i32, [vp, sz, i32, C.POINTER(C.c_float), f32, i32, vp, vp, C.POINTER(C.c_float), vp, vp]),
         "bitnet_hip_lookup_compute": (i32, [i32, vp, sz, vp, sz, vp, sz, vp]),
         "bitnet_hip_packed_size": (sz, [sz]),
         "bitnet_hip_pack_ternary_2bit": (i32, [vp, sz, vp, vp]),
@@ -495,6 +496,9 @@ def _quantize_scaled(x: torch.Tensor, precision: int, scale: float, reference_u8
     return (values.view(torch.uint8) if reference_u8 and precision == QuantizationPrecision.EightBit else values), scales
 
 
+_ACTIVATION_BITS = {QuantizationPrecision.OneFiveFiveBit: 1.58, QuantizationPrecision.EightBit: 8.0}
+
+
 class DynamicActivationQuantizer:
     """DynamicActivationQuantizer (activations.rs:203-454) over the HIP path: the tensor work (abs-max, quantisation with
     the current scale) runs on the device, the state (DynamicScaleState) on the host as in the reference.
@@ -538,8 +542,28 @@ class DynamicActivationQuantizer:
     # -- ActivationQuantizer --------------------------------------------------------------------------------------
     def quantize_dynamic(self, activations: torch.Tensor) -> QuantizedActivation:
         self.state.step_count += 1
+        done = self._quantize_step(activations)
+        if done is not None:
+            return done
         self.update_dynamic_params(activations)
         return self.quantize(activations)
+
+    def _quantize_step(self, x: torch.Tensor) -> Optional[QuantizedActivation]:
+        """Both halves of quantize_dynamic in one native call, for tensors that need no conversion; None where it does not apply."""
+        precision, state = self.config.precision, self.state
+        bits = _ACTIVATION_BITS.get(precision)
+        if bits is None or _native is None or x.dim() < 1:
+            return None
+        average = state.ema_scale
+        r = _native.quantize_dynamic(x, precision, None if average is None else float(average), self.config.ema_decay, self.reference_u8, None)
+        if r is None:
+            return None
+        values, scales, largest = r
+        scale = float(state.update(largest))
+        stats = {"elements_count": x.numel(), "scale_factor": scale, "compression_ratio": 32.0 / bits}
+        if self.reference_u8 and precision == QuantizationPrecision.EightBit:
+            values = values.view(torch.uint8)
+        return QuantizedActivation(values, scales, None, tuple(x.shape), precision, stats)
 
     def quantize_attention(self, attention_scores: torch.Tensor, sequence_length: int) -> QuantizedActivation:
         if not self.config.quantize_attention:

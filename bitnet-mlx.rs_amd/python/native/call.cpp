@@ -301,7 +301,48 @@ PyObject *quantize_scaled(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     }
 }
 
+// quantize_dynamic(x, precision, average or None, decay, reference_u8, stream): (int8 values, scale tensor [1], max |x|)
+PyObject *quantize_dynamic(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
+    c10::Device device(at::kCUDA, -1);
+    if (nargs != 6) return unusual();
+    const at::Tensor *x = plain_f32(args[0], device);
+    const long precision = PyLong_AsLong(args[1]);
+    const bool averaged = args[2] != Py_None;
+    const float average = averaged ? (float)PyFloat_AsDouble(args[2]) : 0.0f, decay = (float)PyFloat_AsDouble(args[3]);
+    const int u8 = PyObject_IsTrue(args[4]);
+    void *stream;
+    if (!x || x->numel() == 0 || PyErr_Occurred() || u8 < 0 || !stream_handle(args[5], device, &stream)) return unusual();
+    try {
+        at::Tensor values, scales, scratch;
+        {
+            at::AutoDispatchBelowADInplaceOrView below;
+            values = at::empty(x->sizes(), x->options().dtype(at::kChar));
+            scales = at::empty({1}, x->options());
+            scratch = at::empty({256}, x->options());
+        }
+        const float *xp = x->const_data_ptr<float>();
+        const size_t count = (size_t)x->numel();
+        int8_t *vp = values.data_ptr<int8_t>();
+        float *sp = scales.data_ptr<float>(), *tp = scratch.data_ptr<float>(), abs_max = 0.0f;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = bitnet_hip_quantize_activations_dynamic(xp, count, (int)precision, averaged ? &average : nullptr, decay, u8, vp, sp, &abs_max, tp, stream);
+        Py_END_ALLOW_THREADS
+        if (rc != BITNET_HIP_OK) return unusual();
+        PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales), *am = PyFloat_FromDouble(abs_max);
+        PyObject *res = v && sc && am ? PyTuple_Pack(3, v, sc, am) : nullptr;
+        Py_XDECREF(v);
+        Py_XDECREF(sc);
+        Py_XDECREF(am);
+        return res;
+    } catch (...) {
+        return unusual();
+    }
+}
+
 PyMethodDef methods[] = {
+    {"quantize_dynamic", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize_dynamic)), METH_FASTCALL, nullptr},
     {"abs_max", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(abs_max)), METH_FASTCALL, nullptr},
     {"quantize_scaled", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize_scaled)), METH_FASTCALL, nullptr},
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},

@@ -76,6 +76,10 @@ extern "C" {
     pub fn bitnet_hip_quantize_activations_scaled_keep(x: *const f32, count: usize, precision: c_int, scale: f32,
                                                        reference_u8: c_int, values: *mut i8, scale_out: *mut f32,
                                                        stream: *mut c_void) -> c_int;
+    pub fn bitnet_hip_quantize_activations_dynamic(x: *const f32, count: usize, precision: c_int, average: *const f32,
+                                                   decay: f32, reference_u8: c_int, values: *mut i8,
+                                                   scale_out: *mut f32, abs_max: *mut f32, scratch: *mut f32,
+                                                   stream: *mut c_void) -> c_int;
     pub fn bitnet_hip_lookup_compute(kind: c_int, weights: *const i8, n_weights: usize, inputs: *const f32,
                                      n_inputs: usize, output: *mut f32, n_output: usize, stream: *mut c_void) -> c_int;
     pub fn bitnet_hip_packed_size(count: usize) -> usize;

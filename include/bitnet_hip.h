@@ -167,6 +167,15 @@ int bitnet_hip_quantize_activations_scaled(const float *x, size_t count, int pre
 int bitnet_hip_quantize_activations_scaled_keep(const float *x, size_t count, int precision, float scale, int reference_u8,
                                                 int8_t *values, float *scale_out, void *stream);
 
+/* A step of DynamicActivationQuantizer::quantize_dynamic in one call (update_dynamic_params :420-433, then quantize): the maximum,
+ * the scale and the values without a wait for the host in between.  The step's own scale s = abs_max / 127 (8-bit) or
+ * abs_max (ternary) is averaged as decay * *average + (1 - decay) * s, or taken as it is where average (HOST) is NULL.
+ *   *scale_out (DEVICE): the scale used;  *abs_max (HOST): the caller's on return, the values follow in stream order;
+ *   scratch: 256 DEVICE floats.  count must not be 0. */
+int bitnet_hip_quantize_activations_dynamic(const float *x, size_t count, int precision, const float *average, float decay,
+                                            int reference_u8, int8_t *values, float *scale_out, float *abs_max,
+                                            float *scratch, void *stream);
+
 /* ---- lookup-table kernels --------------------------------------------------------------------- */
 
 #define BITNET_HIP_LOOKUP_TERNARY 0 /* weights {-1,0,+1}, anything else counts as 0 */

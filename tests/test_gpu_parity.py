@@ -1667,3 +1667,28 @@ def test_forward_of_long_outputs_at_few_tokens_bit_exact(m, n, k):
     layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "long")
     layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
     assert np.array_equal(host(layer.forward(dev(x))), orc.bitlinear_forward(x, pk, n, f32(0.02))[0])
+
+
+@pytest.mark.parametrize("precision", [bh.QuantizationPrecision.OneFiveFiveBit, bh.QuantizationPrecision.EightBit])
+@pytest.mark.parametrize("count,offset", [(1, 0), (4099, 0), (4099, 1), (32767, 0), (32768, 0), (32769, 0), (32800, 1), (700001, 0), (5000000, 0)])
+def test_dynamic_quantiser_step_at_the_edges_of_its_kernels(precision, count, offset):
+    """Tensors held by one workgroup and larger ones, addresses that are no multiple of 16 bytes, NaN and zero maxima, both 8-bit
+    forms, a step with and without an average before it: scale and values as the state and the oracle have them."""
+    rng = np.random.default_rng(count + offset)
+    for u8 in (False, True):
+        cfg = bh.ActivationQuantizationConfig(precision=precision, ema_decay=0.7)
+        quant, model = bh.DynamicActivationQuantizer(cfg, reference_u8=u8), bh.DynamicScaleState(cfg)
+        for step, mag in enumerate((2.0, 0.0, 5.0) if step_sizes_fit(count) else (2.0,)):
+            x = (rng.standard_normal(count) * mag).astype(f32)
+            if step == 2 and count > 1:
+                x[count // 2] = np.nan
+            t = torch.empty((count + offset,), device="cuda")[offset:].copy_(dev(x))
+            out = quant.quantize_dynamic(t)
+            ema = model.update(np.nanmax(np.abs(x)))
+            assert f32(out.stats["scale_factor"]) == ema == f32(host(out.scales)[0])
+            want = orc.quantize_activations_scaled(x, precision, float(ema), reference_u8=u8)
+            assert np.array_equal(host(out.values).view(np.int8), want)
+
+
+def step_sizes_fit(count):
+    return count < 1000000  # one step of the largest tensor is enough
