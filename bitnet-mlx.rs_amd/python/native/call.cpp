@@ -93,7 +93,7 @@ at::Tensor new_f32(at::IntArrayRef shape, const at::Tensor &like)
 }
 
 // forward(key, x, gamma, residual, out, eps, sum_order, stream)
-PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *forward(PyObject *const *args, Py_ssize_t nargs)
 {
     if (nargs != 8) return unusual();
     Layer l;
@@ -112,44 +112,40 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     void *stream;
     if (PyErr_Occurred() || !stream_handle(args[7], device, &stream)) return unusual();
     size_t dims[3] = {(size_t)x->size(0), (size_t)x->size(1), rank == 3 ? (size_t)x->size(2) : 0};
-    try {
-        at::Tensor made;
-        const at::Tensor *y;
-        if (args[4] == Py_None) {
-            const int64_t shape[3] = {x->size(0), rank == 3 ? x->size(1) : l.out, l.out};
-            made = new_f32(at::IntArrayRef(shape, rank), *x);
-            y = &made;
-        } else {
-            y = plain_f32(args[4], device);
-            if (!y || y->dim() != rank || y->size(rank - 1) != l.out || y->numel() != m * l.out || y->size(0) != x->size(0))
-                return unusual();
-        }
-        // scratch only where the call runs the stand-alone quantiser; from torch's allocator, in the order of the stream
-        // the tensors are used on
-        const float *xp = x->const_data_ptr<float>();
-        const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch(l.handle, xp, (size_t)m, gamma, (int)order);
-        at::Tensor ws;
-        if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
-        float *yp = y->data_ptr<float>();
-        void *wp = ws_bytes ? ws.data_ptr() : nullptr;
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = bitnet_hip_bitlinear_forward(l.handle, xp, dims, (int)rank, gamma, (float)eps, (int)order, residual, yp, wp, ws_bytes,
-                                          nullptr, nullptr, nullptr, stream);
-        Py_END_ALLOW_THREADS
-        if (rc != BITNET_HIP_OK) return unusual();
-        if (args[4] != Py_None) {
-            Py_INCREF(args[4]);
-            return args[4];
-        }
-        return THPVariable_Wrap(made);
-    } catch (...) {
-        return unusual();
+    at::Tensor made;
+    const at::Tensor *y;
+    if (args[4] == Py_None) {
+        const int64_t shape[3] = {x->size(0), rank == 3 ? x->size(1) : l.out, l.out};
+        made = new_f32(at::IntArrayRef(shape, rank), *x);
+        y = &made;
+    } else {
+        y = plain_f32(args[4], device);
+        if (!y || y->dim() != rank || y->size(rank - 1) != l.out || y->numel() != m * l.out || y->size(0) != x->size(0))
+            return unusual();
     }
+    // scratch only where the call runs the stand-alone quantiser; from torch's allocator, in the order of the stream
+    // the tensors are used on
+    const float *xp = x->const_data_ptr<float>();
+    const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch(l.handle, xp, (size_t)m, gamma, (int)order);
+    at::Tensor ws;
+    if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+    float *yp = y->data_ptr<float>();
+    void *wp = ws_bytes ? ws.data_ptr() : nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bitnet_hip_bitlinear_forward(l.handle, xp, dims, (int)rank, gamma, (float)eps, (int)order, residual, yp, wp, ws_bytes,
+                                      nullptr, nullptr, nullptr, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != BITNET_HIP_OK) return unusual();
+    if (args[4] != Py_None) {
+        Py_INCREF(args[4]);
+        return args[4];
+    }
+    return THPVariable_Wrap(made);
 }
 
 // forward_multi(layers, x, gamma, eps, sum_order, stream)
-PyObject *forward_multi(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *forward_multi(PyObject *const *args, Py_ssize_t nargs)
 {
     if (nargs != 6) return unusual();
     constexpr Py_ssize_t MOST = 16;
@@ -179,42 +175,38 @@ PyObject *forward_multi(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     const long order = PyLong_AsLong(args[4]);
     void *stream;
     if (PyErr_Occurred() || !stream_handle(args[5], device, &stream)) return unusual();
-    try {
-        at::Tensor outs[MOST];
-        float *ptrs[MOST];
-        for (Py_ssize_t j = 0; j < count; ++j) {
-            outs[j] = new_f32({m, widths[j]}, *x);
-            ptrs[j] = outs[j].data_ptr<float>();
-        }
-        const float *xp = x->const_data_ptr<float>();
-        const size_t ws_bytes = bitnet_hip_bitlinear_forward_multi_scratch(handles, (size_t)count, xp, (size_t)m, gamma, (int)order);
-        at::Tensor ws;
-        if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
-        void *wp = ws_bytes ? ws.data_ptr() : nullptr;
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = bitnet_hip_bitlinear_forward_multi(handles, (size_t)count, xp, (size_t)m, gamma, (float)eps, (int)order, ptrs, wp,
-                                                ws_bytes, stream);
-        Py_END_ALLOW_THREADS
-        if (rc != BITNET_HIP_OK) return unusual();
-        PyObject *res = PyList_New(count);
-        if (!res) return nullptr;
-        for (Py_ssize_t j = 0; j < count; ++j) {
-            PyObject *t = THPVariable_Wrap(outs[j]);
-            if (!t) {
-                Py_DECREF(res);
-                return nullptr;
-            }
-            PyList_SET_ITEM(res, j, t);
-        }
-        return res;
-    } catch (...) {
-        return unusual();
+    at::Tensor outs[MOST];
+    float *ptrs[MOST];
+    for (Py_ssize_t j = 0; j < count; ++j) {
+        outs[j] = new_f32({m, widths[j]}, *x);
+        ptrs[j] = outs[j].data_ptr<float>();
     }
+    const float *xp = x->const_data_ptr<float>();
+    const size_t ws_bytes = bitnet_hip_bitlinear_forward_multi_scratch(handles, (size_t)count, xp, (size_t)m, gamma, (int)order);
+    at::Tensor ws;
+    if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+    void *wp = ws_bytes ? ws.data_ptr() : nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bitnet_hip_bitlinear_forward_multi(handles, (size_t)count, xp, (size_t)m, gamma, (float)eps, (int)order, ptrs, wp,
+                                            ws_bytes, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != BITNET_HIP_OK) return unusual();
+    PyObject *res = PyList_New(count);
+    if (!res) return nullptr;
+    for (Py_ssize_t j = 0; j < count; ++j) {
+        PyObject *t = THPVariable_Wrap(outs[j]);
+        if (!t) {
+            Py_DECREF(res);
+            return nullptr;
+        }
+        PyList_SET_ITEM(res, j, t);
+    }
+    return res;
 }
 
 // decode(decoder, hidden, begin, end, x, out, stream)
-PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *decode(PyObject *const *args, Py_ssize_t nargs)
 {
     if (nargs != 7) return unusual();
     auto *dec = static_cast<bitnet_hip_decoder *>(PyLong_AsVoidPtr(args[0]));
@@ -225,35 +217,31 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     if (!x || x->dim() != 2 || x->size(1) != hidden) return unusual();
     void *stream;
     if (!stream_handle(args[6], device, &stream)) return unusual();
-    try {
-        at::Tensor made;
-        const at::Tensor *y;
-        if (args[5] == Py_None) {
-            made = new_f32(x->sizes(), *x);
-            y = &made;
-        } else {
-            y = plain_f32(args[5], device);
-            if (!y || y->sizes() != x->sizes()) return unusual();
-        }
-        const float *xp = x->const_data_ptr<float>();
-        float *yp = y->data_ptr<float>();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = bitnet_hip_decoder_decode_layers(dec, (size_t)begin, (size_t)end, xp, (size_t)x->size(0), yp, nullptr, nullptr, stream);
-        Py_END_ALLOW_THREADS
-        if (rc != BITNET_HIP_OK) return unusual();
-        if (args[5] != Py_None) {
-            Py_INCREF(args[5]);
-            return args[5];
-        }
-        return THPVariable_Wrap(made);
-    } catch (...) {
-        return unusual();
+    at::Tensor made;
+    const at::Tensor *y;
+    if (args[5] == Py_None) {
+        made = new_f32(x->sizes(), *x);
+        y = &made;
+    } else {
+        y = plain_f32(args[5], device);
+        if (!y || y->sizes() != x->sizes()) return unusual();
     }
+    const float *xp = x->const_data_ptr<float>();
+    float *yp = y->data_ptr<float>();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bitnet_hip_decoder_decode_layers(dec, (size_t)begin, (size_t)end, xp, (size_t)x->size(0), yp, nullptr, nullptr, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != BITNET_HIP_OK) return unusual();
+    if (args[5] != Py_None) {
+        Py_INCREF(args[5]);
+        return args[5];
+    }
+    return THPVariable_Wrap(made);
 }
 
 // abs_max(x, stream): the float, or None
-PyObject *abs_max(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *abs_max(PyObject *const *args, Py_ssize_t nargs)
 {
     c10::Device device(at::kCUDA, -1);
     if (nargs != 2) return unusual();
@@ -271,7 +259,7 @@ PyObject *abs_max(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 }
 
 // quantize_scaled(x, precision, scale, reference_u8, stream): (int8 values, scale tensor [1])
-PyObject *quantize_scaled(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *quantize_scaled(PyObject *const *args, Py_ssize_t nargs)
 {
     c10::Device device(at::kCUDA, -1);
     if (nargs != 5) return unusual();
@@ -281,28 +269,24 @@ PyObject *quantize_scaled(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     const int u8 = PyObject_IsTrue(args[3]);
     void *stream;
     if (!x || PyErr_Occurred() || u8 < 0 || !stream_handle(args[4], device, &stream)) return unusual();
-    try {
-        at::Tensor values, scales;
-        {
-            at::AutoDispatchBelowADInplaceOrView below;
-            values = at::empty(x->sizes(), x->options().dtype(at::kChar));
-            scales = at::empty({1}, x->options());
-        }
-        if (bitnet_hip_quantize_activations_scaled_keep(x->const_data_ptr<float>(), (size_t)x->numel(), (int)precision, (float)scale, u8,
-                                                        values.data_ptr<int8_t>(), scales.data_ptr<float>(), stream) != BITNET_HIP_OK)
-            return unusual();
-        PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales);
-        PyObject *pair = v && sc ? PyTuple_Pack(2, v, sc) : nullptr;
-        Py_XDECREF(v);
-        Py_XDECREF(sc);
-        return pair;
-    } catch (...) {
-        return unusual();
+    at::Tensor values, scales;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        values = at::empty(x->sizes(), x->options().dtype(at::kChar));
+        scales = at::empty({1}, x->options());
     }
+    if (bitnet_hip_quantize_activations_scaled_keep(x->const_data_ptr<float>(), (size_t)x->numel(), (int)precision, (float)scale, u8,
+                                                    values.data_ptr<int8_t>(), scales.data_ptr<float>(), stream) != BITNET_HIP_OK)
+        return unusual();
+    PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales);
+    PyObject *pair = v && sc ? PyTuple_Pack(2, v, sc) : nullptr;
+    Py_XDECREF(v);
+    Py_XDECREF(sc);
+    return pair;
 }
 
 // quantize_dynamic(x, precision, average or None, decay, reference_u8, stream): (int8 values, scale tensor [1], max |x|)
-PyObject *quantize_dynamic(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+PyObject *quantize_dynamic(PyObject *const *args, Py_ssize_t nargs)
 {
     c10::Device device(at::kCUDA, -1);
     if (nargs != 6) return unusual();
@@ -313,41 +297,55 @@ PyObject *quantize_dynamic(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     const int u8 = PyObject_IsTrue(args[4]);
     void *stream;
     if (!x || x->numel() == 0 || PyErr_Occurred() || u8 < 0 || !stream_handle(args[5], device, &stream)) return unusual();
+    at::Tensor values, scales, scratch;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        values = at::empty(x->sizes(), x->options().dtype(at::kChar));
+        scales = at::empty({1}, x->options());
+        scratch = at::empty({256}, x->options());
+    }
+    const float *xp = x->const_data_ptr<float>();
+    const size_t count = (size_t)x->numel();
+    int8_t *vp = values.data_ptr<int8_t>();
+    float *sp = scales.data_ptr<float>(), *tp = scratch.data_ptr<float>(), abs_max = 0.0f;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bitnet_hip_quantize_activations_dynamic(xp, count, (int)precision, averaged ? &average : nullptr, decay, u8, vp, sp, &abs_max, tp, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != BITNET_HIP_OK) return unusual();
+    PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales), *am = PyFloat_FromDouble(abs_max);
+    PyObject *res = v && sc && am ? PyTuple_Pack(3, v, sc, am) : nullptr;
+    Py_XDECREF(v);
+    Py_XDECREF(sc);
+    Py_XDECREF(am);
+    return res;
+}
+
+// What Python calls: a C++ exception (a tensor without storage or strides refuses the question, an allocation fails) must not pass
+// into the interpreter, where it would end the process.
+template <PyObject *(*F)(PyObject *const *, Py_ssize_t)>
+PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t nargs)
+{
     try {
-        at::Tensor values, scales, scratch;
-        {
-            at::AutoDispatchBelowADInplaceOrView below;
-            values = at::empty(x->sizes(), x->options().dtype(at::kChar));
-            scales = at::empty({1}, x->options());
-            scratch = at::empty({256}, x->options());
-        }
-        const float *xp = x->const_data_ptr<float>();
-        const size_t count = (size_t)x->numel();
-        int8_t *vp = values.data_ptr<int8_t>();
-        float *sp = scales.data_ptr<float>(), *tp = scratch.data_ptr<float>(), abs_max = 0.0f;
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = bitnet_hip_quantize_activations_dynamic(xp, count, (int)precision, averaged ? &average : nullptr, decay, u8, vp, sp, &abs_max, tp, stream);
-        Py_END_ALLOW_THREADS
-        if (rc != BITNET_HIP_OK) return unusual();
-        PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales), *am = PyFloat_FromDouble(abs_max);
-        PyObject *res = v && sc && am ? PyTuple_Pack(3, v, sc, am) : nullptr;
-        Py_XDECREF(v);
-        Py_XDECREF(sc);
-        Py_XDECREF(am);
-        return res;
+        return F(args, nargs);
     } catch (...) {
         return unusual();
     }
 }
 
+template <PyObject *(*F)(PyObject *const *, Py_ssize_t)>
+PyMethodDef method(const char *name)
+{
+    return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<F>)), METH_FASTCALL, nullptr};
+}
+
 PyMethodDef methods[] = {
-    {"quantize_dynamic", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize_dynamic)), METH_FASTCALL, nullptr},
-    {"abs_max", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(abs_max)), METH_FASTCALL, nullptr},
-    {"quantize_scaled", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize_scaled)), METH_FASTCALL, nullptr},
-    {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
-    {"forward_multi", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward_multi)), METH_FASTCALL, nullptr},
-    {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, nullptr},
+    method<quantize_dynamic>("quantize_dynamic"),
+    method<abs_max>("abs_max"),
+    method<quantize_scaled>("quantize_scaled"),
+    method<forward>("forward"),
+    method<forward_multi>("forward_multi"),
+    method<decode>("decode"),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
