@@ -195,6 +195,22 @@ def _stream(stream=None):
     return C.c_void_p(s.cuda_stream)
 
 
+def _empty(shape, dtype, device, stream=None) -> torch.Tensor:
+    """A tensor for a call on `stream` to write.  torch hands a block out, and takes it back, in the order of one stream, so on a
+    stream that is not the current one it is asked for there: a block freed by the current stream may still be in use, and
+    scratch that is dropped when the call returns must not reach other work before the call's kernels have run.  The caller may use
+    a result on the current stream too, which torch is told (record_stream)."""
+    if stream is None:
+        return torch.empty(shape, dtype=dtype, device=device)
+    current = torch.cuda.current_stream(device)
+    if stream.cuda_stream == current.cuda_stream:
+        return torch.empty(shape, dtype=dtype, device=device)
+    with torch.cuda.stream(stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(stream.cuda_stream)):
+        t = torch.empty(shape, dtype=dtype, device=device)
+    t.record_stream(current)
+    return t
+
+
 def _dev(t: torch.Tensor, dtype, name: str):
     if not t.is_cuda:
         raise BitLinearError(DEVICE_ERROR, f"{name} must live on the GPU")
@@ -302,10 +318,10 @@ def quantize_activations_i8(x: torch.Tensor, gamma: Optional[torch.Tensor] = Non
     k = src_cols * gqa_group if input_mode == INPUT_GQA_BROADCAST else src_cols
     _opt_dev(gamma, torch.float32, "gamma", k, x)
     _opt_dev(x2, torch.float32, "x2", x.numel(), x)
-    q = torch.empty((m, k), dtype=torch.int8, device=x.device)
-    a_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
-    a_sum = torch.empty((m,), dtype=torch.int32, device=x.device) if want_sum else None
-    y = torch.empty((m, k), dtype=torch.float32, device=x.device) if want_y else None
+    q = _empty((m, k), torch.int8, x.device, stream)
+    a_scale = _empty((m,), torch.float32, x.device, stream)
+    a_sum = _empty((m,), torch.int32, x.device, stream) if want_sum else None
+    y = _empty((m, k), torch.float32, x.device, stream) if want_y else None
     _check(lib.bitnet_hip_quantize_activations_i8(_ptr(x), _ptr(x2), src_cols, m, k, input_mode, gqa_group, head_dim,
                                                   _ptr(gamma), eps, sum_order, _ptr(q), _ptr(a_scale), _ptr(a_sum),
                                                   _ptr(y), _stream(stream)))
@@ -344,8 +360,8 @@ def absmax_quantize_activations(activations: torch.Tensor, precision: Optional[i
     branch loses it).  The per-token int8 quantiser of the BitLinear path is quantize_activations_i8."""
     _dev(activations, torch.float32, "activations")
     precision = QuantizationPrecision.OneFiveFiveBit if precision is None else precision
-    values = torch.empty(activations.shape, dtype=torch.int8, device=activations.device)
-    stats = torch.empty((4,), dtype=torch.float32, device=activations.device)
+    values = _empty(activations.shape, torch.int8, activations.device, stream)
+    stats = _empty((4,), torch.float32, activations.device, stream)
     _check(load_library().bitnet_hip_absmax_quantize_activations(_ptr(activations), activations.numel(), precision,
                                                                  _ptr(values), _ptr(stats), _stream(stream)))
     scale, mse, lo, hi = stats.cpu().tolist()
@@ -489,7 +505,7 @@ def _quantize_scaled(x: torch.Tensor, precision: int, scale: float, reference_u8
     if pair is None:
         lib = load_library()
         _dev(x, torch.float32, "x")
-        pair = (torch.empty(x.shape, dtype=torch.int8, device=x.device), torch.empty((1,), dtype=torch.float32, device=x.device))
+        pair = (_empty(x.shape, torch.int8, x.device, stream), _empty((1,), torch.float32, x.device, stream))
         _check(lib.bitnet_hip_quantize_activations_scaled_keep(_ptr(x), x.numel(), precision, float(scale), 1 if reference_u8 else 0,
                                                                _ptr(pair[0]), _ptr(pair[1]), _stream(stream)))
     values, scales = pair
@@ -609,7 +625,7 @@ def tiled_size(n: int, k: int) -> int:
 
 def pack_ternary_2bit(q: torch.Tensor, stream=None) -> torch.Tensor:
     _dev(q, torch.int8, "q")
-    out = torch.empty((packed_size(q.numel()),), dtype=torch.uint8, device=q.device)
+    out = _empty((packed_size(q.numel()),), torch.uint8, q.device, stream)
     _check(load_library().bitnet_hip_pack_ternary_2bit(_ptr(q), q.numel(), _ptr(out), _stream(stream)))
     return out
 
@@ -618,7 +634,7 @@ def unpack_ternary_2bit(packed: torch.Tensor, count: int, stream=None) -> torch.
     _dev(packed, torch.uint8, "packed")
     if packed.numel() < packed_size(count):
         raise BitLinearError(SHAPE_MISMATCH, "packed buffer too short", [packed_size(count)], [packed.numel()])
-    out = torch.empty((count,), dtype=torch.int8, device=packed.device)
+    out = _empty((count,), torch.int8, packed.device, stream)
     _check(load_library().bitnet_hip_unpack_ternary_2bit(_ptr(packed), count, _ptr(out), _stream(stream)))
     return out
 
@@ -629,7 +645,7 @@ def base3_packed_size(count: int) -> int:
 
 def pack_ternary_base3(q: torch.Tensor, stream=None) -> torch.Tensor:
     _dev(q, torch.int8, "q")
-    out = torch.empty((base3_packed_size(q.numel()),), dtype=torch.uint8, device=q.device)
+    out = _empty((base3_packed_size(q.numel()),), torch.uint8, q.device, stream)
     _check(load_library().bitnet_hip_pack_ternary_base3(_ptr(q), q.numel(), _ptr(out), _stream(stream)))
     return out
 
@@ -638,7 +654,7 @@ def unpack_ternary_base3(packed: torch.Tensor, count: int, stream=None) -> torch
     _dev(packed, torch.uint8, "packed")
     if packed.numel() < base3_packed_size(count):
         raise BitLinearError(SHAPE_MISMATCH, "packed buffer too short", [base3_packed_size(count)], [packed.numel()])
-    out = torch.empty((count,), dtype=torch.int8, device=packed.device)
+    out = _empty((count,), torch.int8, packed.device, stream)
     _check(load_library().bitnet_hip_unpack_ternary_base3(_ptr(packed), count, _ptr(out), _stream(stream)))
     return out
 
@@ -653,7 +669,7 @@ def retile_base3(base3: torch.Tensor, n: int, k: int, stream=None) -> torch.Tens
     _dev(base3, torch.uint8, "base3")
     if base3.numel() < base3_packed_size(n * k):
         raise BitLinearError(SHAPE_MISMATCH, "base-3 buffer too short", [base3_packed_size(n * k)], [base3.numel()])
-    out = torch.empty((base3_tiled_size(n, k),), dtype=torch.uint8, device=base3.device)
+    out = _empty((base3_tiled_size(n, k),), torch.uint8, base3.device, stream)
     _check(load_library().bitnet_hip_retile_base3(_ptr(base3), n, k, _ptr(out), _stream(stream)))
     return out
 
@@ -668,9 +684,9 @@ def gemv_base3(tiled: torch.Tensor, a: torch.Tensor, n: int, w_scale: Optional[t
         raise BitLinearError(SHAPE_MISMATCH, "base-3 tiles", [base3_tiled_size(n, k)], [tiled.numel()])
     _opt_dev(w_scale, torch.float32, "w_scale", 1, a)
     _opt_dev(a_scale, torch.float32, "a_scale", 1, a)
-    acc = torch.empty((n,), dtype=torch.int32, device=a.device) if want_acc else None
+    acc = _empty((n,), torch.int32, a.device, stream) if want_acc else None
     if out is None and w_scale is not None:
-        out = torch.empty((n,), dtype=torch.float32, device=a.device)
+        out = _empty((n,), torch.float32, a.device, stream)
     elif out is not None:
         _dev(out, torch.float32, "out")
         if out.numel() != n or w_scale is None:
@@ -685,9 +701,9 @@ def quantize_weights(w: torch.Tensor, method: int = TERNARY_ABSMEAN_ROUNDCLIP, t
     """Ternarise + pack an [n, k] f32 matrix on the GPU.  Returns (packed u8, w_scale f32[1], q i8 or None)."""
     _dev(w, torch.float32, "w")
     n, k = w.shape
-    packed = torch.empty((packed_size(n * k),), dtype=torch.uint8, device=w.device)
-    w_scale = torch.empty((1,), dtype=torch.float32, device=w.device)
-    q = torch.empty((n, k), dtype=torch.int8, device=w.device) if want_i8 else None
+    packed = _empty((packed_size(n * k),), torch.uint8, w.device, stream)
+    w_scale = _empty((1,), torch.float32, w.device, stream)
+    q = _empty((n, k), torch.int8, w.device, stream) if want_i8 else None
     _check(load_library().bitnet_hip_quantize_weights(_ptr(w), n, k, method, threshold_factor, _ptr(packed),
                                                       _ptr(w_scale), _ptr(q), _stream(stream)))
     return packed, w_scale, q
@@ -759,10 +775,10 @@ class BitNetWeightQuantizer:
         self.validate_input(weights)
         _dev(weights, torch.float32, "weights")
         n, k = weights.shape[0], weights.numel() // weights.shape[0]
-        packed = torch.empty((packed_size(n * k),), dtype=torch.uint8, device=weights.device)
-        w_scale = torch.empty((1,), dtype=torch.float32, device=weights.device)
-        q = torch.empty(weights.shape, dtype=torch.int8, device=weights.device)
-        stats = torch.empty((12,), dtype=torch.float32, device=weights.device)
+        packed = _empty((packed_size(n * k),), torch.uint8, weights.device, stream)
+        w_scale = _empty((1,), torch.float32, weights.device, stream)
+        q = _empty(weights.shape, torch.int8, weights.device, stream)
+        stats = _empty((12,), torch.float32, weights.device, stream)
         c = self.config
         _check(load_library().bitnet_hip_quantize_weights_reference(
             _ptr(weights), n, k, c.ternary_method, int(c.normalize_weights), c.outlier_threshold,
@@ -783,14 +799,14 @@ def retile_weights(packed: torch.Tensor, n: int, k: int, layout: int = LAYOUT_OU
     _dev(packed, torch.uint8, "packed")
     if packed.numel() < packed_size(n * k):
         raise BitLinearError(SHAPE_MISMATCH, "packed buffer too short", [packed_size(n * k)], [packed.numel()])
-    tiled = torch.empty((tiled_size(n, k),), dtype=torch.uint8, device=packed.device)
+    tiled = _empty((tiled_size(n, k),), torch.uint8, packed.device, stream)
     _check(load_library().bitnet_hip_retile_weights(_ptr(packed), n, k, layout, _ptr(tiled), _stream(stream)))
     return tiled
 
 
 def untile_weights(tiled: torch.Tensor, n: int, k: int, stream=None) -> torch.Tensor:
     _dev(tiled, torch.uint8, "tiled")
-    packed = torch.empty((packed_size(n * k),), dtype=torch.uint8, device=tiled.device)
+    packed = _empty((packed_size(n * k),), torch.uint8, tiled.device, stream)
     _check(load_library().bitnet_hip_untile_weights(_ptr(tiled), n, k, _ptr(packed), _stream(stream)))
     return packed
 
@@ -812,8 +828,8 @@ def matmul_w2a8(tiled: torch.Tensor, a: torch.Tensor, n: int, w_scale: Optional[
     _opt_dev(a_sum, torch.int32, "a_sum", m, a)
     _opt_dev(bias, torch.float32, "bias", n, a)
     _opt_dev(residual, torch.float32, "residual", m * n, a)
-    acc = torch.empty((m, n), dtype=torch.int32, device=a.device) if want_acc else None
-    out = torch.empty((m, n), dtype=torch.float32, device=a.device) if want_out else None
+    acc = _empty((m, n), torch.int32, a.device, stream) if want_acc else None
+    out = _empty((m, n), torch.float32, a.device, stream) if want_out else None
     _check(load_library().bitnet_hip_matmul_w2a8(_ptr(tiled), _ptr(a), _ptr(a_sum), m, n, k, _ptr(acc), _ptr(w_scale), _ptr(a_scale),
                                                  _ptr(bias), _ptr(residual), _ptr(out), _stream(stream)))
     return acc, out
@@ -1001,16 +1017,16 @@ class BitLinear:
         for d in x.shape[:-1]:
             m *= d
         if out is None:
-            out = torch.empty(out_shape, dtype=torch.float32, device=x.device)
+            out = _empty(out_shape, torch.float32, x.device, stream)
         else:
             _dev(out, torch.float32, "out")
             if tuple(out.shape) != tuple(out_shape) or not out.is_contiguous():
                 raise BitLinearError(SHAPE_MISMATCH, "out", list(out_shape), list(out.shape))
         q = a_scale = acc = None
         if debug and x.dim() in (2, 3) and x.shape[-1] == self.config.in_features:
-            q = torch.empty((m, self.config.in_features), dtype=torch.int8, device=x.device)
-            a_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
-            acc = torch.empty((m, nout), dtype=torch.int32, device=x.device)
+            q = _empty((m, self.config.in_features), torch.int8, x.device, stream)
+            a_scale = _empty((m,), torch.float32, x.device, stream)
+            acc = _empty((m, nout), torch.int32, x.device, stream)
         # scratch for the quantised activations comes from torch's caching allocator (the library would otherwise
         # allocate stream-ordered memory itself on every call)
         ws_bytes = lib.bitnet_hip_bitlinear_workspace_size(self._h, m) if m > 0 else 0
@@ -1018,7 +1034,7 @@ class BitLinear:
             _dev(workspace, torch.uint8, "workspace")
             ws, ws_bytes = workspace, workspace.numel()  # the library checks the size
         else:
-            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device) if ws_bytes else None
+            ws = _empty((ws_bytes,), torch.uint8, x.device, stream) if ws_bytes else None
         _check(lib.bitnet_hip_bitlinear_forward(self._h, _ptr(x), dims, x.dim(), _ptr(gamma), self.config.rms_norm_eps,
                                                 self.config.sum_order, _ptr(residual), _ptr(out), _ptr(ws), ws_bytes,
                                                 _ptr(q), _ptr(a_scale), _ptr(acc), _stream(stream)))
@@ -1060,10 +1076,10 @@ class BitLinear:
         if a_scale is None:
             raise BitLinearError(NULL_POINTER, "a_scale is required")
         if out is None:
-            out = torch.empty((m, self.config.out_features), dtype=torch.float32, device=a.device)
+            out = _empty((m, self.config.out_features), torch.float32, a.device, stream)
         else:
             _opt_dev(out, torch.float32, "out", m * self.config.out_features, a)
-        acc = torch.empty((m, self.config.out_features), dtype=torch.int32, device=a.device) if want_acc else None
+        acc = _empty((m, self.config.out_features), torch.int32, a.device, stream) if want_acc else None
         _check(load_library().bitnet_hip_bitlinear_matmul(self._h, _ptr(a), _ptr(a_sum), m, _ptr(a_scale), _ptr(residual), _ptr(acc),
                                                           _ptr(out), _stream(stream)))
         return (out, acc) if want_acc else out
@@ -1114,7 +1130,7 @@ def forward_multi(layers: Sequence["BitLinear"], x: torch.Tensor, gamma: Optiona
     if x.shape[1] != layers[0].config.in_features:
         raise BitLinearError(SHAPE_MISMATCH, "last input dimension", [m, layers[0].config.in_features], list(x.shape))
     _opt_dev(gamma, torch.float32, "gamma", layers[0].config.in_features, x)
-    outs = [torch.empty((m, l.config.out_features), dtype=torch.float32, device=x.device) for l in layers]
+    outs = [_empty((m, l.config.out_features), torch.float32, x.device, stream) for l in layers]
     hs = (C.c_void_p * len(layers))(*[l._h for l in layers])
     os_ = (C.c_void_p * len(layers))(*[o.data_ptr() for o in outs])
     cfg = layers[0].config
@@ -1185,13 +1201,13 @@ class DecoderProjections:
         if len(lo_hi) != 2 or not (0 <= lo_hi[0] <= lo_hi[1] <= self.layers):
             raise BitLinearError(INVALID_CONFIG, f"layer range {lo_hi} outside [0, {self.layers}]")
         if out is None:
-            out = torch.empty_like(x)
+            out = _empty(x.shape, x.dtype, x.device, stream)
         else:
             _dev(out, torch.float32, "out")
             if tuple(out.shape) != tuple(x.shape) or out.device != x.device:
                 raise BitLinearError(SHAPE_MISMATCH, "decode output", list(x.shape), list(out.shape))
-        q = torch.empty((m, self.hidden), dtype=torch.float32, device=x.device) if want_qk else None
-        k = torch.empty((m, self.kv_dim), dtype=torch.float32, device=x.device) if want_qk else None
+        q = _empty((m, self.hidden), torch.float32, x.device, stream) if want_qk else None
+        k = _empty((m, self.kv_dim), torch.float32, x.device, stream) if want_qk else None
         lo, hi = (0, self.layers) if layers is None else layers
         _check(load_library().bitnet_hip_decoder_decode_layers(self._h, lo, hi, _ptr(x), m, _ptr(out), _ptr(q), _ptr(k),
                                                                _stream(stream)))
@@ -1279,7 +1295,7 @@ class HipInferenceBackend:
             if t2.dim() != 2 or t2.shape[1] != hidden:
                 raise BitLinearError(SHAPE_MISMATCH, f"input {i}", [t2.shape[0] if t2.dim() else 1, hidden], list(t.shape))
             mats.append(t2)
-        outs = [torch.empty_like(t) for t in mats]
+        outs = [_empty(t.shape, t.dtype, t.device, stream) for t in mats]
         n = len(mats)
         ins = (C.c_void_p * n)(*[t.data_ptr() for t in mats])
         rows = (C.c_size_t * n)(*[t.shape[0] for t in mats])

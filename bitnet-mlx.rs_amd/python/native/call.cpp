@@ -14,7 +14,10 @@
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
+#include <torch/csrc/Stream.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <optional>
 
 #include "../../../include/bitnet_hip.h"
 
@@ -63,7 +66,12 @@ bool optional_f32(PyObject *obj, int64_t count, c10::Device &device, const float
     return true;
 }
 
-bool stream_handle(PyObject *obj, const c10::Device &device, void **stream)
+// The stream a call is made on.  `other` is set where the caller names one that is not the current stream.
+struct CallStream {
+    void *handle = nullptr;
+    std::optional<c10::Stream> other;
+};
+bool call_stream(PyObject *obj, const c10::Device &device, CallStream &s)
 {
     PyObject *v;
     if (obj == Py_None) {
@@ -72,10 +80,16 @@ bool stream_handle(PyObject *obj, const c10::Device &device, void **stream)
         v = PyObject_CallOneArg(raw_stream_of, index);
         Py_DECREF(index);
     } else {
+        if (!THPStream_Check(obj)) return false;
+        const THPStream *given = reinterpret_cast<const THPStream *>(obj);
+        const c10::Stream stream = c10::Stream::unpack3(given->stream_id, static_cast<c10::DeviceIndex>(given->device_index),
+                                                        static_cast<c10::DeviceType>(given->device_type));
+        if (stream.device() != device) return false;
+        if (c10::impl::getDeviceGuardImpl(at::kCUDA)->getStream(device) != stream) s.other = stream;
         v = PyObject_GetAttr(obj, name_cuda_stream);
     }
     if (!v) return false;
-    *stream = PyLong_AsVoidPtr(v);
+    s.handle = PyLong_AsVoidPtr(v);
     Py_DECREF(v);
     return !PyErr_Occurred();
 }
@@ -86,10 +100,28 @@ PyObject *unusual()
     Py_RETURN_NONE;
 }
 
-at::Tensor new_f32(at::IntArrayRef shape, const at::Tensor &like)
+// Memory that the call's kernels use.  The allocator hands a block out, and takes it back, in the order of one stream, so the
+// block is asked for on the stream the call runs on: what is freed there before its kernels have run (scratch, a result the
+// caller drops) goes to later work of that stream only.  The caller may use a result on the current stream as well and drop it
+// there, which the allocator is told.
+at::Tensor new_on(const CallStream &s, at::IntArrayRef shape, const at::TensorOptions &options)
 {
     at::AutoDispatchBelowADInplaceOrView below;
-    return at::empty(shape, like.options());
+    if (!s.other) return at::empty(shape, options);
+    const c10::impl::DeviceGuardImplInterface *impl = c10::impl::getDeviceGuardImpl(at::kCUDA);
+    const c10::Stream current = impl->exchangeStream(*s.other);
+    struct Back {
+        const c10::impl::DeviceGuardImplInterface *impl;
+        c10::Stream current;
+        ~Back() { impl->exchangeStream(current); }
+    };
+    at::Tensor t;
+    {
+        const Back back{impl, current};
+        t = at::empty(shape, options);
+    }
+    impl->recordDataPtrOnStream(t.storage().data_ptr(), current);
+    return t;
 }
 
 // forward(key, x, gamma, residual, out, eps, sum_order, stream)
@@ -109,32 +141,31 @@ PyObject *forward(PyObject *const *args, Py_ssize_t nargs)
         return unusual();
     const double eps = PyFloat_AsDouble(args[5]);
     const long order = PyLong_AsLong(args[6]);
-    void *stream;
-    if (PyErr_Occurred() || !stream_handle(args[7], device, &stream)) return unusual();
+    CallStream stream;
+    if (PyErr_Occurred() || !call_stream(args[7], device, stream)) return unusual();
     size_t dims[3] = {(size_t)x->size(0), (size_t)x->size(1), rank == 3 ? (size_t)x->size(2) : 0};
     at::Tensor made;
     const at::Tensor *y;
     if (args[4] == Py_None) {
         const int64_t shape[3] = {x->size(0), rank == 3 ? x->size(1) : l.out, l.out};
-        made = new_f32(at::IntArrayRef(shape, rank), *x);
+        made = new_on(stream, at::IntArrayRef(shape, rank), x->options());
         y = &made;
     } else {
         y = plain_f32(args[4], device);
         if (!y || y->dim() != rank || y->size(rank - 1) != l.out || y->numel() != m * l.out || y->size(0) != x->size(0))
             return unusual();
     }
-    // scratch only where the call runs the stand-alone quantiser; from torch's allocator, in the order of the stream
-    // the tensors are used on
+    // scratch only where the call runs the stand-alone quantiser
     const float *xp = x->const_data_ptr<float>();
     const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch(l.handle, xp, (size_t)m, gamma, (int)order);
     at::Tensor ws;
-    if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+    if (ws_bytes) ws = new_on(stream, {(int64_t)((ws_bytes + 3) / 4)}, x->options());
     float *yp = y->data_ptr<float>();
     void *wp = ws_bytes ? ws.data_ptr() : nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = bitnet_hip_bitlinear_forward(l.handle, xp, dims, (int)rank, gamma, (float)eps, (int)order, residual, yp, wp, ws_bytes,
-                                      nullptr, nullptr, nullptr, stream);
+                                      nullptr, nullptr, nullptr, stream.handle);
     Py_END_ALLOW_THREADS
     if (rc != BITNET_HIP_OK) return unusual();
     if (args[4] != Py_None) {
@@ -173,23 +204,23 @@ PyObject *forward_multi(PyObject *const *args, Py_ssize_t nargs)
     if (m == 0 || !optional_f32(args[2], k, device, &gamma)) return unusual();
     const double eps = PyFloat_AsDouble(args[3]);
     const long order = PyLong_AsLong(args[4]);
-    void *stream;
-    if (PyErr_Occurred() || !stream_handle(args[5], device, &stream)) return unusual();
+    CallStream stream;
+    if (PyErr_Occurred() || !call_stream(args[5], device, stream)) return unusual();
     at::Tensor outs[MOST];
     float *ptrs[MOST];
     for (Py_ssize_t j = 0; j < count; ++j) {
-        outs[j] = new_f32({m, widths[j]}, *x);
+        outs[j] = new_on(stream, {m, widths[j]}, x->options());
         ptrs[j] = outs[j].data_ptr<float>();
     }
     const float *xp = x->const_data_ptr<float>();
     const size_t ws_bytes = bitnet_hip_bitlinear_forward_multi_scratch(handles, (size_t)count, xp, (size_t)m, gamma, (int)order);
     at::Tensor ws;
-    if (ws_bytes) ws = new_f32({(int64_t)((ws_bytes + 3) / 4)}, *x);
+    if (ws_bytes) ws = new_on(stream, {(int64_t)((ws_bytes + 3) / 4)}, x->options());
     void *wp = ws_bytes ? ws.data_ptr() : nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = bitnet_hip_bitlinear_forward_multi(handles, (size_t)count, xp, (size_t)m, gamma, (float)eps, (int)order, ptrs, wp,
-                                            ws_bytes, stream);
+                                            ws_bytes, stream.handle);
     Py_END_ALLOW_THREADS
     if (rc != BITNET_HIP_OK) return unusual();
     PyObject *res = PyList_New(count);
@@ -215,12 +246,12 @@ PyObject *decode(PyObject *const *args, Py_ssize_t nargs)
     if (PyErr_Occurred() || !dec || begin < 0 || end < begin) return unusual();
     const at::Tensor *x = plain_f32(args[4], device);
     if (!x || x->dim() != 2 || x->size(1) != hidden) return unusual();
-    void *stream;
-    if (!stream_handle(args[6], device, &stream)) return unusual();
+    CallStream stream;
+    if (!call_stream(args[6], device, stream)) return unusual();
     at::Tensor made;
     const at::Tensor *y;
     if (args[5] == Py_None) {
-        made = new_f32(x->sizes(), *x);
+        made = new_on(stream, x->sizes(), x->options());
         y = &made;
     } else {
         y = plain_f32(args[5], device);
@@ -230,7 +261,7 @@ PyObject *decode(PyObject *const *args, Py_ssize_t nargs)
     float *yp = y->data_ptr<float>();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = bitnet_hip_decoder_decode_layers(dec, (size_t)begin, (size_t)end, xp, (size_t)x->size(0), yp, nullptr, nullptr, stream);
+    rc = bitnet_hip_decoder_decode_layers(dec, (size_t)begin, (size_t)end, xp, (size_t)x->size(0), yp, nullptr, nullptr, stream.handle);
     Py_END_ALLOW_THREADS
     if (rc != BITNET_HIP_OK) return unusual();
     if (args[5] != Py_None) {
@@ -246,14 +277,14 @@ PyObject *abs_max(PyObject *const *args, Py_ssize_t nargs)
     c10::Device device(at::kCUDA, -1);
     if (nargs != 2) return unusual();
     const at::Tensor *x = plain_f32(args[0], device);
-    void *stream;
-    if (!x || !stream_handle(args[1], device, &stream)) return unusual();
+    CallStream stream;
+    if (!x || !call_stream(args[1], device, stream)) return unusual();
     const float *xp = x->const_data_ptr<float>();
     const size_t count = (size_t)x->numel();
     float v = 0.0f;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = bitnet_hip_abs_max(xp, count, &v, stream);
+    rc = bitnet_hip_abs_max(xp, count, &v, stream.handle);
     Py_END_ALLOW_THREADS
     return rc == BITNET_HIP_OK ? PyFloat_FromDouble(v) : unusual();
 }
@@ -267,16 +298,11 @@ PyObject *quantize_scaled(PyObject *const *args, Py_ssize_t nargs)
     const long precision = PyLong_AsLong(args[1]);
     const double scale = PyFloat_AsDouble(args[2]);
     const int u8 = PyObject_IsTrue(args[3]);
-    void *stream;
-    if (!x || PyErr_Occurred() || u8 < 0 || !stream_handle(args[4], device, &stream)) return unusual();
-    at::Tensor values, scales;
-    {
-        at::AutoDispatchBelowADInplaceOrView below;
-        values = at::empty(x->sizes(), x->options().dtype(at::kChar));
-        scales = at::empty({1}, x->options());
-    }
+    CallStream stream;
+    if (!x || PyErr_Occurred() || u8 < 0 || !call_stream(args[4], device, stream)) return unusual();
+    const at::Tensor values = new_on(stream, x->sizes(), x->options().dtype(at::kChar)), scales = new_on(stream, {1}, x->options());
     if (bitnet_hip_quantize_activations_scaled_keep(x->const_data_ptr<float>(), (size_t)x->numel(), (int)precision, (float)scale, u8,
-                                                    values.data_ptr<int8_t>(), scales.data_ptr<float>(), stream) != BITNET_HIP_OK)
+                                                    values.data_ptr<int8_t>(), scales.data_ptr<float>(), stream.handle) != BITNET_HIP_OK)
         return unusual();
     PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales);
     PyObject *pair = v && sc ? PyTuple_Pack(2, v, sc) : nullptr;
@@ -295,22 +321,17 @@ PyObject *quantize_dynamic(PyObject *const *args, Py_ssize_t nargs)
     const bool averaged = args[2] != Py_None;
     const float average = averaged ? (float)PyFloat_AsDouble(args[2]) : 0.0f, decay = (float)PyFloat_AsDouble(args[3]);
     const int u8 = PyObject_IsTrue(args[4]);
-    void *stream;
-    if (!x || x->numel() == 0 || PyErr_Occurred() || u8 < 0 || !stream_handle(args[5], device, &stream)) return unusual();
-    at::Tensor values, scales, scratch;
-    {
-        at::AutoDispatchBelowADInplaceOrView below;
-        values = at::empty(x->sizes(), x->options().dtype(at::kChar));
-        scales = at::empty({1}, x->options());
-        scratch = at::empty({256}, x->options());
-    }
+    CallStream stream;
+    if (!x || x->numel() == 0 || PyErr_Occurred() || u8 < 0 || !call_stream(args[5], device, stream)) return unusual();
+    const at::Tensor values = new_on(stream, x->sizes(), x->options().dtype(at::kChar)), scales = new_on(stream, {1}, x->options()),
+                     scratch = new_on(stream, {256}, x->options());
     const float *xp = x->const_data_ptr<float>();
     const size_t count = (size_t)x->numel();
     int8_t *vp = values.data_ptr<int8_t>();
     float *sp = scales.data_ptr<float>(), *tp = scratch.data_ptr<float>(), abs_max = 0.0f;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = bitnet_hip_quantize_activations_dynamic(xp, count, (int)precision, averaged ? &average : nullptr, decay, u8, vp, sp, &abs_max, tp, stream);
+    rc = bitnet_hip_quantize_activations_dynamic(xp, count, (int)precision, averaged ? &average : nullptr, decay, u8, vp, sp, &abs_max, tp, stream.handle);
     Py_END_ALLOW_THREADS
     if (rc != BITNET_HIP_OK) return unusual();
     PyObject *v = THPVariable_Wrap(values), *sc = THPVariable_Wrap(scales), *am = PyFloat_FromDouble(abs_max);
