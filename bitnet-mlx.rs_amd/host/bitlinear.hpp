@@ -379,7 +379,9 @@ inline Result<QuantizedActivation> absmax_quantize_activations(const DeviceTenso
     int rc = bitnet_hip_absmax_quantize_activations(activations.data(), n, static_cast<int>(q.precision), v, st, stream);
     if (rc != BITNET_HIP_OK) return last_error(rc);
     float h[4];
-    (void)hipMemcpy(h, st, sizeof h, hipMemcpyDeviceToHost);
+    // hipMemcpy waits for the null stream, not for a stream created without it
+    if (hipStreamSynchronize(stream) != hipSuccess || hipMemcpy(h, st, sizeof h, hipMemcpyDeviceToHost) != hipSuccess)
+        return BitLinearError{BitLinearError::DeviceError, "reading the quantiser's figures failed", {}, {}};
     q.scales = h[0];
     q.stats = {n, h[1], 32.0f / q.effective_bit_width(), h[2], h[3], h[0]};
     return q;
@@ -540,16 +542,19 @@ public:
                                                        config_.normalize_weights, config_.outlier_threshold,
                                                        config_.custom_threshold_factor.value_or(0.0f), packed, scale, q, nullptr, stream);
         QuantizedWeight out;
+        hipError_t e = hipSuccess;
         if (rc == BITNET_HIP_OK) {
             out.values.resize(n);
             out.packed.resize((n + 3) / 4);
             out.original_shape = weights.dims();
-            (void)hipMemcpy(out.values.data(), q, n, hipMemcpyDeviceToHost);
-            (void)hipMemcpy(out.packed.data(), packed, out.packed.size(), hipMemcpyDeviceToHost);
-            (void)hipMemcpy(&out.scales, scale, sizeof(float), hipMemcpyDeviceToHost);
+            e = hipStreamSynchronize(stream);  // hipMemcpy waits for the null stream, not for a stream created without it
+            if (e == hipSuccess) e = hipMemcpy(out.values.data(), q, n, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(out.packed.data(), packed, out.packed.size(), hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(&out.scales, scale, sizeof(float), hipMemcpyDeviceToHost);
         }
         (void)hipFree(packed); (void)hipFree(q); (void)hipFree(scale);
         if (rc != BITNET_HIP_OK) return last_error(rc);
+        if (e != hipSuccess) return BitLinearError{BitLinearError::DeviceError, "reading the quantised weights failed", {}, {}};
         return out;
     }
 

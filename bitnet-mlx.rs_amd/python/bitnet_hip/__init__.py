@@ -211,6 +211,13 @@ def _empty(shape, dtype, device, stream=None) -> torch.Tensor:
     return t
 
 
+def _finish(stream, device):
+    """Waits for a call on a stream that is not the current one.  A quantiser's figures are read on the current stream, which is not
+    behind that one, and what the weight quantisers return is complete for any stream."""
+    if stream is not None and stream.cuda_stream != torch.cuda.current_stream(device).cuda_stream:
+        stream.synchronize()
+
+
 def _dev(t: torch.Tensor, dtype, name: str):
     if not t.is_cuda:
         raise BitLinearError(DEVICE_ERROR, f"{name} must live on the GPU")
@@ -364,6 +371,7 @@ def absmax_quantize_activations(activations: torch.Tensor, precision: Optional[i
     stats = _empty((4,), torch.float32, activations.device, stream)
     _check(load_library().bitnet_hip_absmax_quantize_activations(_ptr(activations), activations.numel(), precision,
                                                                  _ptr(values), _ptr(stats), _stream(stream)))
+    _finish(stream, activations.device)
     scale, mse, lo, hi = stats.cpu().tolist()
     bits = 1.58 if precision == QuantizationPrecision.OneFiveFiveBit else 8.0
     info = {"elements_count": activations.numel(), "quantization_error": mse, "compression_ratio": 32.0 / bits,
@@ -706,6 +714,7 @@ def quantize_weights(w: torch.Tensor, method: int = TERNARY_ABSMEAN_ROUNDCLIP, t
     q = _empty((n, k), torch.int8, w.device, stream) if want_i8 else None
     _check(load_library().bitnet_hip_quantize_weights(_ptr(w), n, k, method, threshold_factor, _ptr(packed),
                                                       _ptr(w_scale), _ptr(q), _stream(stream)))
+    _finish(stream, w.device)
     return packed, w_scale, q
 
 
@@ -783,6 +792,7 @@ class BitNetWeightQuantizer:
         _check(load_library().bitnet_hip_quantize_weights_reference(
             _ptr(weights), n, k, c.ternary_method, int(c.normalize_weights), c.outlier_threshold,
             c.custom_threshold_factor or 0.0, _ptr(packed), _ptr(w_scale), _ptr(q), _ptr(stats), _stream(stream)))
+        _finish(stream, weights.device)
         return QuantizedWeight(q, w_scale, tuple(weights.shape), packed, dict(zip(WQ_STATS, stats.cpu().tolist())))
 
     def dequantize(self, quantized: QuantizedWeight) -> torch.Tensor:

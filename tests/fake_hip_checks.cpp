@@ -1,0 +1,166 @@
+// Host-side checks of the library and of its C++ mirror against a stand-in for the HIP runtime: no GPU, no kernel runs.  The
+// functions below take the place of the runtime's (the executable's symbols come first), keep device memory on the heap, write down
+// what is called in which order, and can be told to fail.  Each check is named on the command line.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../bitnet-mlx.rs_amd/host/bitlinear.hpp"
+
+namespace fake {
+struct Call {
+    std::string name;
+    hipStream_t stream;
+};
+std::vector<Call> calls;
+hipError_t host_malloc_answer = hipSuccess, launch_answer = hipSuccess;
+int copies_until_failure = -1;  // a copy that fails has moved half of its bytes
+hipStream_t capturing = nullptr;
+hipStreamCaptureMode thread_mode = hipStreamCaptureModeGlobal;
+uintptr_t next_handle = 1;
+
+hipError_t note(const char *name, hipStream_t stream = nullptr, hipError_t answer = hipSuccess)
+{
+    calls.push_back({name, stream});
+    return answer;
+}
+size_t count(const std::string &name)
+{
+    size_t n = 0;
+    for (const Call &c : calls) n += c.name == name;
+    return n;
+}
+// the position of the last call of this name on this stream, or -1
+long last(const std::string &name, hipStream_t stream)
+{
+    for (long i = (long)calls.size() - 1; i >= 0; --i)
+        if (calls[i].name == name && calls[i].stream == stream) return i;
+    return -1;
+}
+hipError_t copy(void *dst, const void *src, size_t bytes)
+{
+    if (copies_until_failure == 0) {
+        memcpy(dst, src, bytes / 2);
+        return hipErrorInvalidValue;
+    }
+    if (copies_until_failure > 0) --copies_until_failure;
+    memcpy(dst, src, bytes);
+    return hipSuccess;
+}
+template <class T>
+hipError_t make(T *out)
+{
+    *out = reinterpret_cast<T>(next_handle++ << 4);
+    return hipSuccess;
+}
+}  // namespace fake
+
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "as told"; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+
+hipError_t hipMalloc(void **p, size_t n) { *p = calloc(1, n); return hipSuccess; }
+hipError_t hipFree(void *p) { free(p); return fake::note("hipFree"); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    *p = fake::host_malloc_answer == hipSuccess ? aligned_alloc(256, (n + 255) / 256 * 256) : nullptr;
+    return fake::note("hipHostMalloc", nullptr, fake::host_malloc_answer);
+}
+hipError_t hipHostFree(void *p) { free(p); return fake::note("hipHostFree"); }
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipMemPoolCreate(hipMemPool_t *p, const hipMemPoolProps *) { return fake::make(p); }
+hipError_t hipMemPoolSetAttribute(hipMemPool_t, hipMemPoolAttr, void *) { return hipSuccess; }
+hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t, hipStream_t) { return hipMalloc(p, n); }
+hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
+hipError_t hipFreeAsync(void *p, hipStream_t) { free(p); return hipSuccess; }
+
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { (void)fake::note("hipMemcpy"); return fake::copy(d, s, n); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st)
+{
+    (void)fake::note("hipMemcpyAsync", st);
+    return fake::copy(d, s, n);
+}
+hipError_t hipMemset(void *d, int v, size_t n) { memset(d, v, n); return fake::note("hipMemset"); }
+
+hipError_t hipDeviceSynchronize() { return fake::note("hipDeviceSynchronize"); }
+hipError_t hipStreamSynchronize(hipStream_t s) { return fake::note("hipStreamSynchronize", s); }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { (void)fake::note("hipStreamCreate"); return fake::make(s); }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return fake::make(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t s) { return fake::note("hipEventRecord", s); }
+hipError_t hipEventSynchronize(hipEvent_t) { return fake::note("hipEventSynchronize"); }
+
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) { std::swap(*m, fake::thread_mode); return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { fake::capturing = s; return fake::note("hipStreamBeginCapture", s); }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { fake::capturing = nullptr; return fake::make(g); }
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st)
+{
+    *st = s && s == fake::capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t *g, hipGraph_t, hipGraphNode_t *, char *, size_t) { (void)fake::note("hipGraphInstantiate"); return fake::make(g); }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) { return fake::note("hipGraphLaunch", s); }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return fake::note("hipGraphExecDestroy"); }
+
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t s) { return fake::note("configure", s); }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *s) { *s = fake::calls.back().stream; return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) { return fake::note("launch", s, fake::launch_answer); }
+}
+
+namespace {
+
+using namespace bitnet;
+int failures = 0;
+#define CHECK(cond) \
+    do { \
+        if (!(cond)) { std::printf("FAIL line %d: %s\n", __LINE__, #cond); ++failures; } \
+    } while (0)
+
+const hipStream_t side = reinterpret_cast<hipStream_t>(0x1000);
+
+// The mirror's quantisers read on the null stream what a kernel on the caller's stream leaves: they wait for that stream first.
+void mirror_waits_for_the_stream_it_was_given()
+{
+    auto x = DeviceTensor::from_vec(std::vector<float>(64 * 64, 1.0f), {64, 64}).unwrap();
+    for (hipStream_t s : {side, hipStream_t(nullptr)}) {
+        fake::calls.clear();
+        CHECK(absmax_quantize_activations(x, std::nullopt, s).is_ok());
+        long launched = fake::last("launch", s), waited = fake::last("hipStreamSynchronize", s);
+        CHECK(launched >= 0 && launched < waited && fake::last("hipMemcpy", nullptr) > waited);
+        fake::calls.clear();
+        CHECK(BitNetWeightQuantizer().quantize(x, s).is_ok());
+        launched = fake::last("launch", s), waited = fake::last("hipStreamSynchronize", s);
+        CHECK(launched >= 0 && launched < waited && fake::count("hipMemcpy") == 3 && fake::last("hipMemcpy", nullptr) == waited + 3);
+    }
+}
+
+struct Check {
+    const char *name;
+    void (*run)();
+};
+const Check checks[] = {
+    {"mirror_waits_for_the_stream_it_was_given", mirror_waits_for_the_stream_it_was_given},
+};
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    for (const Check &c : checks) {
+        if (argc == 2 && std::string(argv[1]) != c.name) continue;
+        if (argc == 1) { std::printf("%s\n", c.name); continue; }
+        c.run();
+        std::printf("%s: %d failed\n", c.name, failures);
+        return failures ? 1 : 0;
+    }
+    return argc == 1 ? 0 : 2;
+}

@@ -110,3 +110,24 @@ def test_calls_on_another_stream_share_no_memory_with_the_current_one(name):
     again = call(xs[1], side)
     torch.cuda.synchronize()
     assert same(read, want[0]) and same(again, want[1])
+
+
+@pytest.mark.gpu
+def test_quantisers_on_another_stream_return_what_their_kernels_wrote():
+    """The figures and bytes of a quantiser on a stream that is held up, read on the current stream as soon as the call is back."""
+    bh.init(0)
+    rng = np.random.default_rng(3)
+    x = torch.from_numpy(synth_weights(rng, 96, 512)).cuda()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    weights = bh.BitNetWeightQuantizer()
+    for call in (lambda s: (a := bh.absmax_quantize_activations(x, stream=s)) and (a.stats, a.values, a.scales),
+                 lambda s: (w := weights.quantize(x, stream=s)) and (w.stats, w.values, w.packed, w.scales),
+                 lambda s: ({}, *bh.quantize_weights(x, stream=s)[:2])):
+        stats, *tensors = call(None)
+        tensors = [t.clone() for t in tensors]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(20_000_000)
+        got, *other = call(side)
+        assert got == stats and all(torch.equal(a, b) for a, b in zip(other, tensors))
