@@ -77,7 +77,8 @@ inline BitLinearError last_error(int status)
 class DeviceTensor {
 public:
     DeviceTensor() = default;
-    static Result<DeviceTensor> zeros(std::vector<size_t> dims)
+    // memory that the caller's kernels fill
+    static Result<DeviceTensor> uninitialised(std::vector<size_t> dims)
     {
         DeviceTensor t;
         t.dims_ = std::move(dims);
@@ -85,13 +86,21 @@ public:
         float *p = nullptr;
         if (hipMalloc(reinterpret_cast<void **>(&p), (n ? n : 1) * sizeof(float)) != hipSuccess)
             return BitLinearError{BitLinearError::MemoryError, "hipMalloc failed", {}, {}};
-        (void)hipMemset(p, 0, n * sizeof(float));
         t.data_.reset(p, [](float *q) { (void)hipFree(q); });
+        return t;
+    }
+    // complete on return: hipMemset only enqueues, and a stream created without the null stream does not wait for it
+    static Result<DeviceTensor> zeros(std::vector<size_t> dims)
+    {
+        auto t = uninitialised(std::move(dims));
+        if (t.is_err()) return t;
+        if (hipMemset(t.unwrap().data(), 0, t.unwrap().elem_count() * sizeof(float)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+            return BitLinearError{BitLinearError::DeviceError, "hipMemset failed", {}, {}};
         return t;
     }
     static Result<DeviceTensor> from_vec(const std::vector<float> &host, std::vector<size_t> dims)
     {
-        auto r = zeros(std::move(dims));
+        auto r = uninitialised(std::move(dims));
         if (r.is_err()) return r;
         if (r.unwrap().elem_count() != host.size())
             return BitLinearError{BitLinearError::ShapeMismatch, "from_vec: element count", {r.unwrap().elem_count()}, {host.size()}};
@@ -182,7 +191,7 @@ public:
     {
         std::vector<size_t> out_dims = input.dims();
         if (!out_dims.empty()) out_dims.back() = config_.out_features;
-        auto out = DeviceTensor::zeros(out_dims.empty() ? std::vector<size_t>{config_.out_features} : out_dims);
+        auto out = DeviceTensor::uninitialised(out_dims.empty() ? std::vector<size_t>{config_.out_features} : out_dims);
         if (out.is_err()) return out;
         // the scratch for the quantised activations is kept by the layer and grown on demand: no allocation per call
         size_t rows = input.dims().empty() ? 0 : input.elem_count() / (input.dims().back() ? input.dims().back() : 1);
@@ -320,7 +329,7 @@ public:
         if (input.dims().size() != 2 || input.dims()[1] != hidden)
             return BitLinearError{BitLinearError::ShapeMismatch, "ffn input", {1, hidden}, input.dims()};
         const size_t m = input.dims()[0];
-        auto gate = DeviceTensor::zeros({m, ffn}), up = DeviceTensor::zeros({m, ffn}), out = DeviceTensor::zeros({m, hidden});
+        auto gate = DeviceTensor::uninitialised({m, ffn}), up = DeviceTensor::uninitialised({m, ffn}), out = DeviceTensor::uninitialised({m, hidden});
         if (gate.is_err() || up.is_err() || out.is_err()) return BitLinearError{BitLinearError::MemoryError, "hipMalloc failed", {}, {}};
         bitnet_hip_bitlinear *layers[2] = {gate_proj->handle(), up_proj->handle()};
         float *outs[2] = {gate.unwrap().data(), up.unwrap().data()};
@@ -596,7 +605,7 @@ public:
     }
     Result<DeviceTensor> decode(const DeviceTensor &x) const
     {
-        auto out = DeviceTensor::zeros(x.dims());
+        auto out = DeviceTensor::uninitialised(x.dims());
         if (out.is_err()) return out;
         int rc = bitnet_hip_decoder_decode(handle_, x.data(), x.dims().empty() ? 0 : x.dims()[0], out.unwrap().data(), nullptr, nullptr, nullptr);
         if (rc != BITNET_HIP_OK) return last_error(rc);
@@ -673,7 +682,7 @@ public:
         for (const DeviceTensor &t : inputs) {
             if (model_ && (t.dims().size() != 2 || t.dims()[1] != model_->hidden))
                 return BitLinearError{BitLinearError::ShapeMismatch, "execute_batch input", {t.dims().empty() ? 1 : t.dims()[0], model_->hidden}, t.dims()};
-            auto o = DeviceTensor::zeros(t.dims());
+            auto o = DeviceTensor::uninitialised(t.dims());
             if (o.is_err()) return o.unwrap_err();
             outs.push_back(o.unwrap());
             in_ptrs.push_back(t.data());

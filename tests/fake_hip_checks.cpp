@@ -143,12 +143,32 @@ void mirror_waits_for_the_stream_it_was_given()
     }
 }
 
+// Nothing that the mirror enqueues on the null stream may still write a result that a kernel on the caller's stream fills.
+void mirror_leaves_nothing_on_the_null_stream()
+{
+    auto ready = [] { return fake::last("hipMemset", nullptr) <= fake::last("hipStreamSynchronize", nullptr); };
+    fake::calls.clear();
+    auto x = DeviceTensor::zeros({40, 64}).unwrap();
+    CHECK(ready());
+    BitLinearConfig c;
+    c.in_features = c.out_features = 64;
+    auto layer = BitLinear::create(c, "layer").unwrap();
+    CHECK(layer->update_weights(std::vector<float>(64 * 64, 0.5f), 64, 64).is_ok());
+    fake::calls.clear();
+    CHECK(layer->forward(x, nullptr, side).is_ok() && fake::count("launch") > 0 && ready());
+    FeedForwardNetwork net;
+    net.up_proj = net.gate_proj = net.down_proj = layer;
+    fake::calls.clear();
+    CHECK(net.forward(x, side).is_ok() && fake::count("launch") > 0 && ready());
+}
+
 struct Check {
     const char *name;
     void (*run)();
 };
 const Check checks[] = {
     {"mirror_waits_for_the_stream_it_was_given", mirror_waits_for_the_stream_it_was_given},
+    {"mirror_leaves_nothing_on_the_null_stream", mirror_leaves_nothing_on_the_null_stream},
 };
 
 }  // namespace
