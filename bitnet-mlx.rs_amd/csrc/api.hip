@@ -797,13 +797,16 @@ int bitnet_hip_bitlinear_set_weights_gguf(bitnet_hip_bitlinear *layer, const uin
     if (offset_out) *offset_out = header[1];
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
-    // The codes start 8 bytes into the tensor; they go to an aligned address, the layer's own bytes, in their own orientation,
-    // and give way there to the canonical form ([out, in] order, code 3 stored as code 1).
+    // The codes start 8 bytes into the tensor; they go to scratch first, in their own orientation, and from there into the tiles and
+    // the canonical bytes ([out, in] order, code 3 stored as code 1).  The layer stays as it is until they are on the device.
+    StreamScratch codes_dev;
     Upload up;
-    int rc = BITNET_HIP_OK;
-    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(layer->packed, data + 8, codes, hipMemcpyDeviceToDevice, s));
-    else rc = up.copy(layer->packed, data + 8, codes, s);
-    if (rc == BITNET_HIP_OK) rc = launch_retile(layer->packed, n, k, layout, layer->tiled, s, layer->packed, header[0], layer->w_scale);
+    int rc = codes_dev.alloc(codes, s);
+    if (rc != BITNET_HIP_OK) return rc;
+    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(codes_dev.ptr, data + 8, codes, hipMemcpyDeviceToDevice, s));
+    else rc = up.copy(codes_dev.ptr, data + 8, codes, s);
+    if (rc == BITNET_HIP_OK)
+        rc = launch_retile(static_cast<const uint8_t *>(codes_dev.ptr), n, k, layout, layer->tiled, s, layer->packed, header[0], layer->w_scale);
     if (rc != BITNET_HIP_OK) return rc;
     BITNET_HIP_TRY(hipStreamSynchronize(s));
     up.done();

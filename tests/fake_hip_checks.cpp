@@ -162,6 +162,29 @@ void mirror_leaves_nothing_on_the_null_stream()
     CHECK(net.forward(x, side).is_ok() && fake::count("launch") > 0 && ready());
 }
 
+// A GGUF tensor whose bytes do not reach the device leaves the layer with the weights it had.
+void failed_gguf_copy_leaves_the_layer_whole()
+{
+    const size_t n = 32, k = 64, codes = n * k / 4;
+    for (int on_device : {0, 1})
+        for (int layout : {BITNET_HIP_LAYOUT_OUT_IN, BITNET_HIP_LAYOUT_IN_OUT}) {
+            bitnet_hip_bitlinear *layer = nullptr;
+            CHECK(bitnet_hip_bitlinear_create(k, n, 0, &layer) == BITNET_HIP_OK);
+            const std::vector<uint8_t> held(codes, 0x61), data(8 + codes, 0x22);
+            CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, held.data(), codes, 0.5f, 0, nullptr) == BITNET_HIP_OK);
+            fake::copies_until_failure = on_device;  // of a device tensor, the header's copy succeeds
+            const size_t rows = layout == BITNET_HIP_LAYOUT_OUT_IN ? n : k, cols = n + k - rows;
+            fake::calls.clear();
+            CHECK(bitnet_hip_bitlinear_set_weights_gguf(layer, data.data(), data.size(), rows, cols, layout, on_device, nullptr, nullptr,
+                                                        nullptr) != BITNET_HIP_OK);
+            fake::copies_until_failure = -1;
+            CHECK(fake::count("launch") == 0);
+            std::vector<uint8_t> back(codes);
+            CHECK(bitnet_hip_bitlinear_get_quantized(layer, nullptr, back.data(), codes) == BITNET_HIP_OK && back == held);
+            bitnet_hip_bitlinear_destroy(layer);
+        }
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -169,6 +192,7 @@ struct Check {
 const Check checks[] = {
     {"mirror_waits_for_the_stream_it_was_given", mirror_waits_for_the_stream_it_was_given},
     {"mirror_leaves_nothing_on_the_null_stream", mirror_leaves_nothing_on_the_null_stream},
+    {"failed_gguf_copy_leaves_the_layer_whole", failed_gguf_copy_leaves_the_layer_whole},
 };
 
 }  // namespace
