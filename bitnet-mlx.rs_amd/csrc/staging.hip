@@ -70,30 +70,41 @@ struct Ring {
         base = on_device = nullptr;
         device = -1;
     }
-    int prepare()
+    // False where there is no pinned memory to be had: the copy then goes through the runtime, which needs none of ours.
+    bool prepare()
     {
         int now = 0;
-        int rc = current_device(&now);
-        if (rc != BITNET_HIP_OK) return rc;
-        if (base && device == now) return BITNET_HIP_OK;
+        if (hipGetDevice(&now) != hipSuccess) return false;
+        if (base && device == now) return true;
         drop();
         void *mapped = nullptr;
         hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&base), CHUNK * CHUNKS + 256, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostGetDevicePointer(&mapped, base, 0);
+        if (e != hipSuccess) base = nullptr;
+        else e = hipHostGetDevicePointer(&mapped, base, 0);
         for (hipEvent_t &ev : passed)
             if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         if (e != hipSuccess) {
             drop();
-            return fail(BITNET_HIP_MEMORY_ERROR, "pinned staging chunks: %s", hipGetErrorString(e));
+            (void)hipGetLastError();
+            return false;
         }
         on_device = static_cast<uint8_t *>(mapped);
         scalar = reinterpret_cast<float *>(base + CHUNK * CHUNKS);
         scalar_on_device = reinterpret_cast<float *>(on_device + CHUNK * CHUNKS);
         device = now;
-        return BITNET_HIP_OK;
+        return true;
     }
 };
 Ring ring;
+
+// Takes the chunks for a copy of `bytes` at the device address `device_side`, where they pay and are there to be had.
+bool take_ring(std::unique_lock<std::mutex> &mine, size_t bytes, const void *device_side)
+{
+    if (bytes < RING_MIN_BYTES || (reinterpret_cast<uintptr_t>(device_side) & 15) != 0 || !mine.try_lock()) return false;
+    if (ring.prepare()) return true;
+    mine.unlock();
+    return false;
+}
 
 std::mutex users_lock;
 size_t users = 0;
@@ -223,13 +234,11 @@ int StreamScratch::alloc(size_t bytes, hipStream_t stream)
 int Upload::copy(void *dst, const void *src, size_t bytes, hipStream_t stream)
 {
     std::unique_lock<std::mutex> mine(ring.lock, std::defer_lock);
-    if (bytes < RING_MIN_BYTES || (reinterpret_cast<uintptr_t>(dst) & 15) != 0 || !mine.try_lock()) {
+    if (!take_ring(mine, bytes, dst)) {
         BITNET_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
         BITNET_HIP_TRY(hipStreamSynchronize(stream));
         return BITNET_HIP_OK;
     }
-    int rc = ring.prepare();
-    if (rc != BITNET_HIP_OK) return rc;
     ring_ = std::move(mine);
     stream_ = stream;
     const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
@@ -262,14 +271,12 @@ Upload::~Upload()
 int download(void *dst, const void *src, size_t bytes, const float *scalar, float *scalar_host, hipStream_t stream)
 {
     std::unique_lock<std::mutex> mine(ring.lock, std::defer_lock);
-    if (bytes < RING_MIN_BYTES || (reinterpret_cast<uintptr_t>(src) & 15) != 0 || !mine.try_lock()) {
+    if (!take_ring(mine, bytes, src)) {
         if (scalar) BITNET_HIP_TRY(hipMemcpyAsync(scalar_host, scalar, sizeof(float), hipMemcpyDeviceToHost, stream));
         BITNET_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
         BITNET_HIP_TRY(hipStreamSynchronize(stream));
         return BITNET_HIP_OK;
     }
-    int rc = ring.prepare();
-    if (rc != BITNET_HIP_OK) return rc;
     hipError_t e = hipSuccess;
     const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
     auto part_of = [&](size_t c) { return c + 1 < chunks ? CHUNK : bytes - c * CHUNK; };

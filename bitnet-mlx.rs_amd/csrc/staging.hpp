@@ -27,8 +27,8 @@ private:
 // the host copies the next.  (4.4 MB: the link alone takes 85 us, the host's copy 56 us; one after the other, as the
 // runtime does it, 138 us.  hipMemcpyAsync and an event per chunk cost the host more than they hide.)  What follows on the
 // stream sees the data; the object holds the chunks until the stream has passed them: done() after the caller's own
-// synchronisation, or the destructor, which waits.  One upload at a time has the chunks; others, and small ones, take the
-// runtime's path.
+// synchronisation, or the destructor, which waits.  One upload at a time has the chunks; others, small ones, and all of
+// them where pinned memory is not to be had, take the runtime's path.
 class Upload {
 public:
     Upload() = default;

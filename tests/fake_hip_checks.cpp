@@ -185,6 +185,26 @@ void failed_gguf_copy_leaves_the_layer_whole()
         }
 }
 
+// Without pinned memory, layers are loaded and saved through the runtime's own copies.
+void loads_and_saves_without_pinned_memory()
+{
+    const size_t n = 1024, k = 2048, codes = n * k / 4;  // more than the chunks are made for
+    bitnet_hip_bitlinear *layer = nullptr;
+    CHECK(bitnet_hip_bitlinear_create(k, n, 0, &layer) == BITNET_HIP_OK);
+    std::vector<uint8_t> held(codes), back(codes);
+    for (size_t i = 0; i < codes; ++i) held[i] = (uint8_t)(i * 7);
+    fake::host_malloc_answer = hipErrorOutOfMemory;
+    CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, held.data(), codes, 0.5f, 0, nullptr) == BITNET_HIP_OK);
+    CHECK(bitnet_hip_bitlinear_get_quantized(layer, nullptr, back.data(), codes) == BITNET_HIP_OK && back == held);
+    CHECK(fake::count("hipHostMalloc") > 0);
+    fake::host_malloc_answer = hipSuccess;
+    // and through the chunks once there is some: a launch moves what is copied here otherwise
+    fake::calls.clear();
+    CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, held.data(), codes, 0.5f, 0, nullptr) == BITNET_HIP_OK);
+    CHECK(fake::count("hipHostMalloc") == 1 && fake::count("hipMemcpyAsync") == 0);
+    bitnet_hip_bitlinear_destroy(layer);
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -193,6 +213,7 @@ const Check checks[] = {
     {"mirror_waits_for_the_stream_it_was_given", mirror_waits_for_the_stream_it_was_given},
     {"mirror_leaves_nothing_on_the_null_stream", mirror_leaves_nothing_on_the_null_stream},
     {"failed_gguf_copy_leaves_the_layer_whole", failed_gguf_copy_leaves_the_layer_whole},
+    {"loads_and_saves_without_pinned_memory", loads_and_saves_without_pinned_memory},
 };
 
 }  // namespace
