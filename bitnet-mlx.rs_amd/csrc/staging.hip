@@ -234,13 +234,13 @@ int StreamScratch::alloc(size_t bytes, hipStream_t stream)
 int Upload::copy(void *dst, const void *src, size_t bytes, hipStream_t stream)
 {
     std::unique_lock<std::mutex> mine(ring.lock, std::defer_lock);
+    stream_ = stream;
+    reading_ = true;
     if (!take_ring(mine, bytes, dst)) {
         BITNET_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
-        BITNET_HIP_TRY(hipStreamSynchronize(stream));
         return BITNET_HIP_OK;
     }
     ring_ = std::move(mine);
-    stream_ = stream;
     const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
     hipError_t e = hipSuccess;
     for (size_t c = 0; c < chunks && e == hipSuccess; ++c) {
@@ -258,14 +258,14 @@ int Upload::copy(void *dst, const void *src, size_t bytes, hipStream_t stream)
 
 void Upload::done()
 {
+    reading_ = false;
     if (ring_.owns_lock()) ring_.unlock();
 }
 
 Upload::~Upload()
 {
-    if (!ring_.owns_lock()) return;
-    (void)hipStreamSynchronize(stream_);  // the chunks' next user must not overwrite what the link still reads
-    ring_.unlock();
+    // the caller's buffer, and the chunks for their next user, must outlive what the link still reads
+    if (reading_) (void)hipStreamSynchronize(stream_);
 }
 
 int download(void *dst, const void *src, size_t bytes, const float *scalar, float *scalar_host, hipStream_t stream)

@@ -26,8 +26,8 @@ private:
 // Pageable host memory to the device through pinned chunks: the host copies a chunk, a kernel pulls it over the link while
 // the host copies the next.  (4.4 MB: the link alone takes 85 us, the host's copy 56 us; one after the other, as the
 // runtime does it, 138 us.  hipMemcpyAsync and an event per chunk cost the host more than they hide.)  What follows on the
-// stream sees the data; the object holds the chunks until the stream has passed them: done() after the caller's own
-// synchronisation, or the destructor, which waits.  One upload at a time has the chunks; others, small ones, and all of
+// stream sees the data; the object holds the chunks, and `src` must stay, until the stream has passed them: done() after the
+// caller's own synchronisation, or the destructor, which waits.  One upload at a time has the chunks; others, small ones, and all of
 // them where pinned memory is not to be had, take the runtime's path.
 class Upload {
 public:
@@ -41,6 +41,7 @@ public:
 private:
     std::unique_lock<std::mutex> ring_;
     hipStream_t stream_ = nullptr;
+    bool reading_ = false;
 };
 // The other way: returns with `dst` complete.  `scalar` (optional): one device float that comes along, into *scalar_host.
 // (4.4 MB into pageable memory through hipMemcpy: 250 us.)

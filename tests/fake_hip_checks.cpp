@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -61,7 +62,7 @@ hipError_t make(T *out)
 
 extern "C" {
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return fake::launch_answer; }
 const char *hipGetErrorString(hipError_t) { return "as told"; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 
@@ -205,6 +206,39 @@ void loads_and_saves_without_pinned_memory()
     bitnet_hip_bitlinear_destroy(layer);
 }
 
+// Loading from host memory waits for the stream once, at the end; and also where a launch behind the copy fails, since the
+// caller's buffer is free on return.
+void loads_wait_for_the_stream_once()
+{
+    for (size_t n : {size_t(64), size_t(1024)}) {  // through the runtime's copy, and through the chunks
+        const size_t k = 2048, codes = n * k / 4;
+        bitnet_hip_bitlinear *layer = nullptr;
+        CHECK(bitnet_hip_bitlinear_create(k, n, 0, &layer) == BITNET_HIP_OK);
+        const std::vector<uint8_t> data(8 + codes, 0x22);
+        const std::vector<float> latent(n * k, 0.5f);
+        const auto packed = [&] { return bitnet_hip_bitlinear_set_weights_packed(layer, data.data(), codes, 0.5f, 0, side); };
+        const auto base3 = [&] { return bitnet_hip_bitlinear_set_weights_base3(layer, data.data(), (n * k + 4) / 5, 0.5f, 0, side); };
+        const auto gguf = [&] {
+            return bitnet_hip_bitlinear_set_weights_gguf(layer, data.data(), data.size(), n, k, BITNET_HIP_LAYOUT_OUT_IN, 0, nullptr, nullptr, side);
+        };
+        const auto f32 = [&] {
+            return bitnet_hip_bitlinear_set_weights_f32(layer, latent.data(), n, k, BITNET_HIP_LAYOUT_OUT_IN, 0, BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP, 0.5f, side);
+        };
+        const std::vector<std::function<int()>> loads = {packed, base3, gguf, f32};
+        for (const auto &load : loads)
+            for (hipError_t answer : {hipSuccess, hipErrorLaunchFailure}) {
+                fake::calls.clear();
+                fake::launch_answer = answer;
+                CHECK((load() == BITNET_HIP_OK) == (answer == hipSuccess));
+                fake::launch_answer = hipSuccess;
+                CHECK(fake::count("hipStreamSynchronize") == 1);
+                CHECK(fake::last("hipStreamSynchronize", side) > fake::last("launch", side));
+                CHECK(fake::last("hipStreamSynchronize", side) > fake::last("hipMemcpyAsync", side));
+            }
+        bitnet_hip_bitlinear_destroy(layer);
+    }
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -214,6 +248,7 @@ const Check checks[] = {
     {"mirror_leaves_nothing_on_the_null_stream", mirror_leaves_nothing_on_the_null_stream},
     {"failed_gguf_copy_leaves_the_layer_whole", failed_gguf_copy_leaves_the_layer_whole},
     {"loads_and_saves_without_pinned_memory", loads_and_saves_without_pinned_memory},
+    {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
 };
 
 }  // namespace
