@@ -1326,6 +1326,21 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
     return rc;
 }
 
+namespace {
+// While one lives, this thread's calls are not held to another thread's capture in the global mode.
+class AnyCaptureMode {
+public:
+    AnyCaptureMode() { known_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+    ~AnyCaptureMode() { if (known_) (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    AnyCaptureMode(const AnyCaptureMode &) = delete;
+    AnyCaptureMode &operator=(const AnyCaptureMode &) = delete;
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;  // the thread's own while this lives
+    bool known_ = false;
+};
+}  // namespace
+
 // The recorded form of a step, or null where it is to be enqueued launch by launch.  A launch costs the host 2.3 to 4.5 us and
 // a block is four to eight of them, which the GPU runs in 12 to 25 us where the model is small or the step one token: the
 // host was the slower side.  A graph costs it 13 us whatever it holds (120 launches of a 30-block step: 15 us).  Recording
@@ -1359,6 +1374,9 @@ static hipGraphExec_t repeated_step_graph(bitnet_hip_decoder *dec, const StepKey
     hipStream_t cs = nullptr;
     hipGraph_t recorded = nullptr;
     hipGraphExec_t exec = nullptr;
+    // Another thread may be capturing a graph of its own in the global mode, under which calls of any thread that are not plain
+    // launches fail or spoil its capture.  What follows touches none of its streams, so this thread steps out of that rule.
+    const AnyCaptureMode unrestricted;
     // on a stream of its own: nothing runs, and what the caller's stream holds is not touched
     bool ok = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) == hipSuccess;
     if (ok && hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) == hipSuccess) {
@@ -1377,8 +1395,8 @@ static hipGraphExec_t repeated_step_graph(bitnet_hip_decoder *dec, const StepKey
         return nullptr;
     }
     if (oldest->exec) {
-        // its last replay may still be running: as when a layer's weights change, an event that is rare waits for the device
-        if (hipDeviceSynchronize() != hipSuccess) {
+        // its last replay may still be running: the steps of a decoder follow each other, and `done` stands behind the last one
+        if (hipEventSynchronize(dec->done) != hipSuccess) {
             (void)hipGraphExecDestroy(exec);
             return nullptr;
         }

@@ -16,17 +16,18 @@ namespace fake {
 struct Call {
     std::string name;
     hipStream_t stream;
+    hipStreamCaptureMode mode;  // of the thread, when it called
 };
 std::vector<Call> calls;
+hipStreamCaptureMode thread_mode = hipStreamCaptureModeGlobal;
 hipError_t host_malloc_answer = hipSuccess, launch_answer = hipSuccess;
 int copies_until_failure = -1;  // a copy that fails has moved half of its bytes
 hipStream_t capturing = nullptr;
-hipStreamCaptureMode thread_mode = hipStreamCaptureModeGlobal;
 uintptr_t next_handle = 1;
 
 hipError_t note(const char *name, hipStream_t stream = nullptr, hipError_t answer = hipSuccess)
 {
-    calls.push_back({name, stream});
+    calls.push_back({name, stream, thread_mode});
     return answer;
 }
 size_t count(const std::string &name)
@@ -239,6 +240,41 @@ void loads_wait_for_the_stream_once()
     }
 }
 
+// Recording a step that repeats, and giving up an old recording, leave a capture of another thread alone: what is no plain launch
+// runs outside the global mode's rule, nothing waits for the whole device, and the thread's own mode is back afterwards.
+void recording_a_step_leaves_other_captures_alone()
+{
+    bitnet_hip_decoder *dec = nullptr;
+    CHECK(bitnet_hip_decoder_create(2, 64, 64, 4, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, 4, &dec) == BITNET_HIP_OK);
+    const std::vector<uint8_t> codes(64 * 64 / 4, 0x22);
+    for (size_t l = 0; l < 2; ++l)
+        for (int p = 0; p < 7; ++p) {
+            bitnet_hip_bitlinear *layer = nullptr;
+            CHECK(bitnet_hip_decoder_projection(dec, l, p, &layer) == BITNET_HIP_OK);
+            CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, codes.data(), codes.size(), 0.5f, 0, nullptr) == BITNET_HIP_OK);
+        }
+    std::vector<float> x(64), outs(8 * 64);
+    const auto step = [&](int i) { CHECK(bitnet_hip_decoder_decode(dec, x.data(), 1, outs.data() + 64 * i, nullptr, nullptr, side) == BITNET_HIP_OK); };
+    fake::calls.clear();
+    for (int i = 0; i < 4; ++i)  // as many recordings as are kept
+        for (int times = 0; times < 3; ++times) step(i);
+    CHECK(fake::count("hipGraphInstantiate") == 4 && fake::count("hipGraphLaunch") == 4);
+    for (int times = 0; times < 64; ++times) step(1 + times % 3);  // replays that earn another recording
+    for (int times = 0; times < 3; ++times) step(5);
+    CHECK(fake::count("hipGraphInstantiate") == 5 && fake::count("hipGraphExecDestroy") == 1);
+    CHECK(fake::count("hipDeviceSynchronize") == 0);
+    bool waited = false;
+    for (const fake::Call &c : fake::calls) {
+        if (c.name == "hipStreamCreate" || c.name == "hipStreamBeginCapture" || c.name == "hipGraphInstantiate" || c.name == "hipGraphExecDestroy")
+            CHECK(c.mode == hipStreamCaptureModeRelaxed);
+        if (c.name == "hipGraphLaunch") waited = false;
+        if (c.name == "hipEventSynchronize") waited = true;
+        if (c.name == "hipGraphExecDestroy") CHECK(waited);
+    }
+    CHECK(fake::thread_mode == hipStreamCaptureModeGlobal);
+    bitnet_hip_decoder_destroy(dec);
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -249,6 +285,7 @@ const Check checks[] = {
     {"failed_gguf_copy_leaves_the_layer_whole", failed_gguf_copy_leaves_the_layer_whole},
     {"loads_and_saves_without_pinned_memory", loads_and_saves_without_pinned_memory},
     {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
+    {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
 };
 
 }  // namespace

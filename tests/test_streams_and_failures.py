@@ -131,3 +131,53 @@ def test_quantisers_on_another_stream_return_what_their_kernels_wrote():
             torch.cuda._sleep(20_000_000)
         got, *other = call(side)
         assert got == stats and all(torch.equal(a, b) for a, b in zip(other, tensors))
+
+
+@pytest.mark.gpu
+def test_a_step_is_recorded_while_another_thread_captures():
+    """The third, recorded call of a step while another thread is in a capture of its own (torch's default, the global mode): the
+    capture is whole afterwards, and so are the step's results."""
+    import threading
+
+    bh.init(0)
+    rng = np.random.default_rng(4)
+    dec = bh.DecoderProjections(3, 256, 512, 4, 2, 64, max_tokens=4)
+    for layer in range(3):
+        for p in range(7):
+            dec.projection(layer, p).update_weights(torch.from_numpy(synth_weights(rng, *dec.proj_shape(p))).cuda())
+    x = torch.from_numpy(synth_activations(rng, 2, 256)).cuda()
+    want, out, a = dec.decode(x), torch.empty_like(x), torch.ones(1000, device="cuda")
+    mine = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(2):
+        dec.decode(x, out=out, stream=mine)
+    mine.synchronize()
+    out.zero_()
+    torch.cuda.synchronize()
+    inside, stepped, errors = threading.Event(), threading.Event(), []
+
+    def steps():
+        try:
+            assert inside.wait(30)
+            for _ in range(2):  # recorded, replayed
+                dec.decode(x, out=out, stream=mine)
+        except BaseException as exc:
+            errors.append(exc)
+        finally:
+            stepped.set()
+
+    worker = threading.Thread(target=steps)
+    worker.start()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        b = a * 2
+        inside.set()
+        assert stepped.wait(30)
+        b = b + 1
+    worker.join()
+    assert not errors
+    for value in (1.0, 4.0):
+        a.fill_(value)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (b == 2 * value + 1).all() and torch.equal(out, want)
