@@ -797,17 +797,23 @@ int bitnet_hip_bitlinear_set_weights_gguf(bitnet_hip_bitlinear *layer, const uin
     if (offset_out) *offset_out = header[1];
     std::unique_lock<std::shared_mutex> guard(layer->lock);
     BITNET_HIP_TRY(hipDeviceSynchronize());  // forwards already queued on any stream still read the old weights
-    // The codes start 8 bytes into the tensor; they go to scratch first, in their own orientation, and from there into the tiles and
-    // the canonical bytes ([out, in] order, code 3 stored as code 1).  The layer stays as it is until they are on the device.
-    StreamScratch codes_dev;
+    // The codes start 8 bytes into the tensor; they go to an aligned address first, in their own orientation, and from there into the
+    // tiles and the canonical bytes ([out, in] order, code 3 stored as code 1).  A layer without weights lends its own bytes for
+    // that.  One that has some stays as it is until the codes are on the device: they go through scratch, for 12 us of a reload.
+    StreamScratch scratch;
     Upload up;
-    int rc = codes_dev.alloc(codes, s);
+    int rc = BITNET_HIP_OK;
+    uint8_t *at = layer->packed;
+    if (layer->has_weights) {
+        rc = scratch.alloc(codes, s);
+        if (rc != BITNET_HIP_OK) return rc;
+        at = static_cast<uint8_t *>(scratch.ptr);
+    }
+    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(at, data + 8, codes, hipMemcpyDeviceToDevice, s));
+    else rc = up.copy(at, data + 8, codes, s);
+    if (rc == BITNET_HIP_OK) rc = launch_retile(at, n, k, layout, layer->tiled, s, layer->packed, header[0], layer->w_scale);
     if (rc != BITNET_HIP_OK) return rc;
-    if (on_device) BITNET_HIP_TRY(hipMemcpyAsync(codes_dev.ptr, data + 8, codes, hipMemcpyDeviceToDevice, s));
-    else rc = up.copy(codes_dev.ptr, data + 8, codes, s);
-    if (rc == BITNET_HIP_OK)
-        rc = launch_retile(static_cast<const uint8_t *>(codes_dev.ptr), n, k, layout, layer->tiled, s, layer->packed, header[0], layer->w_scale);
-    if (rc != BITNET_HIP_OK) return rc;
+    scratch.give_back();
     BITNET_HIP_TRY(hipStreamSynchronize(s));
     up.done();
     layer->has_weights = true;

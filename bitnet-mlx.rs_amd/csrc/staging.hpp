@@ -15,8 +15,14 @@ public:
     StreamScratch() = default;
     StreamScratch(const StreamScratch &) = delete;
     StreamScratch &operator=(const StreamScratch &) = delete;
-    ~StreamScratch() { if (ptr) (void)hipFreeAsync(ptr, stream_); }
+    ~StreamScratch() { give_back(); }
     int alloc(size_t bytes, hipStream_t stream);
+    // Behind the last launch that uses it.  Ahead of a wait for the stream, whose work then hides the 12 us this takes the host.
+    void give_back()
+    {
+        if (ptr) (void)hipFreeAsync(ptr, stream_);
+        ptr = nullptr;
+    }
     void *ptr = nullptr;
 
 private:
