@@ -59,6 +59,7 @@ struct Ring {
     float *scalar = nullptr, *scalar_on_device = nullptr;  // behind the chunks
     hipEvent_t passed[CHUNKS] = {};
     int device = -1;
+    bool used = false;  // since the last layer of some time before was destroyed
 
     void drop()
     {
@@ -101,7 +102,7 @@ Ring ring;
 bool take_ring(std::unique_lock<std::mutex> &mine, size_t bytes, const void *device_side)
 {
     if (bytes < RING_MIN_BYTES || (reinterpret_cast<uintptr_t>(device_side) & 15) != 0 || !mine.try_lock()) return false;
-    if (ring.prepare()) return true;
+    if (ring.prepare()) return ring.used = true;
     mine.unlock();
     return false;
 }
@@ -313,7 +314,8 @@ void staging_release()
     std::lock_guard<std::mutex> guard(users_lock);
     if (--users == 0) {
         std::lock_guard<std::mutex> idle(ring.lock);
-        ring.drop();
+        if (!ring.used) ring.drop();
+        ring.used = false;
     }
 }
 

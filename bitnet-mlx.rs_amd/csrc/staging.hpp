@@ -61,7 +61,10 @@ struct Pieces {
     unsigned count[MOST];  // floats
 };
 hipError_t launch_move_pieces(const Pieces &pieces, int n, hipStream_t stream);
-// The chunks exist while layers do: made by the first copy that wants them, given back with the last layer.
+// How long the chunks (4 MiB a process) live: made by the first copy that wants them, given back when a last layer is destroyed
+// and nothing was copied since the last layer before it was.  Making and freeing them takes 45 to 85 us, which a program that makes
+// a layer, loads it, saves it and drops it, one after the other, does not pay each time (a GGUF tensor of 640 x 2560 through all
+// four: 125 us with the chunks given back each time, 84 so; 2560 x 2560: 255 and 168; 6912 x 2560: 500 and 470).
 void staging_retain();
 void staging_release();
 

@@ -275,6 +275,25 @@ void recording_a_step_leaves_other_captures_alone()
     bitnet_hip_decoder_destroy(dec);
 }
 
+// Layers made, loaded and dropped one after the other share the pinned chunks; they are given back once layers come and go unloaded.
+void chunks_outlive_a_layer_that_used_them()
+{
+    const size_t n = 1024, k = 2048, codes = n * k / 4;
+    const std::vector<uint8_t> data(codes, 0x22);
+    const auto layer = [&](bool load) {
+        bitnet_hip_bitlinear *l = nullptr;
+        CHECK(bitnet_hip_bitlinear_create(k, n, 0, &l) == BITNET_HIP_OK);
+        if (load) CHECK(bitnet_hip_bitlinear_set_weights_packed(l, data.data(), codes, 0.5f, 0, nullptr) == BITNET_HIP_OK);
+        bitnet_hip_bitlinear_destroy(l);
+    };
+    for (int round = 1; round <= 2; ++round) {
+        for (int i = 0; i < 3; ++i) layer(true);
+        CHECK((int)fake::count("hipHostMalloc") == round && (int)fake::count("hipHostFree") == round - 1);
+        layer(false);
+        CHECK((int)fake::count("hipHostMalloc") == round && (int)fake::count("hipHostFree") == round);
+    }
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -286,6 +305,7 @@ const Check checks[] = {
     {"loads_and_saves_without_pinned_memory", loads_and_saves_without_pinned_memory},
     {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
+    {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
 };
 
 }  // namespace
