@@ -791,8 +791,12 @@ int bitnet_hip_bitlinear_set_weights_gguf(bitnet_hip_bitlinear *layer, const uin
     }
     hipStream_t s = as_stream(stream);
     float header[2];  // little-endian host, as f32::from_le_bytes on the reference's targets
-    if (on_device) BITNET_HIP_TRY(hipMemcpy(header, data, 8, hipMemcpyDeviceToHost));
-    else memcpy(header, data, 8);
+    if (on_device) {  // in the order of the stream that the tensor is made on
+        BITNET_HIP_TRY(hipMemcpyAsync(header, data, 8, hipMemcpyDeviceToHost, s));
+        BITNET_HIP_TRY(hipStreamSynchronize(s));
+    } else {
+        memcpy(header, data, 8);
+    }
     if (scale_out) *scale_out = header[0];
     if (offset_out) *offset_out = header[1];
     std::unique_lock<std::shared_mutex> guard(layer->lock);

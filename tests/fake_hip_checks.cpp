@@ -294,6 +294,22 @@ void chunks_outlive_a_layer_that_used_them()
     }
 }
 
+// The header of a GGUF tensor in device memory is read behind the work of the caller's stream, as the codes are.
+void gguf_header_is_read_in_stream_order()
+{
+    const size_t n = 32, k = 64;
+    const std::vector<uint8_t> data(8 + n * k / 4, 0x22);
+    bitnet_hip_bitlinear *layer = nullptr;
+    CHECK(bitnet_hip_bitlinear_create(k, n, 0, &layer) == BITNET_HIP_OK);
+    fake::calls.clear();
+    CHECK(bitnet_hip_bitlinear_set_weights_gguf(layer, data.data(), data.size(), n, k, BITNET_HIP_LAYOUT_OUT_IN, 1, nullptr, nullptr, side) ==
+          BITNET_HIP_OK);
+    CHECK(fake::count("hipMemcpy") == 0 && fake::count("hipMemcpyAsync") == 2);
+    CHECK(fake::calls[0].name == "hipMemcpyAsync" && fake::calls[0].stream == side);
+    CHECK(fake::calls[1].name == "hipStreamSynchronize" && fake::calls[1].stream == side);
+    bitnet_hip_bitlinear_destroy(layer);
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -306,6 +322,7 @@ const Check checks[] = {
     {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
+    {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
 };
 
 }  // namespace
