@@ -1081,10 +1081,15 @@ struct StepGraph {
     uint64_t used = 0;  // step_clock of its last replay
 };
 constexpr int STEP_GRAPHS = 4, STEP_SEEN = 8;
-// Which steps are worth a recording: blocks of up to STEP_SMALL_BLOCK weights from the second block on (896 to 1536 wide: 17 to
-// 40 us a block launch by launch, 12 to 27 us recorded); larger blocks keep the GPU busy for as long as the host needs to
-// enqueue them, and a graph starts 7 us later than a launch, so those only where that is under 2 % of the step.
-constexpr size_t STEP_MIN_BLOCKS = 2, STEP_MIN_LARGE_BLOCKS = 12, STEP_SMALL_BLOCK = 70000000;
+// Which steps are worth a recording.  A recorded step starts about 6 us later than an enqueued one and gains 0.5 us a block back:
+// queued one behind the other, steps are even from 12 blocks on (11 blocks of 69 / 79 / 101 / 107 M weights at one token: 167 / 214 /
+// 223 / 291 us enqueued, 168 / 215 / 225 / 295 recorded).  A caller that waits for each step waits for the host's launches into an idle
+// queue, and gains from the second block on at any size (2 blocks of these: 72 / 97 / 100 / 102 -> 47 / 55 / 58 / 69 us; 11: 206 /
+// 261 / 263 / 322 -> 181 / 229 / 239 / 309).  Below 12 blocks the one stands against the other.  Such a step is recorded where the GPU
+// is done with a block of it, at one token, by the time the host has enqueued the block's four launches, 15 us, so that a queue
+// hangs on the host's launches as well: 15 to 24 M weights take it 12 us, 45 M 12.5, 69 M 14.9; 79 M 19, 82 M 16 to 19, 101 M 20.
+// (Queued steps of few such blocks pay for it: 2 blocks of 69 M 33 -> 39 us; 8 of 24 M gain, 115 -> 106.)
+constexpr size_t STEP_MIN_BLOCKS = 2, STEP_MIN_LARGE_BLOCKS = 12, STEP_SMALL_BLOCK = 74000000;
 }  // namespace
 
 struct bitnet_hip_decoder {

@@ -240,19 +240,43 @@ void loads_wait_for_the_stream_once()
     }
 }
 
-// Recording a step that repeats, and giving up an old recording, leave a capture of another thread alone: what is no plain launch
-// runs outside the global mode's rule, nothing waits for the whole device, and the thread's own mode is back afterwards.
-void recording_a_step_leaves_other_captures_alone()
+bitnet_hip_decoder *decoder_with_weights(size_t layers, size_t hidden, size_t ffn)
 {
     bitnet_hip_decoder *dec = nullptr;
-    CHECK(bitnet_hip_decoder_create(2, 64, 64, 4, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, 4, &dec) == BITNET_HIP_OK);
-    const std::vector<uint8_t> codes(64 * 64 / 4, 0x22);
-    for (size_t l = 0; l < 2; ++l)
+    CHECK(bitnet_hip_decoder_create(layers, hidden, ffn, hidden / 16, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, 4, &dec) == BITNET_HIP_OK);
+    const std::vector<uint8_t> codes(hidden * (hidden > ffn ? hidden : ffn) / 4, 0x22);
+    for (size_t l = 0; l < layers; ++l)
         for (int p = 0; p < 7; ++p) {
             bitnet_hip_bitlinear *layer = nullptr;
             CHECK(bitnet_hip_decoder_projection(dec, l, p, &layer) == BITNET_HIP_OK);
             CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, codes.data(), codes.size(), 0.5f, 0, nullptr) == BITNET_HIP_OK);
         }
+    return dec;
+}
+
+// A step that comes a third time is recorded from two blocks on, and one of large blocks (above 74 M weights) from twelve on.
+void steps_worth_a_recording()
+{
+    const struct {
+        size_t layers, hidden, ffn, blocks;
+        bool recorded;
+    } steps[] = {{2, 64, 64, 1, false}, {2, 64, 64, 2, true}, {11, 2048, 10600, 11, true}, {12, 2048, 10700, 11, false}, {12, 2048, 10700, 12, true}};
+    for (const auto &t : steps) {
+        bitnet_hip_decoder *dec = decoder_with_weights(t.layers, t.hidden, t.ffn);
+        std::vector<float> x(t.hidden), out(t.hidden);
+        fake::calls.clear();
+        for (int times = 0; times < 3; ++times)
+            CHECK(bitnet_hip_decoder_decode_layers(dec, 0, t.blocks, x.data(), 1, out.data(), nullptr, nullptr, side) == BITNET_HIP_OK);
+        CHECK(fake::count("hipGraphLaunch") == (t.recorded ? 1 : 0));
+        bitnet_hip_decoder_destroy(dec);
+    }
+}
+
+// Recording a step that repeats, and giving up an old recording, leave a capture of another thread alone: what is no plain launch
+// runs outside the global mode's rule, nothing waits for the whole device, and the thread's own mode is back afterwards.
+void recording_a_step_leaves_other_captures_alone()
+{
+    bitnet_hip_decoder *dec = decoder_with_weights(2, 64, 64);
     std::vector<float> x(64), outs(8 * 64);
     const auto step = [&](int i) { CHECK(bitnet_hip_decoder_decode(dec, x.data(), 1, outs.data() + 64 * i, nullptr, nullptr, side) == BITNET_HIP_OK); };
     fake::calls.clear();
@@ -320,6 +344,7 @@ const Check checks[] = {
     {"failed_gguf_copy_leaves_the_layer_whole", failed_gguf_copy_leaves_the_layer_whole},
     {"loads_and_saves_without_pinned_memory", loads_and_saves_without_pinned_memory},
     {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
+    {"steps_worth_a_recording", steps_worth_a_recording},
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
