@@ -262,13 +262,19 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
     // In one round of workgroups only: a second one quantises again.  A row of 16 tokens costs a workgroup 0.4 us at 256 columns and
     // 1.0 us at 1024, the launch it saves 0.5 us of the GPU's time in a recorded step and 2.5 us of the host's outside one (9 x 256 ->
     // 2560: 5.1 -> 4.8 us recorded, 7.2 -> 4.7 us as calls; 16 x 1024 -> 2560: 5.1 -> 6.0 recorded, so up to 12288 elements a
-    // token group in a step and any row that fits in a call of its own).  Up to eight tokens
-    // gemv_fused16_kernel already is one launch, and the faster one but for long outputs of the attention (block of the stack
-    // at 8 tokens, 2560 wide: 27.6 -> 26.6 us; 4096 wide: 42.1 -> 39.8).
+    // token group in a step and any row that fits in a call of its own).
     const size_t in_group = m < 16 ? m : 16, tgroups = (m + 15) / 16;
-    if (m < 8 || (m == 8 && (!gqa || k < 2560)) || m > (size_t)GEMV_MAX_M || (blocks + 3) / 4 * tgroups > 256) return false;
+    if (m < 2 || m > (size_t)GEMV_MAX_M || (blocks + 3) / 4 * tgroups > 256) return false;
     if (width % 4 != 0 || ldx != width || width > MAX_WIDTH || (!gqa && !alone && width * in_group > 12288)) return false;
     if (k_tiles(k) > (size_t)MAX_KT || k > 0xffff || blocks > GEMV_ROWS_MAX_BLOCKS) return false;
+    // Up to eight tokens gemv_fused16_kernel may be one launch as well, with a set of workgroups for every token.  It has fewer rows to
+    // quantise but reads the weight tiles once a token, so it is ahead while its workgroups have few tiles to walk.  A decoder block
+    // with the attention output by this kernel instead, where those walk 24 to 40 tiles: 0.5 to 1.0 us slower (1536 to 2560 wide, 2
+    // to 8 tokens); 44 and 48: 0.1 to 0.3 slower (2816 and 3072 wide at 3 to 5); 52: 0.4 to 1.0 faster (3200 at 3 to 5), 56 and 64:
+    // even (3584 and 4096 at 3, 4), 80 and more: 0.6 to 2.0 faster (2560 at 7 and 8, 4096 at 5 to 8, 5120 to 8192 at 2 to 8).  Where
+    // that kernel's workgroups do not fit one round, the other choice is two launches: 6 x 1024 -> 8192 7.5 us a call, 3.7 here.
+    if (gemv_fused_supported(x, nullptr, ldx, m, k, input_mode, head_dim, gamma, sum_order, blocks) && gemv_fused_tiles(m, k, blocks) <= 48)
+        return false;
     return al16(x) && (!gamma || (al16(gamma) && sum_order == BITNET_HIP_SUM_BLOCK256));
 }
 

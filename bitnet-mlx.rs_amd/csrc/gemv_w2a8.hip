@@ -1712,6 +1712,8 @@ int fused16_row_blocks_per_workgroup(size_t m, size_t k, size_t blocks)
     return rbw;
 }
 
+size_t gemv_fused_tiles(size_t m, size_t k, size_t blocks) { return (size_t)fused16_row_blocks_per_workgroup(m, k, blocks) * k_tiles(k); }
+
 bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                           size_t head_dim, const float *gamma, int sum_order, size_t blocks)
 {

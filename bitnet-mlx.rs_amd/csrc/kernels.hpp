@@ -142,6 +142,7 @@ int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m,
 // a_sum_out (each optional) receive the quantiser's results.
 bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                           size_t head_dim, const float *gamma, int sum_order, size_t blocks);
+size_t gemv_fused_tiles(size_t m, size_t k, size_t blocks);  // weight tiles that one workgroup of that launch walks
 // blocks: 16-row blocks of all projections of the launch (of its largest launch group)
 int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const float *x2, size_t ldx, size_t m,
                       size_t k, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,

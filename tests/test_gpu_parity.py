@@ -1692,3 +1692,31 @@ def test_dynamic_quantiser_step_at_the_edges_of_its_kernels(precision, count, of
 
 def step_sizes_fit(count):
     return count < 1000000  # one step of the largest tensor is enough
+
+
+@pytest.mark.parametrize("m", [2, 3, 5, 8])
+@pytest.mark.parametrize("n,k", [(16384, 256), (10300, 516), (6400, 1024), (9600, 1028)])
+def test_forward_of_few_short_rows_and_long_outputs_bit_exact(m, n, k):
+    """Two to eight tokens on both sides of the lines at which the launch quantises every row once a workgroup instead of one row a
+    workgroup, or is two launches; a zero row, one too small and one too large for the short division."""
+    rng = np.random.default_rng(m + n + k)
+    x, pk, g = synth_activations(rng, m, k, outliers=True), random_packed_ternary(rng, n, k), rng.standard_normal(k, dtype=f32)
+    x[1] *= f32(2.0**-70)
+    if m > 3:
+        x[2], x[3] = 0.0, x[3] * f32(2.0**70)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "few rows")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    res = rng.standard_normal((m, n), dtype=f32)
+    assert np.array_equal(host(layer.forward(dev(x), residual=dev(res))), orc.bitlinear_forward(x, pk, n, f32(0.02), residual=res)[0])
+    assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g))), orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, eps=1e-5)[0])
+
+
+@pytest.mark.parametrize("dims", [(2304, 64, 18, 2, 128), (2560, 64, 20, 5, 128), (3200, 64, 25, 5, 128), (5120, 64, 40, 8, 128), (896, 4864, 14, 2, 64)])
+@pytest.mark.parametrize("m", [2, 3, 7, 8])
+def test_decoder_blocks_of_two_to_eight_tokens_match_the_oracle(dims, m):
+    """The attention output projection by either one-launch kernel, on both sides of the line between them, and gate and up of a
+    narrow model where the workgroups of one of them do not fit one round."""
+    rng = np.random.default_rng(m + dims[0])
+    dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
+    x = synth_activations(rng, m, dims[0])
+    assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
