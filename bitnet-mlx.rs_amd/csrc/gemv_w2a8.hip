@@ -1465,8 +1465,14 @@ int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src,
         if (norm) hipLaunchKernelGGL((gemv_fused16_kernel<MODE, true, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
         else hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
     } while (0)
-    if (nchb == 1) BITNET_F16_LAUNCH(1);
-    else BITNET_F16_LAUNCH(2);
+    // rows of more than 16 k-tiles take at most four row blocks a workgroup (fused16_row_blocks_per_workgroup)
+    if constexpr (RBW > 4) {
+        if (nchb != 1) return fail(BITNET_HIP_UNSUPPORTED, "fused GEMV: %d row blocks a workgroup for %d k-tiles", RBW, p.kt_count);
+        BITNET_F16_LAUNCH(1);
+    } else {
+        if (nchb == 1) BITNET_F16_LAUNCH(1);
+        else BITNET_F16_LAUNCH(2);
+    }
 #undef BITNET_F16_LAUNCH
 #undef BITNET_HOT_ARGS
     BITNET_HIP_CHECK_LAUNCH("gemv_fused16_kernel");
