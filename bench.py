@@ -76,7 +76,7 @@ STEP_BYTES = LAYER_BYTES * LAYERS
 # script with --no-extras --calibration-copy), each scaled by what the same counter reads for the plain
 # 256 MiB copy: FETCH_SIZE reads 0.5 KiB per KiB fetched (factor 2.0), WRITE_SIZE 1.0 (factor 1.0).
 # Summary: profiles/decode_layer_b1_gemv_hbm_traffic.md
-MEASURED_TRAFFIC_BYTES_PER_LAUNCH = 4_685_621
+MEASURED_TRAFFIC_BYTES_PER_LAUNCH = 4_658_296
 
 
 def decode_roofline(event_ms, steps):
@@ -227,6 +227,18 @@ def large_gemv_pair(bh, torch, gen, loops=5):
     return out
 
 
+def enqueued_steps(torch, dec, x):
+    """A function that makes one decode() step launch by launch.  A decoder replays steps that come again with the same tensors from a
+    recording of its own, so each step reads the tensor the one before it wrote, in a ring of more than it remembers."""
+    ring, at = [x.clone() for _ in range(16)], [0]
+
+    def step():
+        i = at[0] = (at[0] + 1) % len(ring)
+        return dec.decode(ring[i - 1], out=ring[i])
+
+    return step
+
+
 def stack_latency(bh, torch, dec, gen, reps=20):
     """per-token decode latency through all 30 layers' projections, batch 1 and batch 8, and
     the gate / down projections at M in {1, 4, 16, 64} tokens (activations with 1 % x20 outliers)."""
@@ -239,8 +251,9 @@ def stack_latency(bh, torch, dec, gen, reps=20):
     for m in (1, 8):
         x = torch.randn((m, HIDDEN), generator=gen, device="cuda", dtype=torch.float32)
         y = torch.empty_like(x)
-        big.decode(x, out=y)
-        eager_ms = time_events(torch, lambda: [big.decode(x, out=y) for _ in range(reps)]) / reps
+        step = enqueued_steps(torch, big, x)
+        step()
+        eager_ms = time_events(torch, lambda: [step() for _ in range(reps)]) / reps
         recorded = big.record(x, out=y)
         recorded.replay()
         ms = sorted(time_events(torch, lambda: [recorded.replay() for _ in range(reps)]) / reps for _ in range(3))[1]
@@ -366,16 +379,17 @@ def sequential_order_decode(bh, torch, dec, gen, reps=20):
 def eager_decode(torch, dec, x, reps=20):
     """The headline step with its 120 launches enqueued one by one by the host, and what that enqueue costs the host:
     where the host needs longer per launch than the GPU, the loop runs at the host's pace."""
-    dec.decode(x, out=x)
+    step = enqueued_steps(torch, dec, x)
+    step()
     torch.cuda.synchronize()
     host = []
     for _ in range(9):
         torch.cuda.synchronize()
         t0 = time.perf_counter()
-        dec.decode(x, out=x)
+        step()
         host.append(time.perf_counter() - t0)
     host_us = sorted(host)[len(host) // 2] * 1e6
-    times = sorted(time_events(torch, lambda: [dec.decode(x, out=x) for _ in range(reps)]) / reps for _ in range(5))
+    times = sorted(time_events(torch, lambda: [step() for _ in range(reps)]) / reps for _ in range(5))
     ms = times[len(times) // 2]
     return {"us_per_token_step": round(ms * 1e3, 1), "gbs_packed_weights": round(dec.weight_bytes() / (ms * 1e-3) / 1e9, 1),
             "host_enqueue_us_per_step": round(host_us, 1), "host_enqueue_us_per_launch": round(host_us / LAUNCHES_PER_STEP, 2),
@@ -552,13 +566,14 @@ def main():
     # The step is recorded once (bitnet_hip_decoder_graph_create: the 120 launches of decode() as a HIP graph) and
     # replayed: the same kernels in the same order, enqueued by one host call.
     recorded = None if args.eager else dec.record(x, out=x)
+    eager_step = enqueued_steps(torch, dec, x) if args.eager else None
 
     def run_steps(count):
         """`count` token steps, each one call of the boundary: the seven projections of layers 0..29 in turn, the hidden
         state carried along (four launches per layer)."""
         for _ in range(count):
             if recorded is None:
-                dec.decode(x, out=x)
+                eager_step()
             else:
                 recorded.replay()
 
