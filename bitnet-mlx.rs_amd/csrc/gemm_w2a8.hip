@@ -1025,8 +1025,8 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     //                                           and two loader wavefronts;
     //   otherwise                            -> 64 x 160, four workgroups of 4 wavefronts per compute unit.
     // A long k with few tiles: the 64 x 32 tiles of the launch in three parts of k each (plan_split).  Measured at
-    // 6912 -> 2560: 128 / 192 / 256 tokens 15.7 / 15.7 / 17.9 us -> 12.1 / 13.2 / 14.6 us; from 320 tokens on, and at
-    // k = 2560 at any token count, the partial tiles cost more to exchange than the shorter loops save.
+    // 6912 -> 2560, quantiser included: 97 / 128 / 192 / 256 tokens 18.2 / 18.4 / 18.9 / 21.3 us -> 14.6 / 14.6 / 16.7 / 19.7;
+    // from 320 tokens on, and at k = 2560 at any token count, the partial tiles cost more to exchange than the shorter loops save.
     if (split && split->partials) {
         int nsplit = 0, st_per = 0;
         if (plan_split(m, k, tiles32, &nsplit, &st_per)) return launch_dma_split<64, 32, 4, 4>(p, nsplit, st_per, *split, stream);

@@ -26,10 +26,11 @@
 //   * up to three projections that share the input row (q, k, v or gate, up): the grid is the
 //     concatenation of their row blocks.
 // HBM traffic per call: n*k/4 weight bytes; the input row (K or 4K bytes per workgroup) comes from L2.
-// gemv_fused16_kernel is this launch with 16 wavefronts per workgroup (the default for one token; see its comment).
+// gemv_fused16_kernel is this launch with up to 16 wavefronts per workgroup (the default for one token; see its comment): there the
+// row reaches the MFMA by lane broadcasts, and the tiles are requested behind it.
 //
 // gemv_rows_kernel serves several tokens whose rows the quantiser laid out for it.  gemv_mfma_kernel is the same
-// weight-streaming scheme for 2..16 row-major token rows: the 16 x 16 x 64 int8 MFMA takes
+// weight-streaming scheme for 2..16 row-major token rows, which a caller brings or wants to see: the 16 x 16 x 64 int8 MFMA takes
 // the place of the dot-product chain (its A operand is 16 token rows x 64 columns, loaded straight from the
 // int8 activation matrix, which stays in L2; its B operand is a decoded weight dword, exactly as in the
 // prefill GEMM), so up to 16 tokens cost what one costs in weight traffic and instructions.  A workgroup
