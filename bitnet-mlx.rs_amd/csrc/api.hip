@@ -868,7 +868,6 @@ size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, c
                                             int sum_order)
 {
     if (!layer || m == 0) return 0;
-    const size_t in = layer->in_features;
     if (quantises_in_launch(&layer, 1, x, m, gamma, sum_order)) return 0;
     return bitnet_hip_bitlinear_workspace_size(layer, m);
 }
