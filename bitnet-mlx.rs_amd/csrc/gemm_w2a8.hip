@@ -27,7 +27,7 @@
 // The MFMA takes the weight fragment as its first operand, so a lane ends up with four consecutive output
 // columns of one token row and the epilogue stores 16 bytes per lane.  The epilogue's per-row operands (a_sum,
 // a_scale) arrive by LDS-direct loads in the stage buffer that is free during the last stage; the usual case
-// (f32 output only, n % 4 == 0, scales within the short division's range) is straight-line code
+// (f32 output only, scales within the short division's range) is straight-line code
 // (store_fragments_fast), everything else goes through store_fragments_general: same bits.
 //
 // gemm_ld8_kernel: the same data path with eight multiplying and two loading wavefronts per workgroup, for launches
@@ -291,15 +291,20 @@ __device__ __forceinline__ void fetch_row_operands(const GemmParams &p, int m0, 
     }
 }
 
-// The epilogue of one wavefront's fragments on the usual path: f32 output only, n % 4 == 0, w_scale and every
-// a_scale of the tile suited to the short division (the caller checks).  Straight-line code: per output element
-// a subtraction, a conversion, two multiplications, two FMAs and a sign copy; 16-byte stores, 128 contiguous bytes a row.
+// The epilogue of one wavefront's fragments on the usual path: f32 output only, w_scale and every a_scale of the tile suited to
+// the short division (the caller checks).  Straight-line code: per output element a subtraction,
+// a conversion, two multiplications, two FMAs and one and a half moves; 16-byte stores, 128 contiguous bytes a row.
+// The dividend is float(sum) * w_scale with w_scale > 0: a zero is +0, so the quotient's sign needs no care.
 // Fragment i of lane l holds token row rows[i], columns col0 + 16*j + 0..3.  FULL: the tile lies inside the
-// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.
+// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.  LINES: rows of the output begin at whole lines.
 // The stores are a quarter of a short-k launch (8192 x 2560 x 6912: 118 us of 153 without them), and the loads of the other
 // workgroups of the compute unit wait behind them: so they write whole 128-byte lines, non-temporal.  In 64-byte pieces 1024 x
 // 2560 x 6912 took 26.0 us (now 23.9), 2048 x 6912 x 2560 36.5 (34.8), 333 x 3328 x 8640 21.0 (19.5).
-template <int NI, int FN, bool FULL, bool EXTRA>
+// Rows that begin anywhere (n no multiple of 32) are written by the same 16-byte stores, which need four-byte alignment only, through
+// the cache, where the halves of a line that two stores share meet.  Such rows took 4-byte stores (n odd) or non-temporal ones:
+// 1566 x 256 -> 28790 110 us, now 46, -> 28796 119, now 45; 4000 x 1024 -> 5001 with residual 195, now 62; 439 x 384 -> 23272 27, now 17.
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+template <int NI, int FN, bool FULL, bool EXTRA, bool LINES>
 __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], const int (&rs)[NI], const float (&as)[NI],
                                                      const float (&rcp)[NI], float ws, const GemmProjDev &PJ, int m,
                                                      const int (&rows)[NI], int col0)
@@ -309,7 +314,8 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
     auto scaled4 = [&](const v4i &c, int i) {
         v4f v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = div_by_invariant_unchecked(f32_mul((float)(c[r] - rs[i]), ws), as[i], rcp[i]);
+        for (int r = 0; r < 4; ++r)
+            v[r] = div_by_invariant_unchecked<false>(f32_mul((float)(c[r] - rs[i]), ws), as[i], rcp[i]);
         return v;
     };
     // Store k of fragment row i, FN of them.  Fragments 32 columns apart by pairs (j, j + 1): lanes of rows 8..15 of j change places
@@ -322,7 +328,16 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
         const int second = (k - FIRST) & 1;
         *row = single ? rows[i] : rows[i] - (lr & 8) + 8 * second;
         *col = col0 + (single ? k : k - second + (hi ? 1 : 0)) * 16;
-        return FULL || (*row < m && *col < PJ.n);  // n % 4 == 0: a fragment row is inside or outside as a whole
+        return FULL || (*row < m && *col < PJ.n);
+    };
+    // Four values at src + 0..3, of which those past column n are not there.
+    auto get = [&](const float *src, int col) {
+        if (FULL || col + 4 <= PJ.n) return (v4f)*reinterpret_cast<const v4f_any *>(src);
+        v4f v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+            if (col + r < PJ.n) v[r] = src[r];
+        return v;
     };
     auto run = [&](auto is_odd) {
         constexpr int FIRST = decltype(is_odd)::value ? 1 : 0, PAIRED = (FN - FIRST) / 2 * 2;
@@ -336,7 +351,7 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
                 int row, col;
                 const bool inside = place(is_odd, i, k, &row, &col);
                 res[AHEAD ? i & 1 : 0][k] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-                if (inside) res[AHEAD ? i & 1 : 0][k] = *reinterpret_cast<const v4f *>(PJ.residual + (size_t)row * PJ.n + col);
+                if (inside) res[AHEAD ? i & 1 : 0][k] = get(PJ.residual + (size_t)row * PJ.n + col, col);
             }
         };
         if (AHEAD && EXTRA && PJ.residual) fetch(0);
@@ -350,10 +365,12 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
             for (int j = FIRST; j < FIRST + PAIRED; j += 2)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float a = v[j][r], b = v[j + 1][r];
-                    const int got = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, hi ? a : b), 0x128, 0xf, 0xf, true);
-                    v[j][r] = hi ? __builtin_bit_cast(float, got) : a;
-                    v[j + 1][r] = hi ? b : __builtin_bit_cast(float, got);
+                    // lanes 8..15 of a row of 16 take the partner's value of j + 1, lanes 0..7 the partner's value of j
+                    // (__builtin_bit_cast of a vector's element reads element 0 with this compiler: the elements go through floats)
+                    const float fa = v[j][r], fb = v[j + 1][r];
+                    const int a = __builtin_bit_cast(int, fa), b = __builtin_bit_cast(int, fb);
+                    v[j][r] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false));
+                    v[j + 1][r] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false));
                 }
 #pragma unroll
             for (int k = 0; k < FN; ++k) {
@@ -361,14 +378,21 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
                 if (!place(is_odd, i, k, &row, &col)) continue;
                 v4f y = v[k];
                 if (EXTRA && PJ.bias) {
-                    const v4f b = *reinterpret_cast<const v4f *>(PJ.bias + col);
+                    const v4f b = get(PJ.bias + col, col);
                     y = (v4f){f32_add(y[0], b[0]), f32_add(y[1], b[1]), f32_add(y[2], b[2]), f32_add(y[3], b[3])};
                 }
                 if (EXTRA && PJ.residual) {
                     const v4f q = res[AHEAD ? i & 1 : 0][k];
                     y = (v4f){f32_add(y[0], q[0]), f32_add(y[1], q[1]), f32_add(y[2], q[2]), f32_add(y[3], q[3])};
                 }
-                __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(PJ.out + (size_t)row * PJ.n + col));
+                float *dst = PJ.out + (size_t)row * PJ.n + col;
+                if (LINES) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
+                else if (FULL || col + 4 <= PJ.n) *reinterpret_cast<v4f_any *>(dst) = y;
+                else {
+#pragma unroll
+                    for (int r = 0; r < 3; ++r)
+                        if (col + r < PJ.n) dst[r] = y[r];
+                }
             }
         }
     };
@@ -376,7 +400,7 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
     else run(std::false_type{});
 }
 
-// The epilogue for every other case (int32 accumulator output, n % 4 != 0, scales outside the short division's
+// The epilogue for every other case (int32 accumulator output, scales outside the short division's
 // range): the same arithmetic, choices made per fragment row, a_sum and a_scale read from global memory.
 template <int NI, int FN>
 __device__ __forceinline__ void store_fragments_general(const v4i (&acc)[NI][FN], const int (&rows)[NI], int col0, float ws,
@@ -453,7 +477,7 @@ __device__ __forceinline__ void finish_fragments(const v4i (&acc)[NI][FN], const
     int rows[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) rows[i] = m0 + lrows[i];
-    if (PJ.out && !PJ.acc && (PJ.n & 3) == 0 && ws_fast) {
+    if (PJ.out && !PJ.acc && ws_fast) {
         const int *sum_l = reinterpret_cast<const int *>(rowp);
         const float *scale_l = reinterpret_cast<const float *>(rowp + BM * 4);
         int rs[NI];
@@ -468,10 +492,15 @@ __device__ __forceinline__ void finish_fragments(const v4i (&acc)[NI][FN], const
         }
         if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
             const bool extra = PJ.bias != nullptr || PJ.residual != nullptr;
-            if (full && !extra) store_fragments_fast<NI, FN, true, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-            else if (full) store_fragments_fast<NI, FN, true, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-            else if (!extra) store_fragments_fast<NI, FN, false, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-            else store_fragments_fast<NI, FN, false, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+            auto store = [&](auto lines) {
+                constexpr bool LINES = decltype(lines)::value;
+                if (full && !extra) store_fragments_fast<NI, FN, true, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else if (full) store_fragments_fast<NI, FN, true, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else if (!extra) store_fragments_fast<NI, FN, false, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else store_fragments_fast<NI, FN, false, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+            };
+            if ((PJ.n & 31) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0) store(std::true_type{});
+            else store(std::false_type{});
             return;
         }
     }

@@ -1720,3 +1720,22 @@ def test_decoder_blocks_of_two_to_eight_tokens_match_the_oracle(dims, m):
     dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
     x = synth_activations(rng, m, dims[0])
     assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
+
+
+@pytest.mark.parametrize("m,n,k", [(130, 45, 512), (300, 1001, 256), (1000, 2403, 512), (1000, 2564, 512), (700, 5030, 256), (2100, 6901, 256), (130, 643, 4096)])
+@pytest.mark.parametrize("extras", [False, True], ids=["plain", "bias_residual"])
+def test_gemm_rows_that_begin_inside_a_line(m, n, k, extras):
+    """Output widths that are no multiple of 32 floats, odd ones among them, through every LDS-direct kernel: the last group of four
+    columns cut, bias and residual read at any alignment.  Exact integers and single IEEE operations: the same bits."""
+    rng = np.random.default_rng(m + n)
+    x = synth_activations(rng, m, k, outliers=True)
+    pk = random_packed_ternary(rng, n, k)
+    bias = rng.standard_normal(n, dtype=f32) if extras else None
+    res = rng.standard_normal((m, n), dtype=f32) if extras else None
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=extras), "lines")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    if extras:
+        layer.update_bias(dev(bias))
+    got = host(layer.forward(dev(x), residual=dev(res) if extras else None))
+    ref = orc.bitlinear_forward(x, pk, n, f32(0.02), bias=bias, residual=res)[0]
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
