@@ -77,6 +77,7 @@ struct GemmParams {
     int m, n, k;
     int kt_count;   // 256-column weight tiles per row block
     int tiles_m, tiles_n;
+    int group_rows; // gemm_dma_kernel: row tiles that consecutive tiles go down before the next column (tile_position), 1 or more
     int rotate;     // gemm_dma_kernel: every workgroup of the launch is resident at once (see there)
     // gemm_dma_kernel<..., SPLIT = true>: k split across nsplit workgroups per output tile, st_per (even) stages each
     int nsplit, st_per;
@@ -538,10 +539,26 @@ __device__ __forceinline__ v4i load_shared4(const int *ptr)
     return *(gv4i *)(uintptr_t)ptr;
 }
 
-template <int BM, int BN, int D, int OCC, bool SPLIT = false>
+// Tile -> position.  Consecutive tiles run on one XCD at the same time.  Column by column of a row of tiles, they share one row
+// tile's activations in the XCD's L2 and sweep all of the weights for every row of tiles.  With p.group_rows they go down that many
+// row tiles before the next column, share those rows' activations and a few columns of weights, and the weights are swept once per group.
+// The rule (launch_dma): where the weights do not fit an L2 of 4 MiB, the group's activations do (3 MiB), and an XCD would sweep the weights three
+// times or more.  8192 x 2560 -> 6912 + 6912: loads alone 98 -> 75 us, the whole call 276 -> 264; 3402 x 1664 -> 11968 + 11968 151 -> 146.
+// Elsewhere it gains nothing or loses up to 3 % (4096 x 4096 -> 8192, 1531 x 2816 -> 27824: output rows in more, shorter pieces).
+constexpr int TILE_GROUP = 8;
+__device__ __forceinline__ void tile_position(const GemmParams &p, int tile_id, int *tm, int *tn)
+{
+    const int per = p.group_rows * p.tiles_n, group = tile_id / per, in = tile_id - group * per;
+    const int high = min(p.group_rows, p.tiles_m - group * p.group_rows);
+    *tn = in / high;
+    *tm = group * p.group_rows + in - *tn * high;
+}
+
+// WN: of the four wavefronts, how many lie side by side along n (2: 2 x 2, 4: 1 x 4).
+template <int BM, int BN, int D, int OCC, bool SPLIT = false, int WN = 2>
 __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
 {
-    constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
+    constexpr int WTM = BM * WN / 4, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
     constexpr int P = D - 1, NB = dma_nb<D>();
     constexpr int A_STAGE = BM * DMA_SK;
     constexpr int A_DMA = A_STAGE / 1024 / 4;  // LDS-direct loads per wavefront per activation stage
@@ -554,7 +571,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [D][A_STAGE] then [NB][B_STAGE]
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lg = lane >> 4;
+    const int wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
 
     int tile_id, ks = 0;
     {
@@ -567,7 +584,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
         if (SPLIT) { ks = tile_id % nsplit; tile_id /= nsplit; }  // the parts of a tile are neighbours: one XCD
     }
     // tiles_n counts the column tiles of all projections of the launch, one after the other
-    const int tm = tile_id / p.tiles_n, tn_all = tile_id % p.tiles_n;
+    int tm = tile_id / p.tiles_n, tn_all = tile_id - tm * p.tiles_n;
+    if (BM == 128 && p.group_rows > 1) tile_position(p, tile_id, &tm, &tn_all);
     int pj = 0;
     if (p.nproj > 1 && tn_all >= p.proj[0].tn_end) pj = 1;
     if (p.nproj > 2 && tn_all >= p.proj[1].tn_end) pj = 2;
@@ -733,7 +751,7 @@ hipError_t raise_lds_limit(Kernel kernel, size_t bytes)
     return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-template <int BM, int BN, int D, int OCC>
+template <int BM, int BN, int D, int OCC, int WN = 2>
 int launch_dma(GemmParams p, hipStream_t stream)
 {
     p.tiles_m = (p.m + BM - 1) / BM;
@@ -742,11 +760,13 @@ int launch_dma(GemmParams p, hipStream_t stream)
     const int total = p.tiles_m * p.tiles_n;
     const int grid = ((total + 7) / 8) * 8;
     p.rotate = total <= 256 * OCC && total > 256;
+    p.group_rows = BM == 128 && p.tiles_m >= 3 * 8 && (size_t)p.tiles_n * BN * p.k / 4 > (4u << 20) &&
+                           (size_t)TILE_GROUP * BM * p.k <= (3u << 20) ? TILE_GROUP : 1;
     constexpr size_t lds = dma_lds_bytes<BM, BN, D>();
     static_assert(lds <= 160 * 1024 && lds * OCC <= 160 * 1024 && OCC <= 4, "LDS budget, priorities 0..3");
-    static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC>, lds) : hipSuccess;
+    static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC, false, WN>, lds) : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC>), dim3(grid), dim3(256), lds, stream, p);
+    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC, false, WN>), dim3(grid), dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_dma_kernel");
     return BITNET_HIP_OK;
 }
@@ -778,7 +798,7 @@ int launch_dma_split(GemmParams p, int nsplit, int st_per, const GemmSplitScratc
     if (tiles * nsplit * BM * BN * sizeof(int32_t) > scratch.partial_bytes || tiles > scratch.counter_count)
         return fail(BITNET_HIP_MEMORY_ERROR, "split-k GEMM: scratch of %zu bytes / %zu counters for %zu tiles in %d parts",
                     scratch.partial_bytes, scratch.counter_count, tiles, nsplit);
-    p.nsplit = nsplit; p.st_per = st_per; p.rotate = 0;
+    p.nsplit = nsplit; p.st_per = st_per; p.rotate = 0; p.group_rows = 1;
     p.partials = scratch.partials; p.counters = scratch.counters;
     const int total = (int)tiles * nsplit;
     const int grid = ((total + 7) / 8) * 8;
@@ -1049,7 +1069,7 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     //   2.5 or more tiles per compute unit   -> 128 x 160, three workgroups of 4 wavefronts per compute unit, two
     //                                           activation stages each (more resident wavefronts beat deeper
     //                                           pipelines: 2.45 POP/s at 8192 x 2560 x 6912, against 2.23 with two
-    //                                           workgroups of three stages);
+    //                                           workgroups of three stages), or 128 x 256, two workgroups (below);
     //   0.4 to one tile per compute unit     -> 128 x 160, one workgroup of 8 multiplying wavefronts (k split inside it)
     //                                           and two loader wavefronts;
     //   otherwise                            -> 64 x 160, four workgroups of 4 wavefronts per compute unit.
@@ -1060,7 +1080,20 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
         int nsplit = 0, st_per = 0;
         if (plan_split(m, k, tiles32, &nsplit, &st_per)) return launch_dma_split<64, 32, 4, 4>(p, nsplit, st_per, *split, stream);
     }
-    if (tiles >= 640) return launch_dma<128, 160, 2, 3>(p, stream);
+    if (tiles >= 640) {
+        // 128 x 256 tiles as four wavefronts of 128 x 64 side by side, two workgroups per compute unit: half the unpacking per MFMA
+        // (a weight fragment serves eight token fragments instead of four) and a tenth fewer bytes loaded per output.  Per unit of work it takes
+        // 0.95 of the time of 128 x 160, so it is chosen where the outputs of the fullest compute unit leave that gain:
+        // 8192 x 2560 -> 6912 + 6912 280 -> 264 us, 4096 x 4096 -> 8192 132 -> 122, 3402 x 1664 -> 11968 + 11968 155 -> 146; not
+        // 8192 x 6912 -> 2560 (three tiles of 256 columns where four of 160 come out even: 190 against 180).
+        auto fullest = [&](size_t bn) {
+            size_t count = 0;
+            for (int j = 0; j < nproj; ++j) count += ((m + 127) / 128) * ((projs[j].n + bn - 1) / bn);
+            return (count + 255) / 256 * bn;
+        };
+        if (fullest(256) * 95 <= fullest(160) * 100) return launch_dma<128, 256, 2, 2, 4>(p, stream);
+        return launch_dma<128, 160, 2, 3>(p, stream);
+    }
     // Few tiles: a workgroup walks the whole of k by itself and its time is a chain of load latencies, so small
     // launches take narrow tiles (more workgroups, all resident at once) with four stages of loads in flight.
     // tiles64 / tiles32: 64 x 64 and 64 x 32 tiles of the launch.  Measured at 6912 -> 2560: 384 tokens 35.4 -> 23.3 us,

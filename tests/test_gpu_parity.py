@@ -1739,3 +1739,25 @@ def test_gemm_rows_that_begin_inside_a_line(m, n, k, extras):
     got = host(layer.forward(dev(x), residual=dev(res) if extras else None))
     ref = orc.bitlinear_forward(x, pk, n, f32(0.02), bias=bias, residual=res)[0]
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("m,n,k", [(3100, (6917, 3000), 512), (1030, (32768,), 256), (3073, (16385,), 1024), (3200, (4100, 4100, 33), 2048)])
+def test_gemm_128x256_tiles_and_grouped_rows(m, n, k):
+    """128 x 256 tiles (launches of 640 and more 128 x 160 tiles where they come out even), the last row and column tile cut, and the
+    walk down eight row tiles at a time (24 and more of them, weights above 4 MiB) with an incomplete last group: the same bits as the
+    oracle on rows at both ends, in the middle and on either side of a group, and as each layer by itself."""
+    rng = np.random.default_rng(m + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    layers, packs = [], []
+    for w in n:
+        packs.append(random_packed_ternary(rng, w, k))
+        layers.append(bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=w), "wide"))
+        layers[-1].set_quantized_weights(torch.from_numpy(packs[-1]), 0.02)
+    xd = dev(x)
+    outs = bh.forward_multi(layers, xd) if len(n) > 1 else [layers[0].forward(xd)]
+    rows = sorted({0, 1, 127, 128, 1023, 1024, m // 2, m - 1})
+    for w, pk, out in zip(n, packs, outs):
+        ref = orc.bitlinear_forward(x[rows], pk, w, f32(0.02))[0]
+        assert np.array_equal(host(out)[rows].view(np.uint32), ref.view(np.uint32))
+    single = layers[0].forward(xd[: m // 3].contiguous())
+    assert torch.equal(single, outs[0][: m // 3])
