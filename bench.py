@@ -306,9 +306,8 @@ def rotating_layers(bh, torch, dec, gen, proj):
 
 
 def short_prompt_forward(bh, torch, dec, gen):
-    """Short prompts on the long-k projection (6912 -> 2560 at 128 and 256 tokens): forward (quantiser + GEMM) with the
-    workspace forward asks for, which lets the GEMM split k across workgroups, and with one that holds the quantised
-    activations only (no split)."""
+    """Short prompts on the long-k projection (6912 -> 2560 at 128 and 256 tokens): forward (quantiser + GEMM) with a workspace
+    for the quantised activations."""
     out = {}
     n, k = dec.proj_shape(6)
     bls = rotating_layers(bh, torch, dec, gen, 6)
@@ -316,11 +315,8 @@ def short_prompt_forward(bh, torch, dec, gen):
         x = torch.randn((m, k), generator=gen, device="cuda", dtype=torch.float32)
         y = torch.empty((m, n), device="cuda", dtype=torch.float32)
         quant_only = (m * k + 255) // 256 * 256 + 2 * ((4 * m + 255) // 256 * 256) + 256
-        entry = {}
-        for label, size in (("us", bls[0].workspace_size(m)), ("us_without_k_split", quant_only)):
-            ws = torch.empty((size,), device="cuda", dtype=torch.uint8)
-            ms, how = time_forward_graph(torch, bls, x, y, ws)
-            entry[label] = round(ms * 1e3, 2)
+        ms, how = time_forward_graph(torch, bls, x, y, torch.empty((quant_only,), device="cuda", dtype=torch.uint8))
+        entry = {"us": round(ms * 1e3, 2)}
         entry["tops_incl_quantiser"] = round(2.0 * m * n * k / (entry["us"] * 1e-6) / 1e12, 1)
         entry["timed"] = how
         out[f"down_6912x2560_m{m}_forward"] = entry
@@ -520,7 +516,7 @@ def main():
                     help="run only the 32768 x 16384 one-token GEMV, on 2-bit tiles and on base-3 bytes, LOOPS times over four "
                          "matrices each (profiling runs)")
     ap.add_argument("--only-short-prompt", action="store_true",
-                    help="run only forward at 128 and 256 tokens on the 6912 -> 2560 projection, with and without the k split "
+                    help="run only forward at 128 and 256 tokens on the 6912 -> 2560 projection "
                          "(profiling runs)")
     ap.add_argument("--calibration-copy", action="store_true",
                     help="also run one plain 256 MiB device copy (a kernel of known traffic, to scale rocprofv3 "

@@ -26,18 +26,7 @@ struct ActQuantParams {
     size_t ldq;      // row stride of q: k, or more with the bytes from k on (up to the next multiple of 256) cleared
     int tiled;       // layout of q: see RowPlace
     int seq_in_lds;  // the launch carries LDS for the row's squares (literal summation order: sum_sequential_lds)
-    unsigned *zero;  // optional: zero[0 .. zero_n) is cleared by the first workgroup (counters of the launch that follows)
-    int zero_n;
 };
-
-// The clearing job: the threads of workgroup 0 (any block shape) write the zeros with vector stores.
-__device__ __forceinline__ void clear_counters(const ActQuantParams &p)
-{
-    if (blockIdx.x == 0 && p.zero) {
-        const int flat = threadIdx.y * blockDim.x + threadIdx.x, count = blockDim.x * blockDim.y;
-        for (int i = flat; i < p.zero_n; i += count) p.zero[i] = 0u;
-    }
-}
 
 constexpr size_t ROW_QUANT_MAX_ROWS = 512;
 
@@ -98,7 +87,6 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
     constexpr int NCH = 4;
     const RowSource &src = p.src;
     const int lane = threadIdx.x;
-    clear_counters(p);
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (row >= p.m) return;  // uniform per wavefront: a wavefront is one row
     const int chunks = (src.k + 3) >> 2;
@@ -155,7 +143,6 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
     __shared__ int red_i[4];
     const RowSource &src = p.src;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    clear_counters(p);
     const int k = src.k;
     const int chunks = (k + 3) >> 2;
     const int nloop = NCH > 0 ? NCH : (chunks + 255) >> 8;
@@ -254,11 +241,9 @@ struct RowQuantArgs {
     float *a_scale;
     int32_t *a_sum;
     float *y;
-    unsigned *zero;
-    int zero_n;
     int ldq;
     int tiled;
-    int unused[3];
+    int unused[6];
 };
 static_assert(sizeof(RowQuantArgs) == 64, "one scalar load");
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -288,9 +273,8 @@ __global__ __launch_bounds__(1024) void act_quant_row_kernel(const float *hot_x,
     const global_ptr<int8_t> q = pointer_at<int8_t>(block, 0);
     const global_ptr<float> a_scale = pointer_at<float>(block, 2), y = pointer_at<float>(block, 6);
     const global_ptr<int32_t> a_sum = pointer_at<int32_t>(block, 4);
-    const global_ptr<unsigned> zero = pointer_at<unsigned>(block, 8);
-    const int zero_n = (int)block[10], ldq = (int)block[11];
-    const RowPlace place = row_place(row, (size_t)hot_m, (size_t)ldq, block[12] != 0);
+    const int ldq = (int)block[8];
+    const RowPlace place = row_place(row, (size_t)hot_m, (size_t)ldq, block[9] != 0);
 
     uint32_t packed[NCHB];
     const float scale = row16.quantise(chunks, k_f, k_recip, hot_eps, wave, tid, red_f, packed);
@@ -303,8 +287,6 @@ __global__ __launch_bounds__(1024) void act_quant_row_kernel(const float *hot_x,
         sum = __builtin_amdgcn_sdot4((int)packed[i], 0x01010101, sum, false);
     }
     if (tid == 0) a_scale[row] = scale;
-    if (zero && row == 0)
-        for (int i = tid; i < zero_n; i += 64 * nw) zero[i] = 0u;
     if (a_sum) {
         sum = wave_sum_i32(sum);
         if ((tid & 63) == 0) atomicAdd(&sum_s, sum);
@@ -353,7 +335,7 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
             x2 = reinterpret_cast<const float *>(static_cast<uintptr_t>(magics));
         }
         if (in_range) {
-            const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, p.zero, p.zero_n, (int)p.ldq, p.tiled, {0, 0, 0}};
+            const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, (int)p.ldq, p.tiled, {0, 0, 0, 0, 0, 0}};
             const int kt = (p.src.k + 255) >> 8, nchb = kt > 16 ? 2 : 1;
             const int nw = nchb == 2 ? (kt + 1) / 2 : row_workgroup_waves(p.src.k);
             const dim3 grid((unsigned)p.m), block(64u * (unsigned)nw);
@@ -706,12 +688,11 @@ int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratc
 
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
-                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero, size_t zero_n, ActRows rows)
+                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, ActRows rows)
 {
     ActQuantParams p;
     p.tiled = rows == ActRows::TILES16;
     p.ldq = ldq;
-    p.zero = zero; p.zero_n = (int)zero_n;
     p.src.x = x; p.src.x2 = x2; p.src.gamma = gamma; p.src.ldx = ldx; p.src.k = (int)k;
     p.src.head_dim = (int)(head_dim ? head_dim : 1); p.src.gqa_group = (int)(gqa_group ? gqa_group : 1);
     p.src.sum_order = sum_order; p.src.eps = eps;

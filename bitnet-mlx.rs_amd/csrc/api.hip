@@ -167,7 +167,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
                     size_t m, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,
                     int sum_order, const float *const *residual, float *const *out, int32_t *const *acc, int8_t *q,
                     size_t ldq, float *a_scale, int32_t *a_sum, bool want_quant_outputs, hipStream_t s,
-                    const GemmSplitScratch *split = nullptr, bool alone = true)
+                    bool alone = true)
 {
     size_t k = layers[0]->in_features;
     const bool short_rows = !want_quant_outputs && gemv_rowq_takes(x, ldx, m, k, input_mode, gqa_group, head_dim, gamma, sum_order,
@@ -203,14 +203,10 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
     if (!q || !a_scale || !a_sum) return fail(BITNET_HIP_MEMORY_ERROR, "projection: no scratch for the quantised activations");
     size_t n_blocks = 0;
     for (int j = 0; j < count; ++j) n_blocks += row_blocks(layers[j]->out_features);
-    // A GEMM that splits k across workgroups finds its tile counters zeroed by the quantiser launched in front of it.  One
-    // scratch serves one launch: more projections than one launch takes run without the split.
-    const bool use_split = split && split->counters && count <= GEMM_MAX_PROJ && !gemv_takes(m, ldq, n_blocks, q);
     // Rows for the token GEMV go straight into the order that it reads, unless the caller wants to see them.
     const bool tiles = !want_quant_outputs && gemv_rows_takes(m, ldq, n_blocks, q);
     int rc = launch_act_quant(x, x2, ldx, m, k, input_mode, gqa_group, head_dim, gamma, eps, sum_order, q, ldq, a_scale, tiles ? nullptr : a_sum,
-                              nullptr, s, use_split ? split->counters : nullptr, use_split ? split->counter_count : 0,
-                              tiles ? ActRows::TILES16 : ActRows::ROW_MAJOR);
+                              nullptr, s, tiles ? ActRows::TILES16 : ActRows::ROW_MAJOR);
     if (rc != BITNET_HIP_OK) return rc;
     k = ldq;  // the columns past in_features are zero in the rows and in the tiles
     if (gemv_takes(m, k, n_blocks, q)) {
@@ -227,7 +223,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
         GemvProj pjs[GEMM_MAX_PROJ];
         const int nj = count - j0 < GEMM_MAX_PROJ ? count - j0 : GEMM_MAX_PROJ;
         for (int j = 0; j < nj; ++j) pjs[j] = proj_of(j0 + j);
-        rc = launch_gemm_multi(pjs, nj, q, a_sum, a_scale, m, k, s, use_split ? split : nullptr);  // all of them in one launch where that applies
+        rc = launch_gemm_multi(pjs, nj, q, a_sum, a_scale, m, k, s);  // all of them in one launch where that applies
         if (rc == BITNET_HIP_UNSUPPORTED) {
             for (int j = 0; j < nj; ++j) {
                 const GemvProj &pj = pjs[j];
@@ -259,22 +255,13 @@ QuantScratch carve_scratch(void *ws, size_t m, size_t k)
     return sc;
 }
 
-// Scratch of a GEMM that splits k across workgroups, behind the quantised activations in the same workspace.
-size_t split_scratch_bytes(size_t m, size_t k, size_t n)
+// What workspace_size counts beside the quantised activations for 97 to about 256 tokens on long rows.  A GEMM that split k across workgroups
+// kept its partial tiles and tile counters there; nothing reads it now.  The figure stays what callers have sized their buffers by.
+size_t reserved_bytes(size_t m, size_t k, size_t n)
 {
-    size_t partial_bytes = 0, counters = 0;
-    gemm_split_plan(m, k, &n, 1, &partial_bytes, &counters);
-    return partial_bytes ? partial_bytes + align_up(counters * sizeof(unsigned), 256) : 0;
-}
-GemmSplitScratch carve_split(void *ws, size_t m, size_t k, size_t n)
-{
-    GemmSplitScratch sp;
-    gemm_split_plan(m, k, &n, 1, &sp.partial_bytes, &sp.counter_count);
-    if (sp.partial_bytes == 0) return sp;
-    const uintptr_t base = align_up(reinterpret_cast<uintptr_t>(ws), 256) + quant_scratch_bytes(m, k) - 256;  // behind a_sum: quant_scratch_bytes counts 256 bytes of alignment slack
-    sp.partials = reinterpret_cast<int32_t *>(base);
-    sp.counters = reinterpret_cast<unsigned *>(base + sp.partial_bytes);
-    return sp;
+    const size_t tiles = (m + 63) / 64 * ((n + 31) / 32), stages = k / 128, per = ((stages + 2) / 3 + 1) & ~(size_t)1;
+    if (m <= 96 || k < 4096 || tiles == 0 || tiles > 352) return 0;
+    return align_up(tiles * ((stages + per - 1) / per) * 64 * 32 * sizeof(int32_t), 256) + align_up(tiles * sizeof(unsigned), 256);
 }
 
 }  // namespace
@@ -641,7 +628,7 @@ int bitnet_hip_matmul_w2a8(const uint8_t *tiled, const int8_t *a, const int32_t 
     if (reinterpret_cast<uintptr_t>(tiled) % 16)
         return fail(BITNET_HIP_INVALID_CONFIG, "matmul_w2a8: tiled weights must be 16-byte aligned");
     if (n > 0x7fffffffu || k > 0x7fffffffu) return fail(BITNET_HIP_UNSUPPORTED, "matmul_w2a8: dimension too large");
-    if (gemv_takes(m, k, row_blocks(n), a) || (!a_sum && m <= (size_t)GEMV_MAX_M)) {  // the GEMM that counts the rows' sums itself is slower
+    if (gemv_takes(m, k, row_blocks(n), a, a_sum != nullptr) || (!a_sum && m <= (size_t)GEMV_MAX_M)) {  // the GEMM that counts the rows' sums itself is slower
         GemvProj pj = {tiled, w_scale, bias, residual, out, acc, n};
         return launch_gemv_tiled(&pj, 1, a, a_scale, m, k, as_stream(stream));
     }
@@ -859,9 +846,8 @@ int bitnet_hip_bitlinear_get_quantized(bitnet_hip_bitlinear *layer, float *w_sca
 size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, size_t m)
 {
     if (!layer) return 0;
-    // the quantised activations, and the partial tiles of a GEMM that splits k across workgroups where one would run
     const size_t kp = padded_k(layer->in_features);
-    return quant_scratch_bytes(m, kp) + split_scratch_bytes(m, kp, layer->out_features);
+    return quant_scratch_bytes(m, kp) + reserved_bytes(m, kp, layer->out_features);
 }
 
 size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,
@@ -869,7 +855,7 @@ size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, c
 {
     if (!layer || m == 0) return 0;
     if (quantises_in_launch(&layer, 1, x, m, gamma, sum_order)) return 0;
-    return bitnet_hip_bitlinear_workspace_size(layer, m);
+    return quant_scratch_bytes(m, padded_k(layer->in_features));
 }
 
 size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
@@ -916,24 +902,19 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {dbg_q, dbg_a_scale, nullptr};
-    GemmSplitScratch split;
     size_t ldq = in;
     if (!fused || debug) {  // the fused decode launch needs no scratch unless the caller wants q / a_scale back
         const size_t least = quant_scratch_bytes(m, in);
         if (!dbg_q && (!ws || workspace_bytes >= quant_scratch_bytes(m, padded_k(in)))) ldq = padded_k(in);
-        const size_t need = quant_scratch_bytes(m, ldq), extra = split_scratch_bytes(m, ldq, layer->out_features);
-        bool with_split = extra != 0;
+        const size_t need = quant_scratch_bytes(m, ldq);
         if (!ws) {
-            hipError_t e = hipMallocAsync(&ws, need + extra, s);
-            if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward: hipMallocAsync(%zu) failed: %s", need + extra, hipGetErrorString(e));
+            hipError_t e = hipMallocAsync(&ws, need, s);
+            if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward: hipMallocAsync(%zu) failed: %s", need, hipGetErrorString(e));
             own_ws = true;
         } else if (workspace_bytes < least) {
             return fail(BITNET_HIP_MEMORY_ERROR, "forward: workspace of %zu bytes given, %zu needed", workspace_bytes, least);
-        } else if (workspace_bytes < need + extra) {
-            with_split = false;  // room for the quantised activations only: the GEMM walks k without the split
         }
         sc = carve_scratch(ws, m, ldq);
-        if (with_split) split = carve_split(ws, m, ldq, layer->out_features);
         if (dbg_q) sc.q = dbg_q;
         if (dbg_a_scale) sc.a_scale = dbg_a_scale;
     }
@@ -942,7 +923,7 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     float *outs[1] = {out};
     int32_t *accs[1] = {dbg_acc};
     int rc = run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, split.partials ? &split : nullptr);
+                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -1290,7 +1271,7 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
             const float *res[GEMV_MAX_PROJ] = {res0, nullptr, nullptr};
             rc = run_projections(layers, count, x, x2, ldx, rows, mode, group, dec->head_dim, gamma, dec->eps, dec->sum_order,
                                  res, outs, nullptr, dec->a8 + row0 * widest, padded_k(layers[0]->in_features), dec->a_scale + row0,
-                                 dec->a_sum + row0, false, cs, nullptr, false);
+                                 dec->a_sum + row0, false, cs, false);
         };
         float *qb = dec->qb + row0 * H, *kb = dec->kb + row0 * KV, *vb = dec->vb + row0 * KV, *x1 = dec->x1 + row0 * H;
         float *gate = dec->gate + row0 * F, *up = dec->up + row0 * F, *ping = dec->ping + row0 * H;

@@ -31,7 +31,7 @@
 // (store_fragments_fast), everything else goes through store_fragments_general: same bits.
 //
 // gemm_ld8_kernel: the same data path with eight multiplying and two loading wavefronts per workgroup, for launches
-// with at most one tile per compute unit (see its own comment).
+// that one round of workgroups holds (see its own comment).
 //
 // gemm_tiled_kernel (any shape, computes the row sums itself): activations pass through registers.
 // Activations are staged through LDS one weight tile (256 columns) at a time, double buffered: the global
@@ -49,6 +49,8 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte accesses need four-byte alignment only
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
 struct GemmProjDev {  // one projection of a launch of the LDS-direct kernels
     const uint8_t *w;
@@ -79,10 +81,6 @@ struct GemmParams {
     int tiles_m, tiles_n;
     int group_rows; // gemm_dma_kernel: row tiles that consecutive tiles go down before the next column (tile_position), 1 or more
     int rotate;     // gemm_dma_kernel: every workgroup of the launch is resident at once (see there)
-    // gemm_dma_kernel<..., SPLIT = true>: k split across nsplit workgroups per output tile, st_per (even) stages each
-    int nsplit, st_per;
-    int *partials;        // [tile][part][fragment][thread] int4
-    unsigned *counters;   // one per output tile, zero at launch; the last workgroup of a tile leaves it zero again
 };
 
 constexpr int STAGE_K = 256;              // columns per pipeline stage = one weight tile
@@ -297,18 +295,17 @@ __device__ __forceinline__ void fetch_row_operands(const GemmParams &p, int m0, 
 // a conversion, two multiplications, two FMAs and one and a half moves; 16-byte stores, 128 contiguous bytes a row.
 // The dividend is float(sum) * w_scale with w_scale > 0: a zero is +0, so the quotient's sign needs no care.
 // Fragment i of lane l holds token row rows[i], columns col0 + 16*j + 0..3.  FULL: the tile lies inside the
-// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.  LINES: rows of the output begin at whole lines.
+// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.  lines: rows of the output begin at whole lines.
 // The stores are a quarter of a short-k launch (8192 x 2560 x 6912: 118 us of 153 without them), and the loads of the other
 // workgroups of the compute unit wait behind them: so they write whole 128-byte lines, non-temporal.  In 64-byte pieces 1024 x
 // 2560 x 6912 took 26.0 us (now 23.9), 2048 x 6912 x 2560 36.5 (34.8), 333 x 3328 x 8640 21.0 (19.5).
 // Rows that begin anywhere (n no multiple of 32) are written by the same 16-byte stores, which need four-byte alignment only, through
 // the cache, where the halves of a line that two stores share meet.  Such rows took 4-byte stores (n odd) or non-temporal ones:
 // 1566 x 256 -> 28790 110 us, now 46, -> 28796 119, now 45; 4000 x 1024 -> 5001 with residual 195, now 62; 439 x 384 -> 23272 27, now 17.
-typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
-template <int NI, int FN, bool FULL, bool EXTRA, bool LINES>
+template <int NI, int FN, bool FULL, bool EXTRA>
 __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], const int (&rs)[NI], const float (&as)[NI],
                                                      const float (&rcp)[NI], float ws, const GemmProjDev &PJ, int m,
-                                                     const int (&rows)[NI], int col0)
+                                                     const int (&rows)[NI], int col0, bool lines)
 {
     const int lr = threadIdx.x & 15;
     const bool hi = lr >= 8;
@@ -387,7 +384,7 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
                     y = (v4f){f32_add(y[0], q[0]), f32_add(y[1], q[1]), f32_add(y[2], q[2]), f32_add(y[3], q[3])};
                 }
                 float *dst = PJ.out + (size_t)row * PJ.n + col;
-                if (LINES) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
+                if (FULL && lines) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
                 else if (FULL || col + 4 <= PJ.n) *reinterpret_cast<v4f_any *>(dst) = y;
                 else {
 #pragma unroll
@@ -493,19 +490,110 @@ __device__ __forceinline__ void finish_fragments(const v4i (&acc)[NI][FN], const
         }
         if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
             const bool extra = PJ.bias != nullptr || PJ.residual != nullptr;
-            auto store = [&](auto lines) {
-                constexpr bool LINES = decltype(lines)::value;
-                if (full && !extra) store_fragments_fast<NI, FN, true, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-                else if (full) store_fragments_fast<NI, FN, true, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-                else if (!extra) store_fragments_fast<NI, FN, false, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-                else store_fragments_fast<NI, FN, false, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
-            };
-            if ((PJ.n & 31) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0) store(std::true_type{});
-            else store(std::false_type{});
+            const bool lines = (PJ.n & 31) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0;
+            if (full && !extra) store_fragments_fast<NI, FN, true, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
+            else if (full) store_fragments_fast<NI, FN, true, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
+            else if (!extra) store_fragments_fast<NI, FN, false, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
+            else store_fragments_fast<NI, FN, false, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
             return;
         }
     }
     store_fragments_general<NI, FN>(acc, rows, col0, ws, ws_fast, PJ, p);
+}
+
+// The epilogue by way of LDS, for gemm_ld8_kernel: the workgroup's int32 tile (COPIES partial tiles of different parts of k, added here) is
+// laid down row by row and read back in output order, RP rows at a time.  put(pass) writes this wavefront's fragments of rows RP * pass
+// .. into the area; rowp is the LDS copy of the tile's a_sum and a_scale (outside the area).  Every thread of the workgroup
+// comes here, after a barrier behind the last use of the area; loaders and multipliers store alike.  Against exchanging halves and the
+// epilogue in registers (finish_fragments) a few hundred instructions instead of up to ten thousand that a wavefront runs through
+// once, whole rows of the tile per store at any n, and the residuals of a pass requested ahead of the barrier: 333 x 3328 -> 8640 with bias,
+// 128 x 160 tiles, 24.4 -> 23.6 us.  Non-temporal where a row begins at 16 bytes (128 x 2560 -> 30000: 20.1 us, through the cache 22.1).
+// PITCH: ints per row, padded so that the rows a store instruction touches start in different banks.
+template <int BN>
+constexpr int tile_pitch() { return BN + 4; }
+template <int BN, int COPIES, int RP>
+constexpr size_t tile_area_bytes() { return (size_t)COPIES * RP * tile_pitch<BN>() * 4; }
+
+template <int BM, int BN, int COPIES, int RP, int THREADS, typename Put>
+__device__ __forceinline__ void store_tile(uint8_t *area, const uint8_t *rowp, int m0, int n0, const GemmProjDev &PJ, const GemmParams &p,
+                                           Put put)
+{
+    constexpr int PITCH = tile_pitch<BN>(), QUADS = BN / 4, PER = (RP * QUADS + THREADS - 1) / THREADS;
+    const int *tile = reinterpret_cast<const int *>(area);
+    const int *sum_l = reinterpret_cast<const int *>(rowp);
+    const float *scale_l = reinterpret_cast<const float *>(rowp + BM * 4);
+    const float ws = PJ.out ? *PJ.w_scale : 0.0f;
+    const unsigned ws_expo = (__builtin_bit_cast(unsigned, ws) >> 23) & 0xffu;
+    const bool ws_fast = ws > 0.0f && ws_expo > 64u && ws_expo < 160u;
+    const bool stream = (PJ.n & 3) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int pass = 0; pass < (BM + RP - 1) / RP; ++pass) {
+        if (pass) __syncthreads();  // the pass before has been read
+        put(pass);
+        v4f res[PER];
+        if (PJ.residual) {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const int at = tid + q * THREADS, r = at / QUADS, col = n0 + (at - r * QUADS) * 4, row = m0 + pass * RP + r;
+                res[q] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+                if (r >= RP || row >= p.m || col >= PJ.n) continue;
+                const float *src = PJ.residual + (size_t)row * PJ.n + col;
+                if (col + 4 <= PJ.n) res[q] = *reinterpret_cast<const v4f_any *>(src);
+                else
+                    for (int c = 0; c < 3; ++c)
+                        if (col + c < PJ.n) res[q][c] = src[c];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int at = tid + q * THREADS, r = at / QUADS, quad = at - r * QUADS, col = n0 + quad * 4, lrow = pass * RP + r, row = m0 + lrow;
+            if (r >= RP || row >= p.m || col >= PJ.n) continue;
+            v4i total = *reinterpret_cast<const v4i *>(tile + r * PITCH + quad * 4);
+#pragma unroll
+            for (int c = 1; c < COPIES; ++c) total += *reinterpret_cast<const v4i *>(tile + (c * RP + r) * PITCH + quad * 4);
+            total -= sum_l[lrow];
+            const size_t o = (size_t)row * PJ.n + col;
+            const bool whole = col + 4 <= PJ.n;
+            if (PJ.acc) {
+                if (whole) *reinterpret_cast<v4i_any *>(PJ.acc + o) = total;
+                else
+                    for (int c = 0; c < 3; ++c)
+                        if (col + c < PJ.n) PJ.acc[o + c] = total[c];
+            }
+            if (!PJ.out) continue;
+            const float as = scale_l[lrow];
+            v4f y;
+            // the short division where w_scale and the rows' scales allow it, chosen per wavefront; float(sum) * w_scale of a zero is +0
+            if (ws_fast && __builtin_amdgcn_ballot_w64(!invariant_divisor_ok(as)) == 0) {
+                const float rcp = recip_of_ok_divisor(as);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) y[c] = div_by_invariant_unchecked<false>(f32_mul((float)total[c], ws), as, rcp);
+            } else {
+                for (int c = 0; c < 4; ++c) y[c] = f32_div(f32_mul((float)total[c], ws), as);
+            }
+            if (PJ.bias) {
+                v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (whole) b = *reinterpret_cast<const v4f_any *>(PJ.bias + col);
+                else
+                    for (int c = 0; c < 3; ++c)
+                        if (col + c < PJ.n) b[c] = PJ.bias[col + c];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) y[c] = f32_add(y[c], b[c]);
+            }
+            if (PJ.residual) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) y[c] = f32_add(y[c], res[q][c]);
+            }
+            float *dst = PJ.out + o;
+            if (stream) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
+            else if (whole) *reinterpret_cast<v4f_any *>(dst) = y;
+            else
+                for (int c = 0; c < 3; ++c)
+                    if (col + c < PJ.n) dst[c] = y[c];
+        }
+    }
 }
 
 constexpr int DMA_SK = 128;  // columns per activation stage; a 256-column weight tile serves two stages
@@ -526,19 +614,6 @@ constexpr int dma_in_flight()
     return n;
 }
 
-// Four ints exchanged between workgroups inside one launch: device-scope (relaxed atomic) stores and loads, which the
-// hardware writes through to, and reads from, the level every XCD shares, 8 bytes at a time.
-__device__ __forceinline__ void store_shared4(int *ptr, v4i v)
-{
-    typedef volatile __attribute__((address_space(1))) v4i gv4i;
-    *(gv4i *)(uintptr_t)ptr = v;
-}
-__device__ __forceinline__ v4i load_shared4(const int *ptr)
-{
-    typedef const volatile __attribute__((address_space(1))) v4i gv4i;
-    return *(gv4i *)(uintptr_t)ptr;
-}
-
 // Tile -> position.  Consecutive tiles run on one XCD at the same time.  Column by column of a row of tiles, they share one row
 // tile's activations in the XCD's L2 and sweep all of the weights for every row of tiles.  With p.group_rows they go down that many
 // row tiles before the next column, share those rows' activations and a few columns of weights, and the weights are swept once per group.
@@ -555,7 +630,7 @@ __device__ __forceinline__ void tile_position(const GemmParams &p, int tile_id, 
 }
 
 // WN: of the four wavefronts, how many lie side by side along n (2: 2 x 2, 4: 1 x 4).
-template <int BM, int BN, int D, int OCC, bool SPLIT = false, int WN = 2>
+template <int BM, int BN, int D, int OCC, int WN = 2>
 __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
 {
     constexpr int WTM = BM * WN / 4, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
@@ -573,15 +648,13 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
 
-    int tile_id, ks = 0;
+    int tile_id;
     {
-        const int nsplit = SPLIT ? p.nsplit : 1;
-        const int total = p.tiles_m * p.tiles_n * nsplit;
+        const int total = p.tiles_m * p.tiles_n;
         const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
         const int per_xcd = (total + 7) >> 3;
         tile_id = xcd * per_xcd + idx;
         if (tile_id >= total) return;
-        if (SPLIT) { ks = tile_id % nsplit; tile_id /= nsplit; }  // the parts of a tile are neighbours: one XCD
     }
     // tiles_n counts the column tiles of all projections of the launch, one after the other
     int tm = tile_id / p.tiles_n, tn_all = tile_id - tm * p.tiles_n;
@@ -592,8 +665,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
     const GemmProjDev PJ = p.proj[pj];  // uniform over the workgroup
     const int tn = tn_all - (pj ? p.proj[pj - 1].tn_end : 0);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int s_first = SPLIT ? __builtin_amdgcn_readfirstlane(ks * p.st_per) : 0;  // even
-    const int nstage = SPLIT ? min(p.st_per, p.kt_count * 2 - s_first) : p.kt_count * 2;  // stages of this workgroup (even)
+    const int nstage = p.kt_count * 2;
 
     // Activation loads: load q of this wavefront covers tile rows 8*(wave*A_DMA + q) .. +7; lane l lands in
     // row l/8 at physical 16-byte chunk l%8 and therefore fetches logical chunk (l%8) ^ (row & 7).
@@ -626,11 +698,11 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
             const int kt = s >> 1;
             const uint32_t dst = lds_base + D * A_STAGE + (kt % NB) * B_STAGE;
 #pragma unroll
-            for (int q = 0; q < B_DMA; ++q) dma16(PJ.w + (size_t)(kt + (s_first >> 1)) * 1024, b_off[q], dst + b_dst[q]);
+            for (int q = 0; q < B_DMA; ++q) dma16(PJ.w + (size_t)kt * 1024, b_off[q], dst + b_dst[q]);
         }
         const uint32_t dst = lds_base + (s % D) * A_STAGE + wave * A_DMA * 1024;
 #pragma unroll
-        for (int q = 0; q < A_DMA; ++q) dma16(p.a + (size_t)(s + s_first) * DMA_SK, a_off[q], dst + q * 1024);
+        for (int q = 0; q < A_DMA; ++q) dma16(p.a + (size_t)s * DMA_SK, a_off[q], dst + q * 1024);
     };
 
     v4i acc[FM][FN];
@@ -707,36 +779,6 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
     static_assert(rowp_bytes<BM>() <= A_STAGE, "row operands fit an activation stage");
     wait_vm<0>();
     __syncthreads();
-    if constexpr (SPLIT) {
-        // Every part stores its int32 fragments (device-scope stores: written through to where every XCD reads them),
-        // waits until they have been acknowledged, and draws a ticket from the tile's counter; the part that draws the
-        // last one adds up all parts (integers: any order, same sum), leaves the counter at zero and runs the epilogue.
-        // Nobody waits for anybody.
-        __shared__ int last_ticket;
-        constexpr int SLAB = FM * FN * 256 * 4;
-        int *mine = p.partials + ((size_t)tile_id * p.nsplit + ks) * SLAB;
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) store_shared4(mine + ((i * FN + j) * 256 + tid) * 4, acc[i][j]);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (tid == 0)
-            last_ticket = __hip_atomic_fetch_add(&p.counters[tile_id], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(p.nsplit - 1);
-        __syncthreads();
-        if (!last_ticket) return;  // uniform over the workgroup
-        if (tid == 0) __hip_atomic_store(&p.counters[tile_id], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int *slab = p.partials + (size_t)tile_id * p.nsplit * SLAB;
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = (v4i){0, 0, 0, 0};
-        for (int part = 0; part < p.nsplit; ++part, slab += SLAB)
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] += load_shared4(slab + ((i * FN + j) * 256 + tid) * 4);
-    }
     int lrows[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) lrows[i] = wm * WTM + i * 16 + lr;
@@ -764,56 +806,45 @@ int launch_dma(GemmParams p, hipStream_t stream)
                            (size_t)TILE_GROUP * BM * p.k <= (3u << 20) ? TILE_GROUP : 1;
     constexpr size_t lds = dma_lds_bytes<BM, BN, D>();
     static_assert(lds <= 160 * 1024 && lds * OCC <= 160 * 1024 && OCC <= 4, "LDS budget, priorities 0..3");
-    static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC, false, WN>, lds) : hipSuccess;
+    static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC, WN>, lds) : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC, false, WN>), dim3(grid), dim3(256), lds, stream, p);
+    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC, WN>), dim3(grid), dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_dma_kernel");
     return BITNET_HIP_OK;
 }
 
 // ---- eight MFMA wavefronts per workgroup fed by two loader wavefronts -------------------------------------------
 //
-// For launches with at most one 128 x 160 tile per compute unit.  One wavefront per SIMD cannot keep the MFMA pipe
+// For launches that one round of workgroups holds.  One wavefront per SIMD cannot keep the MFMA pipe
 // busy (its own LDS waits and unpack instructions sit between its MFMAs); two can.  With too few tiles for two
 // workgroups per compute unit the second wavefront per SIMD comes from inside the workgroup: wavefronts 0..3 take
 // columns 0..127 of every 256-column stage and wavefronts 4..7 columns 128..255, each group accumulating the whole
-// BM x BN tile; the two partial tiles are exchanged through LDS at the end (int32 sums: exact), each group
-// finishing half of the fragments.  A stage is one 256-column weight tile plus BM x 256 activation bytes, three
-// stages in LDS, loads two stages ahead.
+// BM x BN tile; the two partial tiles are added in the epilogue (int32 sums: exact).  A stage is one 256-column weight
+// tile plus BM x 256 activation bytes, NST stages in LDS, loads NST - 1 stages ahead (more than three gain nothing).
 // The LDS-direct loads are issued by two further wavefronts (8 and 9) that never multiply.  A wavefront that issues
 // a load while the queue of the load path is full waits at that instruction, and while it waits it issues no MFMA;
 // with the loads spread over the multiplying wavefronts every one of them paid that wait every stage (measured at
 // 2048 x 2560 x 6912: 40.8 us with the loads on the eight wavefronts, 33.6 us with no loads in the loop at all,
 // 35.8 us with the two loaders).  The multiplying wavefronts meet the loaders at the stage barrier and otherwise
 // only read LDS and run MFMAs.
-constexpr int LD8_NST = 3;
-// The same kernel with k split across nsplit workgroups per output tile (st_per stages each; see the kernel's SPLIT branch).
-template <int BM, int BN, int D, int OCC>
-int launch_dma_split(GemmParams p, int nsplit, int st_per, const GemmSplitScratch &scratch, hipStream_t stream)
+// Which tile: choose_ld8.  In place of four-wavefront workgroups of 64 x 32 and 64 x 64 with four stages in flight, and of k split across
+// workgroups (us, quantiser included): 128 x 6912 -> 2560 15.0 -> 12.6, 213 x 13120 -> 3008 36.6 -> 26.2, 378 x 6656 -> 3264 24.5 -> 19.9, 640 x
+// 6912 -> 2560 28.9 -> 23.3, 2100 x 13952 -> 768 65.7 -> 53, 110 x 8192 -> 14336 29 -> 22.6; of 128 x 160 alone 300 x 8192 -> 8192 37.0 -> 33.7.
+// Four multiplying wavefronts of 128 x 80 with their fragments read a half step ahead, and the fragments of the next stage read before the
+// barrier, were measured and are not faster: per compute unit the loop is bound by LDS reads and MFMAs together.
+// Waits until at most `groups` groups of G loads each, MAX at most, are in flight.
+template <int G, int MAX>
+__device__ __forceinline__ void wait_groups(int groups)
 {
-    p.tiles_m = (p.m + BM - 1) / BM;
-    p.tiles_n = 0;
-    for (int j = 0; j < p.nproj; ++j) p.proj[j].tn_end = p.tiles_n += (p.proj[j].n + BN - 1) / BN;
-    const size_t tiles = (size_t)p.tiles_m * p.tiles_n;
-    if (tiles * nsplit * BM * BN * sizeof(int32_t) > scratch.partial_bytes || tiles > scratch.counter_count)
-        return fail(BITNET_HIP_MEMORY_ERROR, "split-k GEMM: scratch of %zu bytes / %zu counters for %zu tiles in %d parts",
-                    scratch.partial_bytes, scratch.counter_count, tiles, nsplit);
-    p.nsplit = nsplit; p.st_per = st_per; p.rotate = 0; p.group_rows = 1;
-    p.partials = scratch.partials; p.counters = scratch.counters;
-    const int total = (int)tiles * nsplit;
-    const int grid = ((total + 7) / 8) * 8;
-    constexpr size_t lds = dma_lds_bytes<BM, BN, D>();
-    static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC, true>, lds) : hipSuccess;
-    BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC, true>), dim3(grid), dim3(256), lds, stream, p);
-    BITNET_HIP_CHECK_LAUNCH("gemm_dma_kernel (k split)");
-    return BITNET_HIP_OK;
+    if constexpr (MAX == 0) wait_vm<0>();
+    else if (groups >= MAX) wait_vm<MAX * G>();
+    else wait_groups<G, MAX - 1>(groups);
 }
 
-template <int BM, int BN>
-constexpr size_t ld8_lds_bytes() { return (size_t)LD8_NST * (BM * 256 + (BN / 16) * 1024) + rowp_bytes<BM>(); }
+template <int BM, int BN, int NST>
+constexpr size_t ld8_lds_bytes() { return (size_t)NST * (BM * 256 + (BN / 16) * 1024) + rowp_bytes<BM>(); }
 
-template <int BM, int BN>
+template <int BM, int BN, int NST>
 __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
 {
     constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
@@ -824,8 +855,8 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
     constexpr int STAGE = A_STAGE + B_STAGE;
     constexpr int A_PER = A_CHUNKS / 2, B_PER = (B_TILES + 1) / 2;  // per loader wavefront
     constexpr int GROUP = A_PER + B_PER;
-    static_assert(A_CHUNKS % 2 == 0 && WTM % 32 == 0 && WTN % 16 == 0 && 2 * GROUP < 64, "tile shape, vmcnt range");
-    static_assert((FM / 2) * FN * 4 * 256 * 8 <= LD8_NST * STAGE, "exchange area");
+    static_assert(A_CHUNKS % 2 == 0 && WTM % 32 == 0 && WTN % 16 == 0 && (NST - 1) * GROUP < 64, "tile shape, vmcnt range");
+    static_assert(tile_area_bytes<BN, 2, WTM>() <= (size_t)NST * STAGE, "epilogue area");
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [NST][A half 0 | A half 1 | B], then the row operands
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
@@ -846,7 +877,7 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
     const GemmProjDev PJ = p.proj[pj];  // uniform over the workgroup
     const int tn = tn_all - (pj ? p.proj[pj - 1].tn_end : 0);
     const int m0 = tm * BM, n0 = tn * BN;
-    constexpr uint32_t ROWP = LD8_NST * STAGE;
+    constexpr uint32_t ROWP = NST * STAGE;
 
     if (wave >= 8) {
         // ---- loader wavefront L: activation chunks A_PER*L .. and weight tiles B_PER*L .. of every stage ----
@@ -872,7 +903,7 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
             b_dst[q] = A_STAGE + tix * 1024;
         }
         auto issue = [&](int kt) {
-            const uint32_t stage = lds_base + (kt % LD8_NST) * STAGE;
+            const uint32_t stage = lds_base + (kt % NST) * STAGE;
 #pragma unroll
             for (int q = 0; q < B_PER; ++q) dma16(PJ.w + (size_t)kt * 1024, b_off[q], stage + b_dst[q]);
 #pragma unroll
@@ -886,15 +917,16 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
             if (L == 0) dma4(p.a_sum, (uint32_t)grow * 4u, lds_base + ROWP + ch * 256);
             else if (p.a_scale) dma4(p.a_scale, (uint32_t)grow * 4u, lds_base + ROWP + BM * 4 + ch * 256);
         }
-        issue(0);
-        if (p.kt_count > 1) issue(1);
+#pragma unroll
+        for (int kt = 0; kt < NST - 1; ++kt)
+            if (kt < p.kt_count) issue(kt);
         for (int kt = 0; kt < p.kt_count; ++kt) {
-            if (kt + 1 < p.kt_count) wait_vm<GROUP>(); else wait_vm<0>();
+            wait_groups<GROUP, NST - 2>(p.kt_count - 1 - kt);
             __syncthreads();
-            if (kt + 2 < p.kt_count) issue(kt + 2);
+            if (kt + NST - 1 < p.kt_count) issue(kt + NST - 1);  // into the buffer of stage kt - 1, which nobody reads any more
         }
-        __syncthreads();  // the two barriers of the exchange
-        __syncthreads();
+        __syncthreads();  // every wavefront is done with the stage buffers
+        store_tile<BM, BN, 2, WTM, 640>(lds, lds + ROWP, m0, n0, PJ, p, [](int) {});
         return;
     }
 
@@ -910,7 +942,7 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
     const int sw = lr & 7;
 
     auto compute = [&](int kt) {
-        const uint8_t *abuf = lds + (kt % LD8_NST) * STAGE;
+        const uint8_t *abuf = lds + (kt % NST) * STAGE;
         const uint8_t *bbuf = abuf + A_STAGE + (wn * FN) * 1024 + lane * 16 + kg * 8;
         uint2 bp[FN];  // dwords 2*kg, 2*kg+1 of the slot: this group's two k-steps
 #pragma unroll
@@ -940,38 +972,18 @@ __global__ __launch_bounds__(640, 1) void gemm_ld8_kernel(GemmParams p)
         compute(kt);
     }
 
-    // ---- exchange: group 0 finishes fragments i < FM/2, group 1 the others ----
     __syncthreads();  // every wavefront is done with the stage buffers
-    constexpr int HALF = FM / 2;
-    {
-        v4i *xch = reinterpret_cast<v4i *>(lds);
-        const int mine = wave, partner = wave ^ 4;
+    store_tile<BM, BN, 2, WTM, 640>(lds, lds + ROWP, m0, n0, PJ, p, [&](int pass) {
+        if (pass != wm) return;
+        int *at = reinterpret_cast<int *>(lds) + (kg * WTM + lr) * tile_pitch<BN>() + wn * WTN + lg * 4;
 #pragma unroll
-        for (int i = 0; i < HALF; ++i)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                xch[((mine * HALF + i) * FN + j) * 64 + lane] = acc[kg == 0 ? i + HALF : i][j];
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < HALF; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const v4i o = xch[((partner * HALF + i) * FN + j) * 64 + lane];
-                if (kg == 0) acc[i][j] += o; else acc[i + HALF][j] += o;
-            }
-    }
-    v4i fin[HALF][FN];
-    int lrows[HALF];
-#pragma unroll
-    for (int ii = 0; ii < HALF; ++ii) {
-        lrows[ii] = wm * WTM + (ii + kg * HALF) * 16 + lr;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) fin[ii][j] = kg == 0 ? acc[ii][j] : acc[ii + HALF][j];
-    }
-    finish_fragments<BM, HALF, FN>(fin, lrows, m0, n0 + wn * WTN + lg * 4, m0 + BM <= p.m && n0 + BN <= PJ.n, lds + ROWP, PJ, p);
+            for (int j = 0; j < FN; ++j) *reinterpret_cast<v4i *>(at + i * 16 * tile_pitch<BN>() + j * 16) = acc[i][j];
+    });
 }
 
-template <int BM, int BN>
+template <int BM, int BN, int NST>
 int launch_ld8(GemmParams p, hipStream_t stream)
 {
     p.tiles_m = (p.m + BM - 1) / BM;
@@ -979,13 +991,41 @@ int launch_ld8(GemmParams p, hipStream_t stream)
     for (int j = 0; j < p.nproj; ++j) p.proj[j].tn_end = p.tiles_n += (p.proj[j].n + BN - 1) / BN;
     const int total = p.tiles_m * p.tiles_n;
     const int grid = ((total + 7) / 8) * 8;
-    constexpr size_t lds = ld8_lds_bytes<BM, BN>();
+    constexpr size_t lds = ld8_lds_bytes<BM, BN, NST>();
     static_assert(lds <= 160 * 1024, "LDS budget");
-    static const hipError_t attr = raise_lds_limit(&gemm_ld8_kernel<BM, BN>, lds);
+    static const hipError_t attr = raise_lds_limit(&gemm_ld8_kernel<BM, BN, NST>, lds);
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_ld8_kernel<BM, BN>), dim3(grid), dim3(640), lds, stream, p);
+    hipLaunchKernelGGL((gemm_ld8_kernel<BM, BN, NST>), dim3(grid), dim3(640), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_ld8_kernel");
     return BITNET_HIP_OK;
+}
+
+// The tiles of gemm_ld8_kernel, with what a stage of 256 columns costs a compute unit in each (ns: the slope over k at few
+// workgroups; the smaller ones are bound by LDS reads per MFMA, the larger ones by unpacking and MFMA).
+struct Ld8Tile {
+    int bm, bn, stage_ns;
+    int per_cu;  // workgroups that a compute unit holds (LDS)
+    int (*launch)(GemmParams, hipStream_t);
+};
+const Ld8Tile LD8_TILES[] = {
+    {64, 32, 140, 2, &launch_ld8<64, 32, 4>},     {64, 64, 250, 2, &launch_ld8<64, 64, 3>},    {64, 96, 330, 2, &launch_ld8<64, 96, 3>},
+    {128, 64, 400, 1, &launch_ld8<128, 64, 3>},   {64, 128, 430, 2, &launch_ld8<64, 128, 3>},  {128, 96, 560, 1, &launch_ld8<128, 96, 3>},
+    {128, 128, 720, 1, &launch_ld8<128, 128, 3>}, {128, 160, 880, 1, &launch_ld8<128, 160, 3>},
+};
+// The tile with which a stage takes least among those that need one round of workgroups: what the fullest compute unit multiplies, or
+// what all of them load at the 24 TB/s that the L2s together give; null: none needs one round.  n: output widths.
+const Ld8Tile *choose_ld8(size_t m, const size_t *n, int nproj, size_t *stage_ns)
+{
+    const Ld8Tile *best = nullptr;
+    for (const Ld8Tile &t : LD8_TILES) {
+        size_t count = 0;
+        for (int j = 0; j < nproj; ++j) count += ((m + t.bm - 1) / t.bm) * ((n[j] + t.bn - 1) / t.bn);
+        const size_t here = (count + 255) / 256, bytes = (size_t)t.bm * 256 + t.bn * 64;
+        if (here > (size_t)t.per_cu) continue;
+        const size_t multiply = here * t.stage_ns, load = count * bytes / 24000, cost = multiply > load ? multiply : load;
+        if (!best || cost < *stage_ns) { best = &t; *stage_ns = cost; }
+    }
+    return best;
 }
 
 template <int BM, int BN>
@@ -1005,45 +1045,24 @@ int launch_tile(GemmParams p, hipStream_t stream)
 
 }  // namespace
 
+size_t gemm_one_round_ns(size_t m, size_t k, size_t n)
+{
+    size_t stage_ns = 0;
+    return choose_ld8(m, &n, 1, &stage_ns) ? GEMM_START_NS + stage_ns * (k / TILE_K) * 11 / 10 : 0;
+}
+
 // Up to GEMM_MAX_PROJ projections of the same activation matrix in one launch of the LDS-direct kernels (q, k, v
 // or gate, up at prefill: small projections alone would leave most compute units idle).  Returns
 // BITNET_HIP_UNSUPPORTED (without a message) when the shapes do not fit those kernels.
-namespace {
-// k split across workgroups: where, and into how many parts of how many 128-column stages (even).  tiles32: 64 x 32
-// tiles of the launch.  One round of workgroups at four per compute unit holds 1024: three parts of at most 352 tiles.
-bool plan_split(size_t m, size_t k, size_t tiles32, int *nsplit, int *st_per)
-{
-    if (m <= 96 || k < 4096 || k % 256 != 0 || tiles32 == 0 || tiles32 > 352) return false;
-    const int nstage = (int)(k / 128);
-    const int per = ((nstage + 2) / 3 + 1) & ~1;
-    const int parts = (nstage + per - 1) / per;
-    if (parts < 2) return false;
-    *nsplit = parts; *st_per = per;
-    return true;
-}
-}  // namespace
-
-void gemm_split_plan(size_t m, size_t k, const size_t *n, int nproj, size_t *partial_bytes, size_t *counters)
-{
-    *partial_bytes = 0; *counters = 0;
-    if (nproj <= 0 || nproj > GEMM_MAX_PROJ) return;
-    size_t tiles32 = 0;
-    for (int j = 0; j < nproj; ++j) tiles32 += ((m + 63) / 64) * ((n[j] + 31) / 32);
-    int nsplit = 0, st_per = 0;
-    if (!plan_split(m, k, tiles32, &nsplit, &st_per)) return;
-    *partial_bytes = (tiles32 * nsplit * 64 * 32 * sizeof(int32_t) + 255) / 256 * 256;
-    *counters = tiles32;
-}
-
 int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const int32_t *a_sum, const float *a_scale,
-                      size_t m, size_t k, hipStream_t stream, const GemmSplitScratch *split)
+                      size_t m, size_t k, hipStream_t stream)
 {
     if (m == 0 || nproj <= 0) return BITNET_HIP_OK;
     if (nproj > GEMM_MAX_PROJ) return BITNET_HIP_UNSUPPORTED;
     // One k-tile is enough for the LDS-direct kernels (two load stages: their prologue issues what there is); the eight-wavefront
     // one wants two.  Through the register-staged kernel 1151 x 256 -> 1024 + 1024 took 37.9 us, now 10.5; 334 x 256 -> 2700
     // with residual 24.7, now 9.6.
-    bool dma_ok = a_sum != nullptr && m > 32 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
+    bool dma_ok = a_sum != nullptr && m > 16 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
                   m * k < (1ull << 32);  // 32-bit lane offsets
     size_t tiles = 0, tiles128 = 0, tiles64 = 0, tiles32 = 0;  // 128 x 160 tiles; 128 x 128 tiles, or 0 if a projection is not a multiple of 128 wide
     bool all128 = true;
@@ -1064,21 +1083,13 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     if (!all128) tiles128 = 0;
     for (int j = nproj; j < GEMM_MAX_PROJ; ++j) p.proj[j] = p.proj[nproj - 1];
     p.nproj = nproj; p.a = a; p.a_sum = a_sum; p.a_scale = a_scale; p.m = (int)m; p.k = (int)k; p.kt_count = (int)k_tiles(k);
-    // Three shapes of the LDS-direct kernel, chosen by how many 128 x 160 tiles the outputs hold (256 compute
-    // units; the MFMA pipe of a SIMD needs two or more resident wavefronts to stay busy).  Measured:
-    //   2.5 or more tiles per compute unit   -> 128 x 160, three workgroups of 4 wavefronts per compute unit, two
-    //                                           activation stages each (more resident wavefronts beat deeper
-    //                                           pipelines: 2.45 POP/s at 8192 x 2560 x 6912, against 2.23 with two
-    //                                           workgroups of three stages), or 128 x 256, two workgroups (below);
-    //   0.4 to one tile per compute unit     -> 128 x 160, one workgroup of 8 multiplying wavefronts (k split inside it)
-    //                                           and two loader wavefronts;
-    //   otherwise                            -> 64 x 160, four workgroups of 4 wavefronts per compute unit.
-    // A long k with few tiles: the 64 x 32 tiles of the launch in three parts of k each (plan_split).  Measured at
-    // 6912 -> 2560, quantiser included: 97 / 128 / 192 / 256 tokens 18.2 / 18.4 / 18.9 / 21.3 us -> 14.6 / 14.6 / 16.7 / 19.7;
-    // from 320 tokens on, and at k = 2560 at any token count, the partial tiles cost more to exchange than the shorter loops save.
-    if (split && split->partials) {
-        int nsplit = 0, st_per = 0;
-        if (plan_split(m, k, tiles32, &nsplit, &st_per)) return launch_dma_split<64, 32, 4, 4>(p, nsplit, st_per, *split, stream);
+    // gemm_ld8_kernel where one round of its workgroups holds the launch (256 compute units); with less than four stages its start and
+    // epilogue cost more than the shorter loop saves (1000 x 512 -> 2560: 11.0 us, 9.6 with the kernels below).
+    if (k >= 1024) {
+        size_t widths[GEMM_MAX_PROJ], stage_ns = 0;
+        for (int j = 0; j < nproj; ++j) widths[j] = projs[j].n;
+        const Ld8Tile *tile = choose_ld8(m, widths, nproj, &stage_ns);
+        if (tile) return tile->launch(p, stream);
     }
     if (tiles >= 640) {
         // 128 x 256 tiles as four wavefronts of 128 x 64 side by side, two workgroups per compute unit: half the unpacking per MFMA
@@ -1094,14 +1105,10 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
         if (fullest(256) * 95 <= fullest(160) * 100) return launch_dma<128, 256, 2, 2, 4>(p, stream);
         return launch_dma<128, 160, 2, 3>(p, stream);
     }
-    // Few tiles: a workgroup walks the whole of k by itself and its time is a chain of load latencies, so small
-    // launches take narrow tiles (more workgroups, all resident at once) with four stages of loads in flight.
-    // tiles64 / tiles32: 64 x 64 and 64 x 32 tiles of the launch.  Measured at 6912 -> 2560: 384 tokens 35.4 -> 23.3 us,
-    // 512 tokens 36.6 -> 25.8 us (64 x 32), 768 tokens 38.0 -> 29.6 us, 1024 tokens 36.8 -> 34.3 us (64 x 64);
-    // 2560 -> 6912 at 192 tokens 17.5 -> 13.6 us, at 384 tokens 20.0 -> 17.7 us.
+    // Short rows with few tiles: narrow tiles (more workgroups, all resident at once), four stages of loads in flight, four or three
+    // workgroups per compute unit.  tiles64 / tiles32: 64 x 64 and 64 x 32 tiles of the launch.
     if (tiles < 100 && tiles32 <= 704) return launch_dma<64, 32, 4, 4>(p, stream);
     if (tiles <= 140 && tiles64 <= 768) return launch_dma<64, 64, 4, 3>(p, stream);
-    if (tiles >= 100 && tiles <= 256 && k >= 512) return launch_ld8<128, 160>(p, stream);
     // between one and 2.5 tiles of 128 x 160 per compute unit: 128 x 128 tiles when they divide every projection and
     // fill the 768 workgroup slots almost three times (q + k + v at 3072 tokens: 33.0 us against 37.9 us with 64 x 160)
     if (tiles > 256 && tiles128 >= 640) return launch_dma<128, 128, 2, 3>(p, stream);

@@ -21,8 +21,7 @@ inline size_t tiled_bytes(size_t n, size_t k) { return row_blocks(n) * k_tiles(k
 enum class ActRows { ROW_MAJOR, TILES16 };
 int launch_act_quant(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,
                      size_t gqa_group, size_t head_dim, const float *gamma, float eps, int sum_order,
-                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, unsigned *zero = nullptr,
-                     size_t zero_n = 0, ActRows rows = ActRows::ROW_MAJOR);  // zero[0 .. zero_n): cleared by the launch (tile counters of the GEMM behind it)
+                     int8_t *q, size_t ldq, float *a_scale, int32_t *a_sum, float *y, hipStream_t stream, ActRows rows = ActRows::ROW_MAJOR);
 // ldq: row stride of q, k or padded_k(k).  Padded rows end in zeros, so the contraction may take padded_k(k) for k: its weight
 // tiles are padded with zero weights, and every width then has the aligned rows the LDS-direct and the batched kernels need.
 inline size_t padded_k(size_t k) { return (k + TILE_K - 1) / TILE_K * TILE_K; }
@@ -100,8 +99,29 @@ inline bool gemm_takes_tokens(size_t m, size_t k, size_t n_blocks, const void *a
     return m > 32 && wgs >= 800 && (tiles32 <= 704 || (wgs >= 1500 && k >= 1536)) && k % TILE_K == 0 && n_blocks * k < (1ull << 29) &&
            (reinterpret_cast<uintptr_t>(a) & 15) == 0;
 }
-inline bool gemv_takes(size_t m, size_t k, size_t n_blocks, const void *a)
+// From 17 tokens on, where one round of gemm_ld8_kernel holds the launch, the two are compared by what they take (ns).  The GEMM: its
+// start and epilogue, and its stages (gemm_one_round_ns).  The token GEMV: its start, and per 16-row block and group of 16 tokens the
+// exchange of the partial results (by wavefronts, up to 16: one per k-tile) and the k-tiles beyond.  Both fitted to kernel times over 10 widths, 10 to
+// 192 tokens, within 20 %; the GEMM's start with 1.5 us on top, what weights that come from HBM cost it more than the GEMV, which asks for
+// all of its tiles at once (blocks of a decoder, each with its own weights, at 18 and 24 tokens of 3072 -> 18048 and 2304 -> 18176).  GEMV / GEMM, quantiser included, in us: 2560 -> 13824 at 32 / 42 / 95 10.1 / 10.6, 12.1 / 11.0, 21.6 / 12.2; 4096 -> 12288
+// at 20 / 42 / 95 12.1 / 12.0, 17.2 / 12.2, 24.3 / 17.6; 8192 -> 8192 at 32 / 42 / 95 11.3 / 15.7, 19.0 / 17.3, 23.6 / 18.2; 2560 -> 30000 at
+// 16 / 20 / 48 10.5 / 12.7, 17.8 / 12.5, 23.6 / 14.5; 6912 -> 2560 at 95 / 112 11.1 / 12.3, 15.7 / 12.5; 2560 -> 2560 at 95 / 192 8.1 / 9.3, 10.5 / 10.3.
+size_t gemm_one_round_ns(size_t m, size_t k, size_t n);  // gemm_w2a8.hip; 0 where no tile of that kernel holds the launch in one round
+constexpr size_t GEMM_START_NS = 6500, GEMM_LEAST_STAGE_NS = 154;
+inline bool gemm_beats_token_gemv(size_t m, size_t k, size_t n_blocks, const void *a)
 {
+    if (m <= 16 || m > (size_t)GEMV_WIDE_MAX_M || k < 1024 || k % TILE_K != 0 || n_blocks * k >= (1ull << 29) || (reinterpret_cast<uintptr_t>(a) & 15) != 0)
+        return false;
+    const size_t kt = k / TILE_K, blocks = n_blocks * ((m + 15) / 16), near = blocks * (kt < 16 ? kt : 16), all = blocks * kt;
+    const size_t gemv_ns = 3300 + near / 4 + (all - near) / 8 + (m > 64 ? 1000 : 0);
+    if (gemv_ns <= GEMM_START_NS + GEMM_LEAST_STAGE_NS * kt) return false;
+    const size_t gemm_ns = gemm_one_round_ns(m, k, n_blocks * 16);
+    return gemm_ns != 0 && gemm_ns < gemv_ns;
+}
+// sums: the caller has the rows' sums, without which the GEMM takes a slower kernel
+inline bool gemv_takes(size_t m, size_t k, size_t n_blocks, const void *a, bool sums = true)
+{
+    if (sums && gemm_beats_token_gemv(m, k, n_blocks, a)) return false;
     if (m <= (size_t)GEMV_MAX_M) return !gemm_takes_tokens(m, k, n_blocks, a);
     if (m > (size_t)GEMV_WIDE_MAX_M || k % 256 != 0 || k > 8192 || (reinterpret_cast<uintptr_t>(a) & 15) != 0) return false;
     const size_t tgroups = (m + 15) / 16, slots = k <= 3072 ? 768 : 256;
@@ -151,19 +171,8 @@ int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const fl
 // gemm_w2a8.hip
 constexpr int GEMM_MAX_PROJ = 3;  // projections sharing one activation matrix per launch of the LDS-direct kernels
 // several projections in one launch; BITNET_HIP_UNSUPPORTED (no message) if the LDS-direct kernels do not apply
-// Scratch of a GEMM launch that splits k across workgroups (gemm_split_plan): int32 partial tiles, and one counter per
-// output tile that MUST be zero when the launch starts (the activation quantiser in front of the GEMM zeroes them:
-// launch_act_quant's zero / zero_n) and is zero again when it ends.  Both belong to the caller's workspace.
-struct GemmSplitScratch {
-    int32_t *partials = nullptr;
-    unsigned *counters = nullptr;
-    size_t partial_bytes = 0, counter_count = 0;
-};
-// What launch_gemm_multi needs to split k for this launch: bytes of partials (a multiple of 256) and the number of
-// counters; both 0 when it would not split.  n: output widths of the projections that share the launch.
-void gemm_split_plan(size_t m, size_t k, const size_t *n, int nproj, size_t *partial_bytes, size_t *counters);
 int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const int32_t *a_sum, const float *a_scale,
-                      size_t m, size_t k, hipStream_t stream, const GemmSplitScratch *split = nullptr);
+                      size_t m, size_t k, hipStream_t stream);
 // a_sum (sum_k a[t, k] per row, from the activation quantiser) may be NULL: the slower kernel then computes it
 int launch_gemm_tiled(const uint8_t *tiled, const int8_t *a, const int32_t *a_sum, size_t m, size_t n, size_t k,
                       int32_t *acc, const float *w_scale, const float *a_scale, const float *bias,

@@ -1761,3 +1761,21 @@ def test_gemm_128x256_tiles_and_grouped_rows(m, n, k):
         assert np.array_equal(host(out)[rows].view(np.uint32), ref.view(np.uint32))
     single = layers[0].forward(xd[: m // 3].contiguous())
     assert torch.equal(single, outs[0][: m // 3])
+
+
+@pytest.mark.parametrize("k", [1024, 1280, 2816])
+@pytest.mark.parametrize("m,n", [(17, 30000), (64, 33), (65, 4100), (130, 1100), (200, 3000), (257, 6000), (333, 8192), (500, 3073), (700, 6500), (1025, 2500),
+                                 (2040, 2560)])
+def test_gemm_tiles_of_one_round_bit_exact(m, n, k):
+    """Launches that one round of the loader-fed workgroups holds: every tile of its table (64 x 32 to 128 x 160, one or two workgroups per
+    compute unit), first and last rows and columns cut, four to eleven stages; int32 and f32 output through matmul, f32 through forward."""
+    rng = np.random.default_rng(m + n + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    pk = random_packed_ternary(rng, n, k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "round")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    ref, q, a_scale, acc_ref = orc.bitlinear_forward(x, pk, n, f32(0.02))
+    assert np.array_equal(host(layer.forward(dev(x))).view(np.uint32), ref.view(np.uint32))
+    acc, out = bh.matmul_w2a8(bh.retile_weights(dev(pk), n, k), dev(q), n, dev(np.array([0.02], dtype=f32)), dev(a_scale),
+                              a_sum=dev(q.astype(np.int32).sum(axis=1).astype(np.int32)))
+    assert np.array_equal(host(acc), acc_ref) and np.array_equal(host(out).view(np.uint32), ref.view(np.uint32))
