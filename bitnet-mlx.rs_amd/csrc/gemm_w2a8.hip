@@ -295,17 +295,17 @@ __device__ __forceinline__ void fetch_row_operands(const GemmParams &p, int m0, 
 // a conversion, two multiplications, two FMAs and one and a half moves; 16-byte stores, 128 contiguous bytes a row.
 // The dividend is float(sum) * w_scale with w_scale > 0: a zero is +0, so the quotient's sign needs no care.
 // Fragment i of lane l holds token row rows[i], columns col0 + 16*j + 0..3.  FULL: the tile lies inside the
-// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.  lines: rows of the output begin at whole lines.
+// matrix, no bounds checks.  EXTRA: bias and / or residual may be present.  LINES: rows of the output begin at whole lines.
 // The stores are a quarter of a short-k launch (8192 x 2560 x 6912: 118 us of 153 without them), and the loads of the other
 // workgroups of the compute unit wait behind them: so they write whole 128-byte lines, non-temporal.  In 64-byte pieces 1024 x
 // 2560 x 6912 took 26.0 us (now 23.9), 2048 x 6912 x 2560 36.5 (34.8), 333 x 3328 x 8640 21.0 (19.5).
 // Rows that begin anywhere (n no multiple of 32) are written by the same 16-byte stores, which need four-byte alignment only, through
 // the cache, where the halves of a line that two stores share meet.  Such rows took 4-byte stores (n odd) or non-temporal ones:
 // 1566 x 256 -> 28790 110 us, now 46, -> 28796 119, now 45; 4000 x 1024 -> 5001 with residual 195, now 62; 439 x 384 -> 23272 27, now 17.
-template <int NI, int FN, bool FULL, bool EXTRA>
+template <int NI, int FN, bool FULL, bool EXTRA, bool LINES>
 __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], const int (&rs)[NI], const float (&as)[NI],
                                                      const float (&rcp)[NI], float ws, const GemmProjDev &PJ, int m,
-                                                     const int (&rows)[NI], int col0, bool lines)
+                                                     const int (&rows)[NI], int col0)
 {
     const int lr = threadIdx.x & 15;
     const bool hi = lr >= 8;
@@ -384,7 +384,7 @@ __device__ __forceinline__ void store_fragments_fast(const v4i (&acc)[NI][FN], c
                     y = (v4f){f32_add(y[0], q[0]), f32_add(y[1], q[1]), f32_add(y[2], q[2]), f32_add(y[3], q[3])};
                 }
                 float *dst = PJ.out + (size_t)row * PJ.n + col;
-                if (FULL && lines) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
+                if (LINES) __builtin_nontemporal_store(y, reinterpret_cast<v4f *>(dst));
                 else if (FULL || col + 4 <= PJ.n) *reinterpret_cast<v4f_any *>(dst) = y;
                 else {
 #pragma unroll
@@ -490,11 +490,16 @@ __device__ __forceinline__ void finish_fragments(const v4i (&acc)[NI][FN], const
         }
         if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
             const bool extra = PJ.bias != nullptr || PJ.residual != nullptr;
-            const bool lines = (PJ.n & 31) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0;
-            if (full && !extra) store_fragments_fast<NI, FN, true, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
-            else if (full) store_fragments_fast<NI, FN, true, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
-            else if (!extra) store_fragments_fast<NI, FN, false, false>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
-            else store_fragments_fast<NI, FN, false, true>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0, lines);
+            // (a run-time choice in place of this one costs the loop of 128 x 160 tiles spilled registers: 10 % of the kernel)
+            auto store = [&](auto lines) {
+                constexpr bool LINES = decltype(lines)::value;
+                if (full && !extra) store_fragments_fast<NI, FN, true, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else if (full) store_fragments_fast<NI, FN, true, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else if (!extra) store_fragments_fast<NI, FN, false, false, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+                else store_fragments_fast<NI, FN, false, true, LINES>(acc, rs, as, rcp, ws, PJ, p.m, rows, col0);
+            };
+            if ((PJ.n & 31) == 0 && (reinterpret_cast<uintptr_t>(PJ.out) & 15) == 0) store(std::true_type{});
+            else store(std::false_type{});
             return;
         }
     }
@@ -635,6 +640,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
 {
     constexpr int WTM = BM * WN / 4, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
     constexpr int P = D - 1, NB = dma_nb<D>();
+    constexpr bool GROUPS = BM == 128 && BN == 256;  // 128 x 160 tiles spill registers with it
     constexpr int A_STAGE = BM * DMA_SK;
     constexpr int A_DMA = A_STAGE / 1024 / 4;  // LDS-direct loads per wavefront per activation stage
     constexpr int B_TILES = BN / 16;           // weight tiles per 256 columns
@@ -646,7 +652,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // [D][A_STAGE] then [NB][B_STAGE]
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
+    const int wm = WN == 2 ? wave >> 1 : 0, wn = WN == 2 ? wave & 1 : wave, lr = lane & 15, lg = lane >> 4;
 
     int tile_id;
     {
@@ -657,8 +663,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_dma_kernel(GemmParams p)
         if (tile_id >= total) return;
     }
     // tiles_n counts the column tiles of all projections of the launch, one after the other
-    int tm = tile_id / p.tiles_n, tn_all = tile_id - tm * p.tiles_n;
-    if (BM == 128 && p.group_rows > 1) tile_position(p, tile_id, &tm, &tn_all);
+    int tm = tile_id / p.tiles_n, tn_all = tile_id % p.tiles_n;
+    if (GROUPS && p.group_rows > 1) tile_position(p, tile_id, &tm, &tn_all);
     int pj = 0;
     if (p.nproj > 1 && tn_all >= p.proj[0].tn_end) pj = 1;
     if (p.nproj > 2 && tn_all >= p.proj[1].tn_end) pj = 2;
@@ -802,7 +808,7 @@ int launch_dma(GemmParams p, hipStream_t stream)
     const int total = p.tiles_m * p.tiles_n;
     const int grid = ((total + 7) / 8) * 8;
     p.rotate = total <= 256 * OCC && total > 256;
-    p.group_rows = BM == 128 && p.tiles_m >= 3 * 8 && (size_t)p.tiles_n * BN * p.k / 4 > (4u << 20) &&
+    p.group_rows = BM == 128 && BN == 256 && p.tiles_m >= 3 * 8 && (size_t)p.tiles_n * BN * p.k / 4 > (4u << 20) &&
                            (size_t)TILE_GROUP * BM * p.k <= (3u << 20) ? TILE_GROUP : 1;
     constexpr size_t lds = dma_lds_bytes<BM, BN, D>();
     static_assert(lds <= 160 * 1024 && lds * OCC <= 160 * 1024 && OCC <= 4, "LDS budget, priorities 0..3");
