@@ -1070,23 +1070,19 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     // with residual 24.7, now 9.6.
     bool dma_ok = a_sum != nullptr && m > 16 && k % 256 == 0 && k > 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
                   m * k < (1ull << 32);  // 32-bit lane offsets
-    size_t tiles = 0, tiles128 = 0, tiles64 = 0, tiles32 = 0;  // 128 x 160 tiles; 128 x 128 tiles, or 0 if a projection is not a multiple of 128 wide
-    bool all128 = true;
+    size_t tiles = 0, tiles64 = 0, tiles32 = 0;  // 128 x 160, 64 x 64 and 64 x 32 tiles of the launch
     GemmParams p = {};
     for (int j = 0; j < nproj && dma_ok; ++j) {
         const GemvProj &s = projs[j];
         dma_ok = s.n > 0 && s.n <= 0x7fffffffu && tiled_bytes(s.n, k) < (1ull << 32);
         tiles += ((m + 127) / 128) * ((s.n + 159) / 160);
-        tiles128 += ((m + 127) / 128) * ((s.n + 127) / 128);
         tiles64 += ((m + 63) / 64) * ((s.n + 63) / 64);
         tiles32 += ((m + 63) / 64) * ((s.n + 31) / 32);
-        all128 = all128 && s.n % 128 == 0;
         GemmProjDev &d = p.proj[j];
         d.w = s.tiled; d.w_scale = s.w_scale; d.bias = s.bias; d.residual = s.residual; d.out = s.out; d.acc = s.acc;
         d.n = (int)s.n; d.tn_end = 0;
     }
     if (!dma_ok) return BITNET_HIP_UNSUPPORTED;
-    if (!all128) tiles128 = 0;
     for (int j = nproj; j < GEMM_MAX_PROJ; ++j) p.proj[j] = p.proj[nproj - 1];
     p.nproj = nproj; p.a = a; p.a_sum = a_sum; p.a_scale = a_scale; p.m = (int)m; p.k = (int)k; p.kt_count = (int)k_tiles(k);
     // gemm_ld8_kernel where one round of its workgroups holds the launch (256 compute units); with less than four stages its start and
@@ -1112,13 +1108,26 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
         return launch_dma<128, 160, 2, 3>(p, stream);
     }
     // Short rows with few tiles: narrow tiles (more workgroups, all resident at once), four stages of loads in flight, four or three
-    // workgroups per compute unit.  tiles64 / tiles32: 64 x 64 and 64 x 32 tiles of the launch.
+    // workgroups per compute unit.
     if (tiles < 100 && tiles32 <= 704) return launch_dma<64, 32, 4, 4>(p, stream);
     if (tiles <= 140 && tiles64 <= 768) return launch_dma<64, 64, 4, 3>(p, stream);
-    // between one and 2.5 tiles of 128 x 160 per compute unit: 128 x 128 tiles when they divide every projection and
-    // fill the 768 workgroup slots almost three times (q + k + v at 3072 tokens: 33.0 us against 37.9 us with 64 x 160)
-    if (tiles > 256 && tiles128 >= 640) return launch_dma<128, 128, 2, 3>(p, stream);
-    return launch_dma<64, 160, 2, 4>(p, stream);
+    // Between one round of loader-fed tiles and 2.5 tiles of 128 x 160 per compute unit: whatever leaves the fullest compute unit least, in
+    // outputs, weighted by what an output costs (64 x 160, two by two wavefronts, unpacks once for two token fragments instead of four and
+    // takes a fifth longer; launches beyond one round of workgroups start over).  In place of 64 x 160 and 128 x 128 (us, quantiser included):
+    // 1024 x 4096 -> 8192 44.1 -> 38.7, 1500 x 8192 -> 4096 62.5 -> 54.5, 1566 x 2560 -> 5000 32.2 -> 28.8, 512 x 4096 -> 14336 38.0 -> 35.1, 6000 x
+    // 1024 -> 1024 21.4 -> 20.0, 1200 x 4096 -> 4096 31.9 -> 30.2, 2600 x 6912 -> 2560 61.0 -> 58.4.
+    struct Shape { size_t bm, bn, slots, cost; int (*launch)(GemmParams, hipStream_t); };
+    static const Shape shapes[] = {{64, 128, 1024, 100, &launch_dma<64, 128, 2, 4, 4>}, {64, 256, 768, 100, &launch_dma<64, 256, 2, 3, 4>},
+                                   {128, 128, 768, 100, &launch_dma<128, 128, 2, 3>},   {64, 160, 1024, 121, &launch_dma<64, 160, 2, 4>}};
+    const Shape *best = nullptr;
+    size_t least = 0;
+    for (const Shape &t : shapes) {
+        size_t count = 0;
+        for (int j = 0; j < nproj; ++j) count += ((m + t.bm - 1) / t.bm) * ((projs[j].n + t.bn - 1) / t.bn);
+        const size_t cost = (count + 255) / 256 * t.bm * t.bn * t.cost * (count > t.slots ? 5 : 4);
+        if (!best || cost < least) { best = &t; least = cost; }
+    }
+    return best->launch(p, stream);
 }
 
 int launch_gemm_tiled(const uint8_t *tiled, const int8_t *a, const int32_t *a_sum, size_t m, size_t n, size_t k,

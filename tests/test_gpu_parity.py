@@ -1779,3 +1779,23 @@ def test_gemm_tiles_of_one_round_bit_exact(m, n, k):
     acc, out = bh.matmul_w2a8(bh.retile_weights(dev(pk), n, k), dev(q), n, dev(np.array([0.02], dtype=f32)), dev(a_scale),
                               a_sum=dev(q.astype(np.int32).sum(axis=1).astype(np.int32)))
     assert np.array_equal(host(acc), acc_ref) and np.array_equal(host(out).view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("m,ns,k", [(1030, (6913,), 256), (1200, (4096,), 512), (800, (13830,), 256), (3072, (2560, 640, 640), 256), (2048, (5120,), 256), (65, (30000,), 768)])
+def test_gemm_launches_between_one_round_and_many_tiles(m, ns, k):
+    """64 x 128, 64 x 256, 128 x 128 and 64 x 160 tiles: launches that no single round of the loader-fed workgroups holds, with fewer than
+    640 tiles of 128 x 160; several projections, tiles cut by rows and columns, one to three weight tiles a row."""
+    rng = np.random.default_rng(m + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    packs = [random_packed_ternary(rng, n, k) for n in ns]
+    layers = []
+    for n, pk in zip(ns, packs):
+        layers.append(bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "between"))
+        layers[-1].set_quantized_weights(torch.from_numpy(pk), 0.02)
+    xd = dev(x)
+    outs = bh.forward_multi(layers, xd) if len(ns) > 1 else [layers[0].forward(xd)]
+    rows = sorted({0, 1, 63, 64, min(127, m - 1), m // 2, m - 2, m - 1})
+    for n, pk, out in zip(ns, packs, outs):
+        assert np.array_equal(host(out)[rows].view(np.uint32), orc.bitlinear_forward(x[rows], pk, n, f32(0.02))[0].view(np.uint32))
+        assert torch.isfinite(out).all()
+    assert torch.equal(layers[0].forward(xd[:40].contiguous()), outs[0][:40])
