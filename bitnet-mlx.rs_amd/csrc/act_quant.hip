@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
 
 // A workgroup of up to 16 wavefronts per row (Row16, rowquant.hpp), for the rows of a decode batch: the launch is as long as one
 // row takes, which is a chain of dependent steps.  What the first loads need arrives preloaded; the other arguments are one
-// scalar load while the row is on its way.  k % 4 == 0 up to 8192, 16-byte aligned rows, the declared summation order.
+// scalar load while the row is on its way.  k % 4 == 0 up to 16384, 16-byte aligned rows, the declared summation order.
 struct RowQuantArgs {
     int8_t *q;
     float *a_scale;
@@ -324,9 +324,13 @@ template <int MODE>
 void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
 {
     const int chunks = (p.src.k + 3) >> 2;
-    // Rows that all run at once: up to 16 wavefronts per row.
+    // Rows that all run at once: up to 16 wavefronts per row, with four chunks a thread above 8192 columns (213 rows of 13120 columns
+    // with norm: 9.8 us in the 256-thread kernel -> 5.6 here; a decoder block with a 13824-wide FFN at 8 tokens: 36.3 -> 31.5).  Rows
+    // that come in many rounds stay with the 256-thread kernel where it is the faster: a compute unit holds fewer of the long rows
+    // here, and with a norm that costs more than the shorter chain gives (6000 x 12288 with norm: 115 us here, 89 there).
     const bool ordered = !p.src.gamma || p.src.sum_order == BITNET_HIP_SUM_BLOCK256;
-    if ((p.m <= ROW_QUANT_MAX_ROWS || chunks > 1792) && vec && ordered && chunks <= 2048 && p.src.ldx < (1u << 31)) {
+    const bool few = p.m <= ROW_QUANT_MAX_ROWS;
+    if ((few || (chunks > 1792 && (chunks <= 2048 || !p.src.gamma))) && vec && ordered && chunks <= 4096 && p.src.ldx < (1u << 31)) {
         const float *x2 = p.src.x2;
         uint64_t magics = 0;
         bool in_range = true;
@@ -336,16 +340,18 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
         }
         if (in_range) {
             const RowQuantArgs args = {p.q, p.a_scale, p.a_sum, p.y, (int)p.ldq, p.tiled, {0, 0, 0, 0, 0, 0}};
-            const int kt = (p.src.k + 255) >> 8, nchb = kt > 16 ? 2 : 1;
-            const int nw = nchb == 2 ? (kt + 1) / 2 : row_workgroup_waves(p.src.k);
+            const int kt = (p.src.k + 255) >> 8, nchb = kt > 32 ? 4 : (kt > 16 ? 2 : 1);
+            const int nw = nchb == 1 ? row_workgroup_waves(p.src.k) : (kt + nchb - 1) / nchb;
             const dim3 grid((unsigned)p.m), block(64u * (unsigned)nw);
 #define BITNET_HOT_ARGS p.src.x, x2, p.src.gamma, p.src.k, p.src.head_dim / 4, nw, (int)p.src.ldx, p.src.eps, (int)p.m, args
             if (p.src.gamma) {
                 if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else if (nchb == 2) hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
             } else {
                 if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else if (nchb == 2) hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
             }
 #undef BITNET_HOT_ARGS
             return;

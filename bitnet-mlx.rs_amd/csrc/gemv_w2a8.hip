@@ -526,7 +526,7 @@ __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, 
     if (tid < RBW * TILE_ROWS) tot[tid >> 4][tid & 15] = 0;
     if (tid < 16 && tid >= nw) red_f[1][tid] = 0.0f;  // the slots of absent wavefronts hold the neutral element
     if (tid == 0) asum_s = 0;
-    float k_f = (float)hot_k, k_recip = recip_of_ok_divisor(k_f);  // k <= 8192: a divisor the short division accepts
+    float k_f = (float)hot_k, k_recip = recip_of_ok_divisor(k_f);  // k <= 16384: a divisor the short division accepts
     asm volatile("" : "+s"(common), "+s"(P), "+v"(k_recip));
     const int kt_count = (int)common[0];
     const float eps = __builtin_bit_cast(float, (unsigned)common[1]);
@@ -1448,8 +1448,8 @@ int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src,
     const bool norm = src.gamma != nullptr;
     const dim3 grid(8u * (unsigned)m, ((unsigned)p.proj[nproj - 1].rb_end + 7u) / 8u);
     // One wavefront per k-tile (at least the four of the summation order) for rows of up to 16 k-tiles, one chunk per
-    // thread; 16 wavefronts and two chunks per thread above.
-    const int nchb = p.kt_count <= 16 ? 1 : 2;
+    // thread; 16 wavefronts and two or four chunks per thread above.
+    const int nchb = p.kt_count <= 16 ? 1 : (p.kt_count <= 32 ? 2 : 4);
     const int nw = p.kt_count <= 16 ? row_workgroup_waves(src.k) : 16;
     const dim3 block(64u * (unsigned)nw);
     const float *x2 = src.x2;
@@ -1472,7 +1472,11 @@ int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src,
         BITNET_F16_LAUNCH(1);
     } else {
         if (nchb == 1) BITNET_F16_LAUNCH(1);
-        else BITNET_F16_LAUNCH(2);
+        else if (nchb == 2) BITNET_F16_LAUNCH(2);
+        else if constexpr (RBW <= 2) {  // what gemv_fused_supported lets through: no norm
+            if (norm) return fail(BITNET_HIP_UNSUPPORTED, "fused GEMV: %d k-tiles with a norm", p.kt_count);
+            hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, 4, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p);
+        } else return fail(BITNET_HIP_UNSUPPORTED, "fused GEMV: %d row blocks a workgroup for %d k-tiles", RBW, p.kt_count);
     }
 #undef BITNET_F16_LAUNCH
 #undef BITNET_HOT_ARGS
@@ -1711,10 +1715,10 @@ int fused16_row_blocks_per_workgroup(size_t m, size_t k, size_t blocks)
         return (blocks > 256 && k <= 4096) ? 2 : 1;
     }
     // Several tokens, each with its own workgroups: the fewest row blocks per workgroup that keep the launch within one
-    // workgroup per compute unit, at most 8 (4 of rows above 4096 columns, whose wavefronts hold two tiles of each).  30-block
-    // step at 2 / 3 / 4 / 6 tokens: 541 / 593 / 667 / 713 us; with launches of up to 512 workgroups 541 / 606 / 670 / 713.
+    // workgroup per compute unit, at most 8 (4 of rows above 4096 columns, whose wavefronts hold two tiles of each, 2 above
+    // 8192).  30-block step at 2 / 3 / 4 / 6 tokens: 541 / 593 / 667 / 713 us; with launches of up to 512 workgroups 541 / 606 / 670 / 713.
     int rbw = 1;
-    const int most = k_tiles(k) > 16 ? 4 : 8;
+    const int most = k_tiles(k) > 32 ? 2 : (k_tiles(k) > 16 ? 4 : 8);
     while (rbw < most && (blocks + rbw - 1) / rbw * m > 256) rbw *= 2;
     return rbw;
 }
@@ -1730,11 +1734,20 @@ bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m,
     // workgroups of all tokens stay within GEMV_FUSED_MAX_WGS.  Otherwise: stand-alone quantiser (rows in parallel) + MFMA GEMV.
     if (m == 0 || m > (size_t)GEMV_FUSED_MAX_ROWS) return false;
     if (m > 1) {
-        if (!((gamma == nullptr || sum_order == BITNET_HIP_SUM_BLOCK256) && k <= 8192 && ldx < ((size_t)1 << 31))) return false;
+        if (!((gamma == nullptr || sum_order == BITNET_HIP_SUM_BLOCK256) && k <= 16384 && ldx < ((size_t)1 << 31))) return false;
         const size_t rbw = (size_t)fused16_row_blocks_per_workgroup(m, k, blocks);
         if ((blocks + rbw - 1) / rbw * m > (size_t)GEMV_FUSED_MAX_WGS) return false;
     }
-    if (k % 4 != 0 || ldx % 4 != 0 || k > (size_t)FUSED_NCH * 1024) return false;
+    // Rows above FUSED_NCH * 1024 columns: only where one round of workgroups serves the launch (each quantises its whole row for
+    // itself), and in the declared summation order; above 8192 columns (four chunks per thread) without a norm, whose registers do
+    // not fit beside the tiles.  A decoder block with 2560-wide rows, in two launches -> here: 8192-wide FFN at 1 / 2 / 3 tokens
+    // 20.3 / 21.5 / 23.4 -> 16.6 / 19.5 / 21.4 us, 13824-wide at 1 / 2 / 3 / 4 tokens 29.4 / 32.8 / 33.2 / 33.9 -> 20.2 / 25.1 /
+    // 25.6 / 29.0 (of which the stand-alone quantiser's four chunks per thread give up to 5).
+    if (k > (size_t)FUSED_NCH * 1024) {
+        if ((m == 1 && blocks > 256) || k > 16384 || ldx >= ((size_t)1 << 31)) return false;
+        if (gamma != nullptr && (sum_order != BITNET_HIP_SUM_BLOCK256 || k > 8192)) return false;
+    }
+    if (k % 4 != 0 || ldx % 4 != 0) return false;
     if (!al16(x) || (x2 && !al16(x2)) || (gamma && !al16(gamma))) return false;
     if (input_mode == BITNET_HIP_INPUT_GQA_BROADCAST && head_dim % 4 != 0) return false;
     return k_tiles(k) * 16 * sizeof(uint4) <= 60 * 1024;
@@ -1749,8 +1762,8 @@ int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const fl
     // workgroup two (short rows only: the tiles of both must fit its registers).
     size_t blocks = 0;
     for (int j = 0; j < nproj; ++j) blocks += row_blocks(projs[j].n);
-    // 16 wavefronts per workgroup (the declared summation order only; k <= 8192: two chunks per thread, 32 k-tiles)
-    if ((gamma == nullptr || sum_order == BITNET_HIP_SUM_BLOCK256) && k <= 8192) {
+    // 16 wavefronts per workgroup (the declared summation order only; k <= 16384: up to four chunks per thread, 64 k-tiles)
+    if ((gamma == nullptr || sum_order == BITNET_HIP_SUM_BLOCK256) && k <= 16384) {
         // row blocks per workgroup: one round of workgroups on the 256 compute units where the row is short enough for
         // a wavefront to hold the tiles of several row blocks (one token, gate alone, 432 row blocks: 4.50 us with one
         // row block per workgroup, 3.82 us with two)

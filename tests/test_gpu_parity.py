@@ -1799,3 +1799,49 @@ def test_gemm_launches_between_one_round_and_many_tiles(m, ns, k):
         assert np.array_equal(host(out)[rows].view(np.uint32), orc.bitlinear_forward(x[rows], pk, n, f32(0.02))[0].view(np.uint32))
         assert torch.isfinite(out).all()
     assert torch.equal(layers[0].forward(xd[:40].contiguous()), outs[0][:40])
+
+
+@pytest.mark.parametrize("m,k", [(3, 8196), (512, 8448), (513, 8448), (2, 12288), (40, 12292), (5, 16384), (3, 16388), (600, 16384)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_activation_quant_of_rows_above_8192_columns(m, k, norm):
+    """Four chunks a thread up to 16384 columns, both sides of the row counts and widths where the other kernels take over."""
+    rng = np.random.default_rng(m + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    g = (1.0 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    q, s, asum, _ = bh.quantize_activations_i8(dev(x), dev(g) if norm else None, eps=1e-5, want_sum=True)
+    q_ref, s_ref, rs_ref = orc.rmsnorm_quantize_i8(x, g, 1e-5, orc.SUM_BLOCK256)
+    assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), rs_ref)
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("n,k", [(17, 7172), (640, 8192), (4100, 8192), (33, 8196), (640, 12292), (2560, 13824), (100, 16384), (4096, 16384), (40, 16388)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_forward_of_few_long_rows_bit_exact(m, n, k, norm):
+    """One to eight tokens on rows above 7168 columns: quantised in the GEMV launch where one round of workgroups serves it (two or four
+    chunks a thread, one to four row blocks a workgroup), by the stand-alone quantiser elsewhere; and through a workspace."""
+    rng = np.random.default_rng(m + n + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    g = (1.0 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    pk = random_packed_ternary(rng, n, k)
+    res = rng.standard_normal((m, n), dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "long")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    gd = None if g is None else dev(g)
+    ref, q_ref, s_ref, acc_ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, residual=res)
+    assert np.array_equal(host(layer.forward(dev(x), gamma=gd, residual=dev(res))), ref)
+    out, q, a_scale, acc = layer.forward(dev(x), gamma=gd, residual=dev(res), debug=True)
+    assert np.array_equal(host(out), ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(a_scale), s_ref) and np.array_equal(host(acc), acc_ref)
+    ws = torch.empty((layer.workspace_size(m),), dtype=torch.uint8, device="cuda")
+    assert np.array_equal(host(layer.forward(dev(x), gamma=gd, residual=dev(res), workspace=ws)), ref)
+
+
+@pytest.mark.parametrize("ffn", [7424, 8192, 8448, 13824, 16640])
+@pytest.mark.parametrize("m", [1, 2, 3, 5, 8, 20])
+def test_decoder_blocks_with_wide_ffn_match_the_oracle(ffn, m):
+    """The down projection of blocks whose FFN is wider than 7168 (relu2-gated input): each of its launches on both sides of the lines
+    between them."""
+    dims = (256, ffn, 4, 2, 64)
+    rng = np.random.default_rng(ffn + m)
+    dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
+    x = synth_activations(rng, m, dims[0])
+    assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
