@@ -24,8 +24,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int WAVES = 16;
 constexpr int MAX_KT = 2 * WAVES;  // k-tiles: two per wavefront
-constexpr int CPR = 4;             // chunks of four columns a lane holds of its row
-constexpr size_t MAX_WIDTH = 256 * CPR;
+constexpr size_t SHORT_WIDTH = 256 * 4, MAX_WIDTH = 256 * 8;  // distinct columns of a row: four or eight chunks of four a lane
 
 struct RowqProj {
     const uint8_t *w;
@@ -46,9 +45,9 @@ struct RowqParams {
 static_assert(sizeof(RowqParams) == 64 * (GEMV_MAX_PROJ + 1), "one scalar load more for the rest");
 constexpr int ROWQ_ARGS_AT = 64;  // offset of RowqParams in the argument buffer: five pointers and five ints before it
 
-// MODE: PLAIN or GQA_BROADCAST.  RB row blocks, NT k-tiles per wavefront.
+// MODE: PLAIN or GQA_BROADCAST.  RB row blocks, NT k-tiles per wavefront, CPR chunks of four columns a lane holds of its row.
 // Counts are packed as for gemv_rows_kernel; hot_blocks_width: row blocks of projection 2, and the distinct columns of a row.
-template <int MODE, bool NORM, int RB, int NT>
+template <int MODE, bool NORM, int RB, int NT, int CPR>
 __global__ __launch_bounds__(1024) void gemv_rowq_kernel(const float *hot_x, const float *hot_gamma, const uint8_t *hot_w0, const uint8_t *hot_w1,
                                                          const uint8_t *hot_w2, unsigned hot_m_kt, unsigned hot_ends, unsigned hot_blocks,
                                                          unsigned hot_blocks_width, unsigned hot_groups, [[maybe_unused]] RowqParams args)
@@ -69,12 +68,14 @@ __global__ __launch_bounds__(1024) void gemv_rowq_kernel(const float *hot_x, con
     const bool has_row = wave < rows_here;  // uniform over the wavefront
 
     // the row first, the weight tiles behind it
+    auto absent_chunk = [&](int i) { return CPR > 4 && 64 * i >= chunks; };  // of every lane: left out above 1024 columns
     float4 v[CPR], g[NORM ? CPR : 1];
     {
         const global_ptr<const v4f> row = (global_ptr<const v4f>)(uintptr_t)(hot_x + (size_t)(tg * 16 + min(wave, rows_here - 1)) * width);
         const global_ptr<const v4f> gamma = (global_ptr<const v4f>)(uintptr_t)hot_gamma;
 #pragma unroll
         for (int i = 0; i < CPR; ++i) {
+            if (absent_chunk(i)) continue;
             const int c = min(lane + 64 * i, chunks - 1);
             const v4f e = row[c];
             v[i] = make_float4(e[0], e[1], e[2], e[3]);
@@ -124,22 +125,31 @@ __global__ __launch_bounds__(1024) void gemv_rowq_kernel(const float *hot_x, con
             // chunk c belongs to virtual lane c % 256 of the declared order: four partial sums a lane
             float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < CPR; ++i) part[i & 3] = sum_squares4(part[i & 3], v[i]);
+            for (int i = 0; i < CPR; ++i) {
+                if (absent_chunk(i)) continue;
+                part[i & 3] = sum_squares4(part[i & 3], v[i]);
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) part[j] = wave_sum_f32(part[j]);
             const float ss = f32_add(f32_add(f32_add(part[0], part[1]), part[2]), part[3]);
             const Divisor rdiv = make_divisor(rms_from_ss(ss, width, __builtin_bit_cast(float, Q[0])));
 #pragma unroll
-            for (int i = 0; i < CPR; ++i)
+            for (int i = 0; i < CPR; ++i) {
+                if (absent_chunk(i)) continue;
                 if (lane + 64 * i < chunks) v[i] = normalize4(v[i], rdiv, g[i]);
+            }
         }
         float amax = 0.0f;
 #pragma unroll
-        for (int i = 0; i < CPR; ++i) amax = absmax4(amax, v[i]);
+        for (int i = 0; i < CPR; ++i) {
+            if (absent_chunk(i)) continue;
+            amax = absmax4(amax, v[i]);
+        }
         const float scale = scale_from_absmax(wave_max_f32(amax));
         int unused = 0;
 #pragma unroll
         for (int i = 0; i < CPR; ++i) {
+            if (absent_chunk(i)) continue;
             const int c = lane + 64 * i, piece = c >> 2;
             const uint32_t packed = quant4_packed(v[i], scale, &unused);
             if (c < chunks) *reinterpret_cast<uint32_t *>(lds + (piece * 16 + (wave ^ (piece & 15))) * 16 + (c & 3) * 4) = packed;
@@ -226,27 +236,37 @@ struct Launch {
     hipStream_t stream;
 };
 
-template <int MODE, bool NORM, int RB, int NT>
+template <int MODE, bool NORM, int RB, int NT, int CPR>
 int launch(const Launch &l)
 {
     const int kt = (int)(l.m_kt >> 16);
     const size_t bytes = l.pieces * 256 + (size_t)(kt < WAVES ? kt : WAVES) * RB * 1024;
     constexpr size_t MOST = (size_t)CPR * 64 / 4 * 256 + (size_t)WAVES * RB * 1024;
-    static const hipError_t attr = MOST > 64 * 1024 ? hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rowq_kernel<MODE, NORM, RB, NT>),
+    static const hipError_t attr = MOST > 64 * 1024 ? hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rowq_kernel<MODE, NORM, RB, NT, CPR>),
                                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST)
                                                     : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemv_rowq_kernel<MODE, NORM, RB, NT>), l.grid, dim3(64 * WAVES), bytes, l.stream, l.x, l.gamma, l.p.proj[0].w, l.p.proj[1].w,
+    hipLaunchKernelGGL((gemv_rowq_kernel<MODE, NORM, RB, NT, CPR>), l.grid, dim3(64 * WAVES), bytes, l.stream, l.x, l.gamma, l.p.proj[0].w, l.p.proj[1].w,
                        l.p.proj[2].w, l.m_kt, l.ends, l.blocks, l.blocks_width, l.groups, l.p);
     BITNET_HIP_CHECK_LAUNCH("gemv_rowq_kernel");
     return BITNET_HIP_OK;
 }
-template <int MODE, bool NORM, int NT>
+template <int MODE, bool NORM, int NT, int CPR>
 int launch_rb(const Launch &l, int rb)
 {
-    if (rb == 4) return launch<MODE, NORM, 4, NT>(l);
-    if (rb == 2) return launch<MODE, NORM, 2, NT>(l);
-    return launch<MODE, NORM, 1, NT>(l);
+    if (rb == 4) return launch<MODE, NORM, 4, NT, CPR>(l);
+    if (rb == 2) return launch<MODE, NORM, 2, NT, CPR>(l);
+    return launch<MODE, NORM, 1, NT, CPR>(l);
+}
+// Workgroups that the fullest compute unit runs, of `groups` groups of row blocks and `tgroups` token groups (the kernel's mapping: a
+// group of row blocks on one XCD of 32).
+size_t rounds_of(size_t groups, size_t tgroups) { return ((groups + 7) / 8 * tgroups + 31) / 32; }
+// The fewest row blocks a workgroup that keep the launch within one round, at most 4.
+size_t row_blocks_per_workgroup(size_t blocks, size_t tgroups)
+{
+    size_t rb = 1;
+    while (rb < 4 && rounds_of((blocks + rb - 1) / rb, tgroups) > 1) rb *= 2;
+    return rb;
 }
 
 }  // namespace
@@ -264,7 +284,16 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
     // 2560: 5.1 -> 4.8 us recorded, 7.2 -> 4.7 us as calls; 16 x 1024 -> 2560: 5.1 -> 6.0 recorded, so up to 12288 elements a
     // token group in a step and any row that fits in a call of its own).
     const size_t in_group = m < 16 ? m : 16, tgroups = (m + 15) / 16;
-    if (m < 2 || m > (size_t)GEMV_MAX_M || (blocks + 3) / 4 * tgroups > 256) return false;
+    if (m < 2 || m > (size_t)GEMV_WIDE_MAX_M || (blocks + 3) / 4 * tgroups > 256) return false;
+    // More than 95 tokens, and rows above 1024 columns without a norm: calls of their own, as long as no compute unit quantises more than
+    // 2048 columns for its 16 tokens (with a norm, in two rounds: not).  In two launches -> here, us as calls / recorded: 104 x 1024 -> 512
+    // 8.0 / 4.6 -> 5.2 / 4.0, 512 x 1024 -> 512 8.0 / 7.1 -> 5.5 / 5.3, 128 x 512 -> 2048 with norm 8.0 / 6.5 -> 6.2 / 6.2, 16 x 1280 -> 2560 8.0 /
+    // 4.8 -> 5.4 / 5.1, 64 x 1280 -> 2560 8.0 / 6.7 -> 6.0 / 5.9, 16 x 2048 -> 2560 8.0 / 4.9 -> 6.0 / 5.9, 40 x 2048 -> 5120 7.8 / 6.3 -> 7.3 / 7.1.
+    // Beyond the line: 16 x 1280 -> 2560 with norm 8.1 / 5.1 -> 7.1 / 7.2, 40 x 2560 -> 5120 9.1 -> 9.1 as calls.
+    if (m > (size_t)GEMV_MAX_M || width > SHORT_WIDTH) {
+        const size_t rb = row_blocks_per_workgroup(blocks, tgroups), rounds = rounds_of((blocks + rb - 1) / rb, tgroups);
+        if (gqa || !alone || (gamma ? rounds > 1 || width > SHORT_WIDTH : rounds * width > MAX_WIDTH)) return false;
+    }
     if (width % 4 != 0 || ldx != width || width > MAX_WIDTH || (!gqa && !alone && width * in_group > 12288)) return false;
     if (k_tiles(k) > (size_t)MAX_KT || k > 0xffff || blocks > GEMV_ROWS_MAX_BLOCKS) return false;
     // Up to eight tokens gemv_fused16_kernel may be one launch as well, with a set of workgroups for every token.  It has fewer rows to
@@ -272,8 +301,9 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
     // with the attention output by this kernel instead, where those walk 24 to 40 tiles: 0.5 to 1.0 us slower (1536 to 2560 wide, 2
     // to 8 tokens); 44 and 48: 0.1 to 0.3 slower (2816 and 3072 wide at 3 to 5); 52: 0.4 to 1.0 faster (3200 at 3 to 5), 56 and 64:
     // even (3584 and 4096 at 3, 4), 80 and more: 0.6 to 2.0 faster (2560 at 7 and 8, 4096 at 5 to 8, 5120 to 8192 at 2 to 8).  Where
-    // that kernel's workgroups do not fit one round, the other choice is two launches: 6 x 1024 -> 8192 7.5 us a call, 3.7 here.
-    if (gemv_fused_supported(x, nullptr, ldx, m, k, input_mode, head_dim, gamma, sum_order, blocks) && gemv_fused_tiles(m, k, blocks) <= 48)
+    // that kernel's workgroups do not fit one round, the other choice is two launches: 6 x 1024 -> 8192 7.5 us a call, 3.7 here.  Above
+    // 1024 columns that kernel keeps what it takes.
+    if (gemv_fused_supported(x, nullptr, ldx, m, k, input_mode, head_dim, gamma, sum_order, blocks) && (width > SHORT_WIDTH || gemv_fused_tiles(m, k, blocks) <= 48))
         return false;
     return al16(x) && (!gamma || (al16(gamma) && sum_order == BITNET_HIP_SUM_BLOCK256));
 }
@@ -286,8 +316,7 @@ int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m,
     const size_t width = gqa ? k / gqa_group : k, kt = k_tiles(k), tgroups = (m + 15) / 16;
     size_t blocks = 0;
     for (int j = 0; j < nproj; ++j) blocks += row_blocks(projs[j].n);
-    int rb = 1;  // as in launch_gemv_rows: the fewest row blocks a workgroup that keep the launch within one round, at most 4
-    while (rb < 4 && (blocks + rb - 1) / rb * tgroups > 256) rb *= 2;
+    const int rb = (int)row_blocks_per_workgroup(blocks, tgroups);
     Launch l = {};
     size_t groups = 0;
     unsigned ends[GEMV_MAX_PROJ] = {}, counts[GEMV_MAX_PROJ] = {};
@@ -312,9 +341,10 @@ int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m,
         auto magic = [](size_t d) { return d == 1 ? 0u : (unsigned)((((uint64_t)1 << 32) + d - 1) / d); };
         l.p.head_pieces = (unsigned)(head_dim / 16);
         l.p.head_magic = magic(head_dim / 16); l.p.span_magic = magic(head_dim / 16 * gqa_group);
-        return kt > WAVES ? launch_rb<BITNET_HIP_INPUT_GQA_BROADCAST, false, 2>(l, rb) : launch_rb<BITNET_HIP_INPUT_GQA_BROADCAST, false, 1>(l, rb);
+        return kt > WAVES ? launch_rb<BITNET_HIP_INPUT_GQA_BROADCAST, false, 2, 4>(l, rb) : launch_rb<BITNET_HIP_INPUT_GQA_BROADCAST, false, 1, 4>(l, rb);
     }
-    return gamma ? launch_rb<BITNET_HIP_INPUT_PLAIN, true, 1>(l, rb) : launch_rb<BITNET_HIP_INPUT_PLAIN, false, 1>(l, rb);
+    if (gamma) return launch_rb<BITNET_HIP_INPUT_PLAIN, true, 1, 4>(l, rb);
+    return width > SHORT_WIDTH ? launch_rb<BITNET_HIP_INPUT_PLAIN, false, 1, 8>(l, rb) : launch_rb<BITNET_HIP_INPUT_PLAIN, false, 1, 4>(l, rb);
 }
 
 }  // namespace bitnet

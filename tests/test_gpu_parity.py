@@ -1845,3 +1845,30 @@ def test_decoder_blocks_with_wide_ffn_match_the_oracle(ffn, m):
     dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
     x = synth_activations(rng, m, dims[0])
     assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
+
+
+@pytest.mark.parametrize("m,n,k", [(96, 512, 1024), (97, 33, 4), (132, 412, 416), (400, 640, 1024), (400, 640, 1028), (512, 500, 768), (513, 500, 768),
+                                   (9, 2560, 1028), (16, 16384, 2048), (16, 16400, 2048), (40, 5120, 2044), (95, 40, 2052), (2, 9000, 1284), (17, 17, 1540)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_forward_of_rows_quantised_by_every_workgroup(m, n, k, norm):
+    """Up to 512 tokens, and rows of up to 2048 columns, in one launch: both sides of the lines beyond which it is two, one and two rounds
+    of workgroups, chunks that no lane has, and several projections of one input."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    g = (1 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    gd = dev(g) if norm else None
+    pk = random_packed_ternary(rng, n, k)
+    bias, res = rng.standard_normal(n, dtype=f32), rng.standard_normal((m, n), dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "workgroup rows")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    layer.update_bias(dev(bias))
+    ref, q_ref, s_ref, acc_ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias, residual=res)
+    assert np.array_equal(host(layer.forward(dev(x), gamma=gd, residual=dev(res))), ref)
+    out, q, a_scale, acc = layer.forward(dev(x), gamma=gd, residual=dev(res), debug=True)
+    assert np.array_equal(host(out), ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(a_scale), s_ref) and np.array_equal(host(acc), acc_ref)
+    other = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=24), "beside")
+    pk2 = random_packed_ternary(rng, 24, k)
+    other.set_quantized_weights(torch.from_numpy(pk2), 0.03)
+    got = bh.forward_multi([other, layer], dev(x), gamma=gd)
+    assert np.array_equal(host(got[0]), orc.bitlinear_forward(x, pk2, 24, f32(0.03), g=g)[0])
+    assert np.array_equal(host(got[1]), orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias)[0])
