@@ -5,9 +5,9 @@
 //   act_quant_block_kernel    256-thread workgroups that take token rows in turn, a row held in registers between the three
 //                             passes (sum of squares, absmax, quantise): 4*K bytes read once, K + 8 bytes written.
 //                             The usual shape, for one row or thousands.
-//   act_quant_row_kernel      a workgroup of up to 16 wavefronts per token row, one chunk of 4 (two above 4096 columns) per
-//                             thread: as many rows as run at once (a decode batch), where the launch is as long as one
-//                             row takes.
+//   act_quant_row_kernel      a workgroup of up to 16 wavefronts per token row, one chunk of 4 (two above 4096 columns, four
+//                             above 8192) per thread: as many rows as run at once (a decode batch), where the launch is as
+//                             long as one row takes.
 //   act_quant_wave_kernel     one wavefront per token row: many rows of at most 1024 columns.
 #include "kernels.hpp"
 #include "rowquant.hpp"

@@ -101,16 +101,19 @@ inline bool gemm_takes_tokens(size_t m, size_t k, size_t n_blocks, const void *a
 }
 // From 17 tokens on, where one round of gemm_ld8_kernel holds the launch, the two are compared by what they take (ns).  The GEMM: its
 // start and epilogue, and its stages (gemm_one_round_ns).  The token GEMV: its start, and per 16-row block and group of 16 tokens the
-// exchange of the partial results (by wavefronts, up to 16: one per k-tile) and the k-tiles beyond.  Both fitted to kernel times over 10 widths, 10 to
-// 192 tokens, within 20 %; the GEMM's start with 2.5 us on top, what weights that come from HBM cost it more than the GEMV, which asks for
-// all of its tiles at once (blocks of a decoder, each with its own weights, at 18 and 24 tokens of 3072 -> 18048 and 2304 -> 18176).  GEMV / GEMM, quantiser included, in us: 2560 -> 13824 at 32 / 42 / 95 10.1 / 10.6, 12.1 / 11.0, 21.6 / 12.2; 4096 -> 12288
-// at 20 / 42 / 95 12.1 / 12.0, 17.2 / 12.2, 24.3 / 17.6; 8192 -> 8192 at 32 / 42 / 95 11.3 / 15.7, 19.0 / 17.3, 23.6 / 18.2; 2560 -> 30000 at
-// 16 / 20 / 48 10.5 / 12.7, 17.8 / 12.5, 23.6 / 14.5; 6912 -> 2560 at 95 / 112 11.1 / 12.3, 15.7 / 12.5; 2560 -> 2560 at 95 / 192 8.1 / 9.3, 10.5 / 10.3.
+// exchange of the partial results (by wavefronts, up to 16: one per k-tile) and the k-tiles beyond.  Both fitted to kernel times over
+// 10 widths, 10 to 192 tokens, within 20 %; the GEMM's start with 2.5 us on top, what weights that come from HBM cost it more than the
+// GEMV, which asks for all of its tiles at once (blocks of a decoder, each with its own weights, at 18 and 24 tokens of 3072 -> 18048
+// and 2304 -> 18176; 42 tokens of 2560 -> 6912 + 6912 by the GEMM: a 30-block step 1060 -> 1115 us).  GEMV / GEMM, quantiser included,
+// in us: 2560 -> 13824 at 32 / 42 / 95 10.1 / 10.6, 12.1 / 11.0, 21.6 / 12.2; 4096 -> 12288 at 20 / 42 / 95 12.1 / 12.0, 17.2 / 12.2,
+// 24.3 / 17.6; 8192 -> 8192 at 32 / 42 / 95 11.3 / 15.7, 19.0 / 17.3, 23.6 / 18.2; 2560 -> 30000 at 16 / 20 / 48 10.5 / 12.7, 17.8 /
+// 12.5, 23.6 / 14.5; 6912 -> 2560 at 95 / 112 11.1 / 12.3, 15.7 / 12.5; 2560 -> 2560 at 95 / 192 8.1 / 9.3, 10.5 / 10.3.
 size_t gemm_one_round_ns(size_t m, size_t k, size_t n);  // gemm_w2a8.hip; 0 where no tile of that kernel holds the launch in one round
 constexpr size_t GEMM_START_NS = 7500, GEMM_LEAST_STAGE_NS = 154;
 inline bool gemm_beats_token_gemv(size_t m, size_t k, size_t n_blocks, const void *a)
 {
-    if (m <= 16 || m > (size_t)GEMV_WIDE_MAX_M || k < 1024 || k % TILE_K != 0 || n_blocks * k >= (1ull << 29) || (reinterpret_cast<uintptr_t>(a) & 15) != 0)
+    if (m <= 16 || m > (size_t)GEMV_WIDE_MAX_M || k < 1024 || k % TILE_K != 0 || n_blocks * k >= (1ull << 29) ||
+        (reinterpret_cast<uintptr_t>(a) & 15) != 0)
         return false;
     const size_t kt = k / TILE_K, blocks = n_blocks * ((m + 15) / 16), near = blocks * (kt < 16 ? kt : 16), all = blocks * kt;
     const size_t gemv_ns = 3300 + near / 4 + (all - near) / 8 + (m > 64 ? 1000 : 0);

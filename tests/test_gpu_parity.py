@@ -575,8 +575,7 @@ def test_gemm_f32_only_epilogue_ragged(m, n, k, extras):
 def test_forward_in_hip_graph_replays_match_eager(m):
     """forward() with caller-supplied output and workspace allocates nothing and records no memset, so a caller may
     capture it into a HIP graph: three replays, with eager work and synchronisations between them, each bit-equal
-    to the eager result and to the oracle.  128 tokens take the GEMM that splits k across workgroups: its tile counters
-    live in the workspace and are cleared by the quantiser kernel of the same call."""
+    to the eager result and to the oracle."""
     rng = np.random.default_rng(900 + m)
     n, k = 2560, 6912
     w = synth_weights(rng, n, k)
@@ -744,11 +743,10 @@ def test_bitlinear_forward_prefill_uses_quantiser_row_sums():
 @pytest.mark.parametrize("m,k,n", [(97, 6912, 2560), (128, 6912, 2560), (200, 4096, 1000), (256, 6912, 2560), (130, 8192, 644),
                                    (255, 5120, 1408), (97, 4096, 16), (256, 8192, 2816), (300, 4352, 2240)])
 def test_forward_split_k_bit_exact(m, k, n):
-    """A long k with few output tiles (97 to 256 tokens at 6912 -> 2560): forward() splits k across workgroups, which
-    exchange int32 partial tiles through the workspace.  Checked against the oracle (activations, accumulators, f32
-    output with bias and residual); with a workspace that holds only the quantised activations (no split: same bits);
-    on a workspace full of ones (the tile counters are cleared by the quantiser of the same call); and on the same
-    workspace three times in a row (the counters are left at zero)."""
+    """A long k with few output tiles (97 to 256 tokens at 6912 -> 2560), for which workspace_size counts more than the
+    quantised activations.  Checked against the oracle (activations, accumulators, f32 output with bias and residual);
+    with a workspace that holds only the quantised activations; on a workspace full of ones; and on the same workspace
+    three times in a row."""
     rng = np.random.default_rng(m + k + n)
     w = synth_weights(rng, n, k)
     x = synth_activations(rng, m, k, outliers=True)
