@@ -266,8 +266,10 @@ __global__ __launch_bounds__(256) void ternarize_pack_kernel(const float *w, siz
 // division by the deviation, which is the same for the whole tensor, and a clamp).  Every tensor-wide sum is carried in f64
 // in the order of the absmean kernels above (per row: lane l adds columns l, l+64, ..., then the butterfly; the row sums
 // the same way), so the f32 scalars have the bits the CPU restatement of the same order has.  The scalars stay on the
-// device in WqState; one workgroup finishes each reduction and derives the next stage's scalars.  The last pass (the
-// scale's sums) knows the threshold, so it writes the codes too where rows start on bytes.
+// device in WqState.  Who finishes a reduction and derives the next stage's scalars: up to WQ_FOLD_MAX_ROWS rows every workgroup of
+// the next pass, for itself (a wavefront adds up to 64 row sums a lane while a launch of its own takes 3.1 us and the gap in front of
+// it); above, and where no pass follows, one workgroup in a launch between the passes.  The last pass (the scale's sums) knows the
+// threshold, so it writes the codes too where rows start on bytes.
 struct WqState {
     float mean, sd;            // normalisation (0, 1 when switched off)
     float clip_mean, clip_mad; // centre and mean |.| of the normalised tensor
@@ -280,6 +282,7 @@ static_assert(sizeof(WqState) == 12 * sizeof(float), "stats are returned as 12 f
 
 enum WqPass { WQ_SUM = 0, WQ_SQDIFF, WQ_CLIP_STATS, WQ_ABS_STATS, WQ_OPTIMAL, WQ_SCALE };
 constexpr int WQ_MAX_ACC = 10;
+constexpr size_t WQ_SCRATCH_SUMS = 4 + WQ_MAX_ACC;  // doubles a row: those of two consecutive passes (two each), and of WQ_OPTIMAL
 
 __device__ __forceinline__ void wq_publish(const WqState &st, int clip, float *w_scale, float *stats)
 {
@@ -297,10 +300,10 @@ struct WqView {
     float recip;
     bool fast, normalize, clip;
 };
-__device__ __forceinline__ WqView wq_view(const WqState *state, int normalize, int clip)
+__device__ __forceinline__ WqView wq_view(const WqState &state, int normalize, int clip)
 {
     WqView v;
-    v.st = *state;
+    v.st = state;
     v.recip = f32_div(1.0f, v.st.sd);
     v.fast = invariant_divisor_ok(v.st.sd);
     v.normalize = normalize != 0;
@@ -328,20 +331,127 @@ __device__ __forceinline__ float wq_code(float x, float thr) { return x > thr ? 
 
 __constant__ float wq_factors[10] = {0.3f, 0.4f, 0.5f, 0.6f, 0.7f, 0.8f, 0.9f, 1.0f, 1.1f, 1.2f};
 
+// Before the first pass (state: none), or what the passes so far have left.
+__device__ __forceinline__ WqState wq_state(const WqState *state)
+{
+    if (state) return *state;
+    WqState st;
+    st.mean = 0.0f; st.sd = 1.0f; st.clip_mean = 0.0f; st.clip_mad = 0.0f; st.lo = -__builtin_inff(); st.hi = __builtin_inff();
+    st.mean_abs = 0.0f; st.max_abs = 0.0f; st.thr = 0.0f; st.num = 0.0f; st.den = 0.0f; st.scale = 1.0f;
+    return st;
+}
+
+// How thresholds and clip bounds come from the sums.  method: TernaryMethod 0..4; custom <= 0: the method's own factor.
+struct WqRule {
+    int method;
+    float outlier_threshold, custom;
+};
+
+// The scalars that the finished sums `tot` (and mx, the largest row_max) of a pass give.
+__device__ __forceinline__ void wq_derive(WqState &st, int pass, const double *tot, float mx, double count, const WqRule &rule)
+{
+    if (pass == WQ_SUM) {
+        st.mean = (float)(tot[0] / count);
+    } else if (pass == WQ_SQDIFF) {
+        const float var = (float)(tot[0] / count);
+        st.sd = f32_sqrt(var + 1e-8f);
+    } else if (pass == WQ_CLIP_STATS) {
+        st.clip_mean = (float)(tot[0] / count);
+        st.clip_mad = (float)(tot[1] / count);
+        const float spread = f32_mul(rule.outlier_threshold, st.clip_mad);
+        st.lo = st.clip_mean - spread;
+        st.hi = st.clip_mean + spread;
+    } else if (pass == WQ_ABS_STATS) {
+        st.mean_abs = (float)(tot[0] / count);
+        st.max_abs = mx;
+        const bool has_custom = rule.custom > 0.0f;
+        float thr;
+        if (rule.method == 1) thr = f32_mul(st.mean_abs, has_custom ? rule.custom : 0.8f);
+        else if (rule.method == 2)
+            thr = has_custom ? f32_mul(st.mean_abs, rule.custom)
+                             : (st.max_abs > f32_mul(3.0f, st.mean_abs) ? f32_mul(st.mean_abs, 0.5f) : f32_mul(st.mean_abs, 0.7f));
+        else thr = f32_mul(st.mean_abs, has_custom ? rule.custom : 0.7f);  // mean, DetSTE; optimal without its search
+        st.thr = thr;
+    } else if (pass == WQ_OPTIMAL) {
+        float best = __builtin_inff(), thr = f32_mul(st.mean_abs, 0.7f);
+#pragma unroll
+        for (int f = 0; f < 10; ++f) {
+            const float mse = (float)(tot[f] / count);
+            if (mse < best) { best = mse; thr = f32_mul(st.mean_abs, wq_factors[f]); }
+        }
+        st.thr = thr;
+    } else {
+        st.num = (float)tot[0];
+        st.den = (float)tot[1];
+        st.scale = fabsf(st.den) < 1.1920929e-07f ? 1.0f : f32_div(st.num, st.den);
+    }
+}
+
+// What a pass with at most WQ_FOLD_MAX_ROWS rows finishes of the pass before it (pass < 0: nothing is left to finish).
+struct WqPrevious {
+    int pass;            // of those with one or two accumulators
+    const double *sums;  // not those this pass writes
+    WqState *state;      // where the state with its scalars goes, for the next pass; not the one this pass reads
+    WqRule rule;
+};
+constexpr size_t WQ_FOLD_MAX_ROWS = 4096;
+
+// By a workgroup of four wavefronts: an accumulator each by the first two (the order of combine_row_sums), the largest row maximum
+// by all of them.
+__device__ __forceinline__ void wq_finish_previous(WqState &st, const WqPrevious &prev, const float *row_max, size_t n, size_t k)
+{
+    __shared__ double tot[2];
+    __shared__ float maxima[4];
+    const int lane = threadIdx.x, wave = threadIdx.y;
+    const int nacc = prev.pass == WQ_CLIP_STATS ? 2 : 1, rows = (int)n;
+    if (wave < nacc) {
+        const double *sums = prev.sums + (size_t)wave * n;
+        double s = 0.0;
+        int row = lane;
+        for (; row + 7 * 64 < rows; row += 8 * 64) {
+            double t[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) t[i] = sums[row + 64 * i];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s = s + t[i];
+        }
+        for (; row < rows; row += 64) s = s + sums[row];
+        s = wave_sum_f64(s);
+        if (lane == 0) tot[wave] = s;
+    }
+    float mx = 0.0f;
+    if (prev.pass == WQ_ABS_STATS) {
+        for (int row = lane + 64 * wave; row < rows; row += 256) mx = fmaxf(mx, row_max[row]);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        if (lane == 0) maxima[wave] = mx;
+    }
+    __syncthreads();
+    if (prev.pass == WQ_ABS_STATS) mx = fmaxf(fmaxf(maxima[0], maxima[1]), fmaxf(maxima[2], maxima[3]));
+    wq_derive(st, prev.pass, tot, mx, (double)n * (double)k, prev.rule);
+}
+
 constexpr int wq_accumulators(int pass) { return pass == WQ_OPTIMAL ? 10 : ((pass == WQ_CLIP_STATS || pass == WQ_SCALE) ? 2 : 1); }
 
 // One wavefront per row; accumulator a of row r goes to row_sums[a * n + r] (and the row's max |.| to row_max[r]).
 // packed (WQ_SCALE, k a multiple of 4, else null): the codes of the row, four columns a byte, put together by the quad of
 // lanes that holds them; q_i8 as ever optional.  Bound by the read of the matrix.
-template <int PASS>
+// FOLD: what WqPrevious says comes first, in every workgroup.
+template <int PASS, bool FOLD>
 __global__ __launch_bounds__(256) void wq_rows_kernel(const float *w, size_t n, size_t k, const WqState *state, int normalize,
-                                                      int clip, double *row_sums, float *row_max, uint8_t *packed, int8_t *q_i8)
+                                                      int clip, double *row_sums, float *row_max, uint8_t *packed, int8_t *q_i8,
+                                                      WqPrevious prev)
 {
     constexpr int NACC = wq_accumulators(PASS);
     const int lane = threadIdx.x;
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
+    WqState st = wq_state(state);
+    if constexpr (FOLD) {
+        if (prev.pass >= 0) wq_finish_previous(st, prev, row_max, n, k);
+        if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *prev.state = st;
+    }
     if (row >= n) return;
-    const WqView p = wq_view(state, normalize, clip);
+    const WqView p = wq_view(st, normalize, clip);
     double acc[NACC];
 #pragma unroll
     for (int a = 0; a < NACC; ++a) acc[a] = 0.0;
@@ -400,13 +510,11 @@ __global__ __launch_bounds__(256) void wq_rows_kernel(const float *w, size_t n, 
     }
 }
 
-// One workgroup: combines the row sums of every accumulator and derives the scalars of the next stage.  method:
-// TernaryMethod 0..4; custom <= 0: the method's own factor.  WQ_SCALE, the last stage, also publishes the scale and
-// (optionally) the twelve scalars.
+// One workgroup: combines the row sums of every accumulator and derives the scalars of the next stage (state: before, next: after,
+// may be the same).  WQ_SCALE, the last stage, also publishes the scale and (optionally) the twelve scalars.
 template <int PASS>
 __global__ __launch_bounds__(1024) void wq_final_kernel(const double *row_sums, const float *row_max, size_t n, size_t k,
-                                                        WqState *state, int method, float outlier_threshold, float custom,
-                                                        int clip, float *w_scale, float *stats)
+                                                        const WqState *state, WqState *next, WqRule rule, int clip, float *w_scale, float *stats)
 {
     constexpr int NACC = wq_accumulators(PASS);
     __shared__ double tot[NACC];
@@ -423,57 +531,16 @@ __global__ __launch_bounds__(1024) void wq_final_kernel(const double *row_sums, 
     if (lane == 0 && wave < NACC) tot[wave] = s;
     __syncthreads();
     if (threadIdx.x != 0) return;
-    const double count = (double)n * (double)k;
-    WqState st = *state;
-    if constexpr (PASS == WQ_SUM) {
-        st.mean = (float)(tot[0] / count);
-    } else if constexpr (PASS == WQ_SQDIFF) {
-        const float var = (float)(tot[0] / count);
-        st.sd = f32_sqrt(var + 1e-8f);
-    } else if constexpr (PASS == WQ_CLIP_STATS) {
-        st.clip_mean = (float)(tot[0] / count);
-        st.clip_mad = (float)(tot[1] / count);
-        const float spread = f32_mul(outlier_threshold, st.clip_mad);
-        st.lo = st.clip_mean - spread;
-        st.hi = st.clip_mean + spread;
-    } else if constexpr (PASS == WQ_ABS_STATS) {
-        float mx = 0.0f;
+    float mx = 0.0f;
+    if constexpr (PASS == WQ_ABS_STATS)
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, maxima[i]);
-        st.mean_abs = (float)(tot[0] / count);
-        st.max_abs = mx;
-        const bool has_custom = custom > 0.0f;
-        float thr;
-        if (method == 1) thr = f32_mul(st.mean_abs, has_custom ? custom : 0.8f);
-        else if (method == 2)
-            thr = has_custom ? f32_mul(st.mean_abs, custom)
-                             : (st.max_abs > f32_mul(3.0f, st.mean_abs) ? f32_mul(st.mean_abs, 0.5f) : f32_mul(st.mean_abs, 0.7f));
-        else thr = f32_mul(st.mean_abs, has_custom ? custom : 0.7f);  // mean, DetSTE; optimal without its search
-        st.thr = thr;
-    } else if constexpr (PASS == WQ_OPTIMAL) {
-        float best = __builtin_inff(), thr = f32_mul(st.mean_abs, 0.7f);
-#pragma unroll
-        for (int f = 0; f < 10; ++f) {
-            const float mse = (float)(tot[f] / count);
-            if (mse < best) { best = mse; thr = f32_mul(st.mean_abs, wq_factors[f]); }
-        }
-        st.thr = thr;
-    } else {
-        st.num = (float)tot[0];
-        st.den = (float)tot[1];
-        st.scale = fabsf(st.den) < 1.1920929e-07f ? 1.0f : f32_div(st.num, st.den);
-        wq_publish(st, clip, w_scale, stats);
-    }
-    *state = st;
+    WqState st = wq_state(state);
+    wq_derive(st, PASS, tot, mx, (double)n * (double)k, rule);
+    if constexpr (PASS == WQ_SCALE) wq_publish(st, clip, w_scale, stats);
+    *next = st;
 }
 
-__global__ void wq_init_kernel(WqState *state, int empty, int clip, float *w_scale, float *stats)
-{
-    WqState st;
-    st.mean = 0.0f; st.sd = 1.0f; st.clip_mean = 0.0f; st.clip_mad = 0.0f; st.lo = -__builtin_inff(); st.hi = __builtin_inff();
-    st.mean_abs = 0.0f; st.max_abs = 0.0f; st.thr = 0.0f; st.num = 0.0f; st.den = 0.0f; st.scale = 1.0f;
-    *state = st;
-    if (empty) wq_publish(st, clip, w_scale, stats);  // an empty tensor: no pass follows
-}
+__global__ void wq_empty_kernel(int clip, float *w_scale, float *stats) { wq_publish(wq_state(nullptr), clip, w_scale, stats); }
 
 // Ternarise the processed tensor with the threshold found, pack; thread b builds byte b (widths that are no multiple of 4,
 // where a byte holds columns of two rows).
@@ -482,7 +549,7 @@ __global__ __launch_bounds__(256) void wq_ternarize_pack_kernel(const float *w, 
 {
     size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nbytes) return;
-    const WqView p = wq_view(state, normalize, clip);
+    const WqView p = wq_view(*state, normalize, clip);
     unsigned byte = 0;
     for (int j = 0; j < 4; ++j) {
         size_t i = 4 * b + j;
@@ -702,41 +769,62 @@ int launch_quantize_weights(const float *w, size_t n, size_t k, int method, floa
 
 size_t quantize_weights_reference_scratch_bytes(size_t n)
 {
-    return sizeof(double) * WQ_MAX_ACC * (n ? n : 1) + sizeof(float) * (n ? n : 1) + 256;
+    return sizeof(double) * WQ_SCRATCH_SUMS * (n ? n : 1) + sizeof(float) * (n ? n : 1) + 256;
 }
 
 int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int method, int normalize, float outlier_threshold,
                                       float custom_factor, void *scratch, uint8_t *packed, float *w_scale, int8_t *q_i8,
                                       float *stats, hipStream_t stream)
 {
-    // scratch: WqState (256 bytes reserved), then WQ_MAX_ACC * n doubles, then n floats
-    WqState *state = static_cast<WqState *>(scratch);
+    // scratch: two WqStates (256 bytes reserved), then WQ_SCRATCH_SUMS * n doubles, then n floats
+    WqState *states = static_cast<WqState *>(scratch);
     double *row_sums = reinterpret_cast<double *>(static_cast<uint8_t *>(scratch) + 256);
-    float *row_max = reinterpret_cast<float *>(row_sums + WQ_MAX_ACC * (n ? n : 1));
+    float *row_max = reinterpret_cast<float *>(row_sums + WQ_SCRATCH_SUMS * (n ? n : 1));
     const int clip = outlier_threshold > 0.0f ? 1 : 0;
     const size_t count = n * k, nbytes = (count + 3) / 4;
-    hipLaunchKernelGGL(wq_init_kernel, dim3(1), dim3(1), 0, stream, state, count == 0 ? 1 : 0, clip, w_scale, stats);
-    BITNET_HIP_CHECK_LAUNCH("wq_init_kernel");
-    if (count == 0) return BITNET_HIP_OK;
+    if (count == 0) {
+        hipLaunchKernelGGL(wq_empty_kernel, dim3(1), dim3(1), 0, stream, clip, w_scale, stats);
+        BITNET_HIP_CHECK_LAUNCH("wq_empty_kernel");
+        return BITNET_HIP_OK;
+    }
     const dim3 rgrid(blocks_for(n, 4)), rblock(64, 4);
     uint8_t *packed_rows = k % 4 == 0 ? packed : nullptr;  // rows of whole bytes: the last pass writes the codes
-#define BITNET_WQ_PASS(PASS)                                                                                              \
+    // A call with the default configuration and the wait for it, with a launch for every reduction -> with those that the next pass finishes:
+    // 256 x 256 92 -> 74 us, 1280 x 2112 95 -> 84, 2048 x 2048 94 -> 84, 2560 x 2560 105 -> 92, 4096 x 4096 149 -> 145; every workgroup
+    // adds all row sums again, so beyond the line it is the other way round: 6912 x 2560 143 and 155, 14045 x 456 133 and 250.
+    const bool fold = n <= WQ_FOLD_MAX_ROWS;
+    const WqState *state = nullptr;  // of the passes so far
+    WqPrevious prev = {-1, nullptr, nullptr, {method, outlier_threshold, custom_factor}};
+    int at = 0;
+    // FINISH: no pass follows that could finish it, or it has more accumulators than a pass finishes
+#define BITNET_WQ_PASS(PASS, FINISH)                                                                                      \
     do {                                                                                                                  \
-        hipLaunchKernelGGL((wq_rows_kernel<PASS>), rgrid, rblock, 0, stream, w, n, k, state, normalize, clip, row_sums,  \
-                           row_max, packed_rows, q_i8);                                                                   \
+        double *sums = row_sums + (PASS == WQ_OPTIMAL ? 4 : 2 * at) * n;                                                  \
+        prev.state = states + at;                                                                                         \
+        if (fold) hipLaunchKernelGGL((wq_rows_kernel<PASS, true>), rgrid, rblock, 0, stream, w, n, k, state, normalize,   \
+                                     clip, sums, row_max, packed_rows, q_i8, prev);                                       \
+        else hipLaunchKernelGGL((wq_rows_kernel<PASS, false>), rgrid, rblock, 0, stream, w, n, k, state, normalize, clip, \
+                                sums, row_max, packed_rows, q_i8, prev);                                                  \
         BITNET_HIP_CHECK_LAUNCH("wq_rows_kernel");                                                                        \
-        hipLaunchKernelGGL((wq_final_kernel<PASS>), dim3(1), dim3(1024), 0, stream, row_sums, row_max, n, k, state,       \
-                           method, outlier_threshold, custom_factor, clip, w_scale, stats);                               \
-        BITNET_HIP_CHECK_LAUNCH("wq_final_kernel");                                                                       \
+        if (fold) state = states + at;                                                                                    \
+        prev.pass = PASS; prev.sums = sums;                                                                               \
+        if (!fold || FINISH) {                                                                                            \
+            hipLaunchKernelGGL((wq_final_kernel<PASS>), dim3(1), dim3(1024), 0, stream, sums, row_max, n, k, state,       \
+                               states + at, prev.rule, clip, w_scale, stats);                                             \
+            BITNET_HIP_CHECK_LAUNCH("wq_final_kernel");                                                                   \
+            state = states + at;                                                                                          \
+            prev.pass = -1;                                                                                               \
+        }                                                                                                                 \
+        at ^= 1;                                                                                                          \
     } while (0)
     if (normalize) {
-        BITNET_WQ_PASS(WQ_SUM);
-        BITNET_WQ_PASS(WQ_SQDIFF);
+        BITNET_WQ_PASS(WQ_SUM, false);
+        BITNET_WQ_PASS(WQ_SQDIFF, false);
     }
-    if (clip) BITNET_WQ_PASS(WQ_CLIP_STATS);
-    BITNET_WQ_PASS(WQ_ABS_STATS);
-    if (method == 3 && !(custom_factor > 0.0f)) BITNET_WQ_PASS(WQ_OPTIMAL);
-    BITNET_WQ_PASS(WQ_SCALE);
+    if (clip) BITNET_WQ_PASS(WQ_CLIP_STATS, false);
+    BITNET_WQ_PASS(WQ_ABS_STATS, false);
+    if (method == 3 && !(custom_factor > 0.0f)) BITNET_WQ_PASS(WQ_OPTIMAL, true);
+    BITNET_WQ_PASS(WQ_SCALE, true);
 #undef BITNET_WQ_PASS
     if (!packed_rows) {
         hipLaunchKernelGGL(wq_ternarize_pack_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, w, count, state,

@@ -1870,3 +1870,20 @@ def test_forward_of_rows_quantised_by_every_workgroup(m, n, k, norm):
     got = bh.forward_multi([other, layer], dev(x), gamma=gd)
     assert np.array_equal(host(got[0]), orc.bitlinear_forward(x, pk2, 24, f32(0.03), g=g)[0])
     assert np.array_equal(host(got[1]), orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias)[0])
+
+
+@pytest.mark.parametrize("n,k", [(1, 4), (3, 258), (64, 260), (513, 64), (4095, 12), (4096, 20), (4097, 20), (4097, 6)])
+@pytest.mark.parametrize("method,normalize,t", [(0, True, 3.0), (3, True, 3.0), (2, False, 2.5), (3, False, 0.0), (1, True, 0.0)])
+def test_reference_weight_pipeline_with_reductions_finished_by_the_next_pass(n, k, method, normalize, t):
+    """Row counts on both sides of the line from which a launch of its own finishes each reduction, fewer and more rows than a wavefront
+    adds at a time, and every order of the passes."""
+    rng = np.random.default_rng(n + k + method)
+    w = (0.2 + 1.3 * rng.standard_normal((n, k))).astype(f32)
+    w[rng.random(w.shape) < 0.01] *= f32(7.0)
+    cfg = bh.WeightQuantizationConfig(normalize_weights=normalize, outlier_threshold=t, ternary_method=method)
+    got = bh.BitNetWeightQuantizer(cfg).quantize(dev(w))
+    q_ref, s_ref, _, st_ref = orc.quantize_weights_reference(w, method=method, normalize=normalize, outlier_threshold=t, want_details=True)
+    assert np.array_equal(host(got.values), q_ref) and np.array_equal(host(got.packed), orc.pack_2bit(q_ref))
+    assert host(got.scales)[0] == s_ref
+    for name, v in st_ref.items():
+        assert f32(got.stats[name]) == v, (name, got.stats[name], v)
