@@ -489,6 +489,8 @@ __device__ __forceinline__ int row_lane(uint32_t packed, int at)
     }
 }
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte accesses need four-byte alignment only
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int MODE, bool NORM, int NCHB, int RBW>
 __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_chunks,
@@ -1193,10 +1195,12 @@ __global__ __launch_bounds__(256) void gemv_mfma_tg_kernel(const int8_t *hot_a, 
 // columns is contiguous, so an A operand is one dense load into the registers the MFMA reads: no copy through LDS, no
 // gathers of 16 bytes per row, and no barrier before the products.  NT tiles are requested at once (LOOP: more than 16 NT tiles,
 // in batches of NT with the next batch in flight).  The rows' sums for the code offset are an MFMA on a constant operand and
-// leave the wavefront subtracted; the partial results of the wavefronts meet in LDS, and every thread finishes its own
-// outputs.  What a launch takes is one trip to memory, the MFMAs of a wavefront and that exchange.  6912 -> 2560, 16 tokens: 4.1 us
-// (gathering the rows from memory 7.6); a block of the 30-block stack: 25.7 us at 8 tokens, 35.8 at 42 (rows copied to LDS first
-// 30.0 and 50.2).
+// leave the wavefront subtracted; the partial results of the wavefronts meet in LDS, and wavefront r finishes row block r, four
+// outputs a lane.  What a launch takes is one trip to memory, the MFMAs of a wavefront and that exchange, and, with more than one
+// workgroup a compute unit, the issue of vector instructions: 10 wavefronts of some 400 hold the four SIMDs for 2 us.  6912 -> 2560, 16
+// tokens: 4.1 us (gathering the rows from memory 7.6); a block of the 30-block stack: 24.8 us at 8 tokens, 29.2 at 24, 33.1 at 42 (with
+// a thread per output, which took a third more instructions and, with four row blocks, 80 registers, so that a compute unit held
+// two workgroups instead of three: 24.9, 30.6 and 35.0; rows copied to LDS first 30.0 at 8 and 50.2 at 42).
 // Everything that the loads need arrives preloaded, the weights' addresses too: a scalar load of an argument takes as long as
 // the weights do, and the two would add up (2560 columns, 160 row blocks: 0.55 us of 3.4).  Counts of row blocks and their
 // groups are packed, 16 bits each: rows and k-tiles; groups of projection 0, and of 0 and 1 (0xffff where there is no next
@@ -1265,32 +1269,31 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
     __builtin_amdgcn_sched_barrier(0);
 
     asm volatile("" : "+s"(P));
-    const global_ptr<const float> scales = (global_ptr<const float>)(uintptr_t)a_scale, absent = scales;
+    const global_ptr<const float> scales = (global_ptr<const float>)(uintptr_t)a_scale;
     const global_ptr<const float> w_scale = pointer_at<const float>(P, 2), bias = pointer_at<const float>(P, 4), residual = pointer_at<const float>(P, 6);
     const global_ptr<float> out = pointer_at<float>(P, 8);
     const global_ptr<int32_t> acc_out = pointer_at<int32_t>(P, 10);
     const int P_n = (int)P[12];
 
-    // Output e of the workgroup: token e / (16 RB), row block (e / 16) % RB, row e % 16.  Thread tid finishes the outputs tid, tid +
-    // 64 nw, ..: RB at most (a workgroup has four wavefronts at least).  Their operands are requested now, behind the tiles.
-    const int outputs = rows_here * RB * TILE_ROWS, step = 64 * nw;
-    float e_ws = 0.0f, e_bias[RB], e_res[RB], e_scale[RB];
-    {
+    // The weights are the first operand of the MFMA, so lane l of a result holds four consecutive outputs, 4 (l / 16) and on, of token
+    // l % 16: wavefront r finishes row block r with loads and stores of 16 bytes.  Its operands are requested behind the tiles, or, where the
+    // registers are full of tiles, behind the products.
+    constexpr bool REQUEST_EARLY = RB < 4 && !LOOP;
+    const bool finishing = wave < RB;  // a workgroup has four wavefronts at least
+    const int n_block = (rb0 + wave) * TILE_ROWS, n_lane = n_block + 4 * (lane >> 4), t_lane = tg * 16 + min(lane & 15, rows_here - 1);
+    const bool whole = n_block + TILE_ROWS <= P_n;
+    float e_ws = 0.0f, e_scale = 1.0f;
+    v4f_any e_bias = {0.0f, 0.0f, 0.0f, 0.0f}, e_res = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto request = [&]() {
+        if (!(finishing && whole && out)) return;  // uniform over the wavefront
         int lane_zero = 0;
         asm volatile("" : "+v"(lane_zero));
-        e_ws = (out ? w_scale : absent)[lane_zero];
-    }
-#pragma unroll
-    for (int s = 0; s < RB; ++s) {
-        e_bias[s] = 0.0f; e_res[s] = 0.0f; e_scale[s] = 1.0f;
-        if (64 * wave + s * step < outputs) {  // uniform over the wavefront
-            const int e = min(tid + s * step, outputs - 1);
-            const int n = min((rb0 + ((e >> 4) & (RB - 1))) * TILE_ROWS + (e & 15), P_n - 1), t = tg * 16 + e / (16 * RB);
-            e_scale[s] = (out ? scales + t : absent)[0];
-            e_bias[s] = (bias ? bias + n : absent)[0];
-            e_res[s] = (residual ? residual + ((size_t)t * P_n + n) : absent)[0];
-        }
-    }
+        e_ws = w_scale[lane_zero];
+        e_scale = scales[t_lane];
+        if (bias) e_bias = *(global_ptr<const v4f_any>)(bias + n_lane);
+        if (residual) e_res = *(global_ptr<const v4f_any>)(residual + ((size_t)t_lane * P_n + n_lane));
+    };
+    if constexpr (REQUEST_EARLY) request();
     __builtin_amdgcn_sched_barrier(0);
 
     v4i acc[RB], sums = {0, 0, 0, 0};
@@ -1303,12 +1306,12 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
             if (kt0 + nw * u >= kt_count) break;  // uniform over the wavefront
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][t], ones, sums, 0, 0, 0);
+                sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, a[u][t], sums, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < RB; ++r) {
                     const unsigned wd = wt[u][r][t];
                     const v4i bf = {(int)(wd & 0x03030303u), (int)((wd >> 2) & 0x03030303u), (int)((wd >> 4) & 0x03030303u), (int)((wd >> 6) & 0x03030303u)};
-                    acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][t], bf, acc[r], 0, 0, 0);
+                    acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf, a[u][t], acc[r], 0, 0, 0);
                 }
             }
         }
@@ -1331,40 +1334,68 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
     } else {
         multiply(af, w, wave);
     }
-    // Component i of a lane's result is token 4 (lane / 16) + i, row lane % 16.  It is stored at component (i + r) % 4, so that the
-    // reads below, of RB row blocks and 16 rows at once, spread over the banks.
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-        const v4i d = acc[r] - sums;
-        part[((size_t)wave * RB + r) * 64 + lane] = (v4i){d[(0 - r) & 3], d[(1 - r) & 3], d[(2 - r) & 3], d[(3 - r) & 3]};
+    if constexpr (!REQUEST_EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        request();
     }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) part[((size_t)wave * RB + r) * 64 + lane] = acc[r] - sums;
     lds_barrier();
-    const int *part_i = reinterpret_cast<const int *>(part);
+    if (!finishing) return;
+    const v4i *from = part + wave * 64 + lane;
+    v4i total = {0, 0, 0, 0};
+    int v = 0;
+    for (; v + 4 <= nw; v += 4) {  // uniform, as the rest is
+        v4i got[4];
 #pragma unroll
-    for (int s = 0; s < RB; ++s) {
-        const int e = tid + s * step;
-        if (e >= outputs) break;
-        const int r = (e >> 4) & (RB - 1), tl = e / (16 * RB), lr = e & 15;
-        const int *from = part_i + r * 256 + ((tl >> 2) * 16 + lr) * 4 + ((tl + r) & 3);
-        int total = 0;
-        for (int v = 0; v < nw; v += 4) {  // past the last wavefront: its slot again, not added
+        for (int i = 0; i < 4; ++i) got[i] = from[(v + i) * (RB * 64)];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int got = from[min(v + j, nw - 1) * (RB * 256)];
-                total += v + j < nw ? got : 0;
-            }
-        }
-        const int n = (rb0 + r) * TILE_ROWS + lr;
-        if (n >= P_n) continue;
-        const size_t o = (size_t)(tg * 16 + tl) * P_n + n;
-        if (acc_out) acc_out[o] = total;
+        for (int i = 0; i < 4; ++i) total = total + got[i];
+    }
+    if (v < nw) {
+        v4i got[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) got[i] = from[min(v + i, nw - 1) * (RB * 64)];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (v + i < nw) total = total + got[i];
+    }
+    if (!row_ok) return;
+    const size_t o = (size_t)t_lane * P_n + n_lane;
+    if (whole) {
+        if (acc_out) *(global_ptr<v4i_any>)(acc_out + o) = total;
         if (out) {
-            const float scaled = f32_mul((float)total, e_ws);
-            float y = div_by_invariant_unchecked(scaled, e_scale[s], recip_of_ok_divisor(e_scale[s]));
-            if (__builtin_expect(!(invariant_divisor_ok(e_scale[s]) && dividend_ok(scaled)), 0)) y = f32_div(scaled, e_scale[s]);
-            if (bias) y = f32_add(y, e_bias[s]);
-            if (residual) y = f32_add(y, e_res[s]);
-            out[o] = y;
+            v4f_any y;
+            bool short_ok = invariant_divisor_ok(e_scale);
+            const float recip = recip_of_ok_divisor(e_scale);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float scaled = f32_mul((float)total[i], e_ws);
+                short_ok = short_ok && dividend_ok(scaled);
+                y[i] = div_by_invariant_unchecked(scaled, e_scale, recip);
+            }
+            if (__builtin_expect(!short_ok, 0)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = f32_div(f32_mul((float)total[i], e_ws), e_scale);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (bias) y[i] = f32_add(y[i], e_bias[i]);
+                if (residual) y[i] = f32_add(y[i], e_res[i]);
+            }
+            *(global_ptr<v4f_any>)(out + o) = y;
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // the last row block of a projection
+        if (n_lane + i >= P_n) break;
+        if (acc_out) acc_out[o + i] = total[i];
+        if (out) {
+            float y = f32_div(f32_mul((float)total[i], w_scale[0]), scales[t_lane]);
+            if (bias) y = f32_add(y, bias[n_lane + i]);
+            if (residual) y = f32_add(y, residual[o + i]);
+            out[o + i] = y;
         }
     }
 }

@@ -1887,3 +1887,24 @@ def test_reference_weight_pipeline_with_reductions_finished_by_the_next_pass(n, 
     assert host(got.scales)[0] == s_ref
     for name, v in st_ref.items():
         assert f32(got.stats[name]) == v, (name, got.stats[name], v)
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 1, 1280), (16, 15, 2560), (17, 40, 2304), (31, 4097, 1536), (33, 2573, 2560), (48, 13827, 2560), (95, 5001, 2304),
+                                   (15, 2561, 6912), (30, 3330, 4352), (20, 20000, 4608), (13, 1023, 12288), (40, 6007, 9216), (300, 1030, 2560)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_token_gemv_outputs_that_end_inside_a_row_block(m, n, k, extras):
+    """Four outputs a lane: rows that start at any multiple of four bytes, last row blocks of 1 to 15 rows, token groups of 1 to 16 rows,
+    one, two and four row blocks a workgroup, k-tiles in one batch and in several."""
+    rng = np.random.default_rng(m + n + k)
+    x = synth_activations(rng, m, k, outliers=True)
+    x[0] *= f32(1e-30)
+    g = (1 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32)
+    nbytes = (n * k + 3) // 4
+    pk = random_packed_ternary(rng, 1, 4 * nbytes)
+    bias, res = (rng.standard_normal(n, dtype=f32), rng.standard_normal((m, n), dtype=f32)) if extras else (None, None)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=extras), "ends")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    if extras:
+        layer.update_bias(dev(bias))
+    ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias, residual=res)[0]
+    assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g), residual=dev(res) if extras else None)), ref)
