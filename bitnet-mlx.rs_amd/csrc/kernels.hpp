@@ -105,9 +105,10 @@ inline bool gemm_takes_tokens(size_t m, size_t k, size_t n_blocks, const void *a
 // 10 widths, 10 to 192 tokens, within 20 %; the GEMM's start with 2.5 us on top, what weights that come from HBM cost it more than the
 // GEMV, which asks for all of its tiles at once (blocks of a decoder, each with its own weights, at 18 and 24 tokens of 3072 -> 18048
 // and 2304 -> 18176; 42 tokens of 2560 -> 6912 + 6912 by the GEMM: a 30-block step 1060 -> 1115 us).  GEMV / GEMM, quantiser included,
-// in us: 2560 -> 13824 at 32 / 42 / 95 10.1 / 10.6, 12.1 / 11.0, 21.6 / 12.2; 4096 -> 12288 at 20 / 42 / 95 12.1 / 12.0, 17.2 / 12.2,
-// 24.3 / 17.6; 8192 -> 8192 at 32 / 42 / 95 11.3 / 15.7, 19.0 / 17.3, 23.6 / 18.2; 2560 -> 30000 at 16 / 20 / 48 10.5 / 12.7, 17.8 /
-// 12.5, 23.6 / 14.5; 6912 -> 2560 at 95 / 112 11.1 / 12.3, 15.7 / 12.5; 2560 -> 2560 at 95 / 192 8.1 / 9.3, 10.5 / 10.3.
+// in us: 2560 -> 13824 at 32 / 42 / 95 7.8 / 9.3, 9.6 / 9.8, 13.8 / 11.8; 4096 -> 12288 at 32 / 42 / 95 9.1 / 11.1, 11.2 / 11.5, 15.7 / 14.0;
+// 8192 -> 8192 at 32 / 42 / 95 9.5 / 13.5, 13.6 / 14.0, 19.1 / 17.3; 2560 -> 30000 at 20 / 42 11.5 / 11.7, 15.0 / 12.5; 6912 -> 2560 at 95
+// 9.6 / 12.4; 2304 -> 6912 at 95 8.5 / 9.7; 1536 -> 12000 at 80 8.3 / 10.0; ten blocks of 4096 columns with a 12288-wide FFN at 32
+// tokens, gate and up by either: 426 / 441.
 size_t gemm_one_round_ns(size_t m, size_t k, size_t n);  // gemm_w2a8.hip; 0 where no tile of that kernel holds the launch in one round
 constexpr size_t GEMM_START_NS = 7500, GEMM_LEAST_STAGE_NS = 154;
 inline bool gemm_beats_token_gemv(size_t m, size_t k, size_t n_blocks, const void *a)
@@ -116,7 +117,7 @@ inline bool gemm_beats_token_gemv(size_t m, size_t k, size_t n_blocks, const voi
         (reinterpret_cast<uintptr_t>(a) & 15) != 0)
         return false;
     const size_t kt = k / TILE_K, blocks = n_blocks * ((m + 15) / 16), near = blocks * (kt < 16 ? kt : 16), all = blocks * kt;
-    const size_t gemv_ns = 3300 + near / 4 + (all - near) / 8 + (m > 64 ? 1000 : 0);
+    const size_t gemv_ns = 3300 + near * 2 / 11 + (all - near) / 8 + (m > 64 ? 1000 : 0);
     if (gemv_ns <= GEMM_START_NS + GEMM_LEAST_STAGE_NS * kt) return false;
     const size_t gemm_ns = gemm_one_round_ns(m, k, n_blocks * 16);
     return gemm_ns != 0 && gemm_ns < gemv_ns;
