@@ -151,11 +151,26 @@ size_t launch_group_blocks(const bitnet_hip_bitlinear *const *layers, size_t cou
 }
 
 // Whether projections of plain rows [m, in] need no scratch: the quantiser runs inside the launch.
-bool quantises_in_launch(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order)
+bool quantises_in_launch(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order,
+                         bool alone = true)
 {
     const size_t in = layers[0]->in_features, blocks = launch_group_blocks(layers, count);
-    return gemv_rowq_takes(x, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, sum_order, blocks, true) ||
+    return gemv_rowq_takes(x, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, sum_order, blocks, alone) ||
            gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, blocks);
+}
+
+// Whether projections that could quantise inside their launch are faster in two launches, since the stream is being captured and a
+// replay costs the host nothing per launch (gemv_rowq_takes).  The stream is asked only where that decides.
+bool recorded_in_two(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order,
+                     hipStream_t s)
+{
+    if (m < 2 || !s || quantises_in_launch(layers, count, x, m, gamma, sum_order, false)) return false;  // the null stream is never captured
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
+        (void)hipGetLastError();  // the launches below must not report it
+        return false;
+    }
+    return capturing == hipStreamCaptureStatusActive;
 }
 
 // Runs `count` projections that share one input row block [m, k].  At decode token counts the quantiser runs
@@ -869,6 +884,18 @@ size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *l
     return quant_scratch_bytes(m, padded_k(in));
 }
 
+size_t bitnet_hip_bitlinear_forward_scratch_on(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
+                                               const float *gamma, int sum_order, void *stream)
+{
+    if (!layers || count == 0 || m == 0) return 0;
+    for (size_t j = 0; j < count; ++j)
+        if (!layers[j]) return 0;
+    if (quantises_in_launch(layers, count, x, m, gamma, sum_order) &&
+        !recorded_in_two(layers, count, x, m, gamma, sum_order, as_stream(stream)))
+        return 0;
+    return quant_scratch_bytes(m, padded_k(layers[0]->in_features));
+}
+
 int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, const size_t *dims, int rank,
                                  const float *gamma, float eps, int sum_order, const float *residual, float *out,
                                  void *workspace, size_t workspace_bytes, int8_t *dbg_q, float *dbg_a_scale,
@@ -898,7 +925,10 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
 
     hipStream_t s = as_stream(stream);
     const bool debug = dbg_q || dbg_a_scale || dbg_acc;
-    const bool fused = quantises_in_launch(&layer, 1, x, m, gamma, sum_order);
+    bool fused = quantises_in_launch(&layer, 1, x, m, gamma, sum_order);
+    const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
+                        recorded_in_two(&layer, 1, x, m, gamma, sum_order, s);
+    fused = fused && !in_two;
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {dbg_q, dbg_a_scale, nullptr};
@@ -923,7 +953,7 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     float *outs[1] = {out};
     int32_t *accs[1] = {dbg_acc};
     int rc = run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s);
+                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, !in_two);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -970,13 +1000,16 @@ int bitnet_hip_bitlinear_forward_noalloc(bitnet_hip_bitlinear *layer, const floa
 
     std::shared_lock<std::shared_mutex> guard(layer->lock);
     if (!layer->has_weights) return fail(BITNET_HIP_NOT_INITIALIZED, "forward_noalloc: the layer has no weights yet");
-    const size_t ldq = quant_scratch_bytes(m, padded_k(in)) <= NOALLOC_SCRATCH_BYTES ? padded_k(in) : in;
+    const bool padded = quant_scratch_bytes(m, padded_k(in)) <= NOALLOC_SCRATCH_BYTES;
+    const size_t ldq = padded ? padded_k(in) : in;
     const QuantScratch sc = carve_scratch(ws, m, ldq);
     bitnet_hip_bitlinear *layers[1] = {layer};
     const float *res[1] = {residual};
     float *outs[1] = {out};
+    const bool in_two = padded && quantises_in_launch(layers, 1, x, m, gamma, sum_order) &&
+                        recorded_in_two(layers, 1, x, m, gamma, sum_order, as_stream(stream));
     return run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                           nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, as_stream(stream));
+                           nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, as_stream(stream), !in_two);
 }
 
 int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
@@ -999,7 +1032,10 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     }
     const size_t in = layers[0]->in_features;
     hipStream_t s = as_stream(stream);
-    const bool fused = quantises_in_launch(layers, count, x, m, gamma, sum_order);
+    bool fused = quantises_in_launch(layers, count, x, m, gamma, sum_order);
+    const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
+                        recorded_in_two(layers, count, x, m, gamma, sum_order, s);
+    fused = fused && !in_two;
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {nullptr, nullptr, nullptr};
@@ -1017,7 +1053,7 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
         sc = carve_scratch(ws, m, ldq);
     }
     int rc = run_projections(layers, (int)count, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order,
-                             nullptr, outs, nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, s);
+                             nullptr, outs, nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, s, !in_two);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)

@@ -279,22 +279,29 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
     if (!gqa && input_mode != BITNET_HIP_INPUT_PLAIN) return false;
     if (gqa && (head_dim % 16 != 0 || gqa_group == 0 || gamma)) return false;
     const size_t width = gqa ? k / gqa_group : k;
-    // In one round of workgroups only: a second one quantises again.  A row of 16 tokens costs a workgroup 0.4 us at 256 columns and
-    // 1.0 us at 1024, the launch it saves 0.5 us of the GPU's time in a recorded step and 2.5 us of the host's outside one (9 x 256 ->
-    // 2560: 5.1 -> 4.8 us recorded, 7.2 -> 4.7 us as calls; 16 x 1024 -> 2560: 5.1 -> 6.0 recorded, so up to 12288 elements a
-    // token group in a step and any row that fits in a call of its own).
+    // In one round of workgroups only: a second one quantises again.  What a workgroup pays for it grows with the columns that it
+    // quantises, those of its up to 16 rows together; what it saves is the quantiser's launch, 0.5 to 1 us of the GPU's time and, in a call
+    // that nothing records, 2.5 us of the host's.  So a call of its own is one launch wherever the kernel takes it, and a recorded one
+    // (alone == false: a decoder step, a capture of the caller's) where the GPU is faster so.  Recorded, two launches -> one, us:
+    // plain rows of up to 1024 columns, any number of tokens: 16 x 1024 -> 2560 4.8 -> 4.2, 64 x 1024 -> 2560 5.5 -> 5.0, 512 x 1024 -> 512 6.4 -> 5.3;
+    // with norm, up to 12288 columns a workgroup: 9 x 256 -> 2560 5.1 -> 4.7, 9 x 1024 -> 9000 6.2 -> 6.0; beyond them 16 x 1024 -> 2560 5.2 -> 6.0,
+    // 64 x 1024 -> 512 5.1 -> 5.8, 128 x 512 -> 512 5.1 -> 5.6;
+    // plain rows above 1024 columns, up to the same 12288: 5 x 2048 -> 9000 6.5 -> 5.8, 9 x 1280 -> 2560 5.1 -> 4.8; beyond them 16 x 1280 -> 2560
+    // 5.1 -> 5.4, 16 x 2048 -> 2560 5.2 -> 6.4, 40 x 2048 -> 5120 6.2 -> 7.4, 256 x 1536 -> 512 5.8 -> 6.0, but above 256 tokens, where the quantiser's
+    // launch is longer itself, 512 x 1280 -> 512 7.0 -> 6.3, 512 x 2048 -> 512 8.3 -> 7.5.
     const size_t in_group = m < 16 ? m : 16, tgroups = (m + 15) / 16;
+    const bool few_columns = width * in_group <= 12288;
     if (m < 2 || m > (size_t)GEMV_WIDE_MAX_M || (blocks + 3) / 4 * tgroups > 256) return false;
-    // More than 95 tokens, and rows above 1024 columns without a norm: calls of their own, as long as no compute unit quantises more than
-    // 2048 columns for its 16 tokens (with a norm, in two rounds: not).  In two launches -> here, us as calls / recorded: 104 x 1024 -> 512
-    // 8.0 / 4.6 -> 5.2 / 4.0, 512 x 1024 -> 512 8.0 / 7.1 -> 5.5 / 5.3, 128 x 512 -> 2048 with norm 8.0 / 6.5 -> 6.2 / 6.2, 16 x 1280 -> 2560 8.0 /
-    // 4.8 -> 5.4 / 5.1, 64 x 1280 -> 2560 8.0 / 6.7 -> 6.0 / 5.9, 16 x 2048 -> 2560 8.0 / 4.9 -> 6.0 / 5.9, 40 x 2048 -> 5120 7.8 / 6.3 -> 7.3 / 7.1.
-    // Beyond the line: 16 x 1280 -> 2560 with norm 8.1 / 5.1 -> 7.1 / 7.2, 40 x 2560 -> 5120 9.1 -> 9.1 as calls.
+    // More than 95 tokens, and rows above 1024 columns without a norm: as long as no compute unit quantises more than 2048 columns for its
+    // 16 tokens (with a norm, in two rounds: not).  In two launches -> here, us a call: 104 x 1024 -> 512 8.0 -> 5.2, 512 x 1024 -> 512 8.0 -> 5.5,
+    // 128 x 512 -> 2048 with norm 8.0 -> 6.2, 16 x 1280 -> 2560 8.0 -> 5.4, 64 x 1280 -> 2560 8.0 -> 6.0, 16 x 2048 -> 2560 8.0 -> 6.0, 40 x 2048 -> 5120
+    // 7.8 -> 7.3.  Beyond the line: 16 x 1280 -> 2560 with norm 8.1 -> 7.1 and recorded 5.1 -> 7.2, 40 x 2560 -> 5120 9.1 -> 9.1.
     if (m > (size_t)GEMV_MAX_M || width > SHORT_WIDTH) {
         const size_t rb = row_blocks_per_workgroup(blocks, tgroups), rounds = rounds_of((blocks + rb - 1) / rb, tgroups);
-        if (gqa || !alone || (gamma ? rounds > 1 || width > SHORT_WIDTH : rounds * width > MAX_WIDTH)) return false;
+        if (gqa || (gamma ? !alone || rounds > 1 || width > SHORT_WIDTH : rounds * width > MAX_WIDTH)) return false;
     }
-    if (width % 4 != 0 || ldx != width || width > MAX_WIDTH || (!gqa && !alone && width * in_group > 12288)) return false;
+    if (width % 4 != 0 || ldx != width || width > MAX_WIDTH) return false;
+    if (!gqa && !alone && !few_columns && (gamma || (width > SHORT_WIDTH && m <= 256))) return false;
     if (k_tiles(k) > (size_t)MAX_KT || k > 0xffff || blocks > GEMV_ROWS_MAX_BLOCKS) return false;
     // Up to eight tokens gemv_fused16_kernel may be one launch as well, with a set of workgroups for every token.  It has fewer rows to
     // quantise but reads the weight tiles once a token, so it is ahead while its workgroups have few tiles to walk.  A decoder block

@@ -157,7 +157,8 @@ inline bool gemv_rows_takes(size_t m, size_t k, size_t n_blocks, const void *a)
 }
 int launch_gemv_rows(const GemvProj *projs, int nproj, const int8_t *a, const float *a_scale, size_t m, size_t k, hipStream_t stream);
 // gemv_rowq.hip: several tokens on short f32 rows, quantised by every workgroup of the one launch.  Only where gemv_rowq_takes()
-// says so; blocks: 16-row blocks of all projections of the launch; alone: the launch is a call of its own, not one of a step.
+// says so; blocks: 16-row blocks of all projections of the launch; alone: the launch is a call of its own, not one of a step or of a
+// caller's capture.
 bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_mode, size_t gqa_group, size_t head_dim,
                      const float *gamma, int sum_order, size_t blocks, bool alone);
 int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m, size_t k, int input_mode, size_t gqa_group, size_t head_dim,

@@ -130,6 +130,7 @@ def load_library() -> C.CDLL:
         "bitnet_hip_bitlinear_workspace_size": (sz, [vp, sz]),
         "bitnet_hip_bitlinear_forward_scratch": (sz, [vp, vp, sz, vp, i32]),
         "bitnet_hip_bitlinear_forward_multi_scratch": (sz, [C.POINTER(vp), sz, vp, sz, vp, i32]),
+        "bitnet_hip_bitlinear_forward_scratch_on": (sz, [C.POINTER(vp), sz, vp, sz, vp, i32, vp]),
         "bitnet_hip_bitlinear_forward": (i32, [vp, vp, C.POINTER(sz), i32, vp, f32, i32, vp, vp, vp, sz, vp, vp, vp, vp]),
         "bitnet_hip_bitlinear_forward_noalloc": (i32, [vp, vp, C.POINTER(sz), i32, vp, f32, i32, vp, vp, vp]),
         "bitnet_hip_bitlinear_forward_multi": (i32, [C.POINTER(vp), sz, vp, sz, vp, f32, i32, C.POINTER(vp), vp, sz, vp]),

@@ -157,7 +157,7 @@ PyObject *forward(PyObject *const *args, Py_ssize_t nargs)
     }
     // scratch only where the call runs the stand-alone quantiser
     const float *xp = x->const_data_ptr<float>();
-    const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch(l.handle, xp, (size_t)m, gamma, (int)order);
+    const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch_on(&l.handle, 1, xp, (size_t)m, gamma, (int)order, stream.handle);
     at::Tensor ws;
     if (ws_bytes) ws = new_on(stream, {(int64_t)((ws_bytes + 3) / 4)}, x->options());
     float *yp = y->data_ptr<float>();
@@ -213,7 +213,7 @@ PyObject *forward_multi(PyObject *const *args, Py_ssize_t nargs)
         ptrs[j] = outs[j].data_ptr<float>();
     }
     const float *xp = x->const_data_ptr<float>();
-    const size_t ws_bytes = bitnet_hip_bitlinear_forward_multi_scratch(handles, (size_t)count, xp, (size_t)m, gamma, (int)order);
+    const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch_on(handles, (size_t)count, xp, (size_t)m, gamma, (int)order, stream.handle);
     at::Tensor ws;
     if (ws_bytes) ws = new_on(stream, {(int64_t)((ws_bytes + 3) / 4)}, x->options());
     void *wp = ws_bytes ? ws.data_ptr() : nullptr;

@@ -135,6 +135,8 @@ extern "C" {
                                                 sum_order: c_int) -> usize;
     pub fn bitnet_hip_bitlinear_forward_multi_scratch(layers: *const *mut bitnet_hip_bitlinear, count: usize, x: *const f32,
                                                       m: usize, gamma: *const f32, sum_order: c_int) -> usize;
+    pub fn bitnet_hip_bitlinear_forward_scratch_on(layers: *const *mut bitnet_hip_bitlinear, count: usize, x: *const f32,
+                                                   m: usize, gamma: *const f32, sum_order: c_int, stream: *mut c_void) -> usize;
     pub fn bitnet_hip_bitlinear_forward(layer: *mut bitnet_hip_bitlinear, x: *const f32, dims: *const usize,
                                         rank: c_int, gamma: *const f32, eps: f32, sum_order: c_int,
                                         residual: *const f32, out: *mut f32, workspace: *mut c_void,

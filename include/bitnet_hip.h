@@ -386,6 +386,11 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
 /* Bytes of workspace that call needs; 0 where it needs none (as bitnet_hip_bitlinear_forward_scratch). */
 size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
                                                   const float *gamma, int sum_order);
+/* Bytes of workspace with which a forward (count = 1) or forward_multi call on `stream` is fastest: as the two functions above say,
+ * and workspace_size(m) as well where the stream is being captured and a replay is faster with the quantiser as a launch of its
+ * own.  A captured call that gets less is one launch, as it is outside a capture. */
+size_t bitnet_hip_bitlinear_forward_scratch_on(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
+                                               const float *gamma, int sum_order, void *stream);
 
 /* The contraction + epilogue of a layer on activations that are already quantised:
  * TernaryProcessor::ternary_matmul (bitnet-inference/src/engine/ternary_operations.rs:87-113) /

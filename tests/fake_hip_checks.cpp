@@ -62,6 +62,7 @@ hipError_t make(T *out)
 }  // namespace fake
 
 extern "C" {
+hipError_t hipGetSymbolAddress(void **p, const void *) { static char held[1 << 21]; *p = held; return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipGetLastError() { return fake::launch_answer; }
 const char *hipGetErrorString(hipError_t) { return "as told"; }
@@ -334,6 +335,53 @@ void gguf_header_is_read_in_stream_order()
     bitnet_hip_bitlinear_destroy(layer);
 }
 
+// A call of several tokens on short rows is one launch in which every workgroup quantises, which saves host time.  Recorded into a
+// caller's graph it is the two launches that the GPU is faster with, as long as the caller gave scratch for them.
+void recorded_calls_on_short_rows()
+{
+    const struct {
+        size_t m, k, n;
+        bool norm;
+        size_t recorded;  // launches
+    } calls[] = {{16, 2048, 2560, false, 2}, {40, 2048, 5120, false, 2}, {16, 1280, 2560, false, 2}, {256, 1536, 512, false, 2}, {16, 1024, 2560, true, 2},
+                 {128, 512, 512, true, 2},   {9, 1280, 2560, false, 1},  {512, 2048, 512, false, 1}, {16, 1024, 2560, false, 1}, {512, 1024, 512, false, 1},
+                 {9, 1024, 2560, true, 1},   {1, 2048, 2560, false, 1}};
+    for (const auto &t : calls) {
+        bitnet_hip_bitlinear *layer = nullptr;
+        CHECK(bitnet_hip_bitlinear_create(t.k, t.n, 0, &layer) == BITNET_HIP_OK);
+        const std::vector<uint8_t> codes(t.n * t.k / 4, 0x22);
+        CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, codes.data(), codes.size(), 0.5f, 0, nullptr) == BITNET_HIP_OK);
+        auto x = DeviceTensor::zeros({t.m, t.k}).unwrap(), out = DeviceTensor::zeros({t.m, t.n}).unwrap(), ones = DeviceTensor::zeros({t.k}).unwrap();
+        const size_t dims[2] = {t.m, t.k}, full = bitnet_hip_bitlinear_workspace_size(layer, t.m);
+        const float *gamma = t.norm ? ones.data() : nullptr;
+        std::vector<uint8_t> ws(full);
+        float *const outs[1] = {out.data()};
+        const auto launches = [&](size_t given) {
+            fake::calls.clear();
+            CHECK(bitnet_hip_bitlinear_forward(layer, x.data(), dims, 2, gamma, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, out.data(), given ? ws.data() : nullptr,
+                                               given, nullptr, nullptr, nullptr, side) == BITNET_HIP_OK);
+            const size_t one = fake::count("launch");
+            fake::calls.clear();
+            CHECK(bitnet_hip_bitlinear_forward_multi(&layer, 1, x.data(), t.m, gamma, 1e-5f, BITNET_HIP_SUM_BLOCK256, outs, given ? ws.data() : nullptr, given,
+                                                     side) == BITNET_HIP_OK);
+            CHECK(fake::count("launch") == one);
+            return one;
+        };
+        const auto static_scratch = [&] {
+            fake::calls.clear();
+            CHECK(bitnet_hip_bitlinear_forward_noalloc(layer, x.data(), dims, 2, gamma, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, out.data(), side) == BITNET_HIP_OK);
+            return fake::count("launch");
+        };
+        const auto scratch = [&](hipStream_t s) { return bitnet_hip_bitlinear_forward_scratch_on(&layer, 1, x.data(), t.m, gamma, BITNET_HIP_SUM_BLOCK256, s); };
+        CHECK(launches(full) == 1 && launches(0) == 1 && static_scratch() == 1 && scratch(side) == 0);
+        fake::capturing = side;
+        CHECK(launches(full) == t.recorded && launches(full - 1) == 1 && launches(0) == 1 && static_scratch() == t.recorded);
+        CHECK(scratch(side) == (t.recorded == 2 ? full : 0) && scratch(nullptr) == 0);
+        fake::capturing = nullptr;
+        bitnet_hip_bitlinear_destroy(layer);
+    }
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -348,6 +396,7 @@ const Check checks[] = {
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
+    {"recorded_calls_on_short_rows", recorded_calls_on_short_rows},
 };
 
 }  // namespace

@@ -609,6 +609,37 @@ def test_forward_in_hip_graph_replays_match_eager(m):
         assert np.array_equal(host(other), ref)
 
 
+@pytest.mark.parametrize("m,n,k,norm", [(16, 2560, 2048, False), (17, 33, 1284, False), (256, 100, 1540, False), (512, 40, 2048, False), (9, 33, 1280, False),
+                                        (16, 300, 1024, True), (96, 33, 260, True), (9, 300, 1024, True)])
+def test_recorded_calls_on_short_rows_replay_the_eager_result(m, n, k, norm):
+    """Short rows on both sides of the line beyond which a captured call takes two launches: with a workspace, with scratch of the
+    graph's own pool (the native call path), in the static scratch and for several layers, three replays each."""
+    rng = np.random.default_rng(m + n + k)
+    pk = random_packed_ternary(rng, n, k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "recorded")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    x, g = synth_activations(rng, m, k, outliers=True), rng.standard_normal(k, dtype=f32) if norm else None
+    ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g)[0]
+    xd, gd = dev(x), dev(g) if norm else None
+    ws = torch.empty((layer.workspace_size(m),), dtype=torch.uint8, device="cuda")
+    outs = [torch.empty((m, n), device="cuda") for _ in range(2)]
+    layer.forward_noalloc(xd, outs[1], gamma=gd)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer.forward(xd, gamma=gd, out=outs[0], workspace=ws)
+        made = [layer.forward(xd, gamma=gd)] + bh.forward_multi([layer, layer], xd, gamma=gd)
+        layer.forward_noalloc(xd, outs[1], gamma=gd)
+    for _ in range(3):
+        for y in outs + made:
+            y.zero_()
+        other = layer.forward(xd, gamma=gd)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(np.array_equal(host(y), ref) for y in outs + made + [other])
+
+
 @pytest.mark.parametrize("n", [1, 4, 5, 6, 1000, 10001, 2560 * 640])
 def test_base3_pack_unpack_bit_exact(n):
     """Base3PackedPacker on the GPU against the oracle, ragged tails included; decoding every byte value."""
