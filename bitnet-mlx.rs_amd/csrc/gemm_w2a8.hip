@@ -1034,6 +1034,9 @@ const Ld8Tile *choose_ld8(size_t m, const size_t *n, int nproj, size_t *stage_ns
     return best;
 }
 
+constexpr size_t LD8_LEAST_K = 1024;      // rows shorter than four stages do not take gemm_ld8_kernel (launch_gemm_multi)
+constexpr size_t LARGE_TILES_FROM = 640;  // tiles of 128 x 160 from which gemm_dma_kernel takes its largest ones
+
 template <int BM, int BN>
 int launch_tile(GemmParams p, hipStream_t stream)
 {
@@ -1051,10 +1054,17 @@ int launch_tile(GemmParams p, hipStream_t stream)
 
 }  // namespace
 
-size_t gemm_one_round_ns(size_t m, size_t k, size_t n)
+// What a launch takes (ns) beyond what the token GEMV takes as well, for the choice between the two (gemm_beats_token_gemv): where one
+// round of gemm_ld8_kernel holds it, its start, its stages (the cost of choose_ld8 is that of a stage alone; with what both kernels do taken
+// off, five eighths of it) and an epilogue by the outputs of whole tiles; elsewhere its start and, per output of a row of tiles (64
+// tokens; 128 from LARGE_TILES_FROM on), the k-tiles.
+size_t gemm_beyond_ns(size_t m, size_t k, size_t n)
 {
+    const size_t kt = k / TILE_K, rows64 = (m + 63) / 64, rows128 = (m + 127) / 128;
     size_t stage_ns = 0;
-    return choose_ld8(m, &n, 1, &stage_ns) ? GEMM_START_NS + stage_ns * (k / TILE_K) * 11 / 10 : 0;
+    if (k >= LD8_LEAST_K && choose_ld8(m, &n, 1, &stage_ns)) return 2800 + stage_ns * kt * 5 / 8 + rows64 * n / 40;
+    const bool large = rows128 * ((n + 159) / 160) >= LARGE_TILES_FROM;
+    return 2300 + (large ? 2 * rows128 : rows64) * n * kt / 85;
 }
 
 // Up to GEMM_MAX_PROJ projections of the same activation matrix in one launch of the LDS-direct kernels (q, k, v
@@ -1087,13 +1097,13 @@ int launch_gemm_multi(const GemvProj *projs, int nproj, const int8_t *a, const i
     p.nproj = nproj; p.a = a; p.a_sum = a_sum; p.a_scale = a_scale; p.m = (int)m; p.k = (int)k; p.kt_count = (int)k_tiles(k);
     // gemm_ld8_kernel where one round of its workgroups holds the launch (256 compute units); with less than four stages its start and
     // epilogue cost more than the shorter loop saves (1000 x 512 -> 2560: 11.0 us, 9.6 with the kernels below).
-    if (k >= 1024) {
+    if (k >= LD8_LEAST_K) {
         size_t widths[GEMM_MAX_PROJ], stage_ns = 0;
         for (int j = 0; j < nproj; ++j) widths[j] = projs[j].n;
         const Ld8Tile *tile = choose_ld8(m, widths, nproj, &stage_ns);
         if (tile) return tile->launch(p, stream);
     }
-    if (tiles >= 640) {
+    if (tiles >= LARGE_TILES_FROM) {
         // 128 x 256 tiles as four wavefronts of 128 x 64 side by side, two workgroups per compute unit: half the unpacking per MFMA
         // (a weight fragment serves eight token fragments instead of four) and a tenth fewer bytes loaded per output.  Per unit of work it takes
         // 0.95 of the time of 128 x 160, so it is chosen where the outputs of the fullest compute unit leave that gain:

@@ -81,52 +81,36 @@ int launch_gemv_base3(const uint8_t *tiled, const int8_t *a, int32_t *acc, float
 // gemv_w2a8.hip
 int launch_gemv_rowmajor(const uint8_t *packed, const int8_t *a, int32_t *out, size_t n, size_t k,
                          hipStream_t stream);
-constexpr int GEMV_MAX_M = 95;      // token rows that the decode-GEMV path takes but for long outputs (gemm_takes_tokens)
-// More rows go to the prefill GEMM, except where the token-group GEMV (gemv_mfma_tg_kernel: k a multiple of 256 up to
-// 8192, 16-byte aligned rows) runs as a single round of workgroups: it then beats a GEMM that is too small to fill the
-// chip (6912 -> 2560 at 96 tokens: 13.6 us against 18.9 us; 2560 -> 2560 up to 192 tokens: 8.4 .. 9.8 us against
-// 10.7 .. 11.0 us), and loses as soon as its workgroups need a second round (6912 -> 2560 at 112 tokens: 21.6 us
-// against 19.1 us).  n_blocks: 16-row blocks of all projections of the launch.  The row blocks per workgroup and
-// the workgroup slots follow launch_gemv_tiled.
-constexpr int GEMV_WIDE_MAX_M = 512;
-// From 33 tokens on a token GEMV of many workgroups (four row blocks by 16 tokens each) is bound by the exchange of its partial results
-// and the GEMM is ahead, where its 64 x 32 tiles fit the chip at once or there is work for its larger ones.  In us, GEMV / GEMM,
-// quantiser included: 1536 -> 16384 at 33 / 49 / 65 tokens 9.0 / 9.5, 11.4 / 9.7, 13.7 / 11.1; 2560 -> 13824 at 33 / 49 / 95 11.0 /
-// 11.4, 14.2 / 11.5, 18.8 / 13.9; 2560 -> 24576 at 33 / 49 / 95 15.9 / 16.9, 21.1 / 17.4, 28.6 / 18.2; 8192 -> 8192 at 95 23.1 / 24.2.
-inline bool gemm_takes_tokens(size_t m, size_t k, size_t n_blocks, const void *a)
-{
-    const size_t wgs = (n_blocks + 3) / 4 * ((m + 15) / 16), tiles32 = (m + 63) / 64 * ((n_blocks + 1) / 2);
-    return m > 32 && wgs >= 800 && (tiles32 <= 704 || (wgs >= 1500 && k >= 1536)) && k % TILE_K == 0 && n_blocks * k < (1ull << 29) &&
-           (reinterpret_cast<uintptr_t>(a) & 15) == 0;
-}
-// From 17 tokens on, where one round of gemm_ld8_kernel holds the launch, the two are compared by what they take (ns).  The GEMM: its
-// start and epilogue, and its stages (gemm_one_round_ns).  The token GEMV: its start, and per 16-row block and group of 16 tokens the
-// exchange of the partial results (by wavefronts, up to 16: one per k-tile) and the k-tiles beyond.  Both fitted to kernel times over
-// 10 widths, 10 to 192 tokens, within 20 %; the GEMM's start with 2.5 us on top, what weights that come from HBM cost it more than the
-// GEMV, which asks for all of its tiles at once (blocks of a decoder, each with its own weights, at 18 and 24 tokens of 3072 -> 18048
-// and 2304 -> 18176; 42 tokens of 2560 -> 6912 + 6912 by the GEMM: a 30-block step 1060 -> 1115 us).  GEMV / GEMM, quantiser included,
-// in us: 2560 -> 13824 at 32 / 42 / 95 7.8 / 9.3, 9.6 / 9.8, 13.8 / 11.8; 4096 -> 12288 at 32 / 42 / 95 9.1 / 11.1, 11.2 / 11.5, 15.7 / 14.0;
-// 8192 -> 8192 at 32 / 42 / 95 9.5 / 13.5, 13.6 / 14.0, 19.1 / 17.3; 2560 -> 30000 at 20 / 42 11.5 / 11.7, 15.0 / 12.5; 6912 -> 2560 at 95
-// 9.6 / 12.4; 2304 -> 6912 at 95 8.5 / 9.7; 1536 -> 12000 at 80 8.3 / 10.0; ten blocks of 4096 columns with a 12288-wide FFN at 32
-// tokens, gate and up by either: 426 / 441.
-size_t gemm_one_round_ns(size_t m, size_t k, size_t n);  // gemm_w2a8.hip; 0 where no tile of that kernel holds the launch in one round
-constexpr size_t GEMM_START_NS = 7500, GEMM_LEAST_STAGE_NS = 154;
+constexpr int GEMV_MAX_M = 95;       // token rows that the token GEMV takes at any width, unless the GEMM is faster
+constexpr int GEMV_WIDE_MAX_M = 512; // and where its workgroups are a single round of the chip (gemv_takes)
+// Between the two from 17 tokens on, by what each takes beyond what both do (launch, quantiser, weights once, outputs once), in ns.
+// The token GEMV, per 16-row block and group of 16 tokens: its part of the exchange of partial results, its k-tiles up to 16 (one per
+// wavefront, whose partial results are exchanged) and those beyond.  The GEMM: gemm_beyond_ns.  Fitted to the recorded times of both:
+// calls of 17 to 512 tokens, 15 widths from 256 to 16384 columns by 14 from 1024 to 131072 outputs, with a pair of layers and with layers
+// that outrun the last-level cache (the mean of the two); and 14 stacks of decoder blocks at 17 to 95 tokens with each launch group
+// by either kernel.  Where they differ, the one chosen is behind the faster one by 0.36 % in the geometric mean of the calls and 0.39 %
+// of the launches in stacks (a rule by workgroups and tiles: 2.0 and 0.6 %, at worst 2.1 times).  GEMV / GEMM, quantiser included, in us:
+// 2560 -> 13824 at 48 / 49 / 95 tokens 10.2 / 10.4, 11.6 / 10.4, 14.5 / 12.7; 1536 -> 16384 at 48 / 64 / 95 7.9 / 8.9, 8.7 / 9.2, 10.7 /
+// 10.3; 4096 -> 13824 at 48 / 49 / 95 12.0 / 12.5, 13.5 / 12.5, 17.6 / 15.0; 8192 -> 8192 at 32 / 48 / 95 10.2 / 13.9, 14.5 / 14.6, 19.6 /
+// 18.6; 6912 -> 2560 at 95 10.1 / 12.8; 256 -> 32768 at 33 / 64 / 95 7.6 / 7.6, 8.9 / 8.2, 11.2 / 9.1; 768 -> 20480 at 33 / 64 / 95 7.3 / 8.4,
+// 8.0 / 8.9, 9.6 / 9.7; 256 -> 131072 at 95 37.0 / 17.3.  A block of a stack with one group by either: 2560 -> 6912 + 6912 at 48 tokens is the
+// GEMV's by 0.3, at 64 the GEMM's by 1.2; 12288 -> 4096 at 95 the GEMV's by 0.3 where the call alone is the GEMM's by 2.1.
+size_t gemm_beyond_ns(size_t m, size_t k, size_t n);  // gemm_w2a8.hip
 inline bool gemm_beats_token_gemv(size_t m, size_t k, size_t n_blocks, const void *a)
 {
-    if (m <= 16 || m > (size_t)GEMV_WIDE_MAX_M || k < 1024 || k % TILE_K != 0 || n_blocks * k >= (1ull << 29) ||
-        (reinterpret_cast<uintptr_t>(a) & 15) != 0)
+    if (m <= 16 || m > (size_t)GEMV_WIDE_MAX_M || k == 0 || k % TILE_K != 0 || n_blocks * k >= (1ull << 29) || (reinterpret_cast<uintptr_t>(a) & 15) != 0)
         return false;
     const size_t kt = k / TILE_K, blocks = n_blocks * ((m + 15) / 16), near = blocks * (kt < 16 ? kt : 16), all = blocks * kt;
-    const size_t gemv_ns = 3300 + near * 2 / 11 + (all - near) / 8 + (m > 64 ? 1000 : 0);
-    if (gemv_ns <= GEMM_START_NS + GEMM_LEAST_STAGE_NS * kt) return false;
-    const size_t gemm_ns = gemm_one_round_ns(m, k, n_blocks * 16);
-    return gemm_ns != 0 && gemm_ns < gemv_ns;
+    const size_t gemv_ns = blocks / 6 + near / 8 + (all - near) / 10;
+    return gemv_ns > 2300 && gemm_beyond_ns(m, k, n_blocks * 16) < gemv_ns;  // the GEMM takes no less anywhere
 }
-// sums: the caller has the rows' sums, without which the GEMM takes a slower kernel
+// sums: the caller has the rows' sums, without which the GEMM takes a slower kernel.  Above 95 tokens (rows of up to 8192 columns) the
+// GEMV is taken only while its workgroups run as a single round, row blocks per workgroup and slots as in launch_gemv_tiled: 2560 ->
+// 2560 at 128 / 192 tokens 8.2 / 9.0, 8.6 / 9.3 us (GEMV / GEMM), 6912 -> 2560 at 96 10.1 / 12.8; a second round: 6912 -> 2560 at 112 13.1 / 12.9.
 inline bool gemv_takes(size_t m, size_t k, size_t n_blocks, const void *a, bool sums = true)
 {
     if (sums && gemm_beats_token_gemv(m, k, n_blocks, a)) return false;
-    if (m <= (size_t)GEMV_MAX_M) return !gemm_takes_tokens(m, k, n_blocks, a);
+    if (m <= (size_t)GEMV_MAX_M) return true;
     if (m > (size_t)GEMV_WIDE_MAX_M || k % 256 != 0 || k > 8192 || (reinterpret_cast<uintptr_t>(a) & 15) != 0) return false;
     const size_t tgroups = (m + 15) / 16, slots = k <= 3072 ? 768 : 256;
     const size_t rb = n_blocks * tgroups > 2 * slots ? 4 : (n_blocks * tgroups > slots ? 2 : 1);

@@ -1,12 +1,16 @@
 // Host-side checks of the library and of its C++ mirror against a stand-in for the HIP runtime: no GPU, no kernel runs.  The
 // functions below take the place of the runtime's (the executable's symbols come first), keep device memory on the heap, write down
-// what is called in which order, and can be told to fail.  Each check is named on the command line.
+// what is called in which order, and can be told to fail.  Each check is named on the command line; `kernels M K N` prints the
+// kernels that M token rows through a K -> N layer launch, by forward and by matmul on quantised rows.
 #include <hip/hip_runtime.h>
+
+#include <cxxabi.h>
 
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -30,6 +34,12 @@ hipError_t note(const char *name, hipStream_t stream = nullptr, hipError_t answe
     calls.push_back({name, stream, thread_mode});
     return answer;
 }
+std::map<const void *, std::string> &kernel_names()  // filled while the library is loaded
+{
+    static std::map<const void *, std::string> names;
+    return names;
+}
+std::vector<std::string> kernels;  // launched, in order
 size_t count(const std::string &name)
 {
     size_t n = 0;
@@ -116,7 +126,17 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t) { return fake::note("hipGraphExec
 
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t s) { return fake::note("configure", s); }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *s) { *s = fake::calls.back().stream; return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) { return fake::note("launch", s, fake::launch_answer); }
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t s)
+{
+    fake::kernels.push_back(fake::kernel_names()[f]);
+    return fake::note("launch", s, fake::launch_answer);
+}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
+{
+    char *plain = abi::__cxa_demangle(name, nullptr, nullptr, nullptr);
+    fake::kernel_names()[f] = plain ? plain : name;
+    free(plain);
+}
 }
 
 namespace {
@@ -403,6 +423,30 @@ const Check checks[] = {
 
 int main(int argc, char **argv)
 {
+    if (argc == 5 && std::string(argv[1]) == "kernels") {
+        const size_t m = std::strtoul(argv[2], nullptr, 10), k = std::strtoul(argv[3], nullptr, 10), n = std::strtoul(argv[4], nullptr, 10);
+        // no kernel runs and no weights are copied in: buffers of a few bytes stand for the matrices, aligned as the real ones
+        bitnet_hip_bitlinear *layer = nullptr;
+        auto some = DeviceTensor::zeros({1024}).unwrap();
+        const size_t dims[2] = {m, k};
+        if (bitnet_hip_bitlinear_create(k, n, 0, &layer) != BITNET_HIP_OK) return 3;
+        if (bitnet_hip_bitlinear_set_weights_f32(layer, some.data(), n, k, BITNET_HIP_LAYOUT_OUT_IN, 1, BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP, 0.5f, side) != BITNET_HIP_OK)
+            return 3;
+        const auto print = [](const char *call) {
+            for (const std::string &name : fake::kernels) std::printf("%s: %s\n", call, name.c_str());
+            fake::kernels.clear();
+        };
+        fake::kernels.clear();
+        if (bitnet_hip_bitlinear_forward(layer, some.data(), dims, 2, nullptr, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, some.data(), nullptr, 0, nullptr, nullptr,
+                                         nullptr, side) != BITNET_HIP_OK)
+            return 3;
+        print("forward");
+        const int8_t *rows = reinterpret_cast<const int8_t *>(some.data());
+        const int32_t *sums = reinterpret_cast<const int32_t *>(some.data());
+        if (bitnet_hip_bitlinear_matmul(layer, rows, sums, m, some.data(), nullptr, nullptr, some.data(), side) != BITNET_HIP_OK) return 3;
+        print("matmul");
+        return 0;
+    }
     for (const Check &c : checks) {
         if (argc == 2 && std::string(argv[1]) != c.name) continue;
         if (argc == 1) { std::printf("%s\n", c.name); continue; }

@@ -1687,9 +1687,10 @@ def test_decoder_output_projection_reads_distinct_heads(dims, m):
     assert np.array_equal(host(dec.decode(dev(x))), oracle_stack(ref, x, *dims)[0])
 
 
-@pytest.mark.parametrize("m,n,k", [(33, 17100, 256), (49, 12900, 300), (65, 10300, 512), (80, 24700, 1600)])
+@pytest.mark.parametrize("m,n,k", [(33, 17100, 256), (49, 12900, 300), (65, 10300, 512), (80, 24700, 1600), (95, 33003, 256), (49, 65540, 260), (90, 103001, 300)])
 def test_forward_of_long_outputs_at_few_tokens_bit_exact(m, n, k):
-    """Few tokens and many outputs: the shapes on which the GEMM takes over below 96 tokens, incomplete row tiles."""
+    """Few tokens and many outputs, on both sides of the line from which the GEMM takes over below 96 tokens: incomplete row tiles, its
+    loader-fed tiles (1600 columns) and those of its other kernel."""
     rng = np.random.default_rng(m)
     x = synth_activations(rng, m, k, outliers=True)
     pk = random_packed_ternary(rng, n, k)

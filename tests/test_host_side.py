@@ -25,3 +25,22 @@ def program(tmp_path_factory):
 def test_host_side(program, name):
     done = subprocess.run([str(program), name], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stdout + done.stderr
+
+
+def kernels_of(program, m, k, n):
+    """{call: the kernel that multiplies, as name<parameters>} of `forward` and `matmul` for m token rows through a k -> n layer."""
+    done = subprocess.run([str(program), "kernels", str(m), str(k), str(n)], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout + done.stderr
+    return {line.split(": ")[0]: re.search(r"\w+_kernel(<[^>]*>)?", line.split(": ", 1)[1]).group() for line in done.stdout.splitlines()}
+
+
+@pytest.mark.parametrize("m,k,n,gemv_us,gemm_us", [
+    (64, 768, 20480, 8.0, 8.9), (48, 768, 27648, 8.2, 9.6), (64, 512, 16384, 7.1, 7.5), (72, 2048, 11008, 9.1, 11.0), (32, 8192, 8192, 10.2, 13.9),
+    (95, 6912, 2560, 10.1, 12.8), (64, 1536, 16384, 8.7, 9.2), (64, 1024, 13824, 7.4, 8.2), (128, 2560, 2560, 8.2, 9.0), (32, 8192, 16384, 15.5, 17.7),
+    (49, 2560, 13824, 11.6, 10.4), (64, 8192, 28672, 38.9, 25.2), (95, 256, 32768, 11.2, 9.1), (64, 256, 65536, 13.1, 9.2), (95, 768, 131072, 41.2, 23.7),
+    (49, 10240, 10240, 24.6, 20.5), (17, 16384, 32768, 49.1, 41.9), (81, 1024, 32768, 12.9, 12.1), (49, 4096, 14336, 13.7, 12.3), (33, 2560, 24576, 13.0, 11.5),
+    (80, 2560, 13824, 13.0, 12.0)])
+def test_the_faster_of_token_gemv_and_gemm_is_launched(program, m, k, n, gemv_us, gemm_us):
+    """Both kernels' recorded times of a forward, quantiser included: the mean of one layer called again and again and of layers that
+    outrun the last-level cache."""
+    assert kernels_of(program, m, k, n)["forward"].startswith("gemv_rows_kernel" if gemv_us < gemm_us else "gemm_")
