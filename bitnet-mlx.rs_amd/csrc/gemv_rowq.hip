@@ -261,7 +261,11 @@ int launch_rb(const Launch &l, int rb)
 // Workgroups that the fullest compute unit runs, of `groups` groups of row blocks and `tgroups` token groups (the kernel's mapping: a
 // group of row blocks on one XCD of 32).
 size_t rounds_of(size_t groups, size_t tgroups) { return ((groups + 7) / 8 * tgroups + 31) / 32; }
-// The fewest row blocks a workgroup that keep the launch within one round, at most 4.
+// The fewest row blocks a workgroup that keep the launch within one round, at most 4.  Counted for the fullest XCD: 84 row blocks by 3
+// token groups are 252 workgroups, but 11 of one XCD by 3 do not fit its 32 compute units.  One / two / four row blocks a workgroup, us a
+// recorded decoder block (this is its attention output projection; 252 to 255 workgroups of one row block): 1344 wide at 33 / 48 tokens
+// 25.4 / 25.3 / 26.1, 27.0 / 25.9 / 26.7; 816 at 80 24.4 / 23.5 / 23.9; 672 at 95 26.3 / 23.2 / 23.7.  Where one fits each XCD (2000 wide
+// at 32) 27.4 / 27.6 / 28.2.
 size_t row_blocks_per_workgroup(size_t blocks, size_t tgroups)
 {
     size_t rb = 1;

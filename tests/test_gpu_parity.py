@@ -1677,10 +1677,11 @@ def test_forward_of_short_rows_in_one_launch_bit_exact(m, n, k):
     assert all(np.array_equal(host(o), ref) for o in outs)
 
 
-@pytest.mark.parametrize("dims,m", [((2560, 256, 20, 5, 128), 8), ((192, 320, 12, 3, 16), 9), ((4352, 64, 34, 2, 128), 17), ((4096, 64, 64, 8, 64), 13)])
+@pytest.mark.parametrize("dims,m", [((2560, 256, 20, 5, 128), 8), ((192, 320, 12, 3, 16), 9), ((4352, 64, 34, 2, 128), 17), ((4096, 64, 64, 8, 64), 13),
+                                    ((1344, 64, 21, 7, 64), 40), ((672, 64, 21, 7, 32), 95)])
 def test_decoder_output_projection_reads_distinct_heads(dims, m):
     """The attention output projection on its distinct columns: groups of one to seventeen query heads, one and two k-tiles a
-    wavefront, heads of one piece, row counts on both sides of a token group."""
+    wavefront, heads of one piece, row counts on both sides of a token group; row blocks that fill the chip but not each of its dies."""
     rng = np.random.default_rng(m)
     dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=m)
     x = synth_activations(rng, m, dims[0])
