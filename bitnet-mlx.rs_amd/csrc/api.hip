@@ -270,15 +270,6 @@ QuantScratch carve_scratch(void *ws, size_t m, size_t k)
     return sc;
 }
 
-// What workspace_size counts beside the quantised activations for 97 to about 256 tokens on long rows.  A GEMM that split k across workgroups
-// kept its partial tiles and tile counters there; nothing reads it now.  The figure stays what callers have sized their buffers by.
-size_t reserved_bytes(size_t m, size_t k, size_t n)
-{
-    const size_t tiles = (m + 63) / 64 * ((n + 31) / 32), stages = k / 128, per = ((stages + 2) / 3 + 1) & ~(size_t)1;
-    if (m <= 96 || k < 4096 || tiles == 0 || tiles > 352) return 0;
-    return align_up(tiles * ((stages + per - 1) / per) * 64 * 32 * sizeof(int32_t), 256) + align_up(tiles * sizeof(unsigned), 256);
-}
-
 }  // namespace
 
 extern "C" {
@@ -860,9 +851,7 @@ int bitnet_hip_bitlinear_get_quantized(bitnet_hip_bitlinear *layer, float *w_sca
 
 size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, size_t m)
 {
-    if (!layer) return 0;
-    const size_t kp = padded_k(layer->in_features);
-    return quant_scratch_bytes(m, kp) + reserved_bytes(m, kp, layer->out_features);
+    return layer ? quant_scratch_bytes(m, padded_k(layer->in_features)) : 0;
 }
 
 size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,

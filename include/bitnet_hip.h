@@ -337,13 +337,12 @@ int bitnet_hip_bitlinear_get_quantized(bitnet_hip_bitlinear *layer, float *w_sca
                                        size_t packed_len);
 
 /* Bytes of device workspace forward needs for m tokens: the quantised activations (int8 rows padded to a multiple of 256
- * bytes, a_scale, a_sum) and, for 97 to about 256 tokens on rows of 4096 and more columns, a reserve that no kernel uses at
- * present.  forward accepts a workspace that holds only unpadded rows (m * in_features rounded up to 256, plus two arrays of
+ * bytes, a_scale, a_sum).  forward accepts a workspace that holds only unpadded rows (m * in_features rounded up to 256, plus two arrays of
  * 4 * m bytes rounded up to 256, plus 256) and then runs without the padding: same results, up to four times slower where
  * in_features is no multiple of 256. */
 size_t bitnet_hip_bitlinear_workspace_size(const bitnet_hip_bitlinear *layer, size_t m);
 /* The same for one particular call: 0 where forward quantises inside its only launch and needs no workspace (decode token
- * counts on aligned rows), else workspace_size(m) without the reserve.  For callers that allocate per call. */
+ * counts on aligned rows), else workspace_size(m).  For callers that allocate per call. */
 size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, const float *x, size_t m, const float *gamma,
                                             int sum_order);
 

@@ -402,6 +402,20 @@ void recorded_calls_on_short_rows()
     }
 }
 
+// A workspace holds the quantised rows and nothing that no kernel reads: workspace_size is what a call of two launches uses.
+void a_workspace_is_what_a_call_uses()
+{
+    for (size_t m : {97, 256, 300})
+        for (size_t k : {4096, 6900}) {
+            bitnet_hip_bitlinear *layer = nullptr;
+            CHECK(bitnet_hip_bitlinear_create(k, 2560, 0, &layer) == BITNET_HIP_OK);
+            auto x = DeviceTensor::zeros({1024}).unwrap();
+            const size_t used = bitnet_hip_bitlinear_forward_scratch(layer, x.data(), m, nullptr, BITNET_HIP_SUM_BLOCK256);
+            CHECK(used != 0 && bitnet_hip_bitlinear_workspace_size(layer, m) == used);
+            bitnet_hip_bitlinear_destroy(layer);
+        }
+}
+
 struct Check {
     const char *name;
     void (*run)();
@@ -417,6 +431,7 @@ const Check checks[] = {
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
     {"recorded_calls_on_short_rows", recorded_calls_on_short_rows},
+    {"a_workspace_is_what_a_call_uses", a_workspace_is_what_a_call_uses},
 };
 
 }  // namespace

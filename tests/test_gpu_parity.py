@@ -773,17 +773,16 @@ def test_bitlinear_forward_prefill_uses_quantiser_row_sums():
 
 @pytest.mark.parametrize("m,k,n", [(97, 6912, 2560), (128, 6912, 2560), (200, 4096, 1000), (256, 6912, 2560), (130, 8192, 644),
                                    (255, 5120, 1408), (97, 4096, 16), (256, 8192, 2816), (300, 4352, 2240)])
-def test_forward_split_k_bit_exact(m, k, n):
-    """A long k with few output tiles (97 to 256 tokens at 6912 -> 2560), for which workspace_size counts more than the
-    quantised activations.  Checked against the oracle (activations, accumulators, f32 output with bias and residual);
-    with a workspace that holds only the quantised activations; on a workspace full of ones; and on the same workspace
-    three times in a row."""
+def test_forward_of_long_rows_in_few_tiles_bit_exact(m, k, n):
+    """A long k with few output tiles (97 to 256 tokens at 6912 -> 2560).  Checked against the oracle (activations,
+    accumulators, f32 output with bias and residual); workspace_size is what the quantised activations take; on a
+    workspace of that size full of ones, three times in a row."""
     rng = np.random.default_rng(m + k + n)
     w = synth_weights(rng, n, k)
     x = synth_activations(rng, m, k, outliers=True)
     bias = rng.standard_normal(n, dtype=f32)
     res = rng.standard_normal((m, n), dtype=f32)
-    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "split")
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "long rows")
     layer.update_weights(dev(w))
     layer.update_bias(dev(bias))
     qw, ws = orc.quantize_weights_absmean(w)
@@ -793,13 +792,10 @@ def test_forward_split_k_bit_exact(m, k, n):
     assert np.array_equal(host(acc), acc_ref)
     assert np.array_equal(host(out), out_ref)
     full = layer.workspace_size(m)
-    quant_only = ((m * k + 255) // 256) * 256 + 2 * (((4 * m) + 255) // 256) * 256 + 256
-    assert full > quant_only, "this shape is expected to take the split"
-    small = torch.full((quant_only,), 1, dtype=torch.uint8, device="cuda")
-    assert np.array_equal(host(layer.forward(dev(x), residual=dev(res), workspace=small)), out_ref)
-    big = torch.full((full,), 1, dtype=torch.uint8, device="cuda")
+    assert full == ((m * k + 255) // 256) * 256 + 2 * (((4 * m) + 255) // 256) * 256 + 256
+    ws = torch.full((full,), 1, dtype=torch.uint8, device="cuda")
     for _ in range(3):
-        assert np.array_equal(host(layer.forward(dev(x), residual=dev(res), workspace=big)), out_ref)
+        assert np.array_equal(host(layer.forward(dev(x), residual=dev(res), workspace=ws)), out_ref)
 
 
 # ---- L1: BitLinear object ----------------------------------------------------------------------------------
