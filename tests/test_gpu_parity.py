@@ -1790,12 +1790,17 @@ def test_gemm_128x256_tiles_and_grouped_rows(m, n, k):
     assert torch.equal(single, outs[0][: m // 3])
 
 
-@pytest.mark.parametrize("k", [1024, 1280, 2816])
-@pytest.mark.parametrize("m,n", [(17, 30000), (64, 33), (65, 4100), (130, 1100), (200, 3000), (257, 6000), (333, 8192), (500, 3073), (700, 6500), (1025, 2500),
-                                 (2040, 2560)])
+ONE_ROUND = [(17, 30000), (64, 33), (65, 4100), (130, 1100), (200, 3000), (257, 6000), (333, 8192), (500, 3073), (700, 6500), (1025, 2500), (2040, 2560),
+             (513, 33), (650, 1101), (520, 1100), (650, 2001), (257, 5999), (333, 8170)]
+ONE_ROUND_K = [1024, 1280, 2816]
+
+
+@pytest.mark.parametrize("k", ONE_ROUND_K)
+@pytest.mark.parametrize("m,n", ONE_ROUND)
 def test_gemm_tiles_of_one_round_bit_exact(m, n, k):
     """Launches that one round of the loader-fed workgroups holds: every tile of its table (64 x 32 to 128 x 160, one or two workgroups per
-    compute unit), first and last rows and columns cut, four to eleven stages; int32 and f32 output through matmul, f32 through forward."""
+    compute unit) with its last row and column tile cut, which test_host_side.py checks, four to eleven stages; and, up to 200 tokens,
+    neighbours that the token GEMV takes; int32 and f32 output through matmul, f32 through forward."""
     rng = np.random.default_rng(m + n + k)
     x = synth_activations(rng, m, k, outliers=True)
     pk = random_packed_ternary(rng, n, k)

@@ -7,6 +7,7 @@ from pathlib import Path
 import pytest
 
 import bitnet_hip as bh
+from test_gpu_parity import ONE_ROUND, ONE_ROUND_K
 
 SOURCE = Path(__file__).with_name("fake_hip_checks.cpp")
 CHECKS = re.findall(r'^    \{"(\w+)", \1\},$', SOURCE.read_text(), flags=re.M)
@@ -44,3 +45,19 @@ def test_the_faster_of_token_gemv_and_gemm_is_launched(program, m, k, n, gemv_us
     """Both kernels' recorded times of a forward, quantiser included: the mean of one layer called again and again and of layers that
     outrun the last-level cache."""
     assert kernels_of(program, m, k, n)["forward"].startswith("gemv_rows_kernel" if gemv_us < gemm_us else "gemm_")
+
+
+def test_the_shapes_of_the_one_round_gemm_test_reach_every_tile(program):
+    """The GPU test that names these shapes runs each tile of gemm_ld8_kernel's table, by forward and by matmul, at every k, with
+    rows and columns left over."""
+    source = (bh.LIB_PATH.parents[1] / "csrc" / "gemm_w2a8.hip").read_text()
+    tiles = re.findall(r"&launch_ld8<(\d+), (\d+), (\d+)>", source)
+    assert len(tiles) == 8
+    for k in ONE_ROUND_K:
+        cut = {call: set() for call in ("forward", "matmul")}
+        for m, n in ONE_ROUND:
+            for call, kernel in kernels_of(program, m, k, n).items():
+                tile = re.fullmatch(r"gemm_ld8_kernel<(\d+), (\d+), (\d+)>", kernel)
+                if tile and m % int(tile[1]) and n % int(tile[2]):
+                    cut[call].add(tile.groups())
+        assert cut["forward"] == cut["matmul"] == set(tiles)
