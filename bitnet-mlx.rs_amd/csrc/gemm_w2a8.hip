@@ -21,9 +21,9 @@
 // quantiser): activations AND weight tiles travel global -> LDS with LDS-direct loads
 // (global_load_lds_dwordx4), never through registers.  D LDS stages of 128 columns are kept in flight;
 // the wait counts are placed by hand (s_waitcnt vmcnt(N)) so that D - 1 stages of loads stay outstanding
-// while one is computed (D = 2 in the shipped instances: a plain double buffer, which leaves LDS and registers for
-// three or four workgroups per compute unit).  An LDS-direct load writes lane l's 16 bytes at base + 16*l, so the XOR swizzle
-// that keeps the fragment reads free of bank conflicts is applied to the global address each lane fetches.
+// while one is computed (D = 2, a plain double buffer, which leaves LDS and registers for two workgroups of the largest
+// tiles and three or four of the others per compute unit; D = 4 for the narrow tiles of short rows).  An
+// LDS-direct load writes lane l's 16 bytes at base + 16*l, so the XOR swizzle that keeps the fragment reads free of bank conflicts is applied to the global address each lane fetches.
 // The MFMA takes the weight fragment as its first operand, so a lane ends up with four consecutive output
 // columns of one token row and the epilogue stores 16 bytes per lane.  The epilogue's per-row operands (a_sum,
 // a_scale) arrive by LDS-direct loads in the stage buffer that is free during the last stage; the usual case
