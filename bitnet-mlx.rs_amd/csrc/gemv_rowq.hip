@@ -286,10 +286,11 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
     // In one round of workgroups only: a second one quantises again.  What a workgroup pays for it grows with the columns that it
     // quantises, those of its up to 16 rows together; what it saves is the quantiser's launch, 0.5 to 1 us of the GPU's time and, in a call
     // that nothing records, 2.5 us of the host's.  So a call of its own is one launch wherever the kernel takes it, and a recorded one
-    // (alone == false: a decoder step, a capture of the caller's) where the GPU is faster so.  Recorded, two launches -> one, us:
+    // (alone == false: a decoder step, a capture of the caller's) up to lines beyond which the GPU is slower so.  Recorded, two launches -> one, us:
     // plain rows of up to 1024 columns, any number of tokens: 16 x 1024 -> 2560 4.8 -> 4.2, 64 x 1024 -> 2560 5.5 -> 5.0, 512 x 1024 -> 512 6.4 -> 5.3;
     // with norm, up to 12288 columns a workgroup: 9 x 256 -> 2560 5.1 -> 4.7, 9 x 1024 -> 9000 6.2 -> 6.0; beyond them 16 x 1024 -> 2560 5.2 -> 6.0,
-    // 64 x 1024 -> 512 5.1 -> 5.8, 128 x 512 -> 512 5.1 -> 5.6;
+    // 64 x 1024 -> 512 5.1 -> 5.8, 128 x 512 -> 512 5.1 -> 5.6 (full groups of 16 rows are behind before the line: 16 x 512 -> 2560 5.05 -> 5.4,
+    // 48 x 768 -> 2560 5.4 -> 5.9);
     // plain rows above 1024 columns, up to the same 12288: 5 x 2048 -> 9000 6.5 -> 5.8, 9 x 1280 -> 2560 5.1 -> 4.8; beyond them 16 x 1280 -> 2560
     // 5.1 -> 5.4, 16 x 2048 -> 2560 5.2 -> 6.4, 40 x 2048 -> 5120 6.2 -> 7.4, 256 x 1536 -> 512 5.8 -> 6.0, but above 256 tokens, where the quantiser's
     // launch is longer itself, 512 x 1280 -> 512 7.0 -> 6.3, 512 x 2048 -> 512 8.3 -> 7.5.
