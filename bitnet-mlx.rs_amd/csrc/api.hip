@@ -7,6 +7,8 @@
 #include <shared_mutex>
 #include <vector>
 
+#include <atomic>
+#include <random>
 #include "kernels.hpp"
 #include "staging.hpp"
 
@@ -159,18 +161,22 @@ bool quantises_in_launch(const bitnet_hip_bitlinear *const *layers, size_t count
            gemv_fused_supported(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, 1, gamma, sum_order, blocks);
 }
 
+bool being_captured(hipStream_t s)
+{
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
+        (void)hipGetLastError();  // the launches that follow must not report it
+        return false;
+    }
+    return capturing == hipStreamCaptureStatusActive;
+}
+
 // Whether projections that could quantise inside their launch are faster in two launches, since the stream is being captured and a
 // replay costs the host nothing per launch (gemv_rowq_takes).  The stream is asked only where that decides.
 bool recorded_in_two(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order,
                      hipStream_t s)
 {
-    if (m < 2 || !s || quantises_in_launch(layers, count, x, m, gamma, sum_order, false)) return false;  // the null stream is never captured
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
-        (void)hipGetLastError();  // the launches below must not report it
-        return false;
-    }
-    return capturing == hipStreamCaptureStatusActive;
+    return m >= 2 && s && !quantises_in_launch(layers, count, x, m, gamma, sum_order, false) && being_captured(s);  // the null stream is never captured
 }
 
 // Runs `count` projections that share one input row block [m, k].  At decode token counts the quantiser runs
@@ -182,7 +188,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
                     size_t m, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,
                     int sum_order, const float *const *residual, float *const *out, int32_t *const *acc, int8_t *q,
                     size_t ldq, float *a_scale, int32_t *a_sum, bool want_quant_outputs, hipStream_t s,
-                    bool alone = true)
+                    bool alone = true, const DieFlags *die = nullptr)
 {
     size_t k = layers[0]->in_features;
     const bool short_rows = !want_quant_outputs && gemv_rowq_takes(x, ldx, m, k, input_mode, gqa_group, head_dim, gamma, sum_order,
@@ -193,6 +199,11 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
                        out[j], acc ? acc[j] : nullptr, bl->out_features};
         return pj;
     };
+    if (die) {
+        GemvProj pjs[GEMV_MAX_PROJ];
+        for (int j = 0; j < count; ++j) pjs[j] = proj_of(j);
+        return launch_gemv_die(pjs, count, x, x2, ldx, m, k, input_mode, gamma, eps, q, a_scale, *die, s);
+    }
     if (short_rows) {
         for (int j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
             GemvProj pjs[GEMV_MAX_PROJ];
@@ -268,6 +279,31 @@ QuantScratch carve_scratch(void *ws, size_t m, size_t k)
     sc.a_scale = reinterpret_cast<float *>(base + align_up(m * k, 256));
     sc.a_sum = reinterpret_cast<int32_t *>(base + align_up(m * k, 256) + align_up(m * sizeof(float), 256));
     return sc;
+}
+
+// Flags behind the scratch of a call that quantises its rows once a die, and the tag that its launch gives them: no other launch of this
+// process has it, and memory that was never a flag holds it by a chance of 2^-64.
+size_t die_flag_bytes(size_t m) { return align_up(sizeof(uint64_t) * GEMV_DIE_SETS * align_up(m, 16), 256); }
+uint64_t next_die_tag()
+{
+    static std::atomic<uint64_t> next{[] {
+        std::random_device any;
+        return ((uint64_t)any() << 32 | any()) | ((uint64_t)1 << 63);
+    }()};
+    return next.fetch_add(1, std::memory_order_relaxed);
+}
+DieFlags call_flags(void *ws, size_t m, size_t ldq)
+{
+    const uintptr_t at = align_up(reinterpret_cast<uintptr_t>(ws), 256) + quant_scratch_bytes(m, ldq) - 256;
+    return {reinterpret_cast<uint64_t *>(at), nullptr, next_die_tag(), (unsigned)align_up(m, 16), GEMV_DIE_LOOKS};
+}
+// Whether plain rows go through one launch that quantises them once a die: a call of its own, on a stream that is not being captured
+// (a replay would find the flags of the one before it).
+bool quantises_on_dies(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m, const float *gamma, int sum_order, hipStream_t s)
+{
+    const size_t in = layers[0]->in_features;
+    return count <= (size_t)GEMV_MAX_PROJ && gemv_die_takes(x, nullptr, in, m, in, BITNET_HIP_INPUT_PLAIN, gamma, sum_order, launch_group_blocks(layers, count), true) &&
+           !(s && being_captured(s));
 }
 
 }  // namespace
@@ -882,7 +918,8 @@ size_t bitnet_hip_bitlinear_forward_scratch_on(bitnet_hip_bitlinear *const *laye
     if (quantises_in_launch(layers, count, x, m, gamma, sum_order) &&
         !recorded_in_two(layers, count, x, m, gamma, sum_order, as_stream(stream)))
         return 0;
-    return quant_scratch_bytes(m, padded_k(layers[0]->in_features));
+    return quant_scratch_bytes(m, padded_k(layers[0]->in_features)) +
+           (quantises_on_dies(layers, count, x, m, gamma, sum_order, as_stream(stream)) ? die_flag_bytes(m) : 0);
 }
 
 int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, const size_t *dims, int rank,
@@ -918,6 +955,9 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
     const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
                         recorded_in_two(&layer, 1, x, m, gamma, sum_order, s);
     fused = fused && !in_two;
+    bitnet_hip_bitlinear *layers[1] = {layer};
+    const bool on_dies = !fused && !in_two && !debug && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
+                         quantises_on_dies(layers, 1, x, m, gamma, sum_order, s);
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {dbg_q, dbg_a_scale, nullptr};
@@ -937,12 +977,12 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
         if (dbg_q) sc.q = dbg_q;
         if (dbg_a_scale) sc.a_scale = dbg_a_scale;
     }
-    bitnet_hip_bitlinear *layers[1] = {layer};
     const float *res[1] = {residual};
     float *outs[1] = {out};
     int32_t *accs[1] = {dbg_acc};
+    const DieFlags flags = on_dies ? call_flags(ws, m, ldq) : DieFlags{};
     int rc = run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
-                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, !in_two);
+                             accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, !in_two, on_dies ? &flags : nullptr);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -1025,6 +1065,8 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
                         recorded_in_two(layers, count, x, m, gamma, sum_order, s);
     fused = fused && !in_two;
+    const bool on_dies = !fused && !in_two && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
+                         quantises_on_dies(layers, count, x, m, gamma, sum_order, s);
     void *ws = workspace;
     bool own_ws = false;
     QuantScratch sc = {nullptr, nullptr, nullptr};
@@ -1041,8 +1083,9 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
         }
         sc = carve_scratch(ws, m, ldq);
     }
+    const DieFlags flags = on_dies ? call_flags(ws, m, ldq) : DieFlags{};
     int rc = run_projections(layers, (int)count, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order,
-                             nullptr, outs, nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, s, !in_two);
+                             nullptr, outs, nullptr, sc.q, ldq, sc.a_scale, sc.a_sum, false, s, !in_two, on_dies ? &flags : nullptr);
     if (own_ws) {
         hipError_t e = hipFreeAsync(ws, s);
         if (rc == BITNET_HIP_OK && e != hipSuccess)
@@ -1109,6 +1152,12 @@ struct bitnet_hip_decoder {
     int32_t *a_sum = nullptr;
     float *qb = nullptr, *kb = nullptr, *vb = nullptr, *x1 = nullptr, *gate = nullptr, *up = nullptr;
     float *ping = nullptr;
+    // Flags of the launches that quantise their rows once a die (gemv_die.hip): two sets used in turn.  Every step leaves the first set
+    // cleared; a step that failed half way does not, and no later one uses them.
+    uint64_t *die_flags = nullptr;
+    bool die_flags_spent = false;
+    int die_looks = GEMV_DIE_LOOKS;
+    size_t die_stride() const { return align_up(max_tokens < (size_t)GEMV_DIE_MAX_M ? max_tokens : (size_t)GEMV_DIE_MAX_M, 16); }
     // One decode at a time: the activation buffers above are shared by every call on this decoder.  The mutex
     // serialises the enqueue; `done` (recorded behind every decode) makes a decode on another stream wait for it.
     std::mutex decode_lock;
@@ -1144,7 +1193,7 @@ struct bitnet_hip_decoder {
     ~bitnet_hip_decoder()
     {
         for (auto *p : proj) delete p;
-        void *bufs[] = {gamma, a8, a_scale, a_sum, qb, kb, vb, x1, gate, up, ping};
+        void *bufs[] = {gamma, a8, a_scale, a_sum, qb, kb, vb, x1, gate, up, ping, die_flags};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
         drop_step_graphs();  // behind the hipFree calls, which wait for the device
@@ -1201,6 +1250,12 @@ int bitnet_hip_decoder_create(size_t layers, size_t hidden, size_t ffn, size_t q
     dev_alloc(&d->gate, sizeof(float) * max_tokens * ffn);
     dev_alloc(&d->up, sizeof(float) * max_tokens * ffn);
     dev_alloc(&d->ping, sizeof(float) * max_tokens * hidden);
+    const size_t die_bytes = sizeof(uint64_t) * 2 * GEMV_DIE_SETS * d->die_stride();
+    dev_alloc(&d->die_flags, die_bytes);
+    if (rc == BITNET_HIP_OK) {
+        hipError_t e = hipMemset(d->die_flags, 0, die_bytes);
+        if (e != hipSuccess) rc = fail(BITNET_HIP_DEVICE_ERROR, "decoder_create: hipMemset failed: %s", hipGetErrorString(e));
+    }
     if (rc == BITNET_HIP_OK) {
         // RMSNorm weights start at one
         std::vector<float> ones(layers * 2 * hidden, 1.0f);
@@ -1236,6 +1291,18 @@ int bitnet_hip_decoder_set_chains(bitnet_hip_decoder *dec, size_t chains)
         return fail(BITNET_HIP_INVALID_CONFIG, "decoder_set_chains: %zu chains, at most %zu", chains, DECODER_MAX_CHAINS);
     std::lock_guard<std::mutex> one_decode(dec->decode_lock);
     dec->chains = chains;
+    return BITNET_HIP_OK;
+}
+
+int bitnet_hip_decoder_set_row_wait(bitnet_hip_decoder *dec, int looks)
+{
+    if (!dec) return fail(BITNET_HIP_NULL_POINTER, "decoder_set_row_wait: dec is NULL");
+    if (looks < 0 || looks > GEMV_DIE_LOOKS)
+        return fail(BITNET_HIP_INVALID_CONFIG, "decoder_set_row_wait: %d looks, 0 to %d", looks, GEMV_DIE_LOOKS);
+    std::lock_guard<std::mutex> one_decode(dec->decode_lock);
+    BITNET_HIP_TRY(hipDeviceSynchronize());  // the steps recorded so far may be running
+    dec->drop_step_graphs();
+    dec->die_looks = looks;
     return BITNET_HIP_OK;
 }
 
@@ -1288,15 +1355,25 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
     // One chain: rows [row0, row0 + rows) through blocks layer_begin .. layer_end-1 on stream cs, in its own rows of the
     // decoder's activation buffers.
     const size_t widest = padded_k(H > F ? H : F);
+    const size_t chains_asked = dec->chains ? dec->chains : 1;
+    size_t die_launches = 0;
     auto run_chain = [&](size_t row0, size_t rows, hipStream_t cs) {
         // one launch group: `count` projections reading the same (transformed) input
         auto run = [&](bitnet_hip_bitlinear *const *layers, int count, const float *x, const float *x2, size_t ldx, int mode,
                        const float *gamma, const float *res0, float *const *outs) {
             if (rc != BITNET_HIP_OK) return;
+            DieFlags flags;
+            const bool on_dies = chains_asked <= 1 && !dec->die_flags_spent &&
+                                 gemv_die_takes(x, x2, ldx, rows, layers[0]->in_features, mode, gamma, dec->sum_order, launch_group_blocks(layers, (size_t)count), false);
+            if (on_dies) {
+                uint64_t *sets[2] = {dec->die_flags, dec->die_flags + GEMV_DIE_SETS * dec->die_stride()};
+                flags = {sets[die_launches & 1], sets[~die_launches & 1], 1, (unsigned)dec->die_stride(), dec->die_looks};
+                ++die_launches;
+            }
             const float *res[GEMV_MAX_PROJ] = {res0, nullptr, nullptr};
             rc = run_projections(layers, count, x, x2, ldx, rows, mode, group, dec->head_dim, gamma, dec->eps, dec->sum_order,
                                  res, outs, nullptr, dec->a8 + row0 * widest, padded_k(layers[0]->in_features), dec->a_scale + row0,
-                                 dec->a_sum + row0, false, cs, false);
+                                 dec->a_sum + row0, false, cs, false, on_dies ? &flags : nullptr);
         };
         float *qb = dec->qb + row0 * H, *kb = dec->kb + row0 * KV, *vb = dec->vb + row0 * KV, *x1 = dec->x1 + row0 * H;
         float *gate = dec->gate + row0 * F, *up = dec->up + row0 * F, *ping = dec->ping + row0 * H;
@@ -1319,11 +1396,13 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
             x = x2;
         }
     };
-    size_t chains = dec->chains ? dec->chains : 1;
+    size_t chains = chains_asked;
     if (chains > m) chains = m;
     if (chains > dec->max_tokens) chains = dec->max_tokens;  // side streams exist for min(max_tokens, 8) chains
     if (chains <= 1) {
         run_chain(0, m, s);
+        if (rc == BITNET_HIP_OK && (die_launches & 1)) rc = launch_clear_die_flags(dec->die_flags, dec->die_stride(), m, s);
+        if (rc != BITNET_HIP_OK && die_launches) dec->die_flags_spent = true;
     } else {
         // fork: the side streams start behind whatever the caller's stream holds; join: it continues behind them all.
         // Recorded into the caller's graph when s is being captured (the events pull the side streams into the capture).
@@ -1605,6 +1684,7 @@ size_t decoder_device_bytes(const bitnet_hip_decoder *d)
     const size_t kv = d->kv_heads * d->head_dim, widest = padded_k(d->hidden > d->ffn ? d->hidden : d->ffn), t = d->max_tokens;
     total += sizeof(float) * d->layers * 2 * d->hidden;                                        // norms
     total += t * widest + 2 * sizeof(float) * t;                                               // a8, a_scale, a_sum
+    total += sizeof(uint64_t) * 2 * GEMV_DIE_SETS * d->die_stride();                                     // die_flags
     total += sizeof(float) * t * (d->hidden /*q*/ + 2 * kv + d->hidden /*x1*/ + 2 * d->ffn + d->hidden /*ping*/);
     return total;
 }

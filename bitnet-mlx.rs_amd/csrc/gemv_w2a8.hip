@@ -38,7 +38,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
-#include "rowquant.hpp"
+#include "rowsgemv.hpp"
 #include "tiledot.hpp"
 #include "ldsdma.hpp"
 
@@ -453,15 +453,6 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvParams p)
 // 23.9 and 22.3.
 
 // The arguments behind the preloaded ones, in blocks of 64 bytes: each is one scalar load.
-struct Fused16Proj {
-    const uint8_t *w;
-    const float *w_scale, *bias, *residual;
-    float *out;
-    int32_t *acc;
-    int n;
-    int rb_end;  // groups of RBW row blocks of projections 0..this one, cumulative
-    uint64_t unused;
-};
 struct Fused16Params {
     int kt_count;
     float eps;
@@ -472,7 +463,7 @@ struct Fused16Params {
     uint64_t unused[3];
     Fused16Proj proj[GEMV_MAX_PROJ];
 };
-static_assert(sizeof(Fused16Proj) == 64 && sizeof(Fused16Params) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
+static_assert(sizeof(Fused16Params) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
 constexpr int FUSED16_ARGS_AT = 48;  // offset of the Fused16Params in the argument buffer: three pointers and six ints before it
 
 // The value of a lane of the own 16 lanes (a constant once unrolled): a row broadcast, 0x150 + lane.
@@ -488,10 +479,6 @@ __device__ __forceinline__ int row_lane(uint32_t packed, int at)
         case 12: return row_lane_at<12>(v); case 13: return row_lane_at<13>(v); case 14: return row_lane_at<14>(v); default: return row_lane_at<15>(v);
     }
 }
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v4i_any __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte accesses need four-byte alignment only
-typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
-
 template <int MODE, bool NORM, int NCHB, int RBW>
 __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_chunks,
                                                            int hot_nw, int hot_ldx, int hot_end0, int hot_end1, [[maybe_unused]] Fused16Params args)
@@ -558,7 +545,6 @@ __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, 
     // The vector memory of a compute unit answers in the order of the requests, whichever wavefront they are from: a tile
     // that comes from memory would hold up the input row of a wavefront that asked a little later.  So all wavefronts meet
     // once their row is requested, and ask for the tiles then.
-    typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
     const global_ptr<const v4u_t> tiles = pointer_at<const v4u_t>(P, 0) + lane;
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -1217,7 +1203,6 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
                                                         [[maybe_unused]] RowsParams args)
 {
     extern __shared__ v4i part[];  // [nw][RB][64]
-    typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
     // workgroup (x, y): token group x / 8, group 8y + x % 8 of row blocks, as in gemv_fused16_kernel: the token groups of one group
     // of row blocks run on the same XCD
     const int tg = (int)(blockIdx.x >> 3);
@@ -1231,25 +1216,8 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
     v16u P = ((arg_ptr)((uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + ROWS_ARGS_AT))[pj];
     __builtin_amdgcn_sched_barrier(0);
     const int rows_here = min(16, m - tg * 16);
-    const bool row_ok = (lane & 15) < rows_here;
-
-    // A operand of lane 16 g + r: row r, columns 16 g .. + 15 of a tile; lanes without a row load nothing (the results of their
-    // row are not used)
-    const global_ptr<const uint8_t> a_lane = (global_ptr<const uint8_t>)(uintptr_t)hot_a + (size_t)tg * 16 * TILE_K * kt_count +
-                                             (unsigned)(((lane >> 4) * rows_here + (lane & 15)) * 16);
-    auto load_a = [&](v4i (&af)[NT][4], int kt0) {
-#pragma unroll
-        for (int u = 0; u < NT; ++u)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) asm("" : "=v"(af[u][t]));
-        if (row_ok) {
-#pragma unroll
-            for (int u = 0; u < NT; ++u)
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    af[u][t] = *(global_ptr<const v4i>)(a_lane + (unsigned)((min(kt0 + nw * u, kt_count - 1) * 4 + t) * 64 * rows_here));
-        }
-    };
+    const global_ptr<const uint8_t> group_rows = (global_ptr<const uint8_t>)(uintptr_t)hot_a + (size_t)tg * 16 * TILE_K * kt_count;
+    auto load_a = [&](v4i (&af)[NT][4], int kt0) { rows_load_a<NT>(af, group_rows, lane, rows_here, kt0, nw, kt_count); };
     v4i af[NT][4];
     load_a(af, wave);
     __builtin_amdgcn_sched_barrier(0);
@@ -1257,72 +1225,32 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
     const int rb0 = (group - (pj == 0 ? 0 : (pj == 1 ? end0 : end1))) * RB;
     const int rb_count = (int)(pj == 0 ? hot_blocks & 0xffffu : (pj == 1 ? hot_blocks >> 16 : hot_blocks_nw & 0xffffu));
     const global_ptr<const v4u_t> tiles = (global_ptr<const v4u_t>)(uintptr_t)(pj == 0 ? hot_w0 : (pj == 1 ? hot_w1 : hot_w2)) + lane;
-    auto load_w = [&](v4u_t (&w)[NT][RB], int kt0) {
-#pragma unroll
-        for (int u = 0; u < NT; ++u)
-#pragma unroll
-            for (int r = 0; r < RB; ++r)
-                w[u][r] = __builtin_nontemporal_load(tiles + ((size_t)min(rb0 + r, rb_count - 1) * kt_count + min(kt0 + nw * u, kt_count - 1)) * 64);
-    };
+    auto load_w = [&](v4u_t (&w)[NT][RB], int kt0) { rows_load_w<RB, NT>(w, tiles, rb0, rb_count, kt0, nw, kt_count); };
     v4u_t w[NT][RB];
     load_w(w, wave);
     __builtin_amdgcn_sched_barrier(0);
 
+    // The epilogue's operands are requested behind the tiles, or, where the registers are full of tiles, behind the products.
     asm volatile("" : "+s"(P));
-    const global_ptr<const float> scales = (global_ptr<const float>)(uintptr_t)a_scale;
-    const global_ptr<const float> w_scale = pointer_at<const float>(P, 2), bias = pointer_at<const float>(P, 4), residual = pointer_at<const float>(P, 6);
-    const global_ptr<float> out = pointer_at<float>(P, 8);
-    const global_ptr<int32_t> acc_out = pointer_at<int32_t>(P, 10);
-    const int P_n = (int)P[12];
-
-    // The weights are the first operand of the MFMA, so lane l of a result holds four consecutive outputs, 4 (l / 16) and on, of token
-    // l % 16: wavefront r finishes row block r with loads and stores of 16 bytes.  Its operands are requested behind the tiles, or, where the
-    // registers are full of tiles, behind the products.
     constexpr bool REQUEST_EARLY = RB < 4 && !LOOP;
-    const bool finishing = wave < RB;  // a workgroup has four wavefronts at least
-    const int n_block = (rb0 + wave) * TILE_ROWS, n_lane = n_block + 4 * (lane >> 4), t_lane = tg * 16 + min(lane & 15, rows_here - 1);
-    const bool whole = n_block + TILE_ROWS <= P_n;
-    float e_ws = 0.0f, e_scale = 1.0f;
-    v4f_any e_bias = {0.0f, 0.0f, 0.0f, 0.0f}, e_res = {0.0f, 0.0f, 0.0f, 0.0f};
+    RowsFinish end(P, a_scale, rb0, RB, wave, lane, tg, rows_here);
     auto request = [&]() {
-        if (!(finishing && whole && out)) return;  // uniform over the wavefront
-        int lane_zero = 0;
-        asm volatile("" : "+v"(lane_zero));
-        e_ws = w_scale[lane_zero];
-        e_scale = scales[t_lane];
-        if (bias) e_bias = *(global_ptr<const v4f_any>)(bias + n_lane);
-        if (residual) e_res = *(global_ptr<const v4f_any>)(residual + ((size_t)t_lane * P_n + n_lane));
+        end.request_operands();
+        end.request_scales();
     };
     if constexpr (REQUEST_EARLY) request();
     __builtin_amdgcn_sched_barrier(0);
 
     v4i acc[RB], sums = {0, 0, 0, 0};
-    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 #pragma unroll
     for (int r = 0; r < RB; ++r) acc[r] = (v4i){0, 0, 0, 0};
-    auto multiply = [&](const v4i (&a)[NT][4], const v4u_t (&wt)[NT][RB], int kt0) {
-#pragma unroll
-        for (int u = 0; u < NT; ++u) {
-            if (kt0 + nw * u >= kt_count) break;  // uniform over the wavefront
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, a[u][t], sums, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < RB; ++r) {
-                    const unsigned wd = wt[u][r][t];
-                    const v4i bf = {(int)(wd & 0x03030303u), (int)((wd >> 2) & 0x03030303u), (int)((wd >> 4) & 0x03030303u), (int)((wd >> 6) & 0x03030303u)};
-                    acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf, a[u][t], acc[r], 0, 0, 0);
-                }
-            }
-        }
-    };
     if constexpr (LOOP) {
         for (int kt0 = wave; kt0 < kt_count; kt0 += nw * NT) {  // uniform over the wavefront
             v4i a_next[NT][4];
             v4u_t w_next[NT][RB];
             load_a(a_next, kt0 + nw * NT);
             load_w(w_next, kt0 + nw * NT);
-            multiply(af, w, kt0);
+            rows_multiply<RB, NT>(af, w, kt0, nw, kt_count, acc, sums);
 #pragma unroll
             for (int u = 0; u < NT; ++u) {
 #pragma unroll
@@ -1332,72 +1260,13 @@ __global__ __launch_bounds__(1024) void gemv_rows_kernel(const int8_t *hot_a, co
             }
         }
     } else {
-        multiply(af, w, wave);
+        rows_multiply<RB, NT>(af, w, wave, nw, kt_count, acc, sums);
     }
     if constexpr (!REQUEST_EARLY) {
         __builtin_amdgcn_sched_barrier(0);
         request();
     }
-#pragma unroll
-    for (int r = 0; r < RB; ++r) part[((size_t)wave * RB + r) * 64 + lane] = acc[r] - sums;
-    lds_barrier();
-    if (!finishing) return;
-    const v4i *from = part + wave * 64 + lane;
-    v4i total = {0, 0, 0, 0};
-    int v = 0;
-    for (; v + 4 <= nw; v += 4) {  // uniform, as the rest is
-        v4i got[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) got[i] = from[(v + i) * (RB * 64)];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) total = total + got[i];
-    }
-    if (v < nw) {
-        v4i got[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) got[i] = from[min(v + i, nw - 1) * (RB * 64)];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            if (v + i < nw) total = total + got[i];
-    }
-    if (!row_ok) return;
-    const size_t o = (size_t)t_lane * P_n + n_lane;
-    if (whole) {
-        if (acc_out) *(global_ptr<v4i_any>)(acc_out + o) = total;
-        if (out) {
-            v4f_any y;
-            bool short_ok = invariant_divisor_ok(e_scale);
-            const float recip = recip_of_ok_divisor(e_scale);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float scaled = f32_mul((float)total[i], e_ws);
-                short_ok = short_ok && dividend_ok(scaled);
-                y[i] = div_by_invariant_unchecked(scaled, e_scale, recip);
-            }
-            if (__builtin_expect(!short_ok, 0)) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[i] = f32_div(f32_mul((float)total[i], e_ws), e_scale);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (bias) y[i] = f32_add(y[i], e_bias[i]);
-                if (residual) y[i] = f32_add(y[i], e_res[i]);
-            }
-            *(global_ptr<v4f_any>)(out + o) = y;
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {  // the last row block of a projection
-        if (n_lane + i >= P_n) break;
-        if (acc_out) acc_out[o + i] = total[i];
-        if (out) {
-            float y = f32_div(f32_mul((float)total[i], w_scale[0]), scales[t_lane]);
-            if (bias) y = f32_add(y, bias[n_lane + i]);
-            if (residual) y = f32_add(y, residual[o + i]);
-            out[o + i] = y;
-        }
-    }
+    end.template finish<RB>(acc, sums, part, wave, lane, nw);
 }
 
 // The reference's flat row-major packing, any n and k (rows need not start on a byte boundary).

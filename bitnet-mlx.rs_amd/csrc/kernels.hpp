@@ -147,6 +147,25 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
                      const float *gamma, int sum_order, size_t blocks, bool alone);
 int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m, size_t k, int input_mode, size_t gqa_group, size_t head_dim,
                      const float *gamma, float eps, hipStream_t stream);
+// gemv_die.hip: several tokens in one launch, their rows quantised once on every die.  Only where gemv_die_takes() says so.
+// flags: 16 dies x stride 64-bit words, none of which holds tag before the launch; clear (optional): a second set of them, cleared for the
+// m rows by the launch; looks: how often a workgroup looks at the flags before it quantises its rows itself.
+constexpr int GEMV_DIE_MAX_M = 128;
+constexpr size_t GEMV_DIE_SETS = 16;  // dies whose flags are kept apart
+constexpr int GEMV_DIE_LOOKS = 4096;
+struct DieFlags {
+    uint64_t *flags, *clear;
+    uint64_t tag;
+    unsigned stride;
+    int looks;
+};
+// blocks: 16-row blocks of all projections of the launch; alone: a call of its own, not one of a step
+bool gemv_die_takes(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode, const float *gamma, int sum_order, size_t blocks,
+                    bool alone);
+int launch_gemv_die(const GemvProj *projs, int nproj, const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode, const float *gamma,
+                    float eps, int8_t *q, float *a_scale, const DieFlags &f, hipStream_t stream);
+// clears the flags of m rows in one set
+int launch_clear_die_flags(uint64_t *flags, size_t stride, size_t m, hipStream_t stream);
 // f32 input quantised inside the GEMV launch; only where gemv_fused_supported() says so.  q_out / a_scale_out /
 // a_sum_out (each optional) receive the quantiser's results.
 bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode,

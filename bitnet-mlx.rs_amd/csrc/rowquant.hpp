@@ -391,7 +391,9 @@ struct Row16 {
     float4 v[NCHB], gm[NORM ? NCHB : 1], vs[NSS];
     int chunk[NCHB];
 
-    // Unconditional loads (clamped indices, values discarded).
+    // Unconditional loads (clamped indices, values discarded), also of the chunks that no virtual lane of a row this short has: a branch for
+    // each costs the kernels that do little else more than the loads (the 30-block stack at 4 / 16 / 42 tokens 668 / 808 / 989 us, 666 / 803 / 986
+    // without; one token even).
     template <int MODE>
     __device__ __forceinline__ void load(const float *row, const float *row2, uint64_t magics, int head_chunks, const float *gamma, int chunks,
                                          int nw, int wave, int tid, int in_tile)
@@ -405,7 +407,7 @@ struct Row16 {
             if (wave < 4) {
 #pragma unroll
                 for (int i = 0; i < NSS; ++i)
-                    if (256 * i < chunks) vs[i] = row16_chunk<MODE>(row, row2, magics, head_chunks, min(tid + 256 * i, chunks - 1));
+                    vs[i] = row16_chunk<MODE>(row, row2, magics, head_chunks, min(tid + 256 * i, chunks - 1));
             }
 #pragma unroll
             for (int i = 0; i < NCHB; ++i) gm[i] = reinterpret_cast<const float4 *>(gamma)[min(chunk[i], chunks - 1)];

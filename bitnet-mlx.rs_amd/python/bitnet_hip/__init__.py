@@ -141,6 +141,7 @@ def load_library() -> C.CDLL:
         "bitnet_hip_decoder_projection": (i32, [vp, sz, i32, C.POINTER(vp)]),
         "bitnet_hip_decoder_set_norm": (i32, [vp, sz, i32, vp, i32, vp]),
         "bitnet_hip_decoder_set_chains": (i32, [vp, sz]),
+        "bitnet_hip_decoder_set_row_wait": (i32, [vp, i32]),
         "bitnet_hip_decoder_weight_bytes": (sz, [vp]),
         "bitnet_hip_decoder_decode": (i32, [vp, vp, sz, vp, vp, vp, vp]),
         "bitnet_hip_decoder_graph_create": (i32, [vp, sz, sz, vp, sz, vp, vp, vp, C.POINTER(vp)]),
@@ -1193,6 +1194,11 @@ class DecoderProjections:
         """Row groups a decode step of several token rows is split into (each a chain of launches on its own stream);
         0 and 1 keep all rows in one chain (the default, and the faster form on the device measured)."""
         _check(load_library().bitnet_hip_decoder_set_chains(self._h, int(chains)))
+
+    def set_row_wait(self, looks: int):
+        """How often a workgroup that waits for rows which others quantise looks for them before it quantises them itself
+        (0 .. 4096; bit-identical results)."""
+        _check(load_library().bitnet_hip_decoder_set_row_wait(self._h, int(looks)))
 
     def weight_bytes(self) -> int:
         return load_library().bitnet_hip_decoder_weight_bytes(self._h)

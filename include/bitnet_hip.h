@@ -435,6 +435,10 @@ int bitnet_hip_decoder_set_norm(bitnet_hip_decoder *dec, size_t layer, int which
  * the caller's stream, which is the faster form on the device measured (kernels this short are started one at a time
  * whatever the number of queues); at most 8. */
 int bitnet_hip_decoder_set_chains(bitnet_hip_decoder *dec, size_t chains);
+/* Launches of a step in which some workgroups quantise the rows that others multiply: how often a waiting workgroup looks for its
+ * rows before it quantises them itself, 0 to 4096 (the default, about 0.5 ms; 0: it always does).  Same results, bit for bit.
+ * Synchronises the device; steps recorded by decoder_graph_create keep what they were recorded with. */
+int bitnet_hip_decoder_set_row_wait(bitnet_hip_decoder *dec, int looks);
 /* Packed-weight bytes one decode step streams (sum of n*k/4 over all projections). */
 size_t bitnet_hip_decoder_weight_bytes(const bitnet_hip_decoder *dec);
 /* One decode step: x_in [m, hidden] -> x_out [m, hidden] through all blocks.  A decoder owns one set of activation

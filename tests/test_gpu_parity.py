@@ -3,6 +3,8 @@
 Bar: int8 activations, packed bytes and int32 accumulators bit-exact; f32 scales and outputs compared
 bit-exact where the oracle and the kernel perform the same IEEE operations, and in any case within
 1e-5 relative error (the tolerance the path's specification states)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -1942,3 +1944,68 @@ def test_token_gemv_outputs_that_end_inside_a_row_block(m, n, k, extras):
         layer.update_bias(dev(bias))
     ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias, residual=res)[0]
     assert np.array_equal(host(layer.forward(dev(x), gamma=dev(g), residual=dev(res) if extras else None)), ref)
+
+
+# ---- rows quantised once a die (gemv_die_kernel) -------------------------------------------------------------
+
+def die_scratch(layer, x, gamma=None):
+    """Bytes of workspace the layer wants for x on the null stream, and those without the flags of a launch on dies."""
+    handles = (ctypes.c_void_p * 1)(layer._h)
+    wanted = bh.load_library().bitnet_hip_bitlinear_forward_scratch_on(handles, 1, x.data_ptr(), x.shape[0], gamma.data_ptr() if gamma is not None else None,
+                                                                       bh.SUM_BLOCK256, None)
+    return wanted, layer.workspace_size(x.shape[0])
+
+
+@pytest.mark.parametrize("m,k,n,norm", [(9, 2308, 2560, False), (9, 1028, 40, True), (16, 6912, 2560, False), (17, 2564, 650, True), (5, 8192, 8200, False),
+                                        (33, 4096, 1000, False), (48, 2560, 2570, True), (31, 8192, 648, True), (95, 1536, 1290, True), (128, 1300, 96, True)])
+def test_rows_quantised_once_a_die_bit_exact(m, k, n, norm):
+    """Rows and columns left over, one and two tiles a wavefront, one to four row blocks a workgroup, up to eight token groups: the
+    oracle's bits, on one workspace through calls with other inputs in between (the flags of an earlier call lie in it)."""
+    rng = np.random.default_rng(m + 3 * k + n)
+    w = synth_weights(rng, n, k)
+    qw, ws = orc.quantize_weights_absmean(w)
+    packed = orc.pack_2bit(qw)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "dies")
+    layer.update_weights(dev(w))
+    bias = rng.standard_normal(n, dtype=f32)
+    layer.update_bias(dev(bias))
+    gamma = (1 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    x = dev(synth_activations(rng, m, k))
+    wanted, plain = die_scratch(layer, x, dev(gamma) if norm else None)
+    assert wanted > plain  # with flags: the launch this test is about
+    scratch = torch.full((wanted,), 255, dtype=torch.uint8, device="cuda")
+    for _ in range(3):
+        xs = synth_activations(rng, m, k, outliers=True)
+        xs[m // 2] = 0.0
+        res = rng.standard_normal((m, n), dtype=f32)
+        want = orc.bitlinear_forward(xs, packed, n, ws, g=gamma, bias=bias, residual=res)[0]
+        g = dev(gamma) if norm else None
+        assert np.array_equal(host(layer.forward(dev(xs), gamma=g, residual=dev(res), workspace=scratch)), want)
+        assert np.array_equal(host(layer.forward(dev(xs), gamma=g, residual=dev(res))), want)
+    least = torch.empty((plain,), dtype=torch.uint8, device="cuda")  # no room for flags: two launches
+    assert np.array_equal(host(layer.forward(dev(xs), gamma=g, residual=dev(res), workspace=least)), want)
+
+
+@pytest.mark.parametrize("dims,layers", [((512, 1408, 8, 2, 64), 3), ((2560, 6912, 20, 5, 128), 1)])
+def test_decoder_rows_quantised_once_a_die(dims, layers):
+    """Steps of several token counts, one after the other and recorded, with workgroups that wait for their rows and (no looks at all)
+    with every one that quantises its rows itself: all equal the oracle's chain bit for bit."""
+    rng = np.random.default_rng(sum(dims))
+    dec, ref = build_decoder_packed(rng, layers, *dims, max_tokens=64)
+    for m in (9, 33, 16, 3, 64, 17):
+        xs = synth_activations(rng, m, dims[0])
+        want = oracle_stack(ref, xs, *dims)[0]
+        for looks in (0, 4096):
+            dec.set_row_wait(looks)
+            x = dev(xs)
+            for _ in range(4):  # the third on is a replay
+                assert np.array_equal(host(dec.decode(x)), want), (m, looks)
+            graph = dec.record(x)
+            for _ in range(3):
+                graph.out.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert np.array_equal(host(graph.out), want), (m, looks)
+    for looks in (-1, 4097):
+        with pytest.raises(bh.BitLinearError):
+            dec.set_row_wait(looks)
