@@ -301,7 +301,7 @@ void launch_wave(const ActQuantParams &p, hipStream_t s)
     const int rows_per_block = 4;
     dim3 block(64, rows_per_block);
     dim3 grid((unsigned)((p.m + rows_per_block - 1) / rows_per_block));
-    hipLaunchKernelGGL((act_quant_wave_kernel<MODE, VEC>), grid, block, 0, s, p);
+    launch_kernel((act_quant_wave_kernel<MODE, VEC>), grid, block, 0, s, p);
 }
 
 // LDS for the row's squares where the literal summation order is asked for and a row fits the default limit
@@ -317,7 +317,7 @@ void launch_block(ActQuantParams p, hipStream_t s)
 {
     const size_t lds = launch_squares_lds(p);
     p.seq_in_lds = lds != 0;
-    hipLaunchKernelGGL((act_quant_block_kernel<MODE, NCH, VEC>), dim3((unsigned)p.m), dim3(256), lds, s, p);
+    launch_kernel((act_quant_block_kernel<MODE, NCH, VEC>), dim3((unsigned)p.m), dim3(256), lds, s, p);
 }
 
 template <int MODE>
@@ -345,13 +345,13 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
             const dim3 grid((unsigned)p.m), block(64u * (unsigned)nw);
 #define BITNET_HOT_ARGS p.src.x, x2, p.src.gamma, p.src.k, p.src.head_dim / 4, nw, (int)p.src.ldx, p.src.eps, (int)p.m, args
             if (p.src.gamma) {
-                if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else if (nchb == 2) hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, true, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
+                if (nchb == 1) launch_kernel((act_quant_row_kernel<MODE, true, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else if (nchb == 2) launch_kernel((act_quant_row_kernel<MODE, true, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else launch_kernel((act_quant_row_kernel<MODE, true, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
             } else {
-                if (nchb == 1) hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else if (nchb == 2) hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
-                else hipLaunchKernelGGL((act_quant_row_kernel<MODE, false, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
+                if (nchb == 1) launch_kernel((act_quant_row_kernel<MODE, false, 1>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else if (nchb == 2) launch_kernel((act_quant_row_kernel<MODE, false, 2>), grid, block, 0, s, BITNET_HOT_ARGS);
+                else launch_kernel((act_quant_row_kernel<MODE, false, 4>), grid, block, 0, s, BITNET_HOT_ARGS);
             }
 #undef BITNET_HOT_ARGS
             return;
@@ -629,7 +629,7 @@ int abs_max_workgroups(size_t n, int most)
 
 int launch_abs_max(const float *x, size_t n, int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream, float *parts)
 {
-    hipLaunchKernelGGL(abs_max_kernel, dim3((unsigned)workgroups), dim3(1024), 0, stream, x, n, answers, ticket, parts);
+    launch_kernel(abs_max_kernel, dim3((unsigned)workgroups), dim3(1024), 0, stream, x, n, answers, ticket, parts);
     BITNET_HIP_CHECK_LAUNCH("abs_max_kernel");
     return BITNET_HIP_OK;
 }
@@ -638,14 +638,14 @@ int launch_dynamic_quantize(const float *x, size_t n, int precision, const Dynam
                             int workgroups, unsigned long long *answers, unsigned ticket, hipStream_t stream)
 {
     if (n <= (size_t)DYNAMIC_SMALL) {
-        hipLaunchKernelGGL(dynamic_quantize_small_kernel, dim3(1), dim3(1024), 0, stream, x, (int)n, precision, d, reference_u8, q, scale_out, answers, ticket);
+        launch_kernel(dynamic_quantize_small_kernel, dim3(1), dim3(1024), 0, stream, x, (int)n, precision, d, reference_u8, q, scale_out, answers, ticket);
         BITNET_HIP_CHECK_LAUNCH("dynamic_quantize_small_kernel");
         return BITNET_HIP_OK;
     }
     const int rc = launch_abs_max(x, n, workgroups, answers, ticket, stream, parts);
     if (rc != BITNET_HIP_OK) return rc;
     const size_t blocks = (n + 1023) / 1024;
-    hipLaunchKernelGGL(dynamic_quantize_kernel, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, stream, x, n, precision, d, parts, workgroups,
+    launch_kernel(dynamic_quantize_kernel, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, stream, x, n, precision, d, parts, workgroups,
                        reference_u8, q, scale_out);
     BITNET_HIP_CHECK_LAUNCH("dynamic_quantize_kernel");
     return BITNET_HIP_OK;
@@ -658,7 +658,7 @@ int launch_scaled_quantize(const float *x, size_t n, int precision, float scale,
     const float recip = (float)(1.0 / (double)scale);
     size_t blocks = (n + 1023) / 1024;
     blocks = blocks < 1 ? 1 : (blocks > 2048 ? 2048 : blocks);
-    hipLaunchKernelGGL(scaled_quantize_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, precision, scale, recip, reference_u8,
+    launch_kernel(scaled_quantize_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, precision, scale, recip, reference_u8,
                        q, scale_out);
     BITNET_HIP_CHECK_LAUNCH("scaled_quantize_kernel");
     return BITNET_HIP_OK;
@@ -678,16 +678,16 @@ int launch_absmax_quantize(const float *x, size_t n, int precision, void *scratc
     const size_t rows = (n + 4095) / 4096;
     int blocks = (int)((n + 255) / 256);
     blocks = blocks < 1 ? 1 : (blocks > 1024 ? 1024 : blocks);
-    hipLaunchKernelGGL(absmax_partial_kernel, dim3(blocks), dim3(256), 0, stream, x, n, part);
+    launch_kernel(absmax_partial_kernel, dim3(blocks), dim3(256), 0, stream, x, n, part);
     BITNET_HIP_CHECK_LAUNCH("absmax_partial_kernel");
-    hipLaunchKernelGGL(absmax_scale_kernel, dim3(1), dim3(64), 0, stream, part, blocks, precision, state);
+    launch_kernel(absmax_scale_kernel, dim3(1), dim3(64), 0, stream, part, blocks, precision, state);
     BITNET_HIP_CHECK_LAUNCH("absmax_scale_kernel");
     if (rows) {
-        hipLaunchKernelGGL(absmax_quantize_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(64, 4), 0, stream, x, n, rows, precision,
+        launch_kernel(absmax_quantize_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(64, 4), 0, stream, x, n, rows, precision,
                            state, q, row_sums);
         BITNET_HIP_CHECK_LAUNCH("absmax_quantize_kernel");
     }
-    hipLaunchKernelGGL(absmax_finish_kernel, dim3(1), dim3(64), 0, stream, row_sums, rows, n, state, stats);
+    launch_kernel(absmax_finish_kernel, dim3(1), dim3(64), 0, stream, row_sums, rows, n, state, stats);
     BITNET_HIP_CHECK_LAUNCH("absmax_finish_kernel");
     return BITNET_HIP_OK;
 }

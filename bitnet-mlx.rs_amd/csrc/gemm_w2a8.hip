@@ -814,7 +814,7 @@ int launch_dma(GemmParams p, hipStream_t stream)
     static_assert(lds <= 160 * 1024 && lds * OCC <= 160 * 1024 && OCC <= 4, "LDS budget, priorities 0..3");
     static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_dma_kernel<BM, BN, D, OCC, WN>, lds) : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, D, OCC, WN>), dim3(grid), dim3(256), lds, stream, p);
+    launch_kernel((gemm_dma_kernel<BM, BN, D, OCC, WN>), dim3(grid), dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_dma_kernel");
     return BITNET_HIP_OK;
 }
@@ -1001,7 +1001,7 @@ int launch_ld8(GemmParams p, hipStream_t stream)
     static_assert(lds <= 160 * 1024, "LDS budget");
     static const hipError_t attr = raise_lds_limit(&gemm_ld8_kernel<BM, BN, NST>, lds);
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_ld8_kernel<BM, BN, NST>), dim3(grid), dim3(640), lds, stream, p);
+    launch_kernel((gemm_ld8_kernel<BM, BN, NST>), dim3(grid), dim3(640), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_ld8_kernel");
     return BITNET_HIP_OK;
 }
@@ -1047,7 +1047,7 @@ int launch_tile(GemmParams p, hipStream_t stream)
     constexpr size_t lds = 2 * BM * LDS_PITCH + BM * sizeof(int);
     static const hipError_t attr = lds > 64 * 1024 ? raise_lds_limit(&gemm_tiled_kernel<BM, BN>, lds) : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemm_tiled_kernel<BM, BN>), dim3(grid), dim3(256), lds, stream, p);
+    launch_kernel((gemm_tiled_kernel<BM, BN>), dim3(grid), dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemm_tiled_kernel");
     return BITNET_HIP_OK;
 }
@@ -1203,8 +1203,8 @@ __global__ __launch_bounds__(512, 1) void mfma_rate_kernel(int iters, int *sink,
 int launch_mfma_rate(bool random_operands, int iters, int compute_units, int *sink, hipStream_t stream)
 {
     const dim3 grid((unsigned)compute_units), block(MFMA_RATE_THREADS);
-    if (random_operands) hipLaunchKernelGGL((mfma_rate_kernel<true>), grid, block, 0, stream, iters, sink, 7u);
-    else hipLaunchKernelGGL((mfma_rate_kernel<false>), grid, block, 0, stream, iters, sink, 7u);
+    if (random_operands) launch_kernel((mfma_rate_kernel<true>), grid, block, 0, stream, iters, sink, 7u);
+    else launch_kernel((mfma_rate_kernel<false>), grid, block, 0, stream, iters, sink, 7u);
     BITNET_HIP_CHECK_LAUNCH("mfma_rate_kernel");
     return BITNET_HIP_OK;
 }

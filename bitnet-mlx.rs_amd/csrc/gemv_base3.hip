@@ -186,7 +186,7 @@ int launch_retile_base3(const uint8_t *flat, size_t n, size_t k, uint8_t *tiled,
     if (total == 0) return BITNET_HIP_OK;
     const size_t blocks = (total + 255) / 256;
     if (blocks > 0x7fffffffu) return fail(BITNET_HIP_INVALID_CONFIG, "retile_base3: %zu x %zu is too large", n, k);
-    hipLaunchKernelGGL(retile_base3_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, flat, n, k, (k + B3_TILE_K - 1) / B3_TILE_K,
+    launch_kernel(retile_base3_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, flat, n, k, (k + B3_TILE_K - 1) / B3_TILE_K,
                        tiled, total);
     BITNET_HIP_CHECK_LAUNCH("retile_base3_kernel");
     return BITNET_HIP_OK;
@@ -203,7 +203,7 @@ int launch_gemv_base3(const uint8_t *tiled, const int8_t *a, int32_t *acc, float
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_base3_kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL(gemv_base3_kernel, dim3((unsigned)row_blocks(n)), dim3(256), lds, stream, tiled, a, acc, out, w_scale, a_scale,
+    launch_kernel(gemv_base3_kernel, dim3((unsigned)row_blocks(n)), dim3(256), lds, stream, tiled, a, acc, out, w_scale, a_scale,
                        (int)n, (int)k, (int)kt_count);
     BITNET_HIP_CHECK_LAUNCH("gemv_base3_kernel");
     return BITNET_HIP_OK;

@@ -253,7 +253,7 @@ int launch(const Launch &l)
                                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST)
                                                      : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemv_die_kernel<MODE, NORM, RB, NT>), l.grid, dim3(64u * (unsigned)l.nw), (size_t)l.nw * RB * 1024, l.stream, l.x, l.x2, l.gamma, l.k,
+    launch_kernel((gemv_die_kernel<MODE, NORM, RB, NT>), l.grid, dim3(64u * (unsigned)l.nw), (size_t)l.nw * RB * 1024, l.stream, l.x, l.x2, l.gamma, l.k,
                        l.nw, l.ldx, l.m_kt, l.ends, l.quantisers_tgroups, l.tg_magic, l.p);
     BITNET_HIP_CHECK_LAUNCH("gemv_die_kernel");
     return BITNET_HIP_OK;
@@ -366,7 +366,7 @@ int launch_gemv_die(const GemvProj *projs, int nproj, const float *x, const floa
 
 int launch_clear_die_flags(uint64_t *flags, size_t stride, size_t m, hipStream_t stream)
 {
-    hipLaunchKernelGGL(clear_die_flags_kernel, dim3((unsigned)GEMV_DIE_SETS), dim3(128), 0, stream, flags, (int)stride, (int)m);
+    launch_kernel(clear_die_flags_kernel, dim3((unsigned)GEMV_DIE_SETS), dim3(128), 0, stream, flags, (int)stride, (int)m);
     BITNET_HIP_CHECK_LAUNCH("clear_die_flags_kernel");
     return BITNET_HIP_OK;
 }

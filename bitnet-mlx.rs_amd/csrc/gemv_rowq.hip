@@ -246,7 +246,7 @@ int launch(const Launch &l)
                                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST)
                                                     : hipSuccess;
     BITNET_HIP_TRY(attr);
-    hipLaunchKernelGGL((gemv_rowq_kernel<MODE, NORM, RB, NT, CPR>), l.grid, dim3(64 * WAVES), bytes, l.stream, l.x, l.gamma, l.p.proj[0].w, l.p.proj[1].w,
+    launch_kernel((gemv_rowq_kernel<MODE, NORM, RB, NT, CPR>), l.grid, dim3(64 * WAVES), bytes, l.stream, l.x, l.gamma, l.p.proj[0].w, l.p.proj[1].w,
                        l.p.proj[2].w, l.m_kt, l.ends, l.blocks, l.blocks_width, l.groups, l.p);
     BITNET_HIP_CHECK_LAUNCH("gemv_rowq_kernel");
     return BITNET_HIP_OK;

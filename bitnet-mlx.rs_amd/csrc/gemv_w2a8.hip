@@ -1315,7 +1315,7 @@ int launch_mb_mode(const GemvParams &p, hipStream_t stream)
 {
     size_t lds = (size_t)MB * p.kt_count * 16 * sizeof(uint4);
     dim3 grid((unsigned)p.proj[p.nproj - 1].rb_end);
-    hipLaunchKernelGGL((gemv_tiled_kernel<MB, MODE>), grid, dim3(256), lds, stream, p);
+    launch_kernel((gemv_tiled_kernel<MB, MODE>), grid, dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemv_tiled_kernel");
     return BITNET_HIP_OK;
 }
@@ -1334,10 +1334,10 @@ int launch_fused_mode(const GemvParams &p, hipStream_t stream)
     const size_t lds_q = (size_t)p.kt_count * 16 * sizeof(uint4), lds_sq = squares_lds_bytes(p.k);
     const size_t lds = (norm && p.src.sum_order == BITNET_HIP_SUM_SEQUENTIAL && lds_sq > lds_q) ? lds_sq : lds_q;
     const dim3 grid((unsigned)p.proj[p.nproj - 1].rb_end);
-    if (norm && small) hipLaunchKernelGGL((gemv_fused_kernel<MODE, true, 3, RBW>), grid, dim3(256), lds, stream, p);
-    else if (norm) hipLaunchKernelGGL((gemv_fused_kernel<MODE, true, FUSED_NCH, RBW>), grid, dim3(256), lds, stream, p);
-    else if (small) hipLaunchKernelGGL((gemv_fused_kernel<MODE, false, 3, RBW>), grid, dim3(256), lds, stream, p);
-    else hipLaunchKernelGGL((gemv_fused_kernel<MODE, false, FUSED_NCH, RBW>), grid, dim3(256), lds, stream, p);
+    if (norm && small) launch_kernel((gemv_fused_kernel<MODE, true, 3, RBW>), grid, dim3(256), lds, stream, p);
+    else if (norm) launch_kernel((gemv_fused_kernel<MODE, true, FUSED_NCH, RBW>), grid, dim3(256), lds, stream, p);
+    else if (small) launch_kernel((gemv_fused_kernel<MODE, false, 3, RBW>), grid, dim3(256), lds, stream, p);
+    else launch_kernel((gemv_fused_kernel<MODE, false, FUSED_NCH, RBW>), grid, dim3(256), lds, stream, p);
     BITNET_HIP_CHECK_LAUNCH("gemv_fused_kernel");
     return BITNET_HIP_OK;
 }
@@ -1363,8 +1363,8 @@ int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src,
 #define BITNET_HOT_ARGS src.x, x2, src.gamma, src.k, src.head_dim / 4, nw, (int)src.ldx, end0, end1
 #define BITNET_F16_LAUNCH(NCHB) \
     do { \
-        if (norm) hipLaunchKernelGGL((gemv_fused16_kernel<MODE, true, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
-        else hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
+        if (norm) launch_kernel((gemv_fused16_kernel<MODE, true, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
+        else launch_kernel((gemv_fused16_kernel<MODE, false, NCHB, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p); \
     } while (0)
     // rows of more than 16 k-tiles take at most four row blocks a workgroup (fused16_row_blocks_per_workgroup)
     if constexpr (RBW > 4) {
@@ -1375,7 +1375,7 @@ int launch_fused16_mode(const Fused16Params &p, int nproj, const RowSource &src,
         else if (nchb == 2) BITNET_F16_LAUNCH(2);
         else if constexpr (RBW <= 2) {  // what gemv_fused_supported lets through: no norm
             if (norm) return fail(BITNET_HIP_UNSUPPORTED, "fused GEMV: %d k-tiles with a norm", p.kt_count);
-            hipLaunchKernelGGL((gemv_fused16_kernel<MODE, false, 4, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p);
+            launch_kernel((gemv_fused16_kernel<MODE, false, 4, RBW>), grid, block, 0, stream, BITNET_HOT_ARGS, p);
         } else return fail(BITNET_HIP_UNSUPPORTED, "fused GEMV: %d row blocks a workgroup for %d k-tiles", RBW, p.kt_count);
     }
 #undef BITNET_F16_LAUNCH
@@ -1411,7 +1411,7 @@ int launch_rows(const RowsParams &p, int nproj, const int8_t *a, const float *a_
     const dim3 grid(8u * (unsigned)((m + 15) / 16), ((unsigned)p.proj[nproj - 1].rb_end + 7u) / 8u);
     const unsigned end0 = nproj > 1 ? (unsigned)p.proj[0].rb_end : 0xffffu, end1 = nproj > 2 ? (unsigned)p.proj[1].rb_end : 0xffffu;
     auto blocks = [&](int j) { return (unsigned)row_blocks((size_t)p.proj[j].n); };
-    hipLaunchKernelGGL((gemv_rows_kernel<RB, NT, LOOP>), grid, dim3(64u * (unsigned)nw), (size_t)nw * RB * 1024, stream, a, p.proj[0].w, p.proj[1].w,
+    launch_kernel((gemv_rows_kernel<RB, NT, LOOP>), grid, dim3(64u * (unsigned)nw), (size_t)nw * RB * 1024, stream, a, p.proj[0].w, p.proj[1].w,
                        p.proj[2].w, (unsigned)m | ((unsigned)p.kt_count << 16), end0 | (end1 << 16), blocks(0) | (blocks(1) << 16),
                        blocks(2) | ((unsigned)nw << 16), a_scale, p);
     BITNET_HIP_CHECK_LAUNCH("gemv_rows_kernel");
@@ -1442,24 +1442,24 @@ int launch_mfma_rb(const GemvProj *projs, int nproj, const int8_t *a, const floa
         const size_t lds = m * (k + 16);
         if (fast && m >= 5 && lds + 4096 * RB + 512 <= 64 * 1024 && (k <= 3072 || (k <= 8192 && m <= 8))) {  // + the kernel's static LDS
             if (k <= 3072)
-                hipLaunchKernelGGL((gemv_mfma_lds_kernel<RB, 0>), dim3((unsigned)end), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, p);
+                launch_kernel((gemv_mfma_lds_kernel<RB, 0>), dim3((unsigned)end), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, p);
             else
-                hipLaunchKernelGGL((gemv_mfma_lds_kernel<RB, 1>), dim3((unsigned)end), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, p);
+                launch_kernel((gemv_mfma_lds_kernel<RB, 1>), dim3((unsigned)end), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, p);
             BITNET_HIP_CHECK_LAUNCH("gemv_mfma_lds_kernel");
             return BITNET_HIP_OK;
         }
         // more than one double-buffered batch per wavefront, but few enough k-tiles for one batch without the second buffer
         constexpr int PF2 = RB == 1 ? 4 : (RB == 2 ? 3 : 2), PF1 = RB == 1 ? 8 : (RB == 2 ? 4 : 3);
         if (fast && p.kt_count > 4 * PF2 && p.kt_count <= 4 * PF1) {
-            hipLaunchKernelGGL((gemv_mfma_kernel<RB, 1, true, true>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
+            launch_kernel((gemv_mfma_kernel<RB, 1, true, true>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
             BITNET_HIP_CHECK_LAUNCH("gemv_mfma_kernel");
             return BITNET_HIP_OK;
         }
     }
     if (fast)
-        hipLaunchKernelGGL((gemv_mfma_kernel<RB, MT, true>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
+        launch_kernel((gemv_mfma_kernel<RB, MT, true>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
     else
-        hipLaunchKernelGGL((gemv_mfma_kernel<RB, MT, false>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
+        launch_kernel((gemv_mfma_kernel<RB, MT, false>), dim3((unsigned)end), dim3(256), 0, stream, p.a, p.k, p.m, p.kt_count, p);
     BITNET_HIP_CHECK_LAUNCH("gemv_mfma_kernel");
     return BITNET_HIP_OK;
 }
@@ -1495,12 +1495,12 @@ int launch_mfma_tg(const GemvProj *projs, int nproj, const int8_t *a, const floa
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_mfma_tg_kernel<RB, 3>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)tg_lds_bytes(3072));
         BITNET_HIP_TRY(attr);
-        hipLaunchKernelGGL((gemv_mfma_tg_kernel<RB, 3>), dim3(grid), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, end, tgroups, p);
+        launch_kernel((gemv_mfma_tg_kernel<RB, 3>), dim3(grid), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, end, tgroups, p);
     } else {
         static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_mfma_tg_kernel<RB, 8>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)tg_lds_bytes(8192));
         BITNET_HIP_TRY(attr);
-        hipLaunchKernelGGL((gemv_mfma_tg_kernel<RB, 8>), dim3(grid), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, end, tgroups, p);
+        launch_kernel((gemv_mfma_tg_kernel<RB, 8>), dim3(grid), dim3(256), lds, stream, p.a, p.k, p.m, p.kt_count, end, tgroups, p);
     }
     BITNET_HIP_CHECK_LAUNCH("gemv_mfma_tg_kernel");
     return BITNET_HIP_OK;
@@ -1512,7 +1512,7 @@ int launch_gemv_rowmajor(const uint8_t *packed, const int8_t *a, int32_t *out, s
                          hipStream_t stream)
 {
     if (n == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(gemv_rowmajor_kernel, dim3((unsigned)((n + 3) / 4)), dim3(64, 4), 0, stream, packed, a,
+    launch_kernel(gemv_rowmajor_kernel, dim3((unsigned)((n + 3) / 4)), dim3(64, 4), 0, stream, packed, a,
                        out, n, k);
     BITNET_HIP_CHECK_LAUNCH("gemv_rowmajor_kernel");
     return BITNET_HIP_OK;

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void move_kernel(uint8_t *dst, const uint8_t *
 hipError_t launch_move(uint8_t *dst, const uint8_t *src, size_t bytes, const float *scalar, float *scalar_out, hipStream_t stream)
 {
     const size_t blocks = (bytes + 16383) / 16384;  // 16 KiB a workgroup: one batch of loads
-    hipLaunchKernelGGL(move_kernel, dim3((unsigned)(blocks ? blocks : 1)), dim3(256), 0, stream, dst, src, bytes, scalar, scalar_out);
+    launch_kernel(move_kernel, dim3((unsigned)(blocks ? blocks : 1)), dim3(256), 0, stream, dst, src, bytes, scalar, scalar_out);
     return hipGetLastError();
 }
 
@@ -214,7 +214,7 @@ hipError_t launch_move_pieces(const Pieces &pieces, int n, hipStream_t stream)
     unsigned most = 0;
     for (int i = 0; i < n; ++i) most = pieces.count[i] > most ? pieces.count[i] : most;
     if (most == 0) return hipSuccess;
-    hipLaunchKernelGGL(move_pieces_kernel, dim3(most / 4096 + (most % 4096 != 0), (unsigned)n), dim3(256), 0, stream, pieces);
+    launch_kernel(move_pieces_kernel, dim3(most / 4096 + (most % 4096 != 0), (unsigned)n), dim3(256), 0, stream, pieces);
     return hipGetLastError();
 }
 

@@ -700,7 +700,7 @@ int launch_pack_2bit(const int8_t *q, size_t count, uint8_t *packed, hipStream_t
 {
     size_t nbytes = (count + 3) / 4;
     if (nbytes == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(pack_2bit_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, q, count, packed, nbytes);
+    launch_kernel(pack_2bit_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, q, count, packed, nbytes);
     BITNET_HIP_CHECK_LAUNCH("pack_2bit_kernel");
     return BITNET_HIP_OK;
 }
@@ -708,7 +708,7 @@ int launch_pack_2bit(const int8_t *q, size_t count, uint8_t *packed, hipStream_t
 int launch_unpack_2bit(const uint8_t *packed, size_t count, int8_t *q, hipStream_t stream)
 {
     if (count == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(unpack_2bit_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, stream, packed, count, q);
+    launch_kernel(unpack_2bit_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, stream, packed, count, q);
     BITNET_HIP_CHECK_LAUNCH("unpack_2bit_kernel");
     return BITNET_HIP_OK;
 }
@@ -716,7 +716,7 @@ int launch_unpack_2bit(const uint8_t *packed, size_t count, int8_t *q, hipStream
 int launch_lookup_compute(int kind, const int8_t *w, const float *x, float *out, size_t n, hipStream_t stream)
 {
     if (n == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(lookup_compute_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, kind, w, x, out, n);
+    launch_kernel(lookup_compute_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, kind, w, x, out, n);
     BITNET_HIP_CHECK_LAUNCH("lookup_compute_kernel");
     return BITNET_HIP_OK;
 }
@@ -725,7 +725,7 @@ int launch_pack_base3(const int8_t *q, size_t count, uint8_t *packed, hipStream_
 {
     size_t nbytes = (count + 4) / 5;
     if (nbytes == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(pack_base3_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, q, count, packed, nbytes);
+    launch_kernel(pack_base3_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, q, count, packed, nbytes);
     BITNET_HIP_CHECK_LAUNCH("pack_base3_kernel");
     return BITNET_HIP_OK;
 }
@@ -733,7 +733,7 @@ int launch_pack_base3(const int8_t *q, size_t count, uint8_t *packed, hipStream_
 int launch_unpack_base3(const uint8_t *packed, size_t count, int8_t *q, hipStream_t stream)
 {
     if (count == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(unpack_base3_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, stream, packed, count, q);
+    launch_kernel(unpack_base3_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, stream, packed, count, q);
     BITNET_HIP_CHECK_LAUNCH("unpack_base3_kernel");
     return BITNET_HIP_OK;
 }
@@ -742,7 +742,7 @@ int launch_base3_to_2bit(const uint8_t *base3, size_t count, uint8_t *packed, hi
 {
     size_t nbytes = (count + 3) / 4;
     if (nbytes == 0) return BITNET_HIP_OK;
-    hipLaunchKernelGGL(base3_to_2bit_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, base3, count, packed, nbytes);
+    launch_kernel(base3_to_2bit_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, base3, count, packed, nbytes);
     BITNET_HIP_CHECK_LAUNCH("base3_to_2bit_kernel");
     return BITNET_HIP_OK;
 }
@@ -751,17 +751,17 @@ int launch_quantize_weights(const float *w, size_t n, size_t k, int method, floa
                             double *row_sums, uint8_t *packed, float *w_scale, int8_t *q_i8, hipStream_t stream)
 {
     if (n > 0 && k > 0) {
-        hipLaunchKernelGGL(absmean_rows_kernel, dim3(blocks_for(n, 4)), dim3(64, 4), 0, stream, w, n, k, row_sums);
+        launch_kernel(absmean_rows_kernel, dim3(blocks_for(n, 4)), dim3(64, 4), 0, stream, w, n, k, row_sums);
         BITNET_HIP_CHECK_LAUNCH("absmean_rows_kernel");
     }
-    hipLaunchKernelGGL(absmean_final_kernel, dim3(1), dim3(1024), 0, stream, row_sums, n, k, w_scale);
+    launch_kernel(absmean_final_kernel, dim3(1), dim3(1024), 0, stream, row_sums, n, k, w_scale);
     BITNET_HIP_CHECK_LAUNCH("absmean_final_kernel");
     const size_t count = n * k;
     if (count == 0) return BITNET_HIP_OK;
     const bool dense = aligned(w, 16) && aligned(packed, 4) && (!q_i8 || aligned(q_i8, 4));
     // at most eight workgroups a compute unit: one round, and no more dispatches than that
     const unsigned blocks = blocks_for(count, 4096);
-    hipLaunchKernelGGL(ternarize_pack_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, stream, w, count,
+    launch_kernel(ternarize_pack_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, stream, w, count,
                        method, threshold_factor, w_scale, packed, q_i8, dense);
     BITNET_HIP_CHECK_LAUNCH("ternarize_pack_kernel");
     return BITNET_HIP_OK;
@@ -783,7 +783,7 @@ int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int me
     const int clip = outlier_threshold > 0.0f ? 1 : 0;
     const size_t count = n * k, nbytes = (count + 3) / 4;
     if (count == 0) {
-        hipLaunchKernelGGL(wq_empty_kernel, dim3(1), dim3(1), 0, stream, clip, w_scale, stats);
+        launch_kernel(wq_empty_kernel, dim3(1), dim3(1), 0, stream, clip, w_scale, stats);
         BITNET_HIP_CHECK_LAUNCH("wq_empty_kernel");
         return BITNET_HIP_OK;
     }
@@ -801,15 +801,15 @@ int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int me
     do {                                                                                                                  \
         double *sums = row_sums + (PASS == WQ_OPTIMAL ? 4 : 2 * at) * n;                                                  \
         prev.state = states + at;                                                                                         \
-        if (fold) hipLaunchKernelGGL((wq_rows_kernel<PASS, true>), rgrid, rblock, 0, stream, w, n, k, state, normalize,   \
+        if (fold) launch_kernel((wq_rows_kernel<PASS, true>), rgrid, rblock, 0, stream, w, n, k, state, normalize,   \
                                      clip, sums, row_max, packed_rows, q_i8, prev);                                       \
-        else hipLaunchKernelGGL((wq_rows_kernel<PASS, false>), rgrid, rblock, 0, stream, w, n, k, state, normalize, clip, \
+        else launch_kernel((wq_rows_kernel<PASS, false>), rgrid, rblock, 0, stream, w, n, k, state, normalize, clip, \
                                 sums, row_max, packed_rows, q_i8, prev);                                                  \
         BITNET_HIP_CHECK_LAUNCH("wq_rows_kernel");                                                                        \
         if (fold) state = states + at;                                                                                    \
         prev.pass = PASS; prev.sums = sums;                                                                               \
         if (!fold || FINISH) {                                                                                            \
-            hipLaunchKernelGGL((wq_final_kernel<PASS>), dim3(1), dim3(1024), 0, stream, sums, row_max, n, k, state,       \
+            launch_kernel((wq_final_kernel<PASS>), dim3(1), dim3(1024), 0, stream, sums, row_max, n, k, state,       \
                                states + at, prev.rule, clip, w_scale, stats);                                             \
             BITNET_HIP_CHECK_LAUNCH("wq_final_kernel");                                                                   \
             state = states + at;                                                                                          \
@@ -827,7 +827,7 @@ int launch_quantize_weights_reference(const float *w, size_t n, size_t k, int me
     BITNET_WQ_PASS(WQ_SCALE, true);
 #undef BITNET_WQ_PASS
     if (!packed_rows) {
-        hipLaunchKernelGGL(wq_ternarize_pack_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, w, count, state,
+        launch_kernel(wq_ternarize_pack_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, w, count, state,
                            normalize, clip, packed, q_i8, nbytes);
         BITNET_HIP_CHECK_LAUNCH("wq_ternarize_pack_kernel");
     }
@@ -843,12 +843,12 @@ int launch_retile(const uint8_t *packed, size_t n, size_t k, int layout, uint8_t
     if (layout == BITNET_HIP_LAYOUT_OUT_IN) {
         const bool dwords = k % 16 == 0 && aligned(packed, 4);
         uint32_t *back = canonical && k % 16 == 0 && aligned(canonical, 4) ? reinterpret_cast<uint32_t *>(canonical) : nullptr;
-        hipLaunchKernelGGL(retile_kernel, rows_grid((kt_count + RETILE_KT - 1) / RETILE_KT, row_blocks(n)), dim3(256), 0, stream, packed, n, k, out, kt_count, dwords,
+        launch_kernel(retile_kernel, rows_grid((kt_count + RETILE_KT - 1) / RETILE_KT, row_blocks(n)), dim3(256), 0, stream, packed, n, k, out, kt_count, dwords,
                            back, w_scale, w_scale_out);
         BITNET_HIP_CHECK_LAUNCH("retile_kernel");
         if (back || !canonical) return BITNET_HIP_OK;
     } else {
-        hipLaunchKernelGGL(retile_in_out_kernel, rows_grid(blocks_for(row_blocks(n), 64), 16 * (size_t)kt_count), dim3(64), 0, stream,
+        launch_kernel(retile_in_out_kernel, rows_grid(blocks_for(row_blocks(n), 64), 16 * (size_t)kt_count), dim3(64), 0, stream,
                            packed, n, k, out, kt_count, n % 16 == 0 && aligned(packed, 4), w_scale, w_scale_out);
         BITNET_HIP_CHECK_LAUNCH("retile_in_out_kernel");
         if (!canonical) return BITNET_HIP_OK;
@@ -862,12 +862,12 @@ int launch_untile(const uint8_t *tiled, size_t n, size_t k, uint8_t *packed, hip
     if (nbytes == 0) return BITNET_HIP_OK;
     const uint32_t *src = reinterpret_cast<const uint32_t *>(tiled);
     if (k % 16 == 0 && aligned(packed, 4)) {
-        hipLaunchKernelGGL(untile_rows_kernel, rows_grid(blocks_for(k / 16, 256), n), dim3(256), 0, stream, src, (unsigned)(k / 16), n,
+        launch_kernel(untile_rows_kernel, rows_grid(blocks_for(k / 16, 256), n), dim3(256), 0, stream, src, (unsigned)(k / 16), n,
                            reinterpret_cast<uint32_t *>(packed), (unsigned)k_tiles(k));
         BITNET_HIP_CHECK_LAUNCH("untile_rows_kernel");
         return BITNET_HIP_OK;
     }
-    hipLaunchKernelGGL(untile_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, src, n, k, packed, k_tiles(k), nbytes);
+    launch_kernel(untile_kernel, dim3(blocks_for(nbytes, 256)), dim3(256), 0, stream, src, n, k, packed, k_tiles(k), nbytes);
     BITNET_HIP_CHECK_LAUNCH("untile_kernel");
     return BITNET_HIP_OK;
 }
