@@ -18,6 +18,8 @@
 // Lanes l, l+16, l+32, l+48 share a row, so the decode GEMV combines them with two shuffles.
 // Positions outside the matrix hold code 1 (weight 0) and code 3 is rewritten to code 1, so the
 // contraction kernels never see code 3.
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace bitnet {
@@ -105,19 +107,29 @@ __device__ __forceinline__ double wave_sum_f64(double p)
 }
 
 // Element c of a row for c = lane, lane + 64, .. below k, in ascending order, with up to U loads in flight: the f64 chains
-// of the row sums fix the order of the additions, not that of the loads.
-template <int U, typename F>
-__device__ __forceinline__ void for_row(const float *row, size_t k, int lane, F &&add)
+// of the row sums fix the order of the additions, not that of the loads.  ready: what is done to the elements of a group, all at once.
+template <int U, typename R, typename F>
+__device__ __forceinline__ void for_row(const float *row, size_t k, int lane, R &&ready, F &&add)
 {
     size_t c = lane;
     for (size_t end = 64 * U; end <= k; end += 64 * U, c += 64 * U) {  // uniform: every lane of the wavefront is in it
         float v[U];
 #pragma unroll
         for (int i = 0; i < U; ++i) v[i] = row[c + 64 * i];
+        ready(v);
 #pragma unroll
         for (int i = 0; i < U; ++i) add(v[i], c + 64 * i);
     }
-    for (; c < k; c += 64) add(row[c], c);
+    for (; c < k; c += 64) {
+        float v[1] = {row[c]};
+        ready(v);
+        add(v[0], c);
+    }
+}
+template <int U, typename F>
+__device__ __forceinline__ void for_row(const float *row, size_t k, int lane, F &&add)
+{
+    for_row<U>(row, k, lane, [](auto &) {}, add);
 }
 
 // Sum of |w| of one row in f64: lane l adds columns l, l+64, ... in ascending order, then the
@@ -210,6 +222,15 @@ __device__ __forceinline__ uint32_t quad_dword(uint32_t byte, int lane)
     w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);
     w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x4E, 0xf, 0xf, true);
     return w;
+}
+
+// Byte j of lane i of four becomes byte i of lane j.
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane)
+{
+    uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+    x = __builtin_amdgcn_perm(y, x, lane & 1 ? 0x03070105u : 0x06020400u);
+    y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+    return __builtin_amdgcn_perm(y, x, lane & 2 ? 0x03020706u : 0x05040100u);
 }
 
 // A wavefront takes 1024 consecutive weights: load i (of four) is one 16-byte chunk a lane, chunks in lane order, so loads
@@ -318,15 +339,37 @@ __device__ __forceinline__ float wq_normalised(float w, const WqView &p)
     if (p.fast && __builtin_amdgcn_ballot_w64(!dividend_ok(d)) == 0) return div_by_invariant_unchecked(d, p.st.sd, p.recip);
     return f32_div(d, p.st.sd);
 }
-__device__ __forceinline__ float wq_processed(float w, const WqView &p)
+// The same for U elements a lane: one look at the largest and the smallest |dividend| (a zero takes the way above) in place of one at each, and
+// U divisions that do not wait for each other.  6912 x 2560, the passes that normalise: 15.3, 16.1 and 22.2 -> 13.8, 14.3 and 19.2 us.
+template <int U>
+__device__ __forceinline__ void wq_normalise(float (&w)[U], const WqView &p)
 {
-    float x = wq_normalised(w, p);
+    if (!p.normalize) return;
+    float d[U], lo = __builtin_inff(), hi = 0.0f;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        d[i] = w[i] - p.st.mean;
+        lo = fminf(lo, fabsf(d[i]));
+        hi = fmaxf(hi, fabsf(d[i]));
+    }
+    if (p.fast && __builtin_amdgcn_ballot_w64(!(lo >= 0x1p-63f && hi < 0x1p63f)) == 0) {
+#pragma unroll
+        for (int i = 0; i < U; ++i) w[i] = div_by_invariant_unchecked(d[i], p.st.sd, p.recip);
+    } else {
+#pragma unroll
+        for (int i = 0; i < U; ++i) w[i] = wq_normalised(w[i], p);
+    }
+}
+// x: normalised.
+__device__ __forceinline__ float wq_clipped(float x, const WqView &p)
+{
     if (p.clip) {
         x = x > p.st.hi ? p.st.hi : x;
         x = x < p.st.lo ? p.st.lo : x;
     }
     return x;
 }
+__device__ __forceinline__ float wq_processed(float w, const WqView &p) { return wq_clipped(wq_normalised(w, p), p); }
 __device__ __forceinline__ float wq_code(float x, float thr) { return x > thr ? 1.0f : (x < -thr ? -1.0f : 0.0f); }
 
 __constant__ float wq_factors[10] = {0.3f, 0.4f, 0.5f, 0.6f, 0.7f, 0.8f, 0.9f, 1.0f, 1.1f, 1.2f};
@@ -408,13 +451,18 @@ __device__ __forceinline__ void wq_finish_previous(WqState &st, const WqPrevious
         const double *sums = prev.sums + (size_t)wave * n;
         double s = 0.0;
         int row = lane;
-        for (; row + 7 * 64 < rows; row += 8 * 64) {
-            double t[8];
+        const auto add = [&](auto batch) {  // so many loads in flight: 32, then 8 (8 throughout: 0.5 us a pass more at 2048 rows)
+            constexpr int U = decltype(batch)::value;
+            for (; row + 63 - lane + (U - 1) * 64 < rows; row += U * 64) {
+                double t[U];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) t[i] = sums[row + 64 * i];
+                for (int i = 0; i < U; ++i) t[i] = sums[row + 64 * i];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s = s + t[i];
-        }
+                for (int i = 0; i < U; ++i) s = s + t[i];
+            }
+        };
+        add(std::integral_constant<int, 32>());
+        add(std::integral_constant<int, 8>());
         for (; row < rows; row += 64) s = s + sums[row];
         s = wave_sum_f64(s);
         if (lane == 0) tot[wave] = s;
@@ -462,32 +510,67 @@ __global__ __launch_bounds__(256) void wq_rows_kernel(const float *w, size_t n, 
 #pragma unroll
         for (int f = 0; f < 10; ++f) cand[f] = f32_mul(p.st.mean_abs, wq_factors[f]);
     }
-    for_row<PASS == WQ_OPTIMAL ? 4 : 10>(w + row * k, k, lane, [&](float v, size_t c) {
+    [[maybe_unused]] const auto scale_step = [&](float v) {
+        const float x = wq_clipped(v, p);
+        const float q = wq_code(x, p.st.thr);
+        acc[0] = acc[0] + (double)f32_mul(x, q);
+        nonzero += __popcll(__builtin_amdgcn_ballot_w64(q != 0.0f));  // sum of q * q: a count, exact in any order
+        return q;
+    };
+    size_t first = 0;  // column
+    if constexpr (PASS == WQ_SCALE) {
+        // Four groups of 64 columns at a time: the quads of lanes exchange codes, so that a lane has four consecutive columns of one group
+        // and stores them as a dword and a byte, in place of a byte store a column and a byte store a group.  This pass on 6912 x 2560:
+        // 25.2 -> 22.2 us, on 14336 x 8192 153 -> 122 (with the normalising above 19.2 and 119; the read alone takes 12 and 85).
+        if (packed && (reinterpret_cast<uintptr_t>(q_i8) & 3) == 0) {
+            for (const float *p4 = w + row * k + lane; first + 256 <= k;) {
+                const int groups = first + 512 <= k ? 8 : 4;  // eight loads in flight
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = p4[first + 64 * min(i, groups - 1)];
+                wq_normalise(v, p);
+#pragma unroll
+                for (int h = 0; h < 8; h += 4) {
+                    if (h >= groups) break;
+                    uint32_t codes = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) codes |= (uint32_t)((int)scale_step(v[h + i]) + 1) << (8 * i);
+                    codes = quad_transpose(codes, lane);
+                    const size_t at = row * k + first + 64 * (h + (lane & 3)) + (lane & ~3);
+                    if (q_i8) *reinterpret_cast<uint32_t *>(q_i8 + at) = ((codes | 0x80808080u) - 0x01010101u) ^ 0x80808080u;
+                    codes |= codes >> 6;
+                    packed[at / 4] = (uint8_t)(codes | (codes >> 12));
+                }
+                first += 64 * groups;
+            }
+        }
+    }
+    const auto ready = [&](auto &v) {
+        if constexpr (PASS != WQ_SUM && PASS != WQ_SQDIFF) wq_normalise(v, p);
+    };
+    for_row<PASS == WQ_OPTIMAL ? 4 : 10>(w + row * k + first, k - first, lane, ready, [&](float v, size_t c) {
         if constexpr (PASS == WQ_SUM) {
             acc[0] = acc[0] + (double)v;
         } else if constexpr (PASS == WQ_SQDIFF) {
             const float d = v - p.st.mean;
             acc[0] = acc[0] + (double)f32_mul(d, d);
         } else if constexpr (PASS == WQ_CLIP_STATS) {
-            const float x = wq_normalised(v, p);
-            acc[0] = acc[0] + (double)x;
-            acc[1] = acc[1] + (double)fabsf(x);
+            acc[0] = acc[0] + (double)v;
+            acc[1] = acc[1] + (double)fabsf(v);
         } else if constexpr (PASS == WQ_ABS_STATS) {
-            const float ax = fabsf(wq_processed(v, p));
+            const float ax = fabsf(wq_clipped(v, p));
             acc[0] = acc[0] + (double)ax;
             mx = fmaxf(mx, ax);
         } else if constexpr (PASS == WQ_OPTIMAL) {
-            const float x = wq_processed(v, p);
+            const float x = wq_clipped(v, p);
 #pragma unroll
             for (int f = 0; f < 10; ++f) {
                 const float d = x - wq_code(x, cand[f]);
                 acc[f] = acc[f] + (double)f32_mul(d, d);
             }
         } else {
-            const float x = wq_processed(v, p);
-            const float q = wq_code(x, p.st.thr);
-            acc[0] = acc[0] + (double)f32_mul(x, q);
-            nonzero += __popcll(__builtin_amdgcn_ballot_w64(q != 0.0f));  // sum of q * q: a count, exact in any order
+            const float q = scale_step(v);
+            c += first;
             if (packed) {  // k % 4 == 0: the four columns of a byte are active together
                 const int t = (int)q;
                 if (q_i8) q_i8[row * k + c] = (int8_t)t;

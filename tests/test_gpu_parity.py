@@ -134,6 +134,31 @@ def test_reference_weight_pipeline_bit_exact(method, normalize, t, custom):
             assert f32(got.stats[name]) == v, (name, got.stats[name], v)
 
 
+@pytest.mark.parametrize("n,k", [(9, 252), (9, 256), (9, 260), (5, 510), (9, 512), (5, 516), (9, 772), (9, 1284), (2113, 260)])
+@pytest.mark.parametrize("kind", ["plain", "constant", "zero_dividend", "far"])
+def test_reference_weight_pipeline_groups_of_columns(n, k, kind):
+    """Widths around the groups of columns that the passes take at once and rows around the batches of row sums; weights equal to the
+    mean (a zero dividend) and dividends out of the short division's range, which take the plain one.  Bit for bit, as above."""
+    rng = np.random.default_rng(n + k)
+    w = (0.3 + 1.7 * rng.standard_normal((n, k))).astype(f32)
+    if kind == "constant":
+        w[:] = f32(0.25)
+    elif kind == "zero_dividend":  # mean exactly 0: a tensor and its negative, with zeros
+        w[rng.random(w.shape) < 0.3] = 0
+        w[n // 2 * 2:] = 0
+        w[1:n // 2 * 2:2] = -w[0:n // 2 * 2:2]
+    elif kind == "far":
+        w[n // 2, k // 3] = f32(2.0) ** 64
+        w *= f32(2.0) ** -4
+    got = bh.BitNetWeightQuantizer().quantize(dev(w))
+    q_ref, s_ref, _, st_ref = orc.quantize_weights_reference(w, method=0, normalize=True, outlier_threshold=3.0, want_details=True)
+    assert np.array_equal(host(got.values), q_ref)
+    assert np.array_equal(host(got.packed), orc.pack_2bit(q_ref))
+    assert host(got.scales)[0] == s_ref
+    for name, v in st_ref.items():
+        assert f32(got.stats[name]) == v, (name, got.stats[name], v)
+
+
 def test_reference_weight_pipeline_through_the_layer():
     """BitLinear with the reference's default quantiser (MeanThreshold, normalise, clip 3.0: layer.rs:53-63): the layer then
     holds the oracle's codes and scale, and forward follows from them."""
