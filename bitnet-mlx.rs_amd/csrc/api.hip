@@ -568,6 +568,14 @@ int bitnet_hip_gemv_base3(const uint8_t *tiled, const int8_t *a, size_t n, size_
 int bitnet_hip_quantize_weights(const float *w, size_t n, size_t k, int method, float threshold_factor,
                                 uint8_t *packed, float *w_scale, int8_t *q_i8, void *stream)
 {
+    return bitnet_hip_quantize_weights_with(w, n, k, method, threshold_factor, packed, w_scale, q_i8, nullptr, 0, stream);
+}
+
+size_t bitnet_hip_quantize_weights_scratch(size_t n) { return sizeof(double) * n; }
+
+int bitnet_hip_quantize_weights_with(const float *w, size_t n, size_t k, int method, float threshold_factor, uint8_t *packed,
+                                     float *w_scale, int8_t *q_i8, void *row_scratch, size_t scratch_bytes, void *stream)
+{
     if (!w_scale) return fail(BITNET_HIP_NULL_POINTER, "quantize_weights: w_scale is required");
     if (n * k != 0 && (!w || !packed)) return fail(BITNET_HIP_NULL_POINTER, "quantize_weights: null buffer");
     if (method >= BITNET_HIP_TERNARY_REF_MEAN_THRESHOLD && method <= BITNET_HIP_TERNARY_REF_DETSTE)
@@ -576,16 +584,18 @@ int bitnet_hip_quantize_weights(const float *w, size_t n, size_t k, int method, 
                                                      threshold_factor, packed, w_scale, q_i8, nullptr, stream);
     if (method != BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP && method != BITNET_HIP_TERNARY_MEAN_THRESHOLD)
         return fail(BITNET_HIP_INVALID_CONFIG, "quantize_weights: unknown method %d", method);
-    // The row sums (8 bytes a row) are done with before the codes are written: they take the codes' place where a row has
-    // 8 bytes of them.
+    // The row sums (8 bytes a row): apart from the codes where the caller has room for them, which saves a launch.  If not they take the
+    // codes' place where a row has 8 bytes of them: they are done with before the codes are written.
     StreamScratch scratch;
     void *row_sums = packed;
-    if (k < 32 || (reinterpret_cast<uintptr_t>(packed) & 7) != 0) {
+    if (row_scratch && scratch_bytes >= sizeof(double) * n && (reinterpret_cast<uintptr_t>(row_scratch) & 7) == 0) {
+        row_sums = row_scratch;
+    } else if (k < 32 || (reinterpret_cast<uintptr_t>(packed) & 7) != 0) {
         int rc = scratch.alloc(sizeof(double) * (n ? n : 1), as_stream(stream));
         if (rc != BITNET_HIP_OK) return rc;
         row_sums = scratch.ptr;
     }
-    return launch_quantize_weights(w, n, k, method, threshold_factor, static_cast<double *>(row_sums), packed,
+    return launch_quantize_weights(w, n, k, method, threshold_factor, static_cast<double *>(row_sums), row_sums != packed, packed,
                                    w_scale, q_i8, as_stream(stream));
 }
 

@@ -56,9 +56,9 @@ int launch_lookup_compute(int kind, const int8_t *w, const float *x, float *out,
 int launch_pack_base3(const int8_t *q, size_t count, uint8_t *packed, hipStream_t stream);
 int launch_unpack_base3(const uint8_t *packed, size_t count, int8_t *q, hipStream_t stream);
 int launch_base3_to_2bit(const uint8_t *base3, size_t count, uint8_t *packed, hipStream_t stream);
-// row_sums: device scratch of n doubles
+// row_sums: device scratch of n doubles; apart: they are not where the codes go
 int launch_quantize_weights(const float *w, size_t n, size_t k, int method, float threshold_factor,
-                            double *row_sums, uint8_t *packed, float *w_scale, int8_t *q_i8,
+                            double *row_sums, bool apart, uint8_t *packed, float *w_scale, int8_t *q_i8,
                             hipStream_t stream);
 // BitNetWeightQuantizer::quantize (weights.rs:568-611): method = TernaryMethod 0..4, custom_factor <= 0 = none;
 // scratch: quantize_weights_reference_scratch_bytes(n) bytes of device memory; stats: 12 floats or null

@@ -233,6 +233,20 @@ __device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane)
     return __builtin_amdgcn_perm(y, x, lane & 2 ? 0x03020706u : 0x05040100u);
 }
 
+// Weights from base (a multiple of 4) up to end by one wavefront, a byte per lane and round.
+__device__ __forceinline__ void ternarize_bytes(const float *w, size_t base, size_t end, const TernaryRule &rule, uint8_t *packed, int8_t *q_i8, int lane)
+{
+    for (size_t e = base + 4 * lane; e < end; e += 256) {
+        unsigned byte = 0;
+        for (int j = 0; j < 4 && e + j < end; ++j) {
+            const int t = ternarize_one(w[e + j], rule);
+            if (q_i8) q_i8[e + j] = (int8_t)t;
+            byte |= (unsigned)(t + 1) << (2 * j);
+        }
+        packed[e / 4] = (uint8_t)byte;
+    }
+}
+
 // A wavefront takes 1024 consecutive weights: load i (of four) is one 16-byte chunk a lane, chunks in lane order, so loads
 // are dense; lane l keeps the dword of group i = l mod 4 of its quad and stores it: 256 bytes a wavefront.  Bound by the
 // read (6912 x 2560: 24 us as a thread per byte with four scalar loads and a division each, 10 us now).
@@ -260,19 +274,93 @@ __global__ __launch_bounds__(256) void ternarize_pack_kernel(const float *w, siz
         }
         *reinterpret_cast<uint32_t *>(packed + base / 4 + 64 * (lane & 3) + (lane & ~3)) = mine;
     }
-    // the end of the matrix, and buffers that are not aligned: a byte per lane and round
-    for (; base < count; base += (size_t)gridDim.x * 4096) {
-        const size_t end = base + 1024 < count ? base + 1024 : count;
-        for (size_t e = base + 4 * lane; e < end; e += 256) {
-            unsigned byte = 0;
-            for (int j = 0; j < 4 && e + j < end; ++j) {
-                const int t = ternarize_one(w[e + j], rule);
-                if (q_i8) q_i8[e + j] = (int8_t)t;
-                byte |= (unsigned)(t + 1) << (2 * j);
+    // the end of the matrix, and buffers that are not aligned
+    for (; base < count; base += (size_t)gridDim.x * 4096) ternarize_bytes(w, base, base + 1024 < count ? base + 1024 : count, rule, packed, q_i8, lane);
+}
+
+// absmean_final_kernel and ternarize_pack_kernel in one launch, for row sums that are not where the codes go: the first wavefront of every
+// workgroup adds the row sums up (lane l rows l, l+64, ..., then the butterfly, as there) while the first weights of the other 15 are on
+// their way.  These have CODES_HELD chunks of 1024 weights each in registers, which is a matrix of 79 MB; of a larger one the next chunk is
+// asked for where one has been used.  Bound by the read of the matrix, the second one.  A call, with the three launches -> with two:
+// 6912 x 2560 27.8 -> 24.9 us (the codes 9.5 behind 3.8 for the sum and a launch, 11.3 now), 4096 x 5120 30.6 -> 27.9, 14336 x 8192 176 -> 174,
+// 2048 x 2048 11.3 -> 9.1, 256 x 512 11.6 -> 9.3 (the host's launches).  With all wavefronts bringing the row sums into LDS ahead of their
+// weights 26.7; the whole quantiser in one launch whose workgroups wait for each other's row sums with the matrix in registers takes 22.1, but
+// two to four such launches on streams of their own keep each other off the compute units: 48 us a call in place of 23.
+constexpr int CODES_HELD = 5, CODES_SUMS = 36;  // chunks and rows of 64 row sums on their way to a wavefront
+constexpr size_t CODES_MAX_ROWS = 65536;        // beyond, every workgroup reading all row sums is what takes the time
+
+// The codes of 1024 consecutive weights, a float4 of each 256 a lane: lane l of a quad ends with the dword of the quad's group l, as above.
+__device__ __forceinline__ void codes_of_chunk(const float4 (&v)[4], float t, uint8_t *packed, size_t chunk, int lane)
+{
+    // A code is 1 where |w| < t, which is the sign of |w| - t, else 0 or 2 by the sign of w: both signs are shifted in, and put right for 16 at a time.
+    uint32_t x = 0;
+    const auto take = [&](float w) {
+        x = __builtin_amdgcn_alignbit(x, __builtin_bit_cast(uint32_t, w), 31);
+        x = __builtin_amdgcn_alignbit(x, __builtin_bit_cast(uint32_t, fabsf(w) - t), 31);
+    };
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        take(v[i].w);
+        take(v[i].z);
+        take(v[i].y);
+        take(v[i].x);
+    }
+    x = t == t ? (x & 0x55555555u) | (~(x | (x << 1)) & 0xaaaaaaaau) : 0x55555555u;
+    *reinterpret_cast<uint32_t *>(packed + chunk * 256 + 64 * (lane & 3) + (lane & ~3)) = quad_transpose(x, lane);
+}
+
+__global__ __launch_bounds__(1024) void absmean_codes_kernel(const float *w, size_t n, size_t k, int method, float factor,
+                                                             const double *row_sums, uint8_t *packed, float *w_scale)
+{
+    __shared__ float scale_s;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t chunks = n * k / 1024, stride = (size_t)gridDim.x * 15;
+    size_t first = (size_t)(wave - 1) * gridDim.x + blockIdx.x;  // as many for every workgroup
+    float4 v[CODES_HELD][4];
+    const auto load = [&](float4 (&to)[4], size_t chunk) {  // zeros past the last one: no branch, so that each chunk is waited for by itself
+        const __amdgpu_buffer_rsrc_t of = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(w + chunk * 1024), 0, chunk < chunks ? 4096 : 0, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) to[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(of, 16 * lane + 1024 * i, 0, 0));
+    };
+    if (wave == 0) {
+        // Zeros past the last row (a sum of absolute values stays what it is), and CODES_SUMS rows of 64 always on their way.
+        const __amdgpu_buffer_rsrc_t sums = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(row_sums), 0, (int)(8 * n), 0x00020000);
+        const auto sum = [&](int row) { return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(sums, 8 * row, 0, 0)); };
+        double total = 0.0, r[CODES_SUMS];
+#pragma unroll
+        for (int i = 0; i < CODES_SUMS; ++i) r[i] = sum(lane + 64 * i);
+        for (int row = lane; row - lane < (int)n; row += 64 * CODES_SUMS) {
+#pragma unroll
+            for (int i = 0; i < CODES_SUMS; ++i) {
+                total = total + r[i];
+                r[i] = sum(row + 64 * (CODES_SUMS + i));
             }
-            packed[e / 4] = (uint8_t)byte;
+        }
+        total = wave_sum_f64(total);
+        if (lane == 0) scale_s = (float)(total / ((double)n * (double)k));
+        first = chunks;
+    } else {
+#pragma unroll
+        for (int h = 0; h < CODES_HELD; ++h) load(v[h], first + h * stride);
+    }
+    __syncthreads();
+    const float scale = scale_s;
+    if (blockIdx.x == 0 && tid == 0) *w_scale = scale;
+    // t > 0, or NaN (every code 0): w > hi, for hi >= 0, is w >= the next float up.
+    const TernaryRule rule = ternary_rule(method, factor, scale);
+    const float t = rule.strict ? __builtin_bit_cast(float, __builtin_bit_cast(int, fabsf(rule.hi)) + 1) : rule.hi;
+    size_t chunk = first;
+    for (; chunk + CODES_HELD * stride < chunks; chunk += CODES_HELD * stride) {
+#pragma unroll
+        for (int h = 0; h < CODES_HELD; ++h) {
+            codes_of_chunk(v[h], t, packed, chunk + h * stride, lane);
+            load(v[h], chunk + (h + CODES_HELD) * stride);
         }
     }
+#pragma unroll
+    for (int h = 0; h < CODES_HELD; ++h)
+        if (chunk + h * stride < chunks) codes_of_chunk(v[h], t, packed, chunk + h * stride, lane);
+    if (blockIdx.x == gridDim.x - 1 && wave == 15) ternarize_bytes(w, chunks * 1024, n * k, rule, packed, nullptr, lane);
 }
 
 // ---- BitNetWeightQuantizer::quantize, the reference's weight pipeline (bitnet-quant/src/quantization/weights.rs:568-611)
@@ -831,17 +919,25 @@ int launch_base3_to_2bit(const uint8_t *base3, size_t count, uint8_t *packed, hi
 }
 
 int launch_quantize_weights(const float *w, size_t n, size_t k, int method, float threshold_factor,
-                            double *row_sums, uint8_t *packed, float *w_scale, int8_t *q_i8, hipStream_t stream)
+                            double *row_sums, bool apart, uint8_t *packed, float *w_scale, int8_t *q_i8, hipStream_t stream)
 {
-    if (n > 0 && k > 0) {
+    const size_t count = n * k;
+    if (count != 0) {
         launch_kernel(absmean_rows_kernel, dim3(blocks_for(n, 4)), dim3(64, 4), 0, stream, w, n, k, row_sums);
         BITNET_HIP_CHECK_LAUNCH("absmean_rows_kernel");
     }
+    const bool dense = aligned(w, 16) && aligned(packed, 4) && (!q_i8 || aligned(q_i8, 4));
+    // No int8 codes, and a threshold that is not negative (what the sign of a difference can tell).
+    if (apart && count != 0 && n <= CODES_MAX_ROWS && dense && !q_i8 && (method == BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP || threshold_factor >= 0.0f)) {
+        const unsigned blocks = blocks_for(count, 2048);  // two wavefronts with a chunk each, up to a workgroup a compute unit
+        launch_kernel(absmean_codes_kernel, dim3(blocks < 256 ? blocks : 256), dim3(1024), 0, stream, w, n, k, method, threshold_factor,
+                      const_cast<const double *>(row_sums), packed, w_scale);
+        BITNET_HIP_CHECK_LAUNCH("absmean_codes_kernel");
+        return BITNET_HIP_OK;
+    }
     launch_kernel(absmean_final_kernel, dim3(1), dim3(1024), 0, stream, row_sums, n, k, w_scale);
     BITNET_HIP_CHECK_LAUNCH("absmean_final_kernel");
-    const size_t count = n * k;
     if (count == 0) return BITNET_HIP_OK;
-    const bool dense = aligned(w, 16) && aligned(packed, 4) && (!q_i8 || aligned(q_i8, 4));
     // at most eight workgroups a compute unit: one round, and no more dispatches than that
     const unsigned blocks = blocks_for(count, 4096);
     launch_kernel(ternarize_pack_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, stream, w, count,

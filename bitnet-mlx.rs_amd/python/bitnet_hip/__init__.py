@@ -110,6 +110,8 @@ def load_library() -> C.CDLL:
         "bitnet_hip_base3_tiled_size": (sz, [sz, sz]),
         "bitnet_hip_retile_base3": (i32, [vp, sz, sz, vp, vp]),
         "bitnet_hip_gemv_base3": (i32, [vp, vp, sz, sz, vp, vp, vp, vp, vp]),
+        "bitnet_hip_quantize_weights_with": (i32, [vp, sz, sz, i32, f32, vp, vp, vp, vp, sz, vp]),
+        "bitnet_hip_quantize_weights_scratch": (sz, [sz]),
         "bitnet_hip_quantize_weights": (i32, [vp, sz, sz, i32, f32, vp, vp, vp, vp]),
         "bitnet_hip_quantize_weights_reference": (i32, [vp, sz, sz, i32, i32, f32, f32, vp, vp, vp, vp, vp]),
         "bitnet_hip_tiled_size": (sz, [sz, sz]),
@@ -714,8 +716,9 @@ def quantize_weights(w: torch.Tensor, method: int = TERNARY_ABSMEAN_ROUNDCLIP, t
     packed = _empty((packed_size(n * k),), torch.uint8, w.device, stream)
     w_scale = _empty((1,), torch.float32, w.device, stream)
     q = _empty((n, k), torch.int8, w.device, stream) if want_i8 else None
-    _check(load_library().bitnet_hip_quantize_weights(_ptr(w), n, k, method, threshold_factor, _ptr(packed),
-                                                      _ptr(w_scale), _ptr(q), _stream(stream)))
+    scratch = None if want_i8 else _empty((n,), torch.float64, w.device, stream)  # the row sums, apart from the codes
+    _check(load_library().bitnet_hip_quantize_weights_with(_ptr(w), n, k, method, threshold_factor, _ptr(packed), _ptr(w_scale),
+                                                           _ptr(q), _ptr(scratch), 0 if scratch is None else 8 * n, _stream(stream)))
     _finish(stream, w.device)
     return packed, w_scale, q
 

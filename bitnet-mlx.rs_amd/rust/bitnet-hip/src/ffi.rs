@@ -94,6 +94,10 @@ extern "C" {
                                  a_scale: *const f32, acc: *mut i32, out: *mut f32, stream: *mut c_void) -> c_int;
     pub fn bitnet_hip_quantize_weights(w: *const f32, n: usize, k: usize, method: c_int, threshold_factor: f32,
                                        packed: *mut u8, w_scale: *mut f32, q_i8: *mut i8, stream: *mut c_void) -> c_int;
+    pub fn bitnet_hip_quantize_weights_scratch(n: usize) -> usize;
+    pub fn bitnet_hip_quantize_weights_with(w: *const f32, n: usize, k: usize, method: c_int, threshold_factor: f32,
+                                            packed: *mut u8, w_scale: *mut f32, q_i8: *mut i8, scratch: *mut c_void,
+                                            scratch_bytes: usize, stream: *mut c_void) -> c_int;
     pub fn bitnet_hip_quantize_weights_reference(w: *const f32, n: usize, k: usize, ternary_method: c_int,
                                                  normalize_weights: c_int, outlier_threshold: f32,
                                                  custom_threshold_factor: f32, packed: *mut u8, w_scale: *mut f32,

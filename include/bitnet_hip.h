@@ -233,6 +233,11 @@ int bitnet_hip_gemv_base3(const uint8_t *tiled, const int8_t *a, size_t n, size_
  *   packed   [(n*k+3)/4] u8 out;  w_scale  1 f32 out (device);  q_i8 [n*k] int8 out or NULL. */
 int bitnet_hip_quantize_weights(const float *w, size_t n, size_t k, int method, float threshold_factor,
                                 uint8_t *packed, float *w_scale, int8_t *q_i8, void *stream);
+/* The same with DEVICE scratch of the caller's for the row sums (quantize_weights_scratch(n) bytes, 8-byte aligned; NULL or fewer: as without),
+ * in use until the call's work on the stream is done: two launches in place of three.  Same results. */
+size_t bitnet_hip_quantize_weights_scratch(size_t n);
+int bitnet_hip_quantize_weights_with(const float *w, size_t n, size_t k, int method, float threshold_factor, uint8_t *packed,
+                                     float *w_scale, int8_t *q_i8, void *scratch, size_t scratch_bytes, void *stream);
 
 /* The reference's weight pipeline with its whole configuration, on the GPU:
  *   replaces BitNetWeightQuantizer::quantize (bitnet-quant/src/quantization/weights.rs:568-611):

@@ -94,6 +94,33 @@ def test_quantize_weights_absmean_bit_exact(n, k):
     assert np.array_equal(host(packed), orc.pack_2bit(q_ref))
 
 
+@pytest.mark.parametrize("n,k", [(1, 4), (3, 127), (16, 64), (33, 1023), (64, 1024), (65, 1028), (2304, 65), (2305, 260), (4099, 4092), (6912, 3072)])
+@pytest.mark.parametrize("method,factor", [(0, 0.5), (1, 0.7), (1, 0.0), (1, -0.25), (1, float("inf"))])
+def test_quantize_weights_with_row_scratch_bit_exact(n, k, method, factor):
+    """Row sums of the caller's, apart from the codes (the sum and the codes in one launch), against those in the codes' place: sizes around a
+    chunk of 1024 weights, around 36 x 64 row sums, and with more chunks than the registers hold; with too little scratch the call is the other one."""
+    lib = bh.load_library()
+    rng = np.random.default_rng(n + k)
+    w = dev(synth_weights(rng, n, k))
+    w.view(-1)[::7] = 0.0
+    need = lib.bitnet_hip_quantize_weights_scratch(n)
+    results = []
+    for room in (need, need - 8, None):
+        packed, scale = torch.full(((n * k + 3) // 4,), 0xAA, dtype=torch.uint8, device="cuda"), torch.zeros(1, device="cuda")
+        scratch = torch.full((need // 8,), float("nan"), dtype=torch.float64, device="cuda")
+        args = (w.data_ptr(), n, k, method, factor, packed.data_ptr(), scale.data_ptr(), None)
+        stream = torch.cuda.current_stream().cuda_stream
+        rc = (lib.bitnet_hip_quantize_weights(*args, stream) if room is None else
+              lib.bitnet_hip_quantize_weights_with(*args, scratch.data_ptr(), room, stream))
+        assert rc == 0
+        results.append((host(packed), host(scale)))
+    for packed, scale in results[1:]:
+        assert np.array_equal(results[0][0], packed) and results[0][1] == scale
+    if method == 0 and n * k < 1 << 20:
+        q_ref, s_ref = orc.quantize_weights_absmean(host(w))
+        assert results[0][1][0] == s_ref and np.array_equal(results[0][0], orc.pack_2bit(q_ref))
+
+
 def test_quantize_weights_reference_vectors():
     c = G["quantize_batch"]
     w = np.array([c["input"]], dtype=f32)
