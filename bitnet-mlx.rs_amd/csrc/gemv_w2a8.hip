@@ -29,6 +29,8 @@
 // gemv_fused16_kernel is this launch with up to 16 wavefronts per workgroup (the default for one token; see its comment): there the
 // row reaches the MFMA by lane broadcasts, and the tiles are requested behind it.
 //
+// gemv_stream.hip is the same for launches of more row blocks than one round of workgroups takes, on rows above 4096 columns.
+//
 // gemv_rows_kernel serves several tokens whose rows the quantiser laid out for it.  gemv_mfma_kernel is the same
 // weight-streaming scheme for 2..16 row-major token rows, which a caller brings or wants to see: the 16 x 16 x 64 int8 MFMA takes
 // the place of the dot-product chain (its A operand is 16 token rows x 64 columns, loaded straight from the
@@ -452,33 +454,6 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(GemvParams p)
 // A block of the 30-block stack (2560 / 6912), replayed, at one token: 16.5 us before these points, 14.8 with them; at four tokens
 // 23.9 and 22.3.
 
-// The arguments behind the preloaded ones, in blocks of 64 bytes: each is one scalar load.
-struct Fused16Params {
-    int kt_count;
-    float eps;
-    uint64_t reserved;
-    int8_t *q_out;  // optional copies of what the prologue produced (written by the first group of row blocks)
-    float *a_scale_out;
-    int32_t *a_sum_out;
-    uint64_t unused[3];
-    Fused16Proj proj[GEMV_MAX_PROJ];
-};
-static_assert(sizeof(Fused16Params) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
-constexpr int FUSED16_ARGS_AT = 48;  // offset of the Fused16Params in the argument buffer: three pointers and six ints before it
-
-// The value of a lane of the own 16 lanes (a constant once unrolled): a row broadcast, 0x150 + lane.
-template <int LANE>
-__device__ __forceinline__ int row_lane_at(int v) { return dpp_i32<0x150 + LANE>(v); }
-__device__ __forceinline__ int row_lane(uint32_t packed, int at)
-{
-    const int v = (int)packed;
-    switch (at) {
-        case 0: return row_lane_at<0>(v); case 1: return row_lane_at<1>(v); case 2: return row_lane_at<2>(v); case 3: return row_lane_at<3>(v);
-        case 4: return row_lane_at<4>(v); case 5: return row_lane_at<5>(v); case 6: return row_lane_at<6>(v); case 7: return row_lane_at<7>(v);
-        case 8: return row_lane_at<8>(v); case 9: return row_lane_at<9>(v); case 10: return row_lane_at<10>(v); case 11: return row_lane_at<11>(v);
-        case 12: return row_lane_at<12>(v); case 13: return row_lane_at<13>(v); case 14: return row_lane_at<14>(v); default: return row_lane_at<15>(v);
-    }
-}
 template <int MODE, bool NORM, int NCHB, int RBW>
 __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, const float *hot_x2, const float *hot_gamma, int hot_k, int hot_head_chunks,
                                                            int hot_nw, int hot_ldx, int hot_end0, int hot_end1, [[maybe_unused]] Fused16Params args)
@@ -1639,12 +1614,12 @@ bool gemv_fused_supported(const float *x, const float *x2, size_t ldx, size_t m,
         if ((blocks + rbw - 1) / rbw * m > (size_t)GEMV_FUSED_MAX_WGS) return false;
     }
     // Rows above FUSED_NCH * 1024 columns: only where one round of workgroups serves the launch (each quantises its whole row for
-    // itself), and in the declared summation order; above 8192 columns (four chunks per thread) without a norm, whose registers do
+    // itself; one token's may walk several row blocks), and in the declared summation order; above 8192 columns (four chunks per thread) without a norm, whose registers do
     // not fit beside the tiles.  A decoder block with 2560-wide rows, in two launches -> here: 8192-wide FFN at 1 / 2 / 3 tokens
     // 20.3 / 21.5 / 23.4 -> 16.6 / 19.5 / 21.4 us, 13824-wide at 1 / 2 / 3 / 4 tokens 29.4 / 32.8 / 33.2 / 33.9 -> 20.2 / 25.1 /
     // 25.6 / 29.0 (of which the stand-alone quantiser's four chunks per thread give up to 5).
     if (k > (size_t)FUSED_NCH * 1024) {
-        if ((m == 1 && blocks > 256) || k > 16384 || ldx >= ((size_t)1 << 31)) return false;
+        if ((m == 1 && blocks > 256 && !gemv_stream_takes(m, k, gamma, sum_order, blocks)) || k > 16384 || ldx >= ((size_t)1 << 31)) return false;
         if (gamma != nullptr && (sum_order != BITNET_HIP_SUM_BLOCK256 || k > 8192)) return false;
     }
     if (k % 4 != 0 || ldx % 4 != 0) return false;
@@ -1667,13 +1642,15 @@ int launch_gemv_fused(const GemvProj *projs, int nproj, const float *x, const fl
         // row blocks per workgroup: one round of workgroups on the 256 compute units where the row is short enough for
         // a wavefront to hold the tiles of several row blocks (one token, gate alone, 432 row blocks: 4.50 us with one
         // row block per workgroup, 3.82 us with two)
-        const int rbw16 = fused16_row_blocks_per_workgroup(m, k, blocks);
+        const bool streams = gemv_stream_takes(m, k, gamma, sum_order, blocks);
+        const int rbw16 = streams ? 1 : fused16_row_blocks_per_workgroup(m, k, blocks);
         Fused16Params p = {};
         if (fill_projs(p, projs, nproj, 0, k, rbw16) == 0) return BITNET_HIP_OK;
         RowSource src = {};
         src.x = x; src.x2 = x2; src.gamma = gamma; src.ldx = ldx; src.k = (int)k;
         src.head_dim = (int)(head_dim ? head_dim : 1); src.gqa_group = (int)(gqa_group ? gqa_group : 1);
         p.eps = eps; p.q_out = q_out; p.a_scale_out = a_scale_out; p.a_sum_out = a_sum_out;
+        if (streams) return launch_gemv_stream(p, nproj, src, input_mode, blocks, stream);
 #define BITNET_F16_MODES(RBW) \
     switch (input_mode) { \
         case BITNET_HIP_INPUT_PLAIN: return launch_fused16_mode<BITNET_HIP_INPUT_PLAIN, RBW>(p, nproj, src, (int)m, stream); \

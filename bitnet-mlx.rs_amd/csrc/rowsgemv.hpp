@@ -1,4 +1,4 @@
-// What the token GEMVs on interleaved rows (ActRows::TILES16) share: the products of one wavefront, and the finish of a workgroup, where
+// What the GEMVs that quantise their one row share (Fused16Params, row_lane), and what the token GEMVs on interleaved rows (ActRows::TILES16) share: the products of one wavefront, and the finish of a workgroup, where
 // the wavefronts' partial results meet in LDS and wavefront r stores row block r, four outputs a lane.  gemv_rows_kernel takes rows
 // that a launch before it wrote; gemv_die_kernel has them quantised by the workgroups of its own die.
 #pragma once
@@ -25,6 +25,38 @@ struct Fused16Proj {
     uint64_t unused;
 };
 static_assert(sizeof(Fused16Proj) == 64, "one scalar load a block");
+
+// The arguments behind the preloaded ones, in blocks of 64 bytes: each is one scalar load.
+struct Fused16Params {
+    int kt_count;
+    float eps;
+    uint64_t reserved;
+    int8_t *q_out;  // optional copies of what the prologue produced (written by the first group of row blocks)
+    float *a_scale_out;
+    int32_t *a_sum_out;
+    uint64_t unused[3];
+    Fused16Proj proj[GEMV_MAX_PROJ];
+};
+static_assert(sizeof(Fused16Params) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
+constexpr int FUSED16_ARGS_AT = 48;  // offset of the Fused16Params in the argument buffer: three pointers and six ints before it
+
+// One token through more row blocks than one round of workgroups takes (gemv_stream.hip); p: projections with a row block each.
+bool gemv_stream_takes(size_t m, size_t k, const float *gamma, int sum_order, size_t blocks);
+int launch_gemv_stream(const Fused16Params &p, int nproj, const RowSource &src, int input_mode, size_t blocks, hipStream_t stream);
+
+// The value of a lane of the own 16 lanes (a constant once unrolled): a row broadcast, 0x150 + lane.
+template <int LANE>
+__device__ __forceinline__ int row_lane_at(int v) { return dpp_i32<0x150 + LANE>(v); }
+__device__ __forceinline__ int row_lane(uint32_t packed, int at)
+{
+    const int v = (int)packed;
+    switch (at) {
+        case 0: return row_lane_at<0>(v); case 1: return row_lane_at<1>(v); case 2: return row_lane_at<2>(v); case 3: return row_lane_at<3>(v);
+        case 4: return row_lane_at<4>(v); case 5: return row_lane_at<5>(v); case 6: return row_lane_at<6>(v); case 7: return row_lane_at<7>(v);
+        case 8: return row_lane_at<8>(v); case 9: return row_lane_at<9>(v); case 10: return row_lane_at<10>(v); case 11: return row_lane_at<11>(v);
+        case 12: return row_lane_at<12>(v); case 13: return row_lane_at<13>(v); case 14: return row_lane_at<14>(v); default: return row_lane_at<15>(v);
+    }
+}
 
 // The A operands of the k-tiles kt0, kt0 + nw, ...: lane 16 g + r takes row r, columns 16 g .. + 15 of a tile; lanes without a row load
 // nothing (the results of their row are not used).  group_rows: the first byte of the token group.

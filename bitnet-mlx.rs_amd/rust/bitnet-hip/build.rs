@@ -5,7 +5,7 @@ use std::path::PathBuf;
 use std::process::Command;
 
 const KERNELS: &[&str] =
-    &["api.hip", "act_quant.hip", "weight_prep.hip", "gemv_w2a8.hip", "gemv_rowq.hip", "gemv_die.hip", "gemm_w2a8.hip", "gemv_base3.hip", "staging.hip",
+    &["api.hip", "act_quant.hip", "weight_prep.hip", "gemv_w2a8.hip", "gemv_rowq.hip", "gemv_die.hip", "gemv_stream.hip", "gemm_w2a8.hip", "gemv_base3.hip", "staging.hip",
       "diag.hip"];
 
 fn main() {

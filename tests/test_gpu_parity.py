@@ -2038,6 +2038,49 @@ def test_rows_quantised_once_a_die_bit_exact(m, k, n, norm):
     assert np.array_equal(host(layer.forward(dev(xs), gamma=g, residual=dev(res), workspace=least)), want)
 
 
+@pytest.mark.parametrize("k,n,norm", [(4100, 4097, True), (4100, 8193, False), (4356, 8201, True), (7168, 12304, False), (7172, 4100, False), (8192, 4129, True),
+                                      (8196, 4112, False), (12288, 8225, False), (16384, 4111, False), (8452, 16401, False), (5120, 20500, True)])
+def test_one_token_through_many_row_blocks(k, n, norm):
+    """Rows of 17 to 64 k-tiles, a few columns past a tile, workgroups with one row block more than others, fewer and more of them than are in
+    flight, last row blocks of 1 to 15 rows, the optional outputs, and two projections that share the row."""
+    rng = np.random.default_rng(k + 3 * n)
+    x = synth_activations(rng, 1, k, outliers=True)
+    g = (1 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    gd = dev(g) if norm else None
+    pk = random_packed_ternary(rng, 1, (n * k + 3) // 4 * 4)
+    bias, res = rng.standard_normal(n, dtype=f32), rng.standard_normal((1, n), dtype=f32)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n, use_bias=True), "many")
+    layer.set_quantized_weights(torch.from_numpy(pk), 0.02)
+    layer.update_bias(dev(bias))
+    ref, q_ref, s_ref, acc_ref = orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias, residual=res)
+    for _ in range(2):
+        assert np.array_equal(host(layer.forward(dev(x), gamma=gd, residual=dev(res))), ref)
+    out, q, a_scale, acc = layer.forward(dev(x), gamma=gd, residual=dev(res), debug=True)
+    assert np.array_equal(host(out), ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(a_scale), s_ref) and np.array_equal(host(acc), acc_ref)
+    other = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=24), "beside")
+    pk2 = random_packed_ternary(rng, 24, k)
+    other.set_quantized_weights(torch.from_numpy(pk2), 0.03)
+    for order in ([other, layer], [layer, other], [other, layer, other]):
+        for one, y in zip(order, bh.forward_multi(order, dev(x), gamma=gd)):
+            want = orc.bitlinear_forward(x, pk2, 24, f32(0.03), g=g)[0] if one is other else orc.bitlinear_forward(x, pk, n, f32(0.02), g=g, bias=bias)[0]
+            assert np.array_equal(host(y), want)
+
+
+@pytest.mark.parametrize("dims", [(4352, 8448, 34, 2, 128), (8320, 512, 65, 5, 128)])
+def test_decoder_blocks_of_many_row_blocks(dims):
+    """One token through wide blocks, as it comes and recorded: gate and up, the relu2-gated down projection, and repeated heads."""
+    rng = np.random.default_rng(sum(dims))
+    dec, ref = build_decoder_packed(rng, 1, *dims, max_tokens=1)
+    x = synth_activations(rng, 1, dims[0])
+    want = oracle_stack(ref, x, *dims)[0]
+    assert np.array_equal(host(dec.decode(dev(x))), want)
+    graph = dec.record(dev(x))
+    for _ in range(3):
+        graph.out.zero_()
+        graph.replay()
+        assert np.array_equal(host(graph.out), want)
+
+
 @pytest.mark.parametrize("dims,layers", [((512, 1408, 8, 2, 64), 3), ((2560, 6912, 20, 5, 128), 1)])
 def test_decoder_rows_quantised_once_a_die(dims, layers):
     """Steps of several token counts, one after the other and recorded, with workgroups that wait for their rows and (no looks at all)
