@@ -1451,7 +1451,7 @@ private:
 }  // namespace
 
 // The recorded form of a step, or null where it is to be enqueued launch by launch.  A launch costs the host 2.3 to 4.5 us and
-// a block is four to eight of them, which the GPU runs in 12 to 25 us where the model is small or the step one token: the
+// a block is four to six of them, which the GPU runs in 12 to 25 us where the model is small or the step one token: the
 // host was the slower side.  A graph costs it 13 us whatever it holds (120 launches of a 30-block step: 15 us).  Recording
 // costs about a millisecond, so only a step that has come twice before is recorded, and, once STEP_GRAPHS have been, no
 // more than one for every 64 replays: a program whose tensors never lie where they lay before does not pay for it.

@@ -1159,9 +1159,10 @@ __global__ __launch_bounds__(256) void gemv_mfma_tg_kernel(const int8_t *hot_a, 
 // leave the wavefront subtracted; the partial results of the wavefronts meet in LDS, and wavefront r finishes row block r, four
 // outputs a lane.  What a launch takes is one trip to memory, the MFMAs of a wavefront and that exchange, and, with more than one
 // workgroup a compute unit, the issue of vector instructions: 10 wavefronts of some 400 hold the four SIMDs for 2 us.  6912 -> 2560, 16
-// tokens: 4.1 us (gathering the rows from memory 7.6); a block of the 30-block stack: 24.8 us at 8 tokens, 29.2 at 24, 33.1 at 42 (with
-// a thread per output, which took a third more instructions and, with four row blocks, 80 registers, so that a compute unit held
-// two workgroups instead of three: 24.9, 30.6 and 35.0; rows copied to LDS first 30.0 at 8 and 50.2 at 42).
+// tokens: 4.1 us (gathering the rows from memory 7.6).  A block of the 30-block stack with this kernel for qkv, gate + up and down: 24.8 us at 8
+// tokens, 29.2 at 24, 33.1 at 42 (with a thread per output, which took a third more instructions and, with four row blocks, 80 registers, so that
+// a compute unit held two workgroups instead of three: 24.9, 30.6 and 35.0; rows copied to LDS first 30.0 at 8 and 50.2 at 42; with
+// gemv_die_kernel where that takes the launch, as now: 21.3, 26.3 and 31.5).
 // Everything that the loads need arrives preloaded, the weights' addresses too: a scalar load of an argument takes as long as
 // the weights do, and the two would add up (2560 columns, 160 row blocks: 0.55 us of 3.4).  Counts of row blocks and their
 // groups are packed, 16 bits each: rows and k-tiles; groups of projection 0, and of 0 and 1 (0xffff where there is no next

@@ -392,7 +392,8 @@ size_t bitnet_hip_bitlinear_forward_multi_scratch(bitnet_hip_bitlinear *const *l
                                                   const float *gamma, int sum_order);
 /* Bytes of workspace with which a forward (count = 1) or forward_multi call on `stream` is fastest: as the two functions above say,
  * and workspace_size(m) as well where the stream is being captured and a replay is faster with the quantiser as a launch of its
- * own.  A captured call that gets less is one launch, as it is outside a capture. */
+ * own.  A captured call that gets less is one launch, as it is outside a capture.  Outside a capture also room, beyond workspace_size(m), for
+ * the flags of 2 to 128 rows that are quantised inside the launch, once on every die; a call that gets less is two launches. */
 size_t bitnet_hip_bitlinear_forward_scratch_on(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
                                                const float *gamma, int sum_order, void *stream);
 
