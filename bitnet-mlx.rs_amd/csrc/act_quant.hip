@@ -79,12 +79,33 @@ __device__ __forceinline__ void clear_pad(const ActQuantParams &p, const RowPlac
     if (4 * (size_t)c < p.ldq) *reinterpret_cast<uint32_t *>(p.q + place.chunk(c)) = 0u;
 }
 
-// One wavefront per row of at most 1024 columns: four chunks a lane, no barriers.  (A workgroup per row leaves most of its
-// threads without a chunk there.)
-template <int MODE, bool VEC>
+// The chunks of a thread (first, first + step, ...; zeros from `chunks` on) normalised together: one look at their range in place of one a chunk.
+template <int NCH>
+__device__ __forceinline__ void normalize_row(float4 (&v)[NCH], const float4 (&gm)[NCH], const Divisor &r, int first, int step, int chunks)
+{
+    bool ok = r.fast;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) ok = ok && (first + step * i >= chunks || chunk_ok(v[i]));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!ok) == 0, 1)) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i)  // no zeros but the padding's
+            v[i] = make_float4(f32_mul(div_by_invariant_unchecked<false>(v[i].x, r.d, r.recip), gm[i].x),
+                               f32_mul(div_by_invariant_unchecked<false>(v[i].y, r.d, r.recip), gm[i].y),
+                               f32_mul(div_by_invariant_unchecked<false>(v[i].z, r.d, r.recip), gm[i].z),
+                               f32_mul(div_by_invariant_unchecked<false>(v[i].w, r.d, r.recip), gm[i].w));
+    } else {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i)
+            if (first + step * i < chunks) v[i] = normalize4(v[i], r, gm[i]);
+    }
+}
+
+// One wavefront per row of at most 256 NCH columns: NCH (two or four) chunks a lane, no barriers.  (A workgroup per row leaves most of its
+// threads without a chunk there.)  With a norm, as below: 65536 x 1024 67.8 -> 59.9 us, 16384 x 1024 18.5 -> 16.0; two chunks where they do: 65536 x 512
+// 33.1 -> 29.1 (36.3 with four).
+template <int MODE, bool VEC, bool NORM, int NCH>
 __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 {
-    constexpr int NCH = 4;
     const RowSource &src = p.src;
     const int lane = threadIdx.x;
     const size_t row = (size_t)blockIdx.x * blockDim.y + threadIdx.y;
@@ -97,21 +118,21 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
         int c = lane + 64 * i;
         v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (src.gamma) {
+    if constexpr (NORM) {
+        float4 gm[NCH];
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) gm[i] = lane + 64 * i < chunks ? load_gamma_chunk(src, lane + 64 * i, VEC) : make_float4(0.f, 0.f, 0.f, 0.f);
         float ss;
         if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
             ss = sum_squares_sequential<MODE>(src, row);
         } else {
             // chunk lane + 64*i belongs to virtual lane lane + 64*i: four partials per lane
-            float part[NCH];
+            float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int i = 0; i < NCH; ++i) part[i] = wave_sum_f32(sum_squares4(0.0f, v[i]));
             ss = f32_add(f32_add(f32_add(part[0], part[1]), part[2]), part[3]);
         }
-        const Divisor rdiv = make_divisor(rms_from_ss(ss, src.k, src.eps));
-#pragma unroll
-        for (int i = 0; i < NCH; ++i)
-            if (lane + 64 * i < chunks) v[i] = normalize4(v[i], rdiv, load_gamma_chunk(src, lane + 64 * i, VEC));
+        normalize_row(v, gm, make_divisor(rms_from_ss(ss, src.k, src.eps)), lane, 64, chunks);
     }
     float amax = 0.0f;
 #pragma unroll
@@ -136,7 +157,10 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 // A workgroup per row; NCH chunks per thread in registers (K <= 1024*NCH), NCH == 0: re-read.  A row is three dependent steps
 // with barriers between them: the loads of one workgroup overlap the arithmetic of the others on the compute unit.  (1024
 // workgroups that take rows in turn and fetch the next one early are slower: 15.8 us against 12.7 us at 2048 x 6912.)
-template <int MODE, int NCH, bool VEC>
+// HELD_NORM: a norm in the declared order, whose weights are asked for with the row and not behind its sum of squares, and whose chunks are divided
+// together; NCH is then exactly what a row takes, since every chunk's weights take registers too.  With a norm, before -> now (without one), us:
+// 4096 x 5120 21.6 -> 17.9 (17.0), 4096 x 4096 18.5 -> 15.2 (14.0), 8192 x 2560 20.3 -> 18.6 (16.4), 2048 x 6912 16.7 -> 15.2 (12.5).
+template <int MODE, int NCH, bool VEC, bool HELD_NORM>
 __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
 {
     __shared__ float red_f[2][4];
@@ -158,15 +182,23 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
             v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : zero4;
         }
     }
+    float4 gm[HELD_NORM ? NCH : 1];
+    if constexpr (HELD_NORM) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int c = tid + 256 * i;
+            gm[i] = c < chunks ? load_gamma_chunk(src, c, VEC) : zero4;
+        }
+    }
     auto chunk_at = [&](int i, int c) -> float4 {
         if constexpr (NCH > 0) return v[i];
         else return c < chunks ? load_chunk<MODE, VEC>(src, row, c) : zero4;
     };
 
     Divisor rdiv = {1.0f, 1.0f, false};
-    if (norm) {
+    if (HELD_NORM || norm) {
         float ss;
-        if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
+        if (!HELD_NORM && src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
             if (p.seq_in_lds) {
                 extern __shared__ float sq_lds[];  // squares_lds_bytes(k)
 #pragma unroll
@@ -192,11 +224,12 @@ __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
     }
 
     float amax = 0.0f;
+    if constexpr (HELD_NORM) normalize_row(v, gm, rdiv, tid, 256, chunks);
 #pragma unroll
     for (int i = 0; i < nloop; ++i) {
         int c = tid + 256 * i;
         float4 e = chunk_at(i, c);
-        if (norm && c < chunks) e = normalize4(e, rdiv, load_gamma_chunk(src, c, VEC));
+        if (!HELD_NORM && norm && c < chunks) e = normalize4(e, rdiv, load_gamma_chunk(src, c, VEC));
         if constexpr (NCH > 0) v[i] = e;
         amax = absmax4(amax, e);
     }
@@ -301,7 +334,11 @@ void launch_wave(const ActQuantParams &p, hipStream_t s)
     const int rows_per_block = 4;
     dim3 block(64, rows_per_block);
     dim3 grid((unsigned)((p.m + rows_per_block - 1) / rows_per_block));
-    launch_kernel((act_quant_wave_kernel<MODE, VEC>), grid, block, 0, s, p);
+    const bool two = p.src.k <= 512 && p.ldq <= 512;  // the padding is cleared by the same lanes
+    if (p.src.gamma && two) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 2>), grid, block, 0, s, p);
+    else if (p.src.gamma) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 4>), grid, block, 0, s, p);
+    else if (two) launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 2>), grid, block, 0, s, p);
+    else launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 4>), grid, block, 0, s, p);
 }
 
 // LDS for the row's squares where the literal summation order is asked for and a row fits the default limit
@@ -317,7 +354,13 @@ void launch_block(ActQuantParams p, hipStream_t s)
 {
     const size_t lds = launch_squares_lds(p);
     p.seq_in_lds = lds != 0;
-    launch_kernel((act_quant_block_kernel<MODE, NCH, VEC>), dim3((unsigned)p.m), dim3(256), lds, s, p);
+    launch_kernel((act_quant_block_kernel<MODE, NCH, VEC, false>), dim3((unsigned)p.m), dim3(256), lds, s, p);
+}
+
+template <int MODE, int NCH>
+void launch_block_norm(const ActQuantParams &p, hipStream_t s)
+{
+    launch_kernel((act_quant_block_kernel<MODE, NCH, true, true>), dim3((unsigned)p.m), dim3(256), 0, s, p);
 }
 
 template <int MODE>
@@ -359,6 +402,17 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
     }
     if (p.m > 32 && chunks <= 256) return vec ? launch_wave<MODE, true>(p, s) : launch_wave<MODE, false>(p, s);
     const int per_thread = (chunks + 255) >> 8;
+    if (vec && p.src.gamma && ordered && per_thread <= 7) {
+        switch (per_thread) {
+            case 1: return launch_block_norm<MODE, 1>(p, s);
+            case 2: return launch_block_norm<MODE, 2>(p, s);
+            case 3: return launch_block_norm<MODE, 3>(p, s);
+            case 4: return launch_block_norm<MODE, 4>(p, s);
+            case 5: return launch_block_norm<MODE, 5>(p, s);
+            case 6: return launch_block_norm<MODE, 6>(p, s);
+            default: return launch_block_norm<MODE, 7>(p, s);
+        }
+    }
     if (vec) {
         if (per_thread <= 3) return launch_block<MODE, 3, true>(p, s);
         if (per_thread <= 7) return launch_block<MODE, 7, true>(p, s);

@@ -331,6 +331,27 @@ def test_activation_quant_sequential_order_bit_exact(m, k):
     assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref)
 
 
+@pytest.mark.parametrize("m,k", [(600, 1028), (600, 1536), (600, 2048), (600, 2052), (520, 3072), (520, 3076), (520, 4100), (520, 5124), (513, 6148), (513, 7168),
+                                 (40, 4), (40, 256), (40, 260), (35, 508), (35, 512), (35, 516), (33, 1020), (33, 1024), (33, 301)])
+def test_activation_quant_with_a_norm_bit_exact(m, k):
+    """Row lengths around each count of chunks a thread, with rows whose dividends are zeros, tiny, huge or not finite (the plain division)."""
+    rng = np.random.default_rng(k + m)
+    x = synth_activations(rng, m, k, outliers=True)
+    x[1, ::3] = 0.0
+    x[2] = -0.0
+    x[3] *= f32(1e-36)
+    x[4, k // 2] = f32(1e30)
+    x[5, k - 1] = np.inf
+    x[6] *= f32(1e12)
+    g = rng.standard_normal(k, dtype=f32)
+    q, s, asum, y = bh.quantize_activations_i8(dev(x), dev(g), want_sum=True, want_y=True)
+    q_ref, s_ref, sum_ref = orc.rmsnorm_quantize_i8(x, g, 1e-5)
+    finite = [r for r in range(m) if r != 5]
+    assert np.array_equal(host(y)[finite].view(np.uint32), orc.rmsnorm(x, g, 1e-5)[finite].view(np.uint32))
+    assert np.array_equal(host(y)[5], orc.rmsnorm(x, g, 1e-5)[5], equal_nan=True)
+    assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), sum_ref)
+
+
 def test_activation_quant_edge_rows():
     x = np.zeros((4, 256), dtype=f32)
     x[1, :9] = [127.0, 0.5, -0.5, 1.5, 2.5, -2.5, 0.49999997, -126.5, 126.4999]
