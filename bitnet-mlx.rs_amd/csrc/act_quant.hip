@@ -119,9 +119,11 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
         v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if constexpr (NORM) {
-        float4 gm[NCH];
+        float4 gm[VEC ? NCH : 1];
+        if constexpr (VEC) {
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) gm[i] = lane + 64 * i < chunks ? load_gamma_chunk(src, lane + 64 * i, VEC) : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int i = 0; i < NCH; ++i) gm[i] = lane + 64 * i < chunks ? load_gamma_chunk(src, lane + 64 * i, VEC) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
         float ss;
         if (src.sum_order == BITNET_HIP_SUM_SEQUENTIAL) {
             ss = sum_squares_sequential<MODE>(src, row);
@@ -132,7 +134,14 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
             for (int i = 0; i < NCH; ++i) part[i] = wave_sum_f32(sum_squares4(0.0f, v[i]));
             ss = f32_add(f32_add(f32_add(part[0], part[1]), part[2]), part[3]);
         }
-        normalize_row(v, gm, make_divisor(rms_from_ss(ss, src.k, src.eps)), lane, 64, chunks);
+        const Divisor rdiv = make_divisor(rms_from_ss(ss, src.k, src.eps));
+        if constexpr (VEC) {
+            normalize_row(v, gm, rdiv, lane, 64, chunks);
+        } else {  // a load per weight: behind the sum they overlap other rows (4776 x 691 in front of it: 0.9 us more)
+#pragma unroll
+            for (int i = 0; i < NCH; ++i)
+                if (lane + 64 * i < chunks) v[i] = normalize4(v[i], rdiv, load_gamma_chunk(src, lane + 64 * i, VEC));
+        }
     }
     float amax = 0.0f;
 #pragma unroll
@@ -159,7 +168,8 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 // workgroups that take rows in turn and fetch the next one early are slower: 15.8 us against 12.7 us at 2048 x 6912.)
 // HELD_NORM: a norm in the declared order, whose weights are asked for with the row and not behind its sum of squares, and whose chunks are divided
 // together; NCH is then exactly what a row takes, since every chunk's weights take registers too.  With a norm, before -> now (without one), us:
-// 4096 x 5120 21.6 -> 17.9 (17.0), 4096 x 4096 18.5 -> 15.2 (14.0), 8192 x 2560 20.3 -> 18.6 (16.4), 2048 x 6912 16.7 -> 15.2 (12.5).
+// (above 14336 columns the registers of a workgroup with held weights leave a compute unit two: 2048 x 16384 37.1 -> 39.4, not taken)
+// 6000 x 12288 85 -> 69 (64.5), 2048 x 10240 25.9 -> 21.7 (16.3), 4096 x 5120 21.6 -> 17.9 (17.0), 4096 x 4096 18.5 -> 15.2 (14.0), 8192 x 2560 20.3 -> 18.6 (16.4), 2048 x 6912 16.7 -> 15.2 (12.5).
 template <int MODE, int NCH, bool VEC, bool HELD_NORM>
 __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
 {
@@ -369,11 +379,11 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
     const int chunks = (p.src.k + 3) >> 2;
     // Rows that all run at once: up to 16 wavefronts per row, with four chunks a thread above 8192 columns (213 rows of 13120 columns
     // with norm: 9.8 us in the 256-thread kernel -> 5.6 here; a decoder block with a 13824-wide FFN at 8 tokens: 36.3 -> 31.5).  Rows
-    // that come in many rounds stay with the 256-thread kernel where it is the faster: a compute unit holds fewer of the long rows
-    // here, and with a norm that costs more than the shorter chain gives (6000 x 12288 with norm: 115 us here, 89 there).
+    // that come in many rounds are here from 7168 columns on without a norm; with one they stay with the 256-thread kernel, of which a compute
+    // unit holds more (8192 x 8192 73.0 us here, 62.2 there, 4096 x 7680 33.1 and 27.0, 6000 x 12288 115 and 69).
     const bool ordered = !p.src.gamma || p.src.sum_order == BITNET_HIP_SUM_BLOCK256;
     const bool few = p.m <= ROW_QUANT_MAX_ROWS;
-    if ((few || (chunks > 1792 && (chunks <= 2048 || !p.src.gamma))) && vec && ordered && chunks <= 4096 && p.src.ldx < (1u << 31)) {
+    if ((few || (chunks > 1792 && !p.src.gamma)) && vec && ordered && chunks <= 4096 && p.src.ldx < (1u << 31)) {
         const float *x2 = p.src.x2;
         uint64_t magics = 0;
         bool in_range = true;
@@ -402,7 +412,7 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
     }
     if (p.m > 32 && chunks <= 256) return vec ? launch_wave<MODE, true>(p, s) : launch_wave<MODE, false>(p, s);
     const int per_thread = (chunks + 255) >> 8;
-    if (vec && p.src.gamma && ordered && per_thread <= 7) {
+    if (vec && p.src.gamma && ordered && per_thread <= 14) {
         switch (per_thread) {
             case 1: return launch_block_norm<MODE, 1>(p, s);
             case 2: return launch_block_norm<MODE, 2>(p, s);
@@ -410,7 +420,11 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
             case 4: return launch_block_norm<MODE, 4>(p, s);
             case 5: return launch_block_norm<MODE, 5>(p, s);
             case 6: return launch_block_norm<MODE, 6>(p, s);
-            default: return launch_block_norm<MODE, 7>(p, s);
+            case 7: return launch_block_norm<MODE, 7>(p, s);
+            case 8: return launch_block_norm<MODE, 8>(p, s);
+            case 9: case 10: return launch_block_norm<MODE, 10>(p, s);
+            case 11: case 12: return launch_block_norm<MODE, 12>(p, s);
+            default: return launch_block_norm<MODE, 14>(p, s);
         }
     }
     if (vec) {

@@ -331,7 +331,7 @@ def test_activation_quant_sequential_order_bit_exact(m, k):
     assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref)
 
 
-@pytest.mark.parametrize("m,k", [(600, 1028), (600, 1536), (600, 2048), (600, 2052), (520, 3072), (520, 3076), (520, 4100), (520, 5124), (513, 6148), (513, 7168),
+@pytest.mark.parametrize("m,k", [(600, 1028), (600, 1536), (600, 2048), (600, 2052), (520, 3072), (520, 3076), (520, 4100), (520, 5124), (513, 6148), (513, 7168), (513, 7172), (513, 8192), (513, 9220), (513, 12292), (514, 14336), (514, 14340),
                                  (40, 4), (40, 256), (40, 260), (35, 508), (35, 512), (35, 516), (33, 1020), (33, 1024), (33, 301)])
 def test_activation_quant_with_a_norm_bit_exact(m, k):
     """Row lengths around each count of chunks a thread, with rows whose dividends are zeros, tiny, huge or not finite (the plain division)."""
