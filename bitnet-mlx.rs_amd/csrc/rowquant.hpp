@@ -140,6 +140,20 @@ __device__ __forceinline__ float load_elem(const RowSource &p, size_t row, int i
     }
 }
 
+// Elements i .. i + 3 of a row of k, zeros from k on, at any alignment of four bytes: one 16-byte load, in the row's last chunk that of its last
+// four elements, shifted.  The quantiser of rows that are no multiple of four columns, as four loads -> as one, us: 8192 x 1023 13.1 -> 11.7 (the
+// host), with a norm 20.3 -> 13.2; 4096 x 5121 26.1 -> 24.1, 43.7 -> 30.4; 2048 x 17001 77.6 -> 49.8, 164 -> 77.
+__device__ __forceinline__ float4 load4_any(const float *row, int i, int k)
+{
+    typedef float v4 __attribute__((ext_vector_type(4), aligned(4)));
+    if (k < 4) return make_float4(row[i], i + 1 < k ? row[i + 1] : 0.0f, i + 2 < k ? row[i + 2] : 0.0f, 0.0f);
+    const int from = min(i, k - 4), shift = i - from;
+    v4 e = *reinterpret_cast<const v4 *>(row + from);
+    if (shift & 1) e = (v4){e[1], e[2], e[3], 0.0f};  // two selects: the compiler's code for a branch a shift lost the shift by three
+    if (shift & 2) e = (v4){e[2], e[3], 0.0f, 0.0f};
+    return make_float4(e[0], e[1], e[2], e[3]);
+}
+
 // Chunk c (elements 4c .. 4c+3).  VEC: 16-byte loads, all four elements inside the row.
 template <int MODE, bool VEC>
 __device__ __forceinline__ float4 load_chunk(const RowSource &p, size_t row, int c)
@@ -158,6 +172,11 @@ __device__ __forceinline__ float4 load_chunk(const RowSource &p, size_t row, int
             return *reinterpret_cast<const float4 *>(p.x + row * p.ldx +
                                                      (size_t)(h / p.gqa_group) * p.head_dim + d);
         }
+    } else if constexpr (MODE == BITNET_HIP_INPUT_PLAIN) {
+        return load4_any(p.x + row * p.ldx, 4 * c, p.k);
+    } else if constexpr (MODE == BITNET_HIP_INPUT_RELU2_MUL) {
+        const float4 g = load4_any(p.x + row * p.ldx, 4 * c, p.k), u = load4_any(p.x2 + row * p.ldx, 4 * c, p.k);
+        return make_float4(relu2_mul(g.x, u.x), relu2_mul(g.y, u.y), relu2_mul(g.z, u.z), relu2_mul(g.w, u.w));
     } else {
         float4 v;
         int i = 4 * c;
@@ -172,13 +191,7 @@ __device__ __forceinline__ float4 load_chunk(const RowSource &p, size_t row, int
 __device__ __forceinline__ float4 load_gamma_chunk(const RowSource &p, int c, bool vec)
 {
     if (vec) return *reinterpret_cast<const float4 *>(p.gamma + 4 * (size_t)c);
-    float4 g;
-    int i = 4 * c;
-    g.x = i + 0 < p.k ? p.gamma[i + 0] : 0.0f;
-    g.y = i + 1 < p.k ? p.gamma[i + 1] : 0.0f;
-    g.z = i + 2 < p.k ? p.gamma[i + 2] : 0.0f;
-    g.w = i + 3 < p.k ? p.gamma[i + 3] : 0.0f;
-    return g;
+    return load4_any(p.gamma, 4 * c, p.k);
 }
 
 __device__ __forceinline__ float sum_squares4(float part, const float4 &e)

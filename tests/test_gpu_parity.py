@@ -352,6 +352,28 @@ def test_activation_quant_with_a_norm_bit_exact(m, k):
     assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), sum_ref)
 
 
+@pytest.mark.parametrize("m,k", [(33, 1), (33, 2), (33, 3), (40, 5), (40, 6), (40, 7), (35, 509), (35, 1021), (35, 1022), (35, 1023), (600, 1029), (600, 1030), (600, 1031),
+                                 (5, 2561), (520, 5121), (513, 7169), (514, 9898), (20, 16385), (513, 16387)])
+@pytest.mark.parametrize("how", ["plain", "norm", "gated", "shifted"])
+def test_activation_quant_of_rows_at_any_alignment_bit_exact(m, k, how):
+    """Rows that are no multiple of four columns, each remainder, and rows that start four bytes past an aligned address: the row's last
+    chunk is read as the last four of its elements."""
+    rng = np.random.default_rng(k + m)
+    x, g, kw = synth_activations(rng, m, k, outliers=True), None, {}
+    ref = x
+    if how == "norm":
+        g = rng.standard_normal(k, dtype=f32)
+    elif how == "gated":
+        up = synth_activations(rng, m, k)
+        kw, ref = {"x2": dev(up), "input_mode": bh.INPUT_RELU2_MUL}, orc.relu2_mul(x, up)
+    xd = dev(x)
+    if how == "shifted":
+        xd = torch.cat([torch.zeros(1, device="cuda"), xd.flatten()])[1:].view(m, k)
+    q, s, asum, _ = bh.quantize_activations_i8(xd, None if g is None else dev(g), want_sum=True, **kw)
+    q_ref, s_ref, sum_ref = orc.quantize_activations_i8(ref) if g is None else orc.rmsnorm_quantize_i8(x, g, 1e-5)
+    assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), sum_ref)
+
+
 def test_activation_quant_edge_rows():
     x = np.zeros((4, 256), dtype=f32)
     x[1, :9] = [127.0, 0.5, -0.5, 1.5, 2.5, -2.5, 0.49999997, -126.5, 126.4999]
