@@ -179,11 +179,28 @@ bool recorded_in_two(const bitnet_hip_bitlinear *const *layers, size_t count, co
     return m >= 2 && s && !quantises_in_launch(layers, count, x, m, gamma, sum_order, false) && being_captured(s);  // the null stream is never captured
 }
 
+// Whether an output of the projections lies over the rows that they quantise (x, x2) or over the norm's weights.  A launch that quantises its
+// rows itself still reads them in some workgroups while others store outputs, so such a call is two launches, whatever its size.
+bool writes_over_input(const bitnet_hip_bitlinear *const *layers, size_t count, const float *x, const float *x2, size_t ldx, size_t m, size_t k,
+                       const float *gamma, const float *const *out, const int32_t *const *acc = nullptr)
+{
+    const auto at = [](const void *p) { return reinterpret_cast<uintptr_t>(p); };
+    const size_t row_bytes = sizeof(float) * ((m - 1) * ldx + (k < ldx ? k : ldx));  // a row of repeated heads is shorter than k
+    for (size_t j = 0; j < count; ++j) {
+        const size_t bytes = sizeof(float) * m * layers[j]->out_features;
+        for (const uintptr_t to : {at(out[j]), acc ? at(acc[j]) : 0}) {
+            const auto meets = [&](const float *from, size_t from_bytes) { return to && from && to < at(from) + from_bytes && at(from) < to + bytes; };
+            if (meets(x, row_bytes) || meets(x2, row_bytes) || meets(gamma, sizeof(float) * k)) return true;
+        }
+    }
+    return false;
+}
+
 // Runs `count` projections that share one input row block [m, k].  At decode token counts the quantiser runs
 // inside the GEMV launch (up to GEMV_MAX_PROJ projections per launch); otherwise the stand-alone quantiser
 // fills q / a_scale / a_sum (scratch the caller provides) and the GEMV or GEMM kernels consume them.
 // residual / out / acc are per-projection arrays (entries of residual and acc may be null, and so may the arrays).  ldq: row
-// stride of q, in_features or padded_k(in_features).
+// stride of q, in_features or padded_k(in_features).  die: only where no output lies over the input.
 int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float *x, const float *x2, size_t ldx,
                     size_t m, int input_mode, size_t gqa_group, size_t head_dim, const float *gamma, float eps,
                     int sum_order, const float *const *residual, float *const *out, int32_t *const *acc, int8_t *q,
@@ -191,7 +208,8 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
                     bool alone = true, const DieFlags *die = nullptr)
 {
     size_t k = layers[0]->in_features;
-    const bool short_rows = !want_quant_outputs && gemv_rowq_takes(x, ldx, m, k, input_mode, gqa_group, head_dim, gamma, sum_order,
+    const bool over = writes_over_input(layers, (size_t)count, x, x2, ldx, m, k, gamma, out, acc);
+    const bool short_rows = !over && !want_quant_outputs && gemv_rowq_takes(x, ldx, m, k, input_mode, gqa_group, head_dim, gamma, sum_order,
                                                                    launch_group_blocks(layers, count), alone);
     auto proj_of = [&](int j) {
         bitnet_hip_bitlinear *bl = layers[j];
@@ -214,7 +232,7 @@ int run_projections(bitnet_hip_bitlinear *const *layers, int count, const float 
         }
         return BITNET_HIP_OK;
     }
-    if (gemv_fused_supported(x, x2, ldx, m, k, input_mode, head_dim, gamma, sum_order, launch_group_blocks(layers, count))) {
+    if (!over && gemv_fused_supported(x, x2, ldx, m, k, input_mode, head_dim, gamma, sum_order, launch_group_blocks(layers, count))) {
         for (int j0 = 0; j0 < count; j0 += GEMV_MAX_PROJ) {
             GemvProj pjs[GEMV_MAX_PROJ];
             const int nj = count - j0 < GEMV_MAX_PROJ ? count - j0 : GEMV_MAX_PROJ;
@@ -961,12 +979,17 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
 
     hipStream_t s = as_stream(stream);
     const bool debug = dbg_q || dbg_a_scale || dbg_acc;
-    bool fused = quantises_in_launch(&layer, 1, x, m, gamma, sum_order);
+    const float *res[1] = {residual};
+    float *outs[1] = {out};
+    int32_t *accs[1] = {dbg_acc};
+    const bool over = writes_over_input(&layer, 1, x, nullptr, in, m, in, gamma, outs, accs);
+    const bool one_launch = quantises_in_launch(&layer, 1, x, m, gamma, sum_order);  // but for an output over the input
+    bool fused = one_launch && !over;
     const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
                         recorded_in_two(&layer, 1, x, m, gamma, sum_order, s);
     fused = fused && !in_two;
     bitnet_hip_bitlinear *layers[1] = {layer};
-    const bool on_dies = !fused && !in_two && !debug && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
+    const bool on_dies = !fused && !in_two && !over && !debug && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
                          quantises_on_dies(layers, 1, x, m, gamma, sum_order, s);
     void *ws = workspace;
     bool own_ws = false;
@@ -976,7 +999,7 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
         const size_t least = quant_scratch_bytes(m, in);
         if (!dbg_q && (!ws || workspace_bytes >= quant_scratch_bytes(m, padded_k(in)))) ldq = padded_k(in);
         const size_t need = quant_scratch_bytes(m, ldq);
-        if (!ws) {
+        if (!ws || (one_launch && over && !debug && workspace_bytes < least)) {  // nobody asked the caller for scratch
             hipError_t e = hipMallocAsync(&ws, need, s);
             if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward: hipMallocAsync(%zu) failed: %s", need, hipGetErrorString(e));
             own_ws = true;
@@ -987,9 +1010,6 @@ int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, co
         if (dbg_q) sc.q = dbg_q;
         if (dbg_a_scale) sc.a_scale = dbg_a_scale;
     }
-    const float *res[1] = {residual};
-    float *outs[1] = {out};
-    int32_t *accs[1] = {dbg_acc};
     const DieFlags flags = on_dies ? call_flags(ws, m, ldq) : DieFlags{};
     int rc = run_projections(layers, 1, x, nullptr, in, m, BITNET_HIP_INPUT_PLAIN, 1, 1, gamma, eps, sum_order, res, outs,
                              accs, sc.q, ldq, sc.a_scale, sc.a_sum, debug, s, !in_two, on_dies ? &flags : nullptr);
@@ -1071,11 +1091,13 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     }
     const size_t in = layers[0]->in_features;
     hipStream_t s = as_stream(stream);
-    bool fused = quantises_in_launch(layers, count, x, m, gamma, sum_order);
+    const bool over = writes_over_input(layers, count, x, nullptr, in, m, in, gamma, outs);
+    const bool one_launch = quantises_in_launch(layers, count, x, m, gamma, sum_order);  // but for an output over the input
+    bool fused = one_launch && !over;
     const bool in_two = fused && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) &&
                         recorded_in_two(layers, count, x, m, gamma, sum_order, s);
     fused = fused && !in_two;
-    const bool on_dies = !fused && !in_two && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
+    const bool on_dies = !fused && !in_two && !over && workspace && workspace_bytes >= quant_scratch_bytes(m, padded_k(in)) + die_flag_bytes(m) &&
                          quantises_on_dies(layers, count, x, m, gamma, sum_order, s);
     void *ws = workspace;
     bool own_ws = false;
@@ -1084,7 +1106,7 @@ int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size
     if (!fused) {
         if (!ws || workspace_bytes >= quant_scratch_bytes(m, padded_k(in))) ldq = padded_k(in);
         const size_t need = quant_scratch_bytes(m, ldq);
-        if (!ws) {
+        if (!ws || (one_launch && over && workspace_bytes < need)) {  // nobody asked the caller for scratch
             hipError_t e = hipMallocAsync(&ws, need, s);
             if (e != hipSuccess) return fail(BITNET_HIP_MEMORY_ERROR, "forward_multi: hipMallocAsync(%zu) failed: %s", need, hipGetErrorString(e));
             own_ws = true;
@@ -1374,6 +1396,7 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
             if (rc != BITNET_HIP_OK) return;
             DieFlags flags;
             const bool on_dies = chains_asked <= 1 && !dec->die_flags_spent &&
+                                 !writes_over_input(layers, (size_t)count, x, x2, ldx, rows, layers[0]->in_features, gamma, outs) &&
                                  gemv_die_takes(x, x2, ldx, rows, layers[0]->in_features, mode, gamma, dec->sum_order, launch_group_blocks(layers, (size_t)count), false);
             if (on_dies) {
                 uint64_t *sets[2] = {dec->die_flags, dec->die_flags + GEMV_DIE_SETS * dec->die_stride()};

@@ -169,10 +169,12 @@ PyObject *forward(PyObject *const *args, Py_ssize_t nargs)
     }
     // scratch only where the call runs the stand-alone quantiser
     const float *xp = x->const_data_ptr<float>();
-    const size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch_on(&l.handle, 1, xp, (size_t)m, gamma, (int)order, stream.handle);
+    size_t ws_bytes = bitnet_hip_bitlinear_forward_scratch_on(&l.handle, 1, xp, (size_t)m, gamma, (int)order, stream.handle);
+    float *yp = y->data_ptr<float>();
+    // a result over the input takes two launches, and scratch, whatever the size
+    if (!ws_bytes && yp < xp + m * l.in && xp < yp + m * l.out) ws_bytes = bitnet_hip_bitlinear_workspace_size(l.handle, (size_t)m);
     at::Tensor ws;
     if (ws_bytes) ws = new_on(stream, {(int64_t)((ws_bytes + 3) / 4)}, x->options());
-    float *yp = y->data_ptr<float>();
     void *wp = ws_bytes ? ws.data_ptr() : nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS

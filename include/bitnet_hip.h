@@ -358,7 +358,9 @@ size_t bitnet_hip_bitlinear_forward_scratch(const bitnet_hip_bitlinear *layer, c
  *   residual   NULL or [m, out] f32 added after the bias
  *   workspace  device buffer of at least workspace_size(m) bytes, or NULL to let the call allocate
  *              stream-ordered scratch itself
- *   debug outputs (each may be NULL): q [m,in] int8, a_scale [m] f32, acc [m,out] int32. */
+ *   debug outputs (each may be NULL): q [m,in] int8, a_scale [m] f32, acc [m,out] int32.
+ *   out may lie over x, or over a part of it: the rows are then quantised in a launch of their own, in the workspace or, where that is too
+ *   small because forward_scratch asked for none, in stream-ordered scratch of the call's. */
 int bitnet_hip_bitlinear_forward(bitnet_hip_bitlinear *layer, const float *x, const size_t *dims, int rank,
                                  const float *gamma, float eps, int sum_order, const float *residual,
                                  float *out, void *workspace, size_t workspace_bytes, int8_t *dbg_q,
@@ -383,7 +385,7 @@ int bitnet_hip_bitlinear_forward_noalloc(bitnet_hip_bitlinear *layer, const floa
  * (bitnet-inference/src/engine/transformer_layers.rs:470-475), FeedForwardNetwork::forward up_proj/gate_proj
  * (:605-611).  The input is quantised once; at decode token counts up to three layers share one kernel
  * launch.  outs[j] is [m, out_features of layers[j]].  All layers must have the same in_features
- * (else SHAPE_MISMATCH).  workspace as for bitnet_hip_bitlinear_forward (sized for layers[0]). */
+ * (else SHAPE_MISMATCH).  workspace, and outputs over x, as for bitnet_hip_bitlinear_forward (sized for layers[0]). */
 int bitnet_hip_bitlinear_forward_multi(bitnet_hip_bitlinear *const *layers, size_t count, const float *x, size_t m,
                                        const float *gamma, float eps, int sum_order, float *const *outs,
                                        void *workspace, size_t workspace_bytes, void *stream);

@@ -2147,3 +2147,59 @@ def test_decoder_rows_quantised_once_a_die(dims, layers):
     for looks in (-1, 4097):
         with pytest.raises(bh.BitLinearError):
             dec.set_row_wait(looks)
+
+
+# ---- outputs over the input ----------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("m,k,norm", [(1, 2560, True), (1, 8192, False), (1, 7424, True), (2, 1024, False), (6, 2560, True), (8, 516, False), (16, 2560, True),
+                                      (64, 2560, False), (33, 4096, True), (200, 1028, True)])
+def test_forward_with_its_output_over_its_input(m, k, norm):
+    """A square layer whose result takes the place of its input, wholly or shifted by one row, with and without a workspace, alone, captured, on the
+    static scratch and among several layers: the oracle's bits at every size that a one-launch kernel takes without the overlap."""
+    rng = np.random.default_rng(m + k)
+    packed = random_packed_ternary(rng, 1, k * k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=k), "over")
+    layer.set_quantized_weights(torch.from_numpy(packed), 0.02)
+    g = (1 + 0.1 * rng.standard_normal(k, dtype=f32)).astype(f32) if norm else None
+    gd = dev(g) if norm else None
+    x = synth_activations(rng, m, k, outliers=True)
+    want = orc.bitlinear_forward(x, packed, k, f32(0.02), g=g)[0]
+    roomy = torch.empty((layer.workspace_size(m) + (1 << 17),), dtype=torch.uint8, device="cuda")
+    for ws in (None, roomy, roomy[: layer.workspace_size(m)]):
+        for _ in range(3):
+            buf = dev(x)
+            assert np.array_equal(host(layer.forward(buf, gamma=gd, out=buf, workspace=ws)), want)
+    rows = torch.empty((m + 1, k), device="cuda")
+    rows[1:] = dev(x)
+    assert np.array_equal(host(layer.forward(rows[1:], gamma=gd, out=rows[:m])), want)
+    buf = dev(x)
+    with_residual = orc.bitlinear_forward(x, packed, k, f32(0.02), g=g, residual=x)[0]
+    assert np.array_equal(host(layer.forward(buf, gamma=gd, residual=buf, out=buf)), with_residual)
+    if m * k <= 1 << 20:
+        buf = dev(x)
+        assert np.array_equal(host(layer.forward_noalloc(buf, buf, gamma=gd)), want)
+    # the C entry without a workspace, and with one of the size that forward_scratch names
+    lib = bh.load_library()
+    handles = (ctypes.c_void_p * 2)(layer._h, layer._h)
+    asked = lib.bitnet_hip_bitlinear_forward_multi_scratch(handles, 2, buf.data_ptr(), m, _pointer(gd), bh.SUM_BLOCK256)
+    for ws in (None, torch.empty((max(asked, 1),), dtype=torch.uint8, device="cuda")):
+        buf, beside = dev(x), torch.empty((m, k), device="cuda")
+        outs = (ctypes.c_void_p * 2)(beside.data_ptr(), buf.data_ptr())
+        assert lib.bitnet_hip_bitlinear_forward_multi(handles, 2, buf.data_ptr(), m, _pointer(gd), 1e-5, bh.SUM_BLOCK256, outs, _pointer(ws),
+                                                      ws.numel() if ws is not None else 0, None) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(host(beside), want) and np.array_equal(host(buf), want)
+    source, buf = dev(x), torch.empty((m, k), device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        buf.copy_(source)
+        layer.forward(buf, gamma=gd, out=buf)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(host(buf), want)
+
+
+def _pointer(t):
+    return t.data_ptr() if t is not None else None
