@@ -1184,10 +1184,11 @@ struct bitnet_hip_decoder {
     int32_t *a_sum = nullptr;
     float *qb = nullptr, *kb = nullptr, *vb = nullptr, *x1 = nullptr, *gate = nullptr, *up = nullptr;
     float *ping = nullptr;
-    // Flags of the launches that quantise their rows once a die (gemv_die.hip): two sets used in turn.  Every step leaves the first set
-    // cleared; a step that failed half way does not, and no later one uses them.
+    // Flags of the launches that quantise their rows once a die (gemv_die.hip): two sets used in turn.  Every step finds the first set
+    // cleared, recorded steps too, and leaves it so; one that fails half way clears it before it returns, or, where that fails as well, the next
+    // step or replay does.
     uint64_t *die_flags = nullptr;
-    bool die_flags_spent = false;
+    bool die_flags_dirty = false;
     int die_looks = GEMV_DIE_LOOKS;
     size_t die_stride() const { return align_up(max_tokens < (size_t)GEMV_DIE_MAX_M ? max_tokens : (size_t)GEMV_DIE_MAX_M, 16); }
     // One decode at a time: the activation buffers above are shared by every call on this decoder.  The mutex
@@ -1395,7 +1396,7 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
                        const float *gamma, const float *res0, float *const *outs) {
             if (rc != BITNET_HIP_OK) return;
             DieFlags flags;
-            const bool on_dies = chains_asked <= 1 && !dec->die_flags_spent &&
+            const bool on_dies = chains_asked <= 1 &&
                                  !writes_over_input(layers, (size_t)count, x, x2, ldx, rows, layers[0]->in_features, gamma, outs) &&
                                  gemv_die_takes(x, x2, ldx, rows, layers[0]->in_features, mode, gamma, dec->sum_order, launch_group_blocks(layers, (size_t)count), false);
             if (on_dies) {
@@ -1435,7 +1436,8 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
     if (chains <= 1) {
         run_chain(0, m, s);
         if (rc == BITNET_HIP_OK && (die_launches & 1)) rc = launch_clear_die_flags(dec->die_flags, dec->die_stride(), m, s);
-        if (rc != BITNET_HIP_OK && die_launches) dec->die_flags_spent = true;
+        if (rc != BITNET_HIP_OK && die_launches && launch_clear_die_flags(dec->die_flags, dec->die_stride(), dec->die_stride(), s) != BITNET_HIP_OK)
+            dec->die_flags_dirty = true;
     } else {
         // fork: the side streams start behind whatever the caller's stream holds; join: it continues behind them all.
         // Recorded into the caller's graph when s is being captured (the events pull the side streams into the capture).
@@ -1456,6 +1458,27 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
         }
     }
     return rc;
+}
+
+// What a step or a replay on s waits for: the step before it, on whatever stream, and flags that one left when it failed.
+static int before_step(bitnet_hip_decoder *dec, hipStream_t s, bool capturing)
+{
+    if (dec->done_recorded && dec->done_stream != s && !capturing) BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));
+    if (dec->die_flags_dirty) {
+        const int rc = launch_clear_die_flags(dec->die_flags, dec->die_stride(), dec->die_stride(), s);
+        if (rc != BITNET_HIP_OK) return rc;
+        dec->die_flags_dirty = capturing;  // what is only recorded clears nothing yet
+    }
+    return BITNET_HIP_OK;
+}
+// What the next one on another stream waits for, also behind a step that failed after some of its launches.
+static int behind_step(bitnet_hip_decoder *dec, hipStream_t s, bool capturing)
+{
+    if (capturing) return BITNET_HIP_OK;
+    BITNET_HIP_TRY(hipEventRecord(dec->done, s));
+    dec->done_stream = s;
+    dec->done_recorded = true;
+    return BITNET_HIP_OK;
 }
 
 namespace {
@@ -1566,21 +1589,17 @@ int bitnet_hip_decoder_decode_layers(bitnet_hip_decoder *dec, size_t layer_begin
             return fail(BITNET_HIP_NOT_INITIALIZED, "decoder_decode: a projection has no weights yet");
     }
     std::lock_guard<std::mutex> one_decode(dec->decode_lock);
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(s, &capturing);
-    if (dec->done_recorded && dec->done_stream != s && capturing == hipStreamCaptureStatusNone)
-        BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));  // the previous decode used these buffers on another stream
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(s, &status);
+    const bool capturing = status != hipStreamCaptureStatusNone;
+    int rc = before_step(dec, s, capturing);
+    if (rc != BITNET_HIP_OK) return rc;
     const StepKey step = {layer_begin, layer_end, m, x_in, x_out, q_last, k_last};
-    int rc = BITNET_HIP_OK;
-    hipGraphExec_t recorded = capturing == hipStreamCaptureStatusNone ? repeated_step_graph(dec, step) : nullptr;
+    hipGraphExec_t recorded = capturing ? nullptr : repeated_step_graph(dec, step);
     if (recorded) BITNET_HIP_TRY(hipGraphLaunch(recorded, s));
     else rc = enqueue_step(dec, step, s);
-    if (rc == BITNET_HIP_OK && capturing == hipStreamCaptureStatusNone) {
-        BITNET_HIP_TRY(hipEventRecord(dec->done, s));
-        dec->done_stream = s;
-        dec->done_recorded = true;
-    }
-    return rc;
+    const int ordered = behind_step(dec, s, capturing);
+    return rc != BITNET_HIP_OK ? rc : ordered;
 }
 
 int bitnet_hip_decoder_decode(bitnet_hip_decoder *dec, const float *x_in, size_t m, float *x_out, float *q_last,
@@ -1666,17 +1685,13 @@ int bitnet_hip_decoder_graph_launch(bitnet_hip_decoder_graph *graph, void *strea
     guards.reserve((graph->layer_end - graph->layer_begin) * 7);
     for (size_t i = graph->layer_begin * 7; i < graph->layer_end * 7; ++i) guards.emplace_back(dec->proj[i]->lock);
     std::lock_guard<std::mutex> one_decode(dec->decode_lock);
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(s, &capturing);
-    if (dec->done_recorded && dec->done_stream != s && capturing == hipStreamCaptureStatusNone)
-        BITNET_HIP_TRY(hipStreamWaitEvent(s, dec->done, 0));
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(s, &status);
+    const bool capturing = status != hipStreamCaptureStatusNone;
+    const int rc = before_step(dec, s, capturing);
+    if (rc != BITNET_HIP_OK) return rc;
     BITNET_HIP_TRY(hipGraphLaunch(graph->exec, s));
-    if (capturing == hipStreamCaptureStatusNone) {
-        BITNET_HIP_TRY(hipEventRecord(dec->done, s));
-        dec->done_stream = s;
-        dec->done_recorded = true;
-    }
-    return BITNET_HIP_OK;
+    return behind_step(dec, s, capturing);
 }
 
 void bitnet_hip_decoder_graph_destroy(bitnet_hip_decoder_graph *graph) { delete graph; }

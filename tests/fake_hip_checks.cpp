@@ -12,6 +12,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../bitnet-mlx.rs_amd/host/bitlinear.hpp"
@@ -53,6 +54,46 @@ long last(const std::string &name, hipStream_t stream)
         if (calls[i].name == name && calls[i].stream == stream) return i;
     return -1;
 }
+// The launches that quantise rows once a die, as far as their flags go (gemv_die.hip): a launch must find none of its rows' flags up, puts them
+// up, and takes down those it is given to clear.  What is launched while the stream is captured does so when the graph is replayed.
+struct DieLaunch {
+    uint64_t *flags, *clear, tag;
+    unsigned stride, m;
+};
+size_t die_launches = 0, stale_flags = 0;
+constexpr unsigned DIES = 16;
+void run(const DieLaunch &l)
+{
+    for (unsigned die = 0; die < DIES; ++die)
+        for (unsigned row = 0; row < l.m; ++row) {
+            if (l.flags) {
+                stale_flags += l.flags[die * l.stride + row] == l.tag;
+                l.flags[die * l.stride + row] = l.tag;
+            }
+            if (l.clear) l.clear[die * l.stride + row] = 0;
+        }
+    die_launches += l.flags != nullptr;
+}
+std::vector<DieLaunch> captured;
+std::map<const void *, std::vector<DieLaunch>> graphs;  // by graph and by executable graph
+void launched(const std::string &name, void **args, hipStream_t s)
+{
+    DieLaunch l = {};
+    if (name.find("gemv_die_kernel") != std::string::npos) {
+        const char *last = static_cast<const char *>(args[10]) + 192;  // the block behind those of the three projections: q, a_scale, flags, ...
+        memcpy(&l.flags, last + 16, 3 * sizeof(uint64_t));
+        memcpy(&l.stride, last + 40, sizeof(unsigned));
+        l.m = *static_cast<unsigned *>(args[6]) & 0xffffu;
+    } else if (name.find("clear_die_flags_kernel") != std::string::npos) {
+        l = {nullptr, *static_cast<uint64_t **>(args[0]), 0, *static_cast<unsigned *>(args[1]), *static_cast<unsigned *>(args[2])};
+    } else {
+        return;
+    }
+    if (s && s == capturing) captured.push_back(l);
+    else run(l);
+}
+int launches_until_failure = -1;  // the launch that fails is queued all the same, and the error is there for whoever asks next
+hipError_t pending = hipSuccess;
 hipError_t copy(void *dst, const void *src, size_t bytes)
 {
     if (copies_until_failure == 0) {
@@ -74,7 +115,7 @@ hipError_t make(T *out)
 extern "C" {
 hipError_t hipGetSymbolAddress(void **p, const void *) { static char held[1 << 21]; *p = held; return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipGetLastError() { return fake::launch_answer; }
+hipError_t hipGetLastError() { return fake::pending != hipSuccess ? std::exchange(fake::pending, hipSuccess) : fake::launch_answer; }
 const char *hipGetErrorString(hipError_t) { return "as told"; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 
@@ -112,23 +153,40 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t s) { return fake::note("hipEve
 hipError_t hipEventSynchronize(hipEvent_t) { return fake::note("hipEventSynchronize"); }
 
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) { std::swap(*m, fake::thread_mode); return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { fake::capturing = s; return fake::note("hipStreamBeginCapture", s); }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { fake::capturing = nullptr; return fake::make(g); }
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { fake::capturing = s; fake::captured.clear(); return fake::note("hipStreamBeginCapture", s); }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g)
+{
+    fake::capturing = nullptr;
+    (void)fake::make(g);
+    fake::graphs[*g] = fake::captured;
+    return hipSuccess;
+}
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st)
 {
     *st = s && s == fake::capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
-hipError_t hipGraphInstantiate(hipGraphExec_t *g, hipGraph_t, hipGraphNode_t *, char *, size_t) { (void)fake::note("hipGraphInstantiate"); return fake::make(g); }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) { return fake::note("hipGraphLaunch", s); }
+hipError_t hipGraphInstantiate(hipGraphExec_t *g, hipGraph_t of, hipGraphNode_t *, char *, size_t)
+{
+    (void)fake::make(g);
+    fake::graphs[*g] = fake::graphs[of];
+    return fake::note("hipGraphInstantiate");
+}
+hipError_t hipGraphLaunch(hipGraphExec_t g, hipStream_t s)
+{
+    for (const fake::DieLaunch &l : fake::graphs[g]) fake::run(l);
+    return fake::note("hipGraphLaunch", s);
+}
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return fake::note("hipGraphExecDestroy"); }
 
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t s) { return fake::note("configure", s); }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *s) { *s = fake::calls.back().stream; return hipSuccess; }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t s)
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s)
 {
     fake::kernels.push_back(fake::kernel_names()[f]);
+    fake::launched(fake::kernels.back(), args, s);
+    if (fake::launches_until_failure >= 0 && fake::launches_until_failure-- == 0) fake::pending = hipErrorLaunchFailure;
     return fake::note("launch", s, fake::launch_answer);
 }
 void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
@@ -261,10 +319,10 @@ void loads_wait_for_the_stream_once()
     }
 }
 
-bitnet_hip_decoder *decoder_with_weights(size_t layers, size_t hidden, size_t ffn)
+bitnet_hip_decoder *decoder_with_weights(size_t layers, size_t hidden, size_t ffn, size_t tokens = 4)
 {
     bitnet_hip_decoder *dec = nullptr;
-    CHECK(bitnet_hip_decoder_create(layers, hidden, ffn, hidden / 16, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, 4, &dec) == BITNET_HIP_OK);
+    CHECK(bitnet_hip_decoder_create(layers, hidden, ffn, hidden / 16, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, tokens, &dec) == BITNET_HIP_OK);
     const std::vector<uint8_t> codes(hidden * (hidden > ffn ? hidden : ffn) / 4, 0x22);
     for (size_t l = 0; l < layers; ++l)
         for (int p = 0; p < 7; ++p) {
@@ -318,6 +376,42 @@ void recording_a_step_leaves_other_captures_alone()
     }
     CHECK(fake::thread_mode == hipStreamCaptureModeGlobal);
     bitnet_hip_decoder_destroy(dec);
+}
+
+// No launch of a step that quantises rows once a die finds a flag of an earlier launch up: not after steps of other sizes, in a replay, nor
+// behind a step that failed after any of its launches, whether its flags could be cleared at once or not.
+void steps_find_their_flags_down()
+{
+    for (size_t layers : {1, 2, 3}) {
+        bitnet_hip_decoder *dec = decoder_with_weights(layers, 512, 1408, 64);
+        std::vector<float> x(64 * 512), out(64 * 512), other(64 * 512);
+        const auto step = [&](size_t m, std::vector<float> &to, size_t end) {
+            return bitnet_hip_decoder_decode_layers(dec, 0, end, x.data(), m, to.data(), nullptr, nullptr, side);
+        };
+        fake::die_launches = fake::stale_flags = 0;
+        for (size_t m : {9, 33, 16, 3, 64, 17, 64})
+            for (int times = 0; times < 4; ++times) CHECK(step(m, out, layers) == BITNET_HIP_OK);
+        bitnet_hip_decoder_graph *graph = nullptr;
+        CHECK(bitnet_hip_decoder_graph_create(dec, 0, layers, x.data(), 12, out.data(), nullptr, nullptr, &graph) == BITNET_HIP_OK);
+        CHECK(bitnet_hip_decoder_graph_launch(graph, side) == BITNET_HIP_OK && fake::die_launches > 0 && fake::stale_flags == 0);
+        for (int at = 0; at < (int)(4 * layers); ++at)
+            for (int clear_fails : {0, 1}) {
+                fake::launches_until_failure = at;
+                if (clear_fails) fake::launch_answer = hipErrorLaunchFailure;  // every launch then reports an error, the first one already
+                CHECK(step(48, other, layers) != BITNET_HIP_OK);
+                fake::launches_until_failure = -1;
+                fake::launch_answer = fake::pending = hipSuccess;
+                fake::stale_flags = 0;
+                if (at % 3 == 0) CHECK(bitnet_hip_decoder_graph_launch(graph, side) == BITNET_HIP_OK);
+                if (at % 3 == 1) CHECK(step(17, out, layers) == BITNET_HIP_OK);
+                CHECK(step(40, other, 1) == BITNET_HIP_OK && step(64, other, layers) == BITNET_HIP_OK);
+                CHECK(fake::stale_flags == 0);
+            }
+        fake::die_launches = 0;
+        CHECK(step(48, other, layers) == BITNET_HIP_OK && fake::die_launches > 0);  // the launches on dies are not given up
+        bitnet_hip_decoder_graph_destroy(graph);
+        bitnet_hip_decoder_destroy(dec);
+    }
 }
 
 // Layers made, loaded and dropped one after the other share the pinned chunks; they are given back once layers come and go unloaded.
@@ -428,6 +522,7 @@ const Check checks[] = {
     {"loads_wait_for_the_stream_once", loads_wait_for_the_stream_once},
     {"steps_worth_a_recording", steps_worth_a_recording},
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
+    {"steps_find_their_flags_down", steps_find_their_flags_down},
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
     {"recorded_calls_on_short_rows", recorded_calls_on_short_rows},
