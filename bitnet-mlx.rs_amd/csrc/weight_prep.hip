@@ -346,9 +346,10 @@ __global__ __launch_bounds__(1024) void absmean_codes_kernel(const float *w, siz
     __syncthreads();
     const float scale = scale_s;
     if (blockIdx.x == 0 && tid == 0) *w_scale = scale;
-    // t > 0, or NaN (every code 0): w > hi, for hi >= 0, is w >= the next float up.
+    // t > 0, or NaN (every code 0): w > hi, for hi >= 0, is w >= the next float up, which is a NaN for an infinite hi.  The next one up of a NaN
+    // whose bits are all ones would be -0.
     const TernaryRule rule = ternary_rule(method, factor, scale);
-    const float t = rule.strict ? __builtin_bit_cast(float, __builtin_bit_cast(int, fabsf(rule.hi)) + 1) : rule.hi;
+    const float t = rule.strict && rule.hi == rule.hi ? __builtin_bit_cast(float, __builtin_bit_cast(unsigned, fabsf(rule.hi)) + 1u) : rule.hi;
     size_t chunk = first;
     for (; chunk + CODES_HELD * stride < chunks; chunk += CODES_HELD * stride) {
 #pragma unroll

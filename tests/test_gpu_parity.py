@@ -121,6 +121,27 @@ def test_quantize_weights_with_row_scratch_bit_exact(n, k, method, factor):
         assert results[0][1][0] == s_ref and np.array_equal(results[0][0], orc.pack_2bit(q_ref))
 
 
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("bits", [0xFFFFFFFF, 0x7FFFFFFF, 0x7FC00000, 0xFFC00001, 0x7F800000, 0xFF800000])
+def test_quantize_weights_with_a_weight_that_is_no_number(bits, method):
+    """A NaN of any payload or an infinity among the weights: with row sums of the caller's the same codes as without, byte for byte."""
+    lib = bh.load_library()
+    rng = np.random.default_rng(bits & 0xFFFF)
+    n, k = 24, 1028
+    w = synth_weights(rng, n, k)
+    w.view(np.uint32)[5, 77] = bits
+    w.view(np.uint32)[23, 1027] = bits
+    w = dev(w)
+    scratch = torch.empty((n,), dtype=torch.float64, device="cuda")
+    results = []
+    for room in (0, 8 * n):
+        packed, scale = torch.full((n * k // 4,), 0xAA, dtype=torch.uint8, device="cuda"), torch.zeros(1, device="cuda")
+        assert lib.bitnet_hip_quantize_weights_with(w.data_ptr(), n, k, method, 0.5, packed.data_ptr(), scale.data_ptr(), None, scratch.data_ptr(), room,
+                                                    torch.cuda.current_stream().cuda_stream) == 0
+        results.append((host(packed), host(scale).view(np.uint32)))
+    assert np.array_equal(results[0][0], results[1][0]) and np.array_equal(results[0][1], results[1][1])
+
+
 def test_quantize_weights_reference_vectors():
     c = G["quantize_batch"]
     w = np.array([c["input"]], dtype=f32)
