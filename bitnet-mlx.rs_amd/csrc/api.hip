@@ -313,7 +313,7 @@ uint64_t next_die_tag()
 DieFlags call_flags(void *ws, size_t m, size_t ldq)
 {
     const uintptr_t at = align_up(reinterpret_cast<uintptr_t>(ws), 256) + quant_scratch_bytes(m, ldq) - 256;
-    return {reinterpret_cast<uint64_t *>(at), nullptr, next_die_tag(), (unsigned)align_up(m, 16), GEMV_DIE_LOOKS};
+    return {reinterpret_cast<uint64_t *>(at), nullptr, 0, next_die_tag(), (unsigned)align_up(m, 16), GEMV_DIE_LOOKS};
 }
 // Whether plain rows go through one launch that quantises them once a die: a call of its own, on a stream that is not being captured
 // (a replay would find the flags of the one before it).
@@ -1141,7 +1141,7 @@ int bitnet_hip_bitlinear_matmul(bitnet_hip_bitlinear *layer, const int8_t *a, co
 // ---------------------------------------------------------------------------------------------------
 // Decoder projections
 // ---------------------------------------------------------------------------------------------------
-constexpr size_t DECODER_MAX_CHAINS = 8;
+constexpr size_t DECODER_MAX_CHAINS = 8, DECODER_FLAG_SETS = 3;
 
 namespace {
 // What the launches of a decode step depend on.
@@ -1184,10 +1184,11 @@ struct bitnet_hip_decoder {
     int32_t *a_sum = nullptr;
     float *qb = nullptr, *kb = nullptr, *vb = nullptr, *x1 = nullptr, *gate = nullptr, *up = nullptr;
     float *ping = nullptr;
-    // Flags of the launches that quantise their rows once a die (gemv_die.hip): two sets used in turn.  Every step finds the first set
+    // Flags of the launches that quantise their rows once a die (gemv_die.hip): three sets (enqueue_step).  Every step finds the first set
     // cleared, recorded steps too, and leaves it so; one that fails half way clears it before it returns, or, where that fails as well, the next
     // step or replay does.
     uint64_t *die_flags = nullptr;
+    uint64_t *die_set(size_t i) const { return die_flags + i * GEMV_DIE_SETS * die_stride(); }
     bool die_flags_dirty = false;
     int die_looks = GEMV_DIE_LOOKS;
     size_t die_stride() const { return align_up(max_tokens < (size_t)GEMV_DIE_MAX_M ? max_tokens : (size_t)GEMV_DIE_MAX_M, 16); }
@@ -1283,7 +1284,7 @@ int bitnet_hip_decoder_create(size_t layers, size_t hidden, size_t ffn, size_t q
     dev_alloc(&d->gate, sizeof(float) * max_tokens * ffn);
     dev_alloc(&d->up, sizeof(float) * max_tokens * ffn);
     dev_alloc(&d->ping, sizeof(float) * max_tokens * hidden);
-    const size_t die_bytes = sizeof(uint64_t) * 2 * GEMV_DIE_SETS * d->die_stride();
+    const size_t die_bytes = sizeof(uint64_t) * DECODER_FLAG_SETS * GEMV_DIE_SETS * d->die_stride();
     dev_alloc(&d->die_flags, die_bytes);
     if (rc == BITNET_HIP_OK) {
         hipError_t e = hipMemset(d->die_flags, 0, die_bytes);
@@ -1388,26 +1389,48 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
     // One chain: rows [row0, row0 + rows) through blocks layer_begin .. layer_end-1 on stream cs, in its own rows of the
     // decoder's activation buffers.
     const size_t widest = padded_k(H > F ? H : F);
-    const size_t chains_asked = dec->chains ? dec->chains : 1;
-    size_t die_launches = 0;
+    size_t chains = dec->chains ? dec->chains : 1;
+    const bool one_chain = chains <= 1;
+    const float *const input_of_block[2] = {x_out, dec->ping};  // of every block but the first, in turn: the last one writes x_out
+    const auto hidden_of = [&](size_t l) { return l == layer_begin ? x_in : input_of_block[(layer_end - l) % 2]; };
+    // Which launch groups quantise their rows once a die, and how many launches of the step do.
+    bitnet_hip_bitlinear **first = &dec->proj[layer_begin * 7];
+    const auto on_dies = [&](int proj, int count, const float *x, const float *x2, size_t ldx, int mode, const float *gamma) {
+        return one_chain && gemv_die_takes(x, x2, ldx, m, first[proj]->in_features, mode, gamma, dec->sum_order,
+                                           launch_group_blocks(&first[proj], (size_t)count), false);
+    };
+    const auto qkv_on_dies = [&](const float *x) { return on_dies(BITNET_HIP_PROJ_Q, 3, x, nullptr, H, BITNET_HIP_INPUT_PLAIN, dec->gamma); };
+    const bool qkv_first = qkv_on_dies(x_in), qkv_other[2] = {qkv_on_dies(x_out), qkv_on_dies(dec->ping)};
+    const bool gate_up_on_dies = on_dies(BITNET_HIP_PROJ_GATE, 2, dec->x1, nullptr, H, BITNET_HIP_INPUT_PLAIN, dec->gamma);
+    const bool down_on_dies = on_dies(BITNET_HIP_PROJ_DOWN, 1, dec->gate, dec->up, F, BITNET_HIP_INPUT_RELU2_MUL, nullptr);
+    const auto qkv_of = [&](size_t l) {
+        if (!(l == layer_begin ? qkv_first : qkv_other[(layer_end - l) % 2])) return false;
+        const float *const wanted[3] = {q_last, k_last, nullptr};  // where the caller's own may lie over the input
+        return l + 1 != layer_end || !(q_last || k_last) ||
+               !writes_over_input(&first[BITNET_HIP_PROJ_Q], 3, hidden_of(l), nullptr, H, m, H, nullptr, wanted);
+    };
+    size_t die_total = (layer_end - layer_begin) * ((size_t)gate_up_on_dies + (size_t)down_on_dies), die_launches = 0;
+    for (size_t l = layer_begin; l < layer_end; ++l) die_total += qkv_of(l);
+    if (die_total == 1) die_total = 0;  // nobody would clear its flags: two launches
     auto run_chain = [&](size_t row0, size_t rows, hipStream_t cs) {
         // one launch group: `count` projections reading the same (transformed) input
         auto run = [&](bitnet_hip_bitlinear *const *layers, int count, const float *x, const float *x2, size_t ldx, int mode,
-                       const float *gamma, const float *res0, float *const *outs) {
+                       const float *gamma, const float *res0, float *const *outs, bool die) {
             if (rc != BITNET_HIP_OK) return;
+            // Launches use sets 0 and 1 in turn, the last of an odd number set 2.  The first one clears sets 1 and 2, which the step before may
+            // have left up, each other one the set of the launch before it: set 0 is down again at the end.
             DieFlags flags;
-            const bool on_dies = chains_asked <= 1 &&
-                                 !writes_over_input(layers, (size_t)count, x, x2, ldx, rows, layers[0]->in_features, gamma, outs) &&
-                                 gemv_die_takes(x, x2, ldx, rows, layers[0]->in_features, mode, gamma, dec->sum_order, launch_group_blocks(layers, (size_t)count), false);
-            if (on_dies) {
-                uint64_t *sets[2] = {dec->die_flags, dec->die_flags + GEMV_DIE_SETS * dec->die_stride()};
-                flags = {sets[die_launches & 1], sets[~die_launches & 1], 1, (unsigned)dec->die_stride(), dec->die_looks};
-                ++die_launches;
+            die = die && die_total;
+            if (die) {
+                const size_t at = die_launches++;
+                const bool alone_in_its_set = at + 1 == die_total && at % 2 == 0;
+                flags = {dec->die_set(alone_in_its_set ? 2 : at % 2), dec->die_set(at ? (at - 1) % 2 : 1), at ? 1u : 2u, 1, (unsigned)dec->die_stride(),
+                         dec->die_looks};
             }
             const float *res[GEMV_MAX_PROJ] = {res0, nullptr, nullptr};
             rc = run_projections(layers, count, x, x2, ldx, rows, mode, group, dec->head_dim, gamma, dec->eps, dec->sum_order,
                                  res, outs, nullptr, dec->a8 + row0 * widest, padded_k(layers[0]->in_features), dec->a_scale + row0,
-                                 dec->a_sum + row0, false, cs, false, on_dies ? &flags : nullptr);
+                                 dec->a_sum + row0, false, cs, false, die ? &flags : nullptr);
         };
         float *qb = dec->qb + row0 * H, *kb = dec->kb + row0 * KV, *vb = dec->vb + row0 * KV, *x1 = dec->x1 + row0 * H;
         float *gate = dec->gate + row0 * F, *up = dec->up + row0 * F, *ping = dec->ping + row0 * H;
@@ -1420,22 +1443,20 @@ static int enqueue_step(bitnet_hip_decoder *dec, const StepKey &step, hipStream_
             // hidden states alternate between x_out and the internal buffer so that the last block writes x_out
             float *x2 = ((layer_end - 1 - l) % 2 == 0) ? xo : ping;
             float *qkv_out[3] = {(last && q_last) ? q_last + row0 * H : qb, (last && k_last) ? k_last + row0 * KV : kb, vb};
-            run(&P[BITNET_HIP_PROJ_Q], 3, x, nullptr, H, BITNET_HIP_INPUT_PLAIN, g_attn, nullptr, qkv_out);
+            run(&P[BITNET_HIP_PROJ_Q], 3, x, nullptr, H, BITNET_HIP_INPUT_PLAIN, g_attn, nullptr, qkv_out, qkv_of(l));
             float *o_out[1] = {x1};
-            run(&P[BITNET_HIP_PROJ_O], 1, vb, nullptr, KV, BITNET_HIP_INPUT_GQA_BROADCAST, nullptr, x, o_out);
+            run(&P[BITNET_HIP_PROJ_O], 1, vb, nullptr, KV, BITNET_HIP_INPUT_GQA_BROADCAST, nullptr, x, o_out, false);
             float *gu_out[2] = {gate, up};
-            run(&P[BITNET_HIP_PROJ_GATE], 2, x1, nullptr, H, BITNET_HIP_INPUT_PLAIN, g_ffn, nullptr, gu_out);
+            run(&P[BITNET_HIP_PROJ_GATE], 2, x1, nullptr, H, BITNET_HIP_INPUT_PLAIN, g_ffn, nullptr, gu_out, gate_up_on_dies);
             float *d_out[1] = {x2};
-            run(&P[BITNET_HIP_PROJ_DOWN], 1, gate, up, F, BITNET_HIP_INPUT_RELU2_MUL, nullptr, x1, d_out);
+            run(&P[BITNET_HIP_PROJ_DOWN], 1, gate, up, F, BITNET_HIP_INPUT_RELU2_MUL, nullptr, x1, d_out, down_on_dies);
             x = x2;
         }
     };
-    size_t chains = chains_asked;
     if (chains > m) chains = m;
     if (chains > dec->max_tokens) chains = dec->max_tokens;  // side streams exist for min(max_tokens, 8) chains
     if (chains <= 1) {
         run_chain(0, m, s);
-        if (rc == BITNET_HIP_OK && (die_launches & 1)) rc = launch_clear_die_flags(dec->die_flags, dec->die_stride(), m, s);
         if (rc != BITNET_HIP_OK && die_launches && launch_clear_die_flags(dec->die_flags, dec->die_stride(), dec->die_stride(), s) != BITNET_HIP_OK)
             dec->die_flags_dirty = true;
     } else {
@@ -1732,7 +1753,7 @@ size_t decoder_device_bytes(const bitnet_hip_decoder *d)
     const size_t kv = d->kv_heads * d->head_dim, widest = padded_k(d->hidden > d->ffn ? d->hidden : d->ffn), t = d->max_tokens;
     total += sizeof(float) * d->layers * 2 * d->hidden;                                        // norms
     total += t * widest + 2 * sizeof(float) * t;                                               // a8, a_scale, a_sum
-    total += sizeof(uint64_t) * 2 * GEMV_DIE_SETS * d->die_stride();                                     // die_flags
+    total += sizeof(uint64_t) * DECODER_FLAG_SETS * GEMV_DIE_SETS * d->die_stride();           // die_flags
     total += sizeof(float) * t * (d->hidden /*q*/ + 2 * kv + d->hidden /*x1*/ + 2 * d->ffn + d->hidden /*ping*/);
     return total;
 }

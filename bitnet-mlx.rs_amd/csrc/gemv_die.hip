@@ -27,8 +27,8 @@
 // only the time does.
 //
 // Flags hold 64-bit tags.  Before a launch none of the flags that it looks at may hold its tag: a call of its own takes a tag that no other
-// launch has; a decoder, whose steps are replayed with the same arguments, passes two sets of flags in turn and tag 1, and every launch
-// clears the set of the launch before it.
+// launch has; a decoder, whose steps are replayed with the same arguments, passes sets of flags in turn and tag 1, and a launch clears the set
+// of the launch before it (enqueue_step says which).
 #include "rowsgemv.hpp"
 
 namespace bitnet {
@@ -45,7 +45,8 @@ struct DieParams {
     unsigned stride;                  // flags of a die
     int looks;
     float eps;
-    unsigned blocks01, blocks2, unused;  // row blocks of projections 0 and 1 (16 bits each), and of 2
+    unsigned blocks01, blocks2;          // row blocks of projections 0 and 1 (16 bits each), and of 2
+    unsigned clear_halves;               // eights of dies whose flags start at clear
 };
 static_assert(sizeof(DieParams) == 64 * (1 + GEMV_MAX_PROJ), "one scalar load a block");
 constexpr int DIE_ARGS_AT = 56;  // its offset in the argument buffer: three pointers and seven 4-byte arguments before it, aligned to eight
@@ -171,9 +172,9 @@ __global__ __launch_bounds__(1024) void gemv_die_kernel(const float *hot_x, cons
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // in L2
         lds_barrier();
         if (tid == 0) d.flags[die * d.stride + row] = d.tag;
-        if (local == 0 && d.clear) {  // both halves of the numbers a die can have
-            for (int i = tid; i < 2 * m; i += 64 * nw) d.clear[(slot + 8 * (i >= m)) * d.stride + (i >= m ? i - m : i)] = 0;
-        }
+        if (local == 0)
+            for (unsigned half = 0; half < C[15]; ++half)
+                for (int i = tid; i < m; i += 64 * nw) d.clear[(slot + 8 * half) * d.stride + i] = 0;
         return;
     }
 
@@ -357,7 +358,7 @@ int launch_gemv_die(const GemvProj *projs, int nproj, const float *x, const floa
     l.quantisers_tgroups = (unsigned)m | ((unsigned)tgroups << 16);
     l.tg_magic = (unsigned)((((uint64_t)1 << 32) + tgroups - 1) / tgroups);  // not used for one group
     l.p.q = reinterpret_cast<uint8_t *>(q); l.p.a_scale = a_scale; l.p.eps = eps;
-    l.p.flags = f.flags; l.p.clear = f.clear; l.p.tag = f.tag; l.p.stride = f.stride; l.p.looks = f.looks;
+    l.p.flags = f.flags; l.p.clear = f.clear; l.p.clear_halves = f.clear ? (unsigned)(f.clear_sets * GEMV_DIE_SETS / 8) : 0; l.p.tag = f.tag; l.p.stride = f.stride; l.p.looks = f.looks;
     l.p.blocks01 = counts[0] | (counts[1] << 16);
     l.p.blocks2 = counts[2];
     if (input_mode == BITNET_HIP_INPUT_RELU2_MUL) return launch_shape<BITNET_HIP_INPUT_RELU2_MUL, false>(l, shape.rb, shape.nt);

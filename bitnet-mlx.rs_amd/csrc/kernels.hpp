@@ -148,13 +148,14 @@ bool gemv_rowq_takes(const float *x, size_t ldx, size_t m, size_t k, int input_m
 int launch_gemv_rowq(const GemvProj *projs, int nproj, const float *x, size_t m, size_t k, int input_mode, size_t gqa_group, size_t head_dim,
                      const float *gamma, float eps, hipStream_t stream);
 // gemv_die.hip: several tokens in one launch, their rows quantised once on every die.  Only where gemv_die_takes() says so.
-// flags: 16 dies x stride 64-bit words, none of which holds tag before the launch; clear (optional): a second set of them, cleared for the
-// m rows by the launch; looks: how often a workgroup looks at the flags before it quantises its rows itself.
+// flags: 16 dies x stride 64-bit words, none of which holds tag before the launch; clear (optional): clear_sets other sets of them, one behind
+// the other, cleared for the m rows by the launch; looks: how often a workgroup looks at the flags before it quantises its rows itself.
 constexpr int GEMV_DIE_MAX_M = 128;
 constexpr size_t GEMV_DIE_SETS = 16;  // dies whose flags are kept apart
 constexpr int GEMV_DIE_LOOKS = 4096;
 struct DieFlags {
     uint64_t *flags, *clear;
+    unsigned clear_sets;
     uint64_t tag;
     unsigned stride;
     int looks;
