@@ -270,6 +270,8 @@ int launch_shape(const Launch &l, int rb, int nt)
 
 namespace {
 
+constexpr size_t DIE_CUS = 32;  // compute units of a die
+
 // Row blocks and k-tiles as in launch_gemv_rows, and the workgroups of a die.
 struct Shape {
     int rb, nt, nw;
@@ -288,7 +290,7 @@ Shape shape_of(size_t m, size_t k, size_t blocks)
     s.multipliers = ((blocks + s.rb - 1) / s.rb + 7) / 8 * tgroups;
     // wavefronts of a compute unit by the kernel's registers: up to 64 with one tile a wavefront; 70, and 90 to 92, with two
     const size_t waves = s.nt == 1 ? 32 : (s.rb == 1 ? 28 : 20);
-    s.slots = 32 * (waves / (size_t)s.nw);
+    s.slots = DIE_CUS * (waves / (size_t)s.nw);
     return s;
 }
 
@@ -307,10 +309,14 @@ bool gemv_die_takes(const float *x, const float *x2, size_t ldx, size_t m, size_
     // Up to eight tokens gemv_fused16_kernel may be one launch as well, which pays while its workgroups have few tiles to walk, and in a call of
     // its own, which takes as long as the host's launch, always (4.4 us against 4.8).  A decoder block with this kernel where that one's
     // workgroups walk 24 to 44 tiles: 0.1 to 1.1 us slower; 48: 0.6 faster to 0.1 slower; 64: 0.2 to 0.7 faster, but at two tokens 0.1 faster to
-    // 0.4 slower; 80 and more: 0.2 to 2.4 faster.
+    // 0.4 slower; 80 and more: 0.2 to 2.4 faster.  At two tokens there is little to gain, and it is lost where that kernel has a workgroup for
+    // every compute unit and the two that quantise are one too many: blocks of 2560 to 4096 columns with gate + up of 30 multiplying workgroups a
+    // die 0.0 to 0.6 us faster, of 31 and 32 0.4 faster to 0.8 slower, of 33 0.1 to 1.3 faster.
     if (gemv_fused_supported(x, x2, ldx, m, k, input_mode, 1, gamma, sum_order, blocks)) {
         const size_t tiles = gemv_fused_tiles(m, k, blocks);
-        return !alone && (tiles >= 80 || (tiles >= 64 && m > 2));
+        if (alone || tiles < (m > 2 ? 64 : 80)) return false;
+        const Shape s = shape_of(m, k, blocks);
+        return m > 2 || s.multipliers > DIE_CUS || s.quantisers + s.multipliers <= DIE_CUS;
     }
     // Otherwise the other choice is two launches, and what decides is whether the workgroups of a die run at once: those that multiply
     // are to be there when the rows are, and a second round of them waits for the first.  Decoder blocks of 512 to 4096 columns at 9 to 64
@@ -326,7 +332,7 @@ bool gemv_die_takes(const float *x, const float *x2, size_t ldx, size_t m, size_
     // 12.7 -> 13.1, 13.6 -> 14.0; long rows of many tokens, whose quantisers fill the die: 8192 -> 640 at 48 7.8 -> 7.3, 8.0 -> 9.2, at 64
     // 7.8 -> 8.2, 8.2 -> 10.1.
     if (s.nt == 2 && m > (gamma ? 32u : 48u)) return false;
-    return 20 * total <= (s.slots == 32 ? 33 : (gamma ? 23 : 28)) * s.slots;
+    return 20 * total <= (s.slots == DIE_CUS ? 33 : (gamma ? 23 : 28)) * s.slots;
 }
 
 int launch_gemv_die(const GemvProj *projs, int nproj, const float *x, const float *x2, size_t ldx, size_t m, size_t k, int input_mode, const float *gamma,

@@ -418,6 +418,25 @@ void steps_find_their_flags_down()
     }
 }
 
+// At two tokens gate and up are quantised on the dies unless the launch without that has just a workgroup for every compute unit.
+void two_tokens_on_dies()
+{
+    const struct {
+        size_t ffn;
+        bool taken;
+    } steps[] = {{6912, true}, {7680, true}, {7936, false}, {8192, false}, {8448, true}};
+    for (const auto &t : steps) {
+        bitnet_hip_decoder *dec = decoder_with_weights(2, 2560, t.ffn);
+        std::vector<float> x(2 * 2560), out(2 * 2560);
+        fake::die_launches = 0;
+        CHECK(bitnet_hip_decoder_decode(dec, x.data(), 2, out.data(), nullptr, nullptr, side) == BITNET_HIP_OK);
+        CHECK(fake::die_launches == (t.taken ? 2 : 0));
+        CHECK(bitnet_hip_decoder_decode_layers(dec, 0, 1, x.data(), 2, out.data(), nullptr, nullptr, side) == BITNET_HIP_OK);
+        CHECK(fake::die_launches == (t.taken ? 2 : 0));  // one alone has no other launch to clear its flags
+        bitnet_hip_decoder_destroy(dec);
+    }
+}
+
 // Layers made, loaded and dropped one after the other share the pinned chunks; they are given back once layers come and go unloaded.
 void chunks_outlive_a_layer_that_used_them()
 {
@@ -527,6 +546,7 @@ const Check checks[] = {
     {"steps_worth_a_recording", steps_worth_a_recording},
     {"recording_a_step_leaves_other_captures_alone", recording_a_step_leaves_other_captures_alone},
     {"steps_find_their_flags_down", steps_find_their_flags_down},
+    {"two_tokens_on_dies", two_tokens_on_dies},
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
     {"recorded_calls_on_short_rows", recorded_calls_on_short_rows},
