@@ -101,9 +101,9 @@ __device__ __forceinline__ void normalize_row(float4 (&v)[NCH], const float4 (&g
 }
 
 // One wavefront per row of at most 256 NCH columns: NCH (two or four) chunks a lane, no barriers.  (A workgroup per row leaves most of its
-// threads without a chunk there.)  With a norm, as below: 65536 x 1024 67.8 -> 59.9 us, 16384 x 1024 18.5 -> 16.0; two chunks where they do: 65536 x 512
-// 33.1 -> 29.1 (36.3 with four).
-template <int MODE, bool VEC, bool NORM, int NCH>
+// threads without a chunk there.)  HELD as HELD_NORM below: 65536 x 1024 67.8 -> 59.9 us, 16384 x 1024 18.3 -> 16.1; two chunks where they do: 65536 x
+// 512 33.1 -> 29.1 (36.3 with four).
+template <int MODE, bool VEC, bool NORM, int NCH, bool HELD>
 __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 {
     const RowSource &src = p.src;
@@ -119,8 +119,8 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
         v[i] = c < chunks ? load_chunk<MODE, VEC>(src, row, c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if constexpr (NORM) {
-        float4 gm[VEC ? NCH : 1];
-        if constexpr (VEC) {
+        float4 gm[HELD ? NCH : 1];
+        if constexpr (HELD) {
 #pragma unroll
             for (int i = 0; i < NCH; ++i) gm[i] = lane + 64 * i < chunks ? load_gamma_chunk(src, lane + 64 * i, VEC) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -135,9 +135,9 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
             ss = f32_add(f32_add(f32_add(part[0], part[1]), part[2]), part[3]);
         }
         const Divisor rdiv = make_divisor(rms_from_ss(ss, src.k, src.eps));
-        if constexpr (VEC) {
+        if constexpr (HELD) {
             normalize_row(v, gm, rdiv, lane, 64, chunks);
-        } else {  // a load per weight: behind the sum they overlap other rows (4776 x 691 in front of it: 0.9 us more)
+        } else {  // unaligned weights too: behind the sum they overlap other rows (4776 x 691 in front of it: 0.9 us more)
 #pragma unroll
             for (int i = 0; i < NCH; ++i)
                 if (lane + 64 * i < chunks) v[i] = normalize4(v[i], rdiv, load_gamma_chunk(src, lane + 64 * i, VEC));
@@ -168,7 +168,8 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(ActQuantParams p)
 // workgroups that take rows in turn and fetch the next one early are slower: 15.8 us against 12.7 us at 2048 x 6912.)
 // HELD_NORM: a norm in the declared order, whose weights are asked for with the row and not behind its sum of squares, and whose chunks are divided
 // together; NCH is then exactly what a row takes, since every chunk's weights take registers too.  With a norm, before -> now (without one), us:
-// (above 14336 columns the registers of a workgroup with held weights leave a compute unit two: 2048 x 16384 37.1 -> 39.4, not taken)
+// (above 14336 columns the registers of a workgroup with held weights leave a compute unit two: 2048 x 16384 37.1 -> 39.4, not taken; fewer rows:
+// held_norm_from)
 // 6000 x 12288 85 -> 69 (64.5), 2048 x 10240 25.9 -> 21.7 (16.3), 4096 x 5120 21.6 -> 17.9 (17.0), 4096 x 4096 18.5 -> 15.2 (14.0), 8192 x 2560 20.3 -> 18.6 (16.4), 2048 x 6912 16.7 -> 15.2 (12.5).
 template <int MODE, int NCH, bool VEC, bool HELD_NORM>
 __global__ __launch_bounds__(256) void act_quant_block_kernel(ActQuantParams p)
@@ -338,6 +339,8 @@ __global__ __launch_bounds__(1024) void act_quant_row_kernel(const float *hot_x,
     }
 }
 
+size_t row_bytes(const ActQuantParams &p) { return p.m * (size_t)p.src.k * sizeof(float); }
+
 template <int MODE, bool VEC>
 void launch_wave(const ActQuantParams &p, hipStream_t s)
 {
@@ -345,10 +348,17 @@ void launch_wave(const ActQuantParams &p, hipStream_t s)
     dim3 block(64, rows_per_block);
     dim3 grid((unsigned)((p.m + rows_per_block - 1) / rows_per_block));
     const bool two = p.src.k <= 512 && p.ldq <= 512;  // the padding is cleared by the same lanes
-    if (p.src.gamma && two) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 2>), grid, block, 0, s, p);
-    else if (p.src.gamma) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 4>), grid, block, 0, s, p);
-    else if (two) launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 2>), grid, block, 0, s, p);
-    else launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 4>), grid, block, 0, s, p);
+    // Two chunks and their weights take few registers: held, 1.07 to 1.12 times as fast from 513 rows to 65536.  Four: where the rows come from
+    // beyond the L2s (32 MB) a row's chain is what counts, and where all of them run at once (12000 x 1024 14.8 -> 13.2 us, 1024 x 1024 4.14 ->
+    // 3.99); between, more wavefronts of fewer registers are the faster (2048 x 640 4.30 held, 3.95 not; 4096 x 1024 5.93 and 5.68; 12000 x 768 11.4
+    // and 11.3; 1024 x 516 3.98 and 3.87).
+    const bool held = VEC && (two || row_bytes(p) > ((size_t)40 << 20) || (p.m <= 1024 && p.src.k > 768));
+    if (p.src.gamma && two && held) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 2, VEC>), grid, block, 0, s, p);
+    else if (p.src.gamma && held) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 4, VEC>), grid, block, 0, s, p);
+    else if (p.src.gamma && two) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 2, false>), grid, block, 0, s, p);
+    else if (p.src.gamma) launch_kernel((act_quant_wave_kernel<MODE, VEC, true, 4, false>), grid, block, 0, s, p);
+    else if (two) launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 2, false>), grid, block, 0, s, p);
+    else launch_kernel((act_quant_wave_kernel<MODE, VEC, false, 4, false>), grid, block, 0, s, p);
 }
 
 // LDS for the row's squares where the literal summation order is asked for and a row fits the default limit
@@ -367,6 +377,26 @@ void launch_block(ActQuantParams p, hipStream_t s)
     launch_kernel((act_quant_block_kernel<MODE, NCH, VEC, false>), dim3((unsigned)p.m), dim3(256), lds, s, p);
 }
 
+// From how many bytes of rows on the 256-thread kernel holds the norm's weights, by chunks a thread.  Beyond the L2s (32 MB) a row's chain waits for
+// memory, and one trip less counts; rows that lie there are the faster the more of them a compute unit holds.  us, not held -> held, around the line:
+// 2560 x 2560 7.61 -> 7.67, 4096 x 2560 12.3 -> 11.3; 1280 x 5120 7.30 -> 7.35, 1792 x 5120 10.9 -> 9.8; 1280 x 6912 10.16 -> 10.35, 1536 x 6912 13.2 -> 12.7;
+// 1792 x 8192 15.5 (16 wavefronts a row) -> 16.0, 2560 x 8192 20.6 -> 20.0; 1024 x 8448 10.9 -> 11.7; 600 x 12288 9.9 -> 10.9, 768 x 12288 12.8 ->
+// 11.7; 1280 x 13824 23.4 -> 23.8, 1536 x 13824 26.5 -> 25.7.  Two and four chunks: at any size, 1.02 to 1.2 times as fast, since the other kernel
+// has registers for three, seven and sixteen.
+size_t held_norm_from(int per_thread)
+{
+    constexpr size_t MB = (size_t)1 << 20;
+    switch (per_thread) {
+        case 3: case 5: case 6: return 29 * MB;
+        case 7: return 36 * MB;
+        case 8: return 60 * MB;
+        case 9: case 10: case 11: return 39 * MB;
+        case 12: return 32 * MB;
+        case 13: case 14: return 72 * MB;
+        default: return 0;
+    }
+}
+
 template <int MODE, int NCH>
 void launch_block_norm(const ActQuantParams &p, hipStream_t s)
 {
@@ -379,11 +409,14 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
     const int chunks = (p.src.k + 3) >> 2;
     // Rows that all run at once: up to 16 wavefronts per row, with four chunks a thread above 8192 columns (213 rows of 13120 columns
     // with norm: 9.8 us in the 256-thread kernel -> 5.6 here; a decoder block with a 13824-wide FFN at 8 tokens: 36.3 -> 31.5).  Rows
-    // that come in many rounds are here from 7168 columns on without a norm; with one they stay with the 256-thread kernel, of which a compute
-    // unit holds more (8192 x 8192 73.0 us here, 62.2 there, 4096 x 7680 33.1 and 27.0, 6000 x 12288 115 and 69).
+    // that come in many rounds are here from 7168 columns on without a norm, and up to 8192 with one as long as the 256-thread kernel does not
+    // hold its weights; that is otherwise the faster, since a compute unit holds more of its rows (8192 x 8192 73.0 us here, 62.2 there, 4096 x 7680
+    // 33.1 and 27.0, 6000 x 12288 115 and 69).
     const bool ordered = !p.src.gamma || p.src.sum_order == BITNET_HIP_SUM_BLOCK256;
     const bool few = p.m <= ROW_QUANT_MAX_ROWS;
-    if ((few || (chunks > 1792 && !p.src.gamma)) && vec && ordered && chunks <= 4096 && p.src.ldx < (1u << 31)) {
+    const int per_thread = (chunks + 255) >> 8;
+    const bool held = vec && p.src.gamma && ordered && per_thread <= 14 && row_bytes(p) >= held_norm_from(per_thread);
+    if ((few || (chunks > 1792 && (!p.src.gamma || (chunks <= 2048 && !held)))) && vec && ordered && chunks <= 4096 && p.src.ldx < (1u << 31)) {
         const float *x2 = p.src.x2;
         uint64_t magics = 0;
         bool in_range = true;
@@ -411,8 +444,7 @@ void launch_mode(const ActQuantParams &p, bool vec, hipStream_t s)
         }
     }
     if (p.m > 32 && chunks <= 256) return vec ? launch_wave<MODE, true>(p, s) : launch_wave<MODE, false>(p, s);
-    const int per_thread = (chunks + 255) >> 8;
-    if (vec && p.src.gamma && ordered && per_thread <= 14) {
+    if (held) {
         switch (per_thread) {
             case 1: return launch_block_norm<MODE, 1>(p, s);
             case 2: return launch_block_norm<MODE, 2>(p, s);

@@ -373,6 +373,13 @@ def test_activation_quant_with_a_norm_bit_exact(m, k):
     assert np.array_equal(host(s), s_ref) and np.array_equal(host(q), q_ref) and np.array_equal(host(asum), sum_ref)
 
 
+@pytest.mark.parametrize("m,k", [(3100, 2564), (1500, 5124), (1300, 6148), (1400, 6916), (2000, 7940), (1150, 8708), (1080, 9980), (1000, 10500), (700, 12284), (1350, 14332),
+                                 (1000, 1020), (1100, 1020), (17000, 644), (1030, 512)])
+def test_activation_quant_with_a_norm_held_bit_exact(m, k):
+    """As many rows as it takes for a workgroup, or a wavefront, to hold the norm's weights, at each count of chunks a thread (the sizes above have fewer)."""
+    test_activation_quant_with_a_norm_bit_exact(m, k)
+
+
 @pytest.mark.parametrize("m,k", [(33, 1), (33, 2), (33, 3), (40, 5), (40, 6), (40, 7), (35, 509), (35, 1021), (35, 1022), (35, 1023), (600, 1029), (600, 1030), (600, 1031),
                                  (5, 2561), (520, 5121), (513, 7169), (514, 9898), (20, 16385), (513, 16387)])
 @pytest.mark.parametrize("how", ["plain", "norm", "gated", "shifted"])
