@@ -281,13 +281,20 @@ __global__ __launch_bounds__(256) void ternarize_pack_kernel(const float *w, siz
 // absmean_final_kernel and ternarize_pack_kernel in one launch, for row sums that are not where the codes go: the first wavefront of every
 // workgroup adds the row sums up (lane l rows l, l+64, ..., then the butterfly, as there) while the first weights of the other 15 are on
 // their way.  These have CODES_HELD chunks of 1024 weights each in registers, which is a matrix of 79 MB; of a larger one the next chunk is
-// asked for where one has been used.  Bound by the read of the matrix, the second one.  A call, with the three launches -> with two:
-// 6912 x 2560 27.8 -> 24.9 us (the codes 9.5 behind 3.8 for the sum and a launch, 11.3 now), 4096 x 5120 30.6 -> 27.9, 14336 x 8192 176 -> 174,
-// 2048 x 2048 11.3 -> 9.1, 256 x 512 11.6 -> 9.3 (the host's launches).  With all wavefronts bringing the row sums into LDS ahead of their
-// weights 26.7; the whole quantiser in one launch whose workgroups wait for each other's row sums with the matrix in registers takes 22.1, but
+// asked for where one has been used.  Bound by the read of the matrix, the second one, and up to 32 MB of weights, which the dies' L2s hold, by the
+// sum's way through one wavefront.  A call, with the three launches -> with two:
+// 6912 x 2560 27.6 -> 23.8 us, 4096 x 4096 27.2 -> 22.2, 4096 x 2560 18.6 -> 11.9, 4096 x 2048 16.6 -> 9.6, 14336 x 4096 77.6 -> 73.1, 256 x 512 8.1 ->
+// 6.9 (the host's launches).  Without the dies' shares, with every chunk on any die: 4096 x 2048 13.6, 6144 x 1024 13.1 (9.5 with, 10.6
+// in three launches, whose two passes went over 1024 columns in the same order); beyond 84 MB the shares only spread the reads: 14336 x 4096 72.9
+// without, 75.2 with, 6144 x 4096 33.6 and 34.2.  A workgroup has 15 chunks where there are so few: as many workgroups as compute units are no faster
+// (1024 x 1024 7.2 and 7.3 us) and keep other launches out (on three streams at once 4.7 and 3.4 us a call).  Beside two more streams of the same
+// calls matrices of few columns are still slower than in three launches, whose first two leave room: 14336 x 256 8.5 -> 11.7 (alone 13.9 -> 12.2),
+// 8192 x 768 9.4 -> 10.9 (16.3 -> 10.4), 2560 x 2560 and larger even.  With all wavefronts bringing the row sums into LDS ahead of their weights 2 us
+// more; the whole quantiser in one launch whose workgroups wait for each other's row sums with the matrix in registers takes 22.1 for 6912 x 2560, but
 // two to four such launches on streams of their own keep each other off the compute units: 48 us a call in place of 23.
 constexpr int CODES_HELD = 5, CODES_SUMS = 36;  // chunks and rows of 64 row sums on their way to a wavefront
 constexpr size_t CODES_MAX_ROWS = 65536;        // beyond, every workgroup reading all row sums is what takes the time
+constexpr size_t CODES_SHARED = 21000000;       // weights up to which a die reads its own rows again
 
 // The codes of 1024 consecutive weights, a float4 of each 256 a lane: lane l of a quad ends with the dword of the quad's group l, as above.
 __device__ __forceinline__ void codes_of_chunk(const float4 (&v)[4], float t, uint8_t *packed, size_t chunk, int lane)
@@ -316,6 +323,15 @@ __global__ __launch_bounds__(1024) void absmean_codes_kernel(const float *w, siz
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t chunks = n * k / 1024, stride = (size_t)gridDim.x * 15;
     size_t first = (size_t)(wave - 1) * gridDim.x + blockIdx.x;  // as many for every workgroup
+    // A workgroup runs on the die of its number modulo eight, here and in absmean_rows_kernel, where it has four rows.  Where those are whole
+    // chunks, the chunks are dealt out so that a die reads again what it has read, from its own L2: groups of eight times `share` chunks.
+    const unsigned share = k % 256 == 0 && n * k <= CODES_SHARED ? (unsigned)(k / 256) : 1, group_chunks = 8 * share;
+    const unsigned grouped = share > 1 ? (unsigned)chunks / group_chunks * group_chunks : 0;
+    const auto chunk_of = [&](size_t turn) -> size_t {
+        if (turn >= grouped) return turn;
+        const unsigned group = (unsigned)turn / group_chunks, at = (unsigned)turn - group * group_chunks;
+        return group * group_chunks + (at & 7) * share + (at >> 3);
+    };
     float4 v[CODES_HELD][4];
     const auto load = [&](float4 (&to)[4], size_t chunk) {  // zeros past the last one: no branch, so that each chunk is waited for by itself
         const __amdgpu_buffer_rsrc_t of = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(w + chunk * 1024), 0, chunk < chunks ? 4096 : 0, 0x00020000);
@@ -341,7 +357,7 @@ __global__ __launch_bounds__(1024) void absmean_codes_kernel(const float *w, siz
         first = chunks;
     } else {
 #pragma unroll
-        for (int h = 0; h < CODES_HELD; ++h) load(v[h], first + h * stride);
+        for (int h = 0; h < CODES_HELD; ++h) load(v[h], chunk_of(first + h * stride));
     }
     __syncthreads();
     const float scale = scale_s;
@@ -354,13 +370,13 @@ __global__ __launch_bounds__(1024) void absmean_codes_kernel(const float *w, siz
     for (; chunk + CODES_HELD * stride < chunks; chunk += CODES_HELD * stride) {
 #pragma unroll
         for (int h = 0; h < CODES_HELD; ++h) {
-            codes_of_chunk(v[h], t, packed, chunk + h * stride, lane);
-            load(v[h], chunk + (h + CODES_HELD) * stride);
+            codes_of_chunk(v[h], t, packed, chunk_of(chunk + h * stride), lane);
+            load(v[h], chunk_of(chunk + (h + CODES_HELD) * stride));
         }
     }
 #pragma unroll
     for (int h = 0; h < CODES_HELD; ++h)
-        if (chunk + h * stride < chunks) codes_of_chunk(v[h], t, packed, chunk + h * stride, lane);
+        if (chunk + h * stride < chunks) codes_of_chunk(v[h], t, packed, chunk_of(chunk + h * stride), lane);
     if (blockIdx.x == gridDim.x - 1 && wave == 15) ternarize_bytes(w, chunks * 1024, n * k, rule, packed, nullptr, lane);
 }
 
@@ -930,7 +946,7 @@ int launch_quantize_weights(const float *w, size_t n, size_t k, int method, floa
     const bool dense = aligned(w, 16) && aligned(packed, 4) && (!q_i8 || aligned(q_i8, 4));
     // No int8 codes, and a threshold that is not negative (what the sign of a difference can tell).
     if (apart && count != 0 && n <= CODES_MAX_ROWS && dense && !q_i8 && (method == BITNET_HIP_TERNARY_ABSMEAN_ROUNDCLIP || threshold_factor >= 0.0f)) {
-        const unsigned blocks = blocks_for(count, 2048);  // two wavefronts with a chunk each, up to a workgroup a compute unit
+        const unsigned blocks = (blocks_for(count, 15 * 1024) + 7) / 8 * 8;  // a chunk a wavefront, up to a workgroup a compute unit
         launch_kernel(absmean_codes_kernel, dim3(blocks < 256 ? blocks : 256), dim3(1024), 0, stream, w, n, k, method, threshold_factor,
                       const_cast<const double *>(row_sums), packed, w_scale);
         BITNET_HIP_CHECK_LAUNCH("absmean_codes_kernel");

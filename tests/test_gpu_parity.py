@@ -121,6 +121,13 @@ def test_quantize_weights_with_row_scratch_bit_exact(n, k, method, factor):
         assert results[0][1][0] == s_ref and np.array_equal(results[0][0], orc.pack_2bit(q_ref))
 
 
+@pytest.mark.parametrize("n,k", [(3, 256), (37, 768), (129, 512), (700, 2560), (33, 8192), (4099, 1024), (4000, 5120), (5130, 4096)])
+def test_quantize_weights_of_whole_chunks_bit_exact(n, k):
+    """Rows that are a quarter of whole chunks: the chunks dealt out by the die that read them, the last ones in order, up to 21 million weights and above."""
+    for method, factor in ((0, 0.5), (1, 0.7)):
+        test_quantize_weights_with_row_scratch_bit_exact(n, k, method, factor)
+
+
 @pytest.mark.parametrize("method", [0, 1])
 @pytest.mark.parametrize("bits", [0xFFFFFFFF, 0x7FFFFFFF, 0x7FC00000, 0xFFC00001, 0x7F800000, 0xFF800000])
 def test_quantize_weights_with_a_weight_that_is_no_number(bits, method):
