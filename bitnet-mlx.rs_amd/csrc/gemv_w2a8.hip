@@ -478,7 +478,7 @@ __global__ __launch_bounds__(1024) void gemv_fused16_kernel(const float *hot_x, 
     // The loads that need no argument but the preloaded ones, unconditional (clamped indices, values discarded).
     const int in_tile = 16 * ((lane >> 2) & 3) + 4 * (lane >> 4) + (lane & 3);
     Row16<NORM, NCHB> row16;
-    row16.template load<MODE>(row, row2, magics, hot_head_chunks, hot_gamma, chunks, nw, wave, tid, in_tile);
+    row16.template load<MODE, (RBW > 1)>(row, row2, magics, hot_head_chunks, hot_gamma, chunks, nw, wave, tid, in_tile);
     __builtin_amdgcn_sched_barrier(0);
 
     // The other arguments, all at once, and pinned here.  Which projection a workgroup serves it knows from the preloaded

@@ -404,10 +404,11 @@ struct Row16 {
     float4 v[NCHB], gm[NORM ? NCHB : 1], vs[NSS];
     int chunk[NCHB];
 
-    // Unconditional loads (clamped indices, values discarded), also of the chunks that no virtual lane of a row this short has: a branch for
-    // each costs the kernels that do little else more than the loads (the 30-block stack at 4 / 16 / 42 tokens 668 / 808 / 989 us, 666 / 803 / 986
-    // without; one token even).
-    template <int MODE>
+    // Unconditional loads (clamped indices, values discarded).  ALL: also of the chunks that no virtual lane of a row this short has.  A branch for
+    // each costs most kernels more than the loads (the 30-block stack at 4 / 16 / 42 tokens 668 / 808 / 989 us, 666 / 803 / 986 without; 8 x 1024 -> 1024
+    // with a norm 2.94 and 2.88), but a fused GEMV whose workgroups have one row block, which is over sooner, less (1 x 1024 -> 1024 2.61 and 2.64,
+    // 1 x 2048 -> 4096 2.96 and 3.01).
+    template <int MODE, bool ALL = true>
     __device__ __forceinline__ void load(const float *row, const float *row2, uint64_t magics, int head_chunks, const float *gamma, int chunks,
                                          int nw, int wave, int tid, int in_tile)
     {
@@ -420,7 +421,7 @@ struct Row16 {
             if (wave < 4) {
 #pragma unroll
                 for (int i = 0; i < NSS; ++i)
-                    vs[i] = row16_chunk<MODE>(row, row2, magics, head_chunks, min(tid + 256 * i, chunks - 1));
+                    if (ALL || 256 * i < chunks) vs[i] = row16_chunk<MODE>(row, row2, magics, head_chunks, min(tid + 256 * i, chunks - 1));
             }
 #pragma unroll
             for (int i = 0; i < NCHB; ++i) gm[i] = reinterpret_cast<const float4 *>(gamma)[min(chunk[i], chunks - 1)];
