@@ -1,5 +1,9 @@
 // extern "C" entry points: argument validation, error records, and the BitLinear / decoder objects.
 // No arithmetic lives here; every result comes from the kernels behind the launch_* functions.
+#include <unistd.h>
+
+#include <atomic>
+#include <chrono>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -7,8 +11,6 @@
 #include <shared_mutex>
 #include <vector>
 
-#include <atomic>
-#include <random>
 #include "kernels.hpp"
 #include "staging.hpp"
 
@@ -305,8 +307,11 @@ size_t die_flag_bytes(size_t m) { return align_up(sizeof(uint64_t) * GEMV_DIE_SE
 uint64_t next_die_tag()
 {
     static std::atomic<uint64_t> next{[] {
-        std::random_device any;
-        return ((uint64_t)any() << 32 | any()) | ((uint64_t)1 << 63);
+        // std::random_device may throw, and nothing may leave a C entry by an exception: this process's start, number and address space, mixed
+        uint64_t v = (uint64_t)std::chrono::system_clock::now().time_since_epoch().count() ^ (uint64_t)getpid() << 40 ^ (uint64_t)reinterpret_cast<uintptr_t>(&v) << 16;
+        v = (v ^ v >> 30) * 0xbf58476d1ce4e5b9u;  // the mixing steps of SplitMix64 (Steele, Lea, Flood 2014)
+        v = (v ^ v >> 27) * 0x94d049bb133111ebu;
+        return (v ^ v >> 31) | ((uint64_t)1 << 63);
     }()};
     return next.fetch_add(1, std::memory_order_relaxed);
 }

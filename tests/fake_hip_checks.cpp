@@ -61,6 +61,7 @@ struct DieLaunch {
     unsigned stride, m, halves;
 };
 size_t die_launches = 0, stale_flags = 0;
+uint64_t last_tag = 0;
 constexpr unsigned DIES = 16;
 void run(const DieLaunch &l)
 {
@@ -73,6 +74,7 @@ void run(const DieLaunch &l)
         }
     for (unsigned die = 0; l.clear && die < 8 * l.halves; ++die) memset(l.clear + die * l.stride, 0, l.m * sizeof(uint64_t));
     die_launches += l.flags != nullptr;
+    if (l.flags) last_tag = l.tag;
 }
 std::vector<DieLaunch> captured;
 std::map<const void *, std::vector<DieLaunch>> graphs;  // by graph and by executable graph
@@ -519,6 +521,72 @@ void recorded_calls_on_short_rows()
     }
 }
 
+// A call on dies gives its flags a tag that no call before it had, since they lie in whatever memory the workspace is; it needs room for them, and
+// is two launches where a replay would find them up, or where the result lies over the rows.
+void calls_on_dies()
+{
+    bitnet_hip_bitlinear *layer = nullptr;
+    const size_t m = 16, k = 4096, full = 2 * k * k / 4;
+    CHECK(bitnet_hip_bitlinear_create(k, k, 0, &layer) == BITNET_HIP_OK);
+    const std::vector<uint8_t> codes(k * k / 4, 0x22);
+    CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, codes.data(), codes.size(), 0.5f, 0, nullptr) == BITNET_HIP_OK);
+    auto x = DeviceTensor::zeros({m + 1, k}).unwrap(), out = DeviceTensor::zeros({m, k}).unwrap();
+    const size_t dims[2] = {m, k}, plain = bitnet_hip_bitlinear_workspace_size(layer, m);
+    const size_t wanted = bitnet_hip_bitlinear_forward_scratch_on(&layer, 1, x.data(), m, nullptr, BITNET_HIP_SUM_BLOCK256, side);
+    CHECK(wanted > plain && wanted < full);
+    std::vector<uint8_t> ws(full);
+    const auto launches = [&](size_t given, float *to) {
+        fake::calls.clear();
+        fake::die_launches = 0;
+        CHECK(bitnet_hip_bitlinear_forward(layer, x.data(), dims, 2, nullptr, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, to, given ? ws.data() : nullptr, given, nullptr,
+                                           nullptr, nullptr, side) == BITNET_HIP_OK);
+        return fake::count("launch");
+    };
+    CHECK(launches(wanted, out.data()) == 1 && fake::die_launches == 1);
+    const uint64_t tag = fake::last_tag;
+    CHECK(launches(full, out.data()) == 1 && fake::die_launches == 1 && fake::last_tag != tag && tag >> 63 == 1 && fake::last_tag >> 63 == 1);
+    CHECK(launches(wanted - 1, out.data()) == 2 && launches(plain, out.data()) == 2 && launches(0, out.data()) == 2);
+    fake::capturing = side;
+    CHECK(bitnet_hip_bitlinear_forward_scratch_on(&layer, 1, x.data(), m, nullptr, BITNET_HIP_SUM_BLOCK256, side) == plain);
+    CHECK(launches(full, out.data()) == 2);
+    fake::capturing = nullptr;
+    for (float *over : {x.data(), x.data() + k, x.data() + (m - 1) * k})
+        CHECK(launches(full, over) == 2 && fake::die_launches == 0);
+    CHECK(launches(full, x.data()) == 2 && launches(0, x.data()) == 2);
+    bitnet_hip_bitlinear_destroy(layer);
+}
+
+// The launches for few tokens that quantise in every workgroup do not take a result over the rows either, whatever scratch the caller was told of.
+void results_over_the_rows()
+{
+    for (const auto &t : {std::pair<size_t, size_t>{1, 2560}, {1, 8192}, {1, 7424}, {2, 1024}, {8, 2560}, {32, 512}}) {
+        bitnet_hip_bitlinear *layer = nullptr;
+        CHECK(bitnet_hip_bitlinear_create(t.second, t.second, 0, &layer) == BITNET_HIP_OK);
+        const std::vector<uint8_t> codes(t.second * t.second / 4, 0x22);
+        CHECK(bitnet_hip_bitlinear_set_weights_packed(layer, codes.data(), codes.size(), 0.5f, 0, nullptr) == BITNET_HIP_OK);
+        auto x = DeviceTensor::zeros({t.first, t.second}).unwrap(), out = DeviceTensor::zeros({t.first, t.second}).unwrap();
+        const size_t dims[2] = {t.first, t.second};
+        CHECK(bitnet_hip_bitlinear_forward_scratch(layer, x.data(), t.first, nullptr, BITNET_HIP_SUM_BLOCK256) == 0);
+        uint8_t byte[1];
+        for (float *to : {out.data(), x.data()})
+            for (size_t given : {0, 1}) {
+                const size_t launches = to == x.data() ? 2 : 1;
+                fake::calls.clear();
+                CHECK(bitnet_hip_bitlinear_forward(layer, x.data(), dims, 2, nullptr, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, to, given ? byte : nullptr, given,
+                                                   nullptr, nullptr, nullptr, side) == BITNET_HIP_OK);
+                CHECK(fake::count("launch") == launches);
+                fake::calls.clear();
+                CHECK(bitnet_hip_bitlinear_forward_multi(&layer, 1, x.data(), t.first, nullptr, 1e-5f, BITNET_HIP_SUM_BLOCK256, &to, given ? byte : nullptr, given,
+                                                         side) == BITNET_HIP_OK);
+                CHECK(fake::count("launch") == launches);
+                fake::calls.clear();
+                CHECK(bitnet_hip_bitlinear_forward_noalloc(layer, x.data(), dims, 2, nullptr, 1e-5f, BITNET_HIP_SUM_BLOCK256, nullptr, to, side) == BITNET_HIP_OK);
+                CHECK(fake::count("launch") == launches);
+            }
+        bitnet_hip_bitlinear_destroy(layer);
+    }
+}
+
 // A workspace holds the quantised rows and nothing that no kernel reads: workspace_size is what a call of two launches uses.
 void a_workspace_is_what_a_call_uses()
 {
@@ -550,6 +618,8 @@ const Check checks[] = {
     {"chunks_outlive_a_layer_that_used_them", chunks_outlive_a_layer_that_used_them},
     {"gguf_header_is_read_in_stream_order", gguf_header_is_read_in_stream_order},
     {"recorded_calls_on_short_rows", recorded_calls_on_short_rows},
+    {"calls_on_dies", calls_on_dies},
+    {"results_over_the_rows", results_over_the_rows},
     {"a_workspace_is_what_a_call_uses", a_workspace_is_what_a_call_uses},
 };
 
