@@ -203,8 +203,12 @@ template <int MODE>
 int launch_mode(const Fused16Params &p, int nproj, const RowSource &src, size_t blocks, hipStream_t stream)
 {
     const int nw = row_workgroup_waves(src.k), kt = p.kt_count;
-    if (kt <= 32) return src.gamma ? launch<MODE, true, 2, 2>(p, nproj, src, blocks, nw, stream) : launch<MODE, false, 2, 2>(p, nproj, src, blocks, nw, stream);
-    if (src.gamma) return fail(BITNET_HIP_UNSUPPORTED, "streaming GEMV: %d k-tiles with a norm", kt);
+    if (src.gamma) {  // plain rows only, and of up to 32 k-tiles: what gemv_stream_takes and the callers let through
+        if constexpr (MODE == BITNET_HIP_INPUT_PLAIN)
+            if (kt <= 32) return launch<MODE, true, 2, 2>(p, nproj, src, blocks, nw, stream);
+        return fail(BITNET_HIP_UNSUPPORTED, "streaming GEMV: %d k-tiles of input mode %d with a norm", kt, MODE);
+    }
+    if (kt <= 32) return launch<MODE, false, 2, 2>(p, nproj, src, blocks, nw, stream);
     // one row block in flight while a workgroup has few of them: 16384 -> 8192 7.7 us against 8.7, -> 32768 21.6 against 20.7
     return blocks > 4 * STREAM_WORKGROUPS ? launch<MODE, false, 4, 2>(p, nproj, src, blocks, nw, stream) : launch<MODE, false, 4, 1>(p, nproj, src, blocks, nw, stream);
 }
