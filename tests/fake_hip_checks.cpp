@@ -1,7 +1,8 @@
 // Host-side checks of the library and of its C++ mirror against a stand-in for the HIP runtime: no GPU, no kernel runs.  The
 // functions below take the place of the runtime's (the executable's symbols come first), keep device memory on the heap, write down
 // what is called in which order, and can be told to fail.  Each check is named on the command line; `kernels M K N` prints the
-// kernels that M token rows through a K -> N layer launch, by forward and by matmul on quantised rows.
+// kernels that M token rows through a K -> N layer launch, by forward and by matmul on quantised rows; `step M LAYERS HIDDEN FFN KV_HEADS
+// HEAD_DIM` how many launches of a decoder's step quantise their rows once a die.
 #include <hip/hip_runtime.h>
 
 #include <cxxabi.h>
@@ -322,10 +323,10 @@ void loads_wait_for_the_stream_once()
     }
 }
 
-bitnet_hip_decoder *decoder_with_weights(size_t layers, size_t hidden, size_t ffn, size_t tokens = 4)
+bitnet_hip_decoder *decoder_with_weights(size_t layers, size_t hidden, size_t ffn, size_t tokens = 4, size_t kv_heads = 2, size_t head_dim = 16)
 {
     bitnet_hip_decoder *dec = nullptr;
-    CHECK(bitnet_hip_decoder_create(layers, hidden, ffn, hidden / 16, 2, 16, 1e-5f, BITNET_HIP_SUM_BLOCK256, tokens, &dec) == BITNET_HIP_OK);
+    CHECK(bitnet_hip_decoder_create(layers, hidden, ffn, hidden / head_dim, kv_heads, head_dim, 1e-5f, BITNET_HIP_SUM_BLOCK256, tokens, &dec) == BITNET_HIP_OK);
     const std::vector<uint8_t> codes(hidden * (hidden > ffn ? hidden : ffn) / 4, 0x22);
     for (size_t l = 0; l < layers; ++l)
         for (int p = 0; p < 7; ++p) {
@@ -649,6 +650,15 @@ int main(int argc, char **argv)
         const int32_t *sums = reinterpret_cast<const int32_t *>(some.data());
         if (bitnet_hip_bitlinear_matmul(layer, rows, sums, m, some.data(), nullptr, nullptr, some.data(), side) != BITNET_HIP_OK) return 3;
         print("matmul");
+        return 0;
+    }
+    if (argc == 8 && std::string(argv[1]) == "step") {
+        size_t v[6];
+        for (int i = 0; i < 6; ++i) v[i] = std::strtoul(argv[2 + i], nullptr, 10);
+        bitnet_hip_decoder *dec = decoder_with_weights(v[1], v[2], v[3], v[0], v[4], v[5]);
+        std::vector<float> x(v[0] * v[2]), out(v[0] * v[2]);
+        if (failures || bitnet_hip_decoder_decode(dec, x.data(), v[0], out.data(), nullptr, nullptr, side) != BITNET_HIP_OK) return 3;
+        std::printf("%zu\n", fake::die_launches);
         return 0;
     }
     for (const Check &c : checks) {

@@ -4,6 +4,7 @@ Bar: int8 activations, packed bytes and int32 accumulators bit-exact; f32 scales
 bit-exact where the oracle and the kernel perform the same IEEE operations, and in any case within
 1e-5 relative error (the tolerance the path's specification states)."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -2159,13 +2160,17 @@ def test_decoder_blocks_of_many_row_blocks(dims):
         assert np.array_equal(host(graph.out), want)
 
 
-@pytest.mark.parametrize("dims,layers", [((512, 1408, 8, 2, 64), 3), ((2560, 6912, 20, 5, 128), 1)])
+DIE_STACKS = [((512, 1408, 8, 2, 64), 3), ((2560, 6912, 20, 5, 128), 1)]  # dimensions and blocks
+DIE_TOKENS = (9, 33, 16, 3, 64, 17)
+
+
+@pytest.mark.parametrize("dims,layers", DIE_STACKS)
 def test_decoder_rows_quantised_once_a_die(dims, layers):
     """Steps of several token counts, one after the other and recorded, with workgroups that wait for their rows and (no looks at all)
     with every one that quantises its rows itself: all equal the oracle's chain bit for bit."""
     rng = np.random.default_rng(sum(dims))
     dec, ref = build_decoder_packed(rng, layers, *dims, max_tokens=64)
-    for m in (9, 33, 16, 3, 64, 17):
+    for m in DIE_TOKENS:
         xs = synth_activations(rng, m, dims[0])
         want = oracle_stack(ref, xs, *dims)[0]
         for looks in (0, 4096):
@@ -2182,6 +2187,86 @@ def test_decoder_rows_quantised_once_a_die(dims, layers):
     for looks in (-1, 4097):
         with pytest.raises(bh.BitLinearError):
             dec.set_row_wait(looks)
+
+
+@pytest.mark.parametrize("looks", [0, 4096])
+def test_decoder_rows_quantised_once_a_die_of_any_magnitude(looks):
+    """Rows of zeros, of tiny and of huge values and with an infinity: a workgroup that quantises rows for itself divides plainly, those that it waits
+    for by the short division with its own rule, and both give the oracle's bits."""
+    dims = (512, 1408, 8, 2, 64)
+    rng = np.random.default_rng(looks)
+    dec, ref = build_decoder_packed(rng, 3, *dims, max_tokens=64)
+    dec.set_row_wait(looks)
+    xs = synth_activations(rng, 20, dims[0], outliers=True)
+    xs[1] = 0.0
+    xs[2] *= f32(1e-36)
+    xs[3] *= f32(1e18)
+    xs[4, 100] = f32(1e30)
+    xs[5, ::2] = -0.0
+    xs[17] = 0.0
+    xs[18, 7] = np.inf
+    want = oracle_stack(ref, xs, *dims)[0]
+    for _ in range(4):
+        assert np.array_equal(host(dec.decode(dev(xs))), want, equal_nan=True)
+
+
+def test_calls_on_dies_from_several_threads():
+    """Launches whose workgroups wait for each other's rows, from three threads on streams of their own: each call's result is its own."""
+    rng = np.random.default_rng(5)
+    shapes = [(16, 6912, 2560), (9, 2560, 6912), (48, 2560, 5120)]
+    jobs = []
+    for m, k, n in shapes:
+        packed = random_packed_ternary(rng, 1, n * k)
+        layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "threads")
+        layer.set_quantized_weights(torch.from_numpy(packed), 0.02)
+        xs = [synth_activations(rng, m, k) for _ in range(3)]
+        jobs.append((layer, [dev(x) for x in xs], [dev(orc.bitlinear_forward(x, packed, n, f32(0.02))[0]) for x in xs]))
+        wanted, plain = die_scratch(layer, jobs[-1][1][0])
+        assert wanted > plain
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(layer, xs, wants):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for i in range(60):
+                y = layer.forward(xs[i % 3])
+                if not torch.equal(y, wants[i % 3]):
+                    wrong.append((layer.config.in_features, i))
+
+    threads = [threading.Thread(target=work, args=job) for job in jobs]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=100)
+    assert not any(th.is_alive() for th in threads) and not wrong
+
+
+def test_a_captured_call_with_room_for_flags():
+    """Flags in the workspace would be up in a second replay: a captured call takes two launches, and every replay multiplies its own rows, with
+    calls on the same workspace between the replays."""
+    rng = np.random.default_rng(6)
+    m, k, n = 16, 6912, 2560
+    packed = random_packed_ternary(rng, 1, n * k)
+    layer = bh.BitLinear(bh.BitLinearConfig(in_features=k, out_features=n), "captured")
+    layer.set_quantized_weights(torch.from_numpy(packed), 0.02)
+    x, out = torch.zeros((m, k), device="cuda"), torch.empty((m, n), device="cuda")
+    wanted, plain = die_scratch(layer, x)
+    scratch = torch.empty((wanted,), dtype=torch.uint8, device="cuda")
+    layer.forward(x, out=out, workspace=scratch)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        layer.forward(x, out=out, workspace=scratch)
+    for i in range(4):
+        xs = synth_activations(rng, m, k)
+        want = orc.bitlinear_forward(xs, packed, n, f32(0.02))[0]
+        x.copy_(dev(xs))
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(host(out), want)
+        assert np.array_equal(host(layer.forward(x, workspace=scratch)), want)
 
 
 # ---- outputs over the input ----------------------------------------------------------------------------------

@@ -7,7 +7,7 @@ from pathlib import Path
 import pytest
 
 import bitnet_hip as bh
-from test_gpu_parity import ONE_ROUND, ONE_ROUND_K
+from test_gpu_parity import DIE_STACKS, DIE_TOKENS, ONE_ROUND, ONE_ROUND_K
 
 SOURCE = Path(__file__).with_name("fake_hip_checks.cpp")
 CHECKS = re.findall(r'^    \{"(\w+)", \1\},$', SOURCE.read_text(), flags=re.M)
@@ -61,3 +61,16 @@ def test_the_shapes_of_the_one_round_gemm_test_reach_every_tile(program):
                 if tile and m % int(tile[1]) and n % int(tile[2]):
                     cut[call].add(tile.groups())
         assert cut["forward"] == cut["matmul"] == set(tiles)
+
+
+@pytest.mark.parametrize("dims,layers", DIE_STACKS)
+def test_the_steps_of_the_die_test_run_on_dies(program, dims, layers):
+    """Of the token counts with which the GPU test compares such steps with the oracle, at least half launch kernels that quantise rows once a die (the
+    three blocks an odd number of them)."""
+    hidden, ffn, _, kv_heads, head_dim = dims
+    counts = []
+    for m in DIE_TOKENS:
+        done = subprocess.run([str(program), "step"] + [str(v) for v in (m, layers, hidden, ffn, kv_heads, head_dim)], capture_output=True, text=True, timeout=60)
+        assert done.returncode == 0, done.stdout + done.stderr
+        counts.append(int(done.stdout))
+    assert sum(c > 0 for c in counts) >= 3 and (layers != 3 or all(c % 2 for c in counts if c)), dict(zip(DIE_TOKENS, counts))
