@@ -8,8 +8,8 @@
 // weight tiles at once and multiply when the rows of their token group have reached the die's L2.  What a launch takes is a row's way
 // through the quantiser (2.9 us with a norm, 2.2 without), the hand-over (0.7) and the products, exchange and epilogue of
 // gemv_rows_kernel (2.5).  gate + up of 2560 -> 2 x 6912 at 8 tokens: 6.0 us from its first workgroup to its last, where quantiser and GEMV
-// took 7.4 with the gap between them.  The 30-block stack of 2560 columns, recorded, at 3 / 4 / 8 / 12 / 16 / 24 / 32 / 42 / 64 tokens: 605 / 665 /
-// 743 / 787 / 815 / 879 / 910 / 995 / 1108 us before, 554 / 585 / 641 / 668 / 702 / 790 / 819 / 945 / 1089 with it.  Calls of their own, us:
+// took 7.4 with the gap between them.  The 30-block stack of 2560 columns, recorded, at 2 / 3 / 4 / 8 / 12 / 16 / 24 / 32 / 42 / 64 tokens: 548 /
+// 605 / 665 / 743 / 787 / 815 / 879 / 910 / 995 / 1108 us before, 543 / 550 / 580 / 629 / 668 / 702 / 790 / 819 / 945 / 1089 with it.  Calls of their own, us:
 // 16 x 6912 -> 2560 7.9 -> 5.6, 32 x 4096 -> 5120 7.8 -> 5.8, 64 x 2560 -> 2560 with norm 8.1 -> 6.2.  (A first form, in which workgroups with
 // products took the rows beside them, was 0.5 to 2 us slower a launch: their tiles came late, and a row's registers beside the tiles' left
 // room for fewer workgroups.)
@@ -330,7 +330,9 @@ bool gemv_die_takes(const float *x, const float *x2, size_t ldx, size_t m, size_
     // norm: 2560 -> 5120 at 64 tokens (1.1 times the slots) 8.0 -> 6.7, 8.2 -> 8.3; 4096 -> 13824 at 32 (1.3) 8.9 -> 8.1, 9.3 -> 9.8; 2560 -> 5120 at 95
     // (1.6) 8.0 -> 8.3, 8.3 -> 9.2; with one workgroup a compute unit 6912 -> 5120 at 32 (1.6) 8.7 -> 8.3, 9.4 -> 9.2, 6912 -> 13824 at 24 (2.4)
     // 12.7 -> 13.1, 13.6 -> 14.0; long rows of many tokens, whose quantisers fill the die: 8192 -> 640 at 48 7.8 -> 7.3, 8.0 -> 9.2, at 64
-    // 7.8 -> 8.2, 8.2 -> 10.1.
+    // 7.8 -> 8.2, 8.2 -> 10.1.  With calls on a second stream beside it, both queued behind long work, the rows' eight copies take the other's compute
+    // units: 48 x 2560 -> 5120 3.7 -> 4.5 us a call, 32 x 6912 -> 5120 5.6 -> 6.2, 24 x 4096 -> 4096 3.75 -> 3.7, 16 x 6912 -> 2560 3.8 -> 3.5; as the host's calls
+    // come from one thread, on one to four streams, 14 -> 11 for each.
     if (s.nt == 2 && m > (gamma ? 32u : 48u)) return false;
     return 20 * total <= (s.slots == DIE_CUS ? 33 : (gamma ? 23 : 28)) * s.slots;
 }
