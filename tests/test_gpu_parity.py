@@ -2191,7 +2191,7 @@ def test_decoder_rows_quantised_once_a_die(dims, layers):
 
 @pytest.mark.parametrize("looks", [0, 4096])
 def test_decoder_rows_quantised_once_a_die_of_any_magnitude(looks):
-    """Rows of zeros, of tiny and of huge values and with an infinity: a workgroup that quantises rows for itself divides plainly, those that it waits
+    """Rows of zeros, of tiny and of huge values, with an infinity and with a NaN: a workgroup that quantises rows for itself divides plainly, those that it waits
     for by the short division with its own rule, and both give the oracle's bits."""
     dims = (512, 1408, 8, 2, 64)
     rng = np.random.default_rng(looks)
@@ -2205,6 +2205,7 @@ def test_decoder_rows_quantised_once_a_die_of_any_magnitude(looks):
     xs[5, ::2] = -0.0
     xs[17] = 0.0
     xs[18, 7] = np.inf
+    xs[19, 3] = np.nan
     want = oracle_stack(ref, xs, *dims)[0]
     for _ in range(4):
         assert np.array_equal(host(dec.decode(dev(xs))), want, equal_nan=True)
